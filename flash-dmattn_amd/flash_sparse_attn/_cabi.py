@@ -7,6 +7,8 @@ CPU or eager fallback behind it.
 """
 import contextlib
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import struct
 from typing import Optional, Sequence
@@ -241,6 +243,31 @@ def _load() -> ctypes.CDLL:
 
 
 lib = _load()
+
+
+_HOST_PATH = os.path.normpath(os.path.join(_HERE, "..", "lib", "_fdma_torch.so"))
+_HOST_CALLS = (
+    "fdma_fwd", "fdma_bwd", "fdma_fwd_workspace_bytes", "fdma_bwd_workspace_bytes", "fdma_fwd_counter_bytes",
+    "fdma_set_stream_min_items", "fdma_varlen_fwd", "fdma_varlen_bwd", "fdma_create_mask", "fdma_dyn_bias_fwd",
+    "fdma_dyn_bias_bwd", "fdma_dyn_bias_bwd_workspace_bytes", "fdma_last_error",
+)
+
+
+def _load_host():
+    """The native host path of the operators (csrc/fdma_torch.cpp), bound to the functions of `lib`: the calls it takes
+    skip the Python below, the others it answers with NotImplemented."""
+    if not os.path.exists(_HOST_PATH):
+        raise ImportError(f"{_HOST_PATH} not found: build it with `make -C flash-dmattn_amd/csrc` (or __graft_entry__.build()); "
+                          "there is no fallback implementation")
+    loader = importlib.machinery.ExtensionFileLoader("_fdma_torch", _HOST_PATH)
+    spec = importlib.util.spec_from_loader("_fdma_torch", loader)
+    mod = importlib.util.module_from_spec(spec)
+    loader.exec_module(mod)
+    mod.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _HOST_CALLS})
+    return mod
+
+
+host = _load_host()
 
 
 def last_error() -> str:

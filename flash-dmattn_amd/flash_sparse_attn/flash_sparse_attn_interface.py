@@ -663,6 +663,11 @@ def flash_sparse_attn_func(
         softmax_lse [optional]: (batch_size, nheads, seqlen), fp32 logsumexp of each score row
             (+inf for rows with no visible key).
     """
+    if not torch.compiler.is_compiling():
+        out = _cabi.host.attention(query, key, value, attn_mask, attn_bias, softmax_scale, is_causal, softcap, deterministic,
+                                   return_attn_probs, _cabi._compact_mode)
+        if out is not NotImplemented:  # (an ordinary call: it has been made; what follows is for all others)
+            return out
     grad_enabled = torch.is_grad_enabled()
     attn_mask, is_causal = _column_causal_form(attn_mask, attn_bias, query, key, is_causal)
     args = (query, key, value, attn_mask, attn_bias, softmax_scale, is_causal, softcap, deterministic, return_attn_probs,
@@ -895,6 +900,11 @@ def flash_sparse_attn_varlen_func(
     Returns out (total_q, nheads, headdim), or (out, softmax_lse (nheads, total_q), S_dmask (empty)) when
     `return_attn_probs` is set.  Paged KV (`block_table`) and softcapping raise RuntimeError.
     """
+    if not torch.compiler.is_compiling():
+        out = _cabi.host.varlen_attention(query, key, value, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale,
+                                          is_causal, softcap, deterministic, return_attn_probs, block_table)
+        if out is not NotImplemented:
+            return out
     grad_enabled = torch.is_grad_enabled()
     args = (query, key, value, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, is_causal, softcap,
             deterministic, return_attn_probs, block_table, grad_enabled)

@@ -124,6 +124,12 @@ def dynamic_mask_bias(
     Returns (batch, num_kv_heads, 1, key_len) in the dtype of value_states, ready to be passed as `attn_bias`
     (and to `create_mask`).  Differentiable in all four inputs.
     """
+    if value_states.is_cuda and not torch.compiler.is_compiling():
+        from .. import _cabi
+
+        bias = _cabi.host.dyn_bias(value_states, dt_proj_weight, A, dt_proj_bias)
+        if bias is not NotImplemented:
+            return bias
     if _native_ok(value_states, dt_proj_weight, A, dt_proj_bias) and value_states.shape[0] * value_states.shape[1] > 0:
         return _DynamicMaskBias.apply(value_states, dt_proj_weight, A, dt_proj_bias)
     return _tensor_program(value_states, dt_proj_weight, A, dt_proj_bias)

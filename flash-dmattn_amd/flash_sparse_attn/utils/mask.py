@@ -57,6 +57,10 @@ def _native_mask(attention_bias, attention_mask, window_size, min_dtype, block_s
         return None
     from .. import _cabi
 
+    if not torch.compiler.is_compiling():
+        keep = _cabi.host.create_mask(attention_bias, attention_mask, window_size, min_dtype, block_size, 0 if kind == "topk" else 1)
+        if keep is not NotImplemented:
+            return keep
     bias = attention_bias.detach()
     shape = tuple(bias.shape) if attention_mask is None else tuple(torch.broadcast_shapes(bias.shape, attention_mask.shape))
     if kind == "topk" and window_size > shape[-1]:

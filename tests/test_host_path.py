@@ -1,0 +1,114 @@
+"""The native host path (csrc/fdma_torch.cpp) against the general Python path it stands in for: the same kernels are
+launched with the same arguments, so outputs and gradients agree bit for bit; calls it was not made for are declined."""
+import pytest
+import torch
+
+DEV = "cuda"
+
+
+def _host():
+    from flash_sparse_attn import _cabi
+    return _cabi.host
+
+
+def test_declines_what_is_not_an_ordinary_device_tensor():
+    q = torch.randn(1, 8, 2, 64, dtype=torch.bfloat16)
+    cu = torch.tensor([0, 8], dtype=torch.int32)
+    assert _host().attention(q, q, q, None, None, None, None, None, None, None, 0) is NotImplemented
+    assert _host().varlen_attention(q[0], q[0], q[0], cu, cu, 8, 8, None, None, None, None, None, None) is NotImplemented
+    assert _host().create_mask(q, None, 4, -1.0, None, 0) is NotImplemented
+    assert _host().dyn_bias(q, q, q, None) is NotImplemented
+    assert _host().attention("q", q, q, None, None, None, None, None, None, None, 0) is NotImplemented
+
+
+def _inputs(B, Lq, Lk, H, Hk, d, rows, dtype, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    def randn(*s): return torch.randn(*s, generator=g, device=DEV).to(dtype)
+    bias = randn(B, Hk, rows, Lk)
+    mask = torch.rand(bias.shape, generator=g, device=DEV) < 0.4
+    return randn(B, Lq, H, d), randn(B, Lk, Hk, d), randn(B, Lk, Hk, d), mask, bias, randn(B, Lq, H, d)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,d,rows,dtype", [
+    (2, 96, 96, 4, 2, 64, 1, torch.bfloat16),     # column mask, tile skipping
+    (1, 512, 1024, 8, 2, 128, 1, torch.float16),  # column mask, compaction (forward workspace reused)
+    (2, 64, 128, 4, 2, 64, 64, torch.bfloat16),   # a mask and bias row per query
+    (3, 1, 4096, 8, 2, 128, 1, torch.bfloat16),   # split-KV decode with its counters
+])
+def test_attention_equals_the_general_path(B, Lq, Lk, H, Hk, d, rows, dtype):
+    from flash_sparse_attn import flash_sparse_attn_interface as itf
+
+    q, k, v, mask, bias, dout = _inputs(B, Lq, Lk, H, Hk, d, rows, dtype)
+    causal = Lq > 1
+    leaves = [t.clone().requires_grad_(True) for t in (q, k, v, bias)]
+    a = _host().attention(leaves[0], leaves[1], leaves[2], mask, leaves[3], None, causal, None, None, None, 0)
+    assert a is not NotImplemented and a.grad_fn is not None
+    b = itf.FlashDMAttnFunc.apply(leaves[0], leaves[1], leaves[2], mask, leaves[3], None, causal, None, None, None)
+    assert torch.equal(a, b)
+    if Lq > 1:
+        ga = torch.autograd.grad(a, leaves, dout)
+        for x, y in zip(ga, torch.autograd.grad(b, leaves, dout)):
+            assert torch.equal(x, y)
+        # an expanded gradient (loss = out.sum()), q without one, and a second backward through a freed graph
+        c = _host().attention(q, leaves[1], leaves[2], mask, leaves[3], 0.1, causal, 0.0, False, False, 0)
+        c.sum().backward()
+        assert leaves[1].grad is not None and leaves[0].grad is None
+        with pytest.raises(RuntimeError, match="second time"):
+            c.sum().backward()
+    with torch.no_grad():
+        n = _host().attention(q, k, v, mask, bias, None, causal, None, None, None, 0)
+        assert torch.equal(n, a.detach()) and n.grad_fn is None
+    with torch.inference_mode():
+        assert torch.equal(_host().attention(q, k, v, mask, bias, None, causal, None, None, None, 0), n)
+
+
+@pytest.mark.gpu
+def test_in_place_change_of_a_saved_input_is_noticed():
+    q, k, v, mask, bias, dout = _inputs(1, 64, 64, 2, 1, 64, 1, torch.bfloat16)
+    k = k.requires_grad_(True)
+    out = _host().attention(q, k, v, mask, bias, None, True, None, None, None, 0)
+    q.add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.backward(dout)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_ragged_batch_equals_the_general_path(dtype):
+    from flash_sparse_attn import flash_sparse_attn_interface as itf
+
+    lens, H, Hk, d = [5, 130, 1, 64], 4, 2, 64
+    g = torch.Generator(device=DEV).manual_seed(1)
+    leaves = [torch.randn(sum(lens), h, d, generator=g, device=DEV).to(dtype).requires_grad_(True) for h in (H, Hk, Hk)]
+    cu = torch.tensor([0, 5, 135, 136, 200], dtype=torch.int32, device=DEV)
+    a = _host().varlen_attention(*leaves, cu, cu, 130, 130, None, True, None, None, None, None)
+    b = itf.FlashAttnVarlenFunc.apply(*leaves, cu, cu, 130, 130, None, True, None, None, None, None)
+    assert torch.equal(a, b)
+    dout = torch.randn(a.shape, generator=g, device=DEV).to(dtype)
+    for x, y in zip(torch.autograd.grad(a, leaves, dout), torch.autograd.grad(b, leaves, dout)):
+        assert torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,pb", [(64, True), (131, False)])
+def test_bias_producer_and_mask_builder_equal_the_general_path(L, pb):
+    from flash_sparse_attn.utils import bias as B, mask as M
+
+    g = torch.Generator(device=DEV).manual_seed(2)
+    def leaf(*s): return torch.randn(*s, generator=g, device=DEV).bfloat16().requires_grad_(True)
+    ins = [leaf(2, L, 4, 64), leaf(4, 256), leaf(4)] + ([leaf(4)] if pb else [])
+    a = _host().dyn_bias(*ins, *([] if pb else [None]))
+    b = B._DynamicMaskBias.apply(*ins, *([] if pb else [None]))
+    assert a.shape == b.shape and torch.equal(a, b)
+    up = torch.randn(a.shape, generator=g, device=DEV).bfloat16()
+    for x, y in zip(torch.autograd.grad(a, ins, up), torch.autograd.grad(b, ins, up)):
+        assert torch.equal(x, y)
+    keep = _host().create_mask(a, None, 40, torch.finfo(a.dtype).min, None, 0)
+    assert int(keep.sum()) == 40 * 2 * 4
+    idx, cnt, count, ld = M.kept_keys_of(keep)  # the record is the one the Python side reads
+    assert ld % 16 == 0 and count.tolist() == [40] * 8
+    row = idx[0, :40].long()
+    assert keep[0, 0, 0, row].all() and torch.equal(row, row.sort().values)
+    keep[0, 0, 0, 0] = ~keep[0, 0, 0, 0]
+    assert M.kept_keys_of(keep) is None
