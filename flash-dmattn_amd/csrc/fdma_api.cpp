@@ -20,6 +20,7 @@ namespace {
 
 thread_local char g_err[512] = "";
 
+constexpr int32_t kMaxColumnFormKeys = 1 << 19;        // what both column-mask directions take (fwd / bwd_colmask_applicable)
 constexpr int64_t kMaxRowStride = (int64_t)1 << 24;  // elements
 
 int fail(int code, const char *fmt, ...) {
@@ -78,18 +79,23 @@ int validate_common(const fdma_fwd_args *a, bool backward) {
     if (!a->q || ((!a->k || !a->v) && a->seqlen_k > 0)) return fail(FDMA_ERR_INVALID, "q, k, v must be device pointers");
     if (!a->out) return fail(FDMA_ERR_INVALID, "out must be a device pointer");
     if (!a->lse) return fail(FDMA_ERR_INVALID, "softmax_lse must be a device pointer");
+    // Rows that all queries share (and a single query's rows) are read element by element or with unaligned loads that
+    // stay inside the row: any address and stride will do.  Rows per query are read in aligned 16-byte vectors.
+    const bool elementwise = a->seqlen_q == 1 || ((!a->mask || a->mask_strides[2] == 0) && (!a->bias || a->bias_strides[2] == 0) &&
+                                                  a->seqlen_k <= kMaxColumnFormKeys);
     if (a->mask) {
         const int hm = a->num_heads_mask;
         if (!(hm == 1 || hm == a->num_heads_k || hm == a->num_heads))
             return fail(FDMA_ERR_INVALID, "Number of heads in mask must be 1, h_k or h");
-        if (!aligned16(a->mask) || !strides_ok(a->mask_strides, 16))
+        if (!elementwise && (!aligned16(a->mask) || !strides_ok(a->mask_strides, 16)))
             return fail(FDMA_ERR_INVALID, "mask must be 16-byte aligned with strides that are multiples of 16 (pad the key dimension)");
     }
     if (a->bias) {
         const int hb = a->num_heads_bias;
         if (!(hb == 1 || hb == a->num_heads_k || hb == a->num_heads))
             return fail(FDMA_ERR_INVALID, "Number of heads in bias must be 1, h_k or h");
-        if (!aligned16(a->bias) || !strides_ok(a->bias_strides, 8))
+        if (elementwise && (reinterpret_cast<uintptr_t>(a->bias) & 1)) return fail(FDMA_ERR_INVALID, "bias must be 2-byte aligned");
+        if (!elementwise && (!aligned16(a->bias) || !strides_ok(a->bias_strides, 8)))
             return fail(FDMA_ERR_INVALID, "bias must be 16-byte aligned with strides that are multiples of 8 (pad the key dimension)");
     }
     if (!aligned16(a->q) || !aligned16(a->k) || !aligned16(a->v) || !aligned16(a->out) || !strides_ok(a->q_strides, 8) ||

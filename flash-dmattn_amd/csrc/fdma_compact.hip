@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) compact_scan_kernel(const FwdPar
     const int pair = blockIdx.x, b = pair / p.Hk, hk = pair % p.Hk;
     const int hm = p.Hm == 1 ? 0 : hk;
     scan_mask_row<SCAN_THREADS>(p.mask + b * p.m_b + hm * p.m_h, p.Lk, idx + (size_t)pair * ld, cnt + (size_t)pair * ld,
-                                count + pair, s_wave, true);
+                                count + pair, s_wave);
 }
 
 // orig: the caller's tensors.  kc / vc: dense [B*Hk, Lk, d] destinations.
@@ -178,10 +178,10 @@ __global__ void __launch_bounds__(256) compact_scan_gather_kernel(const FwdParam
     const uint8_t *mrow = p.mask + b * p.m_b + hm * p.m_h;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int s0 = blockIdx.x * SEG_KEYS;
-    // kept columns in front of the segment (s0 is a multiple of 16; mask rows are readable in 16-byte pieces)
+    // kept columns in front of the segment
     int before = 0;
     for (int c = tid * 16; c < s0; c += 256 * 16) {
-        const u32x4_t mv = *(const u32x4_t *)(mrow + c);
+        const u32x4_t mv = ld_row16(mrow, c, p.Lk);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             // a byte is non-zero <=> bit 7 of ((x & 0x7f) + 0x7f) | x is set
@@ -311,18 +311,17 @@ __global__ void __launch_bounds__(256) compact_image_kernel(const FwdParams p, i
         for (int w = 0; w < KEEP; w++) held[w] = u32x4_t{0, 0, 0, 0};
         int mine = 0;
         if (keep) {
+            int cc[KEEP];
 #pragma unroll
-            for (int w = 0; w < KEEP; w++) {
-                const int c = c0 + 16 * w;
-                if (w * 16 < cpt && c < c1) held[w] = *(const u32x4_t *)(mrow + c);
-            }
+            for (int w = 0; w < KEEP; w++) cc[w] = w * 16 < cpt && c0 + 16 * w < c1 ? c0 + 16 * w : p.Lk;
+            ld_row16(mrow, cc, p.Lk, held);
 #pragma unroll
             for (int w = 0; w < KEEP; w++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) mine += __builtin_popcount(kept_bits(held[w][e], c0 + 16 * w + 4 * e));
         } else {
             for (int c = c0; c < c1; c += 16) {
-                const u32x4_t mv = *(const u32x4_t *)(mrow + c);
+                const u32x4_t mv = ld_row16(mrow, c, p.Lk);
 #pragma unroll
                 for (int e = 0; e < 4; e++) mine += __builtin_popcount(kept_bits(mv[e], c + 4 * e));
             }
@@ -372,7 +371,7 @@ __global__ void __launch_bounds__(256) compact_image_kernel(const FwdParams p, i
                 for (int w = 0; w < KEEP; w++)
                     if (c0 + 16 * w < c1) walk(held[w], c0 + 16 * w);
             } else {
-                for (int c = c0; c < c1; c += 16) walk(*(const u32x4_t *)(mrow + c), c);
+                for (int c = c0; c < c1; c += 16) walk(ld_row16(mrow, c, p.Lk), c);
             }
         }
         // (columns from Lk to the end of the row repeat the total)
@@ -479,11 +478,10 @@ __global__ void __launch_bounds__(256) compact_scan_image_kernel(const FwdParams
     int before = 0;
     for (int c = tid * 16; c < s0; c += 4 * 256 * 16) {
         u32x4_t mv[4];
+        int cc[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int cc = c + u * 256 * 16;
-            mv[u] = cc < s0 ? *(const u32x4_t *)(mrow + cc) : u32x4_t{0, 0, 0, 0};
-        }
+        for (int u = 0; u < 4; u++) cc[u] = c + u * 256 * 16 < s0 ? c + u * 256 * 16 : p.Lk;  // (at the end of the row: zeros)
+        ld_row16(mrow, cc, p.Lk, mv);
 #pragma unroll
         for (int u = 0; u < 4; u++)
 #pragma unroll

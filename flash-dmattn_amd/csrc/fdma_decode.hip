@@ -15,6 +15,8 @@
 // every gathered row is used by all of them: a wave stages 32 gathered K and V rows in its own
 // piece of LDS (no barrier: nobody else reads it), S^T = K Q^T and O^T += V^T P^T run on the matrix
 // pipe, and the vector ALU is left with one exp2 per (key, column).
+#include <type_traits>
+
 #include "fdma_common.h"
 #include "fdma_params.h"
 
@@ -27,6 +29,7 @@ constexpr int DEC_RANGE = 16 * DEC_THREADS;  // keys compacted per pass (16 per 
 constexpr int DEC_NJ = 4;                    // sub-ranges per pass: the mask of 4 x 4096 keys is fetched in one go
 constexpr int DEC_SUPER = DEC_NJ * DEC_RANGE;
 static_assert(DEC_NJ == 4, "the list builder selects among four mask words");
+constexpr int DEC_LIST = DEC_RANGE / 2;       // LISTS: keys per pass (whole column numbers in the same LDS)
 constexpr int DEC_TILE = 32;                 // gathered keys per wave and step
 constexpr int DEC_COLS = 32;                 // query heads per workgroup (columns of the MFMA tile)
 
@@ -61,6 +64,9 @@ __device__ __forceinline__ uint32_t nz_bytes_to_bits(uint32_t x) {
     return ((y >> 7) * 0x10204080u) >> 28;
 }
 
+// LISTS: the caller has handed over the ordered list of kept keys (fdma_kept_keys: the mask builder writes it).  A
+// workgroup then takes its share of the LIST instead of a range of keys and builds nothing: one trip to memory less in a
+// chain of six, and every split has the same number of rows whatever the mask looks like.
 // PERHEAD: mask or bias differ between the query heads of a group, so a lane fetches the mask byte and the
 // bias of its own (key, head) pairs; otherwise one fused value per key serves all columns.
 // out[b,h,:] = sum_s exp(lse_s - lse) * o_s ;  lse = logsumexp_s lse_s  (empty everywhere: 0 / +inf) for one (b, h) row,
@@ -131,7 +137,7 @@ __device__ __forceinline__ void combine_row(const FwdParams &p, int64_t row, int
     __builtin_amdgcn_wave_barrier();  // (s_w is rewritten for the wave's next row)
 }
 
-template <typename T, int D, bool PERHEAD, bool WIDE>
+template <typename T, int D, bool PERHEAD, bool WIDE, bool LISTS>
 __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(const FwdParams p, int keys_per_split) {
     using E = Elem<T>;
     using SM = DecSmem<D>;
@@ -155,14 +161,24 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
     const int h = hk * G + g0 + (col_ok ? r : 0);     // this lane's query head
     const int nchunk = p.d / 8;
 
-    uint16_t *s_idx = (uint16_t *)(smem + SM::OFF_IDX);  // kept keys of the current pass, relative to its first key
+    using Idx = std::conditional_t<LISTS, uint32_t, uint16_t>;
+    Idx *s_idx = (Idx *)(smem + SM::OFF_IDX);  // kept keys of the current pass, relative to its first key (LISTS: absolute)
     char *sK = smem + wave * SM::WAVE_BYTES;
     char *sV = sK + SM::TILE_BYTES;
     float *sB = (float *)(sV + SM::TILE_BYTES);
 
-    const int lo = split * keys_per_split;
-    int hi = lo + keys_per_split;
+    int lo = split * keys_per_split, hi = lo + keys_per_split;
     if (hi > p.Lk) hi = p.Lk;
+    const int32_t *list = nullptr;
+    if (LISTS) {  // this workgroup's share of the list
+        const int srow = (p.m_b == 0 ? 0 : b) * p.Hm + (p.Hm == 1 ? 0 : hk);
+        int n = p.kept_count[srow];  // (lists are device data the host cannot check: held inside the key axis)
+        n = n < 0 ? 0 : (n < p.Lk ? n : p.Lk);
+        list = p.kept_idx + (int64_t)srow * p.kept_ld;
+        const int per = (n + p.splits - 1) / p.splits;
+        lo = split * per < n ? split * per : n;
+        hi = lo + per < n ? lo + per : n;
+    }
 
     // B operands of S^T = K Q^T: lane supplies Q[head r][16 ks + 8 g .. + 7]; columns without a head are zero
     u32x4_t qf[KS];
@@ -208,41 +224,41 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
         return (gptr_t)(((uint64_t)hi32 << 32) | lo32);
     };
 
-    for (int r0 = lo; r0 < hi; r0 += DEC_SUPER) {
-        // ---- phase 1: ordered list of the kept keys of [r0, r0 + DEC_SUPER).  A thread tests 16 keys of each of
-        // the DEC_NJ sub-ranges (one 16-byte mask load per mask row, all of them in flight together); wave scans
-        // and one barrier order the output.  Entries are relative to r0.
-        uint32_t bits[DEC_NJ];
-        {
-            u32x4_t mv[DEC_NJ];
+    // phase 1: the ordered list of the kept keys of a pass
+    uint32_t bits[DEC_NJ];
+    auto scan_pass = [&](int r0, int nj) {
+        // the keys of [r0, r0 + DEC_SUPER): a thread tests 16 keys of each of the DEC_NJ sub-ranges (one 16-byte mask load
+        // per mask row, all of them in flight together); wave scans and one barrier order the output, relative to r0
+        u32x4_t mv[DEC_NJ];
+        int key0[DEC_NJ];
 #pragma unroll
-            for (int j = 0; j < DEC_NJ; j++) {
-                const int key0 = r0 + j * DEC_RANGE + 16 * tid;
-                mv[j] = u32x4_t{0, 0, 0, 0};
-                if (key0 < hi) {
-                    if (!p.mask) {
-                        mv[j] = u32x4_t{~0u, ~0u, ~0u, ~0u};
-                    } else if (!PERHEAD || p.Hm != p.H) {
-                        mv[j] = *(const u32x4_t *)(p.mask + b * p.m_b + (int64_t)(p.Hm == 1 ? 0 : hk) * p.m_h + key0);
-                    } else {  // union of the mask rows of this workgroup's columns
-                        for (int q = 0; q < ncol; q++) {
-                            const u32x4_t x = *(const u32x4_t *)(p.mask + b * p.m_b + (int64_t)(hk * G + g0 + q) * p.m_h + key0);
+        for (int j = 0; j < DEC_NJ; j++) {
+            key0[j] = r0 + j * DEC_RANGE + 16 * tid;
+            key0[j] = key0[j] < hi ? key0[j] : lo;  // (beyond the range: any piece of it, dropped below)
+            mv[j] = u32x4_t{~0u, ~0u, ~0u, ~0u};
+        }
+        if (p.mask && (!PERHEAD || p.Hm != p.H)) {
+            ld_row16(p.mask + b * p.m_b + (int64_t)(p.Hm == 1 ? 0 : hk) * p.m_h, key0, p.Lk, mv);
+        } else if (p.mask) {  // union of the mask rows of this workgroup's columns
 #pragma unroll
-                            for (int e = 0; e < 4; e++) mv[j][e] |= x[e];
-                        }
-                    }
-                }
-            }
+            for (int j = 0; j < DEC_NJ; j++) mv[j] = u32x4_t{0, 0, 0, 0};
+            for (int q = 0; q < ncol; q++) {
+                u32x4_t x[DEC_NJ];
+                ld_row16(p.mask + b * p.m_b + (int64_t)(hk * G + g0 + q) * p.m_h, key0, p.Lk, x);
 #pragma unroll
-            for (int j = 0; j < DEC_NJ; j++) {
-                const int nval = hi - (r0 + j * DEC_RANGE + 16 * tid);  // keys of this thread inside the range
-                const uint32_t inrange = nval >= 16 ? 0xffffu : (nval <= 0 ? 0u : ((1u << nval) - 1u));
-                bits[j] = (nz_bytes_to_bits(mv[j][0]) | (nz_bytes_to_bits(mv[j][1]) << 4) | (nz_bytes_to_bits(mv[j][2]) << 8) |
-                           (nz_bytes_to_bits(mv[j][3]) << 12)) & inrange;
+                for (int j = 0; j < DEC_NJ; j++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) mv[j][e] |= x[j][e];
             }
         }
+#pragma unroll
+        for (int j = 0; j < DEC_NJ; j++) {
+            const int nval = hi - (r0 + j * DEC_RANGE + 16 * tid);  // keys of this thread inside the range
+            const uint32_t inrange = nval >= 16 ? 0xffffu : (nval <= 0 ? 0u : ((1u << nval) - 1u));
+            bits[j] = (nz_bytes_to_bits(mv[j][0]) | (nz_bytes_to_bits(mv[j][1]) << 4) | (nz_bytes_to_bits(mv[j][2]) << 8) |
+                       (nz_bytes_to_bits(mv[j][3]) << 12)) & inrange;
+        }
         // bits[j] also carries, in its upper half, the kept keys of the lower lanes of this wave in sub-range j
-        const int nj = (hi - r0 + DEC_RANGE - 1) / DEC_RANGE < DEC_NJ ? (hi - r0 + DEC_RANGE - 1) / DEC_RANGE : DEC_NJ;
 #pragma unroll
         for (int j = 0; j < DEC_NJ; j++) {
             if (j < nj) {
@@ -254,11 +270,17 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
             }
         }
         __syncthreads();
+    };
+
+    for (int r0 = lo; r0 < hi; r0 += LISTS ? DEC_LIST : DEC_SUPER) {
+        const int nj = (hi - r0 + DEC_RANGE - 1) / DEC_RANGE < DEC_NJ ? (hi - r0 + DEC_RANGE - 1) / DEC_RANGE : DEC_NJ;
+        if (!LISTS) scan_pass(r0, nj);
+        const int key_base = LISTS ? 0 : r0;  // what the list's entries are relative to
 
         // ---- phase 2 (called once the list is complete): a wave takes every fourth batch of 32 kept keys.  The
         // rows of the next batch are in flight (in registers) while the current one is worked on from LDS.
-        const gptr_t kb0 = uniform_ptr(kbase + (int64_t)r0 * p.k_r), vb0 = uniform_ptr(vbase + (int64_t)r0 * p.v_r);
-        const gptr_t bb0 = uniform_ptr(brow ? brow + r0 : kbase);
+        const gptr_t kb0 = uniform_ptr(kbase + (int64_t)key_base * p.k_r), vb0 = uniform_ptr(vbase + (int64_t)key_base * p.v_r);
+        const gptr_t bb0 = uniform_ptr(brow ? brow + key_base : kbase);
         auto process = [&](int total) {
             u32x4_t kreg[NI], vreg[NI];
             uint32_t braw = 0;
@@ -270,7 +292,7 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
                 for (int j = 0; j < NI; j++) {
                     const int t = t0 + j * RPI + srow;
                     const uint32_t rel = s_idx[t < total ? t : total - 1];
-                    if (WIDE) {
+                    if (WIDE || LISTS) {
                         kreg[j] = *(const __attribute__((address_space(1))) u32x4_t *)(kb0 + ((int64_t)rel * p.k_r + scl * 8) * 2);
                         vreg[j] = *(const __attribute__((address_space(1))) u32x4_t *)(vb0 + ((int64_t)rel * p.v_r + scl * 8) * 2);
                     } else {
@@ -302,7 +324,7 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
                         const int t = t0 + 16 * (i >> 3) + 8 * g + (i & 7);
                         badd[i] = -INFINITY;
                         if (t < total) {
-                            const int key = r0 + (int)s_idx[t];
+                            const int key = key_base + (int)s_idx[t];
                             const bool keep = !mrow || mrow[key];
                             const float bv = brow ? E::lo((uint32_t)brow[key]) * kLog2e : 0.f;
                             badd[i] = keep ? bv : -INFINITY;
@@ -371,6 +393,17 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
             }
         };
 
+        if (LISTS) {
+            const int total = hi - r0 < DEC_LIST ? hi - r0 : DEC_LIST;
+            for (int i = tid; i < total; i += DEC_THREADS) {
+                const int32_t key = list[r0 + i];
+                s_idx[i] = (Idx)(key < 0 ? 0 : (key < p.Lk ? key : p.Lk - 1));
+            }
+            __syncthreads();
+            process(total);
+            __syncthreads();
+            continue;
+        }
         // append sub-ranges to the list while they fit, work the list off, go on with the rest (dense masks only)
         for (int j = 0; j < nj;) {
             int total = 0;
@@ -384,7 +417,7 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
                 while (u) {
                     const int k = __builtin_ctz(u);
                     u &= u - 1;
-                    s_idx[pos++] = (uint16_t)(j * DEC_RANGE + 16 * tid + k);
+                    s_idx[pos++] = (Idx)(j * DEC_RANGE + 16 * tid + k);
                 }
                 total += wg_cnt;
             }
@@ -476,12 +509,12 @@ __global__ void __launch_bounds__(CMB_THREADS) decode_combine_kernel(const FwdPa
     if (row < (int64_t)p.B * p.H) combine_row<T, false>(p, row, lane, s_w[wave]);
 }
 
-template <typename T, int D, bool PERHEAD, bool WIDE>
+template <typename T, int D, bool PERHEAD, bool WIDE, bool LISTS>
 hipError_t launch_decode_w(const FwdParams &p, int keys_per_split, hipStream_t stream) {
     const int G = p.H / p.Hk;
     const int chunks = (G + DEC_COLS - 1) / DEC_COLS;
     dim3 grid(p.splits, p.Hk * chunks, p.B);
-    auto kern = decode_kernel<T, D, PERHEAD, WIDE>;
+    auto kern = decode_kernel<T, D, PERHEAD, WIDE, LISTS>;
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, DecSmem<D>::TOTAL);
     if (e != hipSuccess) return e;
@@ -492,9 +525,11 @@ hipError_t launch_decode_w(const FwdParams &p, int keys_per_split, hipStream_t s
 template <typename T, int D, bool PERHEAD>
 hipError_t launch_decode_d(const FwdParams &p, int keys_per_split, hipStream_t stream) {
     // byte offsets of a gathered row relative to the first row of a pass fit 32 bits unless the row stride is huge
+    if (p.kept_idx && p.mask && p.Hm != p.H) return launch_decode_w<T, D, PERHEAD, true, true>(p, keys_per_split, stream);
+    if (p.kept_idx && p.mask && p.H == p.Hk) return launch_decode_w<T, D, false, true, true>(p, keys_per_split, stream);
     const int64_t rmax = p.k_r > p.v_r ? p.k_r : p.v_r;
     const bool wide = ((int64_t)DEC_SUPER * rmax + D) * 2 >= ((int64_t)1 << 32);
-    return wide ? launch_decode_w<T, D, PERHEAD, true>(p, keys_per_split, stream) : launch_decode_w<T, D, PERHEAD, false>(p, keys_per_split, stream);
+    return wide ? launch_decode_w<T, D, PERHEAD, true, false>(p, keys_per_split, stream) : launch_decode_w<T, D, PERHEAD, false, false>(p, keys_per_split, stream);
 }
 
 template <typename T>

@@ -177,14 +177,13 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
         if (j < n_end) {
             if (mrow) {
                 uint32_t any = 0;
+                int col[BN / 16];
+                u32x4_t mv[BN / 16];
 #pragma unroll
-                for (int c = 0; c < BN / 16; c++) {
-                    const int col = j * BN + c * 16;
-                    if (col < LkS) {
-                        u32x4_t mv = *(const u32x4_t *)(mrow + col);
-                        any |= mv[0] | mv[1] | mv[2] | mv[3];
-                    }
-                }
+                for (int c = 0; c < BN / 16; c++) col[c] = j * BN + c * 16;
+                ld_row16(mrow, col, LkS, mv);
+#pragma unroll
+                for (int c = 0; c < BN / 16; c++) any |= mv[c][0] | mv[c][1] | mv[c][2] | mv[c][3];
                 act = any != 0;
             } else {
                 act = true;

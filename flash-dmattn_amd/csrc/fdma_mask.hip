@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
     if (p.kept_idx) {
         __syncthreads();  // the row's stores are visible to the whole workgroup
         scan_mask_row<NT>(orow, Lk, p.kept_idx + (size_t)row * p.kept_ld, p.kept_cnt + (size_t)row * p.kept_ld,
-                          p.kept_count + row, (int *)wave_cnt, false);
+                          p.kept_count + row, (int *)wave_cnt);
     }
 
     // ---- optional third output: the row packed to one bit per key (key j in bit j % 8 of byte j / 8), the form in

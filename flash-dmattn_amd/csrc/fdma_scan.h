@@ -14,29 +14,19 @@ constexpr int SCAN_KEYS = 16;  // mask bytes per thread per pass
 //   irow[c]  = original column of the c-th kept key (ascending), c < *count_out
 //   crow[j]  = kept keys among the columns 0 .. j (inclusive), written for j < round_up(Lk, 16): the row has room
 //   s_wave   : NT / 64 ints of LDS
-// `padded`: the mask row is readable in 16-byte pieces up to round_up(Lk, 16) and 16-byte aligned (the attention
-// entry points require that of their masks); otherwise the last, partial piece is read byte by byte.
 template <int NT>
 __device__ __forceinline__ void scan_mask_row(const uint8_t *mrow, int Lk, int32_t *irow, int32_t *crow,
-                                              int32_t *count_out, int *s_wave, bool padded) {
+                                              int32_t *count_out, int *s_wave) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const bool vec = padded || (((uintptr_t)mrow & 15) == 0);
     int base = 0;
     for (int c0 = 0; c0 < Lk; c0 += NT * SCAN_KEYS) {
         const int col = c0 + tid * SCAN_KEYS;
         uint32_t bits = 0;
         if (col < Lk) {
-            if (vec && (padded || col + SCAN_KEYS <= Lk)) {
-                const u32x4_t mv = *(const u32x4_t *)(mrow + col);
+            const u32x4_t mv = ld_row16(mrow, col, Lk);
 #pragma unroll
-                for (int e = 0; e < SCAN_KEYS; e++) {
-                    const uint32_t byte = (mv[e >> 2] >> (8 * (e & 3))) & 0xffu;
-                    if (byte && col + e < Lk) bits |= 1u << e;
-                }
-            } else {
-                for (int e = 0; e < SCAN_KEYS && col + e < Lk; e++)
-                    if (mrow[col + e]) bits |= 1u << e;
-            }
+            for (int e = 0; e < SCAN_KEYS; e++)
+                if ((mv[e >> 2] >> (8 * (e & 3))) & 0xffu) bits |= 1u << e;
         }
         const int n = __builtin_popcount(bits);
         int incl = n;

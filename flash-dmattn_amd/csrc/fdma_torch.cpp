@@ -293,9 +293,12 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         if (!t->defined()) continue;
         if (t->scalar_type() != (t == &mask ? at::kBool : q.scalar_type()) || t->dim() != 4 || (t->size(0) != B && t->size(0) != 1) ||
             (t->size(1) != 1 && t->size(1) != Hk && t->size(1) != H) || (t->size(2) != 1 && t->size(2) != Lq) ||
-            (t == &mask ? t->size(3) < Lk : t->size(3) != Lk) || !vec_ok(*t, t == &mask ? 16 : 8))
+            (t == &mask ? t->size(3) < Lk : t->size(3) != Lk) || t->stride(3) != 1)
             Py_RETURN_NOTIMPLEMENTED;
     }
+    // (rows that all queries share are taken as they lie, rows per query in aligned vectors: fdma.h)
+    const bool rows = Lq > 1 && ((mask.defined() && mask.size(2) != 1) || (bias.defined() && bias.size(2) != 1) || Lk > (1 << 19));
+    if (rows && ((mask.defined() && !vec_ok(mask, 16)) || (bias.defined() && !vec_ok(bias, 8)))) Py_RETURN_NOTIMPLEMENTED;
     if (mask.defined()) {
         // a row per query head over grouped kv heads (its backward is taken apart), or rows that may turn out to be a
         // column mask under the policy "always": general path

@@ -63,8 +63,9 @@ enum {
  * capture of forward + backward through the tensor library ended in a host crash when the capture was closed; its
  * cause is not known, so the library refuses instead.)
  *
- * Readable lengths of mask and bias rows.  The kernels read mask rows in 16-byte and bias rows in 16-byte
- * (8-element) vectors: each row of `mask` must be readable up to seqlen_k rounded up to 16 bytes, each row of `bias`
+ * Readable lengths of mask and bias rows.  Where mask and bias are broadcast over the queries (or seqlen_q == 1, and up
+ * to 2^19 keys) exactly seqlen_k elements of a row are read, at any address and stride.  Otherwise the kernels read mask
+ * rows in 16-byte and bias rows in 16-byte (8-element) vectors: each row of `mask` must be readable up to seqlen_k rounded up to 16 bytes, each row of `bias`
  * up to seqlen_k rounded up to 8 elements, whatever lies there; this also holds for the last row of the buffer, and for a fully
  * broadcast mask or bias of a single row.  The library cannot check it (it never sees the row length).  The reference
  * asks for more: rows of exactly round_up(seqlen_k, 128) elements (flash_api.cpp:420, 431, 437).  Values beyond
