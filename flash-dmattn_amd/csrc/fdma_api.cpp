@@ -80,8 +80,9 @@ int validate_common(const fdma_fwd_args *a, bool backward) {
     if (!a->out) return fail(FDMA_ERR_INVALID, "out must be a device pointer");
     if (!a->lse) return fail(FDMA_ERR_INVALID, "softmax_lse must be a device pointer");
     // Rows that all queries share (and a single query's rows) are read element by element or with unaligned loads that
-    // stay inside the row: any address and stride will do.  Rows per query are read in aligned 16-byte vectors.
-    const bool elementwise = a->seqlen_q == 1 || ((!a->mask || a->mask_strides[2] == 0) && (!a->bias || a->bias_strides[2] == 0) &&
+    // stay inside the row: any address and stride will do.
+    // (The per-query kernels also take any address, as long as a row has the 8 keys they fetch at a time.)
+    const bool elementwise = a->seqlen_q == 1 || a->seqlen_k >= 8 || ((!a->mask || a->mask_strides[2] == 0) && (!a->bias || a->bias_strides[2] == 0) &&
                                                   a->seqlen_k <= kMaxColumnFormKeys);
     if (a->mask) {
         const int hm = a->num_heads_mask;
@@ -412,11 +413,26 @@ static size_t dbias_accum_bytes(const fdma_bwd_args *a) {
     return dbias_shared(a) ? (size_t)round_up(dbias_accum_elems(a) * sizeof(float), 256) : 0;
 }
 
+// the backward kernels for masks / biases with a row per query take the call
+static bool general_form(const fdma::FwdParams &f) {
+    fdma::BwdParams p;
+    std::memset(&p, 0, sizeof(p));
+    p.f = f;
+    return f.Lq > 0 && f.Lk > 0 && !fdma::bwd_colmask_applicable(p);
+}
+
 size_t fdma_bwd_workspace_bytes(const fdma_bwd_args *a) {
     if (!a) return 0;
     fdma::FwdParams p;
     fill_fwd_params(&a->f, p);
-    return dbias_accum_bytes(a) + (fdma::use_compact(p) ? fdma::compact_bytes(p, true, a->fwd_workspace != nullptr) : 0);
+    size_t bytes = dbias_accum_bytes(a);
+    if (fdma::use_compact(p)) return bytes + fdma::compact_bytes(p, true, a->fwd_workspace != nullptr);
+    if (general_form(p)) {
+        size_t db = 0;
+        bytes += (size_t)round_up(fdma::general_kv_part_bytes(p, &db), 256);
+        bytes += (size_t)round_up(db, 256);
+    }
+    return bytes;
 }
 
 int fdma_bwd(const fdma_bwd_args *a, void *hip_stream) {
@@ -446,6 +462,15 @@ int fdma_bwd(const fdma_bwd_args *a, void *hip_stream) {
         p.dba_r = a->f.bias_strides[2] == 0 ? 0 : lkr;
         p.dba_h = nr * lkr;
         p.dba_b = a->f.bias_strides[0] == 0 ? 0 : p.dba_h * a->f.num_heads_bias;
+    }
+    p.kv_segs = 1;
+    if (!fdma::use_compact(p.f) && general_form(p.f)) {
+        p.kv_segs = fdma::general_kv_segments(p.f);
+        size_t db = 0;
+        const size_t kv = (size_t)round_up(fdma::general_kv_part_bytes(p.f, &db), 256);
+        char *at = static_cast<char *>(a->workspace) + dbias_accum_bytes(a);
+        p.dkv_part = reinterpret_cast<float *>(at);
+        p.db_part = reinterpret_cast<float *>(at + kv);
     }
     hipStream_t stream = static_cast<hipStream_t>(hip_stream);
     hipError_t e;

@@ -77,7 +77,7 @@ template <typename T> struct NegInfPair;
 template <> struct NegInfPair<bf16_tag> { static constexpr uint32_t value = 0xFF80FF80u; };
 template <> struct NegInfPair<fp16_tag> { static constexpr uint32_t value = 0xFC00FC00u; };
 
-template <typename T, int D, bool CAUSAL, bool GSUM>
+template <typename T, int D, bool CAUSAL, bool GSUM, bool ODD>
 __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv_kernel(const BwdParams p) {
     using E = Elem<T>;
     using SM = KvSmem<D, GSUM>;
@@ -92,10 +92,10 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
 
     const FwdParams &f = p.f;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 31, g = lane >> 5;
-    // linear workgroup id -> (key block, kv head, batch), key block OUTERMOST and ascending: under causal masking the low
-    // key blocks are seen by the most queries, so the heaviest workgroups of every head start first
-    const int hb_count = f.Hk * f.B;
-    const int n_block = (int)blockIdx.x / hb_count, hk = ((int)blockIdx.x % hb_count) % f.Hk, b = ((int)blockIdx.x % hb_count) / f.Hk;
+    // linear workgroup id -> (key block, segment, kv head, batch), key block OUTERMOST and ascending: under causal masking
+    // the low key blocks are seen by the most queries, so the heaviest workgroups of every head start first
+    const int hb_count = f.Hk * f.B, segs = p.kv_segs, part_id = (int)blockIdx.x;
+    const int n_block = (int)blockIdx.x / (hb_count * segs), seg = ((int)blockIdx.x / hb_count) % segs, hk = ((int)blockIdx.x % hb_count) % f.Hk, b = ((int)blockIdx.x % hb_count) / f.Hk;
     const int G = f.H / f.Hk;
     const int n0 = n_block * KV_BN;
     const int key = n0 + wave * 32 + r;  // the key column this lane owns
@@ -138,11 +138,12 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
     // row-broadcast dbias wants (g outer, m inner) to keep one column sum per bias head.  Query blocks
     // are walked from the last one down so that neighbouring workgroups stream the same tiles together.
     const bool m_outer = bias_rows;
-    const int n_m = M_blocks - m_start;
+    // (this workgroup's segment of the query blocks that see its keys: fdma_bwd_dkdv_wide.hip has the reasons)
+    const int m_lo = (M_blocks - m_start) * seg / segs, n_m = (M_blocks - m_start) * (seg + 1) / segs - m_lo;
     const int n_steps = n_m * G;
 
     // zero the part of a per-query dbias this workgroup owns but never visits (above the causal diagonal)
-    if (bias_rows && !use_accum && m_start > 0) {
+    if (bias_rows && !use_accum && m_start > 0 && seg == 0) {
         const int ngh = (f.Hb == f.H) ? G : 1;
         for (int gh = 0; gh < ngh; gh++) {
             const int hb = f.Hb == f.H ? hk * G + gh : (f.Hb == 1 ? 0 : hk);
@@ -171,7 +172,7 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
     const uint16_t *bias_ld = has_bias ? (const uint16_t *)f.bias : (const uint16_t *)f.k;
     auto step_head = [&](int step, int &gi, int &mi) {
         gi = m_outer ? step % G : step / n_m;
-        mi = M_blocks - 1 - (m_outer ? step / G : step % n_m);
+        mi = M_blocks - 1 - m_lo - (m_outer ? step / G : step % n_m);
     };
     auto load_step = [&](int step) {
         int gi, mi;
@@ -198,18 +199,19 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
         const int hb = has_bias ? (f.Hb == f.H ? h : (f.Hb == 1 ? 0 : hk)) : 0;
         const int kk = n0 + 8 * bc;
         const int kk_c = kk < f.Lk ? kk : 0;
-        const int64_t moff = f.mask ? b * f.m_b + hm * f.m_h + kk_c : 0;
-        const int64_t boff = has_bias ? b * f.bi_b + hb * f.bi_h + kk_c : 0;
+        const int at = chunk8_at<ODD>(kk, f.Lk);
+        const int64_t moff = f.mask ? b * f.m_b + hm * f.m_h + at : 0;
+        const int64_t boff = has_bias ? b * f.bi_b + hb * f.bi_h + at : 0;
 #pragma unroll
         for (int it = 0; it < FB_IT; it++) {
             int qq = m0 + br0 + 16 * it;
             qq = qq < f.Lq ? qq : f.Lq - 1;
-            braw[it] = *(const u32x4_t *)(bias_ld + boff + (has_bias ? (int64_t)qq * f.bi_r : 0));
+            braw[it] = *(const u32x4_el_t *)(bias_ld + boff + (has_bias ? (int64_t)qq * f.bi_r : 0));
             // (one 8-byte load either way, from an address chosen without a branch: mask bytes of the chunk, or --
             // a mask packed to bits -- the aligned piece of the bit row that holds the chunk's byte)
             const uint8_t *src = (f.mask && f.mbits) ? f.mbits + b * f.mb_b + hm * f.mb_h + (int64_t)qq * f.mb_r + ((kk_c >> 3) & ~7)
                                                      : mask_ld + moff + (f.mask ? (int64_t)qq * f.m_r : 0);
-            mraw[it] = *(const u32x2_t *)src;
+            mraw[it] = *(const u32x2_any_t *)src;
         }
     };
     auto store_step = [&](int buf) {
@@ -229,8 +231,8 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
         const int kk = n0 + 8 * bc;
 #pragma unroll
         for (int it = 0; it < FB_IT; it++) {
-            u32x4_t bv = has_bias ? braw[it] : u32x4_t{0, 0, 0, 0};
-            u32x2_t mv = f.mask ? (f.mbits ? mask_bits_to_bytes(mask_bits_byte(mraw[it], kk < f.Lk ? kk : 0)) : mraw[it])
+            u32x4_t bv = has_bias ? chunk8_fix<ODD>(braw[it], kk, f.Lk) : u32x4_t{0, 0, 0, 0};
+            u32x2_t mv = f.mask ? (f.mbits ? mask_bits_to_bytes(mask_bits_byte(mraw[it], kk < f.Lk ? kk : 0)) : chunk8_fix_mask<ODD>(mraw[it], kk, f.Lk))
                                 : u32x2_t{0x01010101u, 0x01010101u};
             uint64_t keepm = kk < f.Lk ? ~0ull : 0ull;
             if (kk + 8 > f.Lk && kk < f.Lk) keepm = (1ull << (8 * (f.Lk - kk))) - 1ull;  // chunk straddles the end of the keys
@@ -409,7 +411,9 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
                 const bool last_m = (step % n_m) == n_m - 1;
                 if (last_m && (f.Hb == f.H || gi == G - 1)) {
                     const float tot = xhalf_sum(colsum);
-                    if (g == 0 && key < f.Lk) {
+                    if (g == 0 && segs > 1) {
+                        p.db_part[((int64_t)part_id * G + (f.Hb == f.H ? gi : 0)) * KV_BN + wave * 32 + r] = tot;
+                    } else if (g == 0 && key < f.Lk) {
                         if (use_accum) atomicAdd(p.dbias_accum + b * p.dba_b + hb * p.dba_h + key, tot);
                         else ((uint16_t *)p.dbias)[b * p.db_b + hb * p.db_h + key] = (uint16_t)(E::pack2(tot, 0.f) & 0xffffu);
                     }
@@ -463,13 +467,27 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
         __syncthreads();
     }
 
-    // a key block that no query can see still owns its dbias column (row-broadcast case)
-    if (has_bias && !bias_rows && n_steps == 0 && !use_accum && g == 0 && key < f.Lk) {
+    // a key block that no query (of this segment) can see still owns its dbias column (row-broadcast case)
+    if (has_bias && !bias_rows && n_steps == 0 && g == 0) {
         const int ngh = (f.Hb == f.H) ? G : 1;
         for (int gh = 0; gh < ngh; gh++) {
             const int hb = f.Hb == f.H ? hk * G + gh : (f.Hb == 1 ? 0 : hk);
-            ((uint16_t *)p.dbias)[b * p.db_b + hb * p.db_h + key] = 0;
+            if (segs > 1) p.db_part[((int64_t)part_id * G + gh) * KV_BN + wave * 32 + r] = 0.f;
+            else if (!use_accum && key < f.Lk) ((uint16_t *)p.dbias)[b * p.db_b + hb * p.db_h + key] = 0;
         }
+    }
+
+    if (segs > 1) {  // fp32 sums of this segment, in the order the lanes hold them (1 KB per store)
+        f32x4_t *dst = (f32x4_t *)p.dkv_part + (int64_t)part_id * 2 * KV_BN * D / 4 + wave * DB * 4 * 64 + lane;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int at = (db * 4 + q) * 64;
+                dst[at] = f32x4_t{dk[db][4 * q], dk[db][4 * q + 1], dk[db][4 * q + 2], dk[db][4 * q + 3]};
+                dst[at + KV_BN * D / 4] = f32x4_t{dv[db][4 * q], dv[db][4 * q + 1], dv[db][4 * q + 2], dv[db][4 * q + 3]};
+            }
+        return;
     }
 
     // ---- store dK (scaled) and dV
@@ -492,6 +510,50 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
                     *(u32x4_t *)(dvp + c) = wv;
                 }
             }
+    }
+}
+
+// Sums of the segments, in order, to dK (scaled), dV and a row-broadcast dBias.  Thread (kw, db, blk, lane) of a unit owns
+// the eight head-dim elements that lane held in its register block: 2 KB of partial sums per wave and segment, all
+// segments' loads independent; bound by reading them (33 MB in 8 us at 4 segments of 64 units, d = 128).
+template <typename T, int D>
+__global__ void __launch_bounds__(256) bwd_dkdv_sum_kernel(const BwdParams p) {
+    using E = Elem<T>;
+    constexpr int DB = D / 32, PER = KV_BN * D;  // floats of one matrix of a unit
+    const FwdParams &f = p.f;
+    const int segs = p.kv_segs, hb_count = f.Hk * f.B;
+    constexpr int BPU = 2 * PER / 8 / 256;  // workgroups per unit
+    const int unit = (int)blockIdx.x / BPU;
+    const int n_block = unit / hb_count, hk = (unit % hb_count) % f.Hk, b = (unit % hb_count) / f.Hk;
+    const int64_t part0 = (int64_t)n_block * hb_count * segs + unit % hb_count;  // segment s: + s * hb_count
+    const int t = ((int)blockIdx.x % BPU) * 256 + threadIdx.x;
+    const int lane = t & 63, w = t >> 6;  // w = ((mat * 4 + kw) * DB + db) * 2 + blk
+    const int blk = w & 1, db = (w >> 1) % DB, kw = (w >> 1) / DB % 4, mat = (w >> 1) / DB / 4;
+    const float *src = p.dkv_part + part0 * 2 * PER + mat * PER + (((kw * DB + db) * 4 + 2 * blk) * 64 + lane) * 4;
+    f32x4_t a0 = {0, 0, 0, 0}, a1 = {0, 0, 0, 0};
+#pragma unroll 4
+    for (int s = 0; s < segs; s++) {
+        const float *q = src + (int64_t)s * hb_count * 2 * PER;
+        a0 += *(const f32x4_t *)q;
+        a1 += *(const f32x4_t *)(q + 256);
+    }
+    const int key = n_block * KV_BN + kw * 32 + (lane & 31), c = 32 * db + 16 * blk + 8 * (lane >> 5);
+    if (key < f.Lk && c < f.d) {
+        const float m = mat == 0 ? f.scale : 1.f;
+        const u32x4_t o = {E::pack2(a0[0] * m, a0[1] * m), E::pack2(a0[2] * m, a0[3] * m), E::pack2(a1[0] * m, a1[1] * m), E::pack2(a1[2] * m, a1[3] * m)};
+        uint16_t *dst = mat == 0 ? (uint16_t *)p.dk + b * p.dk_b + (int64_t)key * p.dk_r + hk * p.dk_h
+                                 : (uint16_t *)p.dv + b * p.dv_b + (int64_t)key * p.dv_r + hk * p.dv_h;
+        *(u32x4_t *)(dst + c) = o;
+    }
+    if ((int)blockIdx.x % BPU == 0 && f.bias && f.bi_r == 0 && threadIdx.x < KV_BN) {
+        const int G = f.H / f.Hk, ngh = f.Hb == f.H ? G : 1, kc = n_block * KV_BN + threadIdx.x;
+        for (int gh = 0; gh < ngh && kc < f.Lk; gh++) {
+            float tot = 0.f;
+            for (int s = 0; s < segs; s++) tot += p.db_part[((part0 + (int64_t)s * hb_count) * G + gh) * KV_BN + threadIdx.x];
+            const int hb = f.Hb == f.H ? hk * G + gh : (f.Hb == 1 ? 0 : hk);
+            if (p.dbias_accum) atomicAdd(p.dbias_accum + b * p.dba_b + hb * p.dba_h + kc, tot);
+            else ((uint16_t *)p.dbias)[b * p.db_b + hb * p.db_h + kc] = (uint16_t)(E::pack2(tot, 0.f) & 0xffffu);
+        }
     }
 }
 
@@ -542,7 +604,8 @@ hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
     if (f.Lk > 0 && colmask) {
         if ((e = launch_bwd_dkdv_colmask(p, dtype_code, stream)) != hipSuccess) return e;
     } else if (f.Lk > 0) {
-        dim3 grid(((f.Lk + KV_BN - 1) / KV_BN) * f.Hk * f.B);
+        const int units = ((f.Lk + KV_BN - 1) / KV_BN) * f.Hk * f.B;
+        dim3 grid(units * p.kv_segs);
         // a per-query bias shared by several query heads: dS is summed over the group before it is written; one
         // shared by several workgroups (broadcast over the batch or over kv heads) is accumulated with fp32 atomics
         const bool gsum = f.bias != nullptr && f.bi_r != 0 && ((f.Hb != f.H && f.H / f.Hk > 1) || p.dbias_accum != nullptr);
@@ -553,9 +616,21 @@ hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
             hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
             return hipGetLastError();
         };
-        if (gsum) e = f.causal ? launch(bwd_dkdv_kernel<T, D, true, true>, KvSmem<D, true>::TOTAL) : launch(bwd_dkdv_kernel<T, D, false, true>, KvSmem<D, true>::TOTAL);
-        else e = f.causal ? launch(bwd_dkdv_kernel<T, D, true, false>, KvSmem<D, false>::TOTAL) : launch(bwd_dkdv_kernel<T, D, false, false>, KvSmem<D, false>::TOTAL);
+        if constexpr (D == 128) {
+            e = launch_bwd_dkdv_wide(p, dtype_code, gsum, stream);
+        } else {
+            auto pick = [&](auto odd) -> hipError_t {
+                constexpr bool O = decltype(odd)::value;
+                if (gsum) return f.causal ? launch(bwd_dkdv_kernel<T, D, true, true, O>, KvSmem<D, true>::TOTAL) : launch(bwd_dkdv_kernel<T, D, false, true, O>, KvSmem<D, true>::TOTAL);
+                return f.causal ? launch(bwd_dkdv_kernel<T, D, true, false, O>, KvSmem<D, false>::TOTAL) : launch(bwd_dkdv_kernel<T, D, false, false, O>, KvSmem<D, false>::TOTAL);
+            };
+            e = D > 64 || odd_rows(f) ? pick(std::true_type()) : pick(std::bool_constant<(D > 64)>());
+        }
         if (e != hipSuccess) return e;
+        if (p.kv_segs > 1) {
+            hipLaunchKernelGGL((bwd_dkdv_sum_kernel<T, D>), dim3(units * (2 * KV_BN * D / 8 / 256)), dim3(256), 0, stream, p);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
     }
     // 3. dQ (the launch of a compacted backward also sums the dK / dV / dBias partial results of step 2)
     if (colmask) {
@@ -575,6 +650,28 @@ hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
 }
 
 }  // namespace
+
+// Segments of the general dK/dV kernel: as many as it takes to give every CU a workgroup (two at d <= 64, where two fit;
+// a causal launch twice that, since its workgroups are of very different lengths), each at least two query blocks long.
+int general_kv_segments(const FwdParams &f) {
+    if (f.Lk <= 0 || f.Lq <= 0) return 1;
+    const int bm = f.d > 128 ? 32 : 64;
+    const int64_t units = (int64_t)((f.Lk + KV_BN - 1) / KV_BN) * f.Hk * f.B;
+    const int64_t want = (int64_t)device_cus() * (f.d <= 64 ? 2 : 1) * (f.causal ? 2 : 1);
+    int64_t segs = units >= want ? 1 : (want + units - 1) / units;
+    const int64_t most = ((f.Lq + bm - 1) / bm) / 2;
+    segs = segs > most ? most : segs;
+    return segs > 16 ? 16 : (segs < 1 ? 1 : (int)segs);
+}
+
+size_t general_kv_part_bytes(const FwdParams &f, size_t *db_bytes) {
+    const int segs = general_kv_segments(f);
+    if (segs <= 1) return 0;
+    const size_t parts = (size_t)((f.Lk + KV_BN - 1) / KV_BN) * f.Hk * f.B * segs;
+    const int dpad = f.d <= 64 ? 64 : (f.d <= 128 ? 128 : 256);
+    *db_bytes = f.bias && f.bi_r == 0 ? parts * (f.H / f.Hk) * KV_BN * 4 : 0;
+    return parts * 2 * KV_BN * dpad * 4;
+}
 
 hipError_t launch_bwd(const BwdParams &p, int dtype, hipStream_t stream) {
     if (p.f.B <= 0 || p.f.Lq <= 0) return hipSuccess;

@@ -18,9 +18,11 @@ namespace fdma {
 
 namespace {
 
-// Workgroups have 4 waves (128 query rows; two per CU at d <= 64) or, at d = 128 on grids that stay large enough,
-// 8 waves (256 rows): one workgroup fits on a CU there, and a second wave per SIMD hides what a single wave's
-// in-order issue cannot.  Key tiles have 64 keys with 4 waves and 32 with 8 (the 64-key tile's score and dP accumulators
+// Workgroups have 4 waves (128 query rows; two per CU at d <= 64) or, at d = 128, 8: one workgroup fits on a CU there, and
+// a second wave per SIMD hides what a single wave's in-order issue cannot.  On grids that stay large enough the 8 waves
+// cover 256 rows; on smaller ones (KSPLIT) 128 rows, two waves per 32 rows that take the lower and the upper half of every
+// key tile and add their sums through LDS at the end (B = 1, L = 1999, H = 16, d = 128, fp16: 128 us with four waves, 108
+// so, odd rows read where they lie).  Key tiles have 64 keys, and 32 with 256 rows (the 64-key tile's score and dP accumulators
 // do not fit next to dQ and the Q / dO fragments in the 256 registers a wave has when two share a SIMD).
 template <int D, int BM, int BN> struct DqSmem {
     static constexpr int S = D + 8;      // K / V tile row stride (elements)
@@ -35,14 +37,15 @@ template <typename T> struct NegInf2;
 template <> struct NegInf2<bf16_tag> { static constexpr uint32_t value = 0xFF80FF80u; };
 template <> struct NegInf2<fp16_tag> { static constexpr uint32_t value = 0xFC00FC00u; };
 
-template <typename T, int D, bool CAUSAL, int NW>
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, bool ODD>
 __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_kernel(const BwdParams p) {
-    constexpr int NTHREADS = 64 * NW, BM = 32 * NW, BN = (NW == 8 || D > 128) ? 32 : 64;
+    constexpr int NTHREADS = 64 * NW, BM = 32 * NW / KSPLIT, BN = ((NW == 8 && KSPLIT == 1) || D > 128) ? 32 : 64;
+    constexpr int BK = BN / KSPLIT;         // keys of a tile per wave
     constexpr int FCH = BN / 8;             // 8-key chunks per mask / bias row of a tile
     constexpr int F_RPP = NTHREADS / FCH;   // mask / bias rows staged per pass
     using E = Elem<T>;
     using SM = DqSmem<D, BM, BN>;
-    constexpr int KS = D / 16, DB = D / 32, MB = BN / 32, KB = BN / 16;
+    constexpr int KS = D / 16, DB = D / 32, MB = BK / 32, KB = BK / 16;
     constexpr int CH = D / 8;               // 16-byte chunks per K / V row
     constexpr int K_RPP = NTHREADS / CH;    // rows staged per pass
     constexpr int K_IT = BN / K_RPP;
@@ -52,14 +55,17 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
 
     const FwdParams &f = p.f;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 31, g = lane >> 5;
-    // linear workgroup id -> (query block, head, batch) with the query block OUTERMOST and descending: under causal
-    // masking the blocks with the most KV tiles of every head start first, the light ones fill the tail
-    const int hb_count = f.H * f.B;
+    // linear workgroup id -> (query block, member of the kv group, kv head, batch) with the query block OUTERMOST and
+    // descending: under causal masking the blocks with the most KV tiles of every head start first, the light ones fill the
+    // tail.  The members of a group, which read the same K / V and often the same mask and bias, are a multiple of the kv
+    // head count apart: on one XCD (ids are dealt to the 8 XCDs in turn) when that is a multiple of 8.
+    const int hb_count = f.H * f.B, pairs = f.Hk * f.B;
     const int m_block = (int)gridDim.x / hb_count - 1 - (int)blockIdx.x / hb_count;
-    const int h = ((int)blockIdx.x % hb_count) % f.H, b = ((int)blockIdx.x % hb_count) / f.H;
-    const int hk = h / (f.H / f.Hk);
+    const int pair = (int)blockIdx.x % pairs, hk = pair % f.Hk, b = pair / f.Hk;
+    const int h = hk * (f.H / f.Hk) + ((int)blockIdx.x % hb_count) / pairs;
     const int m0 = m_block * BM;
-    const int wrow0 = m0 + wave * 32;
+    const int rw = wave % (BM / 32), kh = wave / (BM / 32);  // row block and key half of this wave
+    const int wrow0 = m0 + rw * 32;
     const int qrow = wrow0 + r;
     const int qrow_c = qrow < f.Lq ? qrow : f.Lq - 1;
     const int shift = f.Lk - f.Lq;
@@ -123,14 +129,15 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         if (!mbase) return;
         int kk = j * BN + 8 * fc;
         kk = kk < f.Lk ? kk : 0;
+        const int at = chunk8_at<ODD>(j * BN + 8 * fc, f.Lk);
 #pragma unroll
         for (int it = 0; it < F_IT; it++) {
             int row = m0 + fr0 + F_RPP * it;
             row = row < f.Lq ? row : f.Lq - 1;
             // (one 8-byte load either way, from an address chosen without a branch: mask bytes of the chunk, or the
             // aligned piece of the bit row that holds the chunk's byte)
-            const uint8_t *src = mbits ? mbits + (int64_t)row * f.mb_r + ((kk >> 3) & ~7) : mbase + (int64_t)row * f.m_r + kk;
-            dst[it] = *(const u32x2_t *)src;
+            const uint8_t *src = mbits ? mbits + (int64_t)row * f.mb_r + ((kk >> 3) & ~7) : mbase + (int64_t)row * f.m_r + at;
+            dst[it] = *(const u32x2_any_t *)src;
         }
     };
     auto finish_mask = [&](int j, u32x2_t (&dst)[F_IT]) -> bool {
@@ -139,7 +146,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
 #pragma unroll
         for (int it = 0; it < F_IT; it++) {
             const int row = m0 + fr0 + F_RPP * it;
-            u32x2_t mv = mbase ? (mbits ? mask_bits_to_bytes(mask_bits_byte(dst[it], kk)) : dst[it]) : u32x2_t{0x01010101u, 0x01010101u};
+            u32x2_t mv = mbase ? (mbits ? mask_bits_to_bytes(mask_bits_byte(dst[it], kk)) : chunk8_fix_mask<ODD>(dst[it], kk, f.Lk)) : u32x2_t{0x01010101u, 0x01010101u};
             const bool ok = row < f.Lq && kk < f.Lk && !(CAUSAL && kk > row + shift);
             uint64_t keepm = ok ? ~0ull : 0ull;
             if (kk + 8 > f.Lk && kk < f.Lk) keepm = (1ull << (8 * (f.Lk - kk))) - 1ull;
@@ -153,13 +160,12 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
     auto load_rest = [&](int j) {
         const int n0 = j * BN;
         if (bbase) {
-            int kk = n0 + 8 * fc;
-            kk = kk < f.Lk ? kk : 0;
+            const int at = chunk8_at<ODD>(n0 + 8 * fc, f.Lk);
 #pragma unroll
             for (int it = 0; it < F_IT; it++) {
                 int row = m0 + fr0 + F_RPP * it;
                 row = row < f.Lq ? row : f.Lq - 1;
-                breg[it] = *(const u32x4_t *)(bbase + (int64_t)row * f.bi_r + kk);
+                breg[it] = *(const u32x4_el_t *)(bbase + (int64_t)row * f.bi_r + at);
             }
         } else {
 #pragma unroll
@@ -173,7 +179,8 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
             vreg[it] = *(const u32x4_t *)(vbase + (int64_t)key * f.v_r + kcol);
         }
     };
-    auto store_stage = [&](int buf, const u32x2_t (&mv)[F_IT]) {
+    auto store_stage = [&](int j, const u32x2_t (&mv)[F_IT]) {
+        const int buf = j & 1, kk = j * BN + 8 * fc;
         char *sK = smem + buf * SM::STAGE;
         char *sV = sK + SM::K_BYTES;
         char *sF = sV + SM::K_BYTES;
@@ -185,7 +192,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         }
 #pragma unroll
         for (int it = 0; it < F_IT; it++) {
-            u32x4_t bv = breg[it];
+            u32x4_t bv = bbase ? chunk8_fix<ODD>(breg[it], kk, f.Lk) : breg[it];
 #pragma unroll
             for (int hlf = 0; hlf < 2; hlf++) {
                 uint32_t x = mv[it][hlf];
@@ -208,10 +215,10 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
     const uint32_t tr_off = (uint32_t)(((8 * g + te) * SM::S + 16 * tdh + 4 * tcp) * 2);
 
     auto compute = [&](int j, int buf) {
-        const int n0 = j * BN;
-        const char *sK = smem + buf * SM::STAGE;
+        const int n0 = j * BN + kh * BK;
+        const char *sK = smem + buf * SM::STAGE + kh * BK * SM::S * 2;
         const char *sV = sK + SM::K_BYTES;
-        const char *sF = sV + SM::K_BYTES + ((wave * 32 + r) * SM::SF + 8 * g) * 2;
+        const char *sF = smem + buf * SM::STAGE + 2 * SM::K_BYTES + ((rw * 32 + r) * SM::SF + kh * BK + 8 * g) * 2;
         // ---- S^T = K Q^T on top of the fused mask+bias tile, dP^T = V dO^T
         f32x16_t s[MB], dp[MB];
 #pragma unroll
@@ -245,7 +252,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
             }
         }
         // ---- dS^T = P^T o (dP^T - D); causal selects on diagonal tiles only (wave-uniform branch)
-        const bool diag = CAUSAL && (n0 + BN - 1 > wrow0 + shift);
+        const bool diag = CAUSAL && (n0 + BK - 1 > wrow0 + shift);
         uint32_t dpk[8 * MB];
 #pragma unroll
         for (int mb = 0; mb < MB; mb++)
@@ -306,7 +313,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
             __builtin_amdgcn_sched_barrier(0);  // loads above, their first use below the compute
             if (act_cur) compute(j, j & 1);
             __builtin_amdgcn_sched_barrier(0);
-            if (have_next) store_stage((j + 1) & 1, m_next);
+            if (have_next) store_stage(j + 1, m_next);
             const bool act_nn = __syncthreads_or(j + 2 < n_end && finish_mask(j + 2, m_new));
             act_cur = have_next;
             act_next = act_nn;
@@ -317,6 +324,27 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         }
     }
 
+    if constexpr (KSPLIT == 2) {  // the upper key half hands over its sums
+        f32x4_t *xo = (f32x4_t *)smem + rw * DB * 4 * 64 + lane;
+        __syncthreads();  // (the tiles' last reads)
+        if (kh == 1) {
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    xo[(db * 4 + q) * 64] = f32x4_t{dq[db][4 * q], dq[db][4 * q + 1], dq[db][4 * q + 2], dq[db][4 * q + 3]};
+        }
+        __syncthreads();
+        if (kh == 1) return;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const f32x4_t v = xo[(db * 4 + q) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; e++) dq[db][4 * q + e] += v[e];
+            }
+    }
     if (qrow < f.Lq) {
         uint16_t *dqp = (uint16_t *)p.dq + b * p.dq_b + (int64_t)qrow * p.dq_r + h * p.dq_h;
 #pragma unroll
@@ -335,10 +363,10 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
     }
 }
 
-template <typename T, int D, bool CAUSAL, int NW>
-hipError_t launch_dq_n(const BwdParams &p, hipStream_t stream) {
-    constexpr int BM = 32 * NW, NTHREADS = 64 * NW, BN = (NW == 8 || D > 128) ? 32 : 64;
-    auto kern = bwd_dq_kernel<T, D, CAUSAL, NW>;
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, bool ODD>
+hipError_t launch_dq_o(const BwdParams &p, hipStream_t stream) {
+    constexpr int BM = 32 * NW / KSPLIT, NTHREADS = 64 * NW, BN = ((NW == 8 && KSPLIT == 1) || D > 128) ? 32 : 64;
+    auto kern = bwd_dq_kernel<T, D, CAUSAL, NW, KSPLIT, ODD>;
     const int smem = DqSmem<D, BM, BN>::TOTAL;
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
@@ -348,13 +376,21 @@ hipError_t launch_dq_n(const BwdParams &p, hipStream_t stream) {
     return hipGetLastError();
 }
 
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT = 1>
+hipError_t launch_dq_n(const BwdParams &p, hipStream_t stream) {
+    if (D > 128 || odd_rows(p.f)) return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, true>(p, stream);
+    return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, D <= 128 ? false : true>(p, stream);
+}
+
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_dq_c(const BwdParams &p, hipStream_t stream) {
     if constexpr (D > 64 && D <= 128) {
         // 256-row workgroups while the grid still covers the chip about twice
         if ((int64_t)p.f.B * p.f.H * ((p.f.Lq + 255) / 256) >= 512) return launch_dq_n<T, D, CAUSAL, 8>(p, stream);
+        return launch_dq_n<T, D, CAUSAL, 8, 2>(p, stream);
+    } else {
+        return launch_dq_n<T, D, CAUSAL, 4>(p, stream);
     }
-    return launch_dq_n<T, D, CAUSAL, 4>(p, stream);
 }
 
 }  // namespace

@@ -243,6 +243,39 @@ __device__ __forceinline__ u32x4_t ld_row16(const uint8_t *row, int c, int n) {
     return v[0];
 }
 
+// The 8-key chunk of a mask or bias row that starts at key kk (a multiple of 8), for rows that may start at any address
+// (mask: any byte, bias: any element).  chunk8_at: the key the chunk is fetched from -- one that keeps the 16-byte load
+// inside a row of at least 8 keys (shorter rows are readable up to 8: fdma.h) -- and chunk8_fix / chunk8_fix_mask put a
+// chunk that was fetched further in front back in place (only the chunk that straddles the end of the row is; the caller
+// drops keys at or beyond the end, and chunks that start there hold anything).  ODD = false: rows of whole, aligned chunks,
+// nothing to put back -- a kernel of its own, because the test for it costs the memory-bound kernels 7 % at head dim 64.
+typedef u32x2_t __attribute__((aligned(1))) u32x2_any_t;
+typedef u32x4_t __attribute__((aligned(2))) u32x4_el_t;
+template <bool ODD> __device__ __forceinline__ int chunk8_at(int kk, int Lk) {
+    if (!ODD) return kk < Lk ? kk : 0;
+    const int last = Lk >= 8 ? Lk - 8 : 0;
+    return kk < last ? kk : last;
+}
+template <bool ODD> __device__ __forceinline__ u32x2_t chunk8_fix_mask(u32x2_t m, int kk, int Lk) {
+    if (!ODD) return m;
+    const int by = kk - chunk8_at<true>(kk, Lk);
+    const uint64_t v = ((uint64_t)m[0] | ((uint64_t)m[1] << 32)) >> (8 * (by < 8 ? by : 0));
+    return u32x2_t{(uint32_t)v, (uint32_t)(v >> 32)};
+}
+template <bool ODD> __device__ __forceinline__ u32x4_t chunk8_fix(u32x4_t b, int kk, int Lk) {
+    if (!ODD) return b;
+    const int by = kk - chunk8_at<true>(kk, Lk);
+    if (by > 0 && by < 8) {
+        uint64_t lo = (uint64_t)b[0] | ((uint64_t)b[1] << 32), hi = (uint64_t)b[2] | ((uint64_t)b[3] << 32);
+        if (by >= 4) { lo = hi; hi = 0; }
+        const int s = 16 * (by & 3);
+        lo = (lo >> s) | ((hi << 1) << (63 - s));
+        hi >>= s;
+        b = u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+    }
+    return b;
+}
+
 // max / sum across the two 32-lane halves of a wave (lanes l and l ^ 32)
 __device__ __forceinline__ float xhalf_max(float x) {
     uint32_t u = __float_as_uint(x);

@@ -901,7 +901,7 @@ size_t compact_bytes(const FwdParams &p, bool backward, bool reuse_fwd) {
 }
 
 // compute units of the current device (cached per device)
-static int device_cus() {
+int device_cus() {
     static std::atomic<int> cus[16];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return 256;

@@ -29,9 +29,11 @@ namespace fdma {
 
 namespace {
 
-// Workgroups have 4 waves (128 query rows; two per CU at d <= 64) or, at d = 128 on grids that stay large enough,
-// 8 waves (256 rows): at d = 128 only one workgroup fits on a CU, and with a single wave per SIMD nothing hides the
-// in-order issue of that wave -- a second wave per SIMD does.
+// Workgroups have 4 waves (128 query rows; two per CU at d <= 64) or, at d = 128, 8: only one workgroup fits on a CU there,
+// and with a single wave per SIMD nothing hides the in-order issue of that wave -- a second wave per SIMD does.  On grids
+// that stay large enough the 8 waves cover 256 rows; on smaller ones (KSPLIT) 128 rows, two waves per 32 rows that take
+// the lower and the upper half of every key tile with a softmax of their own and are merged through LDS at the end
+// (B = 1, L = 1999, H = 16, d = 128, fp16: 108 us with four waves, 88 so, the rows read where they lie).
 constexpr int BN_DEFAULT = 64;  // keys per tile (32 at head dims above 128: LDS)
 
 template <int D, int BM, int BN> struct FwdSmem {
@@ -49,16 +51,16 @@ template <typename T> struct NegInf2;
 template <> struct NegInf2<bf16_tag> { static constexpr uint32_t value = 0xFF80FF80u; };
 template <> struct NegInf2<fp16_tag> { static constexpr uint32_t value = 0xFC00FC00u; };
 
-template <typename T, int D, bool CAUSAL, int NW, int BN>
+template <typename T, int D, bool CAUSAL, int NW, int BN, int KSPLIT, bool ODD>
 __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_kernel(const FwdParams p) {
-    constexpr int NTHREADS = 64 * NW, BM = 32 * NW;
+    constexpr int NTHREADS = 64 * NW, BM = 32 * NW / KSPLIT, BK = BN / KSPLIT;  // (BK: keys of a tile per wave)
     constexpr int FCH = BN / 8;             // 8-key chunks per mask / bias row of a tile
     constexpr int F_RPP = NTHREADS / FCH;   // mask / bias rows staged per pass (FCH threads cover the keys of a row)
     using E = Elem<T>;
     using SM = FwdSmem<D, BM, BN>;
     constexpr int KS = D / 16;  // contraction steps of Q K^T
     constexpr int DB = D / 32;  // 32-wide blocks of the head dimension
-    constexpr int MB = BN / 32, KB = BN / 16;
+    constexpr int MB = BK / 32, KB = BK / 16;
     constexpr int CH = D / 8;               // 16-byte chunks per K row
     constexpr int K_RPP = NTHREADS / CH;    // K rows staged per pass
     constexpr int K_IT = BN / K_RPP;
@@ -67,14 +69,17 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 31, g = lane >> 5;
-    // linear workgroup id -> (query block, head, batch) with the query block OUTERMOST and descending: under causal
-    // masking the blocks with the most KV tiles of every head start first, the light ones fill the tail
-    const int hb_count = p.H * p.B;
+    // linear workgroup id -> (query block, member of the kv group, kv head, batch) with the query block OUTERMOST and
+    // descending: under causal masking the blocks with the most KV tiles of every head start first, the light ones fill the
+    // tail.  The members of a group, which read the same K / V and often the same mask and bias, are a multiple of the kv
+    // head count apart: on one XCD (ids are dealt to the 8 XCDs in turn) when that is a multiple of 8.
+    const int hb_count = p.H * p.B, pairs = p.Hk * p.B;
     const int m_block = (int)gridDim.x / hb_count - 1 - (int)blockIdx.x / hb_count;
-    const int h = ((int)blockIdx.x % hb_count) % p.H, b = ((int)blockIdx.x % hb_count) / p.H;
-    const int hk = h / (p.H / p.Hk);
+    const int pair = (int)blockIdx.x % pairs, hk = pair % p.Hk, b = pair / p.Hk;
+    const int h = hk * (p.H / p.Hk) + ((int)blockIdx.x % hb_count) / pairs;
     const int m0 = m_block * BM;
-    const int wrow0 = m0 + wave * 32;
+    const int rw = wave % (BM / 32), kh = wave / (BM / 32);  // row block and key half of this wave
+    const int wrow0 = m0 + rw * 32;
     const int qrow = wrow0 + r;
     const int shift = p.Lk - p.Lq;  // bottom-right causal alignment
 
@@ -170,13 +175,12 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     auto load_bias = [&](int j, u32x4_t (&dst)[F_IT]) {
         const int n0 = j * BN;
         if (bbase) {
-            int kk = n0 + 8 * fc;
-            kk = kk < p.Lk ? kk : 0;
+            const int at = chunk8_at<ODD>(n0 + 8 * fc, p.Lk);
 #pragma unroll
             for (int it = 0; it < F_IT; it++) {
                 int row = m0 + fr0 + F_RPP * it;
                 row = row < p.Lq ? row : p.Lq - 1;
-                dst[it] = *(const u32x4_t *)(bbase + (int64_t)row * p.bi_r + kk);
+                dst[it] = *(const u32x4_el_t *)(bbase + (int64_t)row * p.bi_r + at);
             }
         } else {
 #pragma unroll
@@ -201,7 +205,8 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
         load_kv(j);
     };
     // registers -> LDS stage `buf`: K and V rows, mask and bias fused (bias where kept, -inf elsewhere)
-    auto store_stage = [&](int buf, const u32x2_t (&mv)[F_IT], const u32x4_t (&bsrc)[F_IT]) {
+    auto store_stage = [&](int j, const u32x2_t (&mv)[F_IT], const u32x4_t (&bsrc)[F_IT]) {
+        const int buf = j & 1, kk = j * BN + 8 * fc;
         char *sK = smem + buf * SM::STAGE;
         char *sVt = sK + SM::K_BYTES;
         char *sF = sVt + SM::VT_BYTES;
@@ -212,7 +217,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
         }
 #pragma unroll
         for (int it = 0; it < F_IT; it++) {
-            u32x4_t bv = bsrc[it];
+            u32x4_t bv = bbase ? chunk8_fix<ODD>(bsrc[it], kk, p.Lk) : bsrc[it];
 #pragma unroll
             for (int hlf = 0; hlf < 2; hlf++) {
                 uint32_t x = mv[it][hlf];
@@ -233,10 +238,10 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
 
     // ---- one tile from LDS stage `buf`
     auto compute = [&](int j, int buf) {
-        const int n0 = j * BN;
-        const char *sK = smem + buf * SM::STAGE;
-        const char *sVt = sK + SM::K_BYTES;
-        const char *sF = sVt + SM::VT_BYTES + ((wave * 32 + r) * SM::SF + 8 * g) * 2;
+        const int n0 = j * BN + kh * BK;
+        const char *sK = smem + buf * SM::STAGE + kh * BK * SM::SK * 2;
+        const char *sVt = smem + buf * SM::STAGE + SM::K_BYTES + kh * BK * LdsTile<D>::ROW_BYTES;
+        const char *sF = smem + buf * SM::STAGE + SM::K_BYTES + SM::VT_BYTES + ((rw * 32 + r) * SM::SF + kh * BK + 8 * g) * 2;
         // scores start from the fused mask+bias tile (exp2 domain)
         f32x16_t s[MB];
 #pragma unroll
@@ -266,7 +271,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             }
         }
         // causal selects on diagonal tiles only (wave-uniform branch)
-        if (CAUSAL && n0 + BN - 1 > wrow0 + shift) {
+        if (CAUSAL && n0 + BK - 1 > wrow0 + shift) {
             asm volatile("" ::: "memory");
             const int lim = qrow + shift - n0 - 8 * g;  // local column limit for this lane
 #pragma unroll
@@ -333,13 +338,13 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
 
     // ---- main loop.  At the top of iteration j: tile j sits in LDS stage j&1 if it is active, `mreg` holds
     // the mask of tile j+1 and `act_next` says whether that tile has any kept element.
-    // DEEP (head dims up to 64, where the registers are there): mask and bias -- the bytes that come from HBM -- stay in
+    // DEEP (head dims up to 64, and two waves per row block: where the registers are there): mask and bias -- the bytes that come from HBM -- stay in
     // flight for TWO iterations instead of one.  With one, every iteration contained a whole trip to memory (the mask
     // requested at its top decided, at its end, whether the tile after the next is fetched at all), and the launch moved
     // what it had in flight once per trip: 64 KB per CU every 3.5 us.  Now the mask of tile j+4 and the bias of tile
     // j+2 are requested at the top of iteration j, behind K / V of tile j+1 (cache hits; waiting for those must not
     // mean waiting for the younger requests: loads come back in the order they were issued).
-    constexpr bool DEEP = D <= 64;
+    constexpr bool DEEP = D <= 64 || KSPLIT == 2;
     if (n_end > 0 && DEEP) {
         u32x2_t m1[F_IT], m2[F_IT], m3[F_IT];            // with mreg: the masks of tiles j .. j+3 at the top of iteration j
         u32x4_t b1[F_IT], b2[F_IT];                      // bias of tiles j+1 (requested an iteration ago), j+2
@@ -369,7 +374,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             __builtin_amdgcn_sched_barrier(0);
             if (act_cur) compute(j, j & 1);
             __builtin_amdgcn_sched_barrier(0);
-            if (have_next) store_stage((j + 1) & 1, ma, ba);
+            if (have_next) store_stage(j + 1, ma, ba);
             const bool act_3 = __syncthreads_or(j + 3 < n_end && finish_mask(j + 3, mc));
             act_cur = have_next;
             act_1 = act_2;
@@ -401,7 +406,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             __builtin_amdgcn_sched_barrier(0);
             if (act_cur) compute(j, j & 1);
             __builtin_amdgcn_sched_barrier(0);
-            if (have_next) store_stage((j + 1) & 1, m_next, breg);
+            if (have_next) store_stage(j + 1, m_next, breg);
             const bool act_nn = __syncthreads_or(j + 2 < n_end && finish_mask(j + 2, m_new));
             act_cur = have_next;
             act_next = act_nn;
@@ -413,7 +418,37 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     }
 
     // ---- epilogue: normalise, store O and LSE
-    const float total = xhalf_sum(row_sum);
+    float total = xhalf_sum(row_sum);
+    if constexpr (KSPLIT == 2) {
+        // the upper key half hands over its sums and O (relative to its own maximum); the lower half merges and stores
+        float *xm = (float *)smem + rw * 64 + lane;                                    // maximum, sum: 2 * BM / 32 * 64 floats
+        f32x4_t *xo = (f32x4_t *)(smem + 2 * (BM / 32) * 256) + rw * DB * 4 * 64 + lane;
+        __syncthreads();  // (the tiles' last reads)
+        if (kh == 1) {
+            xm[0] = row_max;
+            xm[(BM / 32) * 64] = total;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    xo[(db * 4 + q) * 64] = f32x4_t{o[db][4 * q], o[db][4 * q + 1], o[db][4 * q + 2], o[db][4 * q + 3]};
+        }
+        __syncthreads();
+        if (kh == 1) return;
+        const float m1 = xm[0], t1 = xm[(BM / 32) * 64];
+        const float mx = fmaxf(row_max, m1), safe = mx == -INFINITY ? 0.f : mx;
+        const float w0 = fast_exp2(row_max - safe), w1 = fast_exp2(m1 - safe);
+        total = total * w0 + t1 * w1;
+        row_max = mx;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const f32x4_t v = xo[(db * 4 + q) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[db][4 * q + e] = o[db][4 * q + e] * w0 + v[e] * w1;
+            }
+    }
     const float inv = total > 0.f ? 1.f / total : 0.f;
     if (qrow < p.Lq) {
         uint16_t *op = (uint16_t *)p.o + b * p.o_b + (int64_t)qrow * p.o_r + h * p.o_h;
@@ -437,10 +472,10 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     }
 }
 
-template <typename T, int D, bool CAUSAL, int NW>
-hipError_t launch_fwd_c(const FwdParams &p, hipStream_t stream) {
-    constexpr int BM = 32 * NW, NTHREADS = 64 * NW, BN = D > 128 ? 32 : BN_DEFAULT;
-    auto kern = fwd_kernel<T, D, CAUSAL, NW, BN>;
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, bool ODD>
+hipError_t launch_fwd_o(const FwdParams &p, hipStream_t stream) {
+    constexpr int BM = 32 * NW / KSPLIT, NTHREADS = 64 * NW, BN = D > 128 ? 32 : BN_DEFAULT;
+    auto kern = fwd_kernel<T, D, CAUSAL, NW, BN, KSPLIT, ODD>;
     const int smem = FwdSmem<D, BM, BN>::TOTAL;
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
@@ -450,14 +485,22 @@ hipError_t launch_fwd_c(const FwdParams &p, hipStream_t stream) {
     return hipGetLastError();
 }
 
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT = 1>
+hipError_t launch_fwd_c(const FwdParams &p, hipStream_t stream) {
+    if (D > 128 || odd_rows(p)) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, true>(p, stream);
+    return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, D <= 128 ? false : true>(p, stream);
+}
+
 template <typename T, int D>
 hipError_t launch_fwd_t(const FwdParams &p, hipStream_t stream) {
     if constexpr (D > 64 && D <= 128) {
         // 256-row workgroups while the grid still covers the chip about twice
         if ((int64_t)p.B * p.H * ((p.Lq + 255) / 256) >= 512)
             return p.causal ? launch_fwd_c<T, D, true, 8>(p, stream) : launch_fwd_c<T, D, false, 8>(p, stream);
+        return p.causal ? launch_fwd_c<T, D, true, 8, 2>(p, stream) : launch_fwd_c<T, D, false, 8, 2>(p, stream);
+    } else {
+        return p.causal ? launch_fwd_c<T, D, true, 4>(p, stream) : launch_fwd_c<T, D, false, 4>(p, stream);
     }
-    return p.causal ? launch_fwd_c<T, D, true, 4>(p, stream) : launch_fwd_c<T, D, false, 4>(p, stream);
 }
 
 }  // namespace

@@ -188,7 +188,9 @@ struct BwdParams {
     int32_t Lq_rounded;
     float *dbias_accum;        // fp32 scratch at the dbias shape when several workgroups share an element
     int64_t dba_b, dba_h, dba_r;
-    // compacted dK/dV kernel, split mode: per part [2][Dpad][128] fp32 (dK^T, dV^T) and [G][128] fp32 (dBias)
+    int32_t kv_segs;           // general dK/dV kernel: segments of the query blocks (1 = no split; see general_kv_segments)
+    // general dK/dV kernel with segments: per part [2][128][Dpad] fp32 (dK, dV, in register order) and [G][128] fp32 (dBias
+    // columns).  Compacted dK/dV kernel, split mode: per part [2][Dpad][128] fp32 (dK^T, dV^T) and [G][128] fp32 (dBias)
     float *dkv_part;
     float *db_part;
     int32_t dot_done;          // softmax_d has been computed by an earlier launch of this call
@@ -284,6 +286,9 @@ hipError_t launch_bwd_dq_colmask(const BwdParams &p, int dtype, hipStream_t stre
 // and batch entry, dBias written directly): one tile GEMM and no second pass over mask, bias, Q, V, dO
 bool bwd_dq_from_ds_applicable(const BwdParams &p);
 hipError_t launch_bwd_dq_from_ds(const BwdParams &p, int dtype, hipStream_t stream);
+// dK / dV / dBias of the general form at head dims 65 .. 128 (fdma_bwd_dkdv_wide.hip); gsum: a per-query dBias element is
+// shared by several query heads
+hipError_t launch_bwd_dkdv_wide(const BwdParams &p, int dtype, bool gsum, hipStream_t stream);
 // general dQ kernel (mask / bias per query row), fdma_bwd_dq.hip
 hipError_t launch_bwd_dq(const BwdParams &p, int dtype, hipStream_t stream);
 
@@ -329,6 +334,20 @@ inline void dkdv_split_bounds(int pairs, int n_max, int G, int &grid, int &slots
     grid = (int)(8 * lists_per_xcd * items);
     slots = (int)sl;
 }
+
+// general dK/dV kernel: segments its query blocks are cut into, and the bytes of the segments' fp32 sums (and of their dBias
+// columns) the call must provide
+int general_kv_segments(const FwdParams &f);
+size_t general_kv_part_bytes(const FwdParams &f, size_t *db_bytes);
+// general kernels: mask or bias rows that are not made of whole, aligned 8-key chunks (see chunk8_at in fdma_common.h)
+inline bool odd_rows(const FwdParams &f) {
+    if (f.Lk % 8 != 0) return true;
+    const bool m = f.mask && !f.mbits && (((uintptr_t)f.mask | (uintptr_t)f.m_b | (uintptr_t)f.m_h | (uintptr_t)f.m_r) & 7) != 0;
+    const bool b = f.bias && (((uintptr_t)f.bias & 15) != 0 || ((f.bi_b | f.bi_h | f.bi_r) & 7) != 0);
+    return m || b;
+}
+// compute units of the current device (256 where there is none)
+int device_cus();
 
 // number of KV splits the decode path uses for this shape (1 = no workspace needed)
 int decode_num_splits(int B, int Hk, int Lk);

@@ -296,8 +296,8 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             (t == &mask ? t->size(3) < Lk : t->size(3) != Lk) || t->stride(3) != 1)
             Py_RETURN_NOTIMPLEMENTED;
     }
-    // (rows that all queries share are taken as they lie, rows per query in aligned vectors: fdma.h)
-    const bool rows = Lq > 1 && ((mask.defined() && mask.size(2) != 1) || (bias.defined() && bias.size(2) != 1) || Lk > (1 << 19));
+    // (rows are taken as they lie, unless they differ per query and are shorter than a chunk: fdma.h)
+    const bool rows = Lq > 1 && Lk < 8 && ((mask.defined() && mask.size(2) != 1) || (bias.defined() && bias.size(2) != 1));
     if (rows && ((mask.defined() && !vec_ok(mask, 16)) || (bias.defined() && !vec_ok(bias, 8)))) Py_RETURN_NOTIMPLEMENTED;
     if (mask.defined()) {
         // a row per query head over grouped kv heads (its backward is taken apart), or rows that may turn out to be a

@@ -63,13 +63,12 @@ enum {
  * capture of forward + backward through the tensor library ended in a host crash when the capture was closed; its
  * cause is not known, so the library refuses instead.)
  *
- * Readable lengths of mask and bias rows.  Where mask and bias are broadcast over the queries (or seqlen_q == 1, and up
- * to 2^19 keys) exactly seqlen_k elements of a row are read, at any address and stride.  Otherwise the kernels read mask
- * rows in 16-byte and bias rows in 16-byte (8-element) vectors: each row of `mask` must be readable up to seqlen_k rounded up to 16 bytes, each row of `bias`
- * up to seqlen_k rounded up to 8 elements, whatever lies there; this also holds for the last row of the buffer, and for a fully
- * broadcast mask or bias of a single row.  The library cannot check it (it never sees the row length).  The reference
- * asks for more: rows of exactly round_up(seqlen_k, 128) elements (flash_api.cpp:420, 431, 437).  Values beyond
- * seqlen_k are never used, and dbias is only written up to seqlen_k. */
+ * Mask and bias rows.  Rows of at least 8 keys are taken at any address and stride (bias: 2-byte aligned) and exactly
+ * seqlen_k elements of a row are read.  Rows of fewer than 8 keys that differ per query are read in 8-key chunks: then mask
+ * and bias must be 16-byte aligned with strides that are multiples of 16 (mask) or 8 (bias) elements, and readable up to 8
+ * keys per row, whatever lies there.  (The reference asks for rows of exactly round_up(seqlen_k, 128) elements,
+ * flash_api.cpp:420, 431, 437.)  Values beyond seqlen_k are never used; dbias rows hold whole 8-element vectors (aligned,
+ * strides multiples of 8), of which elements beyond seqlen_k may be overwritten. */
 
 /* Column compaction (fdma_fwd_args.compact_mode).  A keep-mask that is broadcast over the queries, with 1 or
  * num_heads_k heads, drops whole key columns; the library can then gather the kept K / V rows into dense copies
