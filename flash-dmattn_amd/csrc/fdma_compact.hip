@@ -653,24 +653,34 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
                                            int Lq, int Lk, int causal, int slots, int cap) {
     constexpr int MAXU = DKDV_ENOUGH_UNITS;  // units are split only below this many (and there are no more pairs than units)
     constexpr int MAXL = 1024;               // ... and with at most this many unit lists (LDS: every block of the launch pays for it)
-    __shared__ int s_sum, s_max, s_n[256], s_units;
+    __shared__ int s_sum, s_max, s_units, s_wsum[4], s_wmax[4];
     __shared__ int s_Gs, s_Sm, s_Q, s_fit, s_q1, s_parts2, s_over2;
     __shared__ int s_first[MAXU + 1], s_nt[MAXU], s_len[MAXU], s_nseg[MAXU], s_uoff[MAXU], s_lcount[MAXL], s_cand[64][8];
-    const int tid = threadIdx.x;
-    // units per pair and their prefix: the counts are fetched 256 at a time by all threads (one memory latency per
-    // chunk instead of one per pair), the prefix over a chunk is then taken from LDS by one thread
-    int u = 0, n_max = 0;  // (meaningful in thread 0)
+    __shared__ int s_pair[MAXU], s_ntx[MAXU];  // pair of a unit; its query blocks and, in the upper half, its XCD
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // units per pair and their prefix, 256 pairs at a time
+    int u = 0, n_max = 0;
     for (int base = 0; base < pairs; base += 256) {
-        if (base + tid < pairs) s_n[tid] = (count[base + tid] + 127) / 128;
+        const int n = base + tid < pairs ? (count[base + tid] + 127) / 128 : 0;
+        int incl = n, mx = n;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int t = __shfl_up(incl, off);
+            if (lane >= off) incl += t;
+            mx = max(mx, __shfl_xor(mx, off));
+        }
+        if (lane == 63) { s_wsum[wave] = incl; s_wmax[wave] = mx; }
         __syncthreads();
-        if (tid == 0) {
-            const int m = pairs - base < 256 ? pairs - base : 256;
-            for (int i = 0; i < m; i++) {
-                plan[DKDV_PLAN_HDR + base + i] = u;
-                if (base + i < MAXU) s_first[base + i] = u;
-                u += s_n[i];
-                n_max = s_n[i] > n_max ? s_n[i] : n_max;
-            }
+        int before = u;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            if (w < wave) before += s_wsum[w];
+            u += s_wsum[w];
+            n_max = max(n_max, s_wmax[w]);
+        }
+        if (base + tid < pairs) {
+            plan[DKDV_PLAN_HDR + base + tid] = before + incl - n;
+            if (base + tid < MAXU) s_first[base + tid] = before + incl - n;
         }
         __syncthreads();
     }
@@ -708,11 +718,20 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
         const int i = pair_of(g);
         const int nt = dkdv_query_blocks(Lq, Lk, causal, idx[(size_t)i * ld + (g - s_first[i]) * 128]);
         s_nt[g] = nt;
+        s_pair[g] = i;
+        s_ntx[g] = nt | (((i * dkdv_lists_per_pair(pairs) + dkdv_list_of(g - s_first[i], dkdv_lists_per_pair(pairs))) & 7) << 24);
         sum += nt;
         mx = nt > mx ? nt : mx;
     }
-    atomicAdd(&s_sum, sum);
-    atomicMax(&s_max, mx);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        sum += __shfl_xor(sum, off);
+        mx = max(mx, __shfl_xor(mx, off));
+    }
+    if (lane == 0) {
+        atomicAdd(&s_sum, sum);
+        atomicMax(&s_max, mx);
+    }
     __syncthreads();
     if (tid == 0) {
         int Q = 1 << 30, fit = 1;
@@ -748,19 +767,23 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
         const int step = (s_max - fit + 61) / 62 > 0 ? (s_max - fit + 61) / 62 : 1;
         const int Qc = cand == 63 ? s_Q : fit + cand * step;
         const float rq = 1.0f / (float)Qc;
-        int c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        int i = 0;
+        // (eight 16-bit counters in four words: at most 384 units of 16 segments)
+        uint32_t c[4] = {0, 0, 0, 0};
+#pragma unroll 4
         for (int g = quarter; g < U; g += 4) {
-            while (s_first[i + 1] <= g) i++;
-            const int x = (i * k + dkdv_list_of(g - s_first[i], k)) & 7;
+            const int ntx = s_ntx[g], x = ntx >> 24;
             // ceil(nt / Qc), exactly: the half keeps the float quotient off the integers
-            int ns = (int)(((float)(s_nt[g] + Qc - 1) + 0.5f) * rq);
+            int ns = (int)(((float)((ntx & 0xffffff) + Qc - 1) + 0.5f) * rq);
             ns = ns < Sm ? ns : Sm;
+            const uint32_t add = (uint32_t)ns << (16 * (x & 1));
 #pragma unroll
-            for (int e = 0; e < 8; e++) c[e] += x == e ? ns : 0;
+            for (int e = 0; e < 4; e++) c[e] += (x >> 1) == e ? add : 0u;
         }
 #pragma unroll
-        for (int e = 0; e < 8; e++) if (c[e]) atomicAdd(&s_cand[cand][e], c[e]);
+        for (int e = 0; e < 8; e++) {
+            const int ce = (int)((c[e >> 1] >> (16 * (e & 1))) & 0xffffu);
+            if (ce) atomicAdd(&s_cand[cand][e], ce);
+        }
         __syncthreads();
         if (tid < 64) {
             int worst = 0, parts = 0;
@@ -806,9 +829,10 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
     }
     __syncthreads();
     for (int g = tid; g < U; g += 256) {
-        const int i = pair_of(g), first = s_first[i], n = s_first[i + 1] - first, un = g - first;
+        const int i = s_pair[g], first = s_first[i], n = s_first[i + 1] - first, un = g - first;
         const int mine = s_len[g], fold = dkdv_list_of(un, k);
         int before = 0;  // parts of the units of the same list that come first
+#pragma unroll 4
         for (int v = 0; v < n; v++) {
             const bool first_v = dkdv_list_of(v, k) == fold && (s_len[first + v] > mine || (s_len[first + v] == mine && v < un));
             before += first_v ? s_nseg[first + v] : 0;
@@ -832,7 +856,7 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
     }
     __syncthreads();
     for (int g = tid; g < U; g += 256) {
-        const int i = pair_of(g), un = g - s_first[i], vl = i * k + dkdv_list_of(un, k), ns = s_nseg[g];
+        const int i = s_pair[g], un = g - s_first[i], vl = i * k + dkdv_list_of(un, k), ns = s_nseg[g];
         int o = s_lcount[vl] + s_uoff[g];
         int32_t *e = lists + 8 + 2 * ((size_t)(vl & 7) * cap);
         for (int gi = 0; gi < Gs0; gi++)
@@ -846,21 +870,24 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
     }
 }
 
-// Everything the compacted backward needs after the scan, in one launch: layer 0 of the grid gathers K / V rows,
-// layer 1 clears the gradients of dropped keys, one workgroup of layer 2 makes the dK/dV plan, and the layers from 3
-// on compute D = rowsum(dO * O), which depends on none of the others.
-// The plan is a chain of dependent steps of a single workgroup (18 us); side by side with the other two it costs nothing.
+// Everything the compacted backward needs after the scan, in one launch: one workgroup of layer 0 of the grid makes the
+// dK/dV plan, layer 1 gathers K / V rows, layer 2 clears the gradients of dropped keys, and the layers from 3 on compute
+// D = rowsum(dO * O), which depends on none of the others.
+// The plan is a chain of dependent steps of a single workgroup: in the FIRST layer it starts with the launch and the others
+// run beside it.  (4 x 2048 tokens, 8 kv heads, d = 64: the chain was the launch, 26 us, most of it the comparison of
+// segment lengths walking the units with a division each; with what a unit contributes made once and the prefixes taken by
+// whole waves the launch takes 12 us.  8192 tokens of 32 heads, d = 128: 30 us, bound by reading dO and O.)
 template <typename T>
 __global__ void __launch_bounds__(256) compact_bwd_prepass_kernel(const BwdParams bp, const int32_t *idx, int32_t *cnt,
                                                                    const int32_t *count, float *fb, uint16_t *kc, uint16_t *vc,
                                                                    int ld, int Hfb, int32_t *plan, int slots, int cap, int do_gather) {
     const FwdParams &f = bp.f;
-    if (blockIdx.z == 0) {
+    if (blockIdx.z == 1) {
         // (not when the lists and copies exist already: made by an earlier launch, or by the forward call)
         if (do_gather) gather_block<T>(f, idx, cnt, count, fb, kc, vc, ld, Hfb, blockIdx.x, blockIdx.y, do_gather == 2);
-    } else if (blockIdx.z == 1) {
-        zero_block(bp, bp.dbias != nullptr && bp.dbias_accum == nullptr, blockIdx.x, blockIdx.y);
     } else if (blockIdx.z == 2) {
+        zero_block(bp, bp.dbias != nullptr && bp.dbias_accum == nullptr, blockIdx.x, blockIdx.y);
+    } else if (blockIdx.z == 0) {
         if (blockIdx.x == 0 && blockIdx.y == 0)
             plan_block(count, idx, ld, plan, f.B * f.Hk, f.H / f.Hk, f.Lq, f.Lk, f.causal, slots, cap);
     } else {  // the blocks of D = rowsum(dO * O), laid out over the remaining layers

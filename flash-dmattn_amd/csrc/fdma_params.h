@@ -96,7 +96,7 @@ __host__ __device__ inline int dkdv_unit_at(int pos, int fold, int k) {
     return 2 * k * (pos >> 1) + ((pos & 1) ? 2 * k - 1 - fold : fold);
 }
 __host__ __device__ inline int dkdv_list_of(int u, int k) {
-    const int rem = u % (2 * k);
+    const int rem = u & (2 * k - 1);  // (k is 1, 2, 4 or 8)
     return rem < k ? rem : 2 * k - 1 - rem;
 }
 __host__ __device__ inline int dkdv_list_len(int units_in_largest_pair, int k) {
