@@ -646,7 +646,7 @@ int fdma_dyn_bias_validate(const fdma_dyn_bias_args *a, int backward) {
     if (a->head_dim <= 0 || a->head_dim % 8 != 0 || (a->num_heads_k * a->head_dim) % 16 != 0)
         return fail(FDMA_ERR_UNSUPPORTED, "head_dim must be a multiple of 8 and num_heads_k * head_dim a multiple of 16");
     const bool empty = (int64_t)a->batch * a->seqlen_k == 0;
-    if (!a->weight || !a->a || (!empty && (!a->value || !a->bias || !a->dt))) return fail(FDMA_ERR_INVALID, "value, weight, a, bias, dt must be device pointers");
+    if (!a->weight || !a->a || (!empty && (!a->value || !a->bias || (backward && !a->dt)))) return fail(FDMA_ERR_INVALID, "value, weight, a, bias, dt must be device pointers");
     if (!aligned16(a->value) || !aligned16(a->weight) || !strides_ok(a->value_strides, 8))
         return fail(FDMA_ERR_INVALID, "value and weight must be 16-byte aligned, value strides multiples of 8 elements");
     if (backward) {

@@ -2,19 +2,25 @@
 // (flash_sparse_attn/utils/mask.py:47-160) as ONE kernel per call instead of masked_fill + topk + zeros + scatter
 // (+ view / sum / copy for the smoothing) through a tensor library.
 //
-// One workgroup (4 or 16 waves) owns one row of `seqlen_k` bias values (16-bit floats).  The `window` largest are
-// found by a two-level radix select on an order-preserving 16-bit key: a 256-bin histogram of the high byte in LDS (one copy per
-// LDS bank: the high byte is sign and exponent, so most of a row falls into a handful of bins),
-// a wave-parallel suffix scan that finds the bin holding the window-th largest value, the same again for the low
-// byte inside that bin.  That yields the exact threshold value T, the number of entries above it and how many
-// entries EQUAL to T are still needed; those are taken in ascending column order (the reference's torch.topk leaves
-// the choice among equal values unspecified).  HBM traffic is one read of the row (the second and third pass hit in
-// L2 / L1) and one write of the mask row.
+// One workgroup owns one row of `seqlen_k` bias values (16-bit floats).  The `window` largest are found by a two-level
+// radix select on an order-preserving 16-bit key: a 256-bin histogram of the high byte in LDS (several copies in different
+// banks: the high byte is sign and exponent, so most of a row falls into a handful of bins), a wave-parallel suffix scan
+// that finds the bin holding the window-th largest value, the same again for the low byte inside that bin.  That yields the
+// exact threshold value T, the number of entries above it and how many entries EQUAL to T are still needed; those are taken
+// in ascending column order (the reference's torch.topk leaves the choice among equal values unspecified).
+//
+// A row is a chain of dependent steps with hardly any bytes, so make_mask_kernel keeps it in registers from the one load
+// to the last output: a thread holds KPT chunks of 8 columns; every wave finds the bins for itself (no broadcast, five
+// barriers in all), and mask, bit row and the list of kept columns come out of one prefix sum over the workgroup.  (Passes
+// over memory for each step, the list from the stored mask: 64 rows of 4093 keys 16.7 us, now 8.1.)  Rows of fewer than 8
+// or more than 65536 keys and block smoothing take make_mask_memory_kernel, which walks the row in memory.
 //
 // As in the reference, entries excluded by an incoming mask are pushed to `min_value` before the selection, and a
 // selected entry whose value equals `min_value` is not kept; the optional block smoothing then replaces every
 // aligned block of `block_size` keys by the majority vote of its entries (a shorter tail block votes over its own
 // length; exactly half is dropped).
+#include <type_traits>
+
 #include "fdma_common.h"
 #include "fdma_params.h"
 #include "fdma_scan.h"
@@ -55,13 +61,235 @@ __device__ __forceinline__ void find_bin(const uint32_t *hist, uint32_t k, uint3
     }
 }
 
-// NT threads own one row.  A thread handles 8 consecutive columns at a time (one 16-byte load of bias, one 8-byte
+// The same by every wave for itself, the answer in scalar registers.  h: 256 bins.
+__device__ __forceinline__ void find_bin_wave(const uint32_t *h, uint32_t k, uint32_t &bin, uint32_t &above) {
+    const int lane = threadIdx.x & 63;
+    uint32_t c[4], s = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        c[j] = h[255 - 4 * lane - j];
+        s += c[j];
+    }
+    uint32_t incl = s;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t t = __shfl_up(incl, off);
+        if (lane >= off) incl += t;
+    }
+    uint32_t a = incl - s, mine_bin = 0, mine_above = 0;
+    const uint64_t who = __ballot(a < k && k <= incl);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (a < k && k <= a + c[j]) {
+            mine_bin = 255 - 4 * lane - j;
+            mine_above = a;
+        }
+        a += c[j];
+    }
+    const int l = who ? __builtin_ctzll(who) : 0;
+    bin = __builtin_amdgcn_readlane(mine_bin, l);
+    above = __builtin_amdgcn_readlane(mine_above, l);
+}
+
+// One row in registers: NT threads, chunk c of thread t = columns (c * NT + t) * 8 .. + 7.  Lk >= 8, Lk <= NT * 8 * KPT.
+template <int NT, int KPT>
+__global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
+    constexpr int NW = NT / 64, REP1 = NT >= 512 ? 16 : 8, REP2 = 4;
+    __shared__ uint32_t hist1[256 * REP1], hist2[256 * REP2], hsum[2][256];
+    __shared__ uint32_t s_tot[2][KPT * NW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = blockIdx.x;
+    const int r = row % p.rows, h = (row / p.rows) % p.heads, b = row / (p.rows * p.heads);
+    const uint16_t *brow = (const uint16_t *)p.bias + b * p.bi_b + h * p.bi_h + (int64_t)r * p.bi_r;
+    const uint8_t *mrow = p.mask_in ? p.mask_in + b * p.mi_b + h * p.mi_h + (int64_t)r * p.mi_r : nullptr;
+    uint8_t *orow = p.mask_out + b * p.mo_b + h * p.mo_h + (int64_t)r * p.mo_r;
+    const int Lk = p.Lk;
+    const uint32_t min_bits = p.min_bits;
+    auto first_col = [&](int c) -> int { return (c * NT + tid) * 8; };
+    // ---- the row, after the masked fill, as bits of the bias type
+    uint32_t v[KPT][4];
+    {
+        u32x4_t raw[KPT];
+        u32x2_t mm[KPT];
+#pragma unroll
+        for (int c = 0; c < KPT; c++) {
+            raw[c] = *(const u32x4_el_t *)(brow + chunk8_at<true>(first_col(c), Lk));
+            if (mrow) mm[c] = *(const u32x2_any_t *)(mrow + chunk8_at<true>(first_col(c), Lk));
+        }
+        for (int i = tid; i < 256 * REP1; i += NT) hist1[i] = 0;
+        for (int i = tid; i < 256 * REP2; i += NT) hist2[i] = 0;
+#pragma unroll
+        for (int c = 0; c < KPT; c++) {
+            const u32x4_t x = chunk8_fix<true>(raw[c], first_col(c), Lk);
+            const u32x2_t m = mrow ? chunk8_fix_mask<true>(mm[c], first_col(c), Lk) : u32x2_t{0x01010101u, 0x01010101u};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t two = m[e >> 1] >> (16 * (e & 1));
+                const uint32_t lo = (two & 0xffu) ? x[e] & 0xffffu : min_bits, hi = (two & 0xff00u) ? x[e] >> 16 : min_bits;
+                v[c][e] = lo | (hi << 16);
+            }
+        }
+    }
+    auto bits_of = [&](int c, int j) -> uint32_t { return (v[c][j >> 1] >> (16 * (j & 1))) & 0xffffu; };
+    auto valid = [&](int c) -> int {  // columns of the chunk inside the row
+        const int n = Lk - first_col(c);
+        return n >= 8 ? 8 : (n < 0 ? 0 : n);
+    };
+    // "is the fill value" compares numerically (+0 == -0)
+    auto is_min = [&](uint32_t x) -> bool { return x == min_bits || (((x | min_bits) & 0x7fffu) == 0); };
+    // exclusive prefix, in column order, of a count per chunk; returns the row's total
+    auto prefix = [&](uint32_t *tot, const int (&n)[KPT], int (&before)[KPT]) -> int {
+#pragma unroll
+        for (int c = 0; c < KPT; c++) {
+            int incl = n[c];
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int t = __shfl_up(incl, off);
+                if (lane >= off) incl += t;
+            }
+            if (lane == 63) tot[c * NW + wave] = incl;
+            before[c] = incl - n[c];
+        }
+        __syncthreads();
+        // every wave sums the (chunk, wave) totals for itself, two per lane
+        constexpr int N = KPT * NW;
+        static_assert(N <= 128, "two totals per lane");
+        const int t0 = 2 * lane < N ? (int)tot[2 * lane] : 0, t1 = 2 * lane + 1 < N ? (int)tot[2 * lane + 1] : 0;
+        int incl = t0 + t1;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int t = __shfl_up(incl, off);
+            if (lane >= off) incl += t;
+        }
+        const int e0 = incl - t0 - t1, e1 = incl - t1;
+#pragma unroll
+        for (int c = 0; c < KPT; c++) {
+            const int i = c * NW + wave;
+            const int a0 = __shfl(e0, i >> 1), a1 = __shfl(e1, i >> 1);
+            before[c] += (i & 1) ? a1 : a0;
+        }
+        return __shfl(incl, 63);
+    };
+
+    uint32_t keep[KPT];  // one bit per column of the chunk
+#pragma unroll
+    for (int c = 0; c < KPT; c++) keep[c] = 0;
+    if (p.type == 1) {  // relu: keep strictly positive values (NaN is not > 0)
+        const uint32_t inf = p.dtype == 0 ? 0x7f80u : 0x7c00u;
+#pragma unroll
+        for (int c = 0; c < KPT; c++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint32_t x = bits_of(c, j), mag = x & 0x7fffu;
+                if (j < valid(c) && !(x & 0x8000u) && mag != 0 && mag <= inf) keep[c] |= 1u << j;
+            }
+    } else if (p.window > 0) {
+        const uint32_t k = (uint32_t)(p.window < Lk ? p.window : Lk);
+        auto fold = [&](const uint32_t *hist, auto rep_c, uint32_t *sum) {
+            constexpr int REP = decltype(rep_c)::value;
+            for (int t = tid; t < 256; t += NT) {
+                uint32_t s = 0;
+#pragma unroll
+                for (int i = 0; i < REP; i++) s += hist[t * REP + ((t + i) & (REP - 1))];  // (the lanes on different banks)
+                sum[t] = s;
+            }
+            __syncthreads();
+        };
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < KPT; c++)
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (j < valid(c)) atomicAdd(&hist1[(order_key(bits_of(c, j)) >> 8) * REP1 + (lane & (REP1 - 1))], 1u);
+        __syncthreads();
+        fold(hist1, std::integral_constant<int, REP1>(), hsum[0]);
+        uint32_t bin1, above1, bin2, above2;
+        find_bin_wave(hsum[0], k, bin1, above1);
+#pragma unroll
+        for (int c = 0; c < KPT; c++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint32_t key = order_key(bits_of(c, j));
+                if (j < valid(c) && (key >> 8) == bin1) atomicAdd(&hist2[(key & 0xffu) * REP2 + (lane & (REP2 - 1))], 1u);
+            }
+        __syncthreads();
+        fold(hist2, std::integral_constant<int, REP2>(), hsum[1]);
+        find_bin_wave(hsum[1], k - above1, bin2, above2);
+        const uint32_t T = (bin1 << 8) | bin2;
+        const uint32_t need_eq = k - above1 - above2;  // >= 1 entries equal to T still to take
+        int rank[KPT];
+        if (need_eq < hsum[1][bin2]) {  // ties across the threshold: the first need_eq of them in column order
+            int eq[KPT];
+#pragma unroll
+            for (int c = 0; c < KPT; c++) {
+                eq[c] = 0;
+#pragma unroll
+                for (int j = 0; j < 8; j++) eq[c] += (j < valid(c) && order_key(bits_of(c, j)) == T) ? 1 : 0;
+            }
+            prefix(s_tot[0], eq, rank);
+        } else {
+#pragma unroll
+            for (int c = 0; c < KPT; c++) rank[c] = -0x40000000;
+        }
+#pragma unroll
+        for (int c = 0; c < KPT; c++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint32_t x = bits_of(c, j), key = order_key(x);
+                const bool in = j < valid(c), eq = in && key == T;
+                if (in && (key > T || (eq && rank[c] < (int)need_eq)) && !is_min(x)) keep[c] |= 1u << j;
+                rank[c] += eq ? 1 : 0;
+            }
+    }
+
+    // ---- the mask row, and its bits (key j of a row in bit j % 8 of byte j / 8)
+#pragma unroll
+    for (int c = 0; c < KPT; c++) {
+        const int col = first_col(c), n = valid(c);
+        const u32x2_t bytes = mask_bits_to_bytes(keep[c]);
+        if (n == 8) {
+            *(u32x2_any_t *)(orow + col) = bytes;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (j < n) orow[col + j] = (uint8_t)((keep[c] >> j) & 1u);
+        }
+        if (p.bits && n > 0) p.bits[(size_t)row * p.bits_row_bytes + (col >> 3)] = (uint8_t)keep[c];
+    }
+    // ---- the row as an ordered list of kept columns with inclusive prefix counts (fdma_scan.h), written up to
+    // round_up(Lk, 16): the row has room
+    if (p.kept_idx) {
+        int32_t *irow = p.kept_idx + (size_t)row * p.kept_ld, *crow = p.kept_cnt + (size_t)row * p.kept_ld;
+        int n[KPT], run[KPT];
+#pragma unroll
+        for (int c = 0; c < KPT; c++) n[c] = __builtin_popcount(keep[c]);
+        const int total = prefix(s_tot[1], n, run);
+#pragma unroll
+        for (int c = 0; c < KPT; c++) {
+            const int col = first_col(c);
+            if (col < (Lk + 15) / 16 * 16) {
+                uint32_t cv[8];
+                int at = run[c];
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    if ((keep[c] >> j) & 1u) irow[at++] = col + j;
+                    cv[j] = (uint32_t)at;
+                }
+                *(u32x4_t *)(crow + col) = u32x4_t{cv[0], cv[1], cv[2], cv[3]};
+                *(u32x4_t *)(crow + col + 4) = u32x4_t{cv[4], cv[5], cv[6], cv[7]};
+            }
+        }
+        if (tid == 0) p.kept_count[row] = total;
+    }
+}
+
+// The row in memory.  NT threads own one row.  A thread handles 8 consecutive columns at a time (one 16-byte load of bias, one 8-byte
 // load of the incoming mask, one 8-byte store of the result when the row addresses allow it).
 // REP copies of the histogram, copy = lane % REP, laid out [bin][copy] so that the copies of a bin sit in different
 // LDS banks: lanes that hit the same bin do not serialise (32 copies for long rows; 8 for short ones, where clearing
 // and folding the copies would cost more than the conflicts).
 template <int NT, int REP>
-__global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
+__global__ void __launch_bounds__(NT) make_mask_memory_kernel(const MaskParams p) {
     __shared__ uint32_t hist[256 * REP];  // [bin][copy]
     __shared__ uint32_t hsum[256];
     __shared__ uint32_t res[4];
@@ -290,10 +518,27 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
 hipError_t launch_make_mask(const MaskParams &p, hipStream_t stream) {
     const int64_t n_rows = (int64_t)p.batch * p.heads * p.rows;
     if (n_rows <= 0 || p.Lk <= 0) return hipSuccess;
+    if (p.Lk >= 8 && p.Lk <= 65536 && p.block_size <= 1) {
+        // few rows: enough threads for one chunk of 8 columns each, up to 16 waves per row (the row is a latency chain);
+        // many rows: 4 waves per row and several rows per CU, each thread with more of the row
+        auto go = [&](auto kern, int nt) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)n_rows), dim3(nt), 0, stream, p);
+            return hipGetLastError();
+        };
+        const bool many = n_rows >= 1024;
+        if (p.Lk <= 2048) return go(make_mask_kernel<256, 1>, 256);
+        if (many && p.Lk <= 4096) return go(make_mask_kernel<256, 2>, 256);
+        if (many && p.Lk <= 8192) return go(make_mask_kernel<256, 4>, 256);
+        if (p.Lk <= 4096) return go(make_mask_kernel<512, 1>, 512);
+        if (p.Lk <= 8192) return go(make_mask_kernel<1024, 1>, 1024);
+        if (p.Lk <= 16384) return go(make_mask_kernel<1024, 2>, 1024);
+        if (p.Lk <= 32768) return go(make_mask_kernel<1024, 4>, 1024);
+        return go(make_mask_kernel<1024, 8>, 1024);
+    }
     // few long rows: 16 waves per row; many rows: 4 waves per row and several rows per CU
-    if (p.Lk >= 8192 && n_rows < 2048) hipLaunchKernelGGL((make_mask_kernel<1024, 32>), dim3((unsigned)n_rows), dim3(1024), 0, stream, p);
-    else if (p.Lk >= 16384) hipLaunchKernelGGL((make_mask_kernel<256, 32>), dim3((unsigned)n_rows), dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((make_mask_kernel<256, 8>), dim3((unsigned)n_rows), dim3(256), 0, stream, p);
+    if (p.Lk >= 8192 && n_rows < 2048) hipLaunchKernelGGL((make_mask_memory_kernel<1024, 32>), dim3((unsigned)n_rows), dim3(1024), 0, stream, p);
+    else if (p.Lk >= 16384) hipLaunchKernelGGL((make_mask_memory_kernel<256, 32>), dim3((unsigned)n_rows), dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((make_mask_memory_kernel<256, 8>), dim3((unsigned)n_rows), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -563,12 +563,13 @@ PyObject *dyn_bias(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     // rows of the bias are handed to the attention kernels' 16-byte loads: a row pitch of whole vectors
     const int64_t lp = round_up(l, 8);
     Tensor bias = at::empty_strided({b, hk, 1, l}, {hk * lp, lp, lp, 1}, opt);
-    Tensor dt = at::empty({b * l, hk}, opt.dtype(at::kFloat));
+    Tensor dt;  // (read by the backward only)
+    if (is_grad) dt = at::empty({b * l, hk}, opt.dtype(at::kFloat));
     fdma_dyn_bias_args a{};
     a.value = v.data_ptr(); a.weight = w.data_ptr(); a.a = av.data_ptr();
     a.proj_bias = has_pb ? pb.data_ptr() : nullptr;
     a.bias = bias.data_ptr();
-    a.dt = (float *)dt.data_ptr();
+    a.dt = is_grad ? (float *)dt.data_ptr() : nullptr;
     strides3(v, a.value_strides);
     a.bias_strides[0] = hk * lp; a.bias_strides[1] = lp;
     a.batch = (int32_t)b; a.seqlen_k = (int32_t)l; a.num_heads_k = (int32_t)hk; a.head_dim = (int32_t)d;

@@ -309,7 +309,7 @@ size_t fdma_sizeof_mask_args(void);
  *   value, dvalue : (batch, seqlen_k, num_heads_k, head_dim), strides {batch, row, head} in elements
  *   weight, dweight : (num_heads_k, num_heads_k * head_dim), contiguous;  a, da, proj_bias, dproj_bias : (num_heads_k)
  *   bias, dbias   : (batch, num_heads_k, 1, >= seqlen_k), strides {batch, head} in elements, key dimension contiguous
- *   dt            : (batch * seqlen_k, num_heads_k) fp32, written by forward and read by backward
+ *   dt            : (batch * seqlen_k, num_heads_k) fp32, written by forward (NULL: not wanted) and read by backward
  * All tensors have the dtype given; num_heads_k <= 32, head_dim % 8 == 0, (num_heads_k * head_dim) % 16 == 0.
  * Backward needs fdma_dyn_bias_bwd_workspace_bytes() of scratch; its sums are folded in a fixed order (bit-reproducible).
  */
