@@ -585,8 +585,10 @@ template <typename T, int D>
 hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
     const FwdParams &f = p.f;
     hipError_t e;
-    // 1. D = rowsum(dO * O)  (the compacted backward has done it in its pre-pass launch)
-    if (!p.dot_done) {
+    // 1. D = rowsum(dO * O)  (the compacted backward has done it in its pre-pass launch; the column-mask form without
+    // compaction makes it in its dQ kernel, which then comes first)
+    const bool colmask = bwd_colmask_applicable(p), dq_first = colmask && !f.cmp.on;
+    if (!p.dot_done && !dq_first) {
         const int rpb = bwd_dot_rows_per_block(f.d);
         dim3 grid(((f.cu_q ? f.total_q : p.Lq_rounded) + rpb - 1) / rpb, f.H, f.cu_q ? 1 : f.B);
         hipLaunchKernelGGL((bwd_dot_kernel<T>), grid, dim3(256), 0, stream, p);
@@ -600,7 +602,7 @@ hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
     }
     // 2. dK, dV, dBias
     const int dtype_code = std::is_same<T, bf16_tag>::value ? 0 : 1;
-    const bool colmask = bwd_colmask_applicable(p);
+    if (dq_first && (e = launch_bwd_dq_colmask(p, dtype_code, stream)) != hipSuccess) return e;
     if (f.Lk > 0 && colmask) {
         if ((e = launch_bwd_dkdv_colmask(p, dtype_code, stream)) != hipSuccess) return e;
     } else if (f.Lk > 0) {
@@ -634,7 +636,7 @@ hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
     }
     // 3. dQ (the launch of a compacted backward also sums the dK / dV / dBias partial results of step 2)
     if (colmask) {
-        if ((e = launch_bwd_dq_colmask(p, dtype_code, stream)) != hipSuccess) return e;
+        if (!dq_first && (e = launch_bwd_dq_colmask(p, dtype_code, stream)) != hipSuccess) return e;
     } else if (f.Lk > 0 && bwd_dq_from_ds_applicable(p)) {
         // (step 2 has written dS itself as dBias: dQ = scale * dS K without a second pass over mask and bias)
         if ((e = launch_bwd_dq_from_ds(p, dtype_code, stream)) != hipSuccess) return e;

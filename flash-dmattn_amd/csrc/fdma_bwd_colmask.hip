@@ -846,7 +846,10 @@ template <int D, int BN> struct DqcSmem {
     static constexpr int TOTAL = OFF_BITS + MAX_TILES / 8;
 };
 
-template <typename T, int D, int BN, bool CAUSAL, bool CMP>
+// BARE: no compaction, no mask, no bias (ragged batches, plain attention): there is no bias column, and the K / V tiles can
+// go the direct way as with compacted keys (a column made from mask bytes and bias values would have to come through
+// registers, whose wait is a wait for every direct load in front of it).
+template <typename T, int D, int BN, bool CAUSAL, bool CMP, bool BARE>
 __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_kernel(const BwdParams p) {
     using E = Elem<T>;
     using SM = DqcSmem<D, BN>;
@@ -856,7 +859,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
     constexpr int MB = BN / 32;
     constexpr int KB = BN / 16;
     constexpr int CH = D / 8, RPP = NTHREADS / CH, K_IT = BN / RPP;
-    // DMA (compacted keys, rows of exactly 256 bytes): the K / V tiles and the fused bias column go from global memory
+    // DMA (rows of exactly 256 bytes): the K / V tiles and, with compacted keys, the fused bias column go from global memory
     // straight into LDS (global_load_lds: a wave writes 64 consecutive 16-byte or 4-byte pieces, so the swizzle of the
     // tile is applied to the GLOBAL address of each lane's piece), TWO tiles ahead, into a third stage: no staging
     // registers, no LDS stores, and a tile has a whole tile time more to arrive.  (Through registers, loaded between the
@@ -864,7 +867,9 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
     // shorter.)  The instruction is written in assembly: issued through the compiler's builtin, every later LDS read
     // waited for ALL direct loads in flight -- the compiler cannot tell which stage they fill -- and the loads of
     // the tile after the next one would be waited for at once.  The waits are placed by hand (publish()).
-    constexpr bool DMA = TL::SWZ && CMP;
+    static_assert(!(CMP && BARE), "compacted keys have a column");
+    constexpr bool DMA = TL::SWZ && (CMP || BARE), DMA_COL = DMA && CMP;
+    constexpr int SLOT = DMA ? 256 : 4 * BN;  // bytes of a bias column's slot
     constexpr int NST = SM::NST;
     static_assert(!DMA || (RPP == 16 && NTHREADS == 256), "the direct loads are laid out for 16 chunks per row and four waves");
 
@@ -1000,7 +1005,24 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
     float lse2 = INFINITY, dd = 0.f;
     if (qrow < LqS) {
         lse2 = f.lse[b * f.lse_b + h * f.lse_h + sq.q0 + qrow] * kLog2e;
-        dd = p.softmax_d[b * p.sd_b + h * p.sd_h + sq.q0 + qrow];
+        if (CMP) dd = p.softmax_d[b * p.sd_b + h * p.sd_h + sq.q0 + qrow];
+    }
+    if constexpr (!CMP) {
+        // D = rowsum(dO * O) is made here, from the dO fragments, and left for the dK/dV kernel, which is launched behind
+        // this one: a launch and a second read of dO less (52 us of 2.8 ms on 16384 ragged tokens x 32 heads).  (With
+        // compacted keys this launch also sums that kernel's partial results and comes second; D is a layer of the pre-pass.)
+        const uint16_t *op = (const uint16_t *)f.o + b * f.o_b + (sq.q0 + qrow_c) * f.o_r + h * f.o_h;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const int c = ks * 16 + g * 8;
+            const u32x4_t ov = *(const u32x4_t *)(op + (c < f.d ? c : 0));  // (dO is zero beyond d and beyond Lq)
+#pragma unroll
+            for (int e = 0; e < 4; e++) dd += E::lo(ov[e]) * E::lo(dof[ks][e]) + E::hi(ov[e]) * E::hi(dof[ks][e]);
+        }
+        dd = xhalf_sum(dd);
+        if (qrow >= LqS) dd = 0.f;
+        // (fixed lengths: padded rows are zero)
+        if (g == 0 && (qrow < LqS || (!f.cu_q && qrow < p.Lq_rounded))) p.softmax_d[b * p.sd_b + h * p.sd_h + sq.q0 + qrow] = dd;
     }
 
     f32x16_t dq[DB];
@@ -1049,7 +1071,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
         tb_k = uniform_ptr(kbase + (int64_t)j * BN * f.k_r);
         tb_v = uniform_ptr(vbase + (int64_t)j * BN * f.v_r);
         t_last = j == j_last;
-        if constexpr (DMA) {
+        if constexpr (DMA_COL) {
             // columns beyond the end of the kept keys read the last one (masked where the column is used)
             tb_b = uniform_ptr(fbrow);
             const int col = j * BN + (lane & 31);
@@ -1077,7 +1099,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
     auto dma4 = [](gptr_t base, uint32_t off, uint32_t dst) {
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(dst));
     };
-    constexpr int N_DMA = 2 * K_IT + 1;  // direct loads of a wave per tile
+    constexpr int N_DMA = 2 * K_IT + (DMA_COL ? 1 : 0);  // direct loads of a wave per tile
     int dma_stage = 0;                   // stage the tile being fetched goes to (DMA)
     auto load_item = [&](int n) {  // 0 .. K_IT-1: K rows, K_IT .. 2*K_IT-1: V rows, 2*K_IT: the bias column (DMA)
         if constexpr (DMA) {
@@ -1117,7 +1139,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
             } else if (bcol_ok && (!mrow || mraw)) {
                 v = brow ? E::lo(braw) * kLog2e : 0.f;
             }
-            lds_st32(lds0 + SM::OFF_BIAS + 4 * (slot * BN + tid), __float_as_uint(v));
+            lds_st32(lds0 + SM::OFF_BIAS + slot * SLOT + 4 * tid, __float_as_uint(v));
         }
     };
 
@@ -1160,7 +1182,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
         const int st = DMA ? i % 3 : (i & 1);
         const uint32_t st_off = (uint32_t)(st * SM::K_BYTES);  // (a multiple of 256: the swizzles stay XORs)
         const uint32_t a_cur = a_off + st_off, tr_cur = tr_off + st_off;
-        const uint32_t bs = lds0 + SM::OFF_BIAS + (DMA ? (i % 3) * 256 + 32 * g : 4 * ((i % 3) * BN + 8 * g));
+        const uint32_t bs = lds0 + SM::OFF_BIAS + (i % 3) * SLOT + 32 * g;
 
         // ---- S^T = K Q^T, dP^T = V dO^T, dS^T = P^T * (dP^T - D), dQ^T += K^T dS^T.  A wave issues in program
         // order, so the vector work has to sit BETWEEN the MFMAs to run under them; the tile is written slot by slot --
@@ -1180,8 +1202,8 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
 #pragma unroll
             for (int blk = 0; blk < 2; blk++) {
                 if (!S_EARLY || i == 0) {
-                    const f32x4_t b0 = __builtin_bit_cast(f32x4_t, lds_ld128(bs + 4 * (32 * mb + 16 * blk)));
-                    const f32x4_t b1 = __builtin_bit_cast(f32x4_t, lds_ld128(bs + 4 * (32 * mb + 16 * blk + 4)));
+                    const f32x4_t b0 = BARE ? f32x4_t{0.f, 0.f, 0.f, 0.f} : __builtin_bit_cast(f32x4_t, lds_ld128(bs + 4 * (32 * mb + 16 * blk)));
+                    const f32x4_t b1 = BARE ? b0 : __builtin_bit_cast(f32x4_t, lds_ld128(bs + 4 * (32 * mb + 16 * blk + 4)));
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         s[mb][8 * blk + e] = b0[e] - lse2;
@@ -1283,20 +1305,20 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
                 if constexpr (S_EARLY) {
                     // the next tile's bias column (slot (i + 1) % 3, complete since the last barrier): read in the slots
                     // of the first key block, used in those of the last
-                    const uint32_t bs_n = lds0 + SM::OFF_BIAS + (uint32_t)(((i + 1) % 3) * 256 + 32 * g);
+                    const uint32_t bs_n = lds0 + SM::OFF_BIAS + (uint32_t)(((i + 1) % 3) * SLOT + 32 * g);
                     // (this wave's own copy of that column was fetched a tile ago, in front of the N_DMA loads of the
                     // tile after it: wait for it alone -- vmcnt N_DMA, no wait for LDS reads or exports)
-                    if (kb == 0 && db == 0) __builtin_amdgcn_s_waitcnt(0x0F70 | N_DMA);
-                    if (kb == 0 && db < 4) nb[db] = __builtin_bit_cast(f32x4_t, lds_ld128(bs_n + 16 * (db & 1) + 64 * (db >> 1)));
+                    if (DMA_COL && kb == 0 && db == 0) __builtin_amdgcn_s_waitcnt(0x0F70 | N_DMA);
+                    if (DMA_COL && kb == 0 && db < 4) nb[db] = __builtin_bit_cast(f32x4_t, lds_ld128(bs_n + 16 * (db & 1) + 64 * (db >> 1)));
                     if (kb == KB - 1 && db < 4) {
 #pragma unroll
-                        for (int e = 0; e < 4; e++) s[0][4 * db + e] = nb[db][e] - lse2;
+                        for (int e = 0; e < 4; e++) s[0][4 * db + e] = DMA_COL ? nb[db][e] - lse2 : -lse2;
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (jn < n_end) store_tile((i + 1) & 1, (i + 1) % 3);
+        if (!DMA && jn < n_end) store_tile((i + 1) & 1, (i + 1) % 3);
         publish();
         i++;
         jc = jn;
@@ -1331,10 +1353,13 @@ template <typename T, int D, bool CAUSAL>
 hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
     const FwdParams &f = p.f;
     constexpr int BN = D > 64 ? 32 : 64;  // at d = 128 a 64-key tile would spill registers
-    auto kern = p.f.cmp.on ? bwd_dq_colmask_kernel<T, D, BN, CAUSAL, true> : bwd_dq_colmask_kernel<T, D, BN, CAUSAL, false>;
+    constexpr bool SWZ = LdsTile<D>::SWZ;
+    const int which = f.cmp.on ? 1 : (SWZ && !f.mask && !f.bias ? 2 : 0);
+    auto kern = which == 1 ? bwd_dq_colmask_kernel<T, D, BN, CAUSAL, true, false>
+                           : (which == 2 ? bwd_dq_colmask_kernel<T, D, BN, CAUSAL, false, SWZ> : bwd_dq_colmask_kernel<T, D, BN, CAUSAL, false, false>);
     const int smem = DqcSmem<D, BN>::TOTAL;
-    static DynSmemLimit smem_limit[2];  // one per instantiation: the limit is a property of the kernel
-    hipError_t e = smem_limit[p.f.cmp.on ? 1 : 0].ensure((const void *)kern, (int)smem);
+    static DynSmemLimit smem_limit[3];  // one per instantiation: the limit is a property of the kernel
+    hipError_t e = smem_limit[which].ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
     const int n_dq = xcd_grid(f.B * f.Hk, (f.Lq + Q_BM - 1) / Q_BM, f.H / f.Hk);  // a multiple of 8
     if (p.f.cmp.on) {

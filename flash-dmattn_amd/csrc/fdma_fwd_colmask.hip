@@ -38,6 +38,11 @@
 // rows per workgroup) four waves stage V and four K and the side rows; one barrier per tile.  Global loads are one
 // instruction each (scalar tile base + a loop-invariant per-thread offset) and sit a whole tile in front of their
 // LDS stores.  Workgroup ids are remapped so that the workgroups sharing one XCD's L2 also share K / V.
+//   Key groups (KG = 2).  A grid of no more 128-row workgroups than CUs leaves a CU with one wave per SIMD, which does not
+// overlap its vector work, its LDS reads and its barriers with its MFMAs (1.4 us per tile of 0.5 us matrix work).  Then a
+// workgroup is two groups of four waves over the SAME query rows, each with its own stages: they take the active tiles in
+// turn, with a softmax of their own, and are merged through LDS at the end.  512 rows x 32 heads against 2048 kept keys,
+// d = 128: 44 us, now @@@.
 #include <type_traits>
 
 #include "fdma_common.h"
@@ -66,9 +71,10 @@ template <int D, int BN> struct CmSmem {
 // CMP: K / V are the compacted copies of the kept columns (see fdma_compact.hip).  The key axis then has
 // `count` columns, all kept; the fused bias vector comes pre-gathered, and the causal limit of a query row
 // is the number of kept columns at or below its diagonal instead of the column index itself.
-template <typename T, int D, int BN, bool CAUSAL, int NW, bool CMP>
-__global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_colmask_kernel(const FwdParams p) {
-    constexpr int NTHREADS = 64 * NW;
+template <typename T, int D, int BN, bool CAUSAL, int NW, bool CMP, int KG>
+__global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1) ? 2 : 1) fwd_colmask_kernel(const FwdParams p) {
+    constexpr int NTHREADS = 64 * NW;         // of a key group
+    static_assert(KG == 1 || NW == 4, "key groups are for small grids, which have 128-row workgroups");
     constexpr int STHREADS = 256;             // threads staging one operand
     constexpr bool SPLIT = NW == 8;           // 8 waves: the first four stage V, the last four K and the side rows
     static_assert(NW == 4 || NW == 8, "staging maps are written for 256 or 512 threads");
@@ -89,11 +95,13 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
     static_assert(!SPLIT || V_IT == 1, "the role split assumes one V item per thread");
     static_assert(!SPLIT || K_IT == 4, "the role split assumes four loads per thread for either operand");
 
-    extern __shared__ __attribute__((aligned(16))) char smem[];
+    extern __shared__ __attribute__((aligned(16))) char smem_all[];
+    const int kgrp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NTHREADS);  // key group of this wave
+    char *const smem = smem_all + kgrp * SM::TOTAL;
     uint32_t *sBits = (uint32_t *)(smem + SM::OFF_BITS);
-    uint32_t *sFlag = (uint32_t *)(smem + SM::OFF_FLAG);
+    uint32_t *sFlag = (uint32_t *)(smem_all + SM::OFF_FLAG);  // (one for all: the groups leave the common path together)
 
-    const int tid = threadIdx.x;
+    const int tid = (int)threadIdx.x - kgrp * NTHREADS;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (tells the compiler that it is wave-uniform)
     const int lane = tid & 63;
     const int r = lane & 31;
@@ -229,6 +237,19 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
         it_word &= it_word - 1;
         return j < n_end ? j : n_end;
     };
+    // The tiles in turns of KG: `lead` is the first of a turn (what ends the loops, alike for all groups), `mine` this
+    // group's -- n_end when the last turn has none left for it: its keys then count as masked, and the tile that is fetched
+    // in its place (any existing one) is not looked at.
+    struct Turn { int lead, mine; };
+    auto next_turn = [&]() -> Turn {
+        Turn t;
+        t.lead = t.mine = next_tile();
+        if (KG == 2) {
+            const int second = next_tile();
+            if (kgrp == 1) t.mine = second;
+        }
+        return t;
+    };
 
     f32x16_t o[DB];
     float row_sum = 0.f;
@@ -279,18 +300,19 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
         return (gptr_t)(((uint64_t)hi << 32) | lo);
     };
     // next fetches: K and the side-row inputs of tile jk / V of tile jv (with split roles a wave has one of the two)
-    auto set_tile_k = [&](int jk) {
+    auto set_tile_k = [&](Turn tk) {
         if (!role_k) return;
+        const int jk = KG == 1 || tk.mine < n_end ? tk.mine : tk.lead;
         tb_k = uniform_ptr((const char *)kbase + (int64_t)jk * BN * p.k_r * 2);
         last_k = jk == j_last;
     };
     // side-row inputs of this thread's column of tile jx: only the raw loads here -- the values are looked at when
     // the row is stored
-    auto set_tile_x = [&](int jx) {
+    auto set_tile_x = [&](Turn tx) {
         if (!role_x) return;
-        const int col = jx * BN + lane;
-        const int cc = col < Lk ? col : 0;
-        bcol_ok = col < Lk;
+        const int col = tx.mine * BN + lane;
+        bcol_ok = col < Lk && (KG == 1 || tx.mine < n_end);
+        const int cc = bcol_ok ? col : 0;
         // (unconditional loads: a load in one arm of a select would have to be waited for right here)
         if (CMP) {
             braw = __float_as_uint(fbrow[cc]);
@@ -299,8 +321,9 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
             braw = brow_ld[cc];
         }
     };
-    auto set_tile_v = [&](int jv) {
+    auto set_tile_v = [&](Turn tv) {
         if (!role_v) return;
+        const int jv = KG == 1 || tv.mine < n_end ? tv.mine : tv.lead;
         tb_v = uniform_ptr((const char *)vbase + (int64_t)jv * BN * p.v_r * 2);
         last_v = jv == j_last;
     };
@@ -473,7 +496,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
     // in front of the MFMAs, left the matrix pipe to the SIMD's other wave alone for a fifth of every tile.  Half tiles
     // on the causal diagonal are masked before the step, in code of their own: only they pay for it.)
     auto step = [&](auto stage_c, auto do_v_c, auto do_k_c, f32x16_t &scur, f32x16_t &snext, uint32_t (&pcur)[8],
-                    const uint32_t (&pprev)[8], int kbuf, int kh, int vbuf, int vh, int j_next, int jx_next) {
+                    const uint32_t (&pprev)[8], int kbuf, int kh, int vbuf, int vh, Turn j_next, Turn jx_next) {
         constexpr bool STAGE = decltype(stage_c)::value;
         constexpr bool DO_V = STAGE && decltype(do_v_c)::value, DO_K = !STAGE && decltype(do_k_c)::value;
         char *const sVt_w = smem + SM::OFF_VT + (vbuf ^ 1) * SM::VT_BYTES;  // V(t) goes to the stage the P V product has left
@@ -559,14 +582,15 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
         if (__any(!(psum <= 16384.f))) *sFlag = 1u;
     };
 
-    const int j0 = next_tile();
+    const Turn j0 = next_turn();
     bool redo = false;
-    if (j0 < n_end) {
+    if (j0.lead < n_end) {
         // ---- common path.  Set-up: the first tile is staged, its scores are computed once just for their row maxima,
         // and the reference point of every row is put kRefMargin above its maximum: probabilities start around
         // 2^-margin, and the rest of the row may exceed the first tile by margin + 14 before the check fails.
-        int jc = j0, jn1 = next_tile(), jn2 = next_tile(), jn3 = next_tile();
-        if (tid == 0) *sFlag = 0u;
+        Turn jc = j0, jn1 = next_turn(), jn2 = next_turn(), jn3 = next_turn();
+        auto or_else = [&](Turn t, Turn e) -> Turn { return t.lead < n_end ? t : e; };
+        if (threadIdx.x == 0) *sFlag = 0u;
         // K(0), K(1) and the side rows of tile 0 go to LDS; the registers then fetch K(2), V(0) (kept until step A)
         // and the side-row inputs of tile 1
         set_tile_k(j0);
@@ -575,7 +599,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
         load_regs(false);
         load_regs(true);
         u32x4_t k1[K_IT];  // K(1) travels in registers of its own, together with K(0)
-        set_tile_k(jn1 < n_end ? jn1 : j0);
+        set_tile_k(or_else(jn1, j0));
         if (role_k) {
 #pragma unroll
             for (int it = 0; it < K_IT; it++)
@@ -583,13 +607,13 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
         }
         store_k(0);
         store_x(0);
-        set_tile_x(jn1 < n_end ? jn1 : j0);
+        set_tile_x(or_else(jn1, j0));
         if (role_k) {
 #pragma unroll
             for (int it = 0; it < K_IT; it++) sreg[it] = k1[it];
         }
         store_k(1);
-        set_tile_k(jn2 < n_end ? jn2 : j0);
+        set_tile_k(or_else(jn2, j0));
         load_regs(false);
         // Q is scaled by softmax_scale * log2(e) once, here (the reference also rounds the scaled Q to the input type,
         // flash_fwd_kernel.h:428-439): the MFMAs then produce exp2-domain scores directly
@@ -610,7 +634,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
         {
             scores_half(sA, 0, 0);
             scores_half(sB, 0, 1);
-            const int col0 = j0 * BN;
+            const int col0 = j0.mine * BN;
             if (CAUSAL && col0 + 32 > vis_wave) causal_mask(sA, col0);
             if (CAUSAL && col0 + 64 > vis_wave) causal_mask(sB, col0 + 32);
             float tmax = -INFINITY;
@@ -651,20 +675,20 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
         auto tile_loop = [&](auto do_v_c, auto do_k_c) {
             while (true) {
                 const int kb = t & 1;
-                const int col0 = jc * BN;
+                const int col0 = jc.mine * BN;
                 if (CAUSAL && col0 + 32 > vis_wave) causal_mask(sA, col0);
                 __builtin_amdgcn_sched_barrier(0);
-                step(yes, do_v_c, do_k_c, sA, sB, pA, pB, kb, 1, kb ^ 1, 1, jn1 < n_end ? jn1 : jc, jn2 < n_end ? jn2 : jc);
+                step(yes, do_v_c, do_k_c, sA, sB, pA, pB, kb, 1, kb ^ 1, 1, or_else(jn1, jc), or_else(jn2, jc));
                 __builtin_amdgcn_sched_barrier(0);
                 __syncthreads();
                 __builtin_amdgcn_sched_barrier(0);
                 if (CAUSAL && col0 + 64 > vis_wave) causal_mask(sB, col0 + 32);
-                step(no, do_v_c, do_k_c, sB, sA, pB, pA, kb ^ 1, 0, kb, 0, jn3 < n_end ? jn3 : jc, 0);
+                step(no, do_v_c, do_k_c, sB, sA, pB, pA, kb ^ 1, 0, kb, 0, or_else(jn3, jc), jc);
                 __builtin_amdgcn_sched_barrier(0);
                 t++;
                 jc = jn1; jn1 = jn2; jn2 = jn3;
-                if (jc >= n_end) break;
-                jn3 = next_tile();
+                if (jc.lead >= n_end) break;
+                jn3 = next_turn();
             }
         };
         const bool do_v = __builtin_amdgcn_readfirstlane((int)(role_v && kt < V_ITEMS)) != 0;
@@ -692,7 +716,7 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
         it_word = 0;
         it_base = -32;
         it_next = 0;
-        for (int j = next_tile(); j < n_end; j = next_tile()) {
+        for (Turn j = next_turn(); j.lead < n_end; j = next_turn()) {
             set_tile_k(j);
             set_tile_v(j);
             set_tile_x(j);
@@ -708,12 +732,12 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
             scores_half(s0, 0, 0);
             scores_half(s1, 0, 1);  // (both against the same pieces: classic() below may replace them)
             const float enc_before = enc_ref;
-            classic(s0, p0, j * BN);
+            classic(s0, p0, j.mine * BN);
             pv_half(p0, 0, 0);  // (before the second half may move the reference and rescale O again)
             const float fix = enc_before - enc_ref;
 #pragma unroll
             for (int i = 0; i < 16; i++) s1[i] += fix;
-            classic(s1, p1, j * BN + 32);
+            classic(s1, p1, j.mine * BN + 32);
             pv_half(p1, 0, 1);
         }
     }
@@ -721,7 +745,36 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
     // ---- epilogue
     {
         const int qrow = wrow0 + r;
-        const float total = xhalf_sum(row_sum);
+        float total = xhalf_sum(row_sum);
+        if constexpr (KG == 2) {
+            // the second group hands over its sums, its reference points and O; the first merges and stores
+            float *xs = (float *)smem_all + wave * 64 + lane;  // sum, reference: 2 * NW * 64 floats
+            f32x4_t *xo = (f32x4_t *)(smem_all + 2 * NW * 256) + wave * DB * 4 * 64 + lane;
+            static_assert(2 * NW * 256 + NW * DB * 4 * 64 * 16 <= SM::OFF_BITS, "the hand-over fits the first group's stages");
+            __syncthreads();  // (the stages' last reads)
+            if (kgrp == 1) {
+                xs[0] = total;
+                xs[NW * 64] = row_ref;
+#pragma unroll
+                for (int db = 0; db < DB; db++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) xo[(db * 4 + q) * 64] = f32x4_t{o[db][4 * q], o[db][4 * q + 1], o[db][4 * q + 2], o[db][4 * q + 3]};
+            }
+            __syncthreads();
+            if (kgrp == 1) return;
+            const float t1 = xs[0], r1 = xs[NW * 64], top = fmaxf(row_ref, r1), safe = top == -INFINITY ? 0.f : top;
+            const float w0 = fast_exp2(row_ref - safe), w1 = fast_exp2(r1 - safe);
+            total = total * w0 + t1 * w1;
+            row_ref = top;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const f32x4_t v = xo[(db * 4 + q) * 64];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[db][4 * q + e] = o[db][4 * q + e] * w0 + v[e] * w1;
+                }
+        }
         const float inv = total > 0.f ? 1.f / total : 0.f;
         if (qrow < LqS) {
             uint16_t *op = (uint16_t *)p.o + b * p.o_b + (sq.q0 + qrow) * p.o_r + h * p.o_h;
@@ -746,11 +799,11 @@ __global__ void __launch_bounds__(64 * NW, (NW == 4 && D <= 128) ? 2 : 1) fwd_co
     }
 }
 
-template <typename T, int D, int BN, bool CAUSAL, bool CMP, int NW = 4>
+template <typename T, int D, int BN, bool CAUSAL, bool CMP, int NW = 4, int KG = 1>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     constexpr int BM = 32 * NW;
-    auto kern = fwd_colmask_kernel<T, D, BN, CAUSAL, NW, CMP>;
-    const int smem = CmSmem<D, BN>::TOTAL;
+    auto kern = fwd_colmask_kernel<T, D, BN, CAUSAL, NW, CMP, KG>;
+    const int smem = KG * CmSmem<D, BN>::TOTAL;
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
@@ -758,7 +811,7 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
     const int k_split = 8 / gcd8;
     dim3 grid(pairs * k_split * ((n_mb + k_split - 1) / k_split) * G);
-    hipLaunchKernelGGL(kern, grid, dim3(64 * NW), smem, stream, p);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * NW * KG), smem, stream, p);
     return hipGetLastError();
 }
 
@@ -770,6 +823,12 @@ hipError_t launch_d(const FwdParams &p, hipStream_t stream) {
     if constexpr (D == 128) if (groups256 >= 512) {
         if (p.cmp.on) return p.causal ? launch_one<T, D, 64, true, true, 8>(p, stream) : launch_one<T, D, 64, false, true, 8>(p, stream);
         return p.causal ? launch_one<T, D, 64, true, false, 8>(p, stream) : launch_one<T, D, 64, false, false, 8>(p, stream);
+    }
+    // no more 128-row workgroups than CUs: two key groups each (a row that sees a single tile gains nothing, and pays
+    // a merge of a microsecond)
+    if constexpr (D <= 128) if ((int64_t)p.B * p.H * ((p.Lq + 127) / 128) <= device_cus() && p.Lk > 128) {
+        if (p.cmp.on) return p.causal ? launch_one<T, D, 64, true, true, 4, 2>(p, stream) : launch_one<T, D, 64, false, true, 4, 2>(p, stream);
+        return p.causal ? launch_one<T, D, 64, true, false, 4, 2>(p, stream) : launch_one<T, D, 64, false, false, 4, 2>(p, stream);
     }
     if (p.cmp.on) return p.causal ? launch_one<T, D, 64, true, true>(p, stream) : launch_one<T, D, 64, false, true>(p, stream);
     return p.causal ? launch_one<T, D, 64, true, false>(p, stream) : launch_one<T, D, 64, false, false>(p, stream);
