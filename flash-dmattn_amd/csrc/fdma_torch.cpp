@@ -15,6 +15,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/TracerMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -61,9 +62,9 @@ inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 // ---- arguments -----------------------------------------------------------------------------------------------------
 
-// Nothing but the device would see a call on plain tensors right now.
+// Nothing but the device would see a call on plain tensors right now (torch.jit.trace would: it records operators).
 bool plain_state() {
-    return c10::impl::TorchDispatchModeTLS::stack_len() == 0 && at::impl::PythonTorchFunctionTLS::stack_len() == 0;
+    return !at::tracer::impl::is_dispatch_enabled() && c10::impl::TorchDispatchModeTLS::stack_len() == 0 && at::impl::PythonTorchFunctionTLS::stack_len() == 0;
 }
 
 // An ordinary torch.Tensor on `dev` (any GPU while dev is negative): not a subclass, not wrapped by functorch or
@@ -99,8 +100,12 @@ void bcast3(const Tensor &t, int64_t *s) {
 
 void *stream_of(int dev) { return c10::hip::getCurrentHIPStream((c10::DeviceIndex)dev).stream(); }
 
-// None: `def`; a bool, number or anything with a truth value otherwise.
-int truth(PyObject *o, int def) { return o == Py_None ? def : PyObject_IsTrue(o); }
+// None: 0; otherwise whether the object is true, -1 (and no exception) where it has no truth value.
+int truth(PyObject *o) {
+    const int t = o == Py_None ? 0 : PyObject_IsTrue(o);
+    if (t < 0) PyErr_Clear();
+    return t;
+}
 
 bool same_shape(const Tensor &t, PyObject *tup) {
     if (!PyTuple_Check(tup) || PyTuple_GET_SIZE(tup) != t.dim()) return false;
@@ -275,8 +280,7 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (!plain_state()) Py_RETURN_NOTIMPLEMENTED;
     for (int i = 0; i < 5; i++)
         if (!(i >= 3 && args[i] == Py_None) && !plain_tensor(args[i], dev)) Py_RETURN_NOTIMPLEMENTED;
-    if (args[7] != Py_None && truth(args[7], 0) != 0) Py_RETURN_NOTIMPLEMENTED;  // softcap
-    if (truth(args[9], 0) != 0) Py_RETURN_NOTIMPLEMENTED;                        // LSE wanted
+    if (truth(args[7]) != 0 || truth(args[9]) != 0 || truth(args[6]) < 0 || truth(args[8]) < 0) Py_RETURN_NOTIMPLEMENTED;  // softcap, LSE wanted
     const Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]);
     const Tensor mask = args[3] == Py_None ? Tensor() : THPVariable_Unpack(args[3]);
     const Tensor bias = args[4] == Py_None ? Tensor() : THPVariable_Unpack(args[4]);
@@ -305,7 +309,7 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         if (mask.size(1) == H && H != Hk) Py_RETURN_NOTIMPLEMENTED;
         if (mask.size(2) != 1 && compact_mode == FDMA_COMPACT_ALWAYS) Py_RETURN_NOTIMPLEMENTED;
     }
-    const bool deterministic = truth(args[8], 0) != 0;
+    const bool deterministic = truth(args[8]) > 0;
     if (deterministic && bias.defined() && ((bias.size(0) == 1 && B > 1) || (bias.size(1) == 1 && Hk > 1))) Py_RETURN_NOTIMPLEMENTED;
     const bool record = at::GradMode::is_enabled();
     const bool is_grad = record && (q.requires_grad() || k.requires_grad() || v.requires_grad());
@@ -319,7 +323,7 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             Py_RETURN_NOTIMPLEMENTED;
         }
     }
-    const bool causal = truth(args[6], 0) != 0;
+    const bool causal = truth(args[6]) > 0;
     SideInputs side;
     if (mask.defined()) side_inputs(args[3], mask, Lk, side);
 
@@ -433,8 +437,7 @@ PyObject *varlen_attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) 
     if (!plain_state()) Py_RETURN_NOTIMPLEMENTED;
     for (int i = 0; i < 5; i++)
         if (!plain_tensor(args[i], dev)) Py_RETURN_NOTIMPLEMENTED;
-    if (args[9] != Py_None && truth(args[9], 0) != 0) Py_RETURN_NOTIMPLEMENTED;
-    if (truth(args[11], 0) != 0 || args[12] != Py_None) Py_RETURN_NOTIMPLEMENTED;
+    if (truth(args[9]) != 0 || truth(args[11]) != 0 || args[12] != Py_None || truth(args[8]) < 0 || truth(args[10]) < 0) Py_RETURN_NOTIMPLEMENTED;
     const Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]);
     const Tensor &cu_q = THPVariable_Unpack(args[3]), &cu_k = THPVariable_Unpack(args[4]);
     if (!half_type(q) || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() || q.dim() != 3 || k.dim() != 3 ||
@@ -455,7 +458,7 @@ PyObject *varlen_attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) 
             Py_RETURN_NOTIMPLEMENTED;
         }
     }
-    const bool causal = truth(args[8], 0) != 0;
+    const bool causal = truth(args[8]) > 0;
     const bool is_grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
     std::shared_ptr<VarlenBackward> node;
     if (is_grad) {
@@ -478,7 +481,7 @@ PyObject *varlen_attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) 
         node->out_ = SavedVariable(out, true);
         node->lse = lse;
         node->max_q = max_q; node->max_k = max_k;
-        node->scale = scale; node->causal = causal; node->deterministic = truth(args[10], 0) != 0;
+        node->scale = scale; node->causal = causal; node->deterministic = truth(args[10]) > 0;
     }
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS

@@ -21,6 +21,44 @@ def test_declines_what_is_not_an_ordinary_device_tensor():
     assert _host().attention("q", q, q, None, None, None, None, None, None, None, 0) is NotImplemented
 
 
+class _NoTruth:
+    def __bool__(self):
+        raise ValueError("no truth value")
+
+
+@pytest.mark.gpu
+def test_declines_flags_without_a_truth_value():
+    q, k, v, mask, bias, _ = _inputs(1, 64, 64, 2, 1, 64, 1, torch.bfloat16)
+    cu = torch.tensor([0, 64], dtype=torch.int32, device=DEV)
+    for at in (6, 7, 8, 9):
+        args = [q, k, v, mask, bias, None, None, None, None, None, 0]
+        args[at] = _NoTruth()
+        assert _host().attention(*args) is NotImplemented
+    for at in (8, 9, 10, 11):
+        args = [q[0], k[0], v[0], cu, cu, 64, 64, None, None, None, None, None, None]
+        args[at] = _NoTruth()
+        assert _host().varlen_attention(*args) is NotImplemented
+
+
+@pytest.mark.gpu
+def test_declines_while_a_trace_records_operators():
+    """torch.jit.trace sees operators of the dispatcher, not launches: a call made here would be recorded as a constant."""
+    q, k, v, mask, bias, _ = _inputs(1, 64, 64, 2, 1, 64, 1, torch.bfloat16)
+    seen = []
+
+    def f(x):
+        seen.append(_host().attention(x, k, v, mask, bias, None, None, None, None, None, 0) is NotImplemented)
+        seen.append(_host().dyn_bias(v, torch.zeros(1, 64, dtype=x.dtype, device=DEV), bias[0, 0, 0, :1], None) is NotImplemented)
+        seen.append(_host().create_mask(bias, None, 8, -1.0, None, 0) is NotImplemented)
+        return x + 1
+
+    torch.jit.trace(f, (q,), check_trace=False)
+    assert seen and all(seen)
+    seen.clear()
+    f(q)
+    assert seen == [False, False, False]
+
+
 def _inputs(B, Lq, Lk, H, Hk, d, rows, dtype, seed=0):
     g = torch.Generator(device=DEV).manual_seed(seed)
     def randn(*s): return torch.randn(*s, generator=g, device=DEV).to(dtype)
