@@ -26,14 +26,16 @@ namespace {
 constexpr int NTHREADS = 256;
 
 // XCD-aware work distribution shared by both kernels: `pairs` independent (batch, kv head) pairs with
-// `n_units` units of work each (heaviest first); see the forward column-mask kernel for the rationale.
+// `n_units` units of work each (heaviest first), `k_split` lists of units per pair; see the forward column-mask kernel for the rationale.
 struct XcdMap {
     int pair, unit;
     bool valid;
 };
-__device__ __forceinline__ XcdMap xcd_map(int lid, int pairs, int n_units, int per_unit) {
+__host__ __device__ __forceinline__ int xcd_lists_per_pair(int pairs) {
     const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
-    const int k_split = 8 / gcd8;
+    return 8 / gcd8;
+}
+__device__ __forceinline__ XcdMap xcd_map(int lid, int k_split, int n_units, int per_unit) {
     const int list_len = ((n_units + k_split - 1) / k_split) * per_unit;
     const int xcd = lid % 8, slot = lid / 8;
     const int vlist = xcd + 8 * (slot / list_len);
@@ -44,9 +46,7 @@ __device__ __forceinline__ XcdMap xcd_map(int lid, int pairs, int n_units, int p
     m.valid = m.unit < n_units;
     return m;
 }
-inline int xcd_grid(int pairs, int n_units, int per_unit) {
-    const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
-    const int k_split = 8 / gcd8;
+inline int xcd_grid(int pairs, int k_split, int n_units, int per_unit) {
     return pairs * k_split * ((n_units + k_split - 1) / k_split) * per_unit;
 }
 
@@ -68,6 +68,10 @@ template <int D> struct KvcSmem {
     static constexpr int OFF_V = 2 * STAGE;
     static constexpr int TOTAL = OFF_V + (V_LDS ? KV_BN * S * 2 : 0);
 };
+
+// Entries of a ragged batch longest first and dealt to all XCDs (fdma_params.h), up to head dim 128: the instantiations
+// at 256 are at the end of their registers (772 bytes of scratch per lane) and keep the plain order.
+template <int D> constexpr bool RAGGED_TURNS = D <= 128;
 
 // CMP: the key axis is the compacted list of kept columns (fdma_compact.hip); a lane still owns one key,
 // reads it from the dense copies, and writes its gradients to the key's original row / column.
@@ -139,10 +143,12 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
         if (per > 1) slot = unit * per + sub;
     } else {
         const int n_nb = (f.Lk + KV_BN - 1) / KV_BN;
-        const XcdMap wm = xcd_map(blockIdx.x, f.B * f.Hk, n_nb, 1);
+        const bool ragged = RAGGED_TURNS<D> && f.cu_q;
+        const XcdMap wm = xcd_map(blockIdx.x, ragged ? ragged_lists_per_pair(f) : xcd_lists_per_pair(f.B * f.Hk), n_nb, 1);
         if (!wm.valid) return;
         n_block = wm.unit;  // low key blocks are seen by the most queries under causal: heaviest first
         pair = wm.pair;
+        if (ragged) pair = ragged_turn(f, pair / f.Hk) * f.Hk + pair % f.Hk;
     }
     const int b = pair / f.Hk, hk = pair % f.Hk;
     const int n0 = n_block * KV_BN;
@@ -818,7 +824,8 @@ hipError_t launch_dkdv_c(const BwdParams &p, hipStream_t stream) {
         hipLaunchKernelGGL(kern, dim3(grid), dim3(NTHREADS), smem, stream, p);
         return hipGetLastError();  // (the partial results are summed by workgroups of the dQ launch)
     }
-    dim3 grid(xcd_grid(f.B * f.Hk, (f.Lk + KV_BN - 1) / KV_BN, 1));
+    const int lists = RAGGED_TURNS<D> && f.cu_q ? ragged_lists_per_pair(f) : xcd_lists_per_pair(f.B * f.Hk);
+    dim3 grid(xcd_grid(f.B * f.Hk, lists, (f.Lk + KV_BN - 1) / KV_BN, 1));
     hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
     return hipGetLastError();
 }
@@ -903,7 +910,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dq_colmask_ker
         }
         lid = o * 8 + (lid & 7);
     }
-    const XcdMap wm = xcd_map(lid, f.B * f.Hk, n_mb, G);
+    const XcdMap wm = xcd_map(lid, xcd_lists_per_pair(f.B * f.Hk), n_mb, G);
     if (!wm.valid) return;
     const int m_block = n_mb - 1 - wm.unit;  // heaviest first under causal
     const int b = wm.pair / f.Hk, hk = wm.pair % f.Hk;
@@ -1361,7 +1368,7 @@ hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
     static DynSmemLimit smem_limit[3];  // one per instantiation: the limit is a property of the kernel
     hipError_t e = smem_limit[which].ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
-    const int n_dq = xcd_grid(f.B * f.Hk, (f.Lq + Q_BM - 1) / Q_BM, f.H / f.Hk);  // a multiple of 8
+    const int n_dq = xcd_grid(f.B * f.Hk, xcd_lists_per_pair(f.B * f.Hk), (f.Lq + Q_BM - 1) / Q_BM, f.H / f.Hk);  // a multiple of 8
     if (p.f.cmp.on) {
         const int units_max = f.B * f.Hk * ((f.Lk + KV_BN - 1) / KV_BN);
         const RedInterleave ri = red_interleave(n_dq / 8, units_max * (D / 16));

@@ -145,6 +145,19 @@ def test_varlen_large_grid_d128(causal):
     _run(lens, lens, 16, 4, 128, causal, seed=6)
 
 
+@pytest.mark.parametrize("lens,H,Hk", [
+    ([130, 64, 130, 1, 64, 300, 7, 130], 2, 1),              # equal lengths, one kv head: every entry on all XCDs
+    ([5 + (37 * i) % 60 for i in range(64)], 2, 2),          # as many entries as a wave has lanes: longest first
+    ([5 + (37 * i) % 60 for i in range(65)], 4, 2),          # one more: in their order
+    ([64, 300, 0, 129], 6, 3),                               # kv heads that do not divide the XCDs, an empty entry
+])
+@pytest.mark.parametrize("D", [64, 128])
+def test_varlen_order_of_entries(lens, H, Hk, D):
+    """The dK/dV kernel takes the entries longest first and deals each to all XCDs: every block of every entry once."""
+    _run(lens, lens, H, Hk, D, True, seed=len(lens))
+    _run(lens, lens[::-1], H, Hk, D, False, seed=len(lens) + 1)
+
+
 def test_varlen_rejects_unsupported_arguments():
     f = _op()
     q, k, v, _ = _make([64], [64], 2, 2, 64, torch.bfloat16, 0)
