@@ -280,18 +280,29 @@ size_t fdma_fwd_counter_bytes(const fdma_fwd_args *a) {
     return (size_t)round_up(fdma::decode_num_counters(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k) * 4, 256);
 }
 
-size_t fdma_fwd_workspace_bytes(const fdma_fwd_args *a) {
+// scratch of a forward call: what it cannot do without, and -- `shares` -- room for the shares of split keys behind it
+static size_t fwd_scratch_bytes(const fdma_fwd_args *a, size_t *shares) {
+    *shares = 0;
     if (!a) return 0;
     if (!fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k)) {
         fdma::FwdParams p, pv;
         fill_fwd_params(a, p);
-        if (fdma::compact_per_query_head(p, pv)) return fdma::compact_bytes(pv, false);
-        return fdma::use_compact(p) ? fdma::compact_bytes(p, false) : 0;
+        if (fdma::compact_per_query_head(p, pv)) p = pv;
+        else if (!fdma::use_compact(p)) return 0;
+        const int splits = fdma::fwd_key_splits(p);
+        if (splits > 1) *shares = (size_t)splits * a->batch * a->num_heads * a->seqlen_q * (size_t)(a->head_dim + 1) * sizeof(float);
+        return (size_t)round_up(fdma::compact_bytes(p, false), 256);
     }
     const int splits = fdma::decode_num_splits(a->batch, a->num_heads_k, a->seqlen_k);
     if (splits <= 1) return 0;
     const size_t rows = (size_t)splits * a->batch * a->num_heads * a->seqlen_q;
     return rows * (size_t)(a->head_dim + 1) * sizeof(float);
+}
+
+size_t fdma_fwd_workspace_bytes(const fdma_fwd_args *a) {
+    size_t shares;
+    const size_t need = fwd_scratch_bytes(a, &shares);
+    return need + shares;
 }
 
 int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
@@ -332,8 +343,17 @@ int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
             const size_t need = fdma::compact_bytes(p, false);
             if (!a->workspace || a->workspace_bytes < need)
                 return fail(FDMA_ERR_WORKSPACE, "forward workspace too small: need %zu bytes, got %zu", need, a->workspace_bytes);
+            // (where the workspace holds the compacted copies but not the shares, the keys stay whole)
+            const int splits = fdma::fwd_key_splits(p);
+            size_t shares;
+            const size_t base = fwd_scratch_bytes(a, &shares);
             if ((e = fdma::compact_setup(p, a->workspace, a->dtype, stream)) != hipSuccess)
                 return fail(FDMA_ERR_LAUNCH, "forward launch failed: %s", hipGetErrorString(e));
+            if (splits > 1 && a->workspace_bytes >= base + shares) {
+                p.splits = splits;
+                p.o_part = reinterpret_cast<float *>(static_cast<char *>(a->workspace) + base);
+                p.lse_part = p.o_part + (size_t)splits * a->batch * a->num_heads * a->seqlen_q * a->head_dim;
+            }
         }
         e = fdma::launch_fwd(p, a->dtype, stream);
     }
@@ -345,7 +365,8 @@ int fdma_fwd_noalloc(const fdma_fwd_args *a, void *hip_stream) {
     g_err[0] = 0;
     int rc = validate_common(a, false);
     if (rc != FDMA_OK) return rc;
-    const size_t need = fdma_fwd_workspace_bytes(a);
+    size_t shares;
+    const size_t need = fwd_scratch_bytes(a, &shares);
     constexpr size_t kUsable = (size_t)FDMA_NOALLOC_SCRATCH_BYTES - FDMA_NOALLOC_COUNTER_BYTES;
     if (need > kUsable)
         return fail(FDMA_ERR_WORKSPACE, "fdma_fwd_noalloc: this problem needs %zu bytes of scratch, the library's static scratch holds %zu",

@@ -908,6 +908,7 @@ bool compact_per_query_head(const FwdParams &p, FwdParams &pv) {
     return use_compact(pv);
 }
 
+constexpr int COMPACT_LONG_KEYS = 1536;
 bool use_compact(const FwdParams &p) {
     const int mode = p.compact_mode;  // 0 = when it pays, 1 = never, 2 = whenever the mask form allows it
     if (mode == 1 || !p.mask || p.m_r != 0) return false;
@@ -918,7 +919,10 @@ bool use_compact(const FwdParams &p) {
     if (mode == 2) return true;
     // the pre-pass costs about one copy of K and V plus a small launch or two; it pays once the attention
     // itself is a few million (query, key) pairs per kv head
-    return p.Lq >= 128 && p.Lk >= 128 && (int64_t)p.Lq * (p.H / p.Hk) * p.Lk >= (int64_t)1 << 21;
+    if (p.Lq >= 128 && p.Lk >= 128 && (int64_t)p.Lq * (p.H / p.Hk) * p.Lk >= (int64_t)1 << 21) return true;
+    // however few the queries, a workgroup of the tile-skipping kernel walks every tile with a kept key, and scattered keys
+    // leave hardly any tile without: 1.6 us per 128 keys.  @@C@@
+    return p.Lk >= COMPACT_LONG_KEYS && p.Lk / 2 >= p.Lq;
 }
 
 size_t compact_bytes(const FwdParams &p, bool backward, bool reuse_fwd) {

@@ -178,6 +178,21 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
         if (ne < n_end) n_end = ne;
     }
 
+    // SPLIT_KEYS: this workgroup's share [t_first, n_end) of the tiles (see fwd_key_splits)
+    constexpr bool SPLIT_KEYS = CMP && KG == 2;
+    int t_first = 0;
+    if (SPLIT_KEYS && p.splits > 1) {
+        // (no share under eight tiles: the shares that are then left over only say so)
+        const int y = (int)blockIdx.y, most = n_end / 8 > 1 ? n_end / 8 : 1, shares = p.splits < most ? p.splits : most;
+        if (y >= shares) {
+            const int row = m0 + (int)threadIdx.x;
+            if ((int)threadIdx.x < BM && row < LqS) p.lse_part[(((int64_t)y * p.B + b) * p.H + h) * p.Lq + row] = -INFINITY;
+            return;
+        }
+        t_first = n_end * y / shares;
+        n_end = n_end * (y + 1) / shares;
+    }
+
     // ---- active-tile bitmap
     for (int base = 0; !CMP && base < n_end; base += NTHREADS) {
         const int j = base + tid;
@@ -218,7 +233,7 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
     // tells the compiler that the value is wave-uniform, so tile numbers, loop conditions and load addresses stay in
     // scalar registers).  Compacted keys have no bitmap: every tile up to n_end is active.
     uint32_t it_word = 0;
-    int it_base = -32, it_next = 0;
+    int it_base = -32, it_next = t_first;
     auto next_tile = [&]() -> int {
         if (CMP) {
             const int j = it_next < n_end ? it_next : n_end;
@@ -715,7 +730,7 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
             for (int i = 0; i < 16; i++) o[db][i] = 0.f;
         it_word = 0;
         it_base = -32;
-        it_next = 0;
+        it_next = t_first;
         for (Turn j = next_turn(); j.lead < n_end; j = next_turn()) {
             set_tile_k(j);
             set_tile_v(j);
@@ -776,6 +791,23 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
                 }
         }
         const float inv = total > 0.f ? 1.f / total : 0.f;
+        if (SPLIT_KEYS && p.splits > 1) {  // this share's O in fp32 and its log2-sum-exp; fwd_merge_kernel adds the shares up
+            if (qrow < LqS) {
+                const int64_t row = (((int64_t)blockIdx.y * p.B + b) * p.H + h) * p.Lq + qrow;
+                float *op = p.o_part + row * p.d;
+#pragma unroll
+                for (int db = 0; db < DB; db++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int c = 32 * db + 16 * (q >> 1) + 8 * g + 4 * (q & 1);
+                        if (c < p.d)
+                            *(f32x4_t *)(op + c) = f32x4_t{o[db][4 * q] * inv, o[db][4 * q + 1] * inv, o[db][4 * q + 2] * inv, o[db][4 * q + 3] * inv};
+                    }
+                // (a sum that is no number has to reach the result: only an empty share is left out)
+                if (g == 0) p.lse_part[row] = total == 0.f ? -INFINITY : row_ref + __builtin_amdgcn_logf(total);
+            }
+            return;
+        }
         if (qrow < LqS) {
             uint16_t *op = (uint16_t *)p.o + b * p.o_b + (sq.q0 + qrow) * p.o_r + h * p.o_h;
 #pragma unroll
@@ -799,6 +831,52 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
     }
 }
 
+// Adds up the shares of a call with split keys: out = sum_s 2^(l_s - l) O_s, l = log2 sum_s 2^l_s (no share with a visible key:
+// 0 and +inf).  A thread has 8 elements of one row; the rows of O of a share without a visible key hold nothing and are not read.
+constexpr int MAX_KEY_SPLITS = 8;
+template <typename T> __global__ void __launch_bounds__(256) fwd_merge_kernel(const FwdParams p) {
+    using E = Elem<T>;
+    const int CH = p.d / 8;
+    const int64_t rows = (int64_t)p.B * p.H * p.Lq, at = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (at >= rows * CH) return;
+    const int64_t row = at / CH;
+    const int c = (int)(at % CH) * 8;
+    float l[MAX_KEY_SPLITS];
+    f32x4_t v[MAX_KEY_SPLITS][2];
+#pragma unroll
+    for (int s = 0; s < MAX_KEY_SPLITS; s++) l[s] = s < p.splits ? p.lse_part[s * rows + row] : -INFINITY;
+#pragma unroll
+    for (int s = 0; s < MAX_KEY_SPLITS; s++) {
+        v[s][0] = v[s][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (l[s] > -INFINITY) {
+            v[s][0] = *(const f32x4_t *)(p.o_part + (s * rows + row) * p.d + c);
+            v[s][1] = *(const f32x4_t *)(p.o_part + (s * rows + row) * p.d + c + 4);
+        }
+    }
+    float top = l[0];
+#pragma unroll
+    for (int s = 1; s < MAX_KEY_SPLITS; s++) top = fmaxf(top, l[s]);
+    float sum = 0.f;
+    f32x4_t a[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int s = 0; s < MAX_KEY_SPLITS; s++) {
+        const float w = l[s] > -INFINITY ? fast_exp2(l[s] - top) : 0.f;
+        sum += w;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            a[0][e] = fmaf(w, v[s][0][e], a[0][e]);
+            a[1][e] = fmaf(w, v[s][1][e], a[1][e]);
+        }
+    }
+    const float inv = sum > 0.f ? 1.f / sum : 0.f;
+    const int q = (int)(row % p.Lq), h = (int)(row / p.Lq % p.H), b = (int)(row / p.Lq / p.H);
+    u32x4_t w;
+#pragma unroll
+    for (int e = 0; e < 4; e++) w[e] = E::pack2(a[e >> 1][2 * (e & 1)] * inv, a[e >> 1][2 * (e & 1) + 1] * inv);
+    *(u32x4_t *)((uint16_t *)p.o + b * p.o_b + q * p.o_r + h * p.o_h + c) = w;
+    if (c == 0) p.lse[b * p.lse_b + h * p.lse_h + q] = sum > 0.f ? (top + __builtin_amdgcn_logf(sum)) * kLn2 : INFINITY;
+}
+
 template <typename T, int D, int BN, bool CAUSAL, bool CMP, int NW = 4, int KG = 1>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     constexpr int BM = 32 * NW;
@@ -810,8 +888,11 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     const int n_mb = (p.Lq + BM - 1) / BM, G = p.H / p.Hk, pairs = p.B * p.Hk;
     const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
     const int k_split = 8 / gcd8;
-    dim3 grid(pairs * k_split * ((n_mb + k_split - 1) / k_split) * G);
+    dim3 grid(pairs * k_split * ((n_mb + k_split - 1) / k_split) * G, CMP && KG == 2 ? p.splits : 1);
     hipLaunchKernelGGL(kern, grid, dim3(64 * NW * KG), smem, stream, p);
+    if ((e = hipGetLastError()) != hipSuccess || grid.y == 1) return e;
+    const int64_t items = (int64_t)p.B * p.H * p.Lq * (p.d / 8);
+    hipLaunchKernelGGL((fwd_merge_kernel<T>), dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -835,6 +916,22 @@ hipError_t launch_d(const FwdParams &p, hipStream_t stream) {
 }
 
 }  // namespace
+
+// Shares that the key tiles of a row block are cut into: a chunk of a prompt against a long cache has too few blocks of 128
+// rows for the chip, and a workgroup's time is 12 us and 1.6 us per turn of two tiles.  (64-row workgroups on twice the CUs
+// were no faster: a turn takes as long for one wave per SIMD as for two.)  The shares' fp32 results cost what they weigh --
+// 256 workgroups write and read 17 MB, 12 us, and two shares of 128 blocks were no faster than none -- so at most 128
+// workgroups, and only from three shares on; a share has at least 1024 keys and (in the kernel) eight tiles of kept keys.
+// Only where the keys are twice the queries or more: a training step keeps the forward's workspace until its backward, which
+// would hold the shares, and has as many queries as keys.  @@M@@
+int fwd_key_splits(const FwdParams &p) {
+    if (p.cu_q || p.d > 128 || p.Lq < 2 || p.Lk / 2 < p.Lq || !use_compact(p) || !fwd_colmask_applicable(p) || fwd_stream_applicable(p)) return 1;
+    const int64_t blocks = (int64_t)p.B * p.H * ((p.Lq + 127) / 128);
+    int64_t s = blocks > 0 ? device_cus() / 2 / blocks : 1;
+    if (s > p.Lk / 1024) s = p.Lk / 1024;
+    if (s > MAX_KEY_SPLITS) s = MAX_KEY_SPLITS;
+    return s < 3 ? 1 : (int)s;
+}
 
 bool fwd_colmask_applicable(const FwdParams &p) {
     const bool mask_ok = !p.mask || p.m_r == 0;

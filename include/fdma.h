@@ -134,7 +134,8 @@ typedef struct fdma_fwd_args {
     float softcap; /* must be 0: softcapping is not built */
     int32_t compact_mode;   /* FDMA_COMPACT_*; 0 = let the library decide */
     void *workspace;        /* split-KV partials (decode) or the compacted K / V copies; may be NULL if bytes == 0 */
-    size_t workspace_bytes; /* >= fdma_fwd_workspace_bytes(args) */
+    size_t workspace_bytes; /* >= fdma_fwd_workspace_bytes(args).  (Few query rows against many keys: the size includes fp32
+                             * partial results of split keys; a workspace that only lacks those is taken, keys unsplit.) */
     fdma_kept_keys kept;    /* optional: the mask's kept columns as lists (see fdma_kept_keys) */
     fdma_mask_bits mask_bits; /* optional: a per-query mask packed to bits (see fdma_mask_bits) */
     /* Optional: arrival counters of the split-KV decode path (seqlen_q == 1), fdma_fwd_counter_bytes(args) bytes of
@@ -186,8 +187,9 @@ int fdma_bwd(const fdma_bwd_args *args, void *hip_stream);
  * partials with torch, flash_api.cpp:340-345).  args->workspace / workspace_bytes are ignored; the scratch of the
  * decode path (split-KV partials) or of the compaction path lives in a static device array of
  * FDMA_NOALLOC_SCRATCH_BYTES inside the library, which every GPU the library runs on holds until the process ends.
- * A problem whose fdma_fwd_workspace_bytes() exceeds that returns FDMA_ERR_WORKSPACE and launches nothing.  The
- * call makes no hipMalloc / hipFree (nor any other allocating call); results are bit-identical to fdma_fwd's.
+ * A problem whose fdma_fwd_workspace_bytes() exceeds that -- without the partial results of split keys -- returns
+ * FDMA_ERR_WORKSPACE and launches nothing.  The call makes no hipMalloc / hipFree (nor any other allocating call); results are
+ * bit-identical to those of fdma_fwd with a workspace of the array's size (it splits keys only where the partial results fit).
  * Every call on a GPU uses that GPU's one array: calls that overlap on one GPU (different streams or host
  * threads) race on it -- serialise them.  The last FDMA_NOALLOC_COUNTER_BYTES of the array are the decode path's
  * arrival counters (args->counters is ignored as well): they are zero when the library is loaded and every call
