@@ -921,7 +921,9 @@ bool use_compact(const FwdParams &p) {
     // itself is a few million (query, key) pairs per kv head
     if (p.Lq >= 128 && p.Lk >= 128 && (int64_t)p.Lq * (p.H / p.Hk) * p.Lk >= (int64_t)1 << 21) return true;
     // however few the queries, a workgroup of the tile-skipping kernel walks every tile with a kept key, and scattered keys
-    // leave hardly any tile without: 1.6 us per 128 keys.  @@C@@
+    // leave hardly any tile without: 1.6 us per 128 keys, 28 us at 1536
+    // keys against 20 with a quarter of them kept (64 rows x 8 heads of 128; 34 with all kept -- at 3072 both are ahead, 27 and
+    // 33 against 47, and at 768 it is 20 against 17 and 25).
     return p.Lk >= COMPACT_LONG_KEYS && p.Lk / 2 >= p.Lq;
 }
 

@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
             mv[j] = u32x4_t{~0u, ~0u, ~0u, ~0u};
         }
         if (p.mask && (!PERHEAD || p.Hm != p.H)) {
-            ld_row16(p.mask + b * p.m_b + (int64_t)(p.Hm == 1 ? 0 : hk) * p.m_h, key0, p.Lk, mv);
+            ld_row16_skip(p.mask + b * p.m_b + (int64_t)(p.Hm == 1 ? 0 : hk) * p.m_h, key0, p.Lk, mv);
         } else if (p.mask) {  // union of the mask rows of this workgroup's columns
 #pragma unroll
             for (int j = 0; j < DEC_NJ; j++) mv[j] = u32x4_t{0, 0, 0, 0};
