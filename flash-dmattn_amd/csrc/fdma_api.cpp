@@ -366,12 +366,21 @@ int fdma_fwd_noalloc(const fdma_fwd_args *a, void *hip_stream) {
     int rc = validate_common(a, false);
     if (rc != FDMA_OK) return rc;
     size_t shares;
-    const size_t need = fwd_scratch_bytes(a, &shares);
+    size_t need = fwd_scratch_bytes(a, &shares);
     constexpr size_t kUsable = (size_t)FDMA_NOALLOC_SCRATCH_BYTES - FDMA_NOALLOC_COUNTER_BYTES;
+    fdma_fwd_args with_scratch = *a;
+    if (need > kUsable && !fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k)) {
+        fdma::FwdParams p, pv;
+        fill_fwd_params(a, p);
+        if (fdma::compact_per_query_head(p, pv)) p = pv;
+        if (fdma::compact_for_long_keys(p)) {  // (skips tiles, which takes no scratch)
+            with_scratch.compact_mode = FDMA_COMPACT_NEVER;
+            need = fwd_scratch_bytes(&with_scratch, &shares);
+        }
+    }
     if (need > kUsable)
         return fail(FDMA_ERR_WORKSPACE, "fdma_fwd_noalloc: this problem needs %zu bytes of scratch, the library's static scratch holds %zu",
                     need, kUsable);
-    fdma_fwd_args with_scratch = *a;
     with_scratch.workspace = nullptr;
     with_scratch.workspace_bytes = 0;
     with_scratch.counters = nullptr;

@@ -909,6 +909,10 @@ bool compact_per_query_head(const FwdParams &p, FwdParams &pv) {
 }
 
 constexpr int COMPACT_LONG_KEYS = 1536;
+static bool enough_pairs(const FwdParams &p) {
+    return p.Lq >= 128 && p.Lk >= 128 && (int64_t)p.Lq * (p.H / p.Hk) * p.Lk >= (int64_t)1 << 21;
+}
+bool compact_for_long_keys(const FwdParams &p) { return p.compact_mode == 0 && use_compact(p) && !enough_pairs(p); }
 bool use_compact(const FwdParams &p) {
     const int mode = p.compact_mode;  // 0 = when it pays, 1 = never, 2 = whenever the mask form allows it
     if (mode == 1 || !p.mask || p.m_r != 0) return false;
@@ -919,7 +923,7 @@ bool use_compact(const FwdParams &p) {
     if (mode == 2) return true;
     // the pre-pass costs about one copy of K and V plus a small launch or two; it pays once the attention
     // itself is a few million (query, key) pairs per kv head
-    if (p.Lq >= 128 && p.Lk >= 128 && (int64_t)p.Lq * (p.H / p.Hk) * p.Lk >= (int64_t)1 << 21) return true;
+    if (enough_pairs(p)) return true;
     // however few the queries, a workgroup of the tile-skipping kernel walks every tile with a kept key, and scattered keys
     // leave hardly any tile without: 1.6 us per 128 keys, 28 us at 1536
     // keys against 20 with a quarter of them kept (64 rows x 8 heads of 128; 34 with all kept -- at 3072 both are ahead, 27 and

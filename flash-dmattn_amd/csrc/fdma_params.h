@@ -307,6 +307,8 @@ hipError_t launch_bwd_dq(const BwdParams &p, int dtype, hipStream_t stream);
 // p.cmp; for a backward call (bp given) the same launch zero-fills the gradient rows / columns of dropped keys
 // and makes the dK/dV plan.
 bool use_compact(const FwdParams &p);
+// ... and does so for the length of the key axis alone (few query rows): without scratch the call can skip tiles instead
+bool compact_for_long_keys(const FwdParams &p);
 // forward only: `p` has a query-broadcast mask with a row per query head and grouped kv heads, and `pv` -- the same
 // problem as the compaction layer takes it (see FwdParams::kv_share) -- is one that use_compact() accepts
 bool compact_per_query_head(const FwdParams &p, FwdParams &pv);

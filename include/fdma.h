@@ -187,9 +187,10 @@ int fdma_bwd(const fdma_bwd_args *args, void *hip_stream);
  * partials with torch, flash_api.cpp:340-345).  args->workspace / workspace_bytes are ignored; the scratch of the
  * decode path (split-KV partials) or of the compaction path lives in a static device array of
  * FDMA_NOALLOC_SCRATCH_BYTES inside the library, which every GPU the library runs on holds until the process ends.
- * A problem whose fdma_fwd_workspace_bytes() exceeds that -- without the partial results of split keys -- returns
- * FDMA_ERR_WORKSPACE and launches nothing.  The call makes no hipMalloc / hipFree (nor any other allocating call); results are
- * bit-identical to those of fdma_fwd with a workspace of the array's size (it splits keys only where the partial results fit).
+ * A problem whose fdma_fwd_workspace_bytes() exceeds that returns FDMA_ERR_WORKSPACE and launches nothing -- unless all that
+ * does not fit are the partial results of split keys (the keys stay whole) or, under FDMA_COMPACT_AUTO, copies that are made
+ * for few query rows against many keys (tiles are skipped instead).  The call makes no hipMalloc / hipFree (nor any other
+ * allocating call); apart from those two, results are bit-identical to fdma_fwd's.
  * Every call on a GPU uses that GPU's one array: calls that overlap on one GPU (different streams or host
  * threads) race on it -- serialise them.  The last FDMA_NOALLOC_COUNTER_BYTES of the array are the decode path's
  * arrival counters (args->counters is ignored as well): they are zero when the library is loaded and every call

@@ -125,3 +125,21 @@ def test_a_workspace_without_room_for_the_shares():
     assert need > _cabi.NOALLOC_SCRATCH_BYTES and torch.equal(results[1], results[2])
     a.workspace, a.workspace_bytes = ws.data_ptr(), 1 << 16
     assert _cabi.lib.fdma_fwd(a, _cabi.current_stream(q.device)) == -3
+
+
+@pytest.mark.parametrize("per_query_head", [False, True])
+def test_no_room_for_the_copies_of_a_long_key_axis(per_query_head):
+    """Few rows against many keys are compacted under the library's own rule; the entry point that allocates nothing, whose
+    scratch does not hold the copies, skips tiles and still takes the call."""
+    from flash_sparse_attn import _cabi
+
+    B, Lq, Lk, H, Hk, D = 1, 64, 16384, 8, 4, 128
+    heads = H if per_query_head else Hk
+    q, k, v, mask, bias = [t.to(DEV) for t in make_inputs(B, Lq, Lk, H, Hk, D, (B, heads, 1, Lk), (B, heads, 1, Lk), 1000, seed=6)]
+    out, lse = torch.full_like(q, float("nan")), torch.empty(B, H, Lq, device=DEV)
+    a = _cabi.FwdArgs()
+    _cabi.fill_fwd(a, q, k, v, mask, bias, out, lse, D ** -0.5, True, 0.0)
+    assert _cabi.lib.fdma_fwd_workspace_bytes(a) > _cabi.NOALLOC_SCRATCH_BYTES
+    assert _cabi.lib.fdma_fwd_noalloc(a, _cabi.current_stream(q.device)) == 0, _cabi.last_error()
+    torch.cuda.synchronize()
+    assert_out_close(out, eager.attention_forward(q, k, v, mask, bias, None, True)[0])
