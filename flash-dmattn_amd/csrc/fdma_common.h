@@ -207,28 +207,21 @@ template <int D> struct LdsTile {
 // fetched further in front and shifted, without a branch, so that all N loads are in flight together (a branch per piece
 // made a trip to memory of each: decode over 65536 keys 23.1 instead of 22.5 us).
 typedef u32x4_t __attribute__((aligned(1))) u32x4_any_t;
-// SKIP: a wave without such a piece branches over the shifts once all its loads are on their way (a mask row of 65536 keys, 8 x 32 heads: 22.79 -> 22.62 us).
-template <int N, bool SKIP = false> __device__ __forceinline__ void ld_row16(const uint8_t *row, const int (&c)[N], int n, u32x4_t (&v)[N]) {
+__device__ __forceinline__ u32x4_t shift_row16(const u32x4_t &v, int past) {  // `past`: bytes of the piece at or beyond the end
+    uint64_t lo = (uint64_t)v[0] | ((uint64_t)v[1] << 32), hi = (uint64_t)v[2] | ((uint64_t)v[3] << 32);
+    if (past >= 8) { lo = hi; hi = 0; }
+    const int s = past > 0 ? 8 * (past & 7) : 0;
+    lo = (lo >> s) | ((hi << 1) << (63 - s));
+    hi >>= s;
+    if (past >= 16) lo = 0;
+    return u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+template <int N> __device__ __forceinline__ void ld_row16(const uint8_t *row, const int (&c)[N], int n, u32x4_t (&v)[N]) {
     if (n >= 16) {
 #pragma unroll
         for (int u = 0; u < N; u++) v[u] = *(const u32x4_any_t *)(row + (c[u] + 16 <= n ? c[u] : n - 16));
-        if (SKIP) {
-            bool cross = false;
 #pragma unroll
-            for (int u = 0; u < N; u++) cross = cross || c[u] + 16 > n;
-            if (!__any(cross)) return;
-        }
-#pragma unroll
-        for (int u = 0; u < N; u++) {
-            const int past = c[u] + 16 - n;  // bytes of the piece at or beyond the end
-            uint64_t lo = (uint64_t)v[u][0] | ((uint64_t)v[u][1] << 32), hi = (uint64_t)v[u][2] | ((uint64_t)v[u][3] << 32);
-            if (past >= 8) { lo = hi; hi = 0; }
-            const int s = past > 0 ? 8 * (past & 7) : 0;
-            lo = (lo >> s) | ((hi << 1) << (63 - s));
-            hi >>= s;
-            if (past >= 16) lo = 0;
-            v[u] = u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
-        }
+        for (int u = 0; u < N; u++) v[u] = shift_row16(v[u], c[u] + 16 - n);
     } else {
 #pragma unroll
         for (int u = 0; u < N; u++) {
@@ -242,9 +235,6 @@ template <int N, bool SKIP = false> __device__ __forceinline__ void ld_row16(con
             }
         }
     }
-}
-template <int N> __device__ __forceinline__ void ld_row16_skip(const uint8_t *row, const int (&c)[N], int n, u32x4_t (&v)[N]) {
-    ld_row16<N, true>(row, c, n, v);
 }
 __device__ __forceinline__ u32x4_t ld_row16(const uint8_t *row, int c, int n) {
     const int cc[1] = {c};
