@@ -833,6 +833,8 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
 
 // Adds up the shares of a call with split keys: out = sum_s 2^(l_s - l) O_s, l = log2 sum_s 2^l_s (no share with a visible key:
 // 0 and +inf).  A thread has 8 elements of one row; the rows of O of a share without a visible key hold nothing and are not read.
+// Only such a share, l_s = -inf, is left out: an l_s that is no number (a NaN among its keys or in the query) has a weight that is
+// none either, which makes the row what the call with whole keys makes it.
 constexpr int MAX_KEY_SPLITS = 8;
 template <typename T> __global__ void __launch_bounds__(256) fwd_merge_kernel(const FwdParams p) {
     using E = Elem<T>;
@@ -848,7 +850,7 @@ template <typename T> __global__ void __launch_bounds__(256) fwd_merge_kernel(co
 #pragma unroll
     for (int s = 0; s < MAX_KEY_SPLITS; s++) {
         v[s][0] = v[s][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        if (l[s] > -INFINITY) {
+        if (l[s] != -INFINITY) {
             v[s][0] = *(const f32x4_t *)(p.o_part + (s * rows + row) * p.d + c);
             v[s][1] = *(const f32x4_t *)(p.o_part + (s * rows + row) * p.d + c + 4);
         }
@@ -860,7 +862,7 @@ template <typename T> __global__ void __launch_bounds__(256) fwd_merge_kernel(co
     f32x4_t a[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int s = 0; s < MAX_KEY_SPLITS; s++) {
-        const float w = l[s] > -INFINITY ? fast_exp2(l[s] - top) : 0.f;
+        const float w = l[s] != -INFINITY ? fast_exp2(l[s] - top) : 0.f;
         sum += w;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
