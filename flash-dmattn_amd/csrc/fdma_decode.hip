@@ -460,14 +460,15 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
         float mx = -INFINITY;
 #pragma unroll
         for (int q = 0; q < 4; q++) mx = fmaxf(mx, s_m[q][col]);
+        // (a wave without keys has sums of 0 and a maximum of -inf; one whose scores are all NaN has that maximum too, and its
+        // sums have to reach the result)
+        const float ms = mx == -INFINITY ? 0.f : mx;
         float lt = 0.f, ot = 0.f;
-        if (mx != -INFINITY) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const float w = fast_exp2(s_m[q][col] - mx);
-                lt += w * s_l[q][col];
-                ot += w * ((const float *)(smem + q * SM::WAVE_BYTES))[col * SM::SO + e];
-            }
+        for (int q = 0; q < 4; q++) {
+            const float w = fast_exp2(s_m[q][col] - ms);
+            lt += w * s_l[q][col];
+            ot += w * ((const float *)(smem + q * SM::WAVE_BYTES))[col * SM::SO + e];
         }
         const int hh = hk * G + g0 + col;
         const float inv = lt > 0.f ? 1.f / lt : 0.f;
