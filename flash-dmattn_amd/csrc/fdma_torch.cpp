@@ -216,10 +216,10 @@ Tensor aligned_grad(const Tensor &g) {  // what the caller's graph hands back ma
 }
 
 struct AttentionBackward : public Node {
-    SavedVariable q_, k_, v_, mask_, bias_, out_;
-    Tensor buf;  // LSE, and behind it the forward's workspace (lists and compacted copies), which the backward reuses
+    SavedVariable q_, k_, v_, mask_, bias_, out_, lse_;
+    Tensor ws;  // the forward's workspace (lists and compacted copies), which the backward reuses
     SideInputs side;
-    size_t ws_off = 0, ws_bytes = 0;
+    size_t ws_bytes = 0;
     double scale = 1;
     bool causal = false, deterministic = false, has_mask = false, has_bias = false;
     int compact_mode = 0, stream_min = 0;
@@ -227,13 +227,13 @@ struct AttentionBackward : public Node {
     std::string name() const override { return "FlashDMAttnFuncBackward"; }
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
-        for (SavedVariable *s : {&q_, &k_, &v_, &mask_, &bias_, &out_}) s->reset_data();
-        buf.reset();
+        for (SavedVariable *s : {&q_, &k_, &v_, &mask_, &bias_, &out_, &lse_}) s->reset_data();
+        ws.reset();
         side = SideInputs{};
     }
     variable_list apply(variable_list &&grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
-        const Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), out = out_.unpack(shared_from_this());
+        const Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), out = out_.unpack(shared_from_this()), lse = lse_.unpack();
         const Tensor mask = has_mask ? mask_.unpack() : Tensor(), bias = has_bias ? bias_.unpack() : Tensor();
         if (!grads[0].defined()) return variable_list(has_bias ? 4 : 3);
         at::NoGradGuard no_grad;
@@ -242,7 +242,7 @@ struct AttentionBackward : public Node {
         // every element of the gradients is written by the kernels: no zero fill
         Tensor dq = at::empty(q.sizes(), opt), dk = at::empty(k.sizes(), opt), dv = at::empty(v.sizes(), opt), dbias;
         fdma_bwd_args a{};
-        fill_fwd(a.f, q, k, v, mask, bias, out, (float *)buf.data_ptr(), scale, causal, compact_mode, side);
+        fill_fwd(a.f, q, k, v, mask, bias, out, (float *)lse.data_ptr(), scale, causal, compact_mode, side);
         a.dout = dout.data_ptr();
         a.dq = dq.data_ptr(); a.dk = dk.data_ptr(); a.dv = dv.data_ptr();
         strides3(dout, a.do_strides); strides3(dq, a.dq_strides); strides3(dk, a.dk_strides); strides3(dv, a.dv_strides);
@@ -255,7 +255,7 @@ struct AttentionBackward : public Node {
         }
         a.deterministic = deterministic;
         if (ws_bytes && stream_min == api.stream_min_items(0)) {
-            a.fwd_workspace = (const char *)buf.data_ptr() + ws_off;
+            a.fwd_workspace = ws.data_ptr();
             a.fwd_workspace_bytes = ws_bytes;
         }
         const size_t d_bytes = up256((size_t)q.size(0) * q.size(2) * round_up(q.size(1), 128) * 4);
@@ -300,7 +300,7 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             (t == &mask ? t->size(3) < Lk : t->size(3) != Lk) || t->stride(3) != 1)
             Py_RETURN_NOTIMPLEMENTED;
     }
-    // (rows are taken as they lie, unless they differ per query and are shorter than a chunk: fdma.h)
+    // (rows are taken as they lie, unless they differ per query and are shorter than a chunk: fdma.h.)
     const bool rows = Lq > 1 && Lk < 8 && ((mask.defined() && mask.size(2) != 1) || (bias.defined() && bias.size(2) != 1));
     if (rows && ((mask.defined() && !vec_ok(mask, 16)) || (bias.defined() && !vec_ok(bias, 8)))) Py_RETURN_NOTIMPLEMENTED;
     if (mask.defined()) {
@@ -336,9 +336,13 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     Tensor out = at::empty(q.sizes(), opt);
     fdma_fwd_args a;
     fill_fwd(a, q, k, v, mask, bias, out, nullptr, scale, causal, compact_mode, side);
-    const size_t need = api.fwd_workspace_bytes(&a), lse_bytes = up256((size_t)B * H * Lq * 4);
-    Tensor buf = at::empty({(int64_t)(lse_bytes + need)}, bytes);
-    a.lse = (float *)buf.data_ptr();
+    // one buffer for LSE and workspace -- but where a backward will want the LSE, it is a tensor of its own, which the node
+    // saves as autograd does (saved-tensor hooks see it: they may move it off the device until then)
+    const size_t need = api.fwd_workspace_bytes(&a), lse_bytes = is_grad ? 0 : up256((size_t)B * H * Lq * 4);
+    Tensor lse, buf;
+    if (is_grad) lse = at::empty({B, H, Lq}, opt.dtype(at::kFloat));
+    if (lse_bytes + need) buf = at::empty({(int64_t)(lse_bytes + need)}, bytes);
+    a.lse = (float *)(is_grad ? lse : buf).data_ptr();
     void *stream = stream_of(dev);
     if (need) {
         a.workspace = (char *)buf.data_ptr() + lse_bytes;
@@ -359,9 +363,9 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         if ((node->has_mask = mask.defined())) node->mask_ = SavedVariable(mask, false);
         if ((node->has_bias = bias.defined())) node->bias_ = SavedVariable(bias, false);
         node->out_ = SavedVariable(out, true);
-        node->buf = buf;
+        node->lse_ = SavedVariable(lse, false);
         node->side = side;
-        if (need && Lq > 1) { node->ws_off = lse_bytes; node->ws_bytes = need; }
+        if (need && Lq > 1) { node->ws = buf; node->ws_bytes = need; }
         node->scale = scale; node->causal = causal; node->deterministic = deterministic;
         node->compact_mode = compact_mode;
         node->stream_min = api.stream_min_items(0);
@@ -392,8 +396,7 @@ void fill_varlen(fdma_varlen_fwd_args &a, const Tensor &q, const Tensor &k, cons
 }
 
 struct VarlenBackward : public Node {
-    SavedVariable q_, k_, v_, out_, cu_q_, cu_k_;
-    Tensor lse;
+    SavedVariable q_, k_, v_, out_, cu_q_, cu_k_, lse_;
     int64_t max_q = 0, max_k = 0;
     double scale = 1;
     bool causal = false, deterministic = false;
@@ -401,13 +404,12 @@ struct VarlenBackward : public Node {
     std::string name() const override { return "FlashAttnVarlenFuncBackward"; }
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
-        for (SavedVariable *s : {&q_, &k_, &v_, &out_, &cu_q_, &cu_k_}) s->reset_data();
-        lse.reset();
+        for (SavedVariable *s : {&q_, &k_, &v_, &out_, &cu_q_, &cu_k_, &lse_}) s->reset_data();
     }
     variable_list apply(variable_list &&grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         const Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), out = out_.unpack(shared_from_this());
-        const Tensor cu_q = cu_q_.unpack(), cu_k = cu_k_.unpack();
+        const Tensor cu_q = cu_q_.unpack(), cu_k = cu_k_.unpack(), lse = lse_.unpack();
         if (!grads[0].defined()) return variable_list(3);
         at::NoGradGuard no_grad;
         const Tensor dout = aligned_grad(grads[0]);
@@ -479,7 +481,7 @@ PyObject *varlen_attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) 
         node->cu_q_ = SavedVariable(cu_q, false);
         node->cu_k_ = SavedVariable(cu_k, false);
         node->out_ = SavedVariable(out, true);
-        node->lse = lse;
+        node->lse_ = SavedVariable(lse, false);
         node->max_q = max_q; node->max_k = max_k;
         node->scale = scale; node->causal = causal; node->deterministic = truth(args[10]) > 0;
     }
@@ -490,19 +492,17 @@ PyObject *varlen_attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) 
 // ---- bias producer -------------------------------------------------------------------------------------------------
 
 struct DynBiasBackward : public Node {
-    SavedVariable v_, w_, a_, pb_;
-    Tensor dt;
+    SavedVariable v_, w_, a_, pb_, dt_;
     bool has_pb = false;
 
     std::string name() const override { return "DynamicMaskBiasBackward"; }
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
-        for (SavedVariable *s : {&v_, &w_, &a_, &pb_}) s->reset_data();
-        dt.reset();
+        for (SavedVariable *s : {&v_, &w_, &a_, &pb_, &dt_}) s->reset_data();
     }
     variable_list apply(variable_list &&grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
-        const Tensor v = v_.unpack(), w = w_.unpack(), av = a_.unpack(), pb = has_pb ? pb_.unpack() : Tensor();
+        const Tensor v = v_.unpack(), w = w_.unpack(), av = a_.unpack(), pb = has_pb ? pb_.unpack() : Tensor(), dt = dt_.unpack();
         const size_t n_in = has_pb ? 4 : 3;
         if (!grads[0].defined()) return variable_list(n_in);
         at::NoGradGuard no_grad;
@@ -584,7 +584,7 @@ PyObject *dyn_bias(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         node->w_ = SavedVariable(w, false);
         node->a_ = SavedVariable(av, false);
         if ((node->has_pb = has_pb)) node->pb_ = SavedVariable(pb, false);
-        node->dt = dt;
+        node->dt_ = SavedVariable(dt, false);
     }
     return THPVariable_Wrap(std::move(bias));
     END_HANDLE_TH_ERRORS

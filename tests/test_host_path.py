@@ -150,3 +150,55 @@ def test_bias_producer_and_mask_builder_equal_the_general_path(L, pb):
     assert keep[0, 0, 0, row].all() and torch.equal(row, row.sort().values)
     keep[0, 0, 0, 0] = ~keep[0, 0, 0, 0]
     assert M.kept_keys_of(keep) is None
+
+
+def _with_hooks(call, leaves, dout):
+    """Gradients with everything that is saved moved to the host in between, and what the hooks were shown."""
+    packed = []
+
+    def pack(t):
+        packed.append((t.dtype, tuple(t.shape)))
+        return t.device, t.detach().cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda p: p[1].to(p[0])):
+        out = call()
+    assert out is not NotImplemented
+    return out.detach(), torch.autograd.grad(out, leaves, dout), packed
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,d,rows", [
+    (2, 96, 96, 4, 2, 64, 1),      # tile skipping: no workspace
+    (1, 512, 1024, 8, 2, 128, 1),  # compaction: a workspace that the backward uses again
+    (1, 40, 72, 2, 2, 64, 40),     # a mask and bias row per query
+])
+def test_saved_tensor_hooks_see_what_the_attention_saves(B, Lq, Lk, H, Hk, d, rows):
+    q, k, v, mask, bias, dout = _inputs(B, Lq, Lk, H, Hk, d, rows, torch.bfloat16)
+    leaves = [t.requires_grad_(True) for t in (q, k, v, bias)]
+    def call(): return _host().attention(q, k, v, mask, bias, None, True, None, None, None, 0)
+    out = call()
+    o, grads, packed = _with_hooks(call, leaves, dout)
+    assert (torch.float32, (B, H, Lq)) in packed and len(packed) == 7  # q, k, v, mask, bias, out, LSE
+    assert torch.equal(o, out)
+    for a, b in zip(grads, torch.autograd.grad(out, leaves, dout)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_saved_tensor_hooks_see_what_ragged_batch_and_bias_producer_save():
+    g = torch.Generator(device=DEV).manual_seed(3)
+    def leaf(*s): return torch.randn(*s, generator=g, device=DEV).bfloat16().requires_grad_(True)
+    cu = torch.tensor([0, 5, 135, 136, 200], dtype=torch.int32, device=DEV)
+    qkv = [leaf(200, h, 64) for h in (4, 2, 2)]
+    vwa = [leaf(2, 131, 4, 64), leaf(4, 256), leaf(4)]
+    for call, leaves, want, n in (
+        (lambda: _host().varlen_attention(*qkv, cu, cu, 130, 130, None, True, None, None, None, None), qkv, (4, 200), 7),
+        (lambda: _host().dyn_bias(*vwa, None), vwa, (2 * 131, 4), 4),
+    ):
+        out = call()
+        dout = torch.randn(out.shape, generator=g, device=DEV).bfloat16()
+        o, grads, packed = _with_hooks(call, leaves, dout)
+        assert (torch.float32, want) in packed and len(packed) == n
+        assert torch.equal(o, out)
+        for a, b in zip(grads, torch.autograd.grad(out, leaves, dout)):
+            assert torch.equal(a, b)
