@@ -300,9 +300,10 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             (t == &mask ? t->size(3) < Lk : t->size(3) != Lk) || t->stride(3) != 1)
             Py_RETURN_NOTIMPLEMENTED;
     }
-    // (rows are taken as they lie, unless they differ per query and are shorter than a chunk: fdma.h.)
+    // (rows are taken as they lie, unless they differ per query and are shorter than a chunk: fdma.h.  Such rows need strides
+    // that a backward may not find again: a saved-tensor hook can hand the tensor back without them)
     const bool rows = Lq > 1 && Lk < 8 && ((mask.defined() && mask.size(2) != 1) || (bias.defined() && bias.size(2) != 1));
-    if (rows && ((mask.defined() && !vec_ok(mask, 16)) || (bias.defined() && !vec_ok(bias, 8)))) Py_RETURN_NOTIMPLEMENTED;
+    if (rows && (at::GradMode::is_enabled() || (mask.defined() && !vec_ok(mask, 16)) || (bias.defined() && !vec_ok(bias, 8)))) Py_RETURN_NOTIMPLEMENTED;
     if (mask.defined()) {
         // a row per query head over grouped kv heads (its backward is taken apart), or rows that may turn out to be a
         // column mask under the policy "always": general path
