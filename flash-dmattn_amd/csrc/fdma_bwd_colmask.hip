@@ -812,6 +812,10 @@ __device__ __forceinline__ void dkdv_reduce_blocks(const BwdParams &p, const int
 // consecutive workgroups (one per XCD) do that instead of dQ work, one such group after every `period - 1` groups
 // of dQ workgroups.  The reduction only moves memory while the dQ workgroups keep the matrix units busy, so side by
 // side it costs next to nothing; as a launch of its own it took as long as its memory traffic.
+// Few query rows against many keys are the other way round: few dQ workgroups, which leave CUs free, and partials by the number
+// of keys.  Interleaved there is at most one summing group per dQ group; all that the items ask for then follow the dQ groups in
+// one piece (period 1).  100 rows of 16 heads over 2048 kept keys, d = 128 (16 dQ workgroups): the launch 361 us with 16
+// summing workgroups, 54 with 1024.
 struct RedInterleave {
     int red_octets, period, start;
 };
@@ -819,6 +823,11 @@ inline RedInterleave red_interleave(int dq_octets, int items) {
     RedInterleave r;
     r.red_octets = (items < 1024 ? items : 1024) / 8;
     if (r.red_octets < 1) r.red_octets = 1;
+    if (8 * dq_octets <= device_cus() && r.red_octets > dq_octets) {
+        r.period = 1;
+        r.start = dq_octets;
+        return r;
+    }
     r.period = (dq_octets + r.red_octets) / r.red_octets;
     r.period = r.period < 2 ? 2 : (r.period > 4 ? 4 : r.period);
     if (r.red_octets > dq_octets / (r.period - 1)) r.red_octets = dq_octets / (r.period - 1);

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import c_oracle, eager
-from _util import assert_out_close, make_inputs, set_compact
+from _util import assert_grad_close, assert_out_close, make_inputs, set_compact
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -143,3 +143,34 @@ def test_no_room_for_the_copies_of_a_long_key_axis(per_query_head):
     assert _cabi.lib.fdma_fwd_noalloc(a, _cabi.current_stream(q.device)) == 0, _cabi.last_error()
     torch.cuda.synchronize()
     assert_out_close(out, eager.attention_forward(q, k, v, mask, bias, None, True)[0])
+
+
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,D,window,dtype", [
+    (1, 100, 4096, 16, 16, 128, 1024, torch.bfloat16),  # 2 groups of dQ workgroups, 128 that sum
+    (1, 2, 3072, 2, 1, 64, 3072, torch.bfloat16),       # the fewest rows and keys, all kept
+    (2, 33, 5000, 4, 2, 96, 900, torch.float16),
+    (4, 64, 3100, 8, 8, 64, 300, torch.bfloat16),
+    (1, 129, 6200, 6, 3, 256, 700, torch.float16),      # two row blocks, one of a single row
+    (1, 300, 3073, 32, 8, 64, 2, torch.bfloat16),       # two kept keys (with one, dQ is zero and has no scale to compare against)
+])
+@pytest.mark.parametrize("causal", [True, False])
+def test_gradients_of_few_rows_against_many_keys(B, Lq, Lk, H, Hk, D, window, dtype, causal):
+    """Under the library's own rule these are compacted; the partial dK / dV are many for few dQ workgroups."""
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func
+
+    q, k, v, mask, bias = [t.to(DEV) for t in make_inputs(B, Lq, Lk, H, Hk, D, (B, Hk, 1, Lk), (B, Hk, 1, Lk), window, seed=Lq + Lk, dtype=dtype)]
+    a = _cabi.FwdArgs()
+    _cabi.fill_fwd(a, q, k, v, mask, bias, q, torch.empty(B, H, Lq, device=DEV), D ** -0.5, causal, 0.0)
+    assert _cabi.lib.fdma_fwd_workspace_bytes(a) > 0  # (compacted)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(1)).to(dtype).to(DEV)
+    ref = eager.attention_forward_backward(q, k, v, mask, bias, None, causal, dout)
+    runs = []
+    for _ in range(2):
+        leaves = [t.detach().clone().requires_grad_(True) for t in (q, k, v, bias)]
+        out = flash_sparse_attn_func(*leaves[:3], mask, leaves[3], None, causal)
+        runs.append((out.detach(),) + torch.autograd.grad(out, leaves, dout))
+    assert_out_close(runs[0][0], ref[0])
+    for got, want, name in zip(runs[0][1:], ref[1:], ("dq", "dk", "dv", "dbias")):
+        assert_grad_close(got, want, name)
+    for x, y in zip(*runs):
+        assert torch.equal(x, y)
