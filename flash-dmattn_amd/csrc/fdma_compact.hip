@@ -908,9 +908,31 @@ bool compact_per_query_head(const FwdParams &p, FwdParams &pv) {
     return use_compact(pv);
 }
 
-constexpr int COMPACT_LONG_KEYS = 1536;
 static bool enough_pairs(const FwdParams &p) {
     return p.Lq >= 128 && p.Lk >= 128 && (int64_t)p.Lq * (p.H / p.Hk) * p.Lk >= (int64_t)1 << 21;
+}
+// Few query rows against many keys.  A workgroup of the tile-skipping kernel walks every tile with a kept key, and scattered
+// keys leave hardly any tile without: 1.6 us per 128 keys, whatever the batch, while there are no more row blocks than CUs.  The
+// copies are read, written and read again: their cost grows with batch x kv heads and with the share of the keys that is
+// kept, which the host does not know.  Tile skipping over compaction, 64 rows, d = 128, a quarter / half / all keys kept
+// (batch x query heads / kv heads):
+//   keys     1 x 8/8           4 x 8/8           1 x 32/8          4 x 32/8          4 x 16/16         16 x 8/8
+//   1536     1.42 1.11 0.80    1.30 0.97 0.71    1.45 1.13 0.81    1.33 0.98 0.72                      1.12 0.78 0.51
+//   4096     1.98 2.05 1.58    1.74 1.69 1.21    2.26 1.94 1.51    1.85 1.25 0.76    1.72 0.97 0.50*   1.38 0.71 0.37
+//   16384    6.52 5.04 3.42    3.91 2.37 1.15    5.49 3.84 2.41    2.60 1.41 0.69    2.18 1.16 0.60*   1.54 0.79 0.41
+// (* 8192 and 32768 keys; d = 64 alike, d = 256 1.8 to 3.6, 0.95 to 1.9, 0.5 to 0.95).  Forward and backward, the same: 1536 keys
+// 0.8 to 1.1 even with a quarter kept, 3072 keys 1.1 to 1.8, 1.0 to 1.6, 0.7 to 1.2.  So:
+//   * from 3072 keys on, and up to 32 pairs of batch entry and kv head: half of the keys kept gain everywhere;
+//   * copies of up to half a gigabyte: they are as large as the caller's whole K and V, and are held until the backward;
+//   * a mask with one row for all of several kv heads is what padding looks like, which keeps nearly everything: from 4096
+//     keys on, and only where the few blocks let the keys be cut into shares (key_shares), which is ahead with all of them
+//     kept (1.15 to 3.5; forward and backward 0.98 to 1.6).
+constexpr int COMPACT_LONG_KEYS = 3072, COMPACT_LONG_KEYS_PADDING = 4096, COMPACT_LONG_PAIRS = 32;
+constexpr int64_t COMPACT_LONG_BYTES = (int64_t)1 << 29;
+static bool few_rows_many_keys(const FwdParams &p) {
+    const int64_t pairs = (int64_t)p.B * p.Hk;
+    if (p.Lk < COMPACT_LONG_KEYS || p.Lk / 2 < p.Lq || pairs > COMPACT_LONG_PAIRS || pairs * p.Lk * p.d * 4 > COMPACT_LONG_BYTES) return false;
+    return p.Hm == p.Hk || (p.Lk >= COMPACT_LONG_KEYS_PADDING && key_shares(p) > 1);
 }
 bool compact_for_long_keys(const FwdParams &p) { return p.compact_mode == 0 && use_compact(p) && !enough_pairs(p); }
 bool use_compact(const FwdParams &p) {
@@ -924,11 +946,7 @@ bool use_compact(const FwdParams &p) {
     // the pre-pass costs about one copy of K and V plus a small launch or two; it pays once the attention
     // itself is a few million (query, key) pairs per kv head
     if (enough_pairs(p)) return true;
-    // however few the queries, a workgroup of the tile-skipping kernel walks every tile with a kept key, and scattered keys
-    // leave hardly any tile without: 1.6 us per 128 keys, 28 us at 1536
-    // keys against 20 with a quarter of them kept (64 rows x 8 heads of 128; 34 with all kept -- at 3072 both are ahead, 27 and
-    // 33 against 47, and at 768 it is 20 against 17 and 25).
-    return p.Lk >= COMPACT_LONG_KEYS && p.Lk / 2 >= p.Lq;
+    return few_rows_many_keys(p);
 }
 
 size_t compact_bytes(const FwdParams &p, bool backward, bool reuse_fwd) {

@@ -927,13 +927,16 @@ hipError_t launch_d(const FwdParams &p, hipStream_t stream) {
 // Only where the keys are twice the queries or more: a training step keeps the forward's workspace until its backward, which
 // would hold the shares, and has as many queries as keys.  32000 keys, 300 kept, 16 rows x 4 heads: 21.6 us; 30000 keys, 4000
 // kept, 33 rows x 32 heads of 64: 30.8 us; 16384 keys, 4096 kept, 512 rows x 8 heads: 60 us whole, 37 us in four shares.
-int fwd_key_splits(const FwdParams &p) {
-    if (p.cu_q || p.d > 128 || p.Lq < 2 || p.Lk / 2 < p.Lq || !use_compact(p) || !fwd_colmask_applicable(p) || fwd_stream_applicable(p)) return 1;
+int key_shares(const FwdParams &p) {
+    if (p.cu_q || p.d > 128 || p.Lq < 2 || p.Lk / 2 < p.Lq) return 1;
     const int64_t blocks = (int64_t)p.B * p.H * ((p.Lq + 127) / 128);
     int64_t s = blocks > 0 ? device_cus() / 2 / blocks : 1;
     if (s > p.Lk / 1024) s = p.Lk / 1024;
     if (s > MAX_KEY_SPLITS) s = MAX_KEY_SPLITS;
     return s < 3 ? 1 : (int)s;
+}
+int fwd_key_splits(const FwdParams &p) {
+    return use_compact(p) && fwd_colmask_applicable(p) && !fwd_stream_applicable(p) ? key_shares(p) : 1;
 }
 
 bool fwd_colmask_applicable(const FwdParams &p) {

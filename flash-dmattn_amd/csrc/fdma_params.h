@@ -278,6 +278,7 @@ hipError_t launch_fwd_colmask(const FwdParams &p, int dtype, hipStream_t stream)
 // compacted forward: shares the keys of a row block are cut into (1: none); p.o_part / p.lse_part then hold
 // splits * B * H * Lq rows of d / 1 floats
 int fwd_key_splits(const FwdParams &p);
+int key_shares(const FwdParams &p);  // ... as far as the sizes go: what they would be if the keys were compacted
 // compacted forward on tile images (fdma_fwd_stream.hip): resident workgroups that walk their share of the
 // (query block, head) items with the tiles of the next item already on their way.  `fwd_stream_applicable` decides from
 // the problem alone (the pre-pass, the forward and the backward of a problem must agree on the workspace layout).

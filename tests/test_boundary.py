@@ -293,6 +293,40 @@ def test_compaction_workspace_rule():
     assert kv_bytes <= need <= 2 * kv_bytes                      # dense K / V copies plus index lists
 
 
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,Hm,D,want", [
+    (1, 64, 3072, 8, 8, 8, 128, True),        # few rows against many keys, a mask row per kv head
+    (1, 64, 3071, 8, 8, 8, 128, False),
+    (4, 64, 16384, 32, 8, 8, 128, True),
+    (4, 2, 32768, 8, 8, 8, 128, True),        # 32 pairs, copies of half a gigabyte
+    (4, 2, 32769, 8, 8, 8, 128, False),
+    (1, 64, 32768, 33, 33, 33, 64, False),    # 33 pairs
+    (16, 4, 32768, 8, 8, 8, 128, False),      # would copy the whole cache
+    (1, 4, 300000, 8, 8, 8, 256, False),
+    (1, 64, 4096, 8, 8, 1, 128, True),        # one mask row for all kv heads (padding): where the keys are cut into shares
+    (1, 64, 4095, 8, 8, 1, 128, False),
+    (4, 64, 8192, 32, 8, 1, 128, False),
+    (1, 64, 8192, 8, 8, 1, 256, False),
+    (1, 64, 8192, 8, 1, 1, 128, True),        # a single kv head: a row per kv head all the same
+    (1, 1600, 3100, 1, 1, 1, 64, True),       # (enough query rows: the other rule)
+    (16, 512, 32768, 32, 8, 1, 64, True),
+])
+def test_which_long_key_axes_are_compacted(B, Lq, Lk, H, Hk, Hm, D, want):
+    """The scratch of a call says whether it is compacted: under the library's own rule few rows against many keys are where
+    that pays with half of the keys kept, and with all of them where the mask may be padding, and never at the price of
+    copies beyond half a gigabyte."""
+    from flash_sparse_attn import _cabi
+
+    a = _valid_fwd()
+    a.batch, a.seqlen_q, a.seqlen_k, a.num_heads, a.num_heads_k, a.head_dim = B, Lq, Lk, H, Hk, D
+    a.mask, a.num_heads_mask = 16, Hm
+    a.mask_strides[:] = (Lk * Hm, Lk, 0)
+    a.bias = None
+    need = _cabi.lib.fdma_fwd_workspace_bytes(a)
+    assert (need > 0) == want
+    if want and B * Hk <= 32:
+        assert need <= 1.25 * max(4 * B * Hk * Lk * D, 1 << 29)
+
+
 def _valid_varlen_fwd():
     from flash_sparse_attn import _cabi
 
