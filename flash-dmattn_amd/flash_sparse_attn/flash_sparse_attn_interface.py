@@ -288,8 +288,10 @@ _wrapped_flash_sparse_attn_forward = _direct_when_eager(_flash_sparse_attn_forwa
 def _per_query_head_groups(q, k, mask, bias) -> int:
     """Query heads per kv head when the backward of this call is to be taken apart by group member (see
     _backward_per_query_head), else 1: a query-broadcast mask with a row per QUERY head over grouped kv heads, next to
-    no bias or a query-broadcast one, on a problem for which the library would compact a mask with a row per kv head
-    (fdma_compact.hip: use_compact -- the same rule, on what one group member sees)."""
+    no bias or a query-broadcast one, on a problem with enough pairs of rows and keys that the library would compact what
+    one group member sees.  Few rows against many keys, which the library's forward compacts as well, stay whole here: G
+    backward calls one after the other cost more than the tiles they save (an eighth / half of the keys kept, 8 query over
+    4 kv heads of 64: 64 rows x 4096 keys 125 / 123 us whole, 304 / 307 in two calls; 100 x 16384 314 / 315 and 315 / 452)."""
     if mask is None or mask.shape[2] != 1 or (bias is not None and bias.shape[2] != 1):
         return 1
     num_heads, num_heads_k = q.shape[2], k.shape[2]

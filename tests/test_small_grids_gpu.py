@@ -174,3 +174,18 @@ def test_gradients_of_few_rows_against_many_keys(B, Lq, Lk, H, Hk, D, window, dt
         assert_grad_close(got, want, name)
     for x, y in zip(*runs):
         assert torch.equal(x, y)
+
+
+def test_gradients_of_few_rows_with_a_mask_row_per_query_head():
+    """The forward compacts per query head; the backward skips tiles, group members together."""
+    from flash_sparse_attn import flash_sparse_attn_func
+
+    B, Lq, Lk, H, Hk, D = 1, 60, 3100, 4, 2, 64
+    q, k, v, mask, bias = [t.to(DEV) for t in make_inputs(B, Lq, Lk, H, Hk, D, (B, Hk, 1, Lk), (B, H, 1, Lk), 700, seed=8)]
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(1)).to(q.dtype).to(DEV)
+    ref = eager.attention_forward_backward(q, k, v, mask, bias, None, True, dout)
+    leaves = [t.detach().clone().requires_grad_(True) for t in (q, k, v, bias)]
+    out = flash_sparse_attn_func(*leaves[:3], mask, leaves[3], None, True)
+    assert_out_close(out, ref[0])
+    for got, want, name in zip(torch.autograd.grad(out, leaves, dout), ref[1:], ("dq", "dk", "dv", "dbias")):
+        assert_grad_close(got, want, name)
