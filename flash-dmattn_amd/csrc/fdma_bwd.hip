@@ -653,16 +653,25 @@ hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
 
 }  // namespace
 
-// Segments of the general dK/dV kernel: as many as it takes to give every CU a workgroup (two at d <= 64, where two fit;
-// a causal launch twice that, since its workgroups are of very different lengths), each at least two query blocks long.
+// Segments of the general dK/dV kernel.  Without them a short or grouped call has a workgroup per 128 keys of a kv head and
+// most CUs idle; each segment costs its fp32 sums, written and read again, and the launch that adds them up.
+//   * As many as the chip holds workgroups at once (two per CU at d <= 64, else one), rounded DOWN: a few workgroups beyond
+//     that are another round of the whole length.  192 key blocks of 700 rows, d = 128: 73.6 us without segments, 92.9 in two.
+//   * A causal call's workgroups are of very different lengths: half as many again, rounded to the nearest from 1280 rows on,
+//     where a workgroup is long against the sums (16 heads of 2000 rows, d = 128: 177 us whole, 155 in two; 1000 rows x 2
+//     batch entries: 95.5 and 104.7).
+//   * At least two query blocks each; three in the eight-wave kernel (64 < d <= 128) where a block is one step (no grouped
+//     heads) and the sums of more than CUs / 8 key blocks weigh (64 of them, 200 rows: 35.4 us whole, 39.0 in two).
+// Swept over 402 calls -- 200 to 3000 rows, 1 to 32 query heads over 1 to 32 (batch entry, kv head) pairs, d = 64, 128, 256, both
+// kinds of mask -- with 1 to 16 segments: never slower than whole, 0.9 % behind the best number on average, a fifth at most.
 int general_kv_segments(const FwdParams &f) {
     if (f.Lk <= 0 || f.Lq <= 0) return 1;
-    const int bm = f.d > 128 ? 32 : 64;
+    const int cus = device_cus(), blocks = f.d > 128 ? (f.Lq + 31) / 32 : (f.Lq + 63) / 64;
     const int64_t units = (int64_t)((f.Lk + KV_BN - 1) / KV_BN) * f.Hk * f.B;
-    const int64_t want = (int64_t)device_cus() * (f.d <= 64 ? 2 : 1) * (f.causal ? 2 : 1);
-    int64_t segs = units >= want ? 1 : (want + units - 1) / units;
-    const int64_t most = ((f.Lq + bm - 1) / bm) / 2;
-    segs = segs > most ? most : segs;
+    const int64_t twice = (int64_t)cus * (f.d <= 64 ? 2 : 1) * (f.causal ? 3 : 2);  // (twice the workgroups wanted)
+    int64_t segs = (twice + (f.causal && f.Lq >= 1280 ? units : 0)) / (2 * units);
+    const int least = f.d > 64 && f.d <= 128 && f.H == f.Hk && units > cus / 8 ? 3 : 2;
+    segs = segs > blocks / least ? blocks / least : segs;
     return segs > 16 ? 16 : (segs < 1 ? 1 : (int)segs);
 }
 

@@ -327,6 +327,36 @@ def test_which_long_key_axes_are_compacted(B, Lq, Lk, H, Hk, Hm, D, want):
         assert need <= 1.25 * max(4 * B * Hk * Lk * D, 1 << 29)
 
 
+@pytest.mark.parametrize("B,L,H,Hk,D,causal,want", [
+    (2, 700, 16, 16, 128, 0, 1),    # 192 key blocks: more than half of the 256 CUs, so whole
+    (1, 700, 16, 16, 128, 0, 2),    # 96 key blocks: 2, not 3 (288 workgroups)
+    (1, 3000, 2, 1, 256, 0, 10),    # 24 key blocks: 240 workgroups, not 264
+    (1, 3000, 8, 2, 64, 0, 10),     # two workgroups per CU
+    (2, 1400, 16, 16, 128, 1, 1),   # causal: half as many again ...
+    (1, 1000, 16, 16, 128, 1, 3),
+    (1, 2000, 16, 16, 128, 1, 2),   # ... and rounded to the nearest for long calls
+    (2, 200, 16, 16, 128, 0, 1),    # at least three query blocks each
+    (2, 200, 16, 16, 64, 0, 2),     # at least two
+    (2, 200, 16, 8, 128, 0, 2),
+    (1, 200, 2, 2, 128, 0, 2),
+    (1, 2000, 2, 1, 64, 1, 16),     # at most 16
+    (1, 90, 2, 1, 64, 1, 1),
+])
+def test_segments_of_the_general_dkdv_kernel(B, L, H, Hk, D, causal, want):
+    """The scratch of the call holds the segments' sums: 2 x 128 x D floats per key block and segment (none when it is whole)."""
+    from flash_sparse_attn import _cabi
+
+    b = _cabi.BwdArgs()
+    a = _valid_fwd()
+    a.batch, a.seqlen_q, a.seqlen_k, a.num_heads, a.num_heads_k, a.head_dim, a.is_causal = B, L, L, H, Hk, D, causal
+    a.mask, a.num_heads_mask = 16, Hk
+    a.mask_strides[:] = (L * L * Hk, L * L, L)
+    a.bias = None
+    ctypes.memmove(ctypes.byref(b.f), ctypes.byref(a), ctypes.sizeof(a))
+    part = (L + 127) // 128 * Hk * B * 2 * 128 * D * 4
+    assert _cabi.lib.fdma_bwd_workspace_bytes(b) == (0 if want == 1 else part * want)
+
+
 def _valid_varlen_fwd():
     from flash_sparse_attn import _cabi
 

@@ -17,7 +17,7 @@ CASES = [
     (1, 70, 130, 4, 2, 128, 4, 2, 70, False),    # group sum, a mask per query head
     (2, 64, 128, 2, 2, 128, 1, 2, 64, True),     # whole tiles, no group
     (1, 33, 257, 8, 2, 96, 2, 8, 33, False),     # a head dim in between, bias per query head
-    (1, 300, 9, 4, 1, 128, 1, 1, 300, False),    # one key block, five query segments
+    (1, 300, 9, 4, 1, 128, 1, 1, 300, False),    # one key block, two query segments
     (1, 513, 129, 2, 1, 128, 0, 1, 513, True),   # no mask
     (1, 200, 190, 4, 2, 128, 2, 2, 1, True),     # bias row shared by the queries: column sums over segments
     (1, 200, 190, 4, 2, 72, 4, 4, 1, False),
@@ -28,6 +28,7 @@ CASES = [
     (2, 257, 77, 4, 4, 40, 1, 4, 257, False),
     (1, 131, 203, 2, 1, 256, 1, 1, 131, True),
     (1, 90, 61, 2, 2, 200, 2, 2, 1, False),
+    (1, 2100, 40, 2, 1, 128, 1, 1, 2100, True),  # the most query segments, of unequal length; rows without visible keys
 ]
 
 
