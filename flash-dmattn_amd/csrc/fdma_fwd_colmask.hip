@@ -925,8 +925,12 @@ hipError_t launch_d(const FwdParams &p, hipStream_t stream) {
 // 256 workgroups write and read 17 MB, 12 us, and two shares of 128 blocks were no faster than none -- so at most 128
 // workgroups, and only from three shares on; a share has at least 1024 keys and (in the kernel) eight tiles of kept keys.
 // Only where the keys are twice the queries or more: a training step keeps the forward's workspace until its backward, which
-// would hold the shares, and has as many queries as keys.  32000 keys, 300 kept, 16 rows x 4 heads: 21.6 us; 30000 keys, 4000
-// kept, 33 rows x 32 heads of 64: 30.8 us; 16384 keys, 4096 kept, 512 rows x 8 heads: 60 us whole, 37 us in four shares.
+// would hold the shares, and has as many queries as keys.  Whole keys / shares in us (a workspace without / with room for them;
+// medians over 1 to 40 blocks of 2 to 300 rows, d = 128; d = 64 is alike), with a sixteenth, a quarter and all of the keys kept:
+//   3072 keys   16.5 / 20.2    24.4 / 27.9    53.0 / 34.4        16384 keys   27.4 / 25.9    65.0 / 31.1    207.5 / 54.8
+//   6144 keys   19.4 / 22.4    34.0 / 26.8    90.2 / 39.3        32768 keys   40.4 / 28.4   114.7 / 40.1    395.4 / 88.2
+// How much is kept is not known here: with under 1024 kept keys there is a single share and the merge costs its 3 to 4 us for
+// nothing; the other way round a share too few costs more.
 int key_shares(const FwdParams &p) {
     if (p.cu_q || p.d > 128 || p.Lq < 2 || p.Lk / 2 < p.Lq) return 1;
     const int64_t blocks = (int64_t)p.B * p.H * ((p.Lq + 127) / 128);
