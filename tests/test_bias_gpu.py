@@ -2,7 +2,7 @@
 
 Checker: the closed form  bias[b, j, 0, l] = A[j] * softplus(V[b, l].flatten() . W[j] + pb[j])  in fp32 with torch
 autograd, on the same 16-bit inputs.  Tolerances: the forward is rounded to the 16-bit output type once (relative
-error <= 2^-8 of the row scale); gradients within rtol 2e-2 of their scale (sums of up to 16 Ki products rounded to 16 bits)."""
+error <= 2^-8 of the row scale); gradients within rtol 2e-2 of their scale (fp32 sums of products, rounded to 16 bits)."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -20,6 +20,11 @@ CASES = [
     (3, 77, 1, 128, True, torch.float16),
     (1, 300, 12, 32, False, torch.bfloat16),
     (2, 129, 32, 16, True, torch.bfloat16),
+    # from 131072 tokens on a wave has 32 of them to itself: either side of the line, a last workgroup of ten tokens behind a
+    # batch boundary inside a wave's tokens with less than a piece of columns, several pieces
+    (1, 131071, 2, 24, True, torch.bfloat16),
+    (2, 65541, 2, 24, True, torch.float16),
+    (1, 131072, 8, 72, False, torch.bfloat16),
 ]
 
 
@@ -88,6 +93,21 @@ def test_bias_producer_is_bit_reproducible_and_feeds_the_operator():
     q = torch.randn(B, L, H, d, device=DEV).to(torch.bfloat16)
     out = flash_sparse_attn_func(q, kv[:, :, 0], kv[:, :, 1], keep, bias, None, True)
     assert torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize("L", [300, 131200])
+def test_value_states_whose_heads_lie_apart(L):
+    """(batch, heads, keys, head dim) value states handed over as a transposed view: a column's head is part of its address."""
+    Hk, d = 4, 40
+    v, w, a, _, gout = _inputs(1, L, Hk, d, False, torch.bfloat16, seed=L)
+    view = v.transpose(1, 2).contiguous().to(DEV).transpose(1, 2).requires_grad_(True)
+    wd, ad = [t.to(DEV).requires_grad_(True) for t in (w, a)]
+    bias = dynamic_mask_bias(view, wd, ad)
+    grads = torch.autograd.grad(bias, (view, wd, ad), gout.to(DEV))
+    rb, rdv, rdw, rda, _ = _reference(v.to(DEV), w.to(DEV), a.to(DEV), None, gout.to(DEV))
+    assert rel_err(bias, rb) <= 2.0 ** -8
+    for got, ref in zip(grads, (rdv, rdw, rda)):
+        assert rel_err(got, ref) <= 2e-2
 
 
 def test_bias_producer_rejects_shapes_it_was_not_built_for():
