@@ -24,7 +24,9 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/version.h>
 
+#include <cstdio>
 #include <list>
 #include <utility>
 
@@ -114,10 +116,16 @@ bool same_shape(const Tensor &t, PyObject *tup) {
     return true;
 }
 
-// Attribute `name` of a plain tensor object, or nullptr (borrowed; no exception is raised for a missing one).
+// Attribute `name` of a plain tensor object's own dictionary, or nullptr (borrowed; no exception is raised for a missing one).
 PyObject *instance_attr(PyObject *o, PyObject *name) {
-    PyObject **dict = _PyObject_GetDictPtr(o);
-    return dict && *dict ? PyDict_GetItem(*dict, name) : nullptr;
+    PyObject *dict = PyObject_GenericGetDict(o, nullptr);
+    if (!dict) {
+        PyErr_Clear();
+        return nullptr;
+    }
+    PyObject *attr = PyDict_GetItem(dict, name);
+    Py_DECREF(dict);  // (the object keeps it)
+    return attr;
 }
 
 // (version, data pointer, shape) left at the end of a record by the mask builder still describe the tensor
@@ -714,5 +722,15 @@ PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fdma_torch", nullptr, -1, met
 PyMODINIT_FUNC PyInit__fdma_torch(void) {
     s_kept = PyUnicode_InternFromString("_fdma_kept");
     s_bits = PyUnicode_InternFromString("_fdma_bits");
-    return PyModule_Create(&module_def);
+    PyObject *mod = PyModule_Create(&module_def);
+    // what this file is tied to (major and minor version of Python); whoever loads it compares
+    char python[16];
+    snprintf(python, sizeof(python), "%d.%d", PY_MAJOR_VERSION, PY_MINOR_VERSION);
+    PyObject *built_for = mod ? Py_BuildValue("(ss)", TORCH_VERSION, python) : nullptr;
+    if (!built_for || PyModule_AddObject(mod, "built_for", built_for) < 0) {
+        Py_XDECREF(built_for);
+        Py_XDECREF(mod);
+        return nullptr;
+    }
+    return mod;
 }

@@ -11,6 +11,8 @@ import importlib.machinery
 import importlib.util
 import os
 import struct
+import sys
+import warnings
 from typing import Optional, Sequence
 
 import torch
@@ -253,16 +255,37 @@ _HOST_CALLS = (
 )
 
 
+class _NoHost:
+    """Stands in for the native host path where it cannot be used: it declines every call, and the operators' Python code
+    makes them all, on the same kernels."""
+
+    @staticmethod
+    def _decline(*args):
+        return NotImplemented
+
+    attention = varlen_attention = dyn_bias = create_mask = _decline
+
+
 def _load_host():
     """The native host path of the operators (csrc/fdma_torch.cpp), bound to the functions of `lib`: the calls it takes
-    skip the Python below, the others it answers with NotImplemented."""
-    if not os.path.exists(_HOST_PATH):
-        raise ImportError(f"{_HOST_PATH} not found: build it with `make -C flash-dmattn_amd/csrc` (or __graft_entry__.build()); "
-                          "there is no fallback implementation")
-    loader = importlib.machinery.ExtensionFileLoader("_fdma_torch", _HOST_PATH)
-    spec = importlib.util.spec_from_loader("_fdma_torch", loader)
-    mod = importlib.util.module_from_spec(spec)
-    loader.exec_module(mod)
+    skip the Python below, the others it answers with NotImplemented.  It is tied to the C++ interface of the torch and to
+    the Python that it was built with; the library of kernels is not, so without a host path that fits the operators warn
+    and take their Python path, which costs a call 10 to 100 us of host time."""
+    why = None
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_fdma_torch", _HOST_PATH)
+        spec = importlib.util.spec_from_loader("_fdma_torch", loader)
+        mod = importlib.util.module_from_spec(spec)
+        loader.exec_module(mod)
+        here = (torch.__version__.split("+")[0], "%d.%d" % sys.version_info[:2])
+        if mod.built_for != here:
+            why = "built for torch %s and Python %s, not torch %s and Python %s" % (mod.built_for + here)
+    except (ImportError, OSError) as e:  # (not built, or symbols that this torch does not have)
+        why = str(e)
+    if why is not None:
+        warnings.warn(f"the native host path of the operators cannot be used ({_HOST_PATH}: {why}); calls take the slower Python path. "
+                      "Build it with `make -C flash-dmattn_amd/csrc` (or __graft_entry__.build())", RuntimeWarning, stacklevel=2)
+        return _NoHost
     mod.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _HOST_CALLS})
     return mod
 

@@ -21,6 +21,55 @@ def test_declines_what_is_not_an_ordinary_device_tensor():
     assert _host().attention("q", q, q, None, None, None, None, None, None, None, 0) is NotImplemented
 
 
+@pytest.mark.parametrize("how", ["missing", "not an extension", "another torch", "another python"])
+def test_without_a_host_path_that_fits_the_operators_warn_and_decline(how, monkeypatch, tmp_path):
+    """The kernels do not depend on torch's C++ interface, so neither does the package."""
+    import sys
+    from flash_sparse_attn import _cabi
+
+    if how == "missing":
+        monkeypatch.setattr(_cabi, "_HOST_PATH", str(tmp_path / "_fdma_torch.so"))
+    elif how == "not an extension":
+        (tmp_path / "_fdma_torch.so").write_bytes(b"not a shared object")
+        monkeypatch.setattr(_cabi, "_HOST_PATH", str(tmp_path / "_fdma_torch.so"))
+    elif how == "another torch":
+        monkeypatch.setattr(torch, "__version__", "1.13.1")
+    else:
+        monkeypatch.setattr(sys, "version_info", (3, 99, 0))
+    with pytest.warns(RuntimeWarning, match="host path"):
+        host = _cabi._load_host()
+    assert host.attention(*[None] * 11) is NotImplemented and host.varlen_attention(*[None] * 13) is NotImplemented
+    assert host.dyn_bias(*[None] * 4) is NotImplemented and host.create_mask(*[None] * 6) is NotImplemented
+
+
+def test_the_built_host_path_fits_this_torch():
+    from flash_sparse_attn import _cabi
+
+    assert _cabi.host is not _cabi._NoHost and _cabi.host.built_for[0] == torch.__version__.split("+")[0]
+
+
+@pytest.mark.gpu
+def test_operators_without_the_host_path(monkeypatch):
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func, flash_sparse_attn_varlen_func
+    from flash_sparse_attn.utils.bias import dynamic_mask_bias
+    from flash_sparse_attn.utils.mask import create_mask
+
+    q, k, v, _, _, dout = _inputs(1, 200, 200, 4, 2, 64, 1, torch.bfloat16)
+    w, a = [torch.randn(*s, device=DEV).bfloat16() * 0.1 for s in ((2, 128), (2,))]
+    cu = torch.tensor([0, 70, 200], dtype=torch.int32, device=DEV)
+    leaves = [t.requires_grad_(True) for t in (q, k, v, w, a)]
+    runs = []
+    for host in (_cabi.host, _cabi._NoHost):
+        monkeypatch.setattr(_cabi, "host", host)
+        bias = dynamic_mask_bias(v, w, a)
+        mask = create_mask(bias, None, 1, 200, 200, 64, torch.finfo(bias.dtype).min)
+        out = flash_sparse_attn_func(q, k, v, mask, bias, is_causal=True)
+        ragged = flash_sparse_attn_varlen_func(q[0], k[0], v[0], cu, cu, 130, 130, is_causal=True)
+        runs.append((mask, out.detach(), ragged.detach()) + torch.autograd.grad((out, ragged), leaves, (dout, dout[0])))
+    for x, y in zip(*runs):
+        assert torch.equal(x, y)
+
+
 class _NoTruth:
     def __bool__(self):
         raise ValueError("no truth value")
