@@ -97,8 +97,14 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
 
     extern __shared__ __attribute__((aligned(16))) char smem_all[];
     const int kgrp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NTHREADS);  // key group of this wave
-    char *const smem = smem_all + kgrp * SM::TOTAL;
-    uint32_t *sBits = (uint32_t *)(smem + SM::OFF_BITS);
+    // This group's LDS.  A lone group at d = 128 addresses the array itself: through the pointer variable the same places took 4
+    // more registers, which the eight-wave kernels do not have (20 bytes spilled; ragged forward of 11 265 tokens x 32 heads
+    // 370.0 -> 367.1 us, of 3 518 x 16 56.0 -> 55.2).  With compacted keys at d = 256 it is 1 % as well (3 000 tokens x 8 heads
+    // 63.1 -> 62.2).  Elsewhere the pointer is ahead by as much (ragged, 18 000 tokens x 16, d = 64: 127.3 and 128.9; 2 800 x 16,
+    // d = 256: 73.9 and 74.8).
+    char *const smem_grp = smem_all + kgrp * SM::TOTAL;
+#define FWD_LDS (KG == 1 && (D == 128 || (D == 256 && CMP)) ? smem_all : smem_grp)
+    uint32_t *sBits = (uint32_t *)(FWD_LDS + SM::OFF_BITS);
     uint32_t *sFlag = (uint32_t *)(smem_all + SM::OFF_FLAG);  // (one for all: the groups leave the common path together)
 
     const int tid = (int)threadIdx.x - kgrp * NTHREADS;
@@ -223,9 +229,9 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
     // stage 1 is cleared as well: the first pipeline step multiplies it with zero probabilities (there is no half tile
     // in front of the first one), and what an earlier workgroup left there need not be a number.  (All of it is made
     // visible by the barrier in front of the main loop.)
-    if (tid < 2 * BN) *(u32x4_t *)(smem + SM::OFF_X + tid * 32 + 16) = u32x4_t{0, 0, 0, 0};
+    if (tid < 2 * BN) *(u32x4_t *)(FWD_LDS + SM::OFF_X + tid * 32 + 16) = u32x4_t{0, 0, 0, 0};
     for (int i = tid; i < SM::VT_BYTES / 16; i += NTHREADS)
-        *(u32x4_t *)(smem + SM::OFF_VT + SM::VT_BYTES + i * 16) = u32x4_t{0, 0, 0, 0};
+        *(u32x4_t *)(FWD_LDS + SM::OFF_VT + SM::VT_BYTES + i * 16) = u32x4_t{0, 0, 0, 0};
     if (!CMP) __syncthreads();  // (compacted keys have no bitmap: every tile up to n_end is active)
 
     // Iterator over the active tiles in ascending order (n_end once they are exhausted).  The current bitmap word
@@ -355,7 +361,7 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
     // registers -> LDS: K into stage kbuf, the side rows into stage xbuf, V^T into stage vbuf
     auto store_k = [&](int kbuf) {
         if (role_k) {
-            char *sK = smem + SM::OFF_K + kbuf * SM::K_BYTES;
+            char *sK = FWD_LDS + SM::OFF_K + kbuf * SM::K_BYTES;
 #pragma unroll
             for (int it = 0; it < K_IT; it++)
                 *(u32x4_t *)(sK + ((kr0 + it * K_RPP) * SM::SK + kc * 8) * 2) = sreg[it];
@@ -377,12 +383,12 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
             row[1] = pc[1] | (E::pack2(0.f, keep ? 0.f : -INFINITY) & 0xffff0000u);
             row[2] = E::pack2(E::kRefWeight, 1.f);
             row[3] = 0;
-            *(u32x4_t *)(smem + SM::OFF_X + xbuf * SM::X_BYTES + lane * 32) = row;
+            *(u32x4_t *)(FWD_LDS + SM::OFF_X + xbuf * SM::X_BYTES + lane * 32) = row;
         }
     };
     auto store_v = [&](int vbuf) {
         if (role_v && kt < V_ITEMS) {  // transpose 4 keys x 8 d in registers, write V^T[d][key quad]
-            char *sVt = smem + SM::OFF_VT + vbuf * SM::VT_BYTES;
+            char *sVt = FWD_LDS + SM::OFF_VT + vbuf * SM::VT_BYTES;
 #pragma unroll
             for (int dj = 0; dj < 8 * V_IT; dj++) {
                 const int j = dj >> 3, dd = dj & 7, w = dd >> 1;
@@ -422,11 +428,11 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
     constexpr int NQK = KS + 1, NPV = 2 * DB, NF = NQK + NPV;
     constexpr int FR = 4;  // fragment reads run FR MFMAs ahead of their MFMAs (8 ahead: 19 spilled registers)
     auto frag_ptr = [&](int f, int kbuf, int kh, int vbuf, int vh) -> const u32x4_t * {
-        if (f == 0) return (const u32x4_t *)(smem + SM::OFF_X + kbuf * SM::X_BYTES + (32 * kh + a_row) * 32 + g * 16);
+        if (f == 0) return (const u32x4_t *)(FWD_LDS + SM::OFF_X + kbuf * SM::X_BYTES + (32 * kh + a_row) * 32 + g * 16);
         if (f < NQK)
-            return (const u32x4_t *)(smem + SM::OFF_K + kbuf * SM::K_BYTES + ((32 * kh + a_row) * SM::SK + (f - 1) * 16 + g * 8) * 2);
+            return (const u32x4_t *)(FWD_LDS + SM::OFF_K + kbuf * SM::K_BYTES + ((32 * kh + a_row) * SM::SK + (f - 1) * 16 + g * 8) * 2);
         const int kb = (f - NQK) / DB, db = (f - NQK) % DB;
-        return (const u32x4_t *)(smem + SM::OFF_VT + vbuf * SM::VT_BYTES + ((32 * db + a_row) * SM::SVT + 32 * vh + 16 * kb + 8 * g) * 2);
+        return (const u32x4_t *)(FWD_LDS + SM::OFF_VT + vbuf * SM::VT_BYTES + ((32 * db + a_row) * SM::SVT + 32 * vh + 16 * kb + 8 * g) * 2);
     };
     const f32x16_t zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
@@ -514,8 +520,8 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
                     const uint32_t (&pprev)[8], int kbuf, int kh, int vbuf, int vh, Turn j_next, Turn jx_next) {
         constexpr bool STAGE = decltype(stage_c)::value;
         constexpr bool DO_V = STAGE && decltype(do_v_c)::value, DO_K = !STAGE && decltype(do_k_c)::value;
-        char *const sVt_w = smem + SM::OFF_VT + (vbuf ^ 1) * SM::VT_BYTES;  // V(t) goes to the stage the P V product has left
-        char *const sK_w = smem + SM::OFF_K + (kbuf ^ 1) * SM::K_BYTES;     // K(t+2) to the stage whose scores are finished
+        char *const sVt_w = FWD_LDS + SM::OFF_VT + (vbuf ^ 1) * SM::VT_BYTES;  // V(t) goes to the stage the P V product has left
+        char *const sK_w = FWD_LDS + SM::OFF_K + (kbuf ^ 1) * SM::K_BYTES;     // K(t+2) to the stage whose scores are finished
         // Order of issue: a wave issues in program order, so the vector instructions have to sit BETWEEN the MFMAs to run
         // under them.  The step is written slot by slot -- one MFMA, the fragment read of the MFMA FR slots later, an even
         // share of the softmax (the two exp2 of a pair of scores in one slot, their conversion to 16 bits and their
@@ -830,6 +836,7 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
         }
     }
 }
+#undef FWD_LDS
 
 // Adds up the shares of a call with split keys: out = sum_s 2^(l_s - l) O_s, l = log2 sum_s 2^l_s (no share with a visible key:
 // 0 and +inf).  A thread has 8 elements of one row; the rows of O of a share without a visible key hold nothing and are not read.
