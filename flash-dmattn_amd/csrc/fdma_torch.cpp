@@ -15,6 +15,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/TracerMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
@@ -227,7 +228,7 @@ struct AttentionBackward : public Node {
     SavedVariable q_, k_, v_, mask_, bias_, out_, lse_;
     Tensor ws;  // the forward's workspace (lists and compacted copies), which the backward reuses
     SideInputs side;
-    size_t ws_bytes = 0;
+    size_t ws_off = 0, ws_bytes = 0;  // (ws_off: of the workspace in `ws` -- the LSE in front of it, unless it is saved as lse_)
     double scale = 1;
     bool causal = false, deterministic = false, has_mask = false, has_bias = false;
     int compact_mode = 0, stream_min = 0;
@@ -241,7 +242,7 @@ struct AttentionBackward : public Node {
     }
     variable_list apply(variable_list &&grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
-        const Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), out = out_.unpack(shared_from_this()), lse = lse_.unpack();
+        const Tensor q = q_.unpack(), k = k_.unpack(), v = v_.unpack(), out = out_.unpack(shared_from_this()), lse = ws_off ? ws : lse_.unpack();
         const Tensor mask = has_mask ? mask_.unpack() : Tensor(), bias = has_bias ? bias_.unpack() : Tensor();
         if (!grads[0].defined()) return variable_list(has_bias ? 4 : 3);
         at::NoGradGuard no_grad;
@@ -263,7 +264,7 @@ struct AttentionBackward : public Node {
         }
         a.deterministic = deterministic;
         if (ws_bytes && stream_min == api.stream_min_items(0)) {
-            a.fwd_workspace = ws.data_ptr();
+            a.fwd_workspace = (const char *)ws.data_ptr() + ws_off;
             a.fwd_workspace_bytes = ws_bytes;
         }
         const size_t d_bytes = up256((size_t)q.size(0) * q.size(2) * round_up(q.size(1), 128) * 4);
@@ -345,13 +346,16 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     Tensor out = at::empty(q.sizes(), opt);
     fdma_fwd_args a;
     fill_fwd(a, q, k, v, mask, bias, out, nullptr, scale, causal, compact_mode, side);
-    // one buffer for LSE and workspace -- but where a backward will want the LSE, it is a tensor of its own, which the node
-    // saves as autograd does (saved-tensor hooks see it: they may move it off the device until then)
-    const size_t need = api.fwd_workspace_bytes(&a), lse_bytes = is_grad ? 0 : up256((size_t)B * H * Lq * 4);
+    // LSE and workspace in one piece -- except where a backward will want the LSE and there is no workspace to go with it, or
+    // saved-tensor hooks are waiting (they may move it off the device until then): it is a tensor of its own there, which the
+    // node saves as autograd does
+    const size_t need = api.fwd_workspace_bytes(&a);
+    const bool apart = is_grad && (need == 0 || Lq == 1 || !at::SavedTensorDefaultHooks::get_tls_state().stack.empty());
+    const size_t lse_bytes = apart ? 0 : up256((size_t)B * H * Lq * 4);
     Tensor lse, buf;
-    if (is_grad) lse = at::empty({B, H, Lq}, opt.dtype(at::kFloat));
+    if (apart) lse = at::empty({B, H, Lq}, opt.dtype(at::kFloat));
     if (lse_bytes + need) buf = at::empty({(int64_t)(lse_bytes + need)}, bytes);
-    a.lse = (float *)(is_grad ? lse : buf).data_ptr();
+    a.lse = (float *)(apart ? lse : buf).data_ptr();
     void *stream = stream_of(dev);
     if (need) {
         a.workspace = (char *)buf.data_ptr() + lse_bytes;
@@ -372,9 +376,9 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         if ((node->has_mask = mask.defined())) node->mask_ = SavedVariable(mask, false);
         if ((node->has_bias = bias.defined())) node->bias_ = SavedVariable(bias, false);
         node->out_ = SavedVariable(out, true);
-        node->lse_ = SavedVariable(lse, false);
+        if (apart) node->lse_ = SavedVariable(lse, false);
         node->side = side;
-        if (need && Lq > 1) { node->ws = buf; node->ws_bytes = need; }
+        if (need && Lq > 1) { node->ws = buf; node->ws_off = lse_bytes; node->ws_bytes = need; }
         node->scale = scale; node->causal = causal; node->deterministic = deterministic;
         node->compact_mode = compact_mode;
         node->stream_min = api.stream_min_items(0);
