@@ -922,11 +922,12 @@ static bool enough_pairs(const FwdParams &p) {
 //   16384    6.52 5.04 3.42    3.91 2.37 1.15    5.49 3.84 2.41    2.60 1.41 0.69    2.18 1.16 0.60*   1.54 0.79 0.41
 // (* 8192 and 32768 keys; d = 64 alike, d = 256 1.8 to 3.6, 0.95 to 1.9, 0.5 to 0.95).  Forward and backward, the same: 1536 keys
 // 0.8 to 1.1 even with a quarter kept, 3072 keys 1.1 to 1.8, 1.0 to 1.6, 0.7 to 1.2.  So:
-//   * from 3072 keys on, and up to 32 pairs of batch entry and kv head: half of the keys kept gain everywhere;
+//   * from 3072 keys on, and up to 32 pairs of batch entry and kv head: half of the keys kept gain everywhere (1.2 to 8.4;
+//     forward and backward 1.0 to 2.8), all of them range from 0.67 to 5.4;
 //   * copies of up to half a gigabyte: they are as large as the caller's whole K and V, and are held until the backward;
 //   * a mask with one row for all of several kv heads is what padding looks like, which keeps nearly everything: from 4096
 //     keys on, and only where the few blocks let the keys be cut into shares (key_shares), which is ahead with all of them
-//     kept (1.15 to 3.5; forward and backward 0.98 to 1.6).
+//     kept (1.13 to 5.4; forward and backward 0.98 to 1.6).
 constexpr int COMPACT_LONG_KEYS = 3072, COMPACT_LONG_KEYS_PADDING = 4096, COMPACT_LONG_PAIRS = 32;
 constexpr int64_t COMPACT_LONG_BYTES = (int64_t)1 << 29;
 static bool few_rows_many_keys(const FwdParams &p) {

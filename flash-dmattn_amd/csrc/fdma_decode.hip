@@ -238,7 +238,8 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
         }
         if (p.mask && p.Lk >= 16 && (!PERHEAD || p.Hm != p.H)) {
             // ld_row16, with nothing fetched beyond the range and, in a wave without a piece that crosses the end of the row,
-            // no shifts behind the loads (8 x 32 heads over 65536 keys 22.79 -> 22.37 us, 12 x 16 over 50000 -1.8 %, 32 over 2049 10.65 -> 10.28)
+            // no shifts behind the loads: what shifts in every wave cost beside aligned rows, which were all the kernel took once
+            // (8 x 32 heads over 65536 keys 22.79 with them, 22.37 without and with aligned rows alone)
             const uint8_t *row = p.mask + b * p.m_b + (int64_t)(p.Hm == 1 ? 0 : hk) * p.m_h;
             bool cross = false;
 #pragma unroll
