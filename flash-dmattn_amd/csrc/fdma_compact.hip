@@ -914,26 +914,29 @@ static bool enough_pairs(const FwdParams &p) {
 // Few query rows against many keys.  A workgroup of the tile-skipping kernel walks every tile with a kept key, and scattered
 // keys leave hardly any tile without: 1.6 us per 128 keys, whatever the batch, while there are no more row blocks than CUs.  The
 // copies are read, written and read again: their cost grows with batch x kv heads and with the share of the keys that is
-// kept, which the host does not know.  Tile skipping over compaction, 64 rows, d = 128, a quarter / half / all keys kept
-// (batch x query heads / kv heads):
-//   keys     1 x 8/8           4 x 8/8           1 x 32/8          4 x 32/8          4 x 16/16         16 x 8/8
-//   1536     1.42 1.11 0.80    1.30 0.97 0.71    1.45 1.13 0.81    1.33 0.98 0.72                      1.12 0.78 0.51
-//   4096     1.98 2.05 1.58    1.74 1.69 1.21    2.26 1.94 1.51    1.85 1.25 0.76    1.72 0.97 0.50*   1.38 0.71 0.37
-//   16384    6.52 5.04 3.42    3.91 2.37 1.15    5.49 3.84 2.41    2.60 1.41 0.69    2.18 1.16 0.60*   1.54 0.79 0.41
-// (* 8192 and 32768 keys; d = 64 alike, d = 256 1.8 to 3.6, 0.95 to 1.9, 0.5 to 0.95).  Forward and backward, the same: 1536 keys
-// 0.8 to 1.1 even with a quarter kept, 3072 keys 1.1 to 1.8, 1.0 to 1.6, 0.7 to 1.2.  So:
-//   * from 3072 keys on, and up to 32 pairs of batch entry and kv head: half of the keys kept gain everywhere (1.2 to 8.4;
-//     forward and backward 1.0 to 2.8), all of them range from 0.67 to 5.4;
-//   * copies of up to half a gigabyte: they are as large as the caller's whole K and V, and are held until the backward;
-//   * a mask with one row for all of several kv heads is what padding looks like, which keeps nearly everything: from 4096
-//     keys on, and only where the few blocks let the keys be cut into shares (key_shares), which is ahead with all of them
-//     kept (1.13 to 5.4; forward and backward 0.98 to 1.6).
-constexpr int COMPACT_LONG_KEYS = 3072, COMPACT_LONG_KEYS_PADDING = 4096, COMPACT_LONG_PAIRS = 32;
-constexpr int64_t COMPACT_LONG_BYTES = (int64_t)1 << 29;
+// kept, which the host does not know.  Tile skipping over compaction, 16 to 100 rows, d = 128, a sixteenth / quarter / half /
+// three quarters / all of the keys kept (batch x query heads / kv heads; - not measured):
+//   keys        1536                      2048                      4096                      8192                      16384
+//   1 x 8/8     1.97 1.42 1.11 -   0.80   2.13 1.63 1.17 0.94 0.82  2.78 1.98 2.05 -   1.58   -                         7.91 6.52 5.04 -   3.42
+//   1 x 32/8    2.00 1.45 1.13 -   0.81   2.25 1.66 1.20 0.97 0.83  2.74 2.26 1.94 -   1.51   -                         7.73 5.49 3.84 -   2.41
+//   4 x 8/8     1.92 1.30 0.97 -   0.71   2.09 1.44 1.06 0.86 0.74  2.62 1.74 1.69 -   1.21   -                         6.54 3.91 2.37 -   1.15
+//   4 x 32/8    1.94 1.33 0.98 -   0.72   2.20 1.47 1.08 0.86 0.75  3.15 1.85 1.25 -   0.76   -                         6.40 2.60 1.41 -   0.69
+//   4 x 16/16   -                         2.03 1.32 0.98 0.75 0.63  -                         4.07 1.66 0.94 0.65 0.49  6.58 2.42 1.13 0.79 0.60
+//   16 x 8/8    1.73 1.12 0.78 -   0.51   1.80 1.18 0.77 0.57 0.43  2.72 1.38 0.71 -   0.37   4.46 1.58 0.84 0.57 0.43  4.24 1.52 0.79 0.53 0.41
+// d = 64 is alike, d = 256 ahead of both (2048 keys, 4 x 32/8: 4.04 2.18 1.39 1.03 0.84).  Forward and backward: 2048 keys 0.8 to 0.9 at d = 64
+// even with a quarter kept, 1.2 to 1.5 at d = 128; 3072 keys 1.1 to 1.8, half 1.0 to 1.6, all 0.7 to 1.2.  So, where the mask has a row
+// per kv head, as one made from a bias of the kv heads has:
+//   * from 2048 keys on (3072 at d <= 64) up to 32 pairs of batch entry and kv head: ahead up to two thirds of the keys kept;
+//   * from 8192 keys on up to 128 pairs: ahead up to 0.4 to 0.6 of them -- a window that is more than a quarter of such an axis is rare;
+//   * copies of up to a gigabyte: they are as large as the caller's whole K and V, and are held until the backward.
+// A mask with one row for all of several kv heads is what padding looks like, which keeps nearly everything: from 4096 keys on and
+// only where the few blocks let the keys be cut into shares (key_shares), which is ahead with all of them kept (1.13 to 5.4; forward
+// and backward 0.98 to 1.6).
 static bool few_rows_many_keys(const FwdParams &p) {
     const int64_t pairs = (int64_t)p.B * p.Hk;
-    if (p.Lk < COMPACT_LONG_KEYS || p.Lk / 2 < p.Lq || pairs > COMPACT_LONG_PAIRS || pairs * p.Lk * p.d * 4 > COMPACT_LONG_BYTES) return false;
-    return p.Hm == p.Hk || (p.Lk >= COMPACT_LONG_KEYS_PADDING && key_shares(p) > 1);
+    if (p.Lk / 2 < p.Lq || pairs * p.Lk * p.d * 4 > (int64_t)1 << 30) return false;
+    if (p.Hm != p.Hk) return p.Lk >= 4096 && pairs <= 32 && key_shares(p) > 1;
+    return pairs <= 32 ? p.Lk >= (p.d <= 64 ? 3072 : 2048) : p.Lk >= 8192 && pairs <= 128;
 }
 bool compact_for_long_keys(const FwdParams &p) { return p.compact_mode == 0 && use_compact(p) && !enough_pairs(p); }
 bool use_compact(const FwdParams &p) {

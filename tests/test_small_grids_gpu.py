@@ -147,7 +147,8 @@ def test_no_room_for_the_copies_of_a_long_key_axis(per_query_head):
 
 @pytest.mark.parametrize("B,Lq,Lk,H,Hk,D,window,dtype", [
     (1, 100, 4096, 16, 16, 128, 1024, torch.bfloat16),  # 2 groups of dQ workgroups, 128 that sum
-    (1, 2, 3072, 2, 1, 64, 3072, torch.bfloat16),       # the fewest rows and keys, all kept
+    (1, 2, 3072, 2, 1, 64, 3072, torch.bfloat16),       # the fewest rows and keys at d <= 64, all kept
+    (1, 2, 2048, 2, 1, 128, 900, torch.bfloat16),       # ... and above
     (2, 33, 5000, 4, 2, 96, 900, torch.float16),
     (4, 64, 3100, 8, 8, 64, 300, torch.bfloat16),
     (1, 129, 6200, 6, 3, 256, 700, torch.float16),      # two row blocks, one of a single row
