@@ -150,6 +150,7 @@ def test_no_room_for_the_copies_of_a_long_key_axis(per_query_head):
     (1, 2, 3072, 2, 1, 64, 3072, torch.bfloat16),       # the fewest rows and keys at d <= 64, all kept
     (1, 2, 2048, 2, 1, 128, 900, torch.bfloat16),       # ... and above
     (2, 33, 5000, 4, 2, 96, 900, torch.float16),
+    (16, 2, 8192, 8, 8, 64, 1500, torch.bfloat16),      # 128 pairs: more units of keys than there are parts to be made
     (4, 64, 3100, 8, 8, 64, 300, torch.bfloat16),
     (1, 129, 6200, 6, 3, 256, 700, torch.float16),      # two row blocks, one of a single row
     (1, 300, 3073, 32, 8, 64, 2, torch.bfloat16),       # two kept keys (with one, dQ is zero and has no scale to compare against)
