@@ -19,7 +19,7 @@ def _library_decides_compaction():
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu where there is one)")
 
 
 def pytest_collection_modifyitems(config, items):

@@ -4,7 +4,7 @@ Run in the build container only (`python tests/golden/make_mask_vectors.py`): it
 /root/reference/flash_sparse_attn/utils/mask.py by file path (the module needs nothing but torch) and calls
 topk_mask / relu_mask / block_smooth / create_mask on small inputs.  What these functions return is not fixed by a
 closed form in two places -- which of several EQUAL values torch.topk selects, and the in-place block vote -- so the
-outputs are frozen here as data.  The fixture holds inputs and expected masks only; the GPU box never sees the reference.
+outputs are frozen here as data.  The fixture holds inputs and expected masks only; no test needs the reference.
 
 Bias values are small integers, exact in bf16 / fp16 / fp32, so the same fixture serves the fp32 tensor program on
 the CPU and the 16-bit device kernel.  Cases named *_distinct have pairwise different values in every row (the
