@@ -465,6 +465,37 @@ size_t fdma_bwd_workspace_bytes(const fdma_bwd_args *a) {
     return bytes;
 }
 
+// Room for the fp32 sums of dK/dV parts, where the column form works on the original key axis (0: whole units)
+static size_t kv_parts_bytes(fdma::BwdParams &p, size_t *kv) {
+    size_t db = 0;
+    *kv = (size_t)round_up(fdma::plan_kv_parts(p, &db), 256);
+    return *kv + (size_t)round_up(db, 256);
+}
+static bool direct_column_form(const fdma::BwdParams &p) {
+    return p.f.Lq > 0 && p.f.Lk > 0 && !fdma::use_compact(p.f) && fdma::bwd_colmask_applicable(p);
+}
+// hands the room at `ws` to the call when it is enough; without it the units stay whole
+static void take_kv_parts(fdma::BwdParams &p, void *ws, size_t bytes) {
+    size_t kv;
+    const size_t need = kv_parts_bytes(p, &kv);
+    if (p.kv_most > 1 && ws && aligned16(ws) && bytes >= need) {
+        p.dkv_part = static_cast<float *>(ws);
+        p.db_part = reinterpret_cast<float *>(static_cast<char *>(ws) + kv);
+    } else {
+        p.kv_most = 1;
+        p.kv_quota = 0;
+    }
+}
+
+size_t fdma_bwd_optional_bytes(const fdma_bwd_args *a) {
+    if (!a || a->f.num_heads_k <= 0) return 0;
+    fdma::BwdParams p;
+    std::memset(&p, 0, sizeof(p));
+    fill_fwd_params(&a->f, p.f);
+    size_t kv;
+    return direct_column_form(p) ? kv_parts_bytes(p, &kv) : 0;
+}
+
 int fdma_bwd(const fdma_bwd_args *a, void *hip_stream) {
     if (int cap = refuse_capture(hip_stream, "fdma_bwd")) return cap;
     int rc = fdma_bwd_validate(a);
@@ -493,7 +524,8 @@ int fdma_bwd(const fdma_bwd_args *a, void *hip_stream) {
         p.dba_h = nr * lkr;
         p.dba_b = a->f.bias_strides[0] == 0 ? 0 : p.dba_h * a->f.num_heads_bias;
     }
-    p.kv_segs = 1;
+    p.kv_segs = p.kv_most = 1;
+    if (direct_column_form(p)) take_kv_parts(p, a->workspace ? static_cast<char *>(a->workspace) + need : nullptr, a->workspace_bytes - need);
     if (!fdma::use_compact(p.f) && general_form(p.f)) {
         p.kv_segs = fdma::general_kv_segments(p.f);
         size_t db = 0;
@@ -557,7 +589,17 @@ int fdma_varlen_bwd_validate(const fdma_varlen_bwd_args *a) {
     return FDMA_OK;
 }
 
-int fdma_varlen_bwd(const fdma_varlen_bwd_args *a, void *hip_stream) {
+size_t fdma_varlen_bwd_optional_bytes(const fdma_varlen_bwd_args *a) {
+    fdma::BwdParams p;
+    std::memset(&p, 0, sizeof(p));
+    if (validate_varlen(a ? &a->f : nullptr, true) != FDMA_OK || fill_varlen_params(&a->f, p.f) != FDMA_OK) return 0;
+    size_t kv;
+    return kv_parts_bytes(p, &kv);
+}
+
+int fdma_varlen_bwd(const fdma_varlen_bwd_args *a, void *hip_stream) { return fdma_varlen_bwd_ws(a, nullptr, 0, hip_stream); }
+
+int fdma_varlen_bwd_ws(const fdma_varlen_bwd_args *a, void *workspace, size_t workspace_bytes, void *hip_stream) {
     if (int cap = refuse_capture(hip_stream, "fdma_varlen_bwd")) return cap;
     int rc = fdma_varlen_bwd_validate(a);
     if (rc != FDMA_OK) return rc;
@@ -576,6 +618,7 @@ int fdma_varlen_bwd(const fdma_varlen_bwd_args *a, void *hip_stream) {
     // Key rows no query can see get zero dK / dV from the dK/dV kernel itself; with no query rows at all, or no
     // key rows at all, one of the two grids is empty and the other kernel still writes its (zero) outputs.
     if (p.f.Lq == 0 && p.f.Lk == 0) return FDMA_OK;
+    take_kv_parts(p, workspace, workspace_bytes);
     if (!fdma::bwd_colmask_applicable(p))
         return fail(FDMA_ERR_UNSUPPORTED, "ragged batches with sequences of more than 2^19 keys are not supported (max_seqlen_k = %d)", a->f.max_seqlen_k);
     hipStream_t stream = static_cast<hipStream_t>(hip_stream);

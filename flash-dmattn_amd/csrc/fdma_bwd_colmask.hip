@@ -73,22 +73,53 @@ template <int D> struct KvcSmem {
 // at 256 are at the end of their registers (772 bytes of scratch per lane) and keep the plain order.
 template <int D> constexpr bool RAGGED_TURNS = D <= 128;
 
-// Entry of a ragged batch that the dK/dV kernel works on in turn `i`: the one with the most query rows first, equal ones in
-// their order.  A block of keys walks the rows of its entry; workgroups start in the order of their ids, and one of a long
-// entry that starts last runs on alone.  16384 tokens in entries of 1 to 5394, the longest last, 32 heads over 8, head
-// dim 128: 1396 -> 1247 us.  Ranks come from one comparison per entry and lane; a batch of more entries than a wave
-// has lanes keeps its order (its units are many and small enough to even out).
-__device__ inline int ragged_turn(const FwdParams &p, int i) {
-    if (p.B > 64) return i;
+// Unit `u` of a kv head's units in a ragged batch: the blocks of 128 keys of its entries, the entry with the most query rows
+// first, equal ones in their order.  A block of keys walks the rows of its entry; workgroups start in the order of their ids, and
+// one of a long entry that starts last runs on alone.  16384 tokens in entries of 1 to 5394, the longest last, 32 heads over 8,
+// head dim 128: 1396 -> 1247 us.  Ranks and first units come from one comparison per entry and lane; a batch of more entries than a
+// wave has lanes keeps its order (its units are many and small enough to even out).  Units beyond the last: block < 0.
+struct RaggedUnit {
+    int entry, block;
+};
+__device__ inline RaggedUnit ragged_unit(const FwdParams &p, int u) {
     const int lane = (int)(threadIdx.x & 63);
-    const int len = lane < p.B ? p.cu_q[lane + 1] - p.cu_q[lane] : -1;
-    int rank = 0;
-    for (int t = 0; t < p.B; t++) {
-        const int other = __builtin_amdgcn_readlane(len, t);
-        rank += (other > len || (other == len && t < lane)) ? 1 : 0;
+    if (p.B > 64) {  // (entry b's units start at cu_k[b] / 128 + b: kv_unit_slot)
+        int e = -1;
+        for (int base = 0; base < p.B; base += 64) {
+            const int b = base + lane;
+            e += __popcll(__ballot(b < p.B && p.cu_k[b] / KV_BN + b <= u));
+        }
+        const int len = p.cu_k[e + 1] - p.cu_k[e], n = u - (p.cu_k[e] / KV_BN + e);
+        return {e, n * KV_BN < len ? n : -1};
     }
-    const uint64_t at = __ballot(lane < p.B && rank == i);
-    return at ? __builtin_ctzll(at) : i;
+    const int b = lane < p.B ? lane : 0, len = lane < p.B ? p.cu_q[b + 1] - p.cu_q[b] : -1;
+    const int n = lane < p.B ? (p.cu_k[b + 1] - p.cu_k[b] + KV_BN - 1) / KV_BN : 0;
+    int first = 0;
+    for (int t = 0; t < p.B; t++) {
+        const int other = __builtin_amdgcn_readlane(len, t), nt = __builtin_amdgcn_readlane(n, t);
+        first += (other > len || (other == len && t < lane)) ? nt : 0;
+    }
+    const uint64_t at = __ballot(u >= first && u < first + n);
+    if (!at) return {0, -1};
+    const int e = __builtin_ctzll(at);
+    return {e, u - __builtin_amdgcn_readlane(first, e)};
+}
+
+// Steps per part of a ragged batch (kv_part_quota of all its units' steps): every lane takes entries, the wave adds up.
+__device__ inline int ragged_part_quota(const FwdParams &p, int bm) {
+    int64_t sum = 0;
+    for (int b = (int)(threadIdx.x & 63); b < p.B; b += 64)
+        sum += kv_head_steps(p.cu_q[b + 1] - p.cu_q[b], p.cu_k[b + 1] - p.cu_k[b], p.causal, bm);
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) sum += __shfl_xor((long long)sum, m);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)sum), hi = __builtin_amdgcn_readfirstlane((uint32_t)(sum >> 32));
+    return kv_part_quota((int64_t)(((uint64_t)hi << 32) | lo) * p.H);
+}
+// Where the sums of a unit's parts lie: unit number within the call (times kv_most).  Ragged: entry b's blocks start at
+// cu_k[b] / 128 + b, which leaves every entry the blocks it has.
+__device__ inline int kv_unit_slot(const BwdParams &p, int b, int hk, int n_block) {
+    const int u = p.f.cu_q ? hk * p.kv_units + p.f.cu_k[b] / KV_BN + b + n_block : (b * p.f.Hk + hk) * p.kv_units + n_block;
+    return u * p.kv_most;
 }
 
 // CMP: the key axis is the compacted list of kept columns (fdma_compact.hip); a lane still owns one key,
@@ -120,7 +151,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
     const int G = f.H / f.Hk;
     // work item: a 128-key block of one (batch, kv head) pair, over query heads [g_lo, g_hi) and segment
     // `seg` of `Sm` of the query range; `slot` >= 0 when the block is shared by several workgroups
-    int pair, n_block, g_lo = 0, g_hi = G, seg = 0, Sm = 1, Q = 1 << 30, slot = -1;
+    int pair, n_block, g_lo = 0, g_hi = G, seg = 0, Sm = 1, Q = 1 << 30, slot = -1, part = 0;
     if (CMP) {
         const int32_t *plan = f.cmp.plan;
         const int Gs = plan[1];
@@ -162,11 +193,31 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
     } else {
         const int n_nb = (f.Lk + KV_BN - 1) / KV_BN;
         const bool ragged = RAGGED_TURNS<D> && f.cu_q;
-        const XcdMap wm = xcd_map(blockIdx.x, ragged ? ragged_lists_per_pair(f) : xcd_lists_per_pair(f.B * f.Hk), n_nb, 1);
+        const int k = ragged ? ragged_lists_per_pair(f) : xcd_lists_per_pair(f.B * f.Hk), n_units = ragged ? p.kv_units : n_nb;
+        XcdMap wm;
+        if (p.kv_most > 1) {
+            // A list holds its units once per part, the LAST parts first: those exist for the longest units only.  Workgroups
+            // side by side go to the shader engines of an XCD in turn, whether they stay or return at once: with the parts of
+            // a unit side by side instead, the engines that got the missing ones idled (ragged, 16384 tokens, two parts at
+            // most: 1966 us instead of 1224 without parts).
+            const int per_list = (n_units + k - 1) / k, pos = (int)(blockIdx.x / 8) % (per_list * p.kv_most);
+            part = p.kv_most - 1 - pos / per_list;
+            const int vlist = (int)(blockIdx.x % 8) + 8 * ((int)(blockIdx.x / 8) / (per_list * p.kv_most));
+            wm.pair = vlist / k;
+            wm.unit = pos % per_list * k + vlist % k;
+            wm.valid = wm.unit < n_units;
+        } else {
+            wm = xcd_map(blockIdx.x, k, n_units, 1);
+        }
         if (!wm.valid) return;
         n_block = wm.unit;  // low key blocks are seen by the most queries under causal: heaviest first
         pair = wm.pair;
-        if (ragged) pair = ragged_turn(f, pair / f.Hk) * f.Hk + pair % f.Hk;
+        if (ragged) {
+            const RaggedUnit ru = ragged_unit(f, n_block);
+            if (ru.block < 0 || ru.block >= n_nb) return;  // (rows beyond the longest length that the caller names: not computed)
+            n_block = ru.block;
+            pair = ru.entry * f.Hk + wm.pair;
+        }
     }
     const int b = pair / f.Hk, hk = pair % f.Hk;
     const int n0 = n_block * KV_BN;
@@ -174,6 +225,18 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
     const int LqS = sq.Lq, LkS = sq.Lk;
     const int Lk = CMP ? f.cmp.count[pair] : LkS;  // key columns on this pair's (possibly compacted) key axis
     if (n0 >= Lk) return;  // the compacted list, or a shorter sequence of a ragged batch, ends before this block
+    // original key axis: this part's steps [first_step, first_step + part_steps) of the unit's
+    int first_step = 0, part_steps = 0;
+    if (!CMP && p.kv_most > 1) {
+        const int steps = G * kv_unit_steps(LqS, LkS, CAUSAL, n0, BM);
+        const int n_parts = kv_parts_of(steps, p.kv_quota ? p.kv_quota : ragged_part_quota(f, BM), p.kv_most);
+        if (part >= n_parts) return;
+        if (n_parts > 1) {
+            first_step = (int)((int64_t)steps * part / n_parts);
+            part_steps = (int)((int64_t)steps * (part + 1) / n_parts) - first_step;
+            slot = kv_unit_slot(p, b, hk, n_block) + part;
+        }
+    }
     const int key = n0 + wave * 32 + r;  // the key column this lane owns
     const int key_c = key < Lk ? key : Lk - 1;
     const int shift = LkS - LqS;
@@ -218,7 +281,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
     const int m_start = M_blocks - dkdv_query_blocks(LqS, LkS, CAUSAL, okey_first);
     // this workgroup's query blocks [m_lo, m_hi): all of them, or one of the unit's equal segments
     int m_lo = m_start, m_hi = M_blocks;
-    if (slot >= 0) {
+    if (CMP && slot >= 0) {
         const int n_seg = dkdv_segments(M_blocks - m_start, Q, Sm);
         if (seg >= n_seg) return;  // the reduce kernel knows that this slot stays unwritten
         const int len = (M_blocks - m_start + n_seg - 1) / n_seg;
@@ -232,7 +295,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
     // (g outer, m inner); the query blocks are walked from the LAST one down, so that the
     // workgroups of one (batch, kv head) pair, which run side by side on an XCD, all begin at the same
     // Q / dO tile and stream the same tiles at the same time (L2 hits instead of re-fetches)
-    const int n_steps = n_m * (g_hi - g_lo);
+    const int n_steps = !CMP && slot >= 0 ? part_steps : n_m * (g_hi - g_lo);
 
     const bool has_bias = f.bias != nullptr;
     const bool use_accum = p.dbias_accum != nullptr;
@@ -299,7 +362,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
     };
     // everything of a step's fetch except the tile loads: block bases, column constant, row statistics
     auto load_step = [&](int step, bool with_tiles) {
-        const int gi = g_lo + step / n_m, mi = s_hi - 1 - step % n_m;  // last query block first: see below
+        const int gi = g_lo + (step + first_step) / n_m, mi = s_hi - 1 - (step + first_step) % n_m;  // last query block first: see below
         const int h = hk * G + gi, m0 = mi * BM;
         column_const_load(h);
         ld_qbase = uniform_ptr((const uint16_t *)f.q + b * f.q_b + h * f.q_h + (sq.q0 + m0) * f.q_r);
@@ -342,14 +405,15 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
     // The steps are walked with counters and running pointers (no division, no 64-bit products per step): inside a
     // query head the query block index falls by one per step, at a head change everything jumps by loop constants.
     typedef const __attribute__((address_space(1))) char *gbytes_t;
-    int dma_gi = g_lo, dma_mi = s_hi - 1;  // head and query block of the step being fetched
+    const int gi0 = CMP || n_steps == 0 ? g_lo : first_step / n_m, mi0 = s_hi - 1 - (CMP || n_steps == 0 ? 0 : first_step % n_m);
+    int dma_gi = gi0, dma_mi = mi0;  // head and query block of the step being fetched
     gbytes_t dma_q = nullptr, dma_do = nullptr, dma_stat = nullptr;  // its Q / dO block bases, this lane's statistic
     char *dma_dst = nullptr;
     const int64_t q_step = -(int64_t)BM * f.q_r * 2, do_step = -(int64_t)BM * p.do_r * 2;
     const int64_t q_head = (int64_t)f.q_h * 2 - (int64_t)(n_m - 1) * q_step, do_head = (int64_t)p.do_h * 2 - (int64_t)(n_m - 1) * do_step;
     const int64_t stat_head = (int64_t)(lane < 32 ? f.lse_h : p.sd_h) * 4 + (int64_t)(n_m - 1) * BM * 4;
     if (DMA && n_steps > 0) {
-        const int h0 = hk * G + g_lo, m00 = dma_mi * BM;
+        const int h0 = hk * G + gi0, m00 = dma_mi * BM;
         dma_q = (gbytes_t)((const uint16_t *)f.q + b * f.q_b + h0 * f.q_h + (sq.q0 + m00) * f.q_r);
         dma_do = (gbytes_t)((const uint16_t *)p.dout + b * p.do_b + h0 * p.do_h + (sq.q0 + m00) * p.do_r);
         dma_stat = (gbytes_t)(lane < 32 ? f.lse + b * f.lse_b + h0 * f.lse_h + sq.q0 + m00 + (lane & 31)
@@ -424,7 +488,7 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
     // CU's address unit while the matrix pipe idles).
     if (n_steps > 0) {
         if constexpr (DMA) {
-            column_const_load(hk * G + g_lo);
+            column_const_load(hk * G + gi0);
             dma_begin(0);
 #pragma unroll
             for (int n = 0; n <= 2 * Q_IT; n++) dma_piece(n);
@@ -439,12 +503,13 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
         publish();
     }
 
-    int cur_gi = g_lo, cur_mi = s_hi - 1;  // (DMA: head and query block of the current step, walked like the fetch)
+    int cur_gi = gi0, cur_mi = mi0;  // (DMA: head and query block of the current step, walked like the fetch)
     // (one step; the LDS stage is a compile-time constant -- the loop below runs the steps in pairs -- so that every
     // stage base folds into the offset field of the LDS instructions instead of costing an addition per access)
     auto one_step = [&](auto buf_c, const int step) {
         constexpr int buf = decltype(buf_c)::value;
-        const int gi = DMA ? cur_gi : g_lo + step / n_m, mi = DMA ? cur_mi : s_hi - 1 - step % n_m;  // last query block first: see below
+        const int gi = DMA ? cur_gi : g_lo + (step + first_step) / n_m;  // last query block first: see below
+        const int mi = DMA ? cur_mi : s_hi - 1 - (step + first_step) % n_m;
         const int h = hk * G + gi;
         const int m0 = mi * BM;
         // The swizzled addresses are these lane constants XOR a compile-time value: recomputed where they are used
@@ -626,12 +691,13 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
 
         // ---- dBias column sum: flush when the bias head changes
         if (has_bias) {
-            const bool last_m = mi == s_lo;
-            if (last_m && (slot >= 0 || f.Hb == f.H || gi == G - 1)) {
+            // (a part: its own last step too; one sum for all its heads where they share the bias)
+            const bool part_end = !CMP && slot >= 0 && step == n_steps - 1;
+            if ((mi == s_lo && ((CMP && slot >= 0) || f.Hb == f.H || (gi == G - 1 && slot < 0))) || part_end) {
                 const float tot = xhalf_sum(colsum);
                 const int hb = f.Hb == f.H ? h : (f.Hb == 1 ? 0 : hk);
                 if (slot >= 0) {  // per-head partial column sums; the reduce kernel folds them
-                    if (g == 0) p.db_part[((int64_t)slot * G + (gi - g_lo)) * KV_BN + (key - n0)] = tot;
+                    if (g == 0) p.db_part[((int64_t)slot * G + (CMP || f.Hb == f.H ? gi - g_lo : 0)) * KV_BN + (key - n0)] = tot;
                 } else if (g == 0 && key < Lk) {
                     if (use_accum) atomicAdd(p.dbias_accum + b * p.dba_b + hb * p.dba_h + okey, tot);
                     else ((uint16_t *)p.dbias)[b * p.db_b + hb * p.db_h + okey] = (uint16_t)(E::pack2(tot, 0.f) & 0xffffu);
@@ -666,8 +732,26 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
         }
     }
 
+    // ---- a part: fp32 sums in the order the lanes hold them (1 KB per store); heads without a step in it have zero columns
+    if (!CMP && slot >= 0) {
+        if (has_bias && f.Hb == f.H && g == 0) {
+            const int g_end = (first_step + part_steps - 1) / n_m;
+            for (int gh = 0; gh < G; gh++)
+                if (gh < gi0 || gh > g_end) p.db_part[((int64_t)slot * G + gh) * KV_BN + (key - n0)] = 0.f;
+        }
+        f32x4_t *dst = (f32x4_t *)p.dkv_part + (int64_t)slot * (2 * KV_BN * D / 4) + wave * DB * 4 * 64 + lane;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int at = (db * 4 + q) * 64;
+                dst[at] = f32x4_t{dk[db][4 * q], dk[db][4 * q + 1], dk[db][4 * q + 2], dk[db][4 * q + 3]};
+                dst[at + KV_BN * D / 4] = f32x4_t{dv[db][4 * q], dv[db][4 * q + 1], dv[db][4 * q + 2], dv[db][4 * q + 3]};
+            }
+        return;
+    }
     // ---- shared block: fp32 partial dK^T / dV^T, [which][d][key] so that a wave writes 128-byte runs
-    if (slot >= 0) {
+    if (CMP && slot >= 0) {
         float *pk = p.dkv_part + (int64_t)slot * 2 * D * KV_BN + (key - n0);
 #pragma unroll
         for (int db = 0; db < DB; db++)
@@ -700,6 +784,70 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
                     *(u32x4_t *)(dvp + c) = wv;
                 }
             }
+    }
+}
+
+// Sums of the parts on the original key axis, in part order, to dK (scaled), dV and dBias.  Thread (matrix, wave, d block, half,
+// lane) of a unit owns the eight head-dim elements that lane held in its register block; a workgroup takes every gridDim-th piece
+// of 256 such threads.
+template <typename T, int D>
+__global__ void __launch_bounds__(NTHREADS) bwd_dkdv_parts_sum_kernel(const BwdParams p) {
+    using E = Elem<T>;
+    constexpr int DB = D / 32, PER = KV_BN * D, BPU = 2 * PER / 8 / NTHREADS;  // floats of one matrix of a part, pieces per unit
+    const FwdParams &f = p.f;
+    const int G = f.H / f.Hk, bm = KvcSmem<D>::BM;
+    const int n_nb = (f.Lk + KV_BN - 1) / KV_BN;
+    const int units = (f.cu_q ? 1 : f.B) * f.Hk * p.kv_units;
+    const int quota = p.kv_quota ? p.kv_quota : ragged_part_quota(f, bm);
+    for (int item = (int)blockIdx.x; item < units * BPU; item += (int)gridDim.x) {
+        const int unit = item / BPU, piece = item % BPU;
+        int n_block = unit % p.kv_units, hk = unit / p.kv_units, b = 0;
+        if (f.cu_q) {
+            const RaggedUnit ru = ragged_unit(f, n_block);
+            b = ru.entry;
+            n_block = ru.block;
+        } else {
+            b = hk / f.Hk;
+            hk = hk % f.Hk;
+        }
+        const SeqInfo sq = seq_info(f, b);
+        const int n0 = n_block * KV_BN;
+        if (n_block < 0 || n_block >= n_nb || n0 >= sq.Lk) continue;
+        const int n = kv_parts_of(G * kv_unit_steps(sq.Lq, sq.Lk, f.causal, n0, bm), quota, p.kv_most);
+        if (n == 1) continue;  // (the dK/dV kernel wrote the results itself)
+        const int slot = kv_unit_slot(p, b, hk, n_block);
+        const int t = piece * NTHREADS + threadIdx.x;
+        const int lane = t & 63, w = t >> 6;  // w = ((mat * 4 + wave) * DB + db) * 2 + blk
+        const int blk = w & 1, db = (w >> 1) % DB, kw = (w >> 1) / DB % 4, mat = (w >> 1) / DB / 4;
+        const float *src = p.dkv_part + (int64_t)slot * 2 * PER + mat * PER + (((kw * DB + db) * 4 + 2 * blk) * 64 + lane) * 4;
+        f32x4_t a0 = {0, 0, 0, 0}, a1 = {0, 0, 0, 0};
+#pragma unroll 4
+        for (int i = 0; i < n; i++) {
+            const float *q = src + (int64_t)i * 2 * PER;
+            a0 += *(const f32x4_t *)q;
+            a1 += *(const f32x4_t *)(q + 256);
+        }
+        const int key = n0 + kw * 32 + (lane & 31), c = 32 * db + 16 * blk + 8 * (lane >> 5);
+        if (key < sq.Lk && c < f.d) {
+            const float m = mat == 0 ? f.scale : 1.f;
+            const u32x4_t o = {E::pack2(a0[0] * m, a0[1] * m), E::pack2(a0[2] * m, a0[3] * m), E::pack2(a1[0] * m, a1[1] * m), E::pack2(a1[2] * m, a1[3] * m)};
+            uint16_t *dst = mat == 0 ? (uint16_t *)p.dk + b * p.dk_b + (sq.k0 + key) * p.dk_r + hk * p.dk_h
+                                     : (uint16_t *)p.dv + b * p.dv_b + (sq.k0 + key) * p.dv_r + hk * p.dv_h;
+            *(u32x4_t *)(dst + c) = o;
+        }
+        // columns of dBias: two query heads per piece where every head has its own, else one sum for all
+        const int ngh = f.Hb == f.H ? G : 1, kk = (int)threadIdx.x & (KV_BN - 1), half = (int)threadIdx.x / KV_BN;
+        if (f.bias && n0 + kk < sq.Lk) {
+            for (int gh = 2 * piece + half; gh < ngh; gh += 2 * BPU) {
+                const float *cp = p.db_part + ((int64_t)slot * G + gh) * KV_BN + kk;
+                float tot = 0.f;
+#pragma unroll 4
+                for (int i = 0; i < n; i++) tot += cp[(int64_t)i * G * KV_BN];
+                const int hb = f.Hb == f.H ? hk * G + gh : (f.Hb == 1 ? 0 : hk);
+                if (p.dbias_accum) atomicAdd(p.dbias_accum + b * p.dba_b + hb * p.dba_h + n0 + kk, tot);
+                else ((uint16_t *)p.dbias)[b * p.db_b + hb * p.db_h + n0 + kk] = (uint16_t)(E::pack2(tot, 0.f) & 0xffffu);
+            }
+        }
     }
 }
 
@@ -851,9 +999,13 @@ hipError_t launch_dkdv_c(const BwdParams &p, hipStream_t stream) {
         hipLaunchKernelGGL(kern, dim3(grid), dim3(NTHREADS), smem, stream, p);
         return hipGetLastError();  // (the partial results are summed by workgroups of the dQ launch)
     }
-    const int lists = RAGGED_TURNS<D> && f.cu_q ? ragged_lists_per_pair(f) : xcd_lists_per_pair(f.B * f.Hk);
-    dim3 grid(xcd_grid(f.B * f.Hk, lists, (f.Lk + KV_BN - 1) / KV_BN, 1));
+    const int n_nb = (f.Lk + KV_BN - 1) / KV_BN;
+    const bool ragged = RAGGED_TURNS<D> && f.cu_q;  // (a kv head's units are numbered over all entries)
+    dim3 grid(ragged ? xcd_grid(f.Hk, ragged_lists_per_pair(f), p.kv_units, p.kv_most) : xcd_grid(f.B * f.Hk, xcd_lists_per_pair(f.B * f.Hk), n_nb, p.kv_most));
     hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
+    if ((e = hipGetLastError()) != hipSuccess || p.kv_most <= 1) return e;
+    const int64_t pieces = (int64_t)(ragged ? 1 : f.B) * f.Hk * p.kv_units * (2 * KV_BN * D / 8 / NTHREADS);
+    hipLaunchKernelGGL((bwd_dkdv_parts_sum_kernel<T, D>), dim3((unsigned)(pieces < 2048 ? pieces : 2048)), dim3(NTHREADS), 0, stream, p);
     return hipGetLastError();
 }
 template <typename T, int D, bool CAUSAL>
@@ -1416,6 +1568,47 @@ bool bwd_colmask_applicable(const BwdParams &p) {
     const bool mask_ok = !p.f.mask || p.f.m_r == 0;
     const bool bias_ok = !p.f.bias || p.f.bi_r == 0;
     return mask_ok && bias_ok && (p.f.Lk + 63) / 64 <= MAX_TILES;
+}
+
+// Parts of the units on the original key axis.  A call has a workgroup per 128 keys of a kv head, whose steps -- query blocks
+// times grouped heads -- follow each other: a call of few heads takes what its first block takes, 1.2 us a step (d = 128; two
+// workgroups on a CU 2 us), with most of the chip idle.  A part costs its start and its sums, written and read again (128 KB
+// at d = 128) and the call the launch that adds them up (5 us):
+// steps per part grow with the square root of the call's steps.  Measured, dK/dV with its sums, whole / rule / best of 13 quotas (us):
+//   d = 128: 1 x 672 x 16/4 heads 110 / 31.6 / 30.8, 1 x 563 x 8/2 96 / 25.5 / 24.2, 4 x 302 x 32/8 62 / 39 / 36, 1 x 1000 x 8/8 47 / 29.6 / 29.6,
+//   not causal 1 x 400 x 32/8 68 / 32.6 / 32.4; ragged, d = 96: 9 entries up to 5397 x 8/2 742 / 288 / 280, 6 up to 4664 x 2/1 323 / 77 / 64;
+//   d = 128, 4 x 2048 x 32/8 417 / 383 / 368; d = 64, 4096 x 32/8 414 / 225 / 218, 962 x 8/4 55 / 24.6 / 22.9.
+// Whole where there are 2.5 units per CU (16384 ragged tokens x 32/8: 1175 whole, 1258 to 1286 in parts of 96 to 140 steps), and, from
+// half a unit per CU on, where the longest is not two and a half parts (1 x 700 x 32/32: 36.5 whole, 39 to 42 cut; d = 64,
+// 2 x 1000 x 16/16: 35.6 and 41 to 49).  Whole up to 20 steps: 25 us at most, and the call is bound by the host, to which a launch
+// more is 2.5 us (256 x 2/1, d = 64, forward and backward: 72.8 whole, 75.5 cut).  At most 16 parts, and 2048 places for sums (256 MB at d = 128).
+size_t plan_kv_parts(BwdParams &p, size_t *db_bytes) {
+    const FwdParams &f = p.f;
+    p.kv_most = 1;
+    p.kv_quota = 0;
+    p.kv_units = f.cu_q ? f.total_k / KV_BN + f.B : (f.Lk + KV_BN - 1) / KV_BN;
+    *db_bytes = 0;
+    if (f.Lq <= 0 || f.Lk <= 0 || f.cmp.on || (f.cu_q && f.d > 128)) return 0;
+    const int G = f.H / f.Hk, bm = kv_step_rows(f.d);
+    const int64_t longest = (int64_t)G * kv_unit_steps(f.Lq, f.Lk, f.causal, 0, bm);
+    const int64_t units = (int64_t)(f.cu_q ? 1 : f.B) * f.Hk * p.kv_units;
+    int64_t total;
+    if (f.cu_q) {  // (at least: the longest entry, and the other rows in entries of one length)
+        const int rest = f.B > 1 ? f.B - 1 : 1, rq = (f.total_q - f.Lq) / rest, rk = (f.total_k - f.Lk) / rest;
+        total = (kv_head_steps(f.Lq, f.Lk, f.causal, bm) + (f.B > 1 ? rest * kv_head_steps(rq, rk, f.causal, bm) : 0)) * f.H;
+    } else {
+        total = kv_head_steps(f.Lq, f.Lk, f.causal, bm) * f.H * f.B;
+    }
+    const int quota = kv_part_quota(total), cus = device_cus();
+    int64_t most = kv_parts_of((int)(longest < (1 << 30) ? longest : 1 << 30), quota, 16);
+    if (longest <= 20 || units >= cus * 5 / 2 || (units >= cus / 2 && 2 * longest <= 5 * (int64_t)quota)) most = 1;
+    if (most * units > 2048) most = 2048 / units;
+    if (most <= 1) return 0;
+    if (!f.cu_q) p.kv_quota = quota;
+    p.kv_most = (int32_t)most;
+    const int dpad = f.d <= 64 ? 64 : (f.d <= 128 ? 128 : 256);
+    if (f.bias) *db_bytes = (size_t)units * most * G * KV_BN * sizeof(float);
+    return (size_t)units * most * 2 * dpad * KV_BN * sizeof(float);
 }
 
 hipError_t launch_bwd_dkdv_colmask(const BwdParams &p, int dtype, hipStream_t stream) {

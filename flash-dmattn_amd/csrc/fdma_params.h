@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <cmath>
 
 namespace fdma {
 
@@ -101,6 +102,36 @@ __host__ __device__ inline int dkdv_list_of(int u, int k) {
 }
 __host__ __device__ inline int dkdv_list_len(int units_in_largest_pair, int k) {
     return 2 * ((units_in_largest_pair + 2 * k - 1) / (2 * k));
+}
+
+constexpr int KV_PART_MIN = 4, KV_PART_TRADE = 18;  // see plan_kv_parts
+// dK/dV kernel on the original key axis (no compaction; ragged batches): a unit is one 128-key block of a (batch, kv head) pair,
+// its steps are the query blocks of `bm` rows that see it, query head after query head.  A unit of many steps is cut into parts of
+// about `quota` steps, which leave fp32 sums that a launch of its own adds up in part order.
+__host__ __device__ inline int kv_step_rows(int d) { return d <= 64 ? 64 : 32; }
+// steps per query head of the unit whose first key is n0 (the kernel walks planning blocks of 64 rows from the first that sees it)
+__host__ __device__ inline int kv_unit_steps(int Lq, int Lk, int causal, int n0, int bm) {
+    const int blocks = (Lq + 63) / 64, first = blocks - dkdv_query_blocks(Lq, Lk, causal, n0);
+    const int steps = (Lq + bm - 1) / bm - first * (64 / bm);
+    return steps > 0 ? steps : 0;
+}
+// all steps of one query head's units (exact without a causal mask and for Lq == Lk up to the rounding of blocks)
+__host__ __device__ inline int64_t kv_head_steps(int Lq, int Lk, int causal, int bm) {
+    const int64_t n = (Lk + 127) / 128, most = kv_unit_steps(Lq, Lk, causal, 0, bm), least = n > 0 ? kv_unit_steps(Lq, Lk, causal, (int)(n - 1) * 128, bm) : 0;
+    return n * (most + least) / 2;
+}
+// Steps per part when a call's units have `total` steps together: the square root of total / KV_PART_TRADE, rounded up.
+__host__ __device__ inline int kv_part_quota(int64_t total) {
+    const int64_t x = (total + KV_PART_TRADE - 1) / KV_PART_TRADE;
+    int64_t q = (int64_t)sqrtf((float)x);
+    while (q * q < x) q++;
+    while (q > 1 && (q - 1) * (q - 1) >= x) q--;  // (the same on the host and on the device, whatever their square roots round to)
+    return (int)(q < KV_PART_MIN ? KV_PART_MIN : q);
+}
+__host__ __device__ inline int kv_parts_of(int steps, int quota, int most) {
+    if (steps <= quota + (quota >> 2)) return 1;
+    const int n = (steps + quota - 1) / quota;
+    return n < most ? n : most;
 }
 
 struct FwdParams {
@@ -200,6 +231,10 @@ struct BwdParams {
     // columns).  Compacted dK/dV kernel, split mode: per part [2][Dpad][128] fp32 (dK^T, dV^T) and [G][128] fp32 (dBias)
     float *dkv_part;
     float *db_part;
+    // dK/dV on the original key axis, cut into parts: most parts of a unit (1 = no cut), steps per part (0: ragged, from the
+    // lengths on the device), units per (batch, kv head) pair -- ragged: per kv head.  Per part [2][Dpad][128] fp32 (dK, dV, in
+    // register order) in dkv_part and [G][128] fp32 (dBias columns) in db_part
+    int32_t kv_most, kv_quota, kv_units;
     int32_t dot_done;          // softmax_d has been computed by an earlier launch of this call
     int32_t red_octets, red_period, red_start;  // compacted backward: workgroups of the dQ launch that sum the dK/dV partials (set by that launch)
 };
@@ -293,6 +328,9 @@ hipError_t launch_bwd(const BwdParams &p, int dtype, hipStream_t stream);
 bool bwd_colmask_applicable(const BwdParams &p);
 hipError_t launch_bwd_dkdv_colmask(const BwdParams &p, int dtype, hipStream_t stream);
 hipError_t launch_bwd_dq_colmask(const BwdParams &p, int dtype, hipStream_t stream);
+// parts the units of the dK/dV kernel on the original key axis are cut into: fills kv_most / kv_quota / kv_units and returns the
+// bytes of their sums (0: whole); *db_bytes: of their dBias columns
+size_t plan_kv_parts(BwdParams &p, size_t *db_bytes);
 // dQ from the dS tiles that the general dK/dV kernel has written as dBias (a per-query bias with a row per query head
 // and batch entry, dBias written directly): one tile GEMM and no second pass over mask, bias, Q, V, dO
 bool bwd_dq_from_ds_applicable(const BwdParams &p);

@@ -45,10 +45,12 @@ struct Api {
     decltype(&::fdma_bwd) bwd;
     decltype(&::fdma_fwd_workspace_bytes) fwd_workspace_bytes;
     decltype(&::fdma_bwd_workspace_bytes) bwd_workspace_bytes;
+    decltype(&::fdma_bwd_optional_bytes) bwd_optional_bytes;
     decltype(&::fdma_fwd_counter_bytes) fwd_counter_bytes;
     decltype(&::fdma_set_stream_min_items) stream_min_items;
     decltype(&::fdma_varlen_fwd) varlen_fwd;
-    decltype(&::fdma_varlen_bwd) varlen_bwd;
+    decltype(&::fdma_varlen_bwd_ws) varlen_bwd_ws;
+    decltype(&::fdma_varlen_bwd_optional_bytes) varlen_bwd_optional_bytes;
     decltype(&::fdma_create_mask) create_mask;
     decltype(&::fdma_dyn_bias_fwd) dyn_bias_fwd;
     decltype(&::fdma_dyn_bias_bwd) dyn_bias_bwd;
@@ -268,7 +270,7 @@ struct AttentionBackward : public Node {
             a.fwd_workspace_bytes = ws_bytes;
         }
         const size_t d_bytes = up256((size_t)q.size(0) * q.size(2) * round_up(q.size(1), 128) * 4);
-        const size_t need = api.bwd_workspace_bytes(&a);
+        const size_t need = api.bwd_workspace_bytes(&a) + api.bwd_optional_bytes(&a);
         Tensor scratch = at::empty({(int64_t)(d_bytes + need)}, opt.dtype(at::kByte));
         a.softmax_d = (float *)scratch.data_ptr();
         if (need) {
@@ -438,7 +440,10 @@ struct VarlenBackward : public Node {
         for (int i = 0; i < 4; i++) { dst[i][0] = src[i]->stride(0); dst[i][1] = src[i]->stride(1); }
         a.softmax_d = (float *)softmax_d.data_ptr();
         a.deterministic = deterministic;
-        check(api.varlen_bwd(&a, stream_of(q.get_device())));
+        const size_t room = api.varlen_bwd_optional_bytes(&a);
+        Tensor scratch;
+        if (room) scratch = at::empty({(int64_t)room}, opt.dtype(at::kByte));
+        check(api.varlen_bwd_ws(&a, room ? scratch.data_ptr() : nullptr, room, stream_of(q.get_device())));
         return {std::move(dq), std::move(dk), std::move(dv)};
     }
 };
@@ -697,9 +702,11 @@ PyObject *bind(PyObject *, PyObject *dict) {
     FDMA_BIND(bwd);
     FDMA_BIND(fwd_workspace_bytes);
     FDMA_BIND(bwd_workspace_bytes);
+    FDMA_BIND(bwd_optional_bytes);
     FDMA_BIND(fwd_counter_bytes);
     FDMA_BIND(varlen_fwd);
-    FDMA_BIND(varlen_bwd);
+    FDMA_BIND(varlen_bwd_ws);
+    FDMA_BIND(varlen_bwd_optional_bytes);
     FDMA_BIND(create_mask);
     FDMA_BIND(dyn_bias_fwd);
     FDMA_BIND(dyn_bias_bwd);

@@ -125,6 +125,7 @@ class DynBiasArgs(ctypes.Structure):
 
 EXPORTS = (
     "fdma_fwd", "fdma_fwd_noalloc", "fdma_bwd", "fdma_fwd_workspace_bytes", "fdma_fwd_counter_bytes", "fdma_bwd_workspace_bytes",
+    "fdma_bwd_optional_bytes", "fdma_varlen_bwd_ws", "fdma_varlen_bwd_optional_bytes",
     "fdma_set_stream_min_items",
     "fdma_fwd_validate", "fdma_bwd_validate", "fdma_last_error", "fdma_abi_version",
     "fdma_sizeof_fwd_args", "fdma_sizeof_bwd_args",
@@ -206,6 +207,8 @@ def _load() -> ctypes.CDLL:
     lib.fdma_set_stream_min_items.restype = ctypes.c_int
     lib.fdma_bwd_workspace_bytes.argtypes = [ctypes.POINTER(BwdArgs)]
     lib.fdma_bwd_workspace_bytes.restype = ctypes.c_size_t
+    lib.fdma_bwd_optional_bytes.argtypes = [ctypes.POINTER(BwdArgs)]
+    lib.fdma_bwd_optional_bytes.restype = ctypes.c_size_t
     lib.fdma_last_error.argtypes = []
     lib.fdma_last_error.restype = ctypes.c_char_p
     lib.fdma_abi_version.restype = ctypes.c_int
@@ -217,6 +220,10 @@ def _load() -> ctypes.CDLL:
     lib.fdma_varlen_fwd.restype = ctypes.c_int
     lib.fdma_varlen_bwd.argtypes = [ctypes.POINTER(VarlenBwdArgs), ctypes.c_void_p]
     lib.fdma_varlen_bwd.restype = ctypes.c_int
+    lib.fdma_varlen_bwd_ws.argtypes = [ctypes.POINTER(VarlenBwdArgs), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+    lib.fdma_varlen_bwd_ws.restype = ctypes.c_int
+    lib.fdma_varlen_bwd_optional_bytes.argtypes = [ctypes.POINTER(VarlenBwdArgs)]
+    lib.fdma_varlen_bwd_optional_bytes.restype = ctypes.c_size_t
     lib.fdma_varlen_fwd_validate.argtypes = [ctypes.POINTER(VarlenFwdArgs)]
     lib.fdma_varlen_fwd_validate.restype = ctypes.c_int
     lib.fdma_varlen_bwd_validate.argtypes = [ctypes.POINTER(VarlenBwdArgs)]
@@ -249,8 +256,8 @@ lib = _load()
 
 _HOST_PATH = os.path.normpath(os.path.join(_HERE, "..", "lib", "_fdma_torch.so"))
 _HOST_CALLS = (
-    "fdma_fwd", "fdma_bwd", "fdma_fwd_workspace_bytes", "fdma_bwd_workspace_bytes", "fdma_fwd_counter_bytes",
-    "fdma_set_stream_min_items", "fdma_varlen_fwd", "fdma_varlen_bwd", "fdma_create_mask", "fdma_dyn_bias_fwd",
+    "fdma_fwd", "fdma_bwd", "fdma_fwd_workspace_bytes", "fdma_bwd_workspace_bytes", "fdma_bwd_optional_bytes", "fdma_fwd_counter_bytes",
+    "fdma_set_stream_min_items", "fdma_varlen_fwd", "fdma_varlen_bwd_ws", "fdma_varlen_bwd_optional_bytes", "fdma_create_mask", "fdma_dyn_bias_fwd",
     "fdma_dyn_bias_bwd", "fdma_dyn_bias_bwd_workspace_bytes", "fdma_last_error",
 )
 

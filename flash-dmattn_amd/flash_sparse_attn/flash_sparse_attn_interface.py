@@ -417,7 +417,7 @@ def _flash_sparse_attn_backward_body(
     args.softmax_d = softmax_d.data_ptr()
     args.deterministic = int(bool(deterministic))
     with _cabi.device_guard(q.device):
-        nbytes = _cabi.lib.fdma_bwd_workspace_bytes(args)
+        nbytes = _cabi.lib.fdma_bwd_workspace_bytes(args) + _cabi.lib.fdma_bwd_optional_bytes(args)
         workspace = None
         if nbytes:
             workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
@@ -799,8 +799,10 @@ def _flash_sparse_attn_varlen_backward_body(
     args.dv_strides[:] = (dv_w.stride(0), dv_w.stride(1))
     args.softmax_d = softmax_d.data_ptr()
     args.deterministic = int(bool(deterministic))
+    nbytes = _cabi.lib.fdma_varlen_bwd_optional_bytes(args)
+    workspace = torch.empty(nbytes, device=q.device, dtype=torch.uint8) if nbytes else None
     with _cabi.device_guard(q.device):
-        _cabi.check(_cabi.lib.fdma_varlen_bwd(args, _cabi.current_stream(q.device)))
+        _cabi.check(_cabi.lib.fdma_varlen_bwd_ws(args, workspace.data_ptr() if nbytes else None, nbytes, _cabi.current_stream(q.device)))
     for given, work in ((dq, dq_w), (dk, dk_w), (dv, dv_w)):
         if given is not None and work is not given:
             given.copy_(work)

@@ -214,6 +214,10 @@ size_t fdma_fwd_workspace_bytes(const fdma_fwd_args *args);
 /* Size of the optional arrival counters (fdma_fwd_args.counters); 0 when the call would not use them. */
 size_t fdma_fwd_counter_bytes(const fdma_fwd_args *args);
 size_t fdma_bwd_workspace_bytes(const fdma_bwd_args *args);
+/* Further scratch that a backward call can use (0: none): with workspace_bytes of at least fdma_bwd_workspace_bytes() plus this
+ * many, key blocks that many queries see are cut into parts, whose fp32 sums lie there; with less they stay whole, and the call
+ * takes longer where the chip is not full. */
+size_t fdma_bwd_optional_bytes(const fdma_bwd_args *args);
 
 /* Argument validation only (no GPU work, callable on a host without a device). */
 int fdma_fwd_validate(const fdma_fwd_args *args);
@@ -258,6 +262,10 @@ typedef struct fdma_varlen_bwd_args {
  * belongs to a sequence is written exactly once. */
 int fdma_varlen_fwd(const fdma_varlen_fwd_args *args, void *hip_stream);
 int fdma_varlen_bwd(const fdma_varlen_bwd_args *args, void *hip_stream);
+/* The same with scratch for the fp32 sums of key blocks cut into parts, 16-byte aligned: used when it holds
+ * fdma_varlen_bwd_optional_bytes() (0: none wanted); NULL or less: the blocks stay whole. */
+int fdma_varlen_bwd_ws(const fdma_varlen_bwd_args *args, void *workspace, size_t workspace_bytes, void *hip_stream);
+size_t fdma_varlen_bwd_optional_bytes(const fdma_varlen_bwd_args *args);
 int fdma_varlen_fwd_validate(const fdma_varlen_fwd_args *args);
 int fdma_varlen_bwd_validate(const fdma_varlen_bwd_args *args);
 size_t fdma_sizeof_varlen_fwd_args(void);
