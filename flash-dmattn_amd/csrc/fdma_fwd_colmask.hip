@@ -42,7 +42,7 @@
 // overlap its vector work, its LDS reads and its barriers with its MFMAs (1.4 us per tile of 0.5 us matrix work).  Then a
 // workgroup is two groups of four waves over the SAME query rows, each with its own stages: they take the active tiles in
 // turn, with a softmax of their own, and are merged through LDS at the end.  512 rows x 32 heads against 2048 kept keys,
-// d = 128: 44 us, now 37.8.
+// d = 128: 44 us with one group, 37.8 with two (and 31 in fdma_fwd_wide.hip, which takes that size).
 #include <type_traits>
 
 #include "fdma_common.h"
@@ -72,7 +72,7 @@ template <int D, int BN> struct CmSmem {
 // `count` columns, all kept; the fused bias vector comes pre-gathered, and the causal limit of a query row
 // is the number of kept columns at or below its diagonal instead of the column index itself.
 template <typename T, int D, int BN, bool CAUSAL, int NW, bool CMP, int KG>
-__global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1) ? 2 : 1) fwd_colmask_kernel(const FwdParams p) {
+__global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fwd_colmask_kernel(const FwdParams p) {
     constexpr int NTHREADS = 64 * NW;         // of a key group
     static_assert(KG == 1 || NW == 4, "key groups are for small grids, which have 128-row workgroups");
     constexpr int STHREADS = 256;             // threads staging one operand
@@ -89,21 +89,19 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
     constexpr int K_RPP = STHREADS / CH;      // K rows staged per pass
     constexpr int K_IT = BN / K_RPP;          // passes (registers) per K tile
     constexpr int V_ITEMS = KQ * CH;          // (key quad, d chunk) items of a V tile
-    constexpr int V_IT = (V_ITEMS + STHREADS - 1) / STHREADS;  // items per staging thread (two at head dims above 128)
-    constexpr int NL = SPLIT ? 4 : K_IT + 4 * V_IT;  // 16-byte loads per thread and tile
+    constexpr int NL = SPLIT ? 4 : K_IT + 4;  // 16-byte loads per thread and tile
     constexpr int VB = SPLIT ? 0 : K_IT;      // first V staging register
-    static_assert(!SPLIT || V_IT == 1, "the role split assumes one V item per thread");
+    static_assert(V_ITEMS <= STHREADS, "one V item per thread");
     static_assert(!SPLIT || K_IT == 4, "the role split assumes four loads per thread for either operand");
 
     extern __shared__ __attribute__((aligned(16))) char smem_all[];
     const int kgrp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NTHREADS);  // key group of this wave
     // This group's LDS.  A lone group at d = 128 addresses the array itself: through the pointer variable the same places took 4
     // more registers, which the eight-wave kernels do not have (20 bytes spilled; ragged forward of 11 265 tokens x 32 heads
-    // 370.0 -> 367.1 us, of 3 518 x 16 56.0 -> 55.2).  With compacted keys at d = 256 it is 1 % as well (3 000 tokens x 8 heads
-    // 63.1 -> 62.2).  Elsewhere the pointer is ahead by as much (ragged, 18 000 tokens x 16, d = 64: 127.3 and 128.9; 2 800 x 16,
-    // d = 256: 73.9 and 74.8).
+    // 370.0 -> 367.1 us, of 3 518 x 16 56.0 -> 55.2).  Elsewhere the pointer is ahead by as much (ragged, 18 000 tokens x 16,
+    // d = 64: 127.3 and 128.9).
     char *const smem_grp = smem_all + kgrp * SM::TOTAL;
-#define FWD_LDS (KG == 1 && (D == 128 || (D == 256 && CMP)) ? smem_all : smem_grp)
+#define FWD_LDS (KG == 1 && D == 128 ? smem_all : smem_grp)
     uint32_t *sBits = (uint32_t *)(FWD_LDS + SM::OFF_BITS);
     uint32_t *sFlag = (uint32_t *)(smem_all + SM::OFF_FLAG);  // (one for all: the groups leave the common path together)
 
@@ -292,7 +290,6 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
     const int vkg = kt % KQ, vc = (kt / KQ) % CH;  // V: key quad and d chunk of this thread
     const uint32_t k_r2 = (uint32_t)(p.k_r * 2), v_r2 = (uint32_t)(p.v_r * 2);  // bytes per row
     const uint32_t kcolb = (kc * 8 < p.d ? kc * 16 : 0);
-    auto vchunk = [&](int j) -> int { return vc + j * (STHREADS / KQ); };  // d chunk of this thread's j-th V item
     const int j_last = Lk > 0 ? (Lk - 1) / BN : 0, last_row = Lk > 0 ? (Lk - 1) % BN : 0;
     uint32_t soff[NL], soff_l[NL];  // byte offsets of this thread's loads inside a full / the last tile
 #pragma unroll
@@ -300,7 +297,7 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
         const bool is_v = SPLIT ? role_v : n >= K_IT;
         const int item = SPLIT ? n : (n >= K_IT ? n - K_IT : n);  // V: four loads (keys of the quad) per item
         const int row = is_v ? 4 * vkg + (item & 3) : kr0 + item * K_RPP;
-        const uint32_t vcolb = (vchunk(item >> 2) * 8 < p.d ? vchunk(item >> 2) * 16 : 0);
+        const uint32_t vcolb = (vc * 8 < p.d ? vc * 16 : 0);
         const uint32_t r2 = is_v ? v_r2 : k_r2, colb = is_v ? vcolb : kcolb;
         soff[n] = (uint32_t)row * r2 + colb;
         soff_l[n] = (uint32_t)(row < last_row ? row : last_row) * r2 + colb;
@@ -390,13 +387,13 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
         if (role_v && kt < V_ITEMS) {  // transpose 4 keys x 8 d in registers, write V^T[d][key quad]
             char *sVt = FWD_LDS + SM::OFF_VT + vbuf * SM::VT_BYTES;
 #pragma unroll
-            for (int dj = 0; dj < 8 * V_IT; dj++) {
-                const int j = dj >> 3, dd = dj & 7, w = dd >> 1;
+            for (int dd = 0; dd < 8; dd++) {
+                const int w = dd >> 1;
                 const uint32_t sel = (dd & 1) ? 0x07060302u : 0x05040100u;
                 u32x2_t out;
-                out[0] = __builtin_amdgcn_perm(sreg[VB + 4 * j + 1][w], sreg[VB + 4 * j + 0][w], sel);
-                out[1] = __builtin_amdgcn_perm(sreg[VB + 4 * j + 3][w], sreg[VB + 4 * j + 2][w], sel);
-                *(u32x2_t *)(sVt + ((vchunk(j) * 8 + dd) * SM::SVT + 4 * vkg) * 2) = out;
+                out[0] = __builtin_amdgcn_perm(sreg[VB + 1][w], sreg[VB][w], sel);
+                out[1] = __builtin_amdgcn_perm(sreg[VB + 3][w], sreg[VB + 2][w], sel);
+                *(u32x2_t *)(sVt + ((vc * 8 + dd) * SM::SVT + 4 * vkg) * 2) = out;
             }
         }
     };
@@ -562,14 +559,14 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && D <= 128 && KG == 1)
             // chunk of K
             if (DO_V) {
 #pragma unroll
-                for (int dj = 0; dj < 8 * V_IT; dj++)
-                    if (f == 1 + dj * ((NF - 1) / (8 * V_IT))) {
-                        const int j = dj >> 3, dd = dj & 7, w = dd >> 1;
+                for (int dd = 0; dd < 8; dd++)
+                    if (f == 1 + dd * ((NF - 1) / 8)) {
+                        const int w = dd >> 1;
                         const uint32_t sel = (dd & 1) ? 0x07060302u : 0x05040100u;
                         u32x2_t out;
-                        out[0] = __builtin_amdgcn_perm(sreg[VB + 4 * j + 1][w], sreg[VB + 4 * j + 0][w], sel);
-                        out[1] = __builtin_amdgcn_perm(sreg[VB + 4 * j + 3][w], sreg[VB + 4 * j + 2][w], sel);
-                        *(u32x2_t *)(sVt_w + ((vchunk(j) * 8 + dd) * SM::SVT + 4 * vkg) * 2) = out;
+                        out[0] = __builtin_amdgcn_perm(sreg[VB + 1][w], sreg[VB][w], sel);
+                        out[1] = __builtin_amdgcn_perm(sreg[VB + 3][w], sreg[VB + 2][w], sel);
+                        *(u32x2_t *)(sVt_w + ((vc * 8 + dd) * SM::SVT + 4 * vkg) * 2) = out;
                     }
             }
             if (DO_K) {
@@ -886,6 +883,12 @@ template <typename T> __global__ void __launch_bounds__(256) fwd_merge_kernel(co
     if (c == 0) p.lse[b * p.lse_b + h * p.lse_h + q] = sum > 0.f ? (top + __builtin_amdgcn_logf(sum)) * kLn2 : INFINITY;
 }
 
+template <typename T> hipError_t launch_merge(const FwdParams &p, hipStream_t stream) {
+    const int64_t items = (int64_t)p.B * p.H * p.Lq * (p.d / 8);
+    hipLaunchKernelGGL((fwd_merge_kernel<T>), dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream, p);
+    return hipGetLastError();
+}
+
 template <typename T, int D, int BN, bool CAUSAL, bool CMP, int NW = 4, int KG = 1>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     constexpr int BM = 32 * NW;
@@ -900,9 +903,7 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     dim3 grid(pairs * k_split * ((n_mb + k_split - 1) / k_split) * G, CMP && KG == 2 ? p.splits : 1);
     hipLaunchKernelGGL(kern, grid, dim3(64 * NW * KG), smem, stream, p);
     if ((e = hipGetLastError()) != hipSuccess || grid.y == 1) return e;
-    const int64_t items = (int64_t)p.B * p.H * p.Lq * (p.d / 8);
-    hipLaunchKernelGGL((fwd_merge_kernel<T>), dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream, p);
-    return hipGetLastError();
+    return launch_merge<T>(p, stream);
 }
 
 template <typename T, int D>
@@ -916,7 +917,7 @@ hipError_t launch_d(const FwdParams &p, hipStream_t stream) {
     }
     // no more 128-row workgroups than CUs: two key groups each (a row that sees a single tile gains nothing, and pays
     // a merge of a microsecond)
-    if constexpr (D <= 128) if ((int64_t)p.B * p.H * ((p.Lq + 127) / 128) <= device_cus() && p.Lk > 128) {
+    if ((int64_t)p.B * p.H * ((p.Lq + 127) / 128) <= device_cus() && p.Lk > 128) {
         if (p.cmp.on) return p.causal ? launch_one<T, D, 64, true, true, 4, 2>(p, stream) : launch_one<T, D, 64, false, true, 4, 2>(p, stream);
         return p.causal ? launch_one<T, D, 64, true, false, 4, 2>(p, stream) : launch_one<T, D, 64, false, false, 4, 2>(p, stream);
     }
@@ -936,6 +937,8 @@ hipError_t launch_d(const FwdParams &p, hipStream_t stream) {
 // medians over 1 to 40 blocks of 2 to 300 rows, d = 128; d = 64 is alike), with a sixteenth, a quarter and all of the keys kept:
 //   3072 keys   16.5 / 20.2    24.4 / 27.9    53.0 / 34.4        16384 keys   27.4 / 25.9    65.0 / 31.1    207.5 / 54.8
 //   6144 keys   19.4 / 22.4    34.0 / 26.8    90.2 / 39.3        32768 keys   40.4 / 28.4   114.7 / 40.1    395.4 / 88.2
+// (As measured with 128-row blocks; at d > 64 the 64-row blocks of fdma_fwd_wide.hip take these calls, whole and in shares, in 0.8 to
+// 0.88 of the time.)
 // How much is kept is not known here: with under 1024 kept keys there is a single share and the merge costs its 3 to 4 us for
 // nothing; the other way round a share too few costs more.
 int key_shares(const FwdParams &p) {
@@ -958,9 +961,20 @@ bool fwd_colmask_applicable(const FwdParams &p) {
 
 hipError_t launch_fwd_colmask(const FwdParams &p, int dtype, hipStream_t stream) {
     if (p.cmp.on && p.cmp.img_kv) return launch_fwd_stream(p, dtype, stream);  // (the pre-pass has written tile images)
-    // head dims up to 64 / 128 / 256 (a head dim in between runs in the next larger instantiation)
-    if (dtype == 0) return p.d <= 64 ? launch_d<bf16_tag, 64>(p, stream) : p.d <= 128 ? launch_d<bf16_tag, 128>(p, stream) : launch_d<bf16_tag, 256>(p, stream);
-    return p.d <= 64 ? launch_d<fp16_tag, 64>(p, stream) : p.d <= 128 ? launch_d<fp16_tag, 128>(p, stream) : launch_d<fp16_tag, 256>(p, stream);
+    // head dims up to 64 / 128 (a head dim in between runs in the next larger instantiation), above in a kernel of their own
+    if (p.d > 128) return launch_fwd_wide(p, dtype, stream);
+    // 64-row workgroups of four key groups, one to a CU, as long as all of them run at once: 1.13 to 1.35 times the 128-row ones
+    // with two groups over 24 calls of 4 to 256 blocks; 352 blocks (2 x 700 rows x 16 heads) 29.9 against 21.6 us.  A row
+    // that sees a single tile gains nothing (128 x 128: 10.7 either way).  (A ragged batch has at most total / 64 blocks per
+    // head and one more per entry.)
+    const int64_t blocks64 = p.cu_q ? (int64_t)p.H * (p.total_q / 64 + p.B) : (int64_t)p.B * p.H * ((p.Lq + 63) / 64);
+    if (p.d > 64 && blocks64 <= device_cus() && p.Lk > 128) {
+        const hipError_t e = launch_fwd_wide(p, dtype, stream);
+        if (e != hipSuccess || !p.cmp.on || p.splits <= 1) return e;
+        return dtype == 0 ? launch_merge<bf16_tag>(p, stream) : launch_merge<fp16_tag>(p, stream);
+    }
+    if (dtype == 0) return p.d <= 64 ? launch_d<bf16_tag, 64>(p, stream) : launch_d<bf16_tag, 128>(p, stream);
+    return p.d <= 64 ? launch_d<fp16_tag, 64>(p, stream) : launch_d<fp16_tag, 128>(p, stream);
 }
 
 }  // namespace fdma

@@ -1,0 +1,483 @@
+// Forward dynamic-mask attention for gfx950, column-mask specialisation with key groups and direct loads: head dims 129 .. 256,
+// and 65 .. 128 where there are no more blocks of 64 query rows than CUs.
+//
+// Same math, inputs and reference counterparts as fdma_fwd_colmask.hip (compute_attn_1rowblock,
+// csrc/flash_sparse_attn/src/flash_fwd_kernel.h:53-804 of the reference; mask and bias absent or broadcast over the query
+// dimension).
+//
+// A workgroup is 8 waves, two to a SIMD: RG groups of 32 query rows times KG = 8 / RG groups of 32 keys, a tile being 32 KG
+// keys.  Wave (rw, kg) takes its rows against its keys of every tile, with a softmax of its own; the key groups are merged
+// through LDS at the end, each finishing its share of the head dim.
+//   * Head dim 256, RG = 4: O alone is 128 registers per lane, Q another 64.  With four waves (one per SIMD, 448 registers,
+//     nothing to hide behind) a step of 128 rows x 64 keys took 3.2 us for 0.85 us of matrix work, here 2.0.
+//   * Head dim 128, RG = 2: 64-row blocks with four key groups are twice as many workgroups with half the chain of tiles.
+//     A tile of 128 keys takes 1.4 us where the eight-wave kernel of fdma_fwd_colmask.hip takes 1.6 for 128 rows, on twice
+//     the CUs.
+//   * K and V tiles go from global memory straight into LDS (global_load_lds, one tile ahead, issued between the MFMAs):
+//     no staging registers.  The 16-byte chunks of a 256-byte row, or of the two halves of a 512-byte one, are swizzled as in
+//     LdsTile<128>; V is row-major like K, and V^T comes from transposing LDS reads.
+//   * The score accumulators start from the fused bias of their keys (fp32, -inf where the mask drops the key), read from an
+//     LDS column; the softmax is the online one, with a reference point that moves only when a score exceeds it by 2^8.  Its
+//     vector work runs under the MFMAs of the SIMD's other wave.
+// LDS: two stages of 64 KB.  Bound by the chain of a tile (scores, softmax, P V, barrier) of two waves per SIMD: without the
+// loads it is 0.25 us shorter, without the softmax 0.1.
+// Before / now (us): 3001 tokens, 8/4 heads, d = 256, 1024 kept, fp16 57 / 38 (with the bias producer and the mask 75.6 / 56.3);
+// 8192 tokens, 8/2 heads, d = 256, 4096 kept 203 / 152; 2300 ragged tokens and others, 16/8 heads, d = 256 152 / 115;
+// d = 128: 512 rows x 32 heads against 2048 kept keys of 16384 42.7 / 35.6, 2000 tokens x 4 heads 39.7 / 32.4, 256 x 32 14.8 / 11.0.
+#include <type_traits>
+
+#include "fdma_common.h"
+#include "fdma_params.h"
+
+namespace fdma {
+
+namespace {
+
+constexpr int NT = 512;
+constexpr int MAX_TILES = 16384;
+
+// RG row groups of 32 query rows, KG = 8 / RG key groups
+template <int D_, int RG> struct Cfg {
+    static constexpr int D = D_, KG = 8 / RG;
+    static constexpr int BM = 32 * RG, BN = 32 * KG;      // query rows per workgroup, keys per tile
+    static constexpr int ROW = D * 2, CH = D / 8;         // bytes and 16-byte chunks of a tile row
+    static constexpr int TILE = BN * ROW;                 // a K or V tile
+    static constexpr int RPP = 64 / CH;                   // rows of a 1 KB piece
+    static constexpr int NP = TILE / 1024 / 8;            // pieces per wave of a K or V tile
+    static constexpr int OFF_V = 2 * TILE;                // two stages of K, two of V
+    static constexpr int OFF_COL = 4 * TILE;              // two stages of the fused bias column
+    static constexpr int OFF_BITS = OFF_COL + 2 * BN * 4;
+    static constexpr int LOOP_BYTES = OFF_BITS + MAX_TILES / 8;
+    static constexpr int DPW = D / 32 / KG;               // merge: 32-wide blocks of O that a wave finishes
+    static constexpr int OFF_SUMS = KG * (KG - 1) * RG * DPW * 4096;  // ... the others' shares of them, then row sums and references
+    static constexpr int MERGE_BYTES = OFF_SUMS + 2 * 8 * 64 * 4;
+    static constexpr int SMEM = LOOP_BYTES > MERGE_BYTES ? LOOP_BYTES : MERGE_BYTES;
+    static_assert(SMEM <= 160 * 1024, "one workgroup per CU");
+    static_assert(8 * RPP % 16 == 0, "a wave's pieces lie rows of one swizzle apart");
+};
+
+// (see LdsTile: the swizzle permutes the 16 chunks of a 256-byte half row, so rows of 512 bytes meet the banks as rows of 256 do)
+__device__ __forceinline__ uint32_t swz(int row) { return (uint32_t)(((row & 3) << 2) | ((row >> 2) & 3)); }
+
+template <typename T, int D, int RG, bool CAUSAL, bool CMP>
+__global__ void __launch_bounds__(NT) fwd_wide_kernel(const FwdParams p) {
+    using E = Elem<T>;
+    using C = Cfg<D, RG>;
+    constexpr int KG = C::KG, BM = C::BM, BN = C::BN, ROW = C::ROW, TILE = C::TILE, NP = C::NP, KS = D / 16, DB = D / 32;
+    constexpr int OFF_V = C::OFF_V, OFF_COL = C::OFF_COL, OFF_BITS = C::OFF_BITS, DPW = C::DPW;
+    extern __shared__ __attribute__((aligned(256))) char smem[];
+    const uint32_t lds0 = lds_addr(smem);  // (a multiple of 256)
+    uint32_t *sBits = (uint32_t *)(smem + OFF_BITS);
+
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = tid & 63, r = lane & 31, g = lane >> 5;
+    const int rw = wave % RG, kg = wave / RG;  // 32-row group and key group of this wave
+
+    // workgroup -> (batch, head, query block): XCD-aware, heaviest query block first (see fwd_colmask_kernel)
+    const int n_mb = (p.Lq + BM - 1) / BM;
+    const int G = p.H / p.Hk, pairs = p.B * p.Hk;
+    const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
+    const int k_split = 8 / gcd8;
+    const int list_len = ((n_mb + k_split - 1) / k_split) * G;
+    const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
+    const int vlist = xcd + 8 * (slot / list_len);
+    const int pos = slot % list_len;
+    const int pair = vlist / k_split;
+    const int mslot = (pos / G) * k_split + vlist % k_split;
+    if (mslot >= n_mb) return;
+    const int b = pair / p.Hk, hk = pair % p.Hk, h = hk * G + pos % G;
+    const int m0 = (n_mb - 1 - mslot) * BM;
+    const SeqInfo sq = seq_info(p, b);
+    const int LqS = sq.Lq, LkS = sq.Lk;
+    if (m0 >= LqS) return;
+    const int shift = LkS - LqS;
+    const int wrow0 = m0 + rw * 32, qrow = wrow0 + r;
+
+    // ---- Q fragments: requested first of all, scaled behind the set-up
+    u32x4_t qf[KS];
+    {
+        const int qc = qrow < LqS ? qrow : LqS - 1;
+        const uint16_t *qp = (const uint16_t *)p.q + b * p.q_b + (sq.q0 + qc) * p.q_r + h * p.q_h;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const int c = ks * 16 + g * 8;
+            qf[ks] = *(const u32x4_t *)(qp + (c < p.d ? c : 0));  // (chunks beyond d are cleared when scaled)
+        }
+    }
+
+    const int hm = p.mask ? (p.Hm == p.H ? h : (p.Hm == 1 ? 0 : h / (p.H / p.Hm))) : 0;
+    const int hb = p.bias ? (p.Hb == p.H ? h : (p.Hb == 1 ? 0 : h / (p.H / p.Hb))) : 0;
+    const uint8_t *mrow = p.mask ? p.mask + b * p.m_b + hm * p.m_h : nullptr;
+    const uint16_t *brow = p.bias ? (const uint16_t *)p.bias + b * p.bi_b + hb * p.bi_h : nullptr;
+    const uint16_t *kbase = (const uint16_t *)p.k + b * p.k_b + sq.k0 * p.k_r + hk * p.k_h;
+    const uint16_t *vbase = (const uint16_t *)p.v + b * p.v_b + sq.k0 * p.v_r + hk * p.v_h;
+
+    // key columns this workgroup iterates over, and the number of them a query row may see
+    const int Lk = CMP ? p.cmp.count[b * p.Hk + hk] : LkS;
+    const int32_t *ccnt = CMP ? p.cmp.cnt + (int64_t)(b * p.Hk + hk) * p.cmp.ld : nullptr;
+    const float *fbrow = CMP ? p.cmp.fb + (int64_t)(b * p.cmp.Hfb + (p.cmp.Hfb == p.H ? h : hk)) * p.cmp.ld : nullptr;
+    auto visible = [&](int row) -> int {  // columns [0, visible(row)) pass the causal test for `row`
+        if (row >= LqS) row = LqS - 1;
+        const int c = row + shift;
+        if (!CMP) return c + 1;
+        if (c < 0) return 0;
+        return ccnt[c < LkS ? c : LkS - 1];
+    };
+    int n_end = (Lk + BN - 1) / BN;
+    if (CAUSAL) {
+        int lim = visible(m0 + BM - 1);
+        if (lim < 0) lim = 0;
+        const int ne = (lim + BN - 1) / BN;
+        if (ne < n_end) n_end = ne;
+    }
+    // this workgroup's share of the tiles (see fwd_key_splits)
+    int t_first = 0;
+    if (CMP && p.splits > 1) {
+        // (no share under 512 keys: the shares that are then left over only say so)
+        const int y = (int)blockIdx.y, most = n_end * BN / 512 > 1 ? n_end * BN / 512 : 1, shares = p.splits < most ? p.splits : most;
+        if (y >= shares) {
+            if (tid < BM && m0 + tid < LqS) p.lse_part[(((int64_t)y * p.B + b) * p.H + h) * p.Lq + m0 + tid] = -INFINITY;
+            return;
+        }
+        t_first = n_end * y / shares;
+        n_end = n_end * (y + 1) / shares;
+    }
+    const int vis_lane = CAUSAL ? visible(qrow) : 0;
+    const int vis_wave = CAUSAL ? visible(wrow0) : 0;
+
+    // ---- active-tile bitmap (compacted keys: every tile is active)
+    for (int base = 0; !CMP && base < n_end; base += NT) {
+        const int j = base + tid;
+        bool act = false;
+        if (j < n_end) {
+            if (mrow) {
+                uint32_t any = 0;
+                int col[BN / 16];
+                u32x4_t mv[BN / 16];
+#pragma unroll
+                for (int c = 0; c < BN / 16; c++) col[c] = j * BN + c * 16;
+                ld_row16(mrow, col, LkS, mv);
+#pragma unroll
+                for (int c = 0; c < BN / 16; c++) any |= mv[c][0] | mv[c][1] | mv[c][2] | mv[c][3];
+                act = any != 0;
+            } else {
+                act = true;
+            }
+        }
+        const uint64_t ball = __ballot(act);
+        if (lane == 0) {
+            const int w0 = (base + wave * 64) >> 5;
+            sBits[w0] = (uint32_t)ball;
+            sBits[w0 + 1] = (uint32_t)(ball >> 32);
+        }
+    }
+    if (!CMP) __syncthreads();
+    auto next_active = [&](int j) -> int {  // wave-uniform
+        if (CMP) return j < n_end ? j : n_end;
+        while (j < n_end) {
+            const uint32_t w = __builtin_amdgcn_readfirstlane(lds_ld32(lds0 + OFF_BITS + 4 * (j >> 5))) >> (j & 31);
+            if (w) {
+                j += __builtin_ctz(w);
+                return j < n_end ? j : n_end;
+            }
+            j = (j | 31) + 1;
+        }
+        return n_end;
+    };
+
+    // ---- staging: a piece is 1 KB, whole rows; wave w fetches pieces w + 8 i of K and of V.  A lane fills chunk position
+    // `lane % CH` of its row, which holds chunk position ^ swz(row) of the global row; rows 16 apart have the same swizzle.  Rows beyond the keys are clamped to the last one (their column says -inf), chunks beyond d to chunk 0 (they
+    // meet zero Q and columns of O that are not stored).
+    typedef const __attribute__((address_space(1))) char *gptr_t;
+    auto uniform_ptr = [](const void *ptr) -> gptr_t {
+        const uint64_t v = (uint64_t)ptr;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+        return (gptr_t)(((uint64_t)hi << 32) | lo);
+    };
+    const int prow = C::RPP * wave + lane / C::CH;
+    const int pchunk = lane % C::CH ^ (int)swz(prow);
+    const uint32_t pcol = pchunk * 8 < p.d ? pchunk * 16 : 0;
+    const uint32_t k_r2 = (uint32_t)(p.k_r * 2), v_r2 = (uint32_t)(p.v_r * 2);
+    gptr_t tb_k = nullptr, tb_v = nullptr;
+    int t_rows = 0, t_stage = 0;     // last row of the tile being fetched, its stage
+    uint32_t braw = 0, mraw = 0;     // first waves: raw bias and mask of key `tid` of that tile
+    bool col_ok = false;
+    auto set_tile = [&](int j, int stage) {
+        tb_k = uniform_ptr(kbase + (int64_t)j * BN * p.k_r);
+        tb_v = uniform_ptr(vbase + (int64_t)j * BN * p.v_r);
+        const int left = Lk - 1 - j * BN;
+        t_rows = left < BN - 1 ? left : BN - 1;
+        t_stage = stage;
+        if (wave < BN / 64) {  // (raw, unconditional loads: an absent mask or bias is read from K and ignored)
+            const int col = j * BN + tid;
+            col_ok = col < Lk;
+            const int cc = col_ok ? col : 0;
+            if (CMP) {
+                braw = __float_as_uint(fbrow[cc]);
+            } else {
+                mraw = (mrow ? mrow : (const uint8_t *)kbase)[cc];
+                braw = (brow ? brow : kbase)[cc];
+            }
+        }
+    };
+    // (in assembly and waited for by hand: behind the compiler's builtin every LDS read waits for all LDS operations in flight)
+    auto dma_piece = [&](int n) {  // NP pieces of K, NP of V
+        const int i = n % NP;
+        const int row = prow + 8 * C::RPP * i, row_c = row < t_rows ? row : t_rows;
+        const uint32_t off = (uint32_t)row_c * (n < NP ? k_r2 : v_r2) + pcol;
+        const uint32_t dst = lds0 + (n < NP ? 0 : OFF_V) + (uint32_t)(t_stage * TILE + (wave + 8 * i) * 1024);
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(n < NP ? tb_k : tb_v), "s"(__builtin_amdgcn_readfirstlane(dst)));
+    };
+    auto publish = [&]() {
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's pieces have landed
+        if (wave < BN / 64) {
+            float v = 0.f;
+            bool keep = col_ok;
+            if (CMP) {
+                v = __uint_as_float(braw);
+            } else {
+                keep = keep && (!mrow || mraw);
+                if (brow) v = E::lo(braw) * kLog2e;
+            }
+            lds_st32(lds0 + OFF_COL + t_stage * BN * 4 + 4 * tid, __float_as_uint(keep ? v : -INFINITY));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+
+    // fragment addresses (stage 0).  K: chunk 2 ks + g of row 32 kg + pi_row(r).  V^T: see LdsTile::tr_base.
+    const int frow = 32 * kg + pi_row(r);
+    uint32_t a_off = lds0 + (uint32_t)frow * ROW + (((uint32_t)g ^ swz(frow)) << 4);
+    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
+    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
+    const int tdh = (lane >> 4) & 1;
+    uint32_t tr_off = lds0 + OFF_V + (uint32_t)(32 * kg + 8 * g + te) * ROW +
+                      (((uint32_t)te << 6) | ((((uint32_t)(2 * tdh + (tcp >> 1))) ^ (uint32_t)(2 * g)) << 4) | ((uint32_t)(tcp & 1) << 3));
+    const uint32_t col_off = lds0 + OFF_COL + 128 * kg + 32 * g;
+
+    f32x16_t o[DB];
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[db][i] = 0.f;
+    float row_sum = 0.f, row_ref = -INFINITY;  // relative to exp2(row_ref); -inf: no visible key met yet
+
+    int jc = next_active(t_first), jn = n_end;
+    if (jc < n_end) {
+        jn = next_active(jc + 1);
+        set_tile(jc, 0);
+#pragma unroll
+        for (int n = 0; n < 2 * NP; n++) dma_piece(n);
+    }
+    // Q is scaled by softmax_scale * log2(e) once (the reference also rounds the scaled Q to the input type,
+    // flash_fwd_kernel.h:428-439)
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+        const bool ok = qrow < LqS && ks * 16 + g * 8 < p.d;
+#pragma unroll
+        for (int e = 0; e < 4; e++) qf[ks][e] = ok ? E::pack2(E::lo(qf[ks][e]) * p.scale_log2, E::hi(qf[ks][e]) * p.scale_log2) : 0u;
+    }
+    if (jc < n_end) publish();
+
+    auto one_tile = [&](auto st_c) {
+        constexpr int st = decltype(st_c)::value;
+        // (the swizzled addresses are these constants XOR a compile-time value, recomputed where used)
+        asm volatile("" : "+v"(a_off), "+v"(tr_off));
+        const int n0 = jc * BN + 32 * kg;
+        set_tile(jn < n_end ? jn : jc, st ^ 1);  // (past the last tile it is fetched again and dropped)
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- S^T = K Q^T on top of the fused bias of the keys
+        f32x16_t s;
+#pragma unroll
+        for (int blk = 0; blk < 2; blk++) {
+            const f32x4_t b0 = __builtin_bit_cast(f32x4_t, lds_ld128(col_off + st * BN * 4 + 64 * blk));
+            const f32x4_t b1 = __builtin_bit_cast(f32x4_t, lds_ld128(col_off + st * BN * 4 + 64 * blk + 16));
+#pragma unroll
+            for (int e = 0; e < 4; e++) { s[8 * blk + e] = b0[e]; s[8 * blk + 4 + e] = b1[e]; }
+        }
+        {
+            constexpr int FR = 4;
+            u32x4_t a[KS];
+            auto frag = [&](int ks) { return lds_ld128((a_off ^ ((uint32_t)(ks & 7) << 5)) + (uint32_t)(st * TILE + (ks >> 3) * 256)); };
+#pragma unroll
+            for (int ks = 0; ks < FR; ks++) a[ks] = frag(ks);
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {
+                if (ks + FR < KS) a[ks + FR] = frag(ks + FR);
+                s = E::mfma(a[ks], qf[ks], s);
+#pragma unroll
+                for (int n = ks * 2 * NP / KS; n < (ks + 1) * 2 * NP / KS; n++) dma_piece(n);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (CAUSAL && n0 + 32 > vis_wave) {
+            asm volatile("" ::: "memory");  // (a branch: only diagonal tiles pay)
+            const int lim = vis_lane - 1 - n0 - 8 * g;  // local columns 16 blk + e <= lim are visible
+#pragma unroll
+            for (int i = 0; i < 16; i++) s[i] = 16 * (i >> 3) + (i & 7) <= lim ? s[i] : -INFINITY;
+        }
+        // ---- online softmax
+        float tmax = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) tmax = fmaxf(tmax, s[i]);
+        tmax = xhalf_max(tmax);
+        const bool move = tmax > row_ref + 8.f || (row_ref == -INFINITY && tmax > -INFINITY);
+        if (__any(move)) {
+            const float alpha = move ? (row_ref == -INFINITY ? 0.f : fast_exp2(row_ref - tmax)) : 1.f;
+            row_ref = move ? tmax : row_ref;
+            row_sum *= alpha;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) o[db][i] *= alpha;
+        }
+        const float ref = row_ref == -INFINITY ? 0.f : row_ref;
+        uint32_t pk[8];
+        float psum0 = 0.f, psum1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float x0 = fast_exp2(s[2 * i] - ref), x1 = fast_exp2(s[2 * i + 1] - ref);
+            psum0 += x0;
+            psum1 += x1;
+            pk[i] = E::pack2(x0, x1);
+        }
+        row_sum += psum0 + psum1;
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- O^T += V^T P^T: V^T through transposing reads, FR2 MFMAs ahead
+        {
+            constexpr int NG = 2 * DB, FR2 = 3;
+            u32x2_t tl[NG], th[NG];
+            auto tr_read = [&](int gi) {
+                const int kb = gi / DB, db = gi % DB;
+                const uint32_t at = (tr_off ^ ((uint32_t)(db & 3) << 6)), hi = (tr_off ^ (((uint32_t)(db & 3) << 6) | 16u));
+                const uint32_t c = (uint32_t)(st * TILE + kb * 16 * ROW + (db >> 2) * 256);
+                tl[gi] = lds_ld_tr16(at + c);
+                th[gi] = lds_ld_tr16(hi + c + 4 * ROW);
+            };
+#pragma unroll
+            for (int gi = 0; gi < FR2; gi++) tr_read(gi);
+#pragma unroll
+            for (int gi = 0; gi < NG; gi++) {
+                if (gi + FR2 < NG) tr_read(gi + FR2);
+                const int kb = gi / DB, db = gi % DB;
+                const u32x4_t bop = {pk[4 * kb], pk[4 * kb + 1], pk[4 * kb + 2], pk[4 * kb + 3]};
+                const u32x4_t av = {tl[gi][0], tl[gi][1], th[gi][0], th[gi][1]};
+                o[db] = E::mfma(av, bop, o[db]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        publish();
+        jc = jn;
+        jn = next_active(jn + 1);
+    };
+    while (jc < n_end) {
+        one_tile(std::integral_constant<int, 0>());
+        if (jc >= n_end) break;
+        one_tile(std::integral_constant<int, 1>());
+    }
+
+    // ---- merge of the key groups: wave (rw, kg) finishes blocks kg DPW .. + DPW - 1 of its rows, the others hand theirs over
+    __syncthreads();
+    float total = xhalf_sum(row_sum);
+    float *xs = (float *)(smem + C::OFF_SUMS) + lane;
+    xs[wave * 64] = total;
+    xs[(8 + wave) * 64] = row_ref;
+    auto shelf = [&](int dst, int src, int j) -> f32x4_t * {  // block j of wave group dst, from group src
+        return (f32x4_t *)smem + (((dst * (KG - 1) + (src + KG - dst - 1) % KG) * RG + rw) * DPW + j) * 4 * 64 + lane;
+    };
+#pragma unroll
+    for (int dst = 0; dst < KG; dst++)
+        if (dst != kg) {
+#pragma unroll
+            for (int j = 0; j < DPW; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const f32x16_t &v = o[dst * DPW + j];
+                    shelf(dst, kg, j)[q * 64] = f32x4_t{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+                }
+        }
+    __syncthreads();
+    float ref[KG], top = -INFINITY, w[KG];
+#pragma unroll
+    for (int x = 0; x < KG; x++) {
+        ref[x] = xs[(8 + x * RG + rw) * 64];
+        top = fmaxf(top, ref[x]);
+    }
+    const float safe = top == -INFINITY ? 0.f : top;
+    total = 0.f;
+#pragma unroll
+    for (int x = 0; x < KG; x++) {
+        w[x] = fast_exp2(ref[x] - safe);
+        total += xs[(x * RG + rw) * 64] * w[x];
+    }
+    if (qrow >= LqS) return;
+    const float inv = total > 0.f ? 1.f / total : 0.f;
+    const bool share = CMP && p.splits > 1;  // this share's O in fp32 and its log2-sum-exp; fwd_merge_kernel adds the shares up
+    const int64_t prow_at = (((int64_t)blockIdx.y * p.B + b) * p.H + h) * p.Lq + qrow;
+    uint16_t *op = (uint16_t *)p.o + b * p.o_b + (sq.q0 + qrow) * p.o_r + h * p.o_h;
+#pragma unroll
+    for (int own = 0; own < KG; own++)
+        if (own == kg) {
+#pragma unroll
+            for (int j = 0; j < DPW; j++)
+#pragma unroll
+                for (int blk = 0; blk < 2; blk++) {
+                    const int c = 32 * (own * DPW + j) + 16 * blk + 8 * g;
+                    f32x4_t y[2];
+#pragma unroll
+                    for (int q = 0; q < 2; q++) {
+                        const f32x16_t &v = o[own * DPW + j];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) y[q][e] = v[8 * blk + 4 * q + e] * w[own];
+#pragma unroll
+                        for (int x = 0; x < KG; x++)
+                            if (x != own) {
+                                const f32x4_t t = shelf(own, x, j)[(2 * blk + q) * 64];
+#pragma unroll
+                                for (int e = 0; e < 4; e++) y[q][e] += t[e] * w[x];
+                            }
+#pragma unroll
+                        for (int e = 0; e < 4; e++) y[q][e] *= inv;
+                    }
+                    if (c < p.d) {
+                        if (share) {
+                            *(f32x4_t *)(p.o_part + prow_at * p.d + c) = y[0];
+                            *(f32x4_t *)(p.o_part + prow_at * p.d + c + 4) = y[1];
+                        } else {
+                            *(u32x4_t *)(op + c) = u32x4_t{E::pack2(y[0][0], y[0][1]), E::pack2(y[0][2], y[0][3]), E::pack2(y[1][0], y[1][1]), E::pack2(y[1][2], y[1][3])};
+                        }
+                    }
+                }
+        }
+    if (g == 0 && kg == 0) {
+        // (a sum that is no number has to reach the result: only an empty share is left out)
+        if (share) p.lse_part[prow_at] = total == 0.f ? -INFINITY : top + __builtin_amdgcn_logf(total);
+        else p.lse[b * p.lse_b + h * p.lse_h + sq.q0 + qrow] = total > 0.f ? (top + __builtin_amdgcn_logf(total)) * kLn2 : INFINITY;
+    }
+}
+
+template <typename T, int D, int RG, bool CAUSAL, bool CMP>
+hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
+    using C = Cfg<D, RG>;
+    auto kern = fwd_wide_kernel<T, D, RG, CAUSAL, CMP>;
+    static DynSmemLimit smem_limit;
+    hipError_t e = smem_limit.ensure((const void *)kern, C::SMEM);
+    if (e != hipSuccess) return e;
+    const int n_mb = (p.Lq + C::BM - 1) / C::BM, G = p.H / p.Hk, pairs = p.B * p.Hk;
+    const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
+    const int k_split = 8 / gcd8;
+    hipLaunchKernelGGL(kern, dim3(pairs * k_split * ((n_mb + k_split - 1) / k_split) * G, CMP ? p.splits : 1), dim3(NT), C::SMEM, stream, p);
+    return hipGetLastError();
+}
+
+template <typename T, int D, int RG> hipError_t launch_t(const FwdParams &p, hipStream_t stream) {
+    if (p.cmp.on) return p.causal ? launch_one<T, D, RG, true, true>(p, stream) : launch_one<T, D, RG, false, true>(p, stream);
+    return p.causal ? launch_one<T, D, RG, true, false>(p, stream) : launch_one<T, D, RG, false, false>(p, stream);
+}
+
+}  // namespace
+
+hipError_t launch_fwd_wide(const FwdParams &p, int dtype, hipStream_t stream) {
+    if (p.d > 128) return dtype == 0 ? launch_t<bf16_tag, 256, 4>(p, stream) : launch_t<fp16_tag, 256, 4>(p, stream);
+    return dtype == 0 ? launch_t<bf16_tag, 128, 2>(p, stream) : launch_t<fp16_tag, 128, 2>(p, stream);
+}
+
+}  // namespace fdma

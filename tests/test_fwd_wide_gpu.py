@@ -1,0 +1,78 @@
+"""The forward with key groups by direct loads (fdma_fwd_wide.hip): head dims above 128, and 65 .. 128 on grids of no more
+64-row blocks than CUs.  Sizes at the edges of its row blocks (64 / 128 rows) and tiles (128 / 64 keys), key groups without a
+kept key, scores that climb from tile to tile (the reference point moves in every one), empty rows."""
+import pytest
+import torch
+
+from oracle import eager
+from _util import assert_out_close, make_inputs, set_compact
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _check(q, k, v, mask, bias, causal):
+    from flash_sparse_attn import flash_sparse_attn_func
+
+    q, k, v, mask, bias = [t if t is None else t.to(DEV) for t in (q, k, v, mask, bias)]
+    out, lse, _ = flash_sparse_attn_func(q, k, v, mask, bias, None, causal, return_attn_probs=True)
+    ro, rl = eager.attention_forward(q, k, v, mask, bias, None, causal)
+    assert_out_close(out, ro)
+    assert torch.equal(torch.isinf(lse), torch.isinf(rl))
+    fin = torch.isfinite(rl)
+    # the scaled Q is rounded to 16 bits: 2^-9 (bf16) of a score's terms, whose sum over d has a standard deviation of one
+    assert (lse[fin] - rl[fin]).abs().max().item() <= 3e-2 * max(1.0, rl[fin].abs().max().item() / 8)
+
+
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,D,causal,dtype", [
+    (1, 64, 129, 2, 1, 128, True, torch.bfloat16),
+    (1, 65, 257, 4, 2, 128, False, torch.float16),
+    (2, 63, 383, 4, 4, 72, True, torch.bfloat16),
+    (1, 127, 130, 2, 1, 128, True, torch.float16),
+    (1, 3, 1000, 8, 2, 104, True, torch.bfloat16),
+    (1, 300, 140, 2, 2, 128, True, torch.bfloat16),     # rows without a key
+    (1, 4100, 4100, 2, 1, 128, True, torch.bfloat16),
+    (1, 1, 64, 2, 1, 256, False, torch.bfloat16),
+    (1, 128, 65, 2, 1, 256, True, torch.float16),
+    (2, 129, 127, 4, 2, 136, True, torch.bfloat16),
+    (1, 33, 63, 2, 2, 200, False, torch.bfloat16),
+    (1, 700, 450, 2, 1, 256, True, torch.float16),
+])
+@pytest.mark.parametrize("mode", ["0", "2"])
+def test_edges(B, Lq, Lk, H, Hk, D, causal, dtype, mode):
+    print(B, Lq, Lk, H, Hk, D, causal, dtype, mode, flush=True)
+    set_compact(mode)
+    q, k, v, mask, bias = make_inputs(B, Lq, Lk, H, Hk, D, (B, Hk, 1, Lk), (B, Hk, 1, Lk), max(1, Lk // 2), seed=Lq + Lk, dtype=dtype)
+    _check(q, k, v, mask, bias, causal)
+
+
+@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("mode", ["0", "2"])
+def test_climbing_scores_and_empty_groups(D, mode):
+    set_compact(mode)
+    B, Lq, Lk, H, Hk = 1, 100, 900, 2, 1
+    q, k, v, mask, _ = make_inputs(B, Lq, Lk, H, Hk, D, None, (B, Hk, 1, Lk), Lk, seed=3)
+    bias = (torch.arange(Lk).float() * 0.25).view(1, 1, 1, Lk).to(torch.bfloat16)  # (32 keys: 8 in log units, 11 in exponents of two)
+    mask[..., 32:96] = False    # whole key groups of a tile
+    mask[..., 256:640] = False  # whole tiles
+    _check(q, k, v, mask, bias, False)
+    _check(q, k, v, mask, bias, True)
+    mask[:] = False
+    mask[..., 77] = True
+    _check(q, k, v, mask, bias, False)
+
+
+def test_ragged_with_few_blocks():
+    from flash_sparse_attn import flash_sparse_attn_varlen_func
+
+    lens, H, Hk, D = [1, 200, 64, 65, 300], 4, 2, 128
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn(sum(lens), H, D, generator=g).to(torch.bfloat16).to(DEV)
+    k, v = [torch.randn(sum(lens), Hk, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2)]
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    out = flash_sparse_attn_varlen_func(q, k, v, cu, cu, max(lens), max(lens), is_causal=True)
+    at = 0
+    for n in lens:
+        s = slice(at, at + n)
+        assert_out_close(out[s], eager.attention_forward(q[None, s], k[None, s], v[None, s], None, None, None, True)[0][0])
+        at += n
