@@ -18,6 +18,7 @@
 
 #include "fdma_common.h"
 #include "fdma_params.h"
+#include "fdma_bwd_units.h"
 
 namespace fdma {
 
@@ -25,37 +26,9 @@ namespace {
 
 constexpr int NTHREADS = 256;
 
-// XCD-aware work distribution shared by both kernels: `pairs` independent (batch, kv head) pairs with
-// `n_units` units of work each (heaviest first), `k_split` lists of units per pair; see the forward column-mask kernel for the rationale.
-struct XcdMap {
-    int pair, unit;
-    bool valid;
-};
-__host__ __device__ __forceinline__ int xcd_lists_per_pair(int pairs) {
-    const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
-    return 8 / gcd8;
-}
-__device__ __forceinline__ XcdMap xcd_map(int lid, int k_split, int n_units, int per_unit) {
-    const int list_len = ((n_units + k_split - 1) / k_split) * per_unit;
-    const int xcd = lid % 8, slot = lid / 8;
-    const int vlist = xcd + 8 * (slot / list_len);
-    const int pos = slot % list_len;
-    XcdMap m;
-    m.pair = vlist / k_split;
-    m.unit = (pos / per_unit) * k_split + vlist % k_split;
-    m.valid = m.unit < n_units;
-    return m;
-}
-inline int xcd_grid(int pairs, int k_split, int n_units, int per_unit) {
-    return pairs * k_split * ((n_units + k_split - 1) / k_split) * per_unit;
-}
-
 // ------------------------------------------------------------------------------------------------
 // dK / dV / dBias
 // ------------------------------------------------------------------------------------------------
-constexpr int KV_BM = 64;   // query rows per planning block (the work split counts these)
-constexpr int KV_BN = 128;  // key columns per workgroup (32 per wave)
-
 // Query rows per step.  At d = 128 the stationary K / V fragments and the dK / dV accumulators alone take 192 registers
 // per lane; with 32-row steps and V parked in LDS (every lane re-reads its own row: a private spill, no sharing) the
 // kernel fits in 256 registers and 70 KB of LDS, so that two workgroups share a CU and fill each other's stalls.
@@ -69,63 +42,13 @@ template <int D> struct KvcSmem {
     static constexpr int TOTAL = OFF_V + (V_LDS ? KV_BN * S * 2 : 0);
 };
 
-// Entries of a ragged batch longest first and dealt to all XCDs (ragged_lists_per_pair), up to head dim 128: the instantiations
-// at 256 are at the end of their registers (772 bytes of scratch per lane) and keep the plain order.
+// Entries of a ragged batch longest first and dealt to all XCDs (ragged_lists_per_pair), up to head dim 128; at 256 the plain order.
 template <int D> constexpr bool RAGGED_TURNS = D <= 128;
-
-// Unit `u` of a kv head's units in a ragged batch: the blocks of 128 keys of its entries, the entry with the most query rows
-// first, equal ones in their order.  A block of keys walks the rows of its entry; workgroups start in the order of their ids, and
-// one of a long entry that starts last runs on alone.  16384 tokens in entries of 1 to 5394, the longest last, 32 heads over 8,
-// head dim 128: 1396 -> 1247 us.  Ranks and first units come from one comparison per entry and lane; a batch of more entries than a
-// wave has lanes keeps its order (its units are many and small enough to even out).  Units beyond the last: block < 0.
-struct RaggedUnit {
-    int entry, block;
-};
-__device__ inline RaggedUnit ragged_unit(const FwdParams &p, int u) {
-    const int lane = (int)(threadIdx.x & 63);
-    if (p.B > 64) {  // (entry b's units start at cu_k[b] / 128 + b: kv_unit_slot)
-        int e = -1;
-        for (int base = 0; base < p.B; base += 64) {
-            const int b = base + lane;
-            e += __popcll(__ballot(b < p.B && p.cu_k[b] / KV_BN + b <= u));
-        }
-        const int len = p.cu_k[e + 1] - p.cu_k[e], n = u - (p.cu_k[e] / KV_BN + e);
-        return {e, n * KV_BN < len ? n : -1};
-    }
-    const int b = lane < p.B ? lane : 0, len = lane < p.B ? p.cu_q[b + 1] - p.cu_q[b] : -1;
-    const int n = lane < p.B ? (p.cu_k[b + 1] - p.cu_k[b] + KV_BN - 1) / KV_BN : 0;
-    int first = 0;
-    for (int t = 0; t < p.B; t++) {
-        const int other = __builtin_amdgcn_readlane(len, t), nt = __builtin_amdgcn_readlane(n, t);
-        first += (other > len || (other == len && t < lane)) ? nt : 0;
-    }
-    const uint64_t at = __ballot(u >= first && u < first + n);
-    if (!at) return {0, -1};
-    const int e = __builtin_ctzll(at);
-    return {e, u - __builtin_amdgcn_readlane(first, e)};
-}
-
-// Steps per part of a ragged batch (kv_part_quota of all its units' steps): every lane takes entries, the wave adds up.
-__device__ inline int ragged_part_quota(const FwdParams &p, int bm) {
-    int64_t sum = 0;
-    for (int b = (int)(threadIdx.x & 63); b < p.B; b += 64)
-        sum += kv_head_steps(p.cu_q[b + 1] - p.cu_q[b], p.cu_k[b + 1] - p.cu_k[b], p.causal, bm);
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) sum += __shfl_xor((long long)sum, m);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)sum), hi = __builtin_amdgcn_readfirstlane((uint32_t)(sum >> 32));
-    return kv_part_quota((int64_t)(((uint64_t)hi << 32) | lo) * p.H);
-}
-// Where the sums of a unit's parts lie: unit number within the call (times kv_most).  Ragged: entry b's blocks start at
-// cu_k[b] / 128 + b, which leaves every entry the blocks it has.
-__device__ inline int kv_unit_slot(const BwdParams &p, int b, int hk, int n_block) {
-    const int u = p.f.cu_q ? hk * p.kv_units + p.f.cu_k[b] / KV_BN + b + n_block : (b * p.f.Hk + hk) * p.kv_units + n_block;
-    return u * p.kv_most;
-}
 
 // CMP: the key axis is the compacted list of kept columns (fdma_compact.hip); a lane still owns one key,
 // reads it from the dense copies, and writes its gradients to the key's original row / column.
 template <typename T, int D, bool CAUSAL, bool CMP>
-__global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_kernel(const BwdParams p) {
+__global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const BwdParams p) {
     using E = Elem<T>;
     using SM = KvcSmem<D>;
     using TL = LdsTile<D>;
@@ -149,76 +72,10 @@ __global__ void __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) bwd_dkdv_colmask_k
     const FwdParams &f = p.f;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = tid & 63, r = lane & 31, g = lane >> 5;
     const int G = f.H / f.Hk;
-    // work item: a 128-key block of one (batch, kv head) pair, over query heads [g_lo, g_hi) and segment
-    // `seg` of `Sm` of the query range; `slot` >= 0 when the block is shared by several workgroups
-    int pair, n_block, g_lo = 0, g_hi = G, seg = 0, Sm = 1, Q = 1 << 30, slot = -1, part = 0;
-    if (CMP) {
-        const int32_t *plan = f.cmp.plan;
-        const int Gs = plan[1];
-        Sm = plan[2];
-        Q = plan[4];
-        const int per = Gs * Sm;
-        int sub;
-        const int x = blockIdx.x % 8, l = blockIdx.x / 8;
-        if (per > 1) {
-            // Split units: the plan holds, per XCD, the list of the parts that exist -- (pair, unit, part of the
-            // unit), longest parts first.  Workgroup l of an XCD takes entry l; consecutive workgroups of an XCD go
-            // to its shader engines in turn, and with the existing parts side by side every engine gets its share.
-            const int cap = gridDim.x / 8;
-            const int32_t *lists = plan + plan[5];
-            if (l >= lists[x]) return;
-            const int32_t *e = lists + 8 + 2 * ((int64_t)x * cap + l);
-            pair = e[0];
-            n_block = e[1] & 0xffff;
-            sub = e[1] >> 16;
-        } else {
-            // unit lists per XCD: the units of a pair are dealt to its k lists, the lists to the XCDs
-            const int P = f.B * f.Hk, k = dkdv_lists_per_pair(P);
-            const int list_len = plan[3];
-            if (list_len == 0) return;
-            const int ls = l / list_len, pos = l % list_len;
-            if (ls >= P * k / 8) return;
-            const int vlist = x + 8 * ls, fold = vlist % k;
-            pair = vlist / k;
-            n_block = dkdv_unit_at(pos, fold, k);
-            if (n_block >= plan[DKDV_PLAN_HDR + pair + 1] - plan[DKDV_PLAN_HDR + pair]) return;
-            sub = 0;
-        }
-        const int unit = plan[DKDV_PLAN_HDR + pair] + n_block;
-        const int gper = G / Gs;
-        g_lo = (sub / Sm) * gper;
-        g_hi = g_lo + gper;
-        seg = sub % Sm;
-        if (per > 1) slot = unit * per + sub;
-    } else {
-        const int n_nb = (f.Lk + KV_BN - 1) / KV_BN;
-        const bool ragged = RAGGED_TURNS<D> && f.cu_q;
-        const int k = ragged ? ragged_lists_per_pair(f) : xcd_lists_per_pair(f.B * f.Hk), n_units = ragged ? p.kv_units : n_nb;
-        XcdMap wm;
-        if (p.kv_most > 1) {
-            // A list holds its units once per part, the LAST parts first: those exist for the longest units only.  Workgroups
-            // side by side go to the shader engines of an XCD in turn, whether they stay or return at once: with the parts of
-            // a unit side by side instead, the engines that got the missing ones idled (ragged, 16384 tokens, two parts at
-            // most: 1966 us instead of 1224 without parts).
-            const int per_list = (n_units + k - 1) / k, pos = (int)(blockIdx.x / 8) % (per_list * p.kv_most);
-            part = p.kv_most - 1 - pos / per_list;
-            const int vlist = (int)(blockIdx.x % 8) + 8 * ((int)(blockIdx.x / 8) / (per_list * p.kv_most));
-            wm.pair = vlist / k;
-            wm.unit = pos % per_list * k + vlist % k;
-            wm.valid = wm.unit < n_units;
-        } else {
-            wm = xcd_map(blockIdx.x, k, n_units, 1);
-        }
-        if (!wm.valid) return;
-        n_block = wm.unit;  // low key blocks are seen by the most queries under causal: heaviest first
-        pair = wm.pair;
-        if (ragged) {
-            const RaggedUnit ru = ragged_unit(f, n_block);
-            if (ru.block < 0 || ru.block >= n_nb) return;  // (rows beyond the longest length that the caller names: not computed)
-            n_block = ru.block;
-            pair = ru.entry * f.Hk + wm.pair;
-        }
-    }
+    const KvItem it = kv_item<CMP>(p, RAGGED_TURNS<D>);
+    if (!it.valid) return;
+    const int pair = it.pair, n_block = it.n_block, g_lo = it.g_lo, g_hi = it.g_hi, seg = it.seg, Sm = it.Sm, Q = it.Q, part = it.part;
+    int slot = it.slot;
     const int b = pair / f.Hk, hk = pair % f.Hk;
     const int n0 = n_block * KV_BN;
     const SeqInfo sq = seq_info(f, b);  // this batch entry's lengths and first rows (ragged batch: from cu_seqlens)
@@ -986,25 +843,33 @@ inline RedInterleave red_interleave(int dq_octets, int items) {
 }
 
 template <typename T, int D, bool CAUSAL, bool CMP>
+hipError_t launch_dkdv_grid(const BwdParams &p, int grid, hipStream_t stream) {
+    if constexpr (D > 128) {
+        return launch_bwd_dkdv_256(p, std::is_same<T, bf16_tag>::value ? 0 : 1, grid, stream);
+    } else {
+        auto kern = bwd_dkdv_colmask_kernel<T, D, CAUSAL, CMP>;
+        const int smem = KvcSmem<D>::TOTAL;
+        static DynSmemLimit smem_limit;
+        hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(NTHREADS), smem, stream, p);
+        return hipGetLastError();
+    }
+}
+template <typename T, int D, bool CAUSAL, bool CMP>
 hipError_t launch_dkdv_c(const BwdParams &p, hipStream_t stream) {
     const FwdParams &f = p.f;
-    auto kern = bwd_dkdv_colmask_kernel<T, D, CAUSAL, CMP>;
-    const int smem = KvcSmem<D>::TOTAL;
-    static DynSmemLimit smem_limit;
-    hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
-    if (e != hipSuccess) return e;
     if (CMP) {
         int grid, slots;
         dkdv_split_bounds(f.B * f.Hk, (f.Lk + KV_BN - 1) / KV_BN, f.H / f.Hk, grid, slots);
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(NTHREADS), smem, stream, p);
-        return hipGetLastError();  // (the partial results are summed by workgroups of the dQ launch)
+        return launch_dkdv_grid<T, D, CAUSAL, CMP>(p, grid, stream);  // (the partial results are summed by workgroups of the dQ launch)
     }
     const int n_nb = (f.Lk + KV_BN - 1) / KV_BN;
-    const bool ragged = RAGGED_TURNS<D> && f.cu_q;  // (a kv head's units are numbered over all entries)
-    dim3 grid(ragged ? xcd_grid(f.Hk, ragged_lists_per_pair(f), p.kv_units, p.kv_most) : xcd_grid(f.B * f.Hk, xcd_lists_per_pair(f.B * f.Hk), n_nb, p.kv_most));
-    hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
-    if ((e = hipGetLastError()) != hipSuccess || p.kv_most <= 1) return e;
-    const int64_t pieces = (int64_t)(ragged ? 1 : f.B) * f.Hk * p.kv_units * (2 * KV_BN * D / 8 / NTHREADS);
+    const bool turns = RAGGED_TURNS<D> && f.cu_q;  // (a kv head's units are numbered over all entries)
+    const int grid = turns ? xcd_grid(f.Hk, ragged_lists_per_pair(f), p.kv_units, p.kv_most) : xcd_grid(f.B * f.Hk, xcd_lists_per_pair(f.B * f.Hk), n_nb, p.kv_most);
+    const hipError_t e = launch_dkdv_grid<T, D, CAUSAL, CMP>(p, grid, stream);
+    if (e != hipSuccess || p.kv_most <= 1) return e;
+    const int64_t pieces = (int64_t)(f.cu_q ? 1 : f.B) * f.Hk * p.kv_units * (2 * KV_BN * D / 8 / NTHREADS);
     hipLaunchKernelGGL((bwd_dkdv_parts_sum_kernel<T, D>), dim3((unsigned)(pieces < 2048 ? pieces : 2048)), dim3(NTHREADS), 0, stream, p);
     return hipGetLastError();
 }
@@ -1588,7 +1453,7 @@ size_t plan_kv_parts(BwdParams &p, size_t *db_bytes) {
     p.kv_quota = 0;
     p.kv_units = f.cu_q ? f.total_k / KV_BN + f.B : (f.Lk + KV_BN - 1) / KV_BN;
     *db_bytes = 0;
-    if (f.Lq <= 0 || f.Lk <= 0 || f.cmp.on || (f.cu_q && f.d > 128)) return 0;
+    if (f.Lq <= 0 || f.Lk <= 0 || f.cmp.on) return 0;
     const int G = f.H / f.Hk, bm = kv_step_rows(f.d);
     const int64_t longest = (int64_t)G * kv_unit_steps(f.Lq, f.Lk, f.causal, 0, bm);
     const int64_t units = (int64_t)(f.cu_q ? 1 : f.B) * f.Hk * p.kv_units;

@@ -328,6 +328,7 @@ hipError_t launch_bwd(const BwdParams &p, int dtype, hipStream_t stream);
 // column-mask specialisations of the two main backward kernels
 bool bwd_colmask_applicable(const BwdParams &p);
 hipError_t launch_bwd_dkdv_colmask(const BwdParams &p, int dtype, hipStream_t stream);
+hipError_t launch_bwd_dkdv_256(const BwdParams &p, int dtype, int grid, hipStream_t stream);  // its kernel at head dims 129 .. 256 (fdma_bwd_dkdv_256.hip)
 hipError_t launch_bwd_dq_colmask(const BwdParams &p, int dtype, hipStream_t stream);
 // parts the units of the dK/dV kernel on the original key axis are cut into: fills kv_most / kv_quota / kv_units and returns the
 // bytes of their sums (0: whole); *db_bytes: of their dBias columns

@@ -82,6 +82,8 @@ def test_column_form(B, Lq, Lk, H, Hk, D, Hb, causal, dtype, monkeypatch):
     ([1000, 2], None, 8, 4, 64, True, torch.float16),
     ([0, 513, 64], [100, 700, 0], 6, 3, 96, False, torch.bfloat16),
     ([257, 500, 1], [900, 129, 128], 4, 2, 128, True, torch.float16),
+    ([300, 1, 700, 33], None, 4, 1, 256, True, torch.bfloat16),
+    ([129, 500], [260, 90], 4, 2, 136, False, torch.float16),
     ([40] * 70 + [900], None, 2, 1, 128, True, torch.bfloat16),   # more entries than a wave has lanes
 ])
 def test_ragged(lens_q, lens_k, H, Hk, D, causal, dtype, monkeypatch):
@@ -115,3 +117,26 @@ def test_ragged(lens_q, lens_k, H, Hk, D, causal, dtype, monkeypatch):
     for x, y in zip(parts, again):
         assert torch.equal(x, y)
     _close(parts, whole, names)
+
+
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,D,Hb,causal,dtype", [
+    (1, 300, 700, 4, 2, 256, 2, True, torch.bfloat16),     # few units: cut by heads and segments
+    (2, 65, 500, 2, 2, 136, 1, False, torch.float16),
+    (1, 513, 513, 6, 2, 200, 6, True, torch.bfloat16),
+    (1, 600, 140, 2, 1, 256, 0, True, torch.float16),      # rows without a key
+    (4, 1100, 1400, 40, 20, 256, 20, True, torch.bfloat16),  # enough units of kept keys: none is cut
+])
+def test_compacted_above_128(B, Lq, Lk, H, Hk, D, Hb, causal, dtype):
+    """The wave pairs of head dims above 128 on compacted keys."""
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func
+
+    print("compacted", B, Lq, Lk, H, Hk, D, Hb, causal, dtype, flush=True)
+    _cabi.set_compact_mode(_cabi.COMPACT_ALWAYS)
+    q, k, v, mask, bias = make_inputs(B, Lq, Lk, H, Hk, D, (B, Hb, 1, Lk) if Hb else None, (B, Hk, 1, Lk), Lk // 2, seed=Lq + D, dtype=dtype)
+    q, k, v, mask = [t.to(DEV) for t in (q, k, v, mask)]
+    leaves = [t.requires_grad_(True) for t in (q, k, v)] + ([bias.to(DEV).requires_grad_(True)] if Hb else [])
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(1)).to(dtype).to(DEV)
+    ref = eager.attention_forward_backward(q.detach(), k.detach(), v.detach(), mask, leaves[3].detach() if Hb else None, None, causal, dout)
+    out = flash_sparse_attn_func(*leaves[:3], mask, leaves[3] if Hb else None, None, causal)
+    for got, want, name in zip(torch.autograd.grad(out, leaves, dout), ref[1:], ("dq", "dk", "dv", "dbias")):
+        assert_grad_close(got, want, name)
