@@ -21,7 +21,10 @@
 //   * everything is double-buffered and fetched a tile ahead, the mask two tiles ahead: the workgroup-wide OR
 //     of the next tile's mask is known before that tile's bias / K / V loads are issued, and a tile without
 //     any kept element costs its mask bytes only (no bias, K, V traffic, no MFMA work);
-//   * one barrier per tile: the OR reduction is that barrier.
+//   * one barrier per tile, which the vote of the OR is published by (__syncthreads_or is three: 6 us of 74 at 1999 x 16 heads,
+//     d = 128).
+#include <type_traits>
+
 #include "fdma_common.h"
 #include "fdma_params.h"
 
@@ -33,27 +36,29 @@ namespace {
 // and with a single wave per SIMD nothing hides the in-order issue of that wave -- a second wave per SIMD does.  On grids
 // that stay large enough the 8 waves cover 256 rows; on smaller ones (KSPLIT) 128 rows, two waves per 32 rows that take
 // the lower and the upper half of every key tile with a softmax of their own and are merged through LDS at the end
-// (B = 1, L = 1999, H = 16, d = 128, fp16: 108 us with four waves, 88 so, the rows read where they lie).
+// (B = 1, L = 1999, H = 16, d = 128, fp16: 108 us with four waves, 88 so, the rows read where they lie; 57 with K / V by direct
+// loads, one barrier per tile and four heads to a workgroup).
 constexpr int BN_DEFAULT = 64;  // keys per tile (32 at head dims above 128: LDS)
 
 template <int D, int BM, int BN> struct FwdSmem {
-    static constexpr int SK = D + 8;     // K tile row stride (elements): conflict-free 16-byte row reads
-    static constexpr int SV = LdsTile<D>::S;  // V tile row stride (row-major like K, read through transposing LDS reads)
     static constexpr int SF = BN + 8;    // fused mask+bias tile row stride
-    static constexpr int K_BYTES = BN * SK * 2;
-    static constexpr int VT_BYTES = BN * SV * 2;
+    static constexpr int K_BYTES = BN * LdsTile<D>::ROW_BYTES;  // a K or V tile (row-major both; V is read through transposing LDS reads)
     static constexpr int F_BYTES = BM * SF * 2;
-    static constexpr int STAGE = K_BYTES + VT_BYTES + F_BYTES;
-    static constexpr int TOTAL = 2 * STAGE;
+    static constexpr int STAGE = (2 * K_BYTES + F_BYTES + 255) / 256 * 256;
+    static constexpr int OFF_VOTE = 2 * STAGE;  // three words: "a tile has a kept element"
+    static constexpr int TOTAL = OFF_VOTE + 16;
 };
 
 template <typename T> struct NegInf2;
 template <> struct NegInf2<bf16_tag> { static constexpr uint32_t value = 0xFF80FF80u; };
 template <> struct NegInf2<fp16_tag> { static constexpr uint32_t value = 0xFC00FC00u; };
 
-template <typename T, int D, bool CAUSAL, int NW, int BN, int KSPLIT, bool ODD>
+// GH query heads of a kv group that share mask and bias rows: a workgroup takes BM / GH query rows of GH heads, so that a fused tile
+// is fetched, fused and stored once for all of them.
+template <typename T, int D, bool CAUSAL, int NW, int BN, int KSPLIT, int GH, bool ODD>
 __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_kernel(const FwdParams p) {
-    constexpr int NTHREADS = 64 * NW, BM = 32 * NW / KSPLIT, BK = BN / KSPLIT;  // (BK: keys of a tile per wave)
+    constexpr int NTHREADS = 64 * NW, BK = BN / KSPLIT;  // (BK: keys of a tile per wave)
+    constexpr int BM = 32 * NW / KSPLIT / GH, RB = BM / 32;  // query rows and 32-row blocks per head
     constexpr int FCH = BN / 8;             // 8-key chunks per mask / bias row of a tile
     constexpr int F_RPP = NTHREADS / FCH;   // mask / bias rows staged per pass (FCH threads cover the keys of a row)
     using E = Elem<T>;
@@ -64,21 +69,31 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     constexpr int CH = D / 8;               // 16-byte chunks per K row
     constexpr int K_RPP = NTHREADS / CH;    // K rows staged per pass
     constexpr int K_IT = BN / K_RPP;
-    constexpr int F_IT = BM * (BN / 8) / NTHREADS;  // 8-key chunks of the mask / bias tile per thread (4)
+    constexpr int F_CHUNKS = BM * (BN / 8);  // 8-key chunks of the mask / bias tile
+    constexpr int F_IT = F_CHUNKS > NTHREADS ? F_CHUNKS / NTHREADS : 1;  // ... per thread (the last waves fetch some again, when there are fewer)
 
-    extern __shared__ __attribute__((aligned(16))) char smem[];
+    using TL = LdsTile<D>;
+    // DMA (rows of exactly 256 bytes): K and V tiles go from global memory straight into LDS (global_load_lds; the swizzle of the
+    // tile is applied to the global address of each lane's piece).  Through registers, their loads and stores were a fifth of
+    // the kernel at head dim 128.
+    constexpr bool DMA = TL::SWZ;
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 31, g = lane >> 5;
+    extern __shared__ __attribute__((aligned(256))) char smem[];
+    const uint32_t lds0 = lds_addr(smem);  // (a multiple of 256)
+
+    const int tid = threadIdx.x, wave = DMA ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : (int)threadIdx.x >> 6, lane = tid & 63, r = lane & 31, g = lane >> 5;
     // linear workgroup id -> (query block, member of the kv group, kv head, batch) with the query block OUTERMOST and
     // descending: under causal masking the blocks with the most KV tiles of every head start first, the light ones fill the
     // tail.  The members of a group, which read the same K / V and often the same mask and bias, are a multiple of the kv
     // head count apart: on one XCD (ids are dealt to the 8 XCDs in turn) when that is a multiple of 8.
-    const int hb_count = p.H * p.B, pairs = p.Hk * p.B;
+    const int hb_count = p.H / GH * p.B, pairs = p.Hk * p.B;
     const int m_block = (int)gridDim.x / hb_count - 1 - (int)blockIdx.x / hb_count;
     const int pair = (int)blockIdx.x % pairs, hk = pair % p.Hk, b = pair / p.Hk;
-    const int h = hk * (p.H / p.Hk) + ((int)blockIdx.x % hb_count) / pairs;
+    const int hs = wave % (RB * GH) / RB;  // head of this wave among the workgroup's
+    const int h = hk * (p.H / p.Hk) + ((int)blockIdx.x % hb_count) / pairs * GH + hs;
     const int m0 = m_block * BM;
-    const int rw = wave % (BM / 32), kh = wave / (BM / 32);  // row block and key half of this wave
+    const int rw = wave % RB, kh = wave / (RB * GH);  // row block and key half of this wave
+    const int xw = wave % (RB * GH);  // (rows and heads: where the halves meet)
     const int wrow0 = m0 + rw * 32;
     const int qrow = wrow0 + r;
     const int shift = p.Lk - p.Lq;  // bottom-right causal alignment
@@ -127,8 +142,8 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     // ---- staging maps
     const int kc = tid % CH, kr0 = tid / CH;             // K: d chunk, first row
     const bool k_dvalid = kc * 8 < p.d;
-    const int fc = tid % FCH, fr0 = tid / FCH;           // mask / bias: 8-key chunk, first row (rows fr0 + F_RPP it)
-    u32x4_t kreg[K_IT], vreg[K_IT], breg[F_IT];
+    const int fc = tid % FCH, fr0 = tid / FCH % BM;      // mask / bias: 8-key chunk, first row (rows fr0 + F_RPP it)
+    u32x4_t kreg[DMA ? 1 : K_IT], vreg[DMA ? 1 : K_IT], breg[F_IT];
     u32x2_t mreg[F_IT], mnext[F_IT];
 
     // All tile loads are unconditional, from clamped (always valid) addresses, so that they can be issued early and
@@ -136,6 +151,9 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     // words are ANDed with a validity pattern when they are consumed, rows of K / V beyond Lk and head-dim chunks
     // beyond d are finite duplicates that meet a -inf score or a zero Q fragment.
     const int kcol = k_dvalid ? kc * 8 : 0;
+    // (DMA: the lane fills chunk POSITION kc of its rows, which holds chunk kc ^ swz(row) of the global row; rows 32 apart have the
+    // same swizzle)
+    const int kc_g = kc ^ (int)TL::swz(kr0), kcol_g = kc_g * 8 < p.d ? kc_g * 8 : 0;
     // (a mask that comes packed to bits: one byte per 8-key chunk instead of eight, expanded where it is looked at)
     const uint8_t *mbits = (mbase && p.mbits) ? p.mbits + b * p.mb_b + hm * p.mb_h : nullptr;
     auto load_mask = [&](int j, u32x2_t (&dst)[F_IT]) {
@@ -187,9 +205,29 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             for (int it = 0; it < F_IT; it++) dst[it] = u32x4_t{0, 0, 0, 0};
         }
     };
-    // K and V of tile j into registers
+    // K and V of tile j into registers, or (DMA) on their way into the tile's stage: in assembly and waited for by hand (kv_landed),
+    // because behind the compiler's builtin every LDS read waits for all LDS operations in flight
+    typedef const __attribute__((address_space(1))) char *gptr_t;
+    auto uniform_ptr = [](const void *ptr) -> gptr_t {
+        const uint64_t v = (uint64_t)ptr;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+        return (gptr_t)(((uint64_t)hi << 32) | lo);
+    };
     auto load_kv = [&](int j) {
         const int n0 = j * BN;
+        if constexpr (DMA) {
+            const gptr_t kb = uniform_ptr(kbase + (int64_t)n0 * p.k_r), vb = uniform_ptr(vbase + (int64_t)n0 * p.v_r);
+            const int last = p.Lk - 1 - n0;
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)((j & 1) * SM::STAGE) + (uint32_t)wave * 1024);
+#pragma unroll
+            for (int it = 0; it < K_IT; it++) {
+                const int row = kr0 + it * K_RPP, row_c = row < last ? row : last;
+                const uint32_t ko = (uint32_t)(row_c * (int)p.k_r + kcol_g) * 2, vo = (uint32_t)(row_c * (int)p.v_r + kcol_g) * 2;
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(ko), "s"(kb), "s"(dst + it * K_RPP * 256) : "memory");
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(vo), "s"(vb), "s"(dst + SM::K_BYTES + it * K_RPP * 256) : "memory");
+            }
+            return;
+        }
 #pragma unroll
         for (int it = 0; it < K_IT; it++) {
             int key = n0 + kr0 + it * K_RPP;
@@ -208,13 +246,16 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     auto store_stage = [&](int j, const u32x2_t (&mv)[F_IT], const u32x4_t (&bsrc)[F_IT]) {
         const int buf = j & 1, kk = j * BN + 8 * fc;
         char *sK = smem + buf * SM::STAGE;
-        char *sVt = sK + SM::K_BYTES;
-        char *sF = sVt + SM::VT_BYTES;
+        char *sV = sK + SM::K_BYTES;
+        char *sF = sV + SM::K_BYTES;
+        if constexpr (!DMA) {
 #pragma unroll
-        for (int it = 0; it < K_IT; it++) {
-            *(u32x4_t *)(sK + ((kr0 + it * K_RPP) * SM::SK + kc * 8) * 2) = kreg[it];
-            *(u32x4_t *)(sVt + LdsTile<D>::chunk(kr0 + it * K_RPP, kc)) = vreg[it];
+            for (int it = 0; it < K_IT; it++) {
+                *(u32x4_t *)(sK + TL::chunk(kr0 + it * K_RPP, kc)) = kreg[it];
+                *(u32x4_t *)(sV + TL::chunk(kr0 + it * K_RPP, kc)) = vreg[it];
+            }
         }
+        if (F_CHUNKS < NTHREADS && wave >= F_CHUNKS / 64) return;
 #pragma unroll
         for (int it = 0; it < F_IT; it++) {
             u32x4_t bv = bbase ? chunk8_fix<ODD>(bsrc[it], kk, p.Lk) : bsrc[it];
@@ -234,14 +275,14 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
 
     const int a_row = pi_row(r);
     // (this lane's part of the address of a transposing read of the V tile)
-    const uint32_t tr_lane = LdsTile<D>::tr_base(g, (lane & 15) >> 2, (lane >> 4) & 1, (lane & 3) == 1 ? 2 : ((lane & 3) == 2 ? 1 : (lane & 3)));
+    const uint32_t tr_lane = TL::tr_base(g, (lane & 15) >> 2, (lane >> 4) & 1, (lane & 3) == 1 ? 2 : ((lane & 3) == 2 ? 1 : (lane & 3)));
 
     // ---- one tile from LDS stage `buf`
     auto compute = [&](int j, int buf) {
         const int n0 = j * BN + kh * BK;
-        const char *sK = smem + buf * SM::STAGE + kh * BK * SM::SK * 2;
-        const char *sVt = smem + buf * SM::STAGE + SM::K_BYTES + kh * BK * LdsTile<D>::ROW_BYTES;
-        const char *sF = smem + buf * SM::STAGE + SM::K_BYTES + SM::VT_BYTES + ((rw * 32 + r) * SM::SF + kh * BK + 8 * g) * 2;
+        const uint32_t a_k = lds0 + (uint32_t)(buf * SM::STAGE + kh * BK * TL::ROW_BYTES) + TL::frag_base(a_row, g);
+        const uint32_t tr_v = lds0 + (uint32_t)(buf * SM::STAGE + SM::K_BYTES + kh * BK * TL::ROW_BYTES) + tr_lane;
+        const char *sF = smem + buf * SM::STAGE + 2 * SM::K_BYTES + ((rw * 32 + r) * SM::SF + kh * BK + 8 * g) * 2;
         // scores start from the fused mask+bias tile (exp2 domain)
         f32x16_t s[MB];
 #pragma unroll
@@ -260,7 +301,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             u32x4_t a[NF];
             auto frag = [&](int f) {
                 const int ks = f / MB, mb = f % MB;
-                return *(const u32x4_t *)(sK + ((32 * mb + a_row) * SM::SK + ks * 16 + g * 8) * 2);
+                return lds_ld128(TL::frag_at(a_k, ks) + (uint32_t)(32 * mb * TL::ROW_BYTES));
             };
 #pragma unroll
             for (int f = 0; f < FR; f++) a[f] = frag(f);
@@ -318,10 +359,9 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             // V^T (rows of the A operand = head dim) through transposing reads of the row-major V tile
             constexpr int NF = KB * DB, FR = NF < 8 ? NF : 8;
             u32x4_t a[NF];
-            const uint32_t tr_v = lds_addr(sVt) + tr_lane;
             auto frag = [&](int f) {
                 const int kb = f / DB, db = f % DB;
-                const u32x2_t lo = lds_ld_tr16(LdsTile<D>::tr_at(tr_v, kb, db, 0)), hi = lds_ld_tr16(LdsTile<D>::tr_at(tr_v, kb, db, 1));
+                const u32x2_t lo = lds_ld_tr16(TL::tr_at(tr_v, kb, db, 0)), hi = lds_ld_tr16(TL::tr_at(tr_v, kb, db, 1));
                 return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
             };
 #pragma unroll
@@ -335,6 +375,28 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             }
         }
     };
+
+    // The end of a step: "has any thread a kept element of that tile", published by the barrier that publishes the step's LDS
+    // stores and direct loads.  (The word of vote i is set in front of barrier i, read behind it, and cleared between barriers i + 1
+    // and i + 2 for vote i + 3.)  `younger`: mask and bias loads that this wave has issued behind the direct loads that must
+    // have landed.
+    int vote_at = 0;
+    if (tid < 3) lds_st32(lds0 + SM::OFF_VOTE + 4 * tid, 0u);
+    auto step_end = [&](bool any, int younger) -> bool {
+        const uint32_t at = lds0 + SM::OFF_VOTE + 4 * vote_at;
+        vote_at = vote_at == 2 ? 0 : vote_at + 1;
+        if (__any(any)) lds_st32(at, 1u);
+        if (tid == 0) lds_st32(lds0 + SM::OFF_VOTE + 4 * vote_at, 0u);
+        if constexpr (DMA) {
+            if (younger >= 2 * F_IT) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(2 * F_IT) : "memory");
+            else if (younger >= F_IT) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(F_IT) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        } else {
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        }
+        return __builtin_amdgcn_readfirstlane(lds_ld32(at)) != 0u;
+    };
+    const int n_mask = mbase ? F_IT : 0, n_bias = bbase ? F_IT : 0;
 
     // ---- main loop.  At the top of iteration j: tile j sits in LDS stage j&1 if it is active, `mreg` holds
     // the mask of tile j+1 and `act_next` says whether that tile has any kept element.
@@ -357,6 +419,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             load_rest(0);
             store_stage(0, mreg, breg);
         }
+        if (DMA) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
         bool act_1 = __syncthreads_or(n_end > 1 && finish_mask(1, m1));
         if (act_1) load_bias(1, b1);
         bool act_2 = __syncthreads_or(n_end > 2 && finish_mask(2, m2));
@@ -375,7 +438,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             if (act_cur) compute(j, j & 1);
             __builtin_amdgcn_sched_barrier(0);
             if (have_next) store_stage(j + 1, ma, ba);
-            const bool act_3 = __syncthreads_or(j + 3 < n_end && finish_mask(j + 3, mc));
+            const bool act_3 = step_end(j + 3 < n_end && finish_mask(j + 3, mc), (j + 4 < n_end ? n_mask : 0) + (j + 2 < n_end && act_2 ? n_bias : 0));
             act_cur = have_next;
             act_1 = act_2;
             act_2 = act_3;
@@ -395,6 +458,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             load_rest(0);
             store_stage(0, mreg, breg);
         }
+        if (DMA) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
         bool act_next = __syncthreads_or(n_end > 1 && finish_mask(1, mnext));
         // one iteration; `m_next` holds the (finished) mask of tile j+1, `m_new` receives the mask of tile j+2.
         // The scheduling barriers keep the loads at the top and their first use below the compute: their
@@ -407,7 +471,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             if (act_cur) compute(j, j & 1);
             __builtin_amdgcn_sched_barrier(0);
             if (have_next) store_stage(j + 1, m_next, breg);
-            const bool act_nn = __syncthreads_or(j + 2 < n_end && finish_mask(j + 2, m_new));
+            const bool act_nn = step_end(j + 2 < n_end && finish_mask(j + 2, m_new), 0);
             act_cur = have_next;
             act_next = act_nn;
         };
@@ -421,12 +485,12 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     float total = xhalf_sum(row_sum);
     if constexpr (KSPLIT == 2) {
         // the upper key half hands over its sums and O (relative to its own maximum); the lower half merges and stores
-        float *xm = (float *)smem + rw * 64 + lane;                                    // maximum, sum: 2 * BM / 32 * 64 floats
-        f32x4_t *xo = (f32x4_t *)(smem + 2 * (BM / 32) * 256) + rw * DB * 4 * 64 + lane;
+        float *xm = (float *)smem + xw * 64 + lane;                                    // maximum, sum: 2 * RB * GH * 64 floats
+        f32x4_t *xo = (f32x4_t *)(smem + 2 * (RB * GH) * 256) + xw * DB * 4 * 64 + lane;
         __syncthreads();  // (the tiles' last reads)
         if (kh == 1) {
             xm[0] = row_max;
-            xm[(BM / 32) * 64] = total;
+            xm[(RB * GH) * 64] = total;
 #pragma unroll
             for (int db = 0; db < DB; db++)
 #pragma unroll
@@ -435,7 +499,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
         }
         __syncthreads();
         if (kh == 1) return;
-        const float m1 = xm[0], t1 = xm[(BM / 32) * 64];
+        const float m1 = xm[0], t1 = xm[(RB * GH) * 64];
         const float mx = fmaxf(row_max, m1), safe = mx == -INFINITY ? 0.f : mx;
         const float w0 = fast_exp2(row_max - safe), w1 = fast_exp2(m1 - safe);
         total = total * w0 + t1 * w1;
@@ -472,23 +536,41 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     }
 }
 
-template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, bool ODD>
+// Query heads per workgroup: 4 or 2 of a kv group, where they share mask and bias rows.  One head / four (us): 1999 x 16/4 heads, d = 128,
+// fp16 70.8 / 57.3, 1231 x 8/2 44.8 / 34.8; d = 64, 4 x 724 x 32/8 39.5 / 28.8, 4096 x 8/2 120 / 107.  Two: d = 128, 2 x 2112 x 8/4
+// 62.7 / 57.7, d = 256, 700 x 32/8 59.2 / 55.2 (four would leave each 32 rows); not at d <= 64 (1984 x 16/8 61.2 / 65.2).
+int shared_rows(const FwdParams &p) {
+    const int G = p.H / p.Hk;
+    if (G > 1 && ((p.mask && p.Hm == p.H) || (p.bias && p.Hb == p.H))) return 1;
+    if (p.d <= 128 && G % 4 == 0) return 4;
+    return p.d > 64 && G % 2 == 0 ? 2 : 1;
+}
+
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD>
 hipError_t launch_fwd_o(const FwdParams &p, hipStream_t stream) {
-    constexpr int BM = 32 * NW / KSPLIT, NTHREADS = 64 * NW, BN = D > 128 ? 32 : BN_DEFAULT;
-    auto kern = fwd_kernel<T, D, CAUSAL, NW, BN, KSPLIT, ODD>;
-    const int smem = FwdSmem<D, BM, BN>::TOTAL;
+    constexpr int BM = 32 * NW / KSPLIT / GH, NTHREADS = 64 * NW, BN = D > 128 ? 32 : BN_DEFAULT;
+    auto kern = fwd_kernel<T, D, CAUSAL, NW, BN, KSPLIT, GH, ODD>;
+    constexpr int merge = KSPLIT == 2 ? (NW / 2) * 512 + (NW / 2) * (D / 32) * 4096 : 0;  // the upper halves' sums
+    constexpr int smem = FwdSmem<D, BM, BN>::TOTAL > merge ? FwdSmem<D, BM, BN>::TOTAL : merge;
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
-    dim3 grid(((p.Lq + BM - 1) / BM) * p.H * p.B);
+    dim3 grid(((p.Lq + BM - 1) / BM) * (p.H / GH) * p.B);
     hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
     return hipGetLastError();
 }
 
 template <typename T, int D, bool CAUSAL, int NW, int KSPLIT = 1>
 hipError_t launch_fwd_c(const FwdParams &p, hipStream_t stream) {
-    if (D > 128 || odd_rows(p)) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, true>(p, stream);
-    return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, D <= 128 ? false : true>(p, stream);
+    const int gh = shared_rows(p);
+    auto pick = [&](auto odd) -> hipError_t {
+        constexpr bool O = decltype(odd)::value;
+        if constexpr (D <= 128) if (gh == 4) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, 4, (D > 64) || O>(p, stream);
+        if constexpr (D > 64) if (gh == 2) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, 2, true>(p, stream);
+        return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, 1, O>(p, stream);
+    };
+    if (D > 128 || odd_rows(p)) return pick(std::true_type());
+    return pick(std::bool_constant<(D > 128)>());
 }
 
 template <typename T, int D>
