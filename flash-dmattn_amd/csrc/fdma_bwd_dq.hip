@@ -11,6 +11,8 @@
 // coalesced loads of every 128 x 64 mask and bias tile, fused in registers into one 16-bit tile in LDS that the score
 // accumulators start from; K, V and the fused tile double-buffered and fetched a tile ahead, the mask two tiles
 // ahead so that a tile without any kept element costs its mask bytes only; one barrier per tile (the OR reduction).
+#include <type_traits>
+
 #include "fdma_common.h"
 #include "fdma_params.h"
 
@@ -22,24 +24,25 @@ namespace {
 // a second wave per SIMD hides what a single wave's in-order issue cannot.  On grids that stay large enough the 8 waves
 // cover 256 rows; on smaller ones (KSPLIT) 128 rows, two waves per 32 rows that take the lower and the upper half of every
 // key tile and add their sums through LDS at the end (B = 1, L = 1999, H = 16, d = 128, fp16: 128 us with four waves, 108
-// so, odd rows read where they lie).  Key tiles have 64 keys, and 32 with 256 rows (the 64-key tile's score and dP accumulators
+// so, odd rows read where they lie; 78 with K / V by direct loads, one barrier per tile and four heads to a workgroup).  Key tiles have 64 keys, and 32 with 256 rows (the 64-key tile's score and dP accumulators
 // do not fit next to dQ and the Q / dO fragments in the 256 registers a wave has when two share a SIMD).
 template <int D, int BM, int BN> struct DqSmem {
-    static constexpr int S = D + 8;      // K / V tile row stride (elements)
     static constexpr int SF = BN + 8;    // fused mask+bias tile row stride
-    static constexpr int K_BYTES = BN * S * 2;
+    static constexpr int K_BYTES = BN * LdsTile<D>::ROW_BYTES;
     static constexpr int F_BYTES = BM * SF * 2;
-    static constexpr int STAGE = 2 * K_BYTES + F_BYTES;
-    static constexpr int TOTAL = 2 * STAGE;
+    static constexpr int STAGE = (2 * K_BYTES + F_BYTES + 255) / 256 * 256;
+    static constexpr int OFF_VOTE = 2 * STAGE;  // three words: "a tile has a kept element"
+    static constexpr int TOTAL = OFF_VOTE + 16;
 };
 
 template <typename T> struct NegInf2;
 template <> struct NegInf2<bf16_tag> { static constexpr uint32_t value = 0xFF80FF80u; };
 template <> struct NegInf2<fp16_tag> { static constexpr uint32_t value = 0xFC00FC00u; };
 
-template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, bool ODD>
+// GH query heads of a kv group that share mask and bias rows: a workgroup takes BM / GH query rows of GH heads (see fwd_kernel).
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD>
 __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_kernel(const BwdParams p) {
-    constexpr int NTHREADS = 64 * NW, BM = 32 * NW / KSPLIT, BN = ((NW == 8 && KSPLIT == 1) || D > 128) ? 32 : 64;
+    constexpr int NTHREADS = 64 * NW, BM = 32 * NW / KSPLIT / GH, RB = BM / 32, BN = ((NW == 8 && KSPLIT == 1) || D > 128) ? 32 : 64;
     constexpr int BK = BN / KSPLIT;         // keys of a tile per wave
     constexpr int FCH = BN / 8;             // 8-key chunks per mask / bias row of a tile
     constexpr int F_RPP = NTHREADS / FCH;   // mask / bias rows staged per pass
@@ -49,22 +52,28 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
     constexpr int CH = D / 8;               // 16-byte chunks per K / V row
     constexpr int K_RPP = NTHREADS / CH;    // rows staged per pass
     constexpr int K_IT = BN / K_RPP;
-    constexpr int F_IT = BM * FCH / NTHREADS;  // 8-key chunks of the mask / bias tile per thread
+    constexpr int F_CHUNKS = BM * FCH;         // 8-key chunks of the mask / bias tile
+    constexpr int F_IT = F_CHUNKS > NTHREADS ? F_CHUNKS / NTHREADS : 1;  // ... per thread (the last waves fetch some again, when there are fewer)
+    using TL = LdsTile<D>;
+    constexpr bool DMA = TL::SWZ;  // K and V tiles by direct loads (see fwd_kernel)
 
-    extern __shared__ __attribute__((aligned(16))) char smem[];
+    extern __shared__ __attribute__((aligned(256))) char smem[];
+    const uint32_t lds0 = lds_addr(smem);  // (a multiple of 256)
 
     const FwdParams &f = p.f;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 31, g = lane >> 5;
+    const int tid = threadIdx.x, wave = DMA ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : (int)threadIdx.x >> 6, lane = tid & 63, r = lane & 31, g = lane >> 5;
     // linear workgroup id -> (query block, member of the kv group, kv head, batch) with the query block OUTERMOST and
     // descending: under causal masking the blocks with the most KV tiles of every head start first, the light ones fill the
     // tail.  The members of a group, which read the same K / V and often the same mask and bias, are a multiple of the kv
     // head count apart: on one XCD (ids are dealt to the 8 XCDs in turn) when that is a multiple of 8.
-    const int hb_count = f.H * f.B, pairs = f.Hk * f.B;
+    const int hb_count = f.H / GH * f.B, pairs = f.Hk * f.B;
     const int m_block = (int)gridDim.x / hb_count - 1 - (int)blockIdx.x / hb_count;
     const int pair = (int)blockIdx.x % pairs, hk = pair % f.Hk, b = pair / f.Hk;
-    const int h = hk * (f.H / f.Hk) + ((int)blockIdx.x % hb_count) / pairs;
+    const int hs = wave % (RB * GH) / RB;  // head of this wave among the workgroup's
+    const int h = hk * (f.H / f.Hk) + ((int)blockIdx.x % hb_count) / pairs * GH + hs;
     const int m0 = m_block * BM;
-    const int rw = wave % (BM / 32), kh = wave / (BM / 32);  // row block and key half of this wave
+    const int rw = wave % RB, kh = wave / (RB * GH);  // row block and key half of this wave
+    const int xw = wave % (RB * GH);  // (rows and heads: where the halves meet)
     const int wrow0 = m0 + rw * 32;
     const int qrow = wrow0 + r;
     const int qrow_c = qrow < f.Lq ? qrow : f.Lq - 1;
@@ -119,8 +128,9 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
     // words are ANDed with a validity pattern when they are consumed
     const int kc = tid % CH, kr0 = tid / CH;
     const int kcol = kc * 8 < f.d ? kc * 8 : 0;
-    const int fc = tid % FCH, fr0 = tid / FCH;  // mask / bias: 8-key chunk, first row (rows fr0 + F_RPP it)
-    u32x4_t kreg[K_IT], vreg[K_IT], breg[F_IT];
+    const int kc_g = kc ^ (int)TL::swz(kr0), kcol_g = kc_g * 8 < f.d ? kc_g * 8 : 0;  // (DMA: what chunk position kc of its rows holds)
+    const int fc = tid % FCH, fr0 = tid / FCH % BM;  // mask / bias: 8-key chunk, first row (rows fr0 + F_RPP it)
+    u32x4_t kreg[DMA ? 1 : K_IT], vreg[DMA ? 1 : K_IT], breg[F_IT];
     u32x2_t mreg[F_IT], mnext[F_IT];
 
     // (a mask that comes packed to bits: one byte per 8-key chunk instead of eight, expanded where it is looked at)
@@ -157,6 +167,12 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         }
         return any != 0;
     };
+    typedef const __attribute__((address_space(1))) char *gptr_t;
+    auto uniform_ptr = [](const void *ptr) -> gptr_t {
+        const uint64_t v = (uint64_t)ptr;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+        return (gptr_t)(((uint64_t)hi << 32) | lo);
+    };
     auto load_rest = [&](int j) {
         const int n0 = j * BN;
         if (bbase) {
@@ -171,6 +187,19 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
 #pragma unroll
             for (int it = 0; it < F_IT; it++) breg[it] = u32x4_t{0, 0, 0, 0};
         }
+        if constexpr (DMA) {
+            const gptr_t kb = uniform_ptr(kbase + (int64_t)n0 * f.k_r), vb = uniform_ptr(vbase + (int64_t)n0 * f.v_r);
+            const int last = f.Lk - 1 - n0;
+            const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)((j & 1) * SM::STAGE) + (uint32_t)wave * 1024);
+#pragma unroll
+            for (int it = 0; it < K_IT; it++) {
+                const int row = kr0 + it * K_RPP, row_c = row < last ? row : last;
+                const uint32_t ko = (uint32_t)(row_c * (int)f.k_r + kcol_g) * 2, vo = (uint32_t)(row_c * (int)f.v_r + kcol_g) * 2;
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(ko), "s"(kb), "s"(dst + it * K_RPP * 256) : "memory");
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(vo), "s"(vb), "s"(dst + SM::K_BYTES + it * K_RPP * 256) : "memory");
+            }
+            return;
+        }
 #pragma unroll
         for (int it = 0; it < K_IT; it++) {
             int key = n0 + kr0 + it * K_RPP;
@@ -184,12 +213,14 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         char *sK = smem + buf * SM::STAGE;
         char *sV = sK + SM::K_BYTES;
         char *sF = sV + SM::K_BYTES;
+        if constexpr (!DMA) {
 #pragma unroll
-        for (int it = 0; it < K_IT; it++) {
-            const int off = ((kr0 + it * K_RPP) * SM::S + kc * 8) * 2;
-            *(u32x4_t *)(sK + off) = kreg[it];
-            *(u32x4_t *)(sV + off) = vreg[it];
+            for (int it = 0; it < K_IT; it++) {
+                *(u32x4_t *)(sK + TL::chunk(kr0 + it * K_RPP, kc)) = kreg[it];
+                *(u32x4_t *)(sV + TL::chunk(kr0 + it * K_RPP, kc)) = vreg[it];
+            }
         }
+        if (F_CHUNKS < NTHREADS && wave >= F_CHUNKS / 64) return;
 #pragma unroll
         for (int it = 0; it < F_IT; it++) {
             u32x4_t bv = bbase ? chunk8_fix<ODD>(breg[it], kk, f.Lk) : breg[it];
@@ -208,16 +239,17 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
     };
 
     const int a_row = pi_row(r);
-    const uint32_t a_off = (uint32_t)((a_row * SM::S + g * 8) * 2);
+    const uint32_t a_off = lds0 + TL::frag_base(a_row, g);
     const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
     const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
     const int tdh = (lane >> 4) & 1;
-    const uint32_t tr_off = (uint32_t)(((8 * g + te) * SM::S + 16 * tdh + 4 * tcp) * 2);
+    const uint32_t tr_off = lds0 + TL::tr_base(g, te, tdh, tcp);
 
     auto compute = [&](int j, int buf) {
         const int n0 = j * BN + kh * BK;
-        const char *sK = smem + buf * SM::STAGE + kh * BK * SM::S * 2;
-        const char *sV = sK + SM::K_BYTES;
+        const uint32_t st = (uint32_t)(buf * SM::STAGE + kh * BK * TL::ROW_BYTES);
+        uint32_t a_cur = a_off + st, tr_cur = tr_off + st;
+        if (TL::SWZ) asm volatile("" : "+v"(a_cur), "+v"(tr_cur));  // (the swizzled addresses are recomputed where used)
         const char *sF = smem + buf * SM::STAGE + 2 * SM::K_BYTES + ((rw * 32 + r) * SM::SF + kh * BK + 8 * g) * 2;
         // ---- S^T = K Q^T on top of the fused mask+bias tile, dP^T = V dO^T
         f32x16_t s[MB], dp[MB];
@@ -235,11 +267,11 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
                 }
             }
         {
-            constexpr int NF = 2 * MB * KS, FR = 8;  // fragment fi: (ks, mb, which) with which = 0: K, 1: V
+            constexpr int NF = 2 * MB * KS, FR = DMA || ODD ? 6 : 8;  // fragment fi: (ks, mb, which) with which = 0: K, 1: V
             u32x4_t a[NF];
             auto frag = [&](int fi) {
                 const int which = fi & 1, mb = (fi >> 1) % MB, ks = (fi >> 1) / MB;
-                return *(const u32x4_t *)((which ? sV : sK) + a_off + (32 * mb * SM::S + ks * 16) * 2);
+                return lds_ld128(TL::frag_at(a_cur, ks) + (uint32_t)(which * SM::K_BYTES + 32 * mb * TL::ROW_BYTES));
             };
 #pragma unroll
             for (int fi = 0; fi < FR; fi++) a[fi] = frag(fi);
@@ -280,8 +312,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
             u32x4_t a[2];
             auto frag = [&](int idx, int slot) {
                 const int kb = idx / DB, db = idx % DB;
-                const uint32_t off = tr_off + (uint32_t)((16 * kb * SM::S + 32 * db) * 2);
-                const u32x2_t lo = lds_read_tr16(sK, off), hi = lds_read_tr16(sK, off + 4 * SM::S * 2);
+                const u32x2_t lo = lds_ld_tr16(TL::tr_at(tr_cur, kb, db, 0)), hi = lds_ld_tr16(TL::tr_at(tr_cur, kb, db, 1));
                 a[slot] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
             };
             frag(0, 0);
@@ -295,6 +326,18 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         }
     };
 
+    // the end of a step (see fwd_kernel): the vote of a tile's mask, published by the barrier that publishes the step's tiles
+    int vote_at = 0;
+    if (tid < 3) lds_st32(lds0 + SM::OFF_VOTE + 4 * tid, 0u);
+    auto step_end = [&](bool any) -> bool {
+        const uint32_t at = lds0 + SM::OFF_VOTE + 4 * vote_at;
+        vote_at = vote_at == 2 ? 0 : vote_at + 1;
+        if (__any(any)) lds_st32(at, 1u);
+        if (tid == 0) lds_st32(lds0 + SM::OFF_VOTE + 4 * vote_at, 0u);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
+        return __builtin_amdgcn_readfirstlane(lds_ld32(at)) != 0u;
+    };
+
     // ---- main loop.  At the top of iteration j: tile j sits in LDS stage j&1 if it is active, the mask of tile j+1 is
     // in registers (finished) and `act_next` says whether that tile has any kept element.
     if (n_end > 0) {
@@ -305,6 +348,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
             load_rest(0);
             store_stage(0, mreg);
         }
+        if (DMA) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
         bool act_next = __syncthreads_or(n_end > 1 && finish_mask(1, mnext));
         auto step = [&](int j, u32x2_t (&m_next)[F_IT], u32x2_t (&m_new)[F_IT]) {
             const bool have_next = j + 1 < n_end && act_next;
@@ -314,7 +358,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
             if (act_cur) compute(j, j & 1);
             __builtin_amdgcn_sched_barrier(0);
             if (have_next) store_stage(j + 1, m_next);
-            const bool act_nn = __syncthreads_or(j + 2 < n_end && finish_mask(j + 2, m_new));
+            const bool act_nn = step_end(j + 2 < n_end && finish_mask(j + 2, m_new));
             act_cur = have_next;
             act_next = act_nn;
         };
@@ -325,7 +369,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
     }
 
     if constexpr (KSPLIT == 2) {  // the upper key half hands over its sums
-        f32x4_t *xo = (f32x4_t *)smem + rw * DB * 4 * 64 + lane;
+        f32x4_t *xo = (f32x4_t *)smem + xw * DB * 4 * 64 + lane;
         __syncthreads();  // (the tiles' last reads)
         if (kh == 1) {
 #pragma unroll
@@ -363,23 +407,31 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
     }
 }
 
-template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, bool ODD>
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD>
 hipError_t launch_dq_o(const BwdParams &p, hipStream_t stream) {
-    constexpr int BM = 32 * NW / KSPLIT, NTHREADS = 64 * NW, BN = ((NW == 8 && KSPLIT == 1) || D > 128) ? 32 : 64;
-    auto kern = bwd_dq_kernel<T, D, CAUSAL, NW, KSPLIT, ODD>;
-    const int smem = DqSmem<D, BM, BN>::TOTAL;
+    constexpr int BM = 32 * NW / KSPLIT / GH, NTHREADS = 64 * NW, BN = ((NW == 8 && KSPLIT == 1) || D > 128) ? 32 : 64;
+    auto kern = bwd_dq_kernel<T, D, CAUSAL, NW, KSPLIT, GH, ODD>;
+    constexpr int merge = KSPLIT == 2 ? (NW / 2) * (D / 32) * 4096 : 0;  // the upper halves' sums
+    constexpr int smem = DqSmem<D, BM, BN>::TOTAL > merge ? DqSmem<D, BM, BN>::TOTAL : merge;
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
-    dim3 grid(((p.f.Lq + BM - 1) / BM) * p.f.H * p.f.B);
+    dim3 grid(((p.f.Lq + BM - 1) / BM) * (p.f.H / GH) * p.f.B);
     hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
     return hipGetLastError();
 }
 
 template <typename T, int D, bool CAUSAL, int NW, int KSPLIT = 1>
 hipError_t launch_dq_n(const BwdParams &p, hipStream_t stream) {
-    if (D > 128 || odd_rows(p.f)) return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, true>(p, stream);
-    return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, D <= 128 ? false : true>(p, stream);
+    const int gh = shared_rows(p.f);
+    auto pick = [&](auto odd) -> hipError_t {
+        constexpr bool O = decltype(odd)::value;
+        if constexpr (D <= 128) if (gh == 4) return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, 4, (D > 64) || O>(p, stream);
+        if constexpr (D > 64) if (gh == 2) return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, 2, true>(p, stream);
+        return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, 1, O>(p, stream);
+    };
+    if (D > 128 || odd_rows(p.f)) return pick(std::true_type());
+    return pick(std::bool_constant<(D > 128)>());
 }
 
 template <typename T, int D, bool CAUSAL>

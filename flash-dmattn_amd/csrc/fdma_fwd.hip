@@ -536,16 +536,6 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     }
 }
 
-// Query heads per workgroup: 4 or 2 of a kv group, where they share mask and bias rows.  One head / four (us): 1999 x 16/4 heads, d = 128,
-// fp16 70.8 / 57.3, 1231 x 8/2 44.8 / 34.8; d = 64, 4 x 724 x 32/8 39.5 / 28.8, 4096 x 8/2 120 / 107.  Two: d = 128, 2 x 2112 x 8/4
-// 62.7 / 57.7, d = 256, 700 x 32/8 59.2 / 55.2 (four would leave each 32 rows); not at d <= 64 (1984 x 16/8 61.2 / 65.2).
-int shared_rows(const FwdParams &p) {
-    const int G = p.H / p.Hk;
-    if (G > 1 && ((p.mask && p.Hm == p.H) || (p.bias && p.Hb == p.H))) return 1;
-    if (p.d <= 128 && G % 4 == 0) return 4;
-    return p.d > 64 && G % 2 == 0 ? 2 : 1;
-}
-
 template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD>
 hipError_t launch_fwd_o(const FwdParams &p, hipStream_t stream) {
     constexpr int BM = 32 * NW / KSPLIT / GH, NTHREADS = 64 * NW, BN = D > 128 ? 32 : BN_DEFAULT;
@@ -586,6 +576,16 @@ hipError_t launch_fwd_t(const FwdParams &p, hipStream_t stream) {
 }
 
 }  // namespace
+
+// Query heads per workgroup: 4 or 2 of a kv group, where they share mask and bias rows.  One head / four (us): 1999 x 16/4 heads, d = 128,
+// fp16 70.8 / 57.3, 1231 x 8/2 44.8 / 34.8; d = 64, 4 x 724 x 32/8 39.5 / 28.8, 4096 x 8/2 120 / 107.  Two: d = 128, 2 x 2112 x 8/4
+// 62.7 / 57.7, d = 256, 700 x 32/8 59.2 / 55.2 (four would leave each 32 rows); not at d <= 64 (1984 x 16/8 61.2 / 65.2).
+int shared_rows(const FwdParams &p) {
+    const int G = p.H / p.Hk;
+    if (G > 1 && ((p.mask && p.Hm == p.H) || (p.bias && p.Hb == p.H))) return 1;
+    if (p.d <= 128 && G % 4 == 0) return 4;
+    return p.d > 64 && G % 2 == 0 ? 2 : 1;
+}
 
 hipError_t launch_fwd(const FwdParams &p, int dtype, hipStream_t stream) {
     if (p.Lq <= 0 || p.B <= 0) return hipSuccess;
