@@ -916,8 +916,8 @@ hipError_t launch_d(const FwdParams &p, hipStream_t stream) {
         return p.causal ? launch_one<T, D, 64, true, false, 8>(p, stream) : launch_one<T, D, 64, false, false, 8>(p, stream);
     }
     // no more 128-row workgroups than CUs: two key groups each (a row that sees a single tile gains nothing, and pays
-    // a merge of a microsecond)
-    if ((int64_t)p.B * p.H * ((p.Lq + 127) / 128) <= device_cus() && p.Lk > 128) {
+    // a merge of a microsecond; at d <= 64 takes_key_groups() has them)
+    if constexpr (D > 64) if ((int64_t)p.B * p.H * ((p.Lq + 127) / 128) <= device_cus() && p.Lk > 128) {
         if (p.cmp.on) return p.causal ? launch_one<T, D, 64, true, true, 4, 2>(p, stream) : launch_one<T, D, 64, false, true, 4, 2>(p, stream);
         return p.causal ? launch_one<T, D, 64, true, false, 4, 2>(p, stream) : launch_one<T, D, 64, false, false, 4, 2>(p, stream);
     }
@@ -959,16 +959,25 @@ bool fwd_colmask_applicable(const FwdParams &p) {
     return mask_ok && bias_ok && (p.Lk + 31) / 32 <= MAX_TILES;
 }
 
+// Whether 64-row workgroups of four key groups (fdma_fwd_wide.hip) take a call at head dims up to 128: twice the workgroups of
+// 128-row ones, with half the chain of tiles and a merge of a microsecond.
+//   * d = 65 .. 128, one to a CU, as long as all of them run at once: 1.13 to 1.35 times as fast over 24 calls of 4 to 256 blocks; 352
+//     blocks (2 x 700 rows x 16 heads) 29.9 against 21.6 us.  A row that sees a single tile gains nothing (128 x 128: 10.7
+//     either way).
+//   * d <= 64, two to a CU: up to two and a half blocks per CU 1.25 to 1.65 times over 11 calls; 768 blocks (2 x 1500 x 16 heads, 700
+//     kept) 29.3 against 27.8 us, ragged 4000 to 1000 x 16 140 against 125.
+// (A ragged batch has at most total / 64 blocks per head and one more per entry.)
+static bool takes_key_groups(const FwdParams &p) {
+    const int64_t blocks64 = p.cu_q ? (int64_t)p.H * (p.total_q / 64 + p.B) : (int64_t)p.B * p.H * ((p.Lq + 63) / 64);
+    if (p.d > 64) return blocks64 <= device_cus() && p.Lk > 128;
+    return 2 * blocks64 <= 5 * (int64_t)device_cus();
+}
+
 hipError_t launch_fwd_colmask(const FwdParams &p, int dtype, hipStream_t stream) {
     if (p.cmp.on && p.cmp.img_kv) return launch_fwd_stream(p, dtype, stream);  // (the pre-pass has written tile images)
     // head dims up to 64 / 128 (a head dim in between runs in the next larger instantiation), above in a kernel of their own
     if (p.d > 128) return launch_fwd_wide(p, dtype, stream);
-    // 64-row workgroups of four key groups, one to a CU, as long as all of them run at once: 1.13 to 1.35 times the 128-row ones
-    // with two groups over 24 calls of 4 to 256 blocks; 352 blocks (2 x 700 rows x 16 heads) 29.9 against 21.6 us.  A row
-    // that sees a single tile gains nothing (128 x 128: 10.7 either way).  (A ragged batch has at most total / 64 blocks per
-    // head and one more per entry.)
-    const int64_t blocks64 = p.cu_q ? (int64_t)p.H * (p.total_q / 64 + p.B) : (int64_t)p.B * p.H * ((p.Lq + 63) / 64);
-    if (p.d > 64 && blocks64 <= device_cus() && p.Lk > 128) {
+    if (takes_key_groups(p)) {
         const hipError_t e = launch_fwd_wide(p, dtype, stream);
         if (e != hipSuccess || !p.cmp.on || p.splits <= 1) return e;
         return dtype == 0 ? launch_merge<bf16_tag>(p, stream) : launch_merge<fp16_tag>(p, stream);

@@ -1,5 +1,5 @@
 // Forward dynamic-mask attention for gfx950, column-mask specialisation with key groups and direct loads: head dims 129 .. 256,
-// and 65 .. 128 where there are no more blocks of 64 query rows than CUs.
+// and below on small grids (takes_key_groups in fdma_fwd_colmask.hip).
 //
 // Same math, inputs and reference counterparts as fdma_fwd_colmask.hip (compute_attn_1rowblock,
 // csrc/flash_sparse_attn/src/flash_fwd_kernel.h:53-804 of the reference; mask and bias absent or broadcast over the query
@@ -13,6 +13,7 @@
 //   * Head dim 128, RG = 2: 64-row blocks with four key groups are twice as many workgroups with half the chain of tiles.
 //     A tile of 128 keys takes 1.4 us where the eight-wave kernel of fdma_fwd_colmask.hip takes 1.6 for 128 rows, on twice
 //     the CUs.
+//   * Head dim 64, RG = 2: two workgroups to a CU.
 //   * K and V tiles go from global memory straight into LDS (global_load_lds, one tile ahead, issued between the MFMAs):
 //     no staging registers.  The 16-byte chunks of a 256-byte row, or of the two halves of a 512-byte one, are swizzled as in
 //     LdsTile<128>; V is row-major like K, and V^T comes from transposing LDS reads.
@@ -23,7 +24,8 @@
 // loads it is 0.25 us shorter, without the softmax 0.1.
 // Before / now (us): 3001 tokens, 8/4 heads, d = 256, 1024 kept, fp16 57 / 38 (with the bias producer and the mask 75.6 / 56.3);
 // 8192 tokens, 8/2 heads, d = 256, 4096 kept 203 / 152; 2300 ragged tokens and others, 16/8 heads, d = 256 152 / 115;
-// d = 128: 512 rows x 32 heads against 2048 kept keys of 16384 42.7 / 35.6, 2000 tokens x 4 heads 39.7 / 32.4, 256 x 32 14.8 / 11.0.
+// d = 128: 512 rows x 32 heads against 2048 kept keys of 16384 42.7 / 35.6, 2000 tokens x 4 heads 39.7 / 32.4, 256 x 32 14.8 / 11.0;
+// d = 64: 2176 x 16 42.4 / 29.4, 4 x 448 x 8 13.7 / 9.9, 512 x 32 against 2048 kept of 16384 32.9 / 25.9, ragged up to 4928 x 2 74 / 45.
 #include <type_traits>
 
 #include "fdma_common.h"
@@ -48,23 +50,28 @@ template <int D_, int RG> struct Cfg {
     static constexpr int OFF_COL = 4 * TILE;              // two stages of the fused bias column
     static constexpr int OFF_BITS = OFF_COL + 2 * BN * 4;
     static constexpr int LOOP_BYTES = OFF_BITS + MAX_TILES / 8;
-    static constexpr int DPW = D / 32 / KG;               // merge: 32-wide blocks of O that a wave finishes
-    static constexpr int OFF_SUMS = KG * (KG - 1) * RG * DPW * 4096;  // ... the others' shares of them, then row sums and references
+    static constexpr int UPW = D / 16 / KG;               // merge: 16-wide units of O that a wave finishes
+    static constexpr int OFF_SUMS = KG * (KG - 1) * RG * UPW * 2048;  // ... the others' shares of them, then row sums and references
     static constexpr int MERGE_BYTES = OFF_SUMS + 2 * 8 * 64 * 4;
     static constexpr int SMEM = LOOP_BYTES > MERGE_BYTES ? LOOP_BYTES : MERGE_BYTES;
     static_assert(SMEM <= 160 * 1024, "one workgroup per CU");
+    static_assert(UPW * KG * 16 == D, "every unit of O is finished by one key group");
     static_assert(8 * RPP % 16 == 0, "a wave's pieces lie rows of one swizzle apart");
 };
 
-// (see LdsTile: the swizzle permutes the 16 chunks of a 256-byte half row, so rows of 512 bytes meet the banks as rows of 256 do)
-__device__ __forceinline__ uint32_t swz(int row) { return (uint32_t)(((row & 3) << 2) | ((row >> 2) & 3)); }
+// Rows of a tile are unpadded, their 16-byte chunks permuted by a XOR with a function of the row (see LdsTile).  Rows of 512 bytes
+// meet the banks as rows of 256 do: the 16 chunks of a half row are permuted.  Two rows of 128 bytes share a line of banks: four
+// consecutive ones lie in different 64-byte quarters (transposing reads), sixteen in different chunks (fragment reads).
+template <int D> __device__ __forceinline__ uint32_t swz(int row) {
+    return D == 64 ? (uint32_t)((((row >> 1) & 1) << 2) | ((row >> 2) & 3)) : (uint32_t)(((row & 3) << 2) | ((row >> 2) & 3));
+}
 
 template <typename T, int D, int RG, bool CAUSAL, bool CMP>
-__global__ void __launch_bounds__(NT) fwd_wide_kernel(const FwdParams p) {
+__global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const FwdParams p) {
     using E = Elem<T>;
     using C = Cfg<D, RG>;
     constexpr int KG = C::KG, BM = C::BM, BN = C::BN, ROW = C::ROW, TILE = C::TILE, NP = C::NP, KS = D / 16, DB = D / 32;
-    constexpr int OFF_V = C::OFF_V, OFF_COL = C::OFF_COL, OFF_BITS = C::OFF_BITS, DPW = C::DPW;
+    constexpr int OFF_V = C::OFF_V, OFF_COL = C::OFF_COL, OFF_BITS = C::OFF_BITS, UPW = C::UPW;
     extern __shared__ __attribute__((aligned(256))) char smem[];
     const uint32_t lds0 = lds_addr(smem);  // (a multiple of 256)
     uint32_t *sBits = (uint32_t *)(smem + OFF_BITS);
@@ -194,7 +201,7 @@ __global__ void __launch_bounds__(NT) fwd_wide_kernel(const FwdParams p) {
         return (gptr_t)(((uint64_t)hi << 32) | lo);
     };
     const int prow = C::RPP * wave + lane / C::CH;
-    const int pchunk = lane % C::CH ^ (int)swz(prow);
+    const int pchunk = lane % C::CH ^ (int)swz<D>(prow);
     const uint32_t pcol = pchunk * 8 < p.d ? pchunk * 16 : 0;
     const uint32_t k_r2 = (uint32_t)(p.k_r * 2), v_r2 = (uint32_t)(p.v_r * 2);
     gptr_t tb_k = nullptr, tb_v = nullptr;
@@ -245,12 +252,12 @@ __global__ void __launch_bounds__(NT) fwd_wide_kernel(const FwdParams p) {
 
     // fragment addresses (stage 0).  K: chunk 2 ks + g of row 32 kg + pi_row(r).  V^T: see LdsTile::tr_base.
     const int frow = 32 * kg + pi_row(r);
-    uint32_t a_off = lds0 + (uint32_t)frow * ROW + (((uint32_t)g ^ swz(frow)) << 4);
+    uint32_t a_off = lds0 + (uint32_t)frow * ROW + (((uint32_t)g ^ swz<D>(frow)) << 4);
     const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
     const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
     const int tdh = (lane >> 4) & 1;
     uint32_t tr_off = lds0 + OFF_V + (uint32_t)(32 * kg + 8 * g + te) * ROW +
-                      (((uint32_t)te << 6) | ((((uint32_t)(2 * tdh + (tcp >> 1))) ^ (uint32_t)(2 * g)) << 4) | ((uint32_t)(tcp & 1) << 3));
+                      ((((uint32_t)(2 * tdh + (tcp >> 1)) ^ swz<D>(8 * g + te)) << 4) | ((uint32_t)(tcp & 1) << 3));
     const uint32_t col_off = lds0 + OFF_COL + 128 * kg + 32 * g;
 
     f32x16_t o[DB];
@@ -374,24 +381,25 @@ __global__ void __launch_bounds__(NT) fwd_wide_kernel(const FwdParams p) {
         one_tile(std::integral_constant<int, 1>());
     }
 
-    // ---- merge of the key groups: wave (rw, kg) finishes blocks kg DPW .. + DPW - 1 of its rows, the others hand theirs over
+    // ---- merge of the key groups: wave (rw, kg) finishes units kg UPW .. + UPW - 1 of its rows, the others hand theirs over
     __syncthreads();
     float total = xhalf_sum(row_sum);
     float *xs = (float *)(smem + C::OFF_SUMS) + lane;
     xs[wave * 64] = total;
     xs[(8 + wave) * 64] = row_ref;
-    auto shelf = [&](int dst, int src, int j) -> f32x4_t * {  // block j of wave group dst, from group src
-        return (f32x4_t *)smem + (((dst * (KG - 1) + (src + KG - dst - 1) % KG) * RG + rw) * DPW + j) * 4 * 64 + lane;
+    auto shelf = [&](int dst, int src, int j) -> f32x4_t * {  // unit j of group dst, from group src
+        return (f32x4_t *)smem + (((dst * (KG - 1) + (src + KG - dst - 1) % KG) * RG + rw) * UPW + j) * 2 * 64 + lane;
     };
 #pragma unroll
     for (int dst = 0; dst < KG; dst++)
         if (dst != kg) {
 #pragma unroll
-            for (int j = 0; j < DPW; j++)
+            for (int j = 0; j < UPW; j++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const f32x16_t &v = o[dst * DPW + j];
-                    shelf(dst, kg, j)[q * 64] = f32x4_t{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+                for (int q = 0; q < 2; q++) {
+                    const int u = dst * UPW + j, e = 8 * (u & 1) + 4 * q;
+                    const f32x16_t &v = o[u >> 1];
+                    shelf(dst, kg, j)[q * 64] = f32x4_t{v[e], v[e + 1], v[e + 2], v[e + 3]};
                 }
         }
     __syncthreads();
@@ -417,35 +425,33 @@ __global__ void __launch_bounds__(NT) fwd_wide_kernel(const FwdParams p) {
     for (int own = 0; own < KG; own++)
         if (own == kg) {
 #pragma unroll
-            for (int j = 0; j < DPW; j++)
+            for (int j = 0; j < UPW; j++) {
+                const int u = own * UPW + j, c = 16 * u + 8 * g;
+                f32x4_t y[2];
 #pragma unroll
-                for (int blk = 0; blk < 2; blk++) {
-                    const int c = 32 * (own * DPW + j) + 16 * blk + 8 * g;
-                    f32x4_t y[2];
+                for (int q = 0; q < 2; q++) {
+                    const f32x16_t &v = o[u >> 1];
 #pragma unroll
-                    for (int q = 0; q < 2; q++) {
-                        const f32x16_t &v = o[own * DPW + j];
+                    for (int e = 0; e < 4; e++) y[q][e] = v[8 * (u & 1) + 4 * q + e] * w[own];
 #pragma unroll
-                        for (int e = 0; e < 4; e++) y[q][e] = v[8 * blk + 4 * q + e] * w[own];
+                    for (int x = 0; x < KG; x++)
+                        if (x != own) {
+                            const f32x4_t t = shelf(own, x, j)[q * 64];
 #pragma unroll
-                        for (int x = 0; x < KG; x++)
-                            if (x != own) {
-                                const f32x4_t t = shelf(own, x, j)[(2 * blk + q) * 64];
-#pragma unroll
-                                for (int e = 0; e < 4; e++) y[q][e] += t[e] * w[x];
-                            }
-#pragma unroll
-                        for (int e = 0; e < 4; e++) y[q][e] *= inv;
-                    }
-                    if (c < p.d) {
-                        if (share) {
-                            *(f32x4_t *)(p.o_part + prow_at * p.d + c) = y[0];
-                            *(f32x4_t *)(p.o_part + prow_at * p.d + c + 4) = y[1];
-                        } else {
-                            *(u32x4_t *)(op + c) = u32x4_t{E::pack2(y[0][0], y[0][1]), E::pack2(y[0][2], y[0][3]), E::pack2(y[1][0], y[1][1]), E::pack2(y[1][2], y[1][3])};
+                            for (int e = 0; e < 4; e++) y[q][e] += t[e] * w[x];
                         }
+#pragma unroll
+                    for (int e = 0; e < 4; e++) y[q][e] *= inv;
+                }
+                if (c < p.d) {
+                    if (share) {
+                        *(f32x4_t *)(p.o_part + prow_at * p.d + c) = y[0];
+                        *(f32x4_t *)(p.o_part + prow_at * p.d + c + 4) = y[1];
+                    } else {
+                        *(u32x4_t *)(op + c) = u32x4_t{E::pack2(y[0][0], y[0][1]), E::pack2(y[0][2], y[0][3]), E::pack2(y[1][0], y[1][1]), E::pack2(y[1][2], y[1][3])};
                     }
                 }
+            }
         }
     if (g == 0 && kg == 0) {
         // (a sum that is no number has to reach the result: only an empty share is left out)
@@ -477,7 +483,8 @@ template <typename T, int D, int RG> hipError_t launch_t(const FwdParams &p, hip
 
 hipError_t launch_fwd_wide(const FwdParams &p, int dtype, hipStream_t stream) {
     if (p.d > 128) return dtype == 0 ? launch_t<bf16_tag, 256, 4>(p, stream) : launch_t<fp16_tag, 256, 4>(p, stream);
-    return dtype == 0 ? launch_t<bf16_tag, 128, 2>(p, stream) : launch_t<fp16_tag, 128, 2>(p, stream);
+    if (p.d > 64) return dtype == 0 ? launch_t<bf16_tag, 128, 2>(p, stream) : launch_t<fp16_tag, 128, 2>(p, stream);
+    return dtype == 0 ? launch_t<bf16_tag, 64, 2>(p, stream) : launch_t<fp16_tag, 64, 2>(p, stream);
 }
 
 }  // namespace fdma

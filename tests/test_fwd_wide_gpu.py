@@ -1,5 +1,4 @@
-"""The forward with key groups by direct loads (fdma_fwd_wide.hip): head dims above 128, and 65 .. 128 on grids of no more
-64-row blocks than CUs.  Sizes at the edges of its row blocks (64 / 128 rows) and tiles (128 / 64 keys), key groups without a
+"""The forward with key groups by direct loads (fdma_fwd_wide.hip): head dims above 128, and below on small grids.  Sizes at the edges of its row blocks (64 / 128 rows) and tiles (128 / 64 keys), key groups without a
 kept key, scores that climb from tile to tile (the reference point moves in every one), empty rows."""
 import pytest
 import torch
@@ -32,6 +31,11 @@ def _check(q, k, v, mask, bias, causal):
     (1, 3, 1000, 8, 2, 104, True, torch.bfloat16),
     (1, 300, 140, 2, 2, 128, True, torch.bfloat16),     # rows without a key
     (1, 4100, 4100, 2, 1, 128, True, torch.bfloat16),
+    (1, 64, 129, 2, 1, 64, True, torch.bfloat16),
+    (1, 65, 257, 4, 2, 64, False, torch.float16),
+    (3, 127, 128, 2, 2, 40, True, torch.bfloat16),
+    (1, 2, 5000, 8, 2, 64, True, torch.float16),
+    (1, 300, 140, 2, 2, 64, True, torch.bfloat16),      # rows without a key
     (1, 1, 64, 2, 1, 256, False, torch.bfloat16),
     (1, 128, 65, 2, 1, 256, True, torch.float16),
     (2, 129, 127, 4, 2, 136, True, torch.bfloat16),
@@ -46,7 +50,7 @@ def test_edges(B, Lq, Lk, H, Hk, D, causal, dtype, mode):
     _check(q, k, v, mask, bias, causal)
 
 
-@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("mode", ["0", "2"])
 def test_climbing_scores_and_empty_groups(D, mode):
     set_compact(mode)
@@ -62,10 +66,14 @@ def test_climbing_scores_and_empty_groups(D, mode):
     _check(q, k, v, mask, bias, False)
 
 
-def test_ragged_with_few_blocks():
+@pytest.mark.parametrize("lens,H,Hk,D", [
+    ([1, 200, 64, 65, 300], 4, 2, 128),
+    ([1, 200, 64, 65, 300], 4, 2, 64),
+    ([2500, 1800], 8, 4, 64),
+])
+def test_ragged(lens, H, Hk, D):
     from flash_sparse_attn import flash_sparse_attn_varlen_func
 
-    lens, H, Hk, D = [1, 200, 64, 65, 300], 4, 2, 128
     g = torch.Generator().manual_seed(5)
     q = torch.randn(sum(lens), H, D, generator=g).to(torch.bfloat16).to(DEV)
     k, v = [torch.randn(sum(lens), Hk, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2)]
