@@ -330,6 +330,7 @@ bool bwd_colmask_applicable(const BwdParams &p);
 hipError_t launch_bwd_dkdv_colmask(const BwdParams &p, int dtype, hipStream_t stream);
 hipError_t launch_bwd_dkdv_256(const BwdParams &p, int dtype, int grid, hipStream_t stream);  // its kernel at head dims 129 .. 256 (fdma_bwd_dkdv_256.hip)
 hipError_t launch_bwd_dq_colmask(const BwdParams &p, int dtype, hipStream_t stream);
+hipError_t launch_bwd_dq_256(const BwdParams &p, int dtype, int grid, hipStream_t stream);  // its kernel at head dims 129 .. 256 (fdma_bwd_dq_256.hip)
 // parts the units of the dK/dV kernel on the original key axis are cut into: fills kv_most / kv_quota / kv_units and returns the
 // bytes of their sums (0: whole); *db_bytes: of their dBias columns
 size_t plan_kv_parts(BwdParams &p, size_t *db_bytes);
