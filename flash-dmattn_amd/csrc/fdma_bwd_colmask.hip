@@ -779,7 +779,7 @@ hipError_t launch_dkdv(const BwdParams &p, hipStream_t stream) {
 // dQ
 // ------------------------------------------------------------------------------------------------
 constexpr int Q_BM = 128;
-constexpr int MAX_TILES = 16384;
+constexpr int DQ_MAX_KEYS = 1 << 20;  // keys that the tile bitmap holds
 
 
 template <int D, int BN> struct DqcSmem {
@@ -790,7 +790,7 @@ template <int D, int BN> struct DqcSmem {
     static constexpr int OFF_V = OFF_K + NST * K_BYTES;
     static constexpr int OFF_BIAS = OFF_V + NST * K_BYTES;
     static constexpr int OFF_BITS = OFF_BIAS + 3 * 256;  // three bias columns (a direct load fills 256 bytes)
-    static constexpr int TOTAL = OFF_BITS + MAX_TILES / 8;
+    static constexpr int TOTAL = OFF_BITS + DQ_MAX_KEYS / BN / 8;
 };
 
 // BARE: no compaction, no mask, no bias (ragged batches, plain attention): there is no bias column, and the K / V tiles can
@@ -1334,7 +1334,7 @@ hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
 bool bwd_colmask_applicable(const BwdParams &p) {
     const bool mask_ok = !p.f.mask || p.f.m_r == 0;
     const bool bias_ok = !p.f.bias || p.f.bi_r == 0;
-    return mask_ok && bias_ok && (p.f.Lk + 63) / 64 <= MAX_TILES;
+    return mask_ok && bias_ok && p.f.Lk <= DQ_MAX_KEYS;
 }
 
 // Parts of the units on the original key axis.  A call has a workgroup per 128 keys of a kv head, whose steps -- query blocks
