@@ -341,6 +341,8 @@ hipError_t launch_bwd_dq_from_ds(const BwdParams &p, int dtype, hipStream_t stre
 // dK / dV / dBias of the general form at head dims 65 .. 128 (fdma_bwd_dkdv_wide.hip); gsum: a per-query dBias element is
 // shared by several query heads
 hipError_t launch_bwd_dkdv_wide(const BwdParams &p, int dtype, bool gsum, hipStream_t stream);
+bool bwd_dkdv_64_applicable(const BwdParams &p);  // general form, head dims up to 64, aligned rows (fdma_bwd_dkdv_64.hip)
+hipError_t launch_bwd_dkdv_64(const BwdParams &p, int dtype, hipStream_t stream);
 // general forward and dQ kernels: query heads to a workgroup (fdma_fwd.hip)
 int shared_rows(const FwdParams &p);
 // general dQ kernel (mask / bias per query row), fdma_bwd_dq.hip
