@@ -967,8 +967,9 @@ bool fwd_colmask_applicable(const FwdParams &p) {
 //   * d <= 64, two to a CU: up to two and a half blocks per CU 1.25 to 1.65 times over 11 calls; 768 blocks (2 x 1500 x 16 heads, 700
 //     kept) 29.3 against 27.8 us, ragged 4000 to 1000 x 16 140 against 125.
 // (A ragged batch has at most total / 64 blocks per head and one more per entry.)
+int64_t fwd_blocks64(const FwdParams &p) { return p.cu_q ? (int64_t)p.H * (p.total_q / 64 + p.B) : (int64_t)p.B * p.H * ((p.Lq + 63) / 64); }
 static bool takes_key_groups(const FwdParams &p) {
-    const int64_t blocks64 = p.cu_q ? (int64_t)p.H * (p.total_q / 64 + p.B) : (int64_t)p.B * p.H * ((p.Lq + 63) / 64);
+    const int64_t blocks64 = fwd_blocks64(p);
     if (p.d > 64) return blocks64 <= device_cus() && p.Lk > 128;
     return 2 * blocks64 <= 5 * (int64_t)device_cus();
 }

@@ -10,6 +10,8 @@
 // through LDS at the end, each finishing its share of the head dim.
 //   * Head dim 256, RG = 4: O alone is 128 registers per lane, Q another 64.  With four waves (one per SIMD, 448 registers,
 //     nothing to hide behind) a step of 128 rows x 64 keys took 3.2 us for 0.85 us of matrix work, here 2.0.
+//     On small grids RG = 2 (see launch_fwd_wide), with one stage: the next K tile is fetched under the softmax and P V, the next V
+//     tile under the scores and the softmax, a barrier more for each.
 //   * Head dim 128, RG = 2: 64-row blocks with four key groups are twice as many workgroups with half the chain of tiles.
 //     A tile of 128 keys takes 1.4 us where the eight-wave kernel of fdma_fwd_colmask.hip takes 1.6 for 128 rows, on twice
 //     the CUs.
@@ -20,7 +22,7 @@
 //   * The score accumulators start from the fused bias of their keys (fp32, -inf where the mask drops the key), read from an
 //     LDS column; the softmax is the online one, with a reference point that moves only when a score exceeds it by 2^8.  Its
 //     vector work runs under the MFMAs of the SIMD's other wave.
-// LDS: two stages of 64 KB.  Bound by the chain of a tile (scores, softmax, P V, barrier) of two waves per SIMD: without the
+// LDS: two stages of 64 KB, or one of 128.  Bound by the chain of a tile (scores, softmax, P V, barrier) of two waves per SIMD: without the
 // loads it is 0.25 us shorter, without the softmax 0.1.
 // Before / now (us): 3001 tokens, 8/4 heads, d = 256, 1024 kept, fp16 57 / 38 (with the bias producer and the mask 75.6 / 56.3);
 // 8192 tokens, 8/2 heads, d = 256, 4096 kept 203 / 152; 2300 ragged tokens and others, 16/8 heads, d = 256 152 / 115;
@@ -46,12 +48,14 @@ template <int D_, int RG> struct Cfg {
     static constexpr int TILE = BN * ROW;                 // a K or V tile
     static constexpr int RPP = 64 / CH;                   // rows of a 1 KB piece
     static constexpr int NP = TILE / 1024 / 8;            // pieces per wave of a K or V tile
-    static constexpr int OFF_V = 2 * TILE;                // two stages of K, two of V
-    static constexpr int OFF_COL = 4 * TILE;              // two stages of the fused bias column
+    static constexpr bool ONE = 4 * TILE > 128 * 1024;    // one stage of K and of V instead of two
+    static constexpr int OFF_V = (ONE ? 1 : 2) * TILE;
+    static constexpr int OFF_COL = 2 * OFF_V;             // two stages of the fused bias column
     static constexpr int OFF_BITS = OFF_COL + 2 * BN * 4;
     static constexpr int LOOP_BYTES = OFF_BITS + MAX_TILES / 8;
     static constexpr int UPW = D / 16 / KG;               // merge: 16-wide units of O that a wave finishes
-    static constexpr int OFF_SUMS = KG * (KG - 1) * RG * UPW * 2048;  // ... the others' shares of them, then row sums and references
+    static constexpr int PASSES = KG * (KG - 1) * RG * UPW * 2048 > 128 * 1024 ? 2 : 1, UPP = UPW / PASSES;  // ... in so many passes
+    static constexpr int OFF_SUMS = KG * (KG - 1) * RG * UPP * 2048;  // the others' shares of a pass's units, then row sums and references
     static constexpr int MERGE_BYTES = OFF_SUMS + 2 * 8 * 64 * 4;
     static constexpr int SMEM = LOOP_BYTES > MERGE_BYTES ? LOOP_BYTES : MERGE_BYTES;
     static_assert(SMEM <= 160 * 1024, "one workgroup per CU");
@@ -71,7 +75,8 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     using E = Elem<T>;
     using C = Cfg<D, RG>;
     constexpr int KG = C::KG, BM = C::BM, BN = C::BN, ROW = C::ROW, TILE = C::TILE, NP = C::NP, KS = D / 16, DB = D / 32;
-    constexpr int OFF_V = C::OFF_V, OFF_COL = C::OFF_COL, OFF_BITS = C::OFF_BITS, UPW = C::UPW;
+    constexpr int OFF_V = C::OFF_V, OFF_COL = C::OFF_COL, OFF_BITS = C::OFF_BITS, UPW = C::UPW, UPP = C::UPP;
+    constexpr bool ONE = C::ONE;
     extern __shared__ __attribute__((aligned(256))) char smem[];
     const uint32_t lds0 = lds_addr(smem);  // (a multiple of 256)
     uint32_t *sBits = (uint32_t *)(smem + OFF_BITS);
@@ -204,6 +209,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     const int pchunk = lane % C::CH ^ (int)swz<D>(prow);
     const uint32_t pcol = pchunk * 8 < p.d ? pchunk * 16 : 0;
     const uint32_t k_r2 = (uint32_t)(p.k_r * 2), v_r2 = (uint32_t)(p.v_r * 2);
+    uint32_t k_row = prow * k_r2, v_row = prow * v_r2;  // (offsets grow with the row: clamped by the last row's)
     gptr_t tb_k = nullptr, tb_v = nullptr;
     int t_rows = 0, t_stage = 0;     // last row of the tile being fetched, its stage
     uint32_t braw = 0, mraw = 0;     // first waves: raw bias and mask of key `tid` of that tile
@@ -229,9 +235,9 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     // (in assembly and waited for by hand: behind the compiler's builtin every LDS read waits for all LDS operations in flight)
     auto dma_piece = [&](int n) {  // NP pieces of K, NP of V
         const int i = n % NP;
-        const int row = prow + 8 * C::RPP * i, row_c = row < t_rows ? row : t_rows;
-        const uint32_t off = (uint32_t)row_c * (n < NP ? k_r2 : v_r2) + pcol;
-        const uint32_t dst = lds0 + (n < NP ? 0 : OFF_V) + (uint32_t)(t_stage * TILE + (wave + 8 * i) * 1024);
+        const uint32_t r2 = n < NP ? k_r2 : v_r2, at = (n < NP ? k_row : v_row) + 8 * C::RPP * i * r2, last = (uint32_t)t_rows * r2;
+        const uint32_t off = (at < last ? at : last) + pcol;
+        const uint32_t dst = lds0 + (n < NP ? 0 : OFF_V) + (uint32_t)((ONE ? 0 : t_stage * TILE) + (wave + 8 * i) * 1024);
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(n < NP ? tb_k : tb_v), "s"(__builtin_amdgcn_readfirstlane(dst)));
     };
     auto publish = [&]() {
@@ -287,7 +293,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     auto one_tile = [&](auto st_c) {
         constexpr int st = decltype(st_c)::value;
         // (the swizzled addresses are these constants XOR a compile-time value, recomputed where used)
-        asm volatile("" : "+v"(a_off), "+v"(tr_off));
+        asm volatile("" : "+v"(a_off), "+v"(tr_off), "+v"(k_row), "+v"(v_row));
         const int n0 = jc * BN + 32 * kg;
         set_tile(jn < n_end ? jn : jc, st ^ 1);  // (past the last tile it is fetched again and dropped)
         __builtin_amdgcn_sched_barrier(0);
@@ -303,17 +309,25 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         {
             constexpr int FR = 4;
             u32x4_t a[KS];
-            auto frag = [&](int ks) { return lds_ld128((a_off ^ ((uint32_t)(ks & 7) << 5)) + (uint32_t)(st * TILE + (ks >> 3) * 256)); };
+            auto frag = [&](int ks) { return lds_ld128((a_off ^ ((uint32_t)(ks & 7) << 5)) + (uint32_t)((ONE ? 0 : st * TILE) + (ks >> 3) * 256)); };
 #pragma unroll
             for (int ks = 0; ks < FR; ks++) a[ks] = frag(ks);
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) {
                 if (ks + FR < KS) a[ks + FR] = frag(ks + FR);
                 s = E::mfma(a[ks], qf[ks], s);
+                if constexpr (!ONE) {
 #pragma unroll
-                for (int n = ks * 2 * NP / KS; n < (ks + 1) * 2 * NP / KS; n++) dma_piece(n);
+                    for (int n = ks * 2 * NP / KS; n < (ks + 1) * 2 * NP / KS; n++) dma_piece(n);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
+        }
+        if constexpr (ONE) {  // everybody has read this K tile: the next one takes its place
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+            for (int n = 0; n < NP; n++) dma_piece(n);
+            __builtin_amdgcn_sched_barrier(0);
         }
         if (CAUSAL && n0 + 32 > vis_wave) {
             asm volatile("" ::: "memory");  // (a branch: only diagonal tiles pay)
@@ -348,6 +362,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         }
         row_sum += psum0 + psum1;
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (ONE) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(NP) : "memory");  // this V tile is there
         // ---- O^T += V^T P^T: V^T through transposing reads, FR2 MFMAs ahead
         {
             constexpr int NG = 2 * DB, FR2 = 3;
@@ -355,7 +370,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
             auto tr_read = [&](int gi) {
                 const int kb = gi / DB, db = gi % DB;
                 const uint32_t at = (tr_off ^ ((uint32_t)(db & 3) << 6)), hi = (tr_off ^ (((uint32_t)(db & 3) << 6) | 16u));
-                const uint32_t c = (uint32_t)(st * TILE + kb * 16 * ROW + (db >> 2) * 256);
+                const uint32_t c = (uint32_t)((ONE ? 0 : st * TILE) + kb * 16 * ROW + (db >> 2) * 256);
                 tl[gi] = lds_ld_tr16(at + c);
                 th[gi] = lds_ld_tr16(hi + c + 4 * ROW);
             };
@@ -372,6 +387,10 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
             }
         }
         publish();
+        if constexpr (ONE) {  // ... and everybody has read this V tile
+#pragma unroll
+            for (int n = NP; n < 2 * NP; n++) dma_piece(n);
+        }
         jc = jn;
         jn = next_active(jn + 1);
     };
@@ -387,22 +406,25 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     float *xs = (float *)(smem + C::OFF_SUMS) + lane;
     xs[wave * 64] = total;
     xs[(8 + wave) * 64] = row_ref;
-    auto shelf = [&](int dst, int src, int j) -> f32x4_t * {  // unit j of group dst, from group src
-        return (f32x4_t *)smem + (((dst * (KG - 1) + (src + KG - dst - 1) % KG) * RG + rw) * UPW + j) * 2 * 64 + lane;
+    auto shelf = [&](int dst, int src, int j) -> f32x4_t * {  // unit j of the pass of group dst, from group src
+        return (f32x4_t *)smem + (((dst * (KG - 1) + (src + KG - dst - 1) % KG) * RG + rw) * UPP + j) * 2 * 64 + lane;
     };
+    auto hand_over = [&](int pass) {
 #pragma unroll
-    for (int dst = 0; dst < KG; dst++)
-        if (dst != kg) {
+        for (int dst = 0; dst < KG; dst++)
+            if (dst != kg) {
 #pragma unroll
-            for (int j = 0; j < UPW; j++)
+                for (int j = 0; j < UPP; j++)
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const int u = dst * UPW + j, e = 8 * (u & 1) + 4 * q;
-                    const f32x16_t &v = o[u >> 1];
-                    shelf(dst, kg, j)[q * 64] = f32x4_t{v[e], v[e + 1], v[e + 2], v[e + 3]};
-                }
-        }
-    __syncthreads();
+                    for (int q = 0; q < 2; q++) {
+                        const int u = dst * UPW + pass * UPP + j, e = 8 * (u & 1) + 4 * q;
+                        const f32x16_t &v = o[u >> 1];
+                        shelf(dst, kg, j)[q * 64] = f32x4_t{v[e], v[e + 1], v[e + 2], v[e + 3]};
+                    }
+            }
+        __syncthreads();
+    };
+    hand_over(0);
     float ref[KG], top = -INFINITY, w[KG];
 #pragma unroll
     for (int x = 0; x < KG; x++) {
@@ -416,44 +438,51 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         w[x] = fast_exp2(ref[x] - safe);
         total += xs[(x * RG + rw) * 64] * w[x];
     }
-    if (qrow >= LqS) return;
+    const bool row_ok = qrow < LqS;
     const float inv = total > 0.f ? 1.f / total : 0.f;
     const bool share = CMP && p.splits > 1;  // this share's O in fp32 and its log2-sum-exp; fwd_merge_kernel adds the shares up
     const int64_t prow_at = (((int64_t)blockIdx.y * p.B + b) * p.H + h) * p.Lq + qrow;
     uint16_t *op = (uint16_t *)p.o + b * p.o_b + (sq.q0 + qrow) * p.o_r + h * p.o_h;
 #pragma unroll
-    for (int own = 0; own < KG; own++)
-        if (own == kg) {
+    for (int pass = 0; pass < C::PASSES; pass++) {
+        if (pass > 0) {
+            __syncthreads();
+            hand_over(pass);
+        }
 #pragma unroll
-            for (int j = 0; j < UPW; j++) {
-                const int u = own * UPW + j, c = 16 * u + 8 * g;
-                f32x4_t y[2];
+        for (int own = 0; own < KG; own++)
+            if (own == kg) {
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const f32x16_t &v = o[u >> 1];
+                for (int j = 0; j < UPP; j++) {
+                    const int u = own * UPW + pass * UPP + j, c = 16 * u + 8 * g;
+                    f32x4_t y[2];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) y[q][e] = v[8 * (u & 1) + 4 * q + e] * w[own];
+                    for (int q = 0; q < 2; q++) {
+                        const f32x16_t &v = o[u >> 1];
 #pragma unroll
-                    for (int x = 0; x < KG; x++)
-                        if (x != own) {
-                            const f32x4_t t = shelf(own, x, j)[q * 64];
+                        for (int e = 0; e < 4; e++) y[q][e] = v[8 * (u & 1) + 4 * q + e] * w[own];
 #pragma unroll
-                            for (int e = 0; e < 4; e++) y[q][e] += t[e] * w[x];
+                        for (int x = 0; x < KG; x++)
+                            if (x != own) {
+                                const f32x4_t t = shelf(own, x, j)[q * 64];
+#pragma unroll
+                                for (int e = 0; e < 4; e++) y[q][e] += t[e] * w[x];
+                            }
+#pragma unroll
+                        for (int e = 0; e < 4; e++) y[q][e] *= inv;
+                    }
+                    if (row_ok && c < p.d) {
+                        if (share) {
+                            *(f32x4_t *)(p.o_part + prow_at * p.d + c) = y[0];
+                            *(f32x4_t *)(p.o_part + prow_at * p.d + c + 4) = y[1];
+                        } else {
+                            *(u32x4_t *)(op + c) = u32x4_t{E::pack2(y[0][0], y[0][1]), E::pack2(y[0][2], y[0][3]), E::pack2(y[1][0], y[1][1]), E::pack2(y[1][2], y[1][3])};
                         }
-#pragma unroll
-                    for (int e = 0; e < 4; e++) y[q][e] *= inv;
-                }
-                if (c < p.d) {
-                    if (share) {
-                        *(f32x4_t *)(p.o_part + prow_at * p.d + c) = y[0];
-                        *(f32x4_t *)(p.o_part + prow_at * p.d + c + 4) = y[1];
-                    } else {
-                        *(u32x4_t *)(op + c) = u32x4_t{E::pack2(y[0][0], y[0][1]), E::pack2(y[0][2], y[0][3]), E::pack2(y[1][0], y[1][1]), E::pack2(y[1][2], y[1][3])};
                     }
                 }
             }
-        }
-    if (g == 0 && kg == 0) {
+    }
+    if (g == 0 && kg == 0 && row_ok) {
         // (a sum that is no number has to reach the result: only an empty share is left out)
         if (share) p.lse_part[prow_at] = total == 0.f ? -INFINITY : top + __builtin_amdgcn_logf(total);
         else p.lse[b * p.lse_b + h * p.lse_h + sq.q0 + qrow] = total > 0.f ? (top + __builtin_amdgcn_logf(total)) * kLn2 : INFINITY;
@@ -481,7 +510,12 @@ template <typename T, int D, int RG> hipError_t launch_t(const FwdParams &p, hip
 
 }  // namespace
 
+// Head dims above 128: 64-row blocks as long as all of them run at once (one to a CU), with half the chain of tiles; then 128-row ones,
+// for which K and V are fetched half as often.  128 / 64 rows (us): 8192 tokens x 2 heads, 2048 kept 62.7 / 54.0; 512 rows x 16 heads
+// against 2000 kept of 8000 63.8 / 54.8; 1500 x 8, all kept 62.2 / 55.2; 2 x 700 x 4 27.7 / 24.6; 1024 x 2 23.8 / 23.9; beyond a block per
+// CU 3001 x 8 (376 blocks) 45.6 / 51.1, 2000 x 16 (512) 34.4 / 45.7.
 hipError_t launch_fwd_wide(const FwdParams &p, int dtype, hipStream_t stream) {
+    if (p.d > 128 && fwd_blocks64(p) <= device_cus()) return dtype == 0 ? launch_t<bf16_tag, 256, 2>(p, stream) : launch_t<fp16_tag, 256, 2>(p, stream);
     if (p.d > 128) return dtype == 0 ? launch_t<bf16_tag, 256, 4>(p, stream) : launch_t<fp16_tag, 256, 4>(p, stream);
     if (p.d > 64) return dtype == 0 ? launch_t<bf16_tag, 128, 2>(p, stream) : launch_t<fp16_tag, 128, 2>(p, stream);
     return dtype == 0 ? launch_t<bf16_tag, 64, 2>(p, stream) : launch_t<fp16_tag, 64, 2>(p, stream);

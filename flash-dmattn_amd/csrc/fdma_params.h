@@ -311,6 +311,7 @@ hipError_t launch_fwd(const FwdParams &p, int dtype, hipStream_t stream);
 bool fwd_colmask_applicable(const FwdParams &p);
 hipError_t launch_fwd_colmask(const FwdParams &p, int dtype, hipStream_t stream);
 hipError_t launch_fwd_wide(const FwdParams &p, int dtype, hipStream_t stream);  // head dims 129 .. 256 (fdma_fwd_wide.hip)
+int64_t fwd_blocks64(const FwdParams &p);  // 64-row blocks of all heads (ragged batches: at most)
 // compacted forward: shares the keys of a row block are cut into (1: none); p.o_part / p.lse_part then hold
 // splits * B * H * Lq rows of d / 1 floats
 int fwd_key_splits(const FwdParams &p);

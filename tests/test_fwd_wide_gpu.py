@@ -41,6 +41,10 @@ def _check(q, k, v, mask, bias, causal):
     (2, 129, 127, 4, 2, 136, True, torch.bfloat16),
     (1, 33, 63, 2, 2, 200, False, torch.bfloat16),
     (1, 700, 450, 2, 1, 256, True, torch.float16),
+    (1, 65, 257, 2, 1, 256, False, torch.bfloat16),
+    (1, 700, 450, 30, 15, 256, True, torch.float16),    # above head dim 128: more 64-row blocks than CUs, 128-row ones
+    (2, 129, 127, 60, 20, 136, True, torch.bfloat16),
+    (4, 65, 65, 36, 9, 200, False, torch.bfloat16),
 ])
 @pytest.mark.parametrize("mode", ["0", "2"])
 def test_edges(B, Lq, Lk, H, Hk, D, causal, dtype, mode):
