@@ -63,8 +63,12 @@ __device__ __forceinline__ void bwd_dot_block(const BwdParams &p, int block_x, i
     }
 #pragma unroll
     for (int i = 0; i < DOT_ROWS; i++) {
-        float a = acc[i];
-        for (int off = lanes / 2; off > 0; off >>= 1) a += __shfl_xor(a, off);
+        float a = acc[i];  // (lane `sub` 0 gets the sum of its row's lanes)
+        auto add = [&](auto ctrl) { a += __uint_as_float(__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(a), decltype(ctrl)::value, 0xf, 0xf, false)); };
+        if (lanes == 16) add(std::integral_constant<int, 0x108>());  // row_shl:8
+        add(std::integral_constant<int, 0x104>());                   // row_shl:4
+        add(std::integral_constant<int, 0x4e>());                    // quad_perm:[2,3,0,1]
+        add(std::integral_constant<int, 0xb1>());                    // quad_perm:[1,0,3,2]
         const int row = row0 + i * rows_per_pass;
         if (sub == 0 && row < n_out) p.softmax_d[b * p.sd_b + h * p.sd_h + row] = a;
     }

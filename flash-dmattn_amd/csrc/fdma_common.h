@@ -13,6 +13,8 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 #include <stdint.h>
 
 namespace fdma {
@@ -287,6 +289,46 @@ __device__ __forceinline__ float xhalf_sum(float x) {
     auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+
+// Inclusive prefix sum of x over the lanes of a wave, and the wave's total (uniform).  Four shifted adds inside
+// each row of 16 lanes (data-parallel primitives: no LDS traffic), then the row totals through scalar registers.
+__device__ __forceinline__ int wave_scan(int x, int lane, int &total) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1 (lanes without a source add 0)
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    const int t0 = __builtin_amdgcn_readlane(x, 15), t1 = __builtin_amdgcn_readlane(x, 31);
+    const int t2 = __builtin_amdgcn_readlane(x, 47), t3 = __builtin_amdgcn_readlane(x, 63);
+    const int row = lane >> 4;
+    x += (row >= 1 ? t0 : 0) + (row >= 2 ? t1 : 0) + (row >= 3 ? t2 : 0);
+    total = t0 + t1 + t2 + t3;
+    return x;
+}
+
+// Reductions over the lanes of a wave, the result in every lane: lane i with i ^ 32, ^ 16, ^ 8, ^ 4, ^ 2, ^ 1, in this order, by lane
+// swaps and data-parallel primitives.  (A shuffle is a trip through the LDS pipe, ten times the latency of one of these: 36
+// of them one behind the other were 1.5 of the 8 us of a mask row.)
+template <typename X, typename Op> __device__ __forceinline__ X wave_reduce(X x, Op op) {
+    static_assert(sizeof(X) == 4, "32-bit values");
+    const uint32_t u = __builtin_bit_cast(uint32_t, x);
+    const auto r32 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    x = op(__builtin_bit_cast(X, (uint32_t)r32[0]), __builtin_bit_cast(X, (uint32_t)r32[1]));
+    const uint32_t w = __builtin_bit_cast(uint32_t, x);
+    const auto r16 = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    x = op(__builtin_bit_cast(X, (uint32_t)r16[0]), __builtin_bit_cast(X, (uint32_t)r16[1]));
+    // (inside a row of 16 the values repeat with the distance last added: rotating is exchanging)
+    auto step = [&](auto ctrl) {
+        x = op(x, __builtin_bit_cast(X, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false)));
+    };
+    step(std::integral_constant<int, 0x128>());  // row_ror:8
+    step(std::integral_constant<int, 0x124>());  // row_ror:4
+    step(std::integral_constant<int, 0x4e>());   // quad_perm:[2,3,0,1]
+    step(std::integral_constant<int, 0xb1>());   // quad_perm:[1,0,3,2]
+    return x;
+}
+template <typename X> __device__ __forceinline__ X wave_sum(X x) { return wave_reduce(x, [](X a, X b) { return a + b; }); }
+__device__ __forceinline__ float wave_max(float x) { return wave_reduce(x, [](float a, float b) { return fmaxf(a, b); }); }
+__device__ __forceinline__ int wave_max(int x) { return wave_reduce(x, [](int a, int b) { return a > b ? a : b; }); }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 

@@ -189,8 +189,7 @@ __global__ void __launch_bounds__(256) compact_scan_gather_kernel(const FwdParam
             before += __builtin_popcount((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u);
         }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off);
+    before = wave_sum(before);
     if (lane == 0) s_wave[wave] = before;
     __syncthreads();
     const int base = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
@@ -326,13 +325,9 @@ __global__ void __launch_bounds__(256) compact_image_kernel(const FwdParams p, i
                 for (int e = 0; e < 4; e++) mine += __builtin_popcount(kept_bits(mv[e], c + 4 * e));
             }
         }
-        int incl = mine;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(incl, off);
-            if (lane >= off) incl += t;
-        }
-        if (lane == 63) s_wave[wave] = incl;
+        int wave_total;
+        const int incl = wave_scan(mine, lane, wave_total);
+        if (lane == 0) s_wave[wave] = wave_total;
         __syncthreads();
         int woff = 0;
         total = 0;
@@ -490,8 +485,7 @@ __global__ void __launch_bounds__(256) compact_scan_image_kernel(const FwdParams
                 before += __builtin_popcount((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u);
             }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off);
+    before = wave_sum(before);
     if (lane == 0) s_wave[wave] = before;
     __syncthreads();
     const int base = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
@@ -662,14 +656,9 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
     int u = 0, n_max = 0;
     for (int base = 0; base < pairs; base += 256) {
         const int n = base + tid < pairs ? (count[base + tid] + 127) / 128 : 0;
-        int incl = n, mx = n;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(incl, off);
-            if (lane >= off) incl += t;
-            mx = max(mx, __shfl_xor(mx, off));
-        }
-        if (lane == 63) { s_wsum[wave] = incl; s_wmax[wave] = mx; }
+        int wave_total;
+        const int incl = wave_scan(n, lane, wave_total), mx = wave_max(n);
+        if (lane == 0) { s_wsum[wave] = wave_total; s_wmax[wave] = mx; }
         __syncthreads();
         int before = u;
 #pragma unroll
@@ -723,11 +712,8 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
         sum += nt;
         mx = nt > mx ? nt : mx;
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        sum += __shfl_xor(sum, off);
-        mx = max(mx, __shfl_xor(mx, off));
-    }
+    sum = wave_sum(sum);
+    mx = wave_max(mx);
     if (lane == 0) {
         atomicAdd(&s_sum, sum);
         atomicMax(&s_max, mx);

@@ -43,21 +43,6 @@ template <int D> struct DecSmem {
     static_assert(DEC_COLS * SO * 4 <= WAVE_BYTES, "a wave's partial output must fit its own piece");
 };
 
-// Inclusive prefix sum of x over the lanes of a wave, and the wave's total (uniform).  Four shifted adds inside
-// each row of 16 lanes (data-parallel primitives: no LDS traffic), then the row totals through scalar registers.
-__device__ __forceinline__ int wave_scan(int x, int lane, int &total) {
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1 (lanes without a source add 0)
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
-    const int t0 = __builtin_amdgcn_readlane(x, 15), t1 = __builtin_amdgcn_readlane(x, 31);
-    const int t2 = __builtin_amdgcn_readlane(x, 47), t3 = __builtin_amdgcn_readlane(x, 63);
-    const int row = lane >> 4;
-    x += (row >= 1 ? t0 : 0) + (row >= 2 ? t1 : 0) + (row >= 3 ? t2 : 0);
-    total = t0 + t1 + t2 + t3;
-    return x;
-}
-
 // nonzero bytes of x -> bit k of the result is set iff byte k of x != 0
 __device__ __forceinline__ uint32_t nz_bytes_to_bits(uint32_t x) {
     uint32_t y = (((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u;
@@ -101,13 +86,9 @@ __device__ __forceinline__ void combine_row(const FwdParams &p, int64_t row, int
         v0[u] = (u < n0 && lane < p.d) ? part_load<COHERENT>(op_row + lane + (int64_t)u * step) : 0.f;
         v1[u] = (u < n0 && lane + 64 < p.d) ? part_load<COHERENT>(op_row + lane + 64 + (int64_t)u * step) : 0.f;
     }
-    float mx = fmaxf(lv0, lv1);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    const float mx = wave_max(fmaxf(lv0, lv1));
     const float w0 = mx == -INFINITY ? 0.f : __expf(lv0 - mx), w1 = mx == -INFINITY ? 0.f : __expf(lv1 - mx);  // exp(-inf) = 0 for empty splits
-    float sum = w0 + w1;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
+    const float sum = wave_sum(w0 + w1);
     s_w[lane] = w0;
     s_w[lane + 64] = w1;
     __builtin_amdgcn_wave_barrier();  // (the LDS operations of one wave execute in order: the weights are readable below)

@@ -42,12 +42,8 @@ __device__ __forceinline__ void find_bin(const uint32_t *hist, uint32_t k, uint3
         c[j] = hist[255 - 4 * lane - j];
         s += c[j];
     }
-    uint32_t incl = s;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t t = __shfl_up(incl, off);
-        if (lane >= off) incl += t;
-    }
+    int total;
+    const uint32_t incl = (uint32_t)wave_scan((int)s, lane, total);
     uint32_t a = incl - s;
     if (a < k && k <= incl) {
 #pragma unroll
@@ -70,12 +66,8 @@ __device__ __forceinline__ void find_bin_wave(const uint32_t *h, uint32_t k, uin
         c[j] = h[255 - 4 * lane - j];
         s += c[j];
     }
-    uint32_t incl = s;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t t = __shfl_up(incl, off);
-        if (lane >= off) incl += t;
-    }
+    int total;
+    const uint32_t incl = (uint32_t)wave_scan((int)s, lane, total);
     uint32_t a = incl - s, mine_bin = 0, mine_above = 0;
     const uint64_t who = __ballot(a < k && k <= incl);
 #pragma unroll
@@ -137,43 +129,36 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
     };
     // "is the fill value" compares numerically (+0 == -0)
     auto is_min = [&](uint32_t x) -> bool { return x == min_bits || (((x | min_bits) & 0x7fffu) == 0); };
-    // exclusive prefix, in column order, of a count per chunk; returns the row's total
-    auto prefix = [&](uint32_t *tot, const int (&n)[KPT], int (&before)[KPT]) -> int {
+    // exclusive prefix, in column order, of a count per chunk: inside the wave (which leaves its totals), and -- behind a
+    // barrier -- of the totals, which every wave sums for itself, two per lane; returns the row's
+    auto prefix_wave = [&](uint32_t *tot, const int (&n)[KPT], int (&before)[KPT]) {
 #pragma unroll
         for (int c = 0; c < KPT; c++) {
-            int incl = n[c];
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int t = __shfl_up(incl, off);
-                if (lane >= off) incl += t;
-            }
-            if (lane == 63) tot[c * NW + wave] = incl;
-            before[c] = incl - n[c];
+            int total;
+            before[c] = wave_scan(n[c], lane, total) - n[c];
+            if (lane == 0) tot[c * NW + wave] = (uint32_t)total;
         }
-        __syncthreads();
-        // every wave sums the (chunk, wave) totals for itself, two per lane
+    };
+    auto prefix_row = [&](const uint32_t *tot, int (&before)[KPT]) -> int {
         constexpr int N = KPT * NW;
         static_assert(N <= 128, "two totals per lane");
         const int t0 = 2 * lane < N ? (int)tot[2 * lane] : 0, t1 = 2 * lane + 1 < N ? (int)tot[2 * lane + 1] : 0;
-        int incl = t0 + t1;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(incl, off);
-            if (lane >= off) incl += t;
-        }
-        const int e0 = incl - t0 - t1, e1 = incl - t1;
+        int total;
+        const int e1 = wave_scan(t0 + t1, lane, total) - t1, e0 = e1 - t0;
 #pragma unroll
         for (int c = 0; c < KPT; c++) {
-            const int i = c * NW + wave;
-            const int a0 = __shfl(e0, i >> 1), a1 = __shfl(e1, i >> 1);
-            before[c] += (i & 1) ? a1 : a0;
+            const int i = c * NW + __builtin_amdgcn_readfirstlane(wave);
+            before[c] += __builtin_amdgcn_readlane((i & 1) ? e1 : e0, i >> 1);
         }
-        return __shfl(incl, 63);
+        return total;
     };
 
-    uint32_t keep[KPT];  // one bit per column of the chunk
+    // one bit per column of the chunk: kept whatever else there is; equal to the threshold, of which `need` are kept
+    uint32_t keep[KPT], ties[KPT];
+    uint32_t need = 0;
+    bool some_ties = false;
 #pragma unroll
-    for (int c = 0; c < KPT; c++) keep[c] = 0;
+    for (int c = 0; c < KPT; c++) keep[c] = ties[c] = 0;
     if (p.type == 1) {  // relu: keep strictly positive values (NaN is not > 0)
         const uint32_t inf = p.dtype == 0 ? 0x7f80u : 0x7c00u;
 #pragma unroll
@@ -216,30 +201,48 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
         fold(hist2, std::integral_constant<int, REP2>(), hsum[1]);
         find_bin_wave(hsum[1], k - above1, bin2, above2);
         const uint32_t T = (bin1 << 8) | bin2;
-        const uint32_t need_eq = k - above1 - above2;  // >= 1 entries equal to T still to take
-        int rank[KPT];
-        if (need_eq < hsum[1][bin2]) {  // ties across the threshold: the first need_eq of them in column order
-            int eq[KPT];
-#pragma unroll
-            for (int c = 0; c < KPT; c++) {
-                eq[c] = 0;
-#pragma unroll
-                for (int j = 0; j < 8; j++) eq[c] += (j < valid(c) && order_key(bits_of(c, j)) == T) ? 1 : 0;
-            }
-            prefix(s_tot[0], eq, rank);
-        } else {
-#pragma unroll
-            for (int c = 0; c < KPT; c++) rank[c] = -0x40000000;
-        }
+        // entries equal to T still to take, >= 1 of hsum[1][bin2]: in column order (none where T is the fill value)
+        const uint32_t t_bits = (T & 0x8000u) ? T ^ 0x8000u : ~T & 0xffffu;
+        need = is_min(t_bits) ? 0u : k - above1 - above2;
+        some_ties = need != 0 && need < hsum[1][bin2];
 #pragma unroll
         for (int c = 0; c < KPT; c++)
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 const uint32_t x = bits_of(c, j), key = order_key(x);
-                const bool in = j < valid(c), eq = in && key == T;
-                if (in && (key > T || (eq && rank[c] < (int)need_eq)) && !is_min(x)) keep[c] |= 1u << j;
-                rank[c] += eq ? 1 : 0;
+                if (j < valid(c) && key > T && !is_min(x)) keep[c] |= 1u << j;
+                if (j < valid(c) && key == T && need != 0) ties[c] |= 1u << j;
             }
+    }
+    // ---- columns kept in front of each chunk, and the first `need` of the ties
+    int run[KPT], total = 0;
+    if (some_ties || p.kept_idx) {
+        int n[KPT], m[KPT], tied[KPT];
+#pragma unroll
+        for (int c = 0; c < KPT; c++) {
+            n[c] = __builtin_popcount(keep[c]);
+            m[c] = __builtin_popcount(ties[c]);
+        }
+        prefix_wave(s_tot[0], n, run);
+        prefix_wave(s_tot[1], m, tied);
+        __syncthreads();
+        total = prefix_row(s_tot[0], run);
+        const int all = prefix_row(s_tot[1], tied);
+        total += all < (int)need ? all : (int)need;
+#pragma unroll
+        for (int c = 0; c < KPT; c++) {
+            int left = (int)need - tied[c];
+            run[c] += left > 0 ? tied[c] : (int)need;
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if ((ties[c] >> j) & 1u) {
+                    if (left > 0) keep[c] |= 1u << j;
+                    left--;
+                }
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < KPT; c++) keep[c] |= ties[c];
     }
 
     // ---- the mask row, and its bits (key j of a row in bit j % 8 of byte j / 8)
@@ -260,10 +263,6 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
     // round_up(Lk, 16): the row has room
     if (p.kept_idx) {
         int32_t *irow = p.kept_idx + (size_t)row * p.kept_ld, *crow = p.kept_cnt + (size_t)row * p.kept_ld;
-        int n[KPT], run[KPT];
-#pragma unroll
-        for (int c = 0; c < KPT; c++) n[c] = __builtin_popcount(keep[c]);
-        const int total = prefix(s_tot[1], n, run);
 #pragma unroll
         for (int c = 0; c < KPT; c++) {
             const int col = first_col(c);
@@ -432,13 +431,9 @@ __global__ void __launch_bounds__(NT) make_mask_memory_kernel(const MaskParams p
 #pragma unroll
                     for (int j = 0; j < 8; j++)
                         if (j < n && order_key(v[j]) == T) mine++;
-                    uint32_t incl = mine;
-#pragma unroll
-                    for (int off = 1; off < 64; off <<= 1) {
-                        const uint32_t t = __shfl_up(incl, off);
-                        if (lane >= off) incl += t;
-                    }
-                    if (lane == 63) wave_cnt[wave] = incl;
+                    int wave_total;
+                    const uint32_t incl = (uint32_t)wave_scan((int)mine, lane, wave_total);
+                    if (lane == 0) wave_cnt[wave] = (uint32_t)wave_total;
                     __syncthreads();
                     uint32_t rank = taken + incl - mine, chunk_total = 0;
                     for (int w = 0; w < NT / 64; w++) {

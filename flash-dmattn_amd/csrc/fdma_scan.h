@@ -29,13 +29,9 @@ __device__ __forceinline__ void scan_mask_row(const uint8_t *mrow, int Lk, int32
                 if ((mv[e >> 2] >> (8 * (e & 3))) & 0xffu) bits |= 1u << e;
         }
         const int n = __builtin_popcount(bits);
-        int incl = n;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(incl, off);
-            if (lane >= off) incl += t;
-        }
-        if (lane == 63) s_wave[wave] = incl;
+        int wave_total;
+        const int incl = wave_scan(n, lane, wave_total);
+        if (lane == 0) s_wave[wave] = wave_total;
         __syncthreads();
         int woff = 0, total = 0;
 #pragma unroll
