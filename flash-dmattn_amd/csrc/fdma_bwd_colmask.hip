@@ -709,33 +709,24 @@ __global__ void __launch_bounds__(NTHREADS) bwd_dkdv_parts_sum_kernel(const BwdP
     }
 }
 
-// The dQ launch of a compacted backward carries the reduction of the dK/dV partials along: `red_octets` groups of 8
-// consecutive workgroups (one per XCD) do that instead of dQ work, one such group after every `period - 1` groups
-// of dQ workgroups.  The reduction only moves memory while the dQ workgroups keep the matrix units busy, so side by
-// side it costs next to nothing; as a launch of its own it took as long as its memory traffic.
+// The dQ launch of a compacted backward carries the reduction of the dK/dV partials along: `red_count` consecutive workgroups
+// (a multiple of 8) do that instead of dQ work.  They only move memory, so side by side with dQ workgroups, which keep the matrix
+// units busy, they cost little; as a launch of its own the reduction took as long as its memory traffic.
+// One to a CU, in front of all others: they are done early, and the dQ workgroups then start heaviest first as if they were
+// alone.  Spread through the launch instead, one beside three dQ workgroups, they kept those from their CUs (half of the CUs' time
+// was idle).  Spread / in front (us, the whole step): 4 x 2048 tokens, 16/8 heads, d = 64 with its layer 174 / 165; 8192 x 8/4, d = 64
+// 117 / 104; d = 128: 8192 x 32/8 724 / 718, 2048 x 32/8 126 / 117, 4096 x 16/4 164 / 149, 2 x 4096 x 8/2 132 / 119, 12000 x 8/2 263 / 240;
+// half as many 0.95 to 1.16 times that, twice as many the same.
 // Few query rows against many keys are the other way round: few dQ workgroups, which leave CUs free, and partials by the number
-// of keys.  Interleaved there is at most one summing group per dQ group; all that the items ask for then follow the dQ groups in
-// one piece (period 1).  100 rows of 16 heads over 2048 kept keys, d = 128 (16 dQ workgroups): the launch 361 us with 16
-// summing workgroups, 54 with 1024.
-struct RedInterleave {
-    int red_octets, period, start;
-};
-inline RedInterleave red_interleave(int dq_octets, int items) {
-    RedInterleave r;
-    r.red_octets = (items < 1024 ? items : 1024) / 8;
-    if (r.red_octets < 1) r.red_octets = 1;
-    if (8 * dq_octets <= device_cus() && r.red_octets > dq_octets) {
-        r.period = 1;
-        r.start = dq_octets;
-        return r;
-    }
-    r.period = (dq_octets + r.red_octets) / r.red_octets;
-    r.period = r.period < 2 ? 2 : (r.period > 4 ? 4 : r.period);
-    if (r.red_octets > dq_octets / (r.period - 1)) r.red_octets = dq_octets / (r.period - 1);
-    if (r.red_octets < 1) r.red_octets = 1;  // (dq_octets >= 1 and period == 2 then)
-    // the interleaved stretch ends with the launch; the dQ groups in front of it are the heaviest ones
-    r.start = dq_octets - r.red_octets * (r.period - 1);
-    return r;
+// of keys.  All that the items ask for then follow the dQ workgroups.  100 rows of 16 heads over 2048 kept keys, d = 128 (16 dQ
+// workgroups): the launch 361 us with 16 summing workgroups, 54 with 1024.  Up to half a dQ workgroup per CU, or one where the keys
+// are more than twice the rows: behind / in front (us, the step) 1300 rows x 16/4 heads over 1500 kept of 4000, d = 128 133.5 / 135.4;
+// 4096 x 8/2, all 4096 keys to choose from, 124 / 121 at d = 128, 98.6 / 96.1 at 64.
+inline void place_reduction(BwdParams &p, int n_dq, int items) {
+    const bool few = (p.f.Lk > 2 * p.f.Lq ? 1 : 2) * n_dq <= device_cus();
+    const int most = few ? 1024 : device_cus();
+    p.red_count = ((items < most ? items : most) + 7) / 8 * 8;
+    p.red_first = few ? n_dq : 0;
 }
 
 template <typename T, int D, bool CAUSAL, bool CMP>
@@ -832,23 +823,13 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
     const int n_mb = (f.Lq + Q_BM - 1) / Q_BM;
     int lid = blockIdx.x;  // index among the dQ workgroups
     if (CMP) {
-        // groups of 8 workgroups (one per XCD): every `period`-th of the first red_octets * period groups sums
-        // partial results of the dK/dV kernel instead
-        const int R = p.red_octets, period = p.red_period;
-        int o = lid >> 3;
-        const int o2 = o - p.red_start;  // the groups before red_start are all dQ groups
-        if (o2 >= 0) {
-            if (o2 < R * period) {
-                if (o2 % period == period - 1) {
-                    dkdv_reduce_blocks<T, D>(p, (o2 / period) * 8 + (lid & 7), R * 8, threadIdx.x);
-                    return;
-                }
-                o -= o2 / period;
-            } else {
-                o -= R;
-            }
+        // some workgroups sum partial results of the dK/dV kernel instead
+        const int at = lid - p.red_first;
+        if (at >= 0 && at < p.red_count) {
+            dkdv_reduce_blocks<T, D>(p, at, p.red_count, threadIdx.x);
+            return;
         }
-        lid = o * 8 + (lid & 7);
+        if (at >= 0) lid -= p.red_count;
     }
     const XcdMap wm = xcd_map(lid, xcd_lists_per_pair(f.B * f.Hk), n_mb, G);
     if (!wm.valid) return;
@@ -1321,12 +1302,9 @@ hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
     const int n_dq = xcd_grid(f.B * f.Hk, xcd_lists_per_pair(f.B * f.Hk), (f.Lq + Q_BM - 1) / Q_BM, f.H / f.Hk);  // a multiple of 8
     if (!f.cmp.on) return launch_dq_grid<T, D, CAUSAL>(p, n_dq, stream);
     const int units_max = f.B * f.Hk * ((f.Lk + KV_BN - 1) / KV_BN);
-    const RedInterleave ri = red_interleave(n_dq / 8, units_max * (D / 16));
     BwdParams pr = p;
-    pr.red_octets = ri.red_octets;
-    pr.red_period = ri.period;
-    pr.red_start = ri.start;
-    return launch_dq_grid<T, D, CAUSAL>(pr, n_dq + 8 * ri.red_octets, stream);
+    place_reduction(pr, n_dq, units_max * (D / 16));
+    return launch_dq_grid<T, D, CAUSAL>(pr, n_dq + pr.red_count, stream);
 }
 
 }  // namespace

@@ -55,22 +55,13 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
     const int G = f.H / f.Hk;
     const int n_mb = (f.Lq + BM - 1) / BM;
     int lid = blockIdx.x;  // index among the dQ workgroups
-    if (CMP) {  // some groups of 8 workgroups sum partial results of the dK/dV kernel instead (see bwd_dq_colmask_kernel)
-        const int R = p.red_octets, period = p.red_period;
-        int o = lid >> 3;
-        const int o2 = o - p.red_start;
-        if (o2 >= 0) {
-            if (o2 < R * period) {
-                if (o2 % period == period - 1) {
-                    dkdv_reduce_blocks<T, D>(p, ((o2 / period) * 8 + (lid & 7)) * 2 + (wave >> 2), R * 16, tid & 255);
-                    return;
-                }
-                o -= o2 / period;
-            } else {
-                o -= R;
-            }
+    if (CMP) {  // some workgroups sum partial results of the dK/dV kernel instead (see place_reduction, fdma_bwd_colmask.hip)
+        const int at = lid - p.red_first;
+        if (at >= 0 && at < p.red_count) {
+            dkdv_reduce_blocks<T, D>(p, at * 2 + (wave >> 2), p.red_count * 2, tid & 255);
+            return;
         }
-        lid = o * 8 + (lid & 7);
+        if (at >= 0) lid -= p.red_count;
     }
     const XcdMap wm = xcd_map(lid, xcd_lists_per_pair(f.B * f.Hk), n_mb, G);
     if (!wm.valid) return;

@@ -104,17 +104,13 @@ __device__ __forceinline__ void dkdv_reduce_item(const BwdParams &p, const int u
     }
 }
 
-// Workgroup `rb` of `nrb` reducing workgroups takes every nrb-th of the U units x D/16 chunk pairs.  The first item
-// goes to the workgroup in the middle: when there are fewer items than workgroups (few units, each cut into many
-// parts: long sums) they run in the middle of the launch's interleaved stretch, neither beside the heaviest dQ
-// workgroups at its start nor in its tail.
+// Workgroup `rb` of `nrb` reducing workgroups takes every nrb-th of the U units x D/16 chunk pairs.
 template <typename T, int D>
 __device__ __forceinline__ void dkdv_reduce_blocks(const BwdParams &p, const int rb, const int nrb, const int tid) {
     const int32_t *plan = p.f.cmp.plan;
     const int U = plan[0];
     if (plan[1] * plan[2] == 1) return;  // no unit was split: the dK/dV kernel wrote the results itself
-    const int first = rb >= nrb / 2 ? rb - nrb / 2 : rb + nrb - nrb / 2;
-    for (int item = first; item < U * (D / 16); item += nrb) dkdv_reduce_item<T, D>(p, item / (D / 16), item % (D / 16), tid);
+    for (int item = rb; item < U * (D / 16); item += nrb) dkdv_reduce_item<T, D>(p, item / (D / 16), item % (D / 16), tid);
 }
 
 }  // namespace
