@@ -649,7 +649,7 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
     constexpr int MAXL = 1024;               // ... and with at most this many unit lists (LDS: every block of the launch pays for it)
     __shared__ int s_sum, s_max, s_units, s_wsum[4], s_wmax[4];
     __shared__ int s_Gs, s_Sm, s_Q, s_fit, s_q1, s_parts2, s_over2;
-    __shared__ int s_first[MAXU + 1], s_nt[MAXU], s_len[MAXU], s_nseg[MAXU], s_uoff[MAXU], s_lcount[MAXL], s_cand[64][8];
+    __shared__ int s_first[MAXU + 1], s_nt[MAXU], s_seg[MAXU], s_uoff[MAXU], s_lcount[MAXL], s_cand[8][64];
     __shared__ int s_pair[MAXU], s_ntx[MAXU];  // pair of a unit; its query blocks and, in the upper half, its XCD
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // units per pair and their prefix, 256 pairs at a time
@@ -734,7 +734,7 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
     }
     if (tid < 64) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) s_cand[tid][e] = 0;
+        for (int e = 0; e < 8; e++) s_cand[e][tid] = 0;
     }
     __syncthreads();
     const int k = dkdv_lists_per_pair(pairs);
@@ -768,15 +768,16 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const int ce = (int)((c[e >> 1] >> (16 * (e & 1))) & 0xffffu);
-            if (ce) atomicAdd(&s_cand[cand][e], ce);
+            if (ce) atomicAdd(&s_cand[e][cand], ce);
         }
         __syncthreads();
         if (tid < 64) {
             int worst = 0, parts = 0;
 #pragma unroll
-            for (int e = 0; e < 8; e++) { worst = s_cand[tid][e] > worst ? s_cand[tid][e] : worst; parts += s_cand[tid][e]; }
-            if (tid == 63) { s_parts2 = parts * Gs0; s_over2 = worst * Gs0 * 8 > slots; }  // (more than one round on some XCD)
-            else if (worst * Gs0 * 8 <= slots) atomicMin(&s_q1, Qc);
+            for (int e = 0; e < 8; e++) { worst = s_cand[e][tid] > worst ? s_cand[e][tid] : worst; parts += s_cand[e][tid]; }
+            const bool over = worst * Gs0 * 8 > slots;  // (more than one round on some XCD)
+            const int q1 = -wave_max(tid < 63 && !over ? -Qc : -(1 << 30));
+            if (tid == 63) { s_parts2 = parts * Gs0; s_over2 = over; s_q1 = q1; }
         }
     }
     __syncthreads();
@@ -810,21 +811,21 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
     const int Q = s_Q, Sm = s_Sm;
     for (int g = tid; g < U; g += 256) {
         const int n_seg = dkdv_segments(s_nt[g], Q, Sm);
-        s_nseg[g] = n_seg;
-        s_len[g] = n_seg > 0 ? (s_nt[g] + n_seg - 1) / n_seg : 0;
+        s_seg[g] = (n_seg > 0 ? (s_nt[g] + n_seg - 1) / n_seg : 0) << 8 | n_seg;  // length of its parts, their number (at most 16)
     }
     __syncthreads();
     for (int g = tid; g < U; g += 256) {
         const int i = s_pair[g], first = s_first[i], n = s_first[i + 1] - first, un = g - first;
-        const int mine = s_len[g], fold = dkdv_list_of(un, k);
+        const int own = s_seg[g], fold = dkdv_list_of(un, k);
         int before = 0;  // parts of the units of the same list that come first
 #pragma unroll 4
         for (int v = 0; v < n; v++) {
-            const bool first_v = dkdv_list_of(v, k) == fold && (s_len[first + v] > mine || (s_len[first + v] == mine && v < un));
-            before += first_v ? s_nseg[first + v] : 0;
+            const int other = s_seg[first + v], longer = (other >> 8) - (own >> 8);
+            const bool first_v = dkdv_list_of(v, k) == fold && (longer > 0 || (longer == 0 && v < un));
+            before += first_v ? other & 0xff : 0;
         }
         s_uoff[g] = Gs0 * before;
-        atomicAdd(&s_lcount[i * k + fold], Gs0 * s_nseg[g]);
+        atomicAdd(&s_lcount[i * k + fold], Gs0 * (own & 0xff));
     }
     __syncthreads();
     int32_t *lists = plan + DKDV_PLAN_HDR + pairs + 1;
@@ -841,44 +842,46 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
         if (off > cap) plan[6] = 1;
     }
     __syncthreads();
-    for (int g = tid; g < U; g += 256) {
-        const int i = s_pair[g], un = g - s_first[i], vl = i * k + dkdv_list_of(un, k), ns = s_nseg[g];
-        int o = s_lcount[vl] + s_uoff[g];
-        int32_t *e = lists + 8 + 2 * ((size_t)(vl & 7) * cap);
-        for (int gi = 0; gi < Gs0; gi++)
-            for (int sg = 0; sg < ns; sg++) {
-                if (o < cap) {
-                    e[2 * o] = i;
-                    e[2 * o + 1] = un | ((gi * Sm + sg) << 16);
-                }
-                o++;
-            }
+    // (a thread per part slot, not per unit: few units have many parts each)
+    const int per = Gs0 * Sm;
+    const float r_per = 1.0f / (float)per, r_sm = 1.0f / (float)Sm;
+    for (int sl = tid; sl < U * per; sl += 256) {
+        const int g = (int)(((float)sl + 0.5f) * r_per), x = sl - g * per, gi = (int)(((float)x + 0.5f) * r_sm), sg = x - gi * Sm;
+        const int i = s_pair[g], un = g - s_first[i], vl = i * k + dkdv_list_of(un, k), ns = s_seg[g] & 0xff;
+        const int o = s_lcount[vl] + s_uoff[g] + gi * ns + sg;
+        if (sg < ns && o < cap) {
+            int32_t *e = lists + 8 + 2 * ((size_t)(vl & 7) * cap + o);
+            e[0] = i;
+            e[1] = un | x << 16;
+        }
     }
 }
 
-// Everything the compacted backward needs after the scan, in one launch: one workgroup of layer 0 of the grid makes the
-// dK/dV plan, layer 1 gathers K / V rows, layer 2 clears the gradients of dropped keys, and the layers from 3 on compute
-// D = rowsum(dO * O), which depends on none of the others.
-// The plan is a chain of dependent steps of a single workgroup: in the FIRST layer it starts with the launch and the others
-// run beside it.  (4 x 2048 tokens, 8 kv heads, d = 64: the chain was the launch, 26 us, most of it the comparison of
-// segment lengths walking the units with a division each; with what a unit contributes made once and the prefixes taken by
-// whole waves the launch takes 12 us.  8192 tokens of 32 heads, d = 128: 30 us, bound by reading dO and O.)
+// Everything the compacted backward needs after the scan, in one launch: the first workgroup of the grid makes the dK/dV plan; of
+// the others (the first column of the grid aside) layer 0 clears the gradients of dropped keys, layer 1 gathers K / V rows where
+// that is not done yet, and the layers behind them compute D = rowsum(dO * O), which depends on none of the others.
+// The plan is a chain of dependent steps of a single workgroup: it starts with the launch and the others run beside it.  On
+// small calls it is the launch: 10 us with candidates counted in one LDS bank and a thread per unit to write the lists, 6.5 with
+// counters side by side and a thread per part (launch, us: 4096 tokens x 8/2 heads, d = 64 12.0 / 7.2, 16000 x 2/1 12 / 7.2).  Larger
+// ones read dO and O: 4 x 2048 x 16/8, d = 64 13.3 with two layers of 1024 workgroups that had nothing to do, 12.5 without;
+// 8192 tokens of 32 heads, d = 128 30.
 template <typename T>
 __global__ void __launch_bounds__(256) compact_bwd_prepass_kernel(const BwdParams bp, const int32_t *idx, int32_t *cnt,
                                                                    const int32_t *count, float *fb, uint16_t *kc, uint16_t *vc,
                                                                    int ld, int Hfb, int32_t *plan, int slots, int cap, int do_gather) {
     const FwdParams &f = bp.f;
-    if (blockIdx.z == 1) {
-        // (not when the lists and copies exist already: made by an earlier launch, or by the forward call)
-        if (do_gather) gather_block<T>(f, idx, cnt, count, fb, kc, vc, ld, Hfb, blockIdx.x, blockIdx.y, do_gather == 2);
-    } else if (blockIdx.z == 2) {
-        zero_block(bp, bp.dbias != nullptr && bp.dbias_accum == nullptr, blockIdx.x, blockIdx.y);
-    } else if (blockIdx.z == 0) {
-        if (blockIdx.x == 0 && blockIdx.y == 0)
+    const int first_dot = do_gather ? 2 : 1, bx = (int)blockIdx.x - 1;
+    if (bx < 0) {
+        if (blockIdx.y == 0 && blockIdx.z == 0)
             plan_block(count, idx, ld, plan, f.B * f.Hk, f.H / f.Hk, f.Lq, f.Lk, f.causal, slots, cap);
+    } else if (blockIdx.z == 0) {
+        zero_block(bp, bp.dbias != nullptr && bp.dbias_accum == nullptr, bx, blockIdx.y);
+    } else if ((int)blockIdx.z < first_dot) {
+        // (not when the lists and copies exist already: made by an earlier launch, or by the forward call)
+        gather_block<T>(f, idx, cnt, count, fb, kc, vc, ld, Hfb, bx, blockIdx.y, do_gather == 2);
     } else {  // the blocks of D = rowsum(dO * O), laid out over the remaining layers
         const int nbx = (bp.Lq_rounded + bwd_dot_rows_per_block(f.d) - 1) / bwd_dot_rows_per_block(f.d);
-        const int64_t lin = ((int64_t)(blockIdx.z - 3) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+        const int64_t lin = ((int64_t)((int)blockIdx.z - first_dot) * gridDim.y + blockIdx.y) * (gridDim.x - 1) + bx;
         if (lin >= (int64_t)nbx * f.H * f.B) return;
         bwd_dot_block<T>(bp, (int)(lin % nbx), (int)((lin / nbx) % f.H), (int)(lin / ((int64_t)nbx * f.H)));
     }
@@ -1037,10 +1040,10 @@ hipError_t compact_setup(FwdParams &p, void *ws, int dtype, hipStream_t stream, 
         const int64_t layer = (int64_t)grid.x * pairs;
         const int64_t dot_layers = (dot_blocks + layer - 1) / layer;
         const bool with_dot = p.cu_q == nullptr && 3 + dot_layers <= 65535;
-        const dim3 grid3(grid.x, pairs, with_dot ? (unsigned)(3 + dot_layers) : 3);
         // 0: lists and copies exist; 1: gather here; 2: the lists are the forward call's, whose copies are tile images --
         // only the row-major K / V copies are made here
         const int do_gather = fwd_ws ? (l.img ? 2 : 0) : (gather_alone ? 0 : 1);
+        const dim3 grid3(grid.x + 1, pairs, (unsigned)((do_gather ? 2 : 1) + (with_dot ? dot_layers : 0)));
         if (dtype == 0)
             hipLaunchKernelGGL((compact_bwd_prepass_kernel<bf16_tag>), grid3, dim3(256), 0, stream, *bp, idx, cnt, count, fb, kc, vc,
                                l.ld, l.Hfb, plan, 2 * device_cus(), plan_cap, do_gather);
