@@ -170,13 +170,23 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
     // wait for it -- and for every load issued before it -- land in front of the matrix work instead of behind it.
     const uint8_t *mask_ld = f.mask ? f.mask : (const uint8_t *)f.k;
     const uint16_t *bias_ld = has_bias ? (const uint16_t *)f.bias : (const uint16_t *)f.k;
-    auto step_head = [&](int step, int &gi, int &mi) {
-        gi = m_outer ? step % G : step / n_m;
-        mi = M_blocks - 1 - m_lo - (m_outer ? step / G : step % n_m);
+    const int mi_last = M_blocks - m_lo - n_m;
+    // Where the step behind (gi, mi), number `step`, is.  Kept up instead of divided out of the step's number: two scalar divisions
+    // are 60 instructions (112 -> 100 us, 1999 tokens, 16 heads over 4 that share their rows, d = 64).  Not in the variant of two
+    // workgroups per CU, whose registers are full (110 against 118 us, 16 heads of their own).
+    constexpr bool DIVIDE = D <= 64 && !GSUM;
+    auto advance = [&](int &gi, int &mi, int step) {  // (without branches: they would put the positions on the stack)
+        if (DIVIDE) {
+            gi = m_outer ? step % G : step / n_m;
+            mi = M_blocks - 1 - m_lo - (m_outer ? step / G : step % n_m);
+            return;
+        }
+        const bool wrap = m_outer ? gi == G - 1 : mi == mi_last;
+        const int gt = m_outer && wrap ? 0 : gi + (m_outer || wrap ? 1 : 0);
+        mi = !m_outer && wrap ? M_blocks - 1 - m_lo : mi - (!m_outer || wrap ? 1 : 0);
+        gi = gt;
     };
-    auto load_step = [&](int step) {
-        int gi, mi;
-        step_head(step, gi, mi);
+    auto load_step = [&](int gi, int mi) {
         const int h = hk * G + gi, m0 = mi * KV_BM;
         const uint16_t *qbase = (const uint16_t *)f.q + b * f.q_b + h * f.q_h + qcol;
         const uint16_t *dobase = (const uint16_t *)p.dout + b * p.do_b + h * p.do_h + qcol;
@@ -268,15 +278,20 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
             for (int i = 0; i < 16; i++) dsum[mb][i] = 0.f;
     }
 
+    int gi = 0, mi = M_blocks - 1 - m_lo;
+    auto load_next = [&](int step) {
+        int gn = gi, mn = mi;
+        advance(gn, mn, step + 1);
+        load_step(gn, mn);
+    };
     if (n_steps > 0) {
-        load_step(0);
+        load_step(gi, mi);
         store_step(0);
         __syncthreads();
     }
 
     for (int step = 0; step < n_steps; step++) {
-        int gi, mi;
-        step_head(step, gi, mi);
+        if (DIVIDE) advance(gi, mi, step);
         const int h = hk * G + gi;
         const int m0 = mi * KV_BM;
         const int buf = step & 1;
@@ -318,7 +333,7 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
         // flight.  The softmax and the dK / dV GEMMs below cover the latency.
         __builtin_amdgcn_sched_barrier(0);
         if (GSUM || D > 64) {
-            if (step + 1 < n_steps) load_step(step + 1);
+            if (step + 1 < n_steps) load_next(step);
             __builtin_amdgcn_sched_barrier(0);
         }
 
@@ -377,7 +392,7 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
         // loads are issued here, behind the softmax; the other workgroup covers what the GEMMs below do not)
         if (!GSUM && D <= 64) {
             __builtin_amdgcn_sched_barrier(0);
-            if (step + 1 < n_steps) load_step(step + 1);
+            if (step + 1 < n_steps) load_next(step);
             __builtin_amdgcn_sched_barrier(0);
         }
         // ---- dV^T += dO^T P ; dK^T += Q^T dS
@@ -408,7 +423,7 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
                         for (int i = 0; i < 16; i++) part += ds[mb][i];
                 }
                 colsum += part;
-                const bool last_m = (step % n_m) == n_m - 1;
+                const bool last_m = DIVIDE ? (step % n_m) == n_m - 1 : mi == mi_last;
                 if (last_m && (f.Hb == f.H || gi == G - 1)) {
                     const float tot = xhalf_sum(colsum);
                     if (g == 0 && segs > 1) {
@@ -465,6 +480,7 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
             }
         }
         __syncthreads();
+        if (!DIVIDE) advance(gi, mi, step + 1);
     }
 
     // a key block that no query (of this segment) can see still owns its dbias column (row-broadcast case)

@@ -24,6 +24,11 @@
 // which bwd_dkdv_sum_kernel (fdma_bwd.hip) adds in segment order.
 // B = 1, L = 1999, H = 16, Hk = 4, d = 128, fp16, mask and bias rows shared by the group: 630 us as 64 workgroups of four
 // waves, 112 + 7 (sums) as 256 of eight; B = 1, L = 4096, H = Hk = 16, bf16, causal: 320 -> 210 us.
+// Positions and bases are kept up from step to step and a lane's offsets are two registers: with divisions of the step's number and
+// the addresses made from scratch a third of the vector instructions of a step were for that.  The first call 116 -> 103 us, 3000 x 8/8,
+// d = 96 122 -> 111, 2048 x 16/4 83 -> 72, 2 x 700 x 8/2 with one bias value per key 49 -> 41.
+// (Wave pairs that share keys by role, as at head dim 256, with P through LDS: 122 us, and 130 with a pair half a step apart: the 32
+// rows of softmax per lane and the sums over heads want the registers that the roles free.)
 #include <type_traits>
 
 #include "fdma_common.h"
@@ -90,16 +95,19 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
     const bool bias_rows = has_bias && f.bi_r != 0;   // per-query bias (and dbias) rows
     const bool use_accum = p.dbias_accum != nullptr;   // several workgroups share a dbias element
     // per-query dbias wants (m outer, g inner) to sum dS over the group in registers; row-broadcast dbias wants
-    // (g outer, m inner) to keep one column sum per bias head
-    const bool m_outer = bias_rows;
+    // (g outer, m inner) to keep one column sum per bias head: see `advance`
     // a fused tile that all query heads of the group share stays for its G steps: its inputs are fetched once, at the first
     // of them (G - 1 more steps until they are needed), and it is replaced -- by dS, then by the next tile -- at the last
     const bool hold = GSUM && bias_rows && f.Hb != f.H && (!f.mask || f.Hm != f.H);
-    auto step_head = [&](int step, int &gi, int &mi) {
-        gi = m_outer ? step % G : step / n_m;
-        mi = M_blocks - 1 - m_lo - (m_outer ? step / G : step % n_m);
+    const int mi_last = M_blocks - m_lo - n_m;
+    auto advance = [&](int &gi, int &mi) {  // (without branches: they would put the positions on the stack)
+        const bool wrap = bias_rows ? gi == G - 1 : mi == mi_last;
+        const int gt = bias_rows && wrap ? 0 : gi + (bias_rows || wrap ? 1 : 0);
+        mi = !bias_rows && wrap ? M_blocks - 1 - m_lo : mi - (!bias_rows || wrap ? 1 : 0);
+        gi = gt;
     };
 
+    const bool per_head = f.Hb == f.H;
     // zero the part of a per-query dbias this workgroup owns but never visits (above the causal diagonal)
     if (bias_rows && !use_accum && m_start > 0 && seg == 0) {
         const int ngh = (f.Hb == f.H) ? G : 1;
@@ -136,34 +144,49 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
         const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
         return (gptr_t)(((uint64_t)hi << 32) | lo);
     };
-    const int m_last = (f.Lq - 1) / BM, row_last = (f.Lq - 1) % BM;
+    // bases of the group's first head, and bytes from one head, and one row, to the next
+    const int h0 = hk * G;
+    const int64_t q_h2 = f.q_h * 2, do_h2 = p.do_h * 2;
+    const char *q_base = (const char *)((const uint16_t *)f.q + b * f.q_b + h0 * f.q_h), *do_base = (const char *)((const uint16_t *)p.dout + b * p.do_b + h0 * p.do_h);
+    const int st_h = wave & 1 ? p.Lq_rounded : f.Lq;
+    const float *st_base = (wave & 1 ? p.softmax_d : f.lse) + ((int64_t)b * f.H + h0) * st_h;
+    // offsets of this lane's pieces: its row (clamped per step: offsets grow with the row), its two columns
+    const uint32_t q_r2 = (uint32_t)(f.q_r * 2), do_r2 = (uint32_t)(p.do_r * 2);
+    uint32_t q_row, do_row, pcol[2];
+    {
+        const int row = 8 * wave + (lane >> 4);
+        q_row = row * q_r2;
+        do_row = row * do_r2;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int chunk = (lane & 15) ^ (int)TL::swz(row + 4 * i);
+            pcol[i] = chunk * 8 < f.d ? chunk * 16 : 0;
+        }
+    }
+    auto least = [](uint32_t x, uint32_t y) { return x < y ? x : y; };
     gptr_t ld_q = nullptr, ld_do = nullptr, ld_stat = nullptr;
-    int ld_rows = 0;  // last existing row of the step being fetched
+    uint32_t ld_rows = 0;  // last existing row of the step being fetched
     uint32_t ld_dst = 0;
-    auto dma_begin = [&](int step, int buf) {
-        int gi, mi;
-        step_head(step, gi, mi);
-        const int h = hk * G + gi, m0 = mi * BM;
-        ld_q = uniform_ptr((const uint16_t *)f.q + b * f.q_b + h * f.q_h + (int64_t)m0 * f.q_r);
-        ld_do = uniform_ptr((const uint16_t *)p.dout + b * p.do_b + h * p.do_h + (int64_t)m0 * p.do_r);
-        ld_stat = uniform_ptr((wave & 1) ? p.softmax_d + ((int64_t)b * f.H + h) * p.Lq_rounded + m0 : f.lse + ((int64_t)b * f.H + h) * f.Lq + m0);
-        ld_rows = mi == m_last ? row_last : BM - 1;
+    auto dma_begin = [&](int gi, int m0, int buf) {
+        ld_q = uniform_ptr(q_base + gi * q_h2 + (int64_t)m0 * q_r2);
+        ld_do = uniform_ptr(do_base + gi * do_h2 + (int64_t)m0 * do_r2);
+        ld_stat = uniform_ptr(st_base + gi * st_h + m0);
+        const int left = f.Lq - 1 - m0;
+        ld_rows = (uint32_t)(left < BM - 1 ? left : BM - 1);
         ld_dst = lds0 + buf * STAGE;
     };
     // (written in assembly and waited for by hand, as in fdma_bwd_colmask.hip: behind the compiler's builtin every LDS read
     // waits for all LDS operations in flight.  m0 carries the LDS address.)
     auto dma_piece = [&](int n) {
         if (n < 4) {
-            const int i = 2 * wave + (n & 1), row = 4 * i + (lane >> 4), row_c = row < ld_rows ? row : ld_rows;
-            const int chunk = (lane & 15) ^ (int)TL::swz(row);
-            const int col = chunk * 8 < f.d ? chunk * 8 : 0;
-            const uint32_t off = (uint32_t)(row_c * (int)(n < 2 ? f.q_r : p.do_r) + col) * 2;
+            const int i = n & 1;
+            const uint32_t r2 = n < 2 ? q_r2 : do_r2;
+            const uint32_t off = least((n < 2 ? q_row : do_row) + 4 * i * r2, ld_rows * r2) + pcol[i];
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         : : "v"(off), "s"(n < 2 ? ld_q : ld_do), "s"(__builtin_amdgcn_readfirstlane(ld_dst + (n < 2 ? 0 : TILE) + i * 1024)));
+                         : : "v"(off), "s"(n < 2 ? ld_q : ld_do), "s"(__builtin_amdgcn_readfirstlane(ld_dst + (n < 2 ? 0 : TILE) + (2 * wave + i) * 1024)));
         } else {
-            const uint32_t off = (uint32_t)(lane < ld_rows ? lane : ld_rows) * 4;
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-                         : : "v"(off), "s"(ld_stat), "s"(__builtin_amdgcn_readfirstlane(ld_dst + 2 * TILE + (wave & 1) * BM * 4)));
+                         : : "v"(least((uint32_t)lane, ld_rows) * 4), "s"(ld_stat), "s"(__builtin_amdgcn_readfirstlane(ld_dst + 2 * TILE + (wave & 1) * BM * 4)));
         }
     };
 
@@ -176,32 +199,29 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
     u32x2_t mraw[2];
     // Every load is unconditional and raw (clamped rows / keys; an absent mask or bias is read from K, any valid address,
     // and ignored later): nothing looks at a value before the step's first barrier.
-    auto fb_load = [&](int step) {
-        int gi, mi;
-        step_head(step, gi, mi);
-        const int h = hk * G + gi, m0 = mi * BM;
-        const int hm = f.mask ? (f.Hm == f.H ? h : (f.Hm == 1 ? 0 : hk)) : 0;
-        const int hb = has_bias ? (f.Hb == f.H ? h : (f.Hb == 1 ? 0 : hk)) : 0;
-        const uint16_t *bias_ld = has_bias ? (const uint16_t *)f.bias + b * f.bi_b + hb * f.bi_h : (const uint16_t *)f.k;
-        const uint8_t *mask_ld = f.mask ? (f.mbits ? f.mbits + b * f.mb_b + hm * f.mb_h : f.mask + b * f.m_b + hm * f.m_h) : (const uint8_t *)f.k;
+    const int hm0 = f.Hm == 1 ? 0 : f.Hm == f.H ? h0 : hk, hb0 = f.Hb == 1 ? 0 : f.Hb == f.H ? h0 : hk;
+    const uint8_t *m_base = !f.mask ? (const uint8_t *)f.k : f.mbits ? f.mbits + b * f.mb_b + hm0 * f.mb_h : f.mask + b * f.m_b + hm0 * f.m_h;
+    const int64_t m_h1 = f.mask && f.Hm == f.H ? (f.mbits ? f.mb_h : f.m_h) : 0, m_r1 = f.mask ? (f.mbits ? f.mb_r : f.m_r) : 0;
+    const uint16_t *bi_base = has_bias ? (const uint16_t *)f.bias + b * f.bi_b + hb0 * f.bi_h : (const uint16_t *)f.k;
+    const int64_t bi_h1 = has_bias && per_head ? f.bi_h : 0, bi_r1 = has_bias ? f.bi_r : 0;
+    auto fb_load = [&](int gi, int m0) {
         asm volatile("" : "+v"(br0), "+v"(kk));
-        const int kk_c = kk < f.Lk ? kk : 0, at = chunk8_at<ODD>(kk, f.Lk);
-        const int64_t b_r = has_bias ? f.bi_r : 0, m_r = f.mask ? (f.mbits ? f.mb_r : f.m_r) : 0;
+        const int at = chunk8_at<ODD>(kk, f.Lk), m_at = !f.mask ? 0 : f.mbits ? ((kk < f.Lk ? kk : 0) >> 3) & ~7 : at, b_at = has_bias ? at : 0;
+        const uint8_t *mp = m_base + gi * m_h1 + m0 * m_r1;
+        const uint16_t *bp = bi_base + gi * bi_h1 + m0 * bi_r1;
 #pragma unroll
         for (int it = 0; it < 2; it++) {
-            int qq = m0 + br0 + 32 * it;
-            qq = qq < f.Lq ? qq : f.Lq - 1;
-            braw[it] = *(const u32x4_el_t *)(bias_ld + (qq * b_r + (has_bias ? at : 0)));
-            mraw[it] = *(const u32x2_any_t *)(mask_ld + (qq * m_r + (f.mask ? (f.mbits ? (kk_c >> 3) & ~7 : at) : 0)));
+            int row = br0 + 32 * it;
+            row = row < f.Lq - m0 ? row : f.Lq - 1 - m0;
+            braw[it] = *(const u32x4_el_t *)(bp + (row * bi_r1 + b_at));
+            mraw[it] = *(const u32x2_any_t *)(mp + (row * m_r1 + m_at));
         }
     };
-    char *fb_chunk = smem + OFF_FB + (br0 * SB + 8 * bc) * 2;
-    auto fb_store = [&](int step) {
-        int gi, mi;
-        step_head(step, gi, mi);
+    const uint32_t fb_chunk = lds0 + OFF_FB + (br0 * SB + 8 * bc) * 2;
+    auto fb_store = [&](int m0) {
 #pragma unroll
         for (int it = 0; it < 2; it++) {
-            const int qq = mi * BM + br0 + 32 * it;
+            const int qq = m0 + br0 + 32 * it;
             u32x4_t bv = has_bias ? chunk8_fix<ODD>(braw[it], kk, f.Lk) : u32x4_t{0, 0, 0, 0};
             u32x2_t mv = f.mask ? (f.mbits ? mask_bits_to_bytes(mask_bits_byte(mraw[it], kk < f.Lk ? kk : 0)) : chunk8_fix_mask<ODD>(mraw[it], kk, f.Lk)) : u32x2_t{0x01010101u, 0x01010101u};
             // keys of the chunk this row may see
@@ -220,7 +240,7 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
                 bv[2 * hlf] = (bv[2 * hlf] & m0w) | (NegInfPair<T>::value & ~m0w);
                 bv[2 * hlf + 1] = (bv[2 * hlf + 1] & m1w) | (NegInfPair<T>::value & ~m1w);
             }
-            *(u32x4_t *)(fb_chunk + 32 * it * SB * 2) = bv;
+            *(__attribute__((address_space(3))) u32x4_t *)(uintptr_t)(fb_chunk + 32 * it * SB * 2) = bv;
         }
     };
 
@@ -251,30 +271,33 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
         for (int i = 0; i < 16; i++) dsum[GSUM ? i : 0] = 0.f;
     }
 
+    int gi = 0, mi = M_blocks - 1 - m_lo;
     if (n_steps > 0) {
-        fb_load(0);
-        dma_begin(0, 0);
+        fb_load(0, mi * BM);
+        dma_begin(0, mi * BM, 0);
 #pragma unroll
         for (int n = 0; n < 5; n++) dma_piece(n);
-        fb_store(0);
+        fb_store(mi * BM);
     }
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
     __syncthreads();
 
     auto one_step = [&](auto buf_c, const int step) {
         constexpr int buf = decltype(buf_c)::value;
-        int gi, mi;
-        step_head(step, gi, mi);
-        const int h = hk * G + gi, m0 = mi * BM;
-        const int hb = has_bias ? (f.Hb == f.H ? h : (f.Hb == 1 ? 0 : hk)) : 0;
-        const int next = step + 1 < n_steps ? step + 1 : step;  // (past the last step its tiles are fetched again and dropped)
+        const int m0 = mi * BM;
+        const int hb = per_head ? h0 + gi : hb0;
+        // the next step (past the last one its tiles are fetched again and dropped), and the step of the next fused tile
+        int gn = gi, mn = mi;
+        advance(gn, mn);
+        gn = step + 1 < n_steps ? gn : gi;
+        mn = step + 1 < n_steps ? mn : mi;
         // (the swizzled addresses are these constants XOR a compile-time value, recomputed where used: hoisted they would
         // cost registers)
         asm volatile("" : "+v"(a_off), "+v"(tr_off), "+v"(kv_off));
         const bool fb_in = !hold || gi == 0, fb_out = !hold || gi == G - 1;  // this step fetches / replaces a fused tile
-        const int fb_next = hold ? (step + G < n_steps ? step + G : step) : next;
-        if (fb_in) fb_load(fb_next);
-        dma_begin(next, buf ^ 1);
+        const int f_gi = hold ? 0 : gn, f_m0 = (hold ? (mi > mi_last ? mi - 1 : mi) : mn) * BM;
+        if (fb_in) fb_load(f_gi, f_m0);
+        dma_begin(gn, mn * BM, buf ^ 1);
         __builtin_amdgcn_sched_barrier(0);
 
         // ---- S = Q K^T and dP = dO V^T (M = query, N = key)
@@ -304,7 +327,10 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
         }
 
         // ---- P = exp2((S*scale + fused)*log2e - LSE*log2e) ; dS = P * (dP - D), 16 query rows (8 per lane) at a time
-        const bool dsum_first = f.Hb == f.H || gi == 0;          // (GSUM) this step starts a sum over the group
+        if (GSUM && (f.Hb == f.H || gi == 0)) {                  // this step starts a sum over the group
+#pragma unroll
+            for (int i = 0; i < 16; i++) dsum[GSUM ? i : 0] = 0.f;
+        }
         const bool dsum_last = f.Hb == f.H || gi == G - 1;       // ... ends one
         uint32_t ppk[8], dpk[8];
         float part = 0.f;
@@ -323,8 +349,13 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
                 const float x = __builtin_fmaf(__builtin_fmaf(s[8 * blk + e], f.scale, fb), kLog2e, -lse * kLog2e);
                 pv[e] = fast_exp2(x);
                 dsv[e] = (dp[8 * blk + e] - dd) * pv[e];
-                if (GSUM && bias_rows) dsum[GSUM ? 8 * blk + e : 0] = dsum_first ? dsv[e] : dsum[GSUM ? 8 * blk + e : 0] + dsv[e];
-                else part += dsv[e];
+            }
+            if (GSUM && bias_rows) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) dsum[GSUM ? 8 * blk + e : 0] += dsv[e];
+            } else if (!bias_rows) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) part += dsv[e];
             }
 #pragma unroll
             for (int e = 0; e < 4; e++) {
@@ -387,8 +418,7 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
             }
         }
         const bool tile_out = bias_rows && !use_accum && (!GSUM || dsum_last);
-        const int last_m = (step % n_m) == n_m - 1;
-        const bool col_out = has_bias && !bias_rows && last_m && (f.Hb == f.H || gi == G - 1);
+        const bool col_out = has_bias && !bias_rows && mi == mi_last && (f.Hb == f.H || gi == G - 1);
         if (has_bias && !bias_rows) {
             colsum += part;
             if (col_out) {
@@ -407,11 +437,11 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
 #pragma unroll
             for (int it = 0; it < 2; it++) {
                 const int qq = m0 + br0 + 32 * it;
-                const u32x4_t v = *(const u32x4_t *)(fb_chunk + 32 * it * SB * 2);
+                const u32x4_t v = lds_ld128(fb_chunk + 32 * it * SB * 2);
                 if (qq < f.Lq && kk < f.Lk) *(u32x4_t *)(dbp + ((int64_t)qq * p.db_r + kk)) = v;
             }
         }
-        if (fb_out) fb_store(next);
+        if (fb_out) fb_store(f_m0);
         if (col_out && tid < BN) {  // (a step's sums are overwritten two steps later at the earliest)
             const float tot = s_col[(step & 1) * 2 * BN + tid] + s_col[((step & 1) * 2 + 1) * BN + tid];
             const int kc = n0 + tid;
@@ -424,6 +454,8 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+        gi = gn;
+        mi = mn;
     };
     for (int step = 0; step < n_steps; step += 2) {
         one_step(std::integral_constant<int, 0>(), step);
