@@ -820,7 +820,6 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
     const FwdParams &f = p.f;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = tid & 63, r = lane & 31, g = lane >> 5;
     const int G = f.H / f.Hk;
-    const int n_mb = (f.Lq + Q_BM - 1) / Q_BM;
     int lid = blockIdx.x;  // index among the dQ workgroups
     if (CMP) {
         // some workgroups sum partial results of the dK/dV kernel instead
@@ -831,12 +830,11 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
         }
         if (at >= 0) lid -= p.red_count;
     }
-    const XcdMap wm = xcd_map(lid, xcd_lists_per_pair(f.B * f.Hk), n_mb, G);
-    if (!wm.valid) return;
-    const int m_block = n_mb - 1 - wm.unit;  // heaviest first under causal
-    const int b = wm.pair / f.Hk, hk = wm.pair % f.Hk;
+    const RowUnit ru = row_unit(f, lid, Q_BM);  // (heaviest first under causal)
+    if (ru.block < 0) return;
+    const int b = ru.pair / f.Hk, hk = ru.pair % f.Hk;
     const int h = hk * G + (lid / 8) % G;
-    const int m0 = m_block * Q_BM;
+    const int m0 = ru.block * Q_BM;
     const SeqInfo sq = seq_info(f, b);  // this batch entry's lengths and first rows (ragged batch: from cu_seqlens)
     const int LqS = sq.Lq, LkS = sq.Lk;
     if (m0 >= LqS) return;
@@ -852,8 +850,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
     const uint16_t *vbase = (const uint16_t *)f.v + b * f.v_b + sq.k0 * f.v_r + hk * f.v_h;
 
     // key columns this workgroup iterates over (the compacted list with CMP), and how many a row may see
-    const int Lk = CMP ? f.cmp.count[wm.pair] : LkS;
-    const int32_t *ccnt = CMP ? f.cmp.cnt + (int64_t)wm.pair * f.cmp.ld : nullptr;
+    const int Lk = CMP ? f.cmp.count[ru.pair] : LkS;
+    const int32_t *ccnt = CMP ? f.cmp.cnt + (int64_t)ru.pair * f.cmp.ld : nullptr;
     const float *fbrow = CMP ? f.cmp.fb + (int64_t)(b * f.cmp.Hfb + (f.cmp.Hfb == f.H ? h : hk)) * f.cmp.ld : nullptr;
     auto visible = [&](int row) -> int {  // columns [0, visible(row)) pass the causal test for `row`
         if (row >= LqS) row = LqS - 1;
@@ -1299,7 +1297,7 @@ hipError_t launch_dq_grid(const BwdParams &p, int grid, hipStream_t stream) {
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
     const FwdParams &f = p.f;
-    const int n_dq = xcd_grid(f.B * f.Hk, xcd_lists_per_pair(f.B * f.Hk), (f.Lq + Q_BM - 1) / Q_BM, f.H / f.Hk);  // a multiple of 8
+    const int n_dq = row_grid(f, Q_BM);  // a multiple of 8
     if (!f.cmp.on) return launch_dq_grid<T, D, CAUSAL>(p, n_dq, stream);
     const int units_max = f.B * f.Hk * ((f.Lk + KV_BN - 1) / KV_BN);
     BwdParams pr = p;

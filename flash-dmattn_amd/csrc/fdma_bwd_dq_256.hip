@@ -53,7 +53,6 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = tid & 63, r = lane & 31, g = lane >> 5;
     const int rw = wave & 3, role = wave >> 2;
     const int G = f.H / f.Hk;
-    const int n_mb = (f.Lq + BM - 1) / BM;
     int lid = blockIdx.x;  // index among the dQ workgroups
     if (CMP) {  // some workgroups sum partial results of the dK/dV kernel instead (see place_reduction, fdma_bwd_colmask.hip)
         const int at = lid - p.red_first;
@@ -63,12 +62,11 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
         }
         if (at >= 0) lid -= p.red_count;
     }
-    const XcdMap wm = xcd_map(lid, xcd_lists_per_pair(f.B * f.Hk), n_mb, G);
-    if (!wm.valid) return;
-    const int m_block = n_mb - 1 - wm.unit;  // heaviest first under causal
-    const int b = wm.pair / f.Hk, hk = wm.pair % f.Hk;
+    const RowUnit ru = row_unit(f, lid, BM);  // (heaviest first under causal)
+    if (ru.block < 0) return;
+    const int b = ru.pair / f.Hk, hk = ru.pair % f.Hk;
     const int h = hk * G + (lid / 8) % G;
-    const int m0 = m_block * BM;
+    const int m0 = ru.block * BM;
     const SeqInfo sq = seq_info(f, b);
     const int LqS = sq.Lq, LkS = sq.Lk;
     if (m0 >= LqS) return;
@@ -84,8 +82,8 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
     const uint16_t *vbase = (const uint16_t *)f.v + b * f.v_b + sq.k0 * f.v_r + hk * f.v_h;
 
     // key columns this workgroup iterates over (the compacted list with CMP), and how many a row may see
-    const int Lk = CMP ? f.cmp.count[wm.pair] : LkS;
-    const int32_t *ccnt = CMP ? f.cmp.cnt + (int64_t)wm.pair * f.cmp.ld : nullptr;
+    const int Lk = CMP ? f.cmp.count[ru.pair] : LkS;
+    const int32_t *ccnt = CMP ? f.cmp.cnt + (int64_t)ru.pair * f.cmp.ld : nullptr;
     const float *fbrow = CMP ? f.cmp.fb + (int64_t)(b * f.cmp.Hfb + (f.cmp.Hfb == f.H ? h : hk)) * f.cmp.ld : nullptr;
     auto visible = [&](int row) -> int {
         if (row >= LqS) row = LqS - 1;

@@ -1,5 +1,5 @@
 // Work items of the column-form dK/dV kernels (fdma_bwd_colmask.hip, fdma_bwd_dkdv_256.hip): which 128 keys, query heads and query
-// blocks a workgroup has, from its id.  (XcdMap: also the dQ kernel's.)
+// blocks a workgroup has, from its id.
 #pragma once
 
 #include "fdma_params.h"

@@ -112,32 +112,18 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
     const int g = lane >> 5;
 
     // Workgroup -> (batch, kv head, query head, query block), XCD-aware.  Workgroups are dealt to the 8
-    // XCDs round-robin by linear id and every XCD has its own L2.  The id is remapped so that the
-    // workgroups running at the same time on one XCD share K / V: the (batch, kv head) pairs are
-    // split into k = 8 / gcd(pairs, 8) interleaved lists of query blocks each, the resulting
-    // multiple-of-8 lists are dealt to the XCDs, and an XCD walks its lists one after the other,
-    // heaviest query block first, the G query heads of a block side by side.  Re-reads of K / V
+    // XCDs round-robin by linear id and every XCD has its own L2.  The id is remapped (row_unit) so that the
+    // workgroups running at the same time on one XCD share K / V: an XCD walks its lists of query blocks one after the
+    // other, heaviest block first, the G query heads of a block side by side.  Re-reads of K / V
     // tiles then hit in that XCD's L2, and every XCD gets the same amount of work.
-    const int n_mb = (p.Lq + BM - 1) / BM;  // p.Lq, p.Lk: the longest sequence of a ragged batch
+    const RowUnit ru = row_unit(p, blockIdx.x, BM);
+    if (ru.block < 0) return;
     const int G = p.H / p.Hk;
-    const int pairs = p.B * p.Hk;
-    const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
-    const int k_split = 8 / gcd8;
-    const int list_len = ((n_mb + k_split - 1) / k_split) * G;  // workgroups per list
-    const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-    const int vlist = xcd + 8 * (slot / list_len);
-    const int pos = slot % list_len;
-    const int pair = vlist / k_split;
-    const int mslot = (pos / G) * k_split + vlist % k_split;
-    if (mslot >= n_mb) return;
-    const int m_block = n_mb - 1 - mslot;
-    const int b = pair / p.Hk;
-    const int h = (pair % p.Hk) * G + pos % G;
-    const int hk = h / (p.H / p.Hk);
-    const int m0 = m_block * BM;
+    const int b = ru.pair / p.Hk, hk = ru.pair % p.Hk;
+    const int h = hk * G + (int)(blockIdx.x / 8) % G;
+    const int m0 = ru.block * BM;
     const SeqInfo sq = seq_info(p, b);  // this batch entry's lengths and first rows (ragged batch: from cu_seqlens)
     const int LqS = sq.Lq, LkS = sq.Lk;
-    if (m0 >= LqS) return;
     const int shift = LkS - LqS;
     const int wrow0 = m0 + wave * 32;  // first query row of this wave
 
@@ -897,10 +883,7 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
-    const int n_mb = (p.Lq + BM - 1) / BM, G = p.H / p.Hk, pairs = p.B * p.Hk;
-    const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
-    const int k_split = 8 / gcd8;
-    dim3 grid(pairs * k_split * ((n_mb + k_split - 1) / k_split) * G, CMP && KG == 2 ? p.splits : 1);
+    const dim3 grid(row_grid(p, BM), CMP && KG == 2 ? p.splits : 1);
     hipLaunchKernelGGL(kern, grid, dim3(64 * NW * KG), smem, stream, p);
     if ((e = hipGetLastError()) != hipSuccess || grid.y == 1) return e;
     return launch_merge<T>(p, stream);

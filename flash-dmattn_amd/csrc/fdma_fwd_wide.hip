@@ -84,23 +84,13 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = tid & 63, r = lane & 31, g = lane >> 5;
     const int rw = wave % RG, kg = wave / RG;  // 32-row group and key group of this wave
 
-    // workgroup -> (batch, head, query block): XCD-aware, heaviest query block first (see fwd_colmask_kernel)
-    const int n_mb = (p.Lq + BM - 1) / BM;
-    const int G = p.H / p.Hk, pairs = p.B * p.Hk;
-    const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
-    const int k_split = 8 / gcd8;
-    const int list_len = ((n_mb + k_split - 1) / k_split) * G;
-    const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-    const int vlist = xcd + 8 * (slot / list_len);
-    const int pos = slot % list_len;
-    const int pair = vlist / k_split;
-    const int mslot = (pos / G) * k_split + vlist % k_split;
-    if (mslot >= n_mb) return;
-    const int b = pair / p.Hk, hk = pair % p.Hk, h = hk * G + pos % G;
-    const int m0 = (n_mb - 1 - mslot) * BM;
+    const RowUnit ru = row_unit(p, blockIdx.x, BM);
+    if (ru.block < 0) return;
+    const int G = p.H / p.Hk;
+    const int b = ru.pair / p.Hk, hk = ru.pair % p.Hk, h = hk * G + (int)(blockIdx.x / 8) % G;
+    const int m0 = ru.block * BM;
     const SeqInfo sq = seq_info(p, b);
     const int LqS = sq.Lq, LkS = sq.Lk;
-    if (m0 >= LqS) return;
     const int shift = LkS - LqS;
     const int wrow0 = m0 + rw * 32, qrow = wrow0 + r;
 
@@ -496,10 +486,7 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, C::SMEM);
     if (e != hipSuccess) return e;
-    const int n_mb = (p.Lq + C::BM - 1) / C::BM, G = p.H / p.Hk, pairs = p.B * p.Hk;
-    const int gcd8 = (pairs % 8 == 0) ? 8 : ((pairs % 4 == 0) ? 4 : ((pairs % 2 == 0) ? 2 : 1));
-    const int k_split = 8 / gcd8;
-    hipLaunchKernelGGL(kern, dim3(pairs * k_split * ((n_mb + k_split - 1) / k_split) * G, CMP ? p.splits : 1), dim3(NT), C::SMEM, stream, p);
+    hipLaunchKernelGGL(kern, dim3(row_grid(p, C::BM), CMP ? p.splits : 1), dim3(NT), C::SMEM, stream, p);
     return hipGetLastError();
 }
 

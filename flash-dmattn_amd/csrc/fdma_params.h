@@ -205,6 +205,39 @@ __device__ inline SeqInfo seq_info(const FwdParams &p, int b) {
     return s;
 }
 
+// Workgroup -> (batch, kv head) pair and block of `bm` query rows, for the kernels that walk the keys of their rows (G workgroups per
+// block: the query heads of the group), heaviest block first.  The blocks of a pair are dealt to k lists, the lists go to the XCDs in
+// turn (a workgroup's XCD is its id % 8).  k is as small as it can be with all lists coming out even, which keeps a pair's K / V in few
+// L2s: over all pairs where they have one length, over the kv heads of an entry where the batch is ragged -- otherwise the XCD
+// that has the longest entry works alone.  The lists of a ragged entry go on where the blocks of those in front of it have ended.
+// Over all pairs / over the heads, forward (us): entries of 18, 256, 1774, 4, 2696, 73, 22, 2677 x 2/1 heads, d = 128 60.0 / 39.3; 1000,
+// 300, 500, 2000 x 8/2, d = 256 82 / 59; 4000, 100, 30, 200, 5, 60 x 8/2, d = 64 63.8 / 39.8; eight of 600 x 16/4, d = 256 57.9 / 62.1.
+__host__ __device__ inline int row_lists_per_pair(const FwdParams &p) {
+    const int n = p.cu_q ? p.Hk : p.B * p.Hk;
+    return n % 8 == 0 ? 1 : (n % 4 == 0 ? 2 : (n % 2 == 0 ? 4 : 8));
+}
+inline int row_grid(const FwdParams &p, int bm) {
+    const int k = row_lists_per_pair(p), n_mb = (p.Lq + bm - 1) / bm;
+    return p.B * p.Hk * k * ((n_mb + k - 1) / k) * (p.H / p.Hk);
+}
+struct RowUnit {
+    int pair, block;  // block < 0: none
+};
+__host__ __device__ inline RowUnit row_unit(const FwdParams &p, int id, int bm) {
+    const int k = row_lists_per_pair(p), G = p.H / p.Hk, n_mb = (p.Lq + bm - 1) / bm;
+    const int list_len = ((n_mb + k - 1) / k) * G;
+    const int slot = id / 8, vlist = id % 8 + 8 * (slot / list_len), pos = slot % list_len;
+    const int pair = vlist / k;
+    int blocks = n_mb, fold = vlist % k;  // of this pair; this list
+    if (p.cu_q) {
+        const int b = pair / p.Hk, q0 = p.cu_q[b], own = (p.cu_q[b + 1] - q0 + bm - 1) / bm;
+        blocks = own < n_mb ? own : n_mb;  // (rows beyond the longest length that the caller names are not computed)
+        fold = (fold - q0 / bm - b) & (k - 1);
+    }
+    const int rank = (pos / G) * k + fold;  // from the last block down
+    return {pair, rank < blocks ? blocks - 1 - rank : -1};
+}
+
 // Lists of units per (batch, kv head) pair, so that the lists of a ragged batch fill the 8 XCDs: the heads of ONE entry go to
 // all of them (8 entries with one kv head each would otherwise put an entry on each XCD, and the call takes as long as the
 // longest entry needs on 32 CUs).
