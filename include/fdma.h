@@ -258,7 +258,7 @@ typedef struct fdma_varlen_bwd_args {
     int32_t deterministic;
 } fdma_varlen_bwd_args;
 
-/* Forward / backward over a ragged batch.  No workspace is needed.  Every row of out / lse / dq / dk / dv that
+/* Forward / backward over a ragged batch.  No workspace is needed (fdma_varlen_bwd_ws can use one).  Every row of out / lse / dq / dk / dv that
  * belongs to a sequence is written exactly once. */
 int fdma_varlen_fwd(const fdma_varlen_fwd_args *args, void *hip_stream);
 int fdma_varlen_bwd(const fdma_varlen_bwd_args *args, void *hip_stream);
