@@ -140,7 +140,18 @@ template <bool CMP> __device__ __forceinline__ KvItem kv_item(const BwdParams &p
         const bool ragged = turns && f.cu_q;
         const int k = ragged ? ragged_lists_per_pair(f) : xcd_lists_per_pair(f.B * f.Hk), n_units = ragged ? p.kv_units : n_nb;
         XcdMap wm;
-        if (p.kv_most > 1) {
+        if (ragged) {
+            // All lists of an XCD side by side: the long entries of all its heads are under way before the short ones start.
+            // One list after the other / side by side, forward + backward (us): 4000, 3000, 700, 1 x 16/16 heads, d = 64 386 / 355;
+            // 900, 6000, 30 x 48/12, d = 64 1443 / 1332; six entries up to 4000 x 32/32, d = 128 1250 / 1207.  (Up to 8 lists: alike.)
+            // The last parts first, see below.
+            const int per_list = (n_units + k - 1) / k, nl = f.Hk * k / 8, at = (int)(blockIdx.x / 8), pos = at % (per_list * nl);
+            w.part = p.kv_most - 1 - at / (per_list * nl);
+            const int vlist = (int)(blockIdx.x % 8) + 8 * (pos % nl);
+            wm.pair = vlist / k;
+            wm.unit = pos / nl * k + vlist % k;
+            wm.valid = wm.unit < n_units;
+        } else if (p.kv_most > 1) {
             // A list holds its units once per part, the LAST parts first: those exist for the longest units only.  Workgroups
             // side by side go to the shader engines of an XCD in turn, whether they stay or return at once: with the parts of
             // a unit side by side instead, the engines that got the missing ones idled (ragged, 16384 tokens, two parts at

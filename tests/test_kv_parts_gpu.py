@@ -85,6 +85,8 @@ def test_column_form(B, Lq, Lk, H, Hk, D, Hb, causal, dtype, monkeypatch):
     ([300, 1, 700, 33], None, 4, 1, 256, True, torch.bfloat16),
     ([129, 500], [260, 90], 4, 2, 136, False, torch.float16),
     ([40] * 70 + [900], None, 2, 1, 128, True, torch.bfloat16),   # more entries than a wave has lanes
+    ([300, 1, 1500, 33], None, 64, 16, 64, True, torch.float16),     # two and three lists of units per XCD
+    ([33, 1500, 1, 300], [300, 1100, 129, 60], 48, 12, 128, False, torch.bfloat16),
 ])
 def test_ragged(lens_q, lens_k, H, Hk, D, causal, dtype, monkeypatch):
     from flash_sparse_attn import flash_sparse_attn_varlen_func
