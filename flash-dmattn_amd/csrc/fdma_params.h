@@ -226,7 +226,10 @@ struct RowUnit {
 __host__ __device__ inline RowUnit row_unit(const FwdParams &p, int id, int bm) {
     const int k = row_lists_per_pair(p), G = p.H / p.Hk, n_mb = (p.Lq + bm - 1) / bm;
     const int list_len = ((n_mb + k - 1) / k) * G;
-    const int slot = id / 8, vlist = id % 8 + 8 * (slot / list_len), pos = slot % list_len;
+    // Of a ragged batch an XCD's lists of one entry run side by side, heaviest blocks first (more than 8 kv heads; one after the other /
+    // side by side, forward: seven entries of 300 and one of 2000 x 12/12, d = 128 78 / 56; 2500 and 2500 x 24/12, d = 96 114 / 102).
+    const int side = p.cu_q ? p.Hk * k / 8 : 1, slot = id / 8, at = slot % (list_len * side) / G;
+    const int vlist = id % 8 + 8 * (slot / (list_len * side) * side + at % side), pos = at / side;
     const int pair = vlist / k;
     int blocks = n_mb, fold = vlist % k;  // of this pair; this list
     if (p.cu_q) {
@@ -234,7 +237,7 @@ __host__ __device__ inline RowUnit row_unit(const FwdParams &p, int id, int bm) 
         blocks = own < n_mb ? own : n_mb;  // (rows beyond the longest length that the caller names are not computed)
         fold = (fold - q0 / bm - b) & (k - 1);
     }
-    const int rank = (pos / G) * k + fold;  // from the last block down
+    const int rank = pos * k + fold;  // from the last block down
     return {pair, rank < blocks ? blocks - 1 - rank : -1};
 }
 
