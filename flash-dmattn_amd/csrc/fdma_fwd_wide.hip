@@ -377,9 +377,11 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
             }
         }
         publish();
-        if constexpr (ONE) {  // ... and everybody has read this V tile
+        if constexpr (ONE) {  // ... and everybody has read this V tile (past the last tile nothing is fetched: the merge is next)
+            if (jn < n_end) {
 #pragma unroll
-            for (int n = NP; n < 2 * NP; n++) dma_piece(n);
+                for (int n = NP; n < 2 * NP; n++) dma_piece(n);
+            }
         }
         jc = jn;
         jn = next_active(jn + 1);
@@ -391,6 +393,10 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     }
 
     // ---- merge of the key groups: wave (rw, kg) finishes units kg UPW .. + UPW - 1 of its rows, the others hand theirs over
+    // (no direct load may be in flight here: it would land in the sums and shares of O that the merge puts where the tiles were.  The
+    // compiler does not know of loads issued in assembly, and __syncthreads() does not wait for them.  None is in flight, so the
+    // wait is free.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     float total = xhalf_sum(row_sum);
     float *xs = (float *)(smem + C::OFF_SUMS) + lane;
