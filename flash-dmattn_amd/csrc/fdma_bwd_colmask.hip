@@ -1324,7 +1324,8 @@ bool bwd_colmask_applicable(const BwdParams &p) {
 // Whole where there are 2.5 units per CU (16384 ragged tokens x 32/8: 1175 whole, 1258 to 1286 in parts of 96 to 140 steps), and, from
 // half a unit per CU on, where the longest is not two and a half parts (1 x 700 x 32/32: 36.5 whole, 39 to 42 cut; d = 64,
 // 2 x 1000 x 16/16: 35.6 and 41 to 49).  Whole up to 20 steps: 25 us at most, and the call is bound by the host, to which a launch
-// more is 2.5 us (256 x 2/1, d = 64, forward and backward: 72.8 whole, 75.5 cut).  At most 16 parts, and 2048 places for sums (256 MB at d = 128).
+// more is 2.5 us (256 x 2/1, d = 64, forward and backward: 72.8 whole, 75.5 cut).  At most 16 parts, and 2048 places for sums: up to 128 / 256 / 512 MB
+// at d = 64 / 128 / 256, which callers offer where they have it.
 size_t plan_kv_parts(BwdParams &p, size_t *db_bytes) {
     const FwdParams &f = p.f;
     p.kv_most = 1;

@@ -20,6 +20,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/util/Exception.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -64,6 +65,18 @@ void check(int rc) { TORCH_CHECK(rc == FDMA_OK, api.last_error()); }
 
 inline size_t up256(size_t x) { return (x + 255) / 256 * 256; }
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
+
+// Scratch of `need` bytes and, where the device has that much left, of `room` more, which the call can do without (then 0).
+Tensor scratch_with_room(size_t need, size_t &room, const at::TensorOptions &opt) {
+    if (room) {
+        try {
+            return at::empty({(int64_t)(need + room)}, opt.dtype(at::kByte));
+        } catch (const c10::OutOfMemoryError &) {
+            room = 0;
+        }
+    }
+    return need ? at::empty({(int64_t)need}, opt.dtype(at::kByte)) : Tensor();
+}
 
 // ---- arguments -----------------------------------------------------------------------------------------------------
 
@@ -270,12 +283,13 @@ struct AttentionBackward : public Node {
             a.fwd_workspace_bytes = ws_bytes;
         }
         const size_t d_bytes = up256((size_t)q.size(0) * q.size(2) * round_up(q.size(1), 128) * 4);
-        const size_t need = api.bwd_workspace_bytes(&a) + api.bwd_optional_bytes(&a);
-        Tensor scratch = at::empty({(int64_t)(d_bytes + need)}, opt.dtype(at::kByte));
+        const size_t need = api.bwd_workspace_bytes(&a);
+        size_t room = api.bwd_optional_bytes(&a);
+        Tensor scratch = scratch_with_room(d_bytes + need, room, opt);
         a.softmax_d = (float *)scratch.data_ptr();
-        if (need) {
+        if (need + room) {
             a.workspace = (char *)scratch.data_ptr() + d_bytes;
-            a.workspace_bytes = need;
+            a.workspace_bytes = need + room;
         }
         check(api.bwd(&a, stream_of(q.get_device())));
         if (has_bias) return {std::move(dq), std::move(dk), std::move(dv), std::move(dbias)};
@@ -440,9 +454,8 @@ struct VarlenBackward : public Node {
         for (int i = 0; i < 4; i++) { dst[i][0] = src[i]->stride(0); dst[i][1] = src[i]->stride(1); }
         a.softmax_d = (float *)softmax_d.data_ptr();
         a.deterministic = deterministic;
-        const size_t room = api.varlen_bwd_optional_bytes(&a);
-        Tensor scratch;
-        if (room) scratch = at::empty({(int64_t)room}, opt.dtype(at::kByte));
+        size_t room = api.varlen_bwd_optional_bytes(&a);
+        const Tensor scratch = scratch_with_room(0, room, opt);
         check(api.varlen_bwd_ws(&a, room ? scratch.data_ptr() : nullptr, room, stream_of(q.get_device())));
         return {std::move(dq), std::move(dk), std::move(dv)};
     }

@@ -213,6 +213,16 @@ def _decode_buffers(device: torch.device, stream: int, nbytes: int, cbytes: int)
     return ws, counters
 
 
+def _scratch_with_room(need: int, room: int, device: torch.device) -> Optional[torch.Tensor]:
+    """Scratch of `need` bytes and, where the device has that much left, of `room` more, which the call can do without."""
+    if room:
+        try:
+            return torch.empty(need + room, dtype=torch.uint8, device=device)
+        except torch.cuda.OutOfMemoryError:
+            pass
+    return torch.empty(need, dtype=torch.uint8, device=device) if need else None
+
+
 def _flash_sparse_attn_forward_body(
     q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[torch.Tensor], bias: Optional[torch.Tensor],
     softmax_scale: float, is_causal: bool, softcap: float, return_softmax: bool,
@@ -417,11 +427,9 @@ def _flash_sparse_attn_backward_body(
     args.softmax_d = softmax_d.data_ptr()
     args.deterministic = int(bool(deterministic))
     with _cabi.device_guard(q.device):
-        nbytes = _cabi.lib.fdma_bwd_workspace_bytes(args) + _cabi.lib.fdma_bwd_optional_bytes(args)
-        workspace = None
-        if nbytes:
-            workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-            args.workspace, args.workspace_bytes = workspace.data_ptr(), nbytes
+        workspace = _scratch_with_room(_cabi.lib.fdma_bwd_workspace_bytes(args), _cabi.lib.fdma_bwd_optional_bytes(args), q.device)
+        if workspace is not None:
+            args.workspace, args.workspace_bytes = workspace.data_ptr(), workspace.numel()
         else:
             args.workspace, args.workspace_bytes = None, 0
         if seqlen_q > 0:
@@ -799,10 +807,10 @@ def _flash_sparse_attn_varlen_backward_body(
     args.dv_strides[:] = (dv_w.stride(0), dv_w.stride(1))
     args.softmax_d = softmax_d.data_ptr()
     args.deterministic = int(bool(deterministic))
-    nbytes = _cabi.lib.fdma_varlen_bwd_optional_bytes(args)
-    workspace = torch.empty(nbytes, device=q.device, dtype=torch.uint8) if nbytes else None
     with _cabi.device_guard(q.device):
-        _cabi.check(_cabi.lib.fdma_varlen_bwd_ws(args, workspace.data_ptr() if nbytes else None, nbytes, _cabi.current_stream(q.device)))
+        workspace = _scratch_with_room(0, _cabi.lib.fdma_varlen_bwd_optional_bytes(args), q.device)
+        at, nbytes = (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel())
+        _cabi.check(_cabi.lib.fdma_varlen_bwd_ws(args, at, nbytes, _cabi.current_stream(q.device)))
     for given, work in ((dq, dq_w), (dk, dk_w), (dv, dv_w)):
         if given is not None and work is not given:
             given.copy_(work)

@@ -216,7 +216,7 @@ size_t fdma_fwd_counter_bytes(const fdma_fwd_args *args);
 size_t fdma_bwd_workspace_bytes(const fdma_bwd_args *args);
 /* Further scratch that a backward call can use (0: none): with workspace_bytes of at least fdma_bwd_workspace_bytes() plus this
  * many, key blocks that many queries see are cut into parts, whose fp32 sums lie there; with less they stay whole, and the call
- * takes longer where the chip is not full. */
+ * takes longer where the chip is not full.  Up to 512 MB and the parts' dBias columns: a caller that is short of memory leaves it out. */
 size_t fdma_bwd_optional_bytes(const fdma_bwd_args *args);
 
 /* Argument validation only (no GPU work, callable on a host without a device). */

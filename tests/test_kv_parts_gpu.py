@@ -142,3 +142,41 @@ def test_compacted_above_128(B, Lq, Lk, H, Hk, D, Hb, causal, dtype):
     out = flash_sparse_attn_func(*leaves[:3], mask, leaves[3] if Hb else None, None, causal)
     for got, want, name in zip(torch.autograd.grad(out, leaves, dout), ref[1:], ("dq", "dk", "dv", "dbias")):
         assert_grad_close(got, want, name)
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("ragged", [True, False])
+def test_no_memory_for_parts(ragged, native, monkeypatch):
+    """The room for parts is optional: a backward that the device has no such room for runs with whole blocks."""
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func, flash_sparse_attn_varlen_func
+
+    _cabi.set_compact_mode(_cabi.COMPACT_NEVER)
+    if not native:
+        monkeypatch.setattr(_cabi, "host", _cabi._NoHost)
+    L, H, Hk, D = 4096, 8, 2, 128
+    g = torch.Generator(device=DEV).manual_seed(7)
+    q = torch.randn(1, L, H, D, generator=g, device=DEV).bfloat16().requires_grad_(True)
+    k, v = [torch.randn(1, L, Hk, D, generator=g, device=DEV).bfloat16().requires_grad_(True) for _ in range(2)]
+    dout = torch.randn(1, L, H, D, generator=g, device=DEV).bfloat16()
+    cu = torch.tensor([0, L], dtype=torch.int32, device=DEV)
+
+    def grads():
+        out = flash_sparse_attn_varlen_func(q[0], k[0], v[0], cu, cu, L, L, is_causal=True) if ragged else flash_sparse_attn_func(q, k, v, is_causal=True)
+        return torch.autograd.grad(out, (q, k, v), dout[0] if ragged else dout)
+
+    def peak():
+        torch.cuda.empty_cache()
+        torch.cuda.reset_peak_memory_stats()
+        got = grads()
+        return got, torch.cuda.max_memory_reserved()
+
+    parts, most = peak()
+    kept, held = 64 << 20, torch.cuda.memory_allocated()  # outputs, gradients, D and the forward's: 8 + 8 + 4 + 20 MB and the allocator's pieces
+    assert most > held + 2 * kept  # (or this is no such call)
+    try:
+        torch.cuda.empty_cache()
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + kept) / torch.cuda.get_device_properties(0).total_memory)
+        whole = grads()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    _close(parts, whole, ("dq", "dk", "dv"))
