@@ -168,21 +168,6 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
         if (ne < n_end) n_end = ne;
     }
 
-    // SPLIT_KEYS: this workgroup's share [t_first, n_end) of the tiles (see fwd_key_splits)
-    constexpr bool SPLIT_KEYS = CMP && KG == 2;
-    int t_first = 0;
-    if (SPLIT_KEYS && p.splits > 1) {
-        // (no share under eight tiles: the shares that are then left over only say so)
-        const int y = (int)blockIdx.y, most = n_end / 8 > 1 ? n_end / 8 : 1, shares = p.splits < most ? p.splits : most;
-        if (y >= shares) {
-            const int row = m0 + (int)threadIdx.x;
-            if ((int)threadIdx.x < BM && row < LqS) p.lse_part[(((int64_t)y * p.B + b) * p.H + h) * p.Lq + row] = -INFINITY;
-            return;
-        }
-        t_first = n_end * y / shares;
-        n_end = n_end * (y + 1) / shares;
-    }
-
     // ---- active-tile bitmap
     for (int base = 0; !CMP && base < n_end; base += NTHREADS) {
         const int j = base + tid;
@@ -223,7 +208,7 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
     // tells the compiler that the value is wave-uniform, so tile numbers, loop conditions and load addresses stay in
     // scalar registers).  Compacted keys have no bitmap: every tile up to n_end is active.
     uint32_t it_word = 0;
-    int it_base = -32, it_next = t_first;
+    int it_base = -32, it_next = 0;
     auto next_tile = [&]() -> int {
         if (CMP) {
             const int j = it_next < n_end ? it_next : n_end;
@@ -719,7 +704,7 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
             for (int i = 0; i < 16; i++) o[db][i] = 0.f;
         it_word = 0;
         it_base = -32;
-        it_next = t_first;
+        it_next = 0;
         for (Turn j = next_turn(); j.lead < n_end; j = next_turn()) {
             set_tile_k(j);
             set_tile_v(j);
@@ -780,23 +765,6 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
                 }
         }
         const float inv = total > 0.f ? 1.f / total : 0.f;
-        if (SPLIT_KEYS && p.splits > 1) {  // this share's O in fp32 and its log2-sum-exp; fwd_merge_kernel adds the shares up
-            if (qrow < LqS) {
-                const int64_t row = (((int64_t)blockIdx.y * p.B + b) * p.H + h) * p.Lq + qrow;
-                float *op = p.o_part + row * p.d;
-#pragma unroll
-                for (int db = 0; db < DB; db++)
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        const int c = 32 * db + 16 * (q >> 1) + 8 * g + 4 * (q & 1);
-                        if (c < p.d)
-                            *(f32x4_t *)(op + c) = f32x4_t{o[db][4 * q] * inv, o[db][4 * q + 1] * inv, o[db][4 * q + 2] * inv, o[db][4 * q + 3] * inv};
-                    }
-                // (a sum that is no number has to reach the result: only an empty share is left out)
-                if (g == 0) p.lse_part[row] = total == 0.f ? -INFINITY : row_ref + __builtin_amdgcn_logf(total);
-            }
-            return;
-        }
         if (qrow < LqS) {
             uint16_t *op = (uint16_t *)p.o + b * p.o_b + (sq.q0 + qrow) * p.o_r + h * p.o_h;
 #pragma unroll
@@ -883,10 +851,8 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
-    const dim3 grid(row_grid(p, BM), CMP && KG == 2 ? p.splits : 1);
-    hipLaunchKernelGGL(kern, grid, dim3(64 * NW * KG), smem, stream, p);
-    if ((e = hipGetLastError()) != hipSuccess || grid.y == 1) return e;
-    return launch_merge<T>(p, stream);
+    hipLaunchKernelGGL(kern, dim3(row_grid(p, BM)), dim3(64 * NW * KG), smem, stream, p);
+    return hipGetLastError();
 }
 
 template <typename T, int D>
@@ -961,7 +927,7 @@ hipError_t launch_fwd_colmask(const FwdParams &p, int dtype, hipStream_t stream)
     if (p.cmp.on && p.cmp.img_kv) return launch_fwd_stream(p, dtype, stream);  // (the pre-pass has written tile images)
     // head dims up to 64 / 128 (a head dim in between runs in the next larger instantiation), above in a kernel of their own
     if (p.d > 128) return launch_fwd_wide(p, dtype, stream);
-    if (takes_key_groups(p)) {
+    if (takes_key_groups(p)) {  // (and all calls in shares: three shares are at most a third of a 64-row block per CU, see key_shares)
         const hipError_t e = launch_fwd_wide(p, dtype, stream);
         if (e != hipSuccess || !p.cmp.on || p.splits <= 1) return e;
         return dtype == 0 ? launch_merge<bf16_tag>(p, stream) : launch_merge<fp16_tag>(p, stream);

@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     using C = Cfg<D, RG>;
     constexpr int KG = C::KG, BM = C::BM, BN = C::BN, ROW = C::ROW, TILE = C::TILE, NP = C::NP, KS = D / 16, DB = D / 32;
     constexpr int OFF_V = C::OFF_V, OFF_COL = C::OFF_COL, OFF_BITS = C::OFF_BITS, UPW = C::UPW, UPP = C::UPP;
-    constexpr bool ONE = C::ONE;
+    constexpr bool ONE = C::ONE, SHARES = CMP && D <= 128;  // (key_shares cuts nothing above)
     extern __shared__ __attribute__((aligned(256))) char smem[];
     const uint32_t lds0 = lds_addr(smem);  // (a multiple of 256)
     uint32_t *sBits = (uint32_t *)(smem + OFF_BITS);
@@ -133,7 +133,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     }
     // this workgroup's share of the tiles (see fwd_key_splits)
     int t_first = 0;
-    if (CMP && p.splits > 1) {
+    if (SHARES && p.splits > 1) {
         // (no share under 512 keys: the shares that are then left over only say so)
         const int y = (int)blockIdx.y, most = n_end * BN / 512 > 1 ? n_end * BN / 512 : 1, shares = p.splits < most ? p.splits : most;
         if (y >= shares) {
@@ -436,7 +436,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     }
     const bool row_ok = qrow < LqS;
     const float inv = total > 0.f ? 1.f / total : 0.f;
-    const bool share = CMP && p.splits > 1;  // this share's O in fp32 and its log2-sum-exp; fwd_merge_kernel adds the shares up
+    const bool share = SHARES && p.splits > 1;  // this share's O in fp32 and its log2-sum-exp; fwd_merge_kernel adds the shares up
     const int64_t prow_at = (((int64_t)blockIdx.y * p.B + b) * p.H + h) * p.Lq + qrow;
     uint16_t *op = (uint16_t *)p.o + b * p.o_b + (sq.q0 + qrow) * p.o_r + h * p.o_h;
 #pragma unroll
@@ -492,7 +492,7 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, C::SMEM);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(row_grid(p, C::BM), CMP ? p.splits : 1), dim3(NT), C::SMEM, stream, p);
+    hipLaunchKernelGGL(kern, dim3(row_grid(p, C::BM), CMP && D <= 128 ? p.splits : 1), dim3(NT), C::SMEM, stream, p);
     return hipGetLastError();
 }
 
