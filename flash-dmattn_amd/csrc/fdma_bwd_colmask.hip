@@ -1297,10 +1297,10 @@ hipError_t launch_dq_grid(const BwdParams &p, int grid, hipStream_t stream) {
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
     const FwdParams &f = p.f;
-    const int n_dq = row_grid(f, Q_BM);  // a multiple of 8
-    if (!f.cmp.on) return launch_dq_grid<T, D, CAUSAL>(p, n_dq, stream);
-    const int units_max = f.B * f.Hk * ((f.Lk + KV_BN - 1) / KV_BN);
     BwdParams pr = p;
+    const int n_dq = row_grid(pr.f, Q_BM);  // a multiple of 8
+    if (!f.cmp.on) return launch_dq_grid<T, D, CAUSAL>(pr, n_dq, stream);
+    const int units_max = f.B * f.Hk * ((f.Lk + KV_BN - 1) / KV_BN);
     place_reduction(pr, n_dq, units_max * (D / 16));
     return launch_dq_grid<T, D, CAUSAL>(pr, n_dq + pr.red_count, stream);
 }

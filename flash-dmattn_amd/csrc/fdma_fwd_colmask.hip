@@ -851,7 +851,9 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(row_grid(p, BM)), dim3(64 * NW * KG), smem, stream, p);
+    FwdParams pr = p;
+    const int grid = row_grid(pr, BM);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW * KG), smem, stream, pr);
     return hipGetLastError();
 }
 

@@ -492,7 +492,9 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, C::SMEM);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(row_grid(p, C::BM), CMP && D <= 128 ? p.splits : 1), dim3(NT), C::SMEM, stream, p);
+    FwdParams pr = p;
+    const int grid = row_grid(pr, C::BM);
+    hipLaunchKernelGGL(kern, dim3(grid, CMP && D <= 128 ? p.splits : 1), dim3(NT), C::SMEM, stream, pr);
     return hipGetLastError();
 }
 

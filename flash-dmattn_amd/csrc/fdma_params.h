@@ -178,6 +178,7 @@ struct FwdParams {
     // broadcast like the mask
     const uint8_t *mbits;
     int64_t mb_b, mb_h, mb_r;
+    int32_t row_lists;  // log2 of the lists that the row blocks of a pair are dealt to, -1: whole ragged entries (set by row_grid)
 };
 
 // the caller's kv head behind head `hk` of the compaction layer (see FwdParams::kv_share)
@@ -212,32 +213,42 @@ __device__ inline SeqInfo seq_info(const FwdParams &p, int b) {
 // that has the longest entry works alone.  The lists of a ragged entry go on where the blocks of those in front of it have ended.
 // Over all pairs / over the heads, forward (us): entries of 18, 256, 1774, 4, 2696, 73, 22, 2677 x 2/1 heads, d = 128 60.0 / 39.3; 1000,
 // 300, 500, 2000 x 8/2, d = 256 82 / 59; 4000, 100, 30, 200, 5, 60 x 8/2, d = 64 63.8 / 39.8; eight of 600 x 16/4, d = 256 57.9 / 62.1.
-__host__ __device__ inline int row_lists_per_pair(const FwdParams &p) {
-    const int n = p.cu_q ? p.Hk : p.B * p.Hk;
-    return n % 8 == 0 ? 1 : (n % 4 == 0 ? 2 : (n % 2 == 0 ? 4 : 8));
-}
-inline int row_grid(const FwdParams &p, int bm) {
-    const int k = row_lists_per_pair(p), n_mb = (p.Lq + bm - 1) / bm;
-    return p.B * p.Hk * k * ((n_mb + k - 1) / k) * (p.H / p.Hk);
+// Where the longest entry has fewer blocks than there are lists, most lists of an entry would be empty, and a workgroup without a block
+// holds its place on a CU until it has seen that: whole entries go to the XCDs in turn there, eight pairs a turn, each turn from the
+// next XCD on.  Lists of every entry / whole entries, forward (us): 64 entries of 60 to 128 rows x 8/1 heads, d = 128 41 / 22, d = 64 20.2 /
+// 10.4; 256 of 64 x 16/2 178 / 129; 33 of 100 x 6/3, d = 96 14.2 / 9.8; 13 of 300 to 700 x 12/3 33.6 / 29.8.  (Whole entries up to 32
+// workgroups each in batches of eight times the longest: 8 of 600 x 16/4 36.3 / 32.0, 16 of 2000 x 8/2 181 / 160, but 9 of 900 x 16/16 71 /
+// 86, 200 of 20 to 400 x 8/4 137 / 165, 20 of 100 to 600 x 16/4, d = 256 78 / 88.)
+inline int row_grid(FwdParams &p, int bm) {
+    const int n = p.cu_q ? p.Hk : p.B * p.Hk, n_mb = (p.Lq + bm - 1) / bm;
+    const int log_k = n % 8 == 0 ? 0 : (n % 4 == 0 ? 1 : (n % 2 == 0 ? 2 : 3)), k = 1 << log_k;
+    const bool whole = p.cu_q && n_mb < k;
+    p.row_lists = whole ? -1 : log_k;
+    return (whole ? (p.B * p.Hk + 7) / 8 * 8 * n_mb : p.B * p.Hk * k * ((n_mb + k - 1) / k)) * (p.H / p.Hk);
 }
 struct RowUnit {
     int pair, block;  // block < 0: none
 };
 __host__ __device__ inline RowUnit row_unit(const FwdParams &p, int id, int bm) {
-    const int k = row_lists_per_pair(p), G = p.H / p.Hk, n_mb = (p.Lq + bm - 1) / bm;
-    const int list_len = ((n_mb + k - 1) / k) * G;
+    const bool whole = p.row_lists < 0;
+    const int log_k = whole ? 0 : p.row_lists, k = 1 << log_k, G = p.H / p.Hk, n_mb = (p.Lq + bm - 1) / bm;
+    const int list_len = ((n_mb + k - 1) >> log_k) * G;
     // Of a ragged batch an XCD's lists of one entry run side by side, heaviest blocks first (more than 8 kv heads; one after the other /
     // side by side, forward: seven entries of 300 and one of 2000 x 12/12, d = 128 78 / 56; 2500 and 2500 x 24/12, d = 96 114 / 102).
-    const int side = p.cu_q ? p.Hk * k / 8 : 1, slot = id / 8, at = slot % (list_len * side) / G;
+    const int side = p.cu_q && !whole ? (p.Hk << log_k) / 8 : 1, slot = id / 8, at = slot % (list_len * side) / G;
     const int vlist = id % 8 + 8 * (slot / (list_len * side) * side + at % side), pos = at / side;
-    const int pair = vlist / k;
-    int blocks = n_mb, fold = vlist % k;  // of this pair; this list
+    int pair = vlist >> log_k;
+    if (whole) {
+        pair = (pair & ~7) | ((pair - (pair >> 3)) & 7);
+        if (pair >= p.B * p.Hk) return {0, -1};
+    }
+    int blocks = n_mb, fold = vlist & (k - 1);  // of this pair; this list
     if (p.cu_q) {
         const int b = pair / p.Hk, q0 = p.cu_q[b], own = (p.cu_q[b + 1] - q0 + bm - 1) / bm;
         blocks = own < n_mb ? own : n_mb;  // (rows beyond the longest length that the caller names are not computed)
         fold = (fold - q0 / bm - b) & (k - 1);
     }
-    const int rank = pos * k + fold;  // from the last block down
+    const int rank = (pos << log_k) + fold;  // from the last block down
     return {pair, rank < blocks ? blocks - 1 - rank : -1};
 }
 

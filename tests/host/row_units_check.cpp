@@ -1,0 +1,64 @@
+// Host-side check of the mapping from workgroups to blocks of query rows (row_grid / row_unit in flash-dmattn_amd/csrc/fdma_params.h, built and
+// run by tests/test_row_units.py with g++), over random batches of one length and ragged ones: every block of rows that a
+// call computes has exactly one workgroup per query head, no other workgroup names one, a launch is made of whole turns over the 8 XCDs,
+// and rounding the blocks of the longest entry up to its lists no more than doubles it.
+#include <cstdio>
+#include <cstring>
+#include <vector>
+
+#include "fdma_params.h"
+
+using namespace fdma;
+
+int main() {
+    unsigned rng = 1u;
+    auto next = [&]() { rng = rng * 1664525u + 1013904223u; return (int)(rng >> 8); };
+    long long checked = 0, whole = 0;
+    for (int rep = 0; rep < 12000; rep++) {
+        FwdParams p;
+        std::memset(&p, 0, sizeof(p));
+        const int G = 1 + next() % 4, bm = (next() & 1) ? 64 : ((next() & 1) ? 128 : 256), longest = 1 + next() % ((next() & 1) ? 3000 : 300);
+        p.Hk = 1 + next() % 34;
+        p.H = p.Hk * G;
+        p.B = 1 + next() % ((next() & 1) ? 12 : 70);
+        std::vector<int> cu(p.B + 1, 0);
+        int most = 1;
+        for (int b = 0; b < p.B; b++) {
+            const int n = next() % 4 == 0 ? 0 : next() % (longest + 1);
+            cu[b + 1] = cu[b] + n;
+            most = n > most ? n : most;
+        }
+        const bool ragged = next() % 3 != 0;
+        p.Lq = ragged ? (next() % 8 ? most : 1 + next() % most) : longest;  // (a caller may name less than the longest: the rest is not computed)
+        if (ragged) p.cu_q = cu.data();
+        p.total_q = cu[p.B];
+        const int n_mb = (p.Lq + bm - 1) / bm, grid = row_grid(p, bm), all = p.B * p.Hk * n_mb * G;
+        whole += p.row_lists < 0;
+        if (grid % 8 || grid > 2 * all + 8 * n_mb * G + (ragged ? 0 : 8 * p.B * p.Hk * G)) {
+            std::printf("FAILED: %d workgroups for B %d Hk %d G %d blocks %d ragged %d\n", grid, p.B, p.Hk, G, n_mb, ragged);
+            return 1;
+        }
+        std::vector<int> seen((size_t)p.B * p.H * n_mb, 0);
+        for (int id = 0; id < grid; id++) {
+            const RowUnit u = row_unit(p, id, bm);
+            if (u.block < 0) continue;
+            if (u.pair < 0 || u.pair >= p.B * p.Hk || u.block >= n_mb) {
+                std::printf("FAILED: workgroup %d has block %d of pair %d\n", id, u.block, u.pair);
+                return 1;
+            }
+            seen[((size_t)(u.pair / p.Hk) * p.H + u.pair % p.Hk * G + (id / 8) % G) * n_mb + u.block]++;
+        }
+        for (int b = 0; b < p.B; b++)
+            for (int i = 0; i < p.H * n_mb; i++) {
+                const int want = i % n_mb * bm < (ragged ? cu[b + 1] - cu[b] : p.Lq) ? 1 : 0;
+                if (seen[(size_t)b * p.H * n_mb + i] != want) {
+                    std::printf("FAILED: B %d Hk %d G %d ragged %d: entry %d, head %d, block %d has %d workgroups\n", p.B, p.Hk, G, ragged, b, i / n_mb, i % n_mb,
+                                seen[(size_t)b * p.H * n_mb + i]);
+                    return 1;
+                }
+            }
+        checked += grid;
+    }
+    std::printf("%s (%lld workgroups, %lld batches of whole entries)\n", whole > 100 ? "OK" : "FAILED", checked, whole);
+    return whole > 100 ? 0 : 1;
+}

@@ -158,6 +158,17 @@ def test_varlen_order_of_entries(lens, H, Hk, D):
     _run(lens, lens[::-1], H, Hk, D, False, seed=len(lens) + 1)
 
 
+@pytest.mark.parametrize("lens,H,Hk", [
+    ([100, 64, 0, 128, 77, 1, 33, 90, 128], 6, 3),           # 27 pairs: the last turn over the XCDs lacks five
+    ([128] * 8, 4, 1),                                       # one full turn
+    ([65, 200], 12, 2),                                      # two blocks of 128 rows, four of 64
+])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_varlen_entries_of_fewer_blocks_than_lists(lens, H, Hk, D):
+    """Row blocks of short entries: whole entries go to the XCDs in turn."""
+    _run(lens, lens, H, Hk, D, True, seed=len(lens) + D)
+
+
 def test_varlen_rejects_unsupported_arguments():
     f = _op()
     q, k, v, _ = _make([64], [64], 2, 2, 64, torch.bfloat16, 0)
