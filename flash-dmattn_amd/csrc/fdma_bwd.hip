@@ -77,7 +77,7 @@ template <typename T> struct NegInfPair;
 template <> struct NegInfPair<bf16_tag> { static constexpr uint32_t value = 0xFF80FF80u; };
 template <> struct NegInfPair<fp16_tag> { static constexpr uint32_t value = 0xFC00FC00u; };
 
-template <typename T, int D, bool CAUSAL, bool GSUM>
+template <typename T, int D, bool CAUSAL, bool GSUM, bool ODD>
 __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv_kernel(const BwdParams p) {
     using E = Elem<T>;
     using SM = KvSmem<D, GSUM>;
@@ -209,7 +209,7 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
         const int hb = has_bias ? (f.Hb == f.H ? h : (f.Hb == 1 ? 0 : hk)) : 0;
         const int kk = n0 + 8 * bc;
         const int kk_c = kk < f.Lk ? kk : 0;
-        const int at = chunk8_at<true>(kk, f.Lk);
+        const int at = chunk8_at<ODD>(kk, f.Lk);
         const int64_t moff = f.mask ? b * f.m_b + hm * f.m_h + at : 0;
         const int64_t boff = has_bias ? b * f.bi_b + hb * f.bi_h + at : 0;
 #pragma unroll
@@ -241,8 +241,8 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
         const int kk = n0 + 8 * bc;
 #pragma unroll
         for (int it = 0; it < FB_IT; it++) {
-            u32x4_t bv = has_bias ? chunk8_fix<true>(braw[it], kk, f.Lk) : u32x4_t{0, 0, 0, 0};
-            u32x2_t mv = f.mask ? (f.mbits ? mask_bits_to_bytes(mask_bits_byte(mraw[it], kk < f.Lk ? kk : 0)) : chunk8_fix_mask<true>(mraw[it], kk, f.Lk))
+            u32x4_t bv = has_bias ? chunk8_fix<ODD>(braw[it], kk, f.Lk) : u32x4_t{0, 0, 0, 0};
+            u32x2_t mv = f.mask ? (f.mbits ? mask_bits_to_bytes(mask_bits_byte(mraw[it], kk < f.Lk ? kk : 0)) : chunk8_fix_mask<ODD>(mraw[it], kk, f.Lk))
                                 : u32x2_t{0x01010101u, 0x01010101u};
             uint64_t keepm = kk < f.Lk ? ~0ull : 0ull;
             if (kk + 8 > f.Lk && kk < f.Lk) keepm = (1ull << (8 * (f.Lk - kk))) - 1ull;  // chunk straddles the end of the keys
@@ -638,8 +638,16 @@ hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
             e = launch_bwd_dkdv_wide(p, dtype_code, gsum, stream);
         } else {
             if (D == 64 && bwd_dkdv_64_applicable(p)) e = launch_bwd_dkdv_64(p, dtype_code, stream);
-            else if (gsum) e = f.causal ? launch(bwd_dkdv_kernel<T, D, true, true>, KvSmem<D, true>::TOTAL) : launch(bwd_dkdv_kernel<T, D, false, true>, KvSmem<D, true>::TOTAL);
-            else e = f.causal ? launch(bwd_dkdv_kernel<T, D, true, false>, KvSmem<D, false>::TOTAL) : launch(bwd_dkdv_kernel<T, D, false, false>, KvSmem<D, false>::TOTAL);
+            else {
+                // (whole aligned chunks / rows read where they lie, d = 64, forward and backward, us: 3000 tokens x 8/8 heads 301 / 330, 2056 x
+                // 16/16, causal 220 / 225, 1000 x 8/2 without a bias 105 / 106)
+                auto pick = [&](auto odd) -> hipError_t {
+                    constexpr bool O = decltype(odd)::value;
+                    if (gsum) return f.causal ? launch(bwd_dkdv_kernel<T, D, true, true, O>, KvSmem<D, true>::TOTAL) : launch(bwd_dkdv_kernel<T, D, false, true, O>, KvSmem<D, true>::TOTAL);
+                    return f.causal ? launch(bwd_dkdv_kernel<T, D, true, false, O>, KvSmem<D, false>::TOTAL) : launch(bwd_dkdv_kernel<T, D, false, false, O>, KvSmem<D, false>::TOTAL);
+                };
+                e = D > 128 || odd_rows(f) ? pick(std::true_type()) : pick(std::bool_constant<(D > 128)>());
+            }
         }
         if (e != hipSuccess) return e;
         if (p.kv_segs > 1) {

@@ -553,10 +553,12 @@ hipError_t launch_fwd_o(const FwdParams &p, hipStream_t stream) {
 template <typename T, int D, bool CAUSAL, int NW, int KSPLIT = 1>
 hipError_t launch_fwd_c(const FwdParams &p, hipStream_t stream) {
     const int gh = shared_rows(p);
+    // (at d = 65 .. 128 whole aligned chunks / rows read where they lie, us: 2000 tokens x 16/8 heads 54.7 / 56.4, x 16/4 52.9 / 53.7,
+    // 1024 x 16/8, causal 30.9 / 31.6)
     auto pick = [&](auto odd) -> hipError_t {
         constexpr bool O = decltype(odd)::value;
-        if constexpr (D <= 128) if (gh == 4) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, 4, (D > 64) || O>(p, stream);
-        if constexpr (D > 64) if (gh == 2) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, 2, true>(p, stream);
+        if constexpr (D <= 128) if (gh == 4) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, 4, O>(p, stream);
+        if constexpr (D > 64) if (gh == 2) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, 2, O>(p, stream);
         return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, 1, O>(p, stream);
     };
     if (D > 128 || odd_rows(p)) return pick(std::true_type());

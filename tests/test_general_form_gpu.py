@@ -68,3 +68,44 @@ def test_general_form_vs_oracle(case, dtype):
     for i, (a, b) in enumerate(zip(*runs)):  # odd rows and padded rows: other kernels, the same arithmetic
         if not (atomics and i == 4):
             assert torch.equal(a, b), ("out", "dq", "dk", "dv", "dbias")[i]
+
+
+def _off_by_one(t):
+    """The same values as a view whose rows start an element behind 16-byte boundaries, a row apart like whole chunks."""
+    big = torch.full((*t.shape[:-1], t.shape[-1] + 16), True if t.dtype == torch.bool else float("nan"), dtype=t.dtype, device=t.device)
+    big[..., 1:t.shape[-1] + 1] = t
+    return big[..., 1:t.shape[-1] + 1]
+
+
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,d,hm,hb,rows,causal,one_batch", [
+    (1, 70, 136, 8, 2, 128, 2, 2, 70, True, False),    # four heads of a group to a workgroup
+    (2, 300, 264, 4, 1, 96, 1, 0, 0, False, False),    # ... no bias
+    (1, 129, 200, 4, 2, 128, 2, 2, 129, True, False),  # two heads
+    (1, 65, 128, 6, 3, 128, 3, 3, 1, False, False),    # ... a bias value per key
+    (1, 131, 200, 4, 4, 64, 4, 4, 131, True, False),   # head dims up to 64, rows of half a piece: dK/dV with tiles through registers
+    (1, 300, 72, 4, 2, 64, 2, 2, 300, False, False),
+    (1, 150, 264, 4, 1, 40, 1, 1, 1, True, False),
+    (2, 90, 136, 4, 2, 64, 2, 2, 90, True, True),      # one bias for the batch: dBias by fp32 atomics
+    (2, 90, 136, 8, 2, 128, 2, 2, 90, False, True),
+])
+def test_rows_of_whole_chunks_at_any_address(B, Lq, Lk, H, Hk, d, hm, hb, rows, causal, one_batch):
+    """Aligned rows of whole 8-key chunks have kernels of their own: the same results as rows that start anywhere."""
+    from flash_sparse_attn import flash_sparse_attn_func
+
+    print("chunks", B, Lq, Lk, H, Hk, d, hm, hb, rows, causal, one_batch, flush=True)
+    g = torch.Generator().manual_seed(Lq * 1000 + Lk)
+    r = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    q, k, v, dout = r(B, Lq, H, d), r(B, Lk, Hk, d), r(B, Lk, Hk, d), r(B, Lq, H, d)
+    mask = torch.rand(B, hm, Lq, Lk, generator=g) < 0.5
+    bias = r(1 if one_batch else B, hb, rows, Lk) if hb else None
+    ref = (c_oracle.forward(q, k, v, mask, bias, d ** -0.5, causal)[0],) + tuple(c_oracle.backward(q, k, v, dout, mask, bias, d ** -0.5, causal))
+    runs = []
+    for shape in (lambda t: t, _off_by_one):
+        leaves = [t.to(DEV).requires_grad_(True) for t in (q, k, v)] + ([shape(bias.to(DEV)).requires_grad_(True)] if hb else [])
+        out = flash_sparse_attn_func(*leaves[:3], shape(mask.to(DEV)), leaves[3] if hb else None, None, causal)
+        runs.append((out,) + torch.autograd.grad(out, leaves, dout.to(DEV)))
+    assert_out_close(runs[0][0].cpu(), ref[0])
+    for got, want, name in zip(runs[0][1:], ref[1:], ("dq", "dk", "dv", "dbias")):
+        assert_grad_close(got.cpu(), want, name)
+    for a, b, name in zip(*runs, ("out", "dq", "dk", "dv", "dbias")):
+        assert (one_batch and name == "dbias") or torch.equal(a, b), name
