@@ -263,10 +263,8 @@ __global__ void __launch_bounds__(NTHREADS, (D <= 64 && !GSUM) ? 2 : 1) bwd_dkdv
     };
 
     const int a_row = pi_row(r);
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    const uint32_t tr_off = (uint32_t)(((8 * g + te) * SM::S + 16 * tdh + 4 * tcp) * 2);
+    const TrLane tr = tr_lane(lane);
+    const uint32_t tr_off = (uint32_t)(((8 * g + tr.te) * SM::S + 16 * tr.tdh + 4 * tr.tcp) * 2);
     const uint32_t a_off = (uint32_t)((a_row * SM::S + g * 8) * 2);
 
     float colsum = 0.f;       // row-broadcast dbias: sum over queries of dS for this lane's key

@@ -190,12 +190,6 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const Bwd
     // Byte offsets of this thread's loads inside a 64-row block are loop invariants -- one set for full blocks, one
     // for the (only) partial block at the end of the queries, whose rows beyond Lq are clamped to the last row
     // (finite duplicates, cancelled by LSE = +inf) -- so a load is one instruction with a scalar block base.
-    typedef const __attribute__((address_space(1))) char *gptr_t;
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     const int m_last = (LqS - 1) / BM, row_last = (LqS - 1) % BM;
     uint32_t qoff[Q_IT], qoff_l[Q_IT], dooff[Q_IT], dooff_l[Q_IT];
 #pragma unroll
@@ -262,19 +256,18 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const Bwd
     typedef const __attribute__((address_space(1))) void gvoid_t;
     // The steps are walked with counters and running pointers (no division, no 64-bit products per step): inside a
     // query head the query block index falls by one per step, at a head change everything jumps by loop constants.
-    typedef const __attribute__((address_space(1))) char *gbytes_t;
     const int gi0 = CMP || n_steps == 0 ? g_lo : first_step / n_m, mi0 = s_hi - 1 - (CMP || n_steps == 0 ? 0 : first_step % n_m);
     int dma_gi = gi0, dma_mi = mi0;  // head and query block of the step being fetched
-    gbytes_t dma_q = nullptr, dma_do = nullptr, dma_stat = nullptr;  // its Q / dO block bases, this lane's statistic
+    gptr_t dma_q = nullptr, dma_do = nullptr, dma_stat = nullptr;  // its Q / dO block bases, this lane's statistic
     char *dma_dst = nullptr;
     const int64_t q_step = -(int64_t)BM * f.q_r * 2, do_step = -(int64_t)BM * p.do_r * 2;
     const int64_t q_head = (int64_t)f.q_h * 2 - (int64_t)(n_m - 1) * q_step, do_head = (int64_t)p.do_h * 2 - (int64_t)(n_m - 1) * do_step;
     const int64_t stat_head = (int64_t)(lane < 32 ? f.lse_h : p.sd_h) * 4 + (int64_t)(n_m - 1) * BM * 4;
     if (DMA && n_steps > 0) {
         const int h0 = hk * G + gi0, m00 = dma_mi * BM;
-        dma_q = (gbytes_t)((const uint16_t *)f.q + b * f.q_b + h0 * f.q_h + (sq.q0 + m00) * f.q_r);
-        dma_do = (gbytes_t)((const uint16_t *)p.dout + b * p.do_b + h0 * p.do_h + (sq.q0 + m00) * p.do_r);
-        dma_stat = (gbytes_t)(lane < 32 ? f.lse + b * f.lse_b + h0 * f.lse_h + sq.q0 + m00 + (lane & 31)
+        dma_q = (gptr_t)((const uint16_t *)f.q + b * f.q_b + h0 * f.q_h + (sq.q0 + m00) * f.q_r);
+        dma_do = (gptr_t)((const uint16_t *)p.dout + b * p.do_b + h0 * p.do_h + (sq.q0 + m00) * p.do_r);
+        dma_stat = (gptr_t)(lane < 32 ? f.lse + b * f.lse_b + h0 * f.lse_h + sq.q0 + m00 + (lane & 31)
                                         : p.softmax_d + b * p.sd_b + h0 * p.sd_h + sq.q0 + m00 + (lane & 31));
     }
     // sets up the fetch of the step the counters stand at (into stage `buf`)
@@ -303,17 +296,14 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const Bwd
     auto dma_piece = [&](int n) {
         const uint32_t dst = lds_addr(dma_dst);
         if (n < Q_IT) {
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         : : "v"(ld_partial ? qoff_l[n] : qoff[n]), "s"(ld_qbase), "s"(__builtin_amdgcn_readfirstlane(dst + (2 * wave + n) * 1024)));
+            load_lds16(ld_partial ? qoff_l[n] : qoff[n], ld_qbase, __builtin_amdgcn_readfirstlane(dst + (2 * wave + n) * 1024));
         } else if (n < 2 * Q_IT) {
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         : : "v"(ld_partial ? dooff_l[n - Q_IT] : dooff[n - Q_IT]), "s"(ld_dobase),
-                             "s"(__builtin_amdgcn_readfirstlane(dst + SM::Q_BYTES + (2 * wave + n - Q_IT) * 1024)));
+            load_lds16(ld_partial ? dooff_l[n - Q_IT] : dooff[n - Q_IT], ld_dobase, __builtin_amdgcn_readfirstlane(dst + SM::Q_BYTES + (2 * wave + n - Q_IT) * 1024));
         } else {
             // (every wave fetches the same 256 bytes: cheaper than a branch in the middle of the MFMAs.)  In the last,
             // partial block the rows beyond the end of the queries read the last row's numbers (masked where used).
             const int over = ld_partial ? (lane & 31) - row_last : 0;
-            gbytes_t sp = dma_stat - (over > 0 ? over * 4 : 0);
+            gptr_t sp = dma_stat - (over > 0 ? over * 4 : 0);
             asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
                          : : "v"(sp), "s"(__builtin_amdgcn_readfirstlane(dst + 2 * SM::Q_BYTES)));
         }
@@ -329,10 +319,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const Bwd
     };
 
     const int a_row = pi_row(r);
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    uint32_t tr_off = lds0 + TL::tr_base(g, te, tdh, tcp);  // (absolute LDS addresses of stage 0's Q tile)
+    const TrLane tr = tr_lane(lane);
+    uint32_t tr_off = lds0 + TL::tr_base(g, tr);  // (absolute LDS addresses of stage 0's Q tile)
     uint32_t a_off = lds0 + TL::frag_base(a_row, g);
     const uint32_t stat_off = lds0 + 32 * g;  // this lane's eight rows of a block of sixteen row statistics
 
@@ -969,12 +957,6 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
     // loads of the next tile can be issued one by one between the MFMAs of the current one.  The bias / mask of the
     // thread's column travel as raw, unconditional loads (an absent one is read from K and ignored) and are looked
     // at when they are stored.
-    typedef const __attribute__((address_space(1))) char *gptr_t;
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     const int j_last = Lk > 0 ? (Lk - 1) / BN : 0, last_row = Lk > 0 ? (Lk - 1) % BN : 0;
     uint32_t koff[K_IT], koff_l[K_IT], voff[K_IT], voff_l[K_IT];
 #pragma unroll
@@ -1020,10 +1002,10 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
     // (wave-uniform) onwards, lane after lane.  (m0 carries the LDS address; it is a reserved register that nothing
     // else in this kernel uses, and it is written immediately in front of every use.)
     auto dma16 = [](gptr_t base, uint32_t off, uint32_t dst) {
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst));
+        load_lds16(off, base, dst);
     };
     auto dma4 = [](gptr_t base, uint32_t off, uint32_t dst) {
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(dst));
+        load_lds4(off, base, dst);
     };
     constexpr int N_DMA = 2 * K_IT + (DMA_COL ? 1 : 0);  // direct loads of a wave per tile
     int dma_stage = 0;                   // stage the tile being fetched goes to (DMA)
@@ -1071,10 +1053,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
 
     const int a_row = pi_row(r);
     const uint32_t a_off = lds0 + SM::OFF_K + TL::frag_base(a_row, g);  // (absolute, stage 0 of K)
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    const uint32_t tr_off = lds0 + SM::OFF_K + TL::tr_base(g, te, tdh, tcp);
+    const TrLane tr = tr_lane(lane);
+    const uint32_t tr_off = lds0 + SM::OFF_K + TL::tr_base(g, tr);
 
     // A wave waits for its own pieces of the next tile, then the barrier publishes everybody's (DMA: by hand -- the
     // N_DMA loads of the tile after that, issued later, stay in flight; vmcnt in bits 3:0, lgkmcnt 0, expcnt not

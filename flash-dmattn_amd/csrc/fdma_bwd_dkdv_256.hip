@@ -37,7 +37,6 @@ constexpr int OFF_P = OFF_STAT + NST * 512;
 constexpr int SMEM = OFF_P + 4 * 4096;
 constexpr int N_DMA = 5;               // direct loads of a wave per step: 2 of Q, 2 of dO, the statistics
 
-__device__ __forceinline__ uint32_t swz(int row) { return (uint32_t)(((row & 3) << 2) | ((row >> 2) & 3)); }  // (see fdma_fwd_wide.hip)
 
 template <typename T, bool CAUSAL, bool CMP>
 __global__ void __launch_bounds__(NT) bwd_dkdv_256_kernel(const BwdParams p) {
@@ -132,16 +131,10 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_256_kernel(const BwdParams p) {
     };
 
     // ---- direct loads of a step: piece i of a tile is rows 2 i, 2 i + 1; wave w fetches pieces w and w + 8 of Q and of dO.
-    // A lane fills chunk position lane % 32 of its row, which holds chunk position ^ swz(row) of the global row.  Rows beyond the
+    // A lane fills chunk position lane % 32 of its row, which holds chunk position ^ chunk_swz(row) of the global row.  Rows beyond the
     // queries repeat the last one (masked where used), chunks beyond d repeat chunk 0 (they meet zeros).
-    typedef const __attribute__((address_space(1))) char *gptr_t;
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     const int prow = 2 * wave + (lane >> 5);
-    const int pchunk = (lane & 31) ^ (int)swz(prow);
+    const int pchunk = (lane & 31) ^ (int)chunk_swz<256>(prow);
     const uint32_t pcol = pchunk * 8 < f.d ? pchunk * 16 : 0;
     const uint32_t q_r2 = (uint32_t)(f.q_r * 2), do_r2 = (uint32_t)(p.do_r * 2);
     int dma_gi = gi0, dma_mi = mi0, dma_stage = 0;  // the step being fetched
@@ -154,13 +147,12 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_256_kernel(const BwdParams p) {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const int row = prow + 16 * i, row_c = row < rows ? row : rows;
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"((uint32_t)row_c * q_r2 + pcol), "s"(qb), "s"(dst + i * 8192));
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"((uint32_t)row_c * do_r2 + pcol), "s"(db), "s"(dst + TILE + i * 8192));
+            load_lds16((uint32_t)row_c * q_r2 + pcol, qb, dst + i * 8192);
+            load_lds16((uint32_t)row_c * do_r2 + pcol, db, dst + TILE + i * 8192);
         }
         // (even waves fetch the LSE values, odd ones D, all the same)
         const gptr_t sp = uniform_ptr(wave & 1 ? p.softmax_d + b * p.sd_b + h * p.sd_h + sq.q0 + m0 : f.lse + b * f.lse_b + h * f.lse_h + sq.q0 + m0);
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"((uint32_t)(lane < rows ? lane : rows) * 4), "s"(sp),
-                     "s"(__builtin_amdgcn_readfirstlane(lds0 + OFF_STAT + dma_stage * 512 + (wave & 1) * 256)));
+        load_lds4((uint32_t)(lane < rows ? lane : rows) * 4, sp, __builtin_amdgcn_readfirstlane(lds0 + OFF_STAT + dma_stage * 512 + (wave & 1) * 256));
         dma_stage = dma_stage == NST - 1 ? 0 : dma_stage + 1;
         if (more) {
             if (dma_mi == s_lo) { dma_mi = s_hi - 1; dma_gi++; } else dma_mi--;
@@ -169,12 +161,8 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_256_kernel(const BwdParams p) {
 
     // fragment addresses (stage 0): rows of Q (scores) or dO (dP); transposing reads of dO (dV) or Q (dK)
     const int frow = pi_row(r);
-    const uint32_t a_off = lds0 + (role ? TILE : 0) + (uint32_t)frow * ROW + (((uint32_t)g ^ swz(frow)) << 4);
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    const uint32_t tr_off = lds0 + (role ? 0 : TILE) + (uint32_t)(8 * g + te) * ROW +
-                            (((uint32_t)te << 6) | ((((uint32_t)(2 * tdh + (tcp >> 1))) ^ (uint32_t)(2 * g)) << 4) | ((uint32_t)(tcp & 1) << 3));
+    const uint32_t a_off = lds0 + (role ? TILE : 0) + (uint32_t)frow * ROW + (((uint32_t)g ^ chunk_swz<256>(frow)) << 4);
+    const uint32_t tr_off = lds0 + (role ? 0 : TILE) + tr_chunk<256>(g, tr_lane(lane));
     const uint32_t stat_off = lds0 + OFF_STAT + role * 256 + 32 * g;
     const uint32_t p_off = lds0 + OFF_P + kw * 4096 + lane * 16;
 

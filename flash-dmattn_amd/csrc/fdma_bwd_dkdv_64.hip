@@ -51,7 +51,6 @@ template <int BIAS> struct Smem {
     static_assert(2 * TOTAL <= 160 * 1024, "two workgroups per CU");
 };
 
-__device__ __forceinline__ uint32_t swz(int row) { return (uint32_t)((((row >> 1) & 1) << 2) | ((row >> 2) & 3)); }  // (see fdma_fwd_wide.hip)
 
 typedef int v2i32_t __attribute__((ext_vector_type(2)));
 // sixteen lanes read an 8 x 16 tile of bytes: lane i passes the address of bytes 8 (i & 1) .. of row i / 2 and gets column i
@@ -150,22 +149,16 @@ __global__ void __launch_bounds__(NT, 2) bwd_dkdv_64_kernel(const BwdParams p) {
     };
 
     // ---- direct loads of a step.  Q, dO: wave w fetches rows 8 w .. 8 w + 7; a lane fills chunk position lane % 8 of its row, which
-    // holds chunk position ^ swz(row) of the global row.  Rows beyond the queries repeat the last one, and chunks beyond the keys a
+    // holds chunk position ^ chunk_swz(row) of the global row.  Rows beyond the queries repeat the last one, and chunks beyond the keys a
     // valid one (masked where used); chunks beyond d repeat chunk 0 (they meet zeros).
-    typedef const __attribute__((address_space(1))) char *gptr_t;
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     auto load16 = [](uint32_t off, gptr_t base, uint32_t dst) {
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)));
+        load_lds16(off, base, __builtin_amdgcn_readfirstlane(dst));
     };
     auto load4 = [](uint32_t off, gptr_t base, uint32_t dst) {
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)));
+        load_lds4(off, base, __builtin_amdgcn_readfirstlane(dst));
     };
     const int prow = 8 * wave + (lane >> 3);
-    const int pchunk = (lane & 7) ^ (int)swz(prow);
+    const int pchunk = (lane & 7) ^ (int)chunk_swz<64>(prow);
     const uint32_t pcol = pchunk * 8 < f.d ? pchunk * 16 : 0;
     const uint32_t q_r2 = (uint32_t)(f.q_r * 2), do_r2 = (uint32_t)(p.do_r * 2);
     const uint32_t bi_r2 = ROWS ? (uint32_t)(f.bi_r * 2) : 0, m_r1 = BITS ? (uint32_t)f.mb_r : (has_mask ? (uint32_t)f.m_r : 0);
@@ -221,14 +214,12 @@ __global__ void __launch_bounds__(NT, 2) bwd_dkdv_64_kernel(const BwdParams p) {
 
     // fragment addresses (stage 0): rows of Q (dO: + TILE); transposing reads of either, of the wave's bias and of its mask
     const int frow = pi_row(r);
-    const uint32_t a_off = lds0 + (uint32_t)frow * ROW + (((uint32_t)g ^ swz(frow)) << 4);
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    const uint32_t tr_off = lds0 + (uint32_t)(8 * g + te) * ROW + (((uint32_t)(2 * tdh + (tcp >> 1)) ^ swz(8 * g + te)) << 4) + ((uint32_t)(tcp & 1) << 3);
+    const uint32_t a_off = lds0 + (uint32_t)frow * ROW + (((uint32_t)g ^ chunk_swz<64>(frow)) << 4);
+    const TrLane tr = tr_lane(lane);
+    const uint32_t tr_off = lds0 + tr_chunk<64>(g, tr);
     const uint32_t w_off = lds0 + SM::OFF_WAVE + wave * SM::WAVE;
-    const uint32_t bt_off = w_off + (8 * g + te) * 64 + 32 * tdh + 8 * tc;
-    const uint32_t mt_off = w_off + SM::WB + (BITS ? 32 * g : (8 * g + (tj >> 1)) * 32 + 16 * tdh + 8 * (tj & 1));
+    const uint32_t bt_off = w_off + (8 * g + tr.te) * 64 + 32 * tr.tdh + 8 * tr.tc;
+    const uint32_t mt_off = w_off + SM::WB + (BITS ? 32 * g : (8 * g + ((lane & 15) >> 1)) * 32 + 16 * tr.tdh + 8 * (lane & 1));
     const uint32_t ds_off = w_off + (8 * g) * 64 + 2 * r;
     const uint32_t stat_off = lds0 + SM::OFF_STAT + 32 * g;
 

@@ -138,12 +138,6 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
     // ---- direct loads of a step's tiles: load n = 2 * wave + i of a tile fills LDS bytes [1024 n, 1024 n + 1024), i.e.
     // rows 4n .. 4n+3, lane l the chunk POSITION l % 16 of row 4n + l / 16 -- which holds chunk position ^ swz(row) of the
     // global row.  One more 4-byte load per wave: the 64 LSE values (even waves) or D values (odd waves).
-    typedef const __attribute__((address_space(1))) char *gptr_t;
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     // bases of the group's first head, and bytes from one head, and one row, to the next
     const int h0 = hk * G;
     const int64_t q_h2 = f.q_h * 2, do_h2 = p.do_h * 2;
@@ -182,11 +176,9 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
             const int i = n & 1;
             const uint32_t r2 = n < 2 ? q_r2 : do_r2;
             const uint32_t off = least((n < 2 ? q_row : do_row) + 4 * i * r2, ld_rows * r2) + pcol[i];
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         : : "v"(off), "s"(n < 2 ? ld_q : ld_do), "s"(__builtin_amdgcn_readfirstlane(ld_dst + (n < 2 ? 0 : TILE) + (2 * wave + i) * 1024)));
+            load_lds16(off, n < 2 ? ld_q : ld_do, __builtin_amdgcn_readfirstlane(ld_dst + (n < 2 ? 0 : TILE) + (2 * wave + i) * 1024));
         } else {
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
-                         : : "v"(least((uint32_t)lane, ld_rows) * 4), "s"(ld_stat), "s"(__builtin_amdgcn_readfirstlane(ld_dst + 2 * TILE + (wave & 1) * BM * 4)));
+            load_lds4(least((uint32_t)lane, ld_rows) * 4, ld_stat, __builtin_amdgcn_readfirstlane(ld_dst + 2 * TILE + (wave & 1) * BM * 4));
         }
     };
 
@@ -253,14 +245,12 @@ __global__ void __launch_bounds__(NT) bwd_dkdv_wide_kernel(const BwdParams p) {
     // fragment addresses (see LdsTile): Q / dO rows of this wave's half, K / V rows of its keys
     uint32_t a_off = lds0 + 32 * qh * TL::ROW_BYTES + TL::frag_base(pi_row(r), g);
     uint32_t kv_off = lds0 + OFF_K + TL::frag_base(kw * 32 + r, g);
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    uint32_t tr_off = lds0 + 32 * qh * TL::ROW_BYTES + TL::tr_base(g, te, tdh, tcp);
+    const TrLane tr = tr_lane(lane);
+    uint32_t tr_off = lds0 + 32 * qh * TL::ROW_BYTES + TL::tr_base(g, tr);
     const uint32_t stat_off = lds0 + 2 * TILE + (32 * qh + 8 * g) * 4;
     // fused tile: rows 32 qh + 16 blk + 8 g + .., this lane's column.  Read through transposing reads (lane (te, tc) of 16
     // supplies four elements of row te, lane i receives rows 0 .. 3 of column i), written back element by element.
-    const uint32_t fb_tr = lds0 + OFF_FB + ((32 * qh + 8 * g + te) * SB + kw * 32 + 16 * tdh + 4 * tc) * 2;
+    const uint32_t fb_tr = lds0 + OFF_FB + ((32 * qh + 8 * g + tr.te) * SB + kw * 32 + 16 * tr.tdh + 4 * tr.tc) * 2;
     uint16_t *fb_col = (uint16_t *)(smem + OFF_FB) + (32 * qh + 8 * g) * SB + kw * 32 + r;
     float *s_col = (float *)(smem + OFF_COL);
 

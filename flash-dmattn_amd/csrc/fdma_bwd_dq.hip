@@ -167,12 +167,6 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         }
         return any != 0;
     };
-    typedef const __attribute__((address_space(1))) char *gptr_t;
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     auto load_rest = [&](int j) {
         const int n0 = j * BN;
         if (bbase) {
@@ -195,8 +189,8 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
             for (int it = 0; it < K_IT; it++) {
                 const int row = kr0 + it * K_RPP, row_c = row < last ? row : last;
                 const uint32_t ko = (uint32_t)(row_c * (int)f.k_r + kcol_g) * 2, vo = (uint32_t)(row_c * (int)f.v_r + kcol_g) * 2;
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(ko), "s"(kb), "s"(dst + it * K_RPP * 256) : "memory");
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(vo), "s"(vb), "s"(dst + SM::K_BYTES + it * K_RPP * 256) : "memory");
+                load_lds16<true>(ko, kb, dst + it * K_RPP * 256);
+                load_lds16<true>(vo, vb, dst + SM::K_BYTES + it * K_RPP * 256);
             }
             return;
         }
@@ -240,10 +234,8 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
 
     const int a_row = pi_row(r);
     const uint32_t a_off = lds0 + TL::frag_base(a_row, g);
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    const uint32_t tr_off = lds0 + TL::tr_base(g, te, tdh, tcp);
+    const TrLane tr = tr_lane(lane);
+    const uint32_t tr_off = lds0 + TL::tr_base(g, tr);
 
     auto compute = [&](int j, int buf) {
         const int n0 = j * BN + kh * BK;

@@ -39,7 +39,6 @@ constexpr int OFF_DS = OFF_P + 4 * 4096;
 constexpr int OFF_BITS = OFF_DS + 4 * 2048;
 constexpr int SMEM = OFF_BITS + (1 << 20) / BN / 8;  // (bwd_colmask_applicable: 2^20 keys at most)
 
-__device__ __forceinline__ uint32_t swz(int row) { return (uint32_t)(((row & 3) << 2) | ((row >> 2) & 3)); }  // (see fdma_fwd_wide.hip)
 
 template <typename T, bool CAUSAL, bool CMP>
 __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
@@ -184,14 +183,8 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
 
     // ---- staging: piece i of a tile is rows 2 i, 2 i + 1; wave w fetches pieces w and w + 8 of K and of V (see
     // fdma_bwd_dkdv_256.hip).  The column: with compacted keys as it is in memory, else made by wave 0 from mask and bias.
-    typedef const __attribute__((address_space(1))) char *gptr_t;
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     const int prow = 2 * wave + (lane >> 5);
-    const int pchunk = (lane & 31) ^ (int)swz(prow);
+    const int pchunk = (lane & 31) ^ (int)chunk_swz<256>(prow);
     const uint32_t pcol = pchunk * 8 < f.d ? pchunk * 16 : 0;
     const uint32_t k_r2 = (uint32_t)(f.k_r * 2), v_r2 = (uint32_t)(f.v_r * 2);
     auto load_tile = [&](int j, int stage) {
@@ -210,22 +203,17 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const int row = prow + 16 * i, row_c = row < rows ? row : rows;
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"((uint32_t)row_c * k_r2 + pcol), "s"(kb), "s"(dst + i * 8192));
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"((uint32_t)row_c * v_r2 + pcol), "s"(vb), "s"(dst + TILE + i * 8192));
+            load_lds16((uint32_t)row_c * k_r2 + pcol, kb, dst + i * 8192);
+            load_lds16((uint32_t)row_c * v_r2 + pcol, vb, dst + TILE + i * 8192);
         }
         if (CMP)  // (columns beyond the kept keys repeat the last one: masked where used)
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"((uint32_t)(r < rows ? r : rows) * 4), "s"(uniform_ptr(fbrow + j * BN)),
-                         "s"(__builtin_amdgcn_readfirstlane(lds0 + OFF_COL + (uint32_t)stage * 256)));
+            load_lds4((uint32_t)(r < rows ? r : rows) * 4, uniform_ptr(fbrow + j * BN), __builtin_amdgcn_readfirstlane(lds0 + OFF_COL + (uint32_t)stage * 256));
     };
 
     // fragment addresses (stage 0): rows of K or V; transposing reads of K, this role's half of the head dim
     const int frow = pi_row(r);
-    const uint32_t a_off = lds0 + (role ? TILE : 0) + (uint32_t)frow * ROW + (((uint32_t)g ^ swz(frow)) << 4);
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    const uint32_t tr_off = lds0 + (uint32_t)role * 256 + (uint32_t)(8 * g + te) * ROW +
-                            (((uint32_t)(2 * tdh + (tcp >> 1)) ^ swz(8 * g + te)) << 4) + ((uint32_t)(tcp & 1) << 3);
+    const uint32_t a_off = lds0 + (role ? TILE : 0) + (uint32_t)frow * ROW + (((uint32_t)g ^ chunk_swz<256>(frow)) << 4);
+    const uint32_t tr_off = lds0 + (uint32_t)role * 256 + tr_chunk<256>(g, tr_lane(lane));
     const uint32_t col_off = lds0 + OFF_COL + 32 * g;
     const uint32_t p_off = lds0 + OFF_P + rw * 4096 + lane * 16, ds_off = lds0 + OFF_DS + rw * 2048 + lane * 16;
 

@@ -116,10 +116,8 @@ __global__ void __launch_bounds__(DS_THREADS) bwd_dq_ds_kernel(const BwdParams p
     };
 
     // transposing reads of the row-major K rows (see fdma_common.h): A operand = K^T, 32 head-dim rows x 16 keys
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    const uint32_t tr_off = (uint32_t)(((8 * g + te) * SM::S + 16 * tdh + 4 * tcp) * 2);
+    const TrLane tr = tr_lane(lane);
+    const uint32_t tr_off = (uint32_t)(((8 * g + tr.te) * SM::S + 16 * tr.tdh + 4 * tr.tcp) * 2);
     // B operand = dS^T: keys 16 kb + 8 g .. + 7 of this lane's query row
     const uint32_t b_off = (uint32_t)(SM::TILE_BYTES + ((wave * 32 + r) * SM::SD + 8 * g) * 2);
 

@@ -165,6 +165,52 @@ __device__ __forceinline__ uint32_t mask_bits_byte(u32x2_t piece, int kk) {
     return ((sh & 32) ? piece[1] >> (sh & 31) : piece[0] >> sh) & 0xffu;
 }
 
+// A pointer that all lanes share, in scalar registers (the global address space survives the integer round trip).
+typedef const __attribute__((address_space(1))) char *gptr_t;
+__device__ __forceinline__ gptr_t uniform_ptr(const void *ptr) {
+    const uint64_t v = (uint64_t)ptr;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (gptr_t)(((uint64_t)hi << 32) | lo);
+}
+
+// Direct loads: every lane's 16 or 4 bytes at `base` + off go to LDS, lane after lane from address `dst` on (both the same for all lanes).
+// In assembly, because behind the compiler's builtin every LDS read waits for all LDS operations in flight.  So the compiler
+// neither waits for them nor knows that they write LDS: a kernel waits by hand (s_waitcnt vmcnt) in front of the barrier that publishes
+// them, AND, for those that are still in flight behind its last tile, in front of whatever it puts into that LDS next; no barrier does
+// it.  MEMORY: other accesses stay on their side of the load.  m0 carries the address; nothing else in these kernels uses it.
+template <bool MEMORY = false> __device__ __forceinline__ void load_lds16(uint32_t off, gptr_t base, uint32_t dst) {
+    if constexpr (MEMORY) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst) : "memory");
+    else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(dst));
+}
+__device__ __forceinline__ void load_lds4(uint32_t off, gptr_t base, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(dst));
+}
+
+// What a lane supplies to a transposing read (lds_ld_tr16): row te of four, its 8-byte piece tc of a 32-byte half row tdh.  tcp: the
+// piece in the order in which the results are rows of an accumulator (see pi_row).
+struct TrLane {
+    int te, tc, tcp, tdh;
+};
+__device__ __forceinline__ TrLane tr_lane(int lane) {
+    const int tj = lane & 15, tc = tj & 3;
+    return {tj >> 2, tc, (tc == 1) ? 2 : (tc == 2 ? 1 : tc), (lane >> 4) & 1};
+}
+
+// Swizzle of tiles with unpadded rows: chunk c of 16 bytes lives at chunk c ^ chunk_swz(row) (see LdsTile).  Rows of 512 bytes meet the
+// banks as rows of 256 do: the 16 chunks of a half row are permuted.  Two rows of 128 bytes share a line of banks: four
+// consecutive ones lie in different 64-byte quarters (transposing reads), sixteen in different chunks (fragment reads).
+template <int D> __device__ __forceinline__ uint32_t chunk_swz(int row) {
+    return D == 64 ? (uint32_t)((((row >> 1) & 1) << 2) | ((row >> 2) & 3)) : (uint32_t)(((row & 3) << 2) | ((row >> 2) & 3));
+}
+
+// Where a lane's piece of a transposing read lies in such a tile: row 8 g + te, elements 16 tdh + 4 tcp .. + 3 of its first 32.
+template <int D> __device__ __forceinline__ uint32_t tr_chunk(int g, const TrLane &t) {
+    const int row = 8 * g + t.te, c = 2 * t.tdh + (t.tcp >> 1);
+    // (above 64 the same as c ^ chunk_swz(row), in the form that costs the kernels fewest registers)
+    const uint32_t at = D == 64 ? ((uint32_t)c ^ chunk_swz<D>(row)) << 4 : ((uint32_t)t.te << 6) | (((uint32_t)c ^ (uint32_t)(2 * g)) << 4);
+    return (uint32_t)row * (2 * D) + (at | ((uint32_t)(t.tcp & 1) << 3));
+}
+
 // Row-major LDS tile of 16-bit elements ([row][head dim]) that is read two ways: as MFMA fragments (ds_read_b128:
 // lane (r, g) takes the 16 bytes of chunk 2*ks + g of row pi_row(r)) and through transposing reads (lds_read_tr16:
 // 16 lanes take four 8-byte pieces of each of four consecutive rows), and written row by row (16 lanes per row).
@@ -179,7 +225,7 @@ template <int D> struct LdsTile {
     static constexpr bool SWZ = D == 128;
     static constexpr int S = SWZ ? D : D + 8;  // row stride, elements
     static constexpr int ROW_BYTES = S * 2;
-    static __device__ __forceinline__ uint32_t swz(int row) { return (uint32_t)(((row & 3) << 2) | ((row >> 2) & 3)); }
+    static __device__ __forceinline__ uint32_t swz(int row) { return chunk_swz<128>(row); }
     // 16-byte chunk c of a row (tile writes)
     static __device__ __forceinline__ uint32_t chunk(int row, int c) {
         return SWZ ? (uint32_t)row * 256u + ((((uint32_t)c) ^ swz(row)) << 4) : (uint32_t)((row * S + c * 8) * 2);
@@ -191,12 +237,10 @@ template <int D> struct LdsTile {
     static __device__ __forceinline__ uint32_t frag_at(uint32_t base, int ks) {
         return SWZ ? (base ^ ((uint32_t)ks << 5)) : base + (uint32_t)ks * 32u;
     }
-    // transposing reads: lane (g, te, tdh, tcp) supplies row 8*g + te, elements 16*tdh + 4*tcp .. +3 of a 32-element
-    // block db, in 16-row block rb; hi = 1: the same four rows further down
-    static __device__ __forceinline__ uint32_t tr_base(int g, int te, int tdh, int tcp) {
-        return SWZ ? (uint32_t)(8 * g + te) * 256u + (((uint32_t)te << 6) | ((((uint32_t)(2 * tdh + (tcp >> 1))) ^ (uint32_t)(2 * g)) << 4) |
-                                                     ((uint32_t)(tcp & 1) << 3))
-                   : (uint32_t)(((8 * g + te) * S + 16 * tdh + 4 * tcp) * 2);
+    // transposing reads: lane (g, t) supplies row 8*g + te, elements 16*tdh + 4*tcp .. +3 of a 32-element block db, in 16-row
+    // block rb; hi = 1: the same four rows further down
+    static __device__ __forceinline__ uint32_t tr_base(int g, const TrLane &t) {
+        return SWZ ? tr_chunk<128>(g, t) : (uint32_t)(((8 * g + t.te) * S + 16 * t.tdh + 4 * t.tcp) * 2);
     }
     static __device__ __forceinline__ uint32_t tr_at(uint32_t base, int rb, int db, int hi) {
         return SWZ ? (base ^ (((uint32_t)db << 6) | ((uint32_t)hi << 4))) + (uint32_t)(hi * 4 * 256 + rb * 16 * 256)

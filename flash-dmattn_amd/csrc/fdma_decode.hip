@@ -188,22 +188,14 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
 
     // fragment addresses inside a staged tile (see fdma_common.h)
     const uint32_t a_off = (uint32_t)((pi_row(r) * SM::S + g * 8) * 2);
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    const uint32_t tr_off = (uint32_t)(((8 * g + te) * SM::S + 16 * tdh + 4 * tcp) * 2);
+    const TrLane tr = tr_lane(lane);
+    const uint32_t tr_off = (uint32_t)(((8 * g + tr.te) * SM::S + 16 * tr.tdh + 4 * tr.tcp) * 2);
     // staging: this lane's row within a load instruction and its chunk
     const int srow = lane / CH, sc = lane % CH;
     const uint32_t st_off = (uint32_t)((srow * SM::S + sc * 8) * 2);
     const bool pad_lane = sc >= nchunk;             // head dimension below D: these lanes stage zeros
     const int scl = pad_lane ? nchunk - 1 : sc;
 
-    typedef const __attribute__((address_space(1))) char *gptr_t;  // global address space survives the integer round trip
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo32 = __builtin_amdgcn_readfirstlane((uint32_t)v), hi32 = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi32 << 32) | lo32);
-    };
 
     // phase 1: the ordered list of the kept keys of a pass
     uint32_t bits[DEC_NJ];

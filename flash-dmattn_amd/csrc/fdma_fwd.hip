@@ -207,12 +207,6 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     };
     // K and V of tile j into registers, or (DMA) on their way into the tile's stage: in assembly and waited for by hand (kv_landed),
     // because behind the compiler's builtin every LDS read waits for all LDS operations in flight
-    typedef const __attribute__((address_space(1))) char *gptr_t;
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     auto load_kv = [&](int j) {
         const int n0 = j * BN;
         if constexpr (DMA) {
@@ -223,8 +217,8 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             for (int it = 0; it < K_IT; it++) {
                 const int row = kr0 + it * K_RPP, row_c = row < last ? row : last;
                 const uint32_t ko = (uint32_t)(row_c * (int)p.k_r + kcol_g) * 2, vo = (uint32_t)(row_c * (int)p.v_r + kcol_g) * 2;
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(ko), "s"(kb), "s"(dst + it * K_RPP * 256) : "memory");
-                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(vo), "s"(vb), "s"(dst + SM::K_BYTES + it * K_RPP * 256) : "memory");
+                load_lds16<true>(ko, kb, dst + it * K_RPP * 256);
+                load_lds16<true>(vo, vb, dst + SM::K_BYTES + it * K_RPP * 256);
             }
             return;
         }
@@ -275,13 +269,13 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
 
     const int a_row = pi_row(r);
     // (this lane's part of the address of a transposing read of the V tile)
-    const uint32_t tr_lane = TL::tr_base(g, (lane & 15) >> 2, (lane >> 4) & 1, (lane & 3) == 1 ? 2 : ((lane & 3) == 2 ? 1 : (lane & 3)));
+    const uint32_t tr_base = TL::tr_base(g, tr_lane(lane));
 
     // ---- one tile from LDS stage `buf`
     auto compute = [&](int j, int buf) {
         const int n0 = j * BN + kh * BK;
         const uint32_t a_k = lds0 + (uint32_t)(buf * SM::STAGE + kh * BK * TL::ROW_BYTES) + TL::frag_base(a_row, g);
-        const uint32_t tr_v = lds0 + (uint32_t)(buf * SM::STAGE + SM::K_BYTES + kh * BK * TL::ROW_BYTES) + tr_lane;
+        const uint32_t tr_v = lds0 + (uint32_t)(buf * SM::STAGE + SM::K_BYTES + kh * BK * TL::ROW_BYTES) + tr_base;
         const char *sF = smem + buf * SM::STAGE + 2 * SM::K_BYTES + ((rw * 32 + r) * SM::SF + kh * BK + 8 * g) * 2;
         // scores start from the fused mask+bias tile (exp2 domain)
         f32x16_t s[MB];

@@ -279,15 +279,9 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
     const uint8_t *mrow_ld = mrow ? mrow : (const uint8_t *)kbase;
     const uint16_t *brow_ld = brow ? brow : kbase;
     bool bcol_ok = false;
-    typedef const __attribute__((address_space(1))) char *gptr_t;  // global address space survives the integer round trip
     gptr_t tb_k = nullptr, tb_v = nullptr;        // tile bases (wave-uniform, in scalar registers)
     bool last_k = false, last_v = false;          // the K / V tile in flight is the partial one
 
-    auto uniform_ptr = [](const char *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     // next fetches: K and the side-row inputs of tile jk / V of tile jv (with split roles a wave has one of the two)
     auto set_tile_k = [&](Turn tk) {
         if (!role_k) return;

@@ -166,16 +166,9 @@ __global__ void __launch_bounds__(ST_THREADS, 1) fwd_stream_kernel(const FwdPara
     // address `dst` (wave-uniform) onwards, lane after lane.  Written in assembly: issued through the compiler's
     // builtin, every later LDS read would wait for all direct loads in flight (the compiler cannot tell which slot they
     // fill); the waits are placed by hand (publish()).  m0 carries the LDS address; nothing else here uses it.
-    typedef const __attribute__((address_space(1))) char *gptr_t;
     const uint32_t lane16 = (uint32_t)lane * 16u;
     auto dma16 = [&](gptr_t base, uint32_t dst) {
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                     : : "v"(lane16), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory");
-    };
-    auto uniform_ptr = [](const char *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
+        load_lds16<true>(lane16, base, __builtin_amdgcn_readfirstlane(dst));
     };
     // Fetch cursor: the tile fetched next is tile f_tile of the item of round f_round (f_nt tiles), at f_kv / f_x; it goes
     // to ring slot f_pos & 3.  Past the last tile of the last item the last tile is fetched again (the slot is free by

@@ -63,13 +63,6 @@ template <int D_, int RG> struct Cfg {
     static_assert(8 * RPP % 16 == 0, "a wave's pieces lie rows of one swizzle apart");
 };
 
-// Rows of a tile are unpadded, their 16-byte chunks permuted by a XOR with a function of the row (see LdsTile).  Rows of 512 bytes
-// meet the banks as rows of 256 do: the 16 chunks of a half row are permuted.  Two rows of 128 bytes share a line of banks: four
-// consecutive ones lie in different 64-byte quarters (transposing reads), sixteen in different chunks (fragment reads).
-template <int D> __device__ __forceinline__ uint32_t swz(int row) {
-    return D == 64 ? (uint32_t)((((row >> 1) & 1) << 2) | ((row >> 2) & 3)) : (uint32_t)(((row & 3) << 2) | ((row >> 2) & 3));
-}
-
 template <typename T, int D, int RG, bool CAUSAL, bool CMP>
 __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const FwdParams p) {
     using E = Elem<T>;
@@ -187,16 +180,10 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     };
 
     // ---- staging: a piece is 1 KB, whole rows; wave w fetches pieces w + 8 i of K and of V.  A lane fills chunk position
-    // `lane % CH` of its row, which holds chunk position ^ swz(row) of the global row; rows 16 apart have the same swizzle.  Rows beyond the keys are clamped to the last one (their column says -inf), chunks beyond d to chunk 0 (they
+    // `lane % CH` of its row, which holds chunk position ^ chunk_swz(row) of the global row; rows 16 apart have the same swizzle.  Rows beyond the keys are clamped to the last one (their column says -inf), chunks beyond d to chunk 0 (they
     // meet zero Q and columns of O that are not stored).
-    typedef const __attribute__((address_space(1))) char *gptr_t;
-    auto uniform_ptr = [](const void *ptr) -> gptr_t {
-        const uint64_t v = (uint64_t)ptr;
-        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-        return (gptr_t)(((uint64_t)hi << 32) | lo);
-    };
     const int prow = C::RPP * wave + lane / C::CH;
-    const int pchunk = lane % C::CH ^ (int)swz<D>(prow);
+    const int pchunk = lane % C::CH ^ (int)chunk_swz<D>(prow);
     const uint32_t pcol = pchunk * 8 < p.d ? pchunk * 16 : 0;
     const uint32_t k_r2 = (uint32_t)(p.k_r * 2), v_r2 = (uint32_t)(p.v_r * 2);
     uint32_t k_row = prow * k_r2, v_row = prow * v_r2;  // (offsets grow with the row: clamped by the last row's)
@@ -228,7 +215,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         const uint32_t r2 = n < NP ? k_r2 : v_r2, at = (n < NP ? k_row : v_row) + 8 * C::RPP * i * r2, last = (uint32_t)t_rows * r2;
         const uint32_t off = (at < last ? at : last) + pcol;
         const uint32_t dst = lds0 + (n < NP ? 0 : OFF_V) + (uint32_t)((ONE ? 0 : t_stage * TILE) + (wave + 8 * i) * 1024);
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(n < NP ? tb_k : tb_v), "s"(__builtin_amdgcn_readfirstlane(dst)));
+        load_lds16(off, n < NP ? tb_k : tb_v, __builtin_amdgcn_readfirstlane(dst));
     };
     auto publish = [&]() {
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's pieces have landed
@@ -248,12 +235,8 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
 
     // fragment addresses (stage 0).  K: chunk 2 ks + g of row 32 kg + pi_row(r).  V^T: see LdsTile::tr_base.
     const int frow = 32 * kg + pi_row(r);
-    uint32_t a_off = lds0 + (uint32_t)frow * ROW + (((uint32_t)g ^ swz<D>(frow)) << 4);
-    const int tj = lane & 15, te = tj >> 2, tc = tj & 3;
-    const int tcp = (tc == 1) ? 2 : (tc == 2 ? 1 : tc);
-    const int tdh = (lane >> 4) & 1;
-    uint32_t tr_off = lds0 + OFF_V + (uint32_t)(32 * kg + 8 * g + te) * ROW +
-                      ((((uint32_t)(2 * tdh + (tcp >> 1)) ^ swz<D>(8 * g + te)) << 4) | ((uint32_t)(tcp & 1) << 3));
+    uint32_t a_off = lds0 + (uint32_t)frow * ROW + (((uint32_t)g ^ chunk_swz<D>(frow)) << 4);
+    uint32_t tr_off = lds0 + OFF_V + (uint32_t)(32 * kg) * ROW + tr_chunk<D>(g, tr_lane(lane));
     const uint32_t col_off = lds0 + OFF_COL + 128 * kg + 32 * g;
 
     f32x16_t o[DB];
