@@ -1328,7 +1328,7 @@ size_t plan_kv_parts(BwdParams &p, size_t *db_bytes) {
     // Ragged, d = 65 .. 128: while the longest block runs, a CU's other units, two at a time, fill it with less than 60 steps each;
     // what parts save then is less than their sums.  Over 37 calls, whole / parts (us): 11 entries up to 1187 x 32/16 (2.4 units per CU, longest 76
     // steps) 222 / 242, five of 800 x 64/16 (2.3, 128) 411 / 430, 11 entries x 8/8 (1.2, 38) 123 / 130; on the other side 11 entries x 48/12 (1.8,
-    // 152) 354 / 318, the same x 16/8 (1.2, 76) 177 / 157; worst kept five of 800 x 48/12 (1.7, 128) 339 / 351 and 4000, 3000, 700, 1 x 8/8 (2, 125) 379 / 383.  At d <= 64 parts lose nowhere.
+    // 152) 354 / 318, the same x 16/8 (1.2, 76) 177 / 157; worst kept five of 800 x 48/12 (1.7, 128) 339 / 351 and 4000, 3000, 700, 1 x 8/8 (2, 125) 375 / 390.  At d <= 64 parts lose nowhere.
     if (f.cu_q && f.d > 64 && f.d <= 128 && longest * cus < 60 * units) most = 1;
     if (longest <= 20 || units >= cus * 5 / 2 || (units >= cus / 2 && 2 * longest <= 5 * (int64_t)quota)) most = 1;
     if (most * units > 2048) most = 2048 / units;

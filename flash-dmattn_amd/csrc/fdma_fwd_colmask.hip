@@ -872,18 +872,17 @@ hipError_t launch_d(const FwdParams &p, hipStream_t stream) {
 
 }  // namespace
 
-// Shares that the key tiles of a row block are cut into: a chunk of a prompt against a long cache has too few blocks of 128
-// rows for the chip, and a workgroup's time is 12 us and 1.6 us per turn of two tiles.  (64-row workgroups on twice the CUs
-// were no faster: a turn takes as long for one wave per SIMD as for two.)  The shares' fp32 results cost what they weigh --
-// 256 workgroups write and read 17 MB, 12 us, and two shares of 128 blocks were no faster than none -- so at most 128
-// workgroups, and only from three shares on; a share has at least 1024 keys and (in the kernel) eight tiles of kept keys.
+// Shares that the key tiles of a row block are cut into: a chunk of a prompt against a long cache has too few row blocks for the
+// chip, and a workgroup's time is the chain of its tiles.  The shares' fp32 results cost what they weigh -- 256 workgroups of 128 rows
+// wrote and read 17 MB, 12 us, and two shares of 128 blocks were no faster than none -- so at most 128 blocks of 128 rows, and only
+// from three shares on; a share has at least 1024 keys and (in the kernel) 512 kept ones.  The kernel is that of 64-row blocks
+// (takes_key_groups).
 // Only where the keys are twice the queries or more: a training step keeps the forward's workspace until its backward, which
 // would hold the shares, and has as many queries as keys.  Whole keys / shares in us (a workspace without / with room for them;
-// medians over 1 to 40 blocks of 2 to 300 rows, d = 128; d = 64 is alike), with a sixteenth, a quarter and all of the keys kept:
-//   3072 keys   16.5 / 20.2    24.4 / 27.9    53.0 / 34.4        16384 keys   27.4 / 25.9    65.0 / 31.1    207.5 / 54.8
-//   6144 keys   19.4 / 22.4    34.0 / 26.8    90.2 / 39.3        32768 keys   40.4 / 28.4   114.7 / 40.1    395.4 / 88.2
-// (As measured with 128-row blocks; at d > 64 the 64-row blocks of fdma_fwd_wide.hip take these calls, whole and in shares, in 0.8 to
-// 0.88 of the time.)
+// medians over 1 to 40 blocks of 2 to 300 rows, d = 128; at d = 64 0.7 to 0.85 of that), with a sixteenth, a quarter and all of the
+// keys kept:
+//   3072 keys   13.1 / 16.3    19.1 / 22.7    41.2 / 28.4        16384 keys   21.5 / 20.9    49.7 / 26.2    157.2 / 45.7
+//   6144 keys   15.2 / 18.6    26.0 / 21.0    70.0 / 33.7        32768 keys   31.6 / 23.1    87.3 / 34.2    297.6 / 70.2
 // How much is kept is not known here: with under 1024 kept keys there is a single share and the merge costs its 3 to 4 us for
 // nothing; the other way round a share too few costs more.
 int key_shares(const FwdParams &p) {
