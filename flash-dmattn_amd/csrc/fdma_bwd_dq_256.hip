@@ -192,12 +192,10 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
         const int left = Lk - 1 - j * BN, rows = left < BN - 1 ? left : BN - 1;
         if (!CMP && wave == 0) {
             const int col = j * BN + r;
-            const bool ok = col < Lk;
-            const int cc = ok ? col : 0;
-            float v = ok ? 0.f : -INFINITY;
-            if (mrow && !mrow[cc]) v = -INFINITY;
-            if (brow) v += E::lo((uint32_t)brow[cc]) * kLog2e;
-            lds_st32(lds0 + OFF_COL + (uint32_t)stage * 256 + 4 * lane, __float_as_uint(ok && v != -INFINITY ? v : -INFINITY));
+            const int cc = col < Lk ? col : 0;
+            const bool keep = col < Lk && (!mrow || mrow[cc]);  // (a dropped key's bias is not looked at: it need not be a number)
+            const float v = brow ? E::lo((uint32_t)brow[cc]) * kLog2e : 0.f;
+            lds_st32(lds0 + OFF_COL + (uint32_t)stage * 256 + 4 * lane, __float_as_uint(keep ? v : -INFINITY));
         }
         const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(stage * STAGE + wave * 1024));
 #pragma unroll

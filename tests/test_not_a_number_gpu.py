@@ -113,3 +113,26 @@ def test_every_row_that_sees_it_and_no_other(route, where, request):
     assert torch.isnan(bdk[0, at, 0]).all()
     for good, got in ((dk, bdk), (dv, bdv)):  # (the other kv heads)
         assert rel_err(got[:, :, 1:], good[:, :, 1:]) <= GRAD_RTOL
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("route", [r for r in ROUTES if ROUTES[r][0] != "none"])
+def test_bias_of_dropped_keys(route, value, request):
+    """What the mask drops may have any bias: the results are those of a zero there, to the bit."""
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func
+
+    rows, mode, Lq, Lk, H, Hk, D, window = ROUTES[route]
+    set_compact(mode)
+    before = _cabi.stream_min_items(1 if route == "tile images" else 0)
+    request.addfinalizer(lambda: _cabi.stream_min_items(before))
+    shape = (1, Hk, Lq if rows == "query" else 1, Lk)
+    q, k, v, mask, bias = [t.to(DEV) for t in make_inputs(1, Lq, Lk, H, Hk, D, shape, shape, window, seed=Lq + Lk)]
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(7)).to(torch.bfloat16).to(DEV)
+    results = []
+    for fill in (0.0, value):
+        leaves = [t.detach().clone().requires_grad_(True) for t in (q, k, v, torch.where(mask, bias, fill))]
+        out = flash_sparse_attn_func(*leaves[:3], mask, leaves[3], None, Lq > 1)
+        results.append((out.detach(),) + torch.autograd.grad(out, leaves, dout))
+    for a, b, name in zip(*results, ("out", "dq", "dk", "dv", "dbias")):
+        assert torch.equal(a, b), name
+    assert not results[1][4][~mask].any()
