@@ -113,9 +113,8 @@ __global__ void __launch_bounds__(NT, 2) bwd_dkdv_64_kernel(const BwdParams p) {
         z_col = (uint32_t)(z_key + 8 * (tid & 15) < f.Lk ? 16 * (tid & 15) : 0);
     }
     auto clear_one = [&]() {
-        int row = z_row + (tid >> 4);
-        row = row < z_rows ? row : z_rows - 1;
-        __builtin_nontemporal_store(u32x4_t{0, 0, 0, 0}, (u32x4_t *)(z_base + ((uint32_t)row * db_r2 + z_col)));
+        const RowPiece at = row_piece(z_row, z_rows, tid >> 4, db_r2);
+        __builtin_nontemporal_store(u32x4_t{0, 0, 0, 0}, (u32x4_t *)(z_base + at.base + (at.off + z_col)));
         z_left--;
         z_row += 16;
         if (z_row >= z_rows) {
@@ -455,7 +454,7 @@ template <typename T> hipError_t launch_t(const BwdParams &p, hipStream_t stream
 
 }  // namespace
 
-// Direct loads take aligned 16-byte pieces (bits: 4 bytes) with 32-bit offsets inside a step's rows; a per-query dBias that several
+// Direct loads take aligned 16-byte pieces (bits: 4 bytes) with 32-bit offsets inside the rows of a step (or of a piece to clear); a per-query dBias that several
 // workgroups add to goes through fp32 atomics, which bwd_dkdv_kernel has.
 bool bwd_dkdv_64_applicable(const BwdParams &p) {
     const FwdParams &f = p.f;

@@ -134,6 +134,18 @@ __host__ __device__ inline int kv_parts_of(int steps, int quota, int most) {
     return n < most ? n : most;
 }
 
+// Row `i` of the piece of 16 rows that starts at row `first` of a matrix of `rows` (the last one where it has fewer), in bytes: where
+// the piece starts, the same for all lanes and of any size (a per-query dBias of 46352 keys has 4 GiB), and a lane's way from there
+// (rows below 2^25 bytes).
+struct RowPiece {
+    int64_t base;
+    uint32_t off;
+};
+__host__ __device__ inline RowPiece row_piece(int first, int rows, int i, uint32_t row_bytes) {
+    const int last = rows - 1 - first;
+    return {(int64_t)first * row_bytes, (uint32_t)(i < last ? i : last) * row_bytes};
+}
+
 struct FwdParams {
     const void *q, *k, *v;
     const uint8_t *mask;  // nullptr = absent

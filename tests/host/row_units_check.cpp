@@ -1,7 +1,8 @@
 // Host-side check of the mapping from workgroups to blocks of query rows (row_grid / row_unit in flash-dmattn_amd/csrc/fdma_params.h, built and
 // run by tests/test_row_units.py with g++), over random batches of one length and ragged ones: every block of rows that a
 // call computes has exactly one workgroup per query head, no other workgroup names one, a launch is made of whole turns over the 8 XCDs,
-// and rounding the blocks of the longest entry up to its lists no more than doubles it.
+// and rounding the blocks of the longest entry up to its lists no more than doubles it.  And of the places of rows in pieces of 16 (row_piece),
+// where a matrix has more bytes than 32 bits count.
 #include <cstdio>
 #include <cstring>
 #include <vector>
@@ -59,6 +60,18 @@ int main() {
             }
         checked += grid;
     }
+    // rows of a matrix in pieces of 16, at any size: where 32 bits hold neither the matrix nor the way to a row
+    for (int rows : {1, 15, 16, 17, 300, 46352, 65536, 131071})
+        for (uint32_t row_bytes : {16u, 2u * 46352u, 2u * 65536u, (1u << 25) - 16u})
+            for (int first = 0; first < rows; first += 16)
+                for (int i = 0; i < 16; i++) {
+                    const RowPiece at = row_piece(first, rows, i, row_bytes);
+                    const int row = first + i < rows ? first + i : rows - 1;
+                    if (at.base + (int64_t)at.off != (int64_t)row * row_bytes || at.off > (15u << 25)) {
+                        std::printf("FAILED: row %d of %d, %u bytes each, lies at %lld + %u\n", row, rows, row_bytes, (long long)at.base, at.off);
+                        return 1;
+                    }
+                }
     std::printf("%s (%lld workgroups, %lld batches of whole entries)\n", whole > 100 ? "OK" : "FAILED", checked, whole);
     return whole > 100 ? 0 : 1;
 }

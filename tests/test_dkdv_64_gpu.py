@@ -53,3 +53,28 @@ def test_against_oracle(B, Lq, Lk, H, Hk, d, hm, hb, rows, causal, bits, dtype):
     for got, again, want, name in zip(*runs, ref, ("dq", "dk", "dv", "dbias")):
         assert_grad_close(got.cpu(), want, name)
         assert torch.equal(got, again), name
+
+
+def test_dbias_of_more_than_4_gib():
+    """Rows above the diagonal are cleared wherever they lie: L = 46400, the first pieces of the last rows lie beyond 2^32 bytes."""
+    from flash_sparse_attn import flash_sparse_attn_func
+
+    L, D = 46400, 64
+    g = torch.Generator(device=DEV).manual_seed(46)
+    q, k, v, dout = [torch.randn(1, L, 1, D, generator=g, device=DEV).bfloat16() for _ in range(4)]
+    bias = torch.empty(1, 1, L, L, dtype=torch.bfloat16, device=DEV)
+    for r in range(0, L, 6400):
+        bias[0, 0, r:r + 6400] = torch.randn(min(6400, L - r), L, generator=g, device=DEV)
+    leaves = [k.requires_grad_(True), bias.requires_grad_(True)]
+    out = flash_sparse_attn_func(q, k, v, None, bias, None, True)
+    torch.full((L, L), float("nan"), dtype=torch.bfloat16, device=DEV)  # (what the gradient's memory may hold before)
+    dbias = torch.autograd.grad(out, leaves, dout)[1][0, 0]
+    k = k.detach()
+    for r in range(0, L, 6400):
+        rows = dbias[r:r + 6400]
+        assert torch.isfinite(rows).all() and not torch.triu(rows, r + 1).any()
+    rows = torch.tensor([0, 1, 31, 32, 200, 20000, L - 65, L - 17, L - 16, L - 1], device=DEV)
+    s = q[0, rows, 0].float() @ k[0, :, 0].float().T * D ** -0.5 + bias.detach()[0, 0, rows].float()
+    p = s.masked_fill(torch.arange(L, device=DEV)[None] > rows[:, None], float("-inf")).softmax(-1)
+    dp = dout[0, rows, 0].float() @ v[0, :, 0].float().T
+    assert_grad_close(dbias[rows], p * (dp - (p * dp).sum(-1, keepdim=True)), "dbias")
