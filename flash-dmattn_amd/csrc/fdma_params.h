@@ -117,6 +117,7 @@ __host__ __device__ inline int kv_unit_steps(int Lq, int Lk, int causal, int n0,
 }
 // all steps of one query head's units (exact without a causal mask and for Lq == Lk up to the rounding of blocks)
 __host__ __device__ inline int64_t kv_head_steps(int Lq, int Lk, int causal, int bm) {
+    if (Lq <= 0 || Lk <= 0) return 0;  // (what a ragged batch has beside its longest entry, when the caller names more than there is)
     const int64_t n = (Lk + 127) / 128, most = kv_unit_steps(Lq, Lk, causal, 0, bm), least = n > 0 ? kv_unit_steps(Lq, Lk, causal, (int)(n - 1) * 128, bm) : 0;
     return n * (most + least) / 2;
 }

@@ -2,7 +2,7 @@
 // run by tests/test_row_units.py with g++), over random batches of one length and ragged ones: every block of rows that a
 // call computes has exactly one workgroup per query head, no other workgroup names one, a launch is made of whole turns over the 8 XCDs,
 // and rounding the blocks of the longest entry up to its lists no more than doubles it.  And of the places of rows in pieces of 16 (row_piece),
-// where a matrix has more bytes than 32 bits count.
+// where a matrix has more bytes than 32 bits count, and of the steps of an entry (kv_head_steps) for lengths below zero.
 #include <cstdio>
 #include <cstring>
 #include <vector>
@@ -60,6 +60,17 @@ int main() {
             }
         checked += grid;
     }
+    // steps of an entry, and per part of a batch, whatever lengths come out of a caller's longest length and totals
+    for (int lq : {-5000, -64, -1, 0, 1, 64, 700})
+        for (int lk : {-90000, -128, -1, 0, 1, 129, 3000})
+            for (int causal = 0; causal < 2; causal++)
+                for (int bm : {32, 64}) {
+                    const int64_t steps = kv_head_steps(lq, lk, causal, bm);
+                    if (steps < 0 || ((lq <= 0 || lk <= 0) && steps != 0) || kv_part_quota(steps * 64) < KV_PART_MIN) {
+                        std::printf("FAILED: %lld steps for %d rows, %d keys\n", (long long)steps, lq, lk);
+                        return 1;
+                    }
+                }
     // rows of a matrix in pieces of 16, at any size: where 32 bits hold neither the matrix nor the way to a row
     for (int rows : {1, 15, 16, 17, 300, 46352, 65536, 131071})
         for (uint32_t row_bytes : {16u, 2u * 46352u, 2u * 65536u, (1u << 25) - 16u})
