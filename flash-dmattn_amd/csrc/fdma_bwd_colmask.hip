@@ -955,7 +955,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
     // Byte offsets of this thread's loads inside a tile are loop invariants -- one set for full tiles, one for the
     // (only) partial tile at the end of the keys -- so a load is one instruction with a scalar tile base, and the
     // loads of the next tile can be issued one by one between the MFMAs of the current one.  The bias / mask of the
-    // thread's column travel as raw, unconditional loads (an absent one is read from K and ignored) and are looked
+    // thread's column travel as raw, unconditional loads (an absent one is the first element of K, ignored) and are looked
     // at when they are stored.
     const int j_last = Lk > 0 ? (Lk - 1) / BN : 0, last_row = Lk > 0 ? (Lk - 1) % BN : 0;
     uint32_t koff[K_IT], koff_l[K_IT], voff[K_IT], voff_l[K_IT];
@@ -993,8 +993,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
             if (CMP) {
                 braw = __float_as_uint(fbrow[cc]);
             } else {
-                mraw = mrow_ld[cc];
-                braw = brow_ld[cc];
+                mraw = mrow_ld[mrow ? cc : 0];
+                braw = brow_ld[brow ? cc : 0];
             }
         }
     };

@@ -275,7 +275,8 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
     }
     u32x4_t sreg[NL];             // staging registers
     uint32_t braw = 0, mraw = 0;  // raw bias / mask of this thread's column of the tile whose side rows are in flight
-    // an absent mask / bias is read from K instead (any valid address) and ignored when the value is used
+    // an absent mask / bias is the first element of K instead (its rows may lie on each other: nothing behind them is K's) and ignored
+    // when the value is used
     const uint8_t *mrow_ld = mrow ? mrow : (const uint8_t *)kbase;
     const uint16_t *brow_ld = brow ? brow : kbase;
     bool bcol_ok = false;
@@ -300,8 +301,8 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
         if (CMP) {
             braw = __float_as_uint(fbrow[cc]);
         } else {
-            mraw = mrow_ld[cc];
-            braw = brow_ld[cc];
+            mraw = mrow_ld[mrow ? cc : 0];
+            braw = brow_ld[brow ? cc : 0];
         }
     };
     auto set_tile_v = [&](Turn tv) {

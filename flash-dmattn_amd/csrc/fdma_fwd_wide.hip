@@ -197,15 +197,15 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         const int left = Lk - 1 - j * BN;
         t_rows = left < BN - 1 ? left : BN - 1;
         t_stage = stage;
-        if (wave < BN / 64) {  // (raw, unconditional loads: an absent mask or bias is read from K and ignored)
+        if (wave < BN / 64) {  // (raw, unconditional loads: an absent mask or bias is the first element of K, ignored)
             const int col = j * BN + tid;
             col_ok = col < Lk;
             const int cc = col_ok ? col : 0;
             if (CMP) {
                 braw = __float_as_uint(fbrow[cc]);
             } else {
-                mraw = (mrow ? mrow : (const uint8_t *)kbase)[cc];
-                braw = (brow ? brow : kbase)[cc];
+                mraw = (mrow ? mrow : (const uint8_t *)kbase)[mrow ? cc : 0];
+                braw = (brow ? brow : kbase)[brow ? cc : 0];
             }
         }
     };

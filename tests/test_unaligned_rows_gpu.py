@@ -1,6 +1,7 @@
 """Masks and biases that all queries share are taken at any address and row stride (run with `-m gpu`): the same values in
 rows of an odd length and in padded, 16-byte aligned rows give the same results bit for bit; and decode from the mask
-builder's list of kept keys against the C oracle."""
+builder's list of kept keys against the C oracle.  K and V rows that lie on each other (stride 0): there is one row of memory, and nothing
+behind it is read in the place of an absent mask or bias."""
 import pytest
 import torch
 
@@ -60,3 +61,23 @@ def test_decode_from_the_list_of_kept_keys(B, Lk, H, Hk, d, window, bias_heads):
         out = flash_sparse_attn_func(q.to(DEV), k.to(DEV), v.to(DEV), keep, bias.to(DEV))
     ref, _ = c_oracle.forward(q, k, v, keep.cpu(), bias, d ** -0.5, False)
     assert_out_close(out.cpu(), ref)
+
+
+@pytest.mark.parametrize("Lq,Lk,H,Hk,d", [(1, 3000, 8, 2, 128), (100, 3000, 4, 2, 64), (100, 3000, 4, 2, 128), (100, 3000, 4, 2, 256),
+                                          (2100, 700, 32, 4, 64), (2100, 700, 32, 4, 128), (2100, 700, 32, 4, 256)])
+@pytest.mark.parametrize("what", ["nothing", "mask", "bias"])
+def test_one_row_of_keys_for_all(Lq, Lk, H, Hk, d, what):
+    from flash_sparse_attn import flash_sparse_attn_func
+
+    print("one row", Lq, Lk, H, Hk, d, what, flush=True)
+    set_compact("0")
+    q, k, v, mask, bias, dout = [t.to(DEV) for t in _case(1, Lq, Lk, H, Hk, d, 0.5, torch.bfloat16, seed=Lk)]
+    mask, bias = mask if what == "mask" else None, bias if what == "bias" else None
+    res = []
+    for shape in (lambda t: t[:, :1].expand_as(t), lambda t: t[:, :1].expand_as(t).contiguous()):
+        leaves = [t.detach().requires_grad_(True) for t in (q, shape(k), shape(v))]
+        out = flash_sparse_attn_func(*leaves, mask, bias, None, Lq > 1)
+        res.append((out.detach(),) + torch.autograd.grad(out, leaves, dout))
+    assert leaves[1].stride(1) != 0 and not res[0][0].isnan().any()
+    for a, b, name in zip(*res, ("out", "dq", "dk", "dv")):
+        assert torch.equal(a, b), name
