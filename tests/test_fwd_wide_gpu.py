@@ -88,3 +88,25 @@ def test_ragged(lens, H, Hk, D):
         s = slice(at, at + n)
         assert_out_close(out[s], eager.attention_forward(q[None, s], k[None, s], v[None, s], None, None, None, True)[0][0])
         at += n
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("lens,H,Hk,D", [
+    ([1, 200, 64, 65, 300], 4, 2, 136),    # 64-row blocks with one stage of K and V
+    ([1, 200, 64, 65, 300], 4, 2, 256),
+    ([129, 1, 700, 127, 900], 16, 8, 256),  # more of them than CUs: 128-row ones with two stages
+])
+def test_ragged_above_head_dim_128(lens, H, Hk, D, causal):
+    from flash_sparse_attn import flash_sparse_attn_varlen_func
+
+    print(lens, H, Hk, D, causal, flush=True)
+    g = torch.Generator().manual_seed(6)
+    q = torch.randn(sum(lens), H, D, generator=g).to(torch.bfloat16).to(DEV)
+    k, v = [torch.randn(sum(lens), Hk, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2)]
+    cu = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    out = flash_sparse_attn_varlen_func(q, k, v, cu, cu, max(lens), max(lens), is_causal=causal)
+    at = 0
+    for n in lens:
+        s = slice(at, at + n)
+        assert_out_close(out[s], eager.attention_forward(q[None, s], k[None, s], v[None, s], None, None, None, causal)[0][0])
+        at += n
