@@ -17,6 +17,8 @@
 #include <type_traits>
 #include <stdint.h>
 
+#include "fdma_params.h"
+
 namespace fdma {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -290,18 +292,12 @@ __device__ __forceinline__ u32x4_t ld_row16(const uint8_t *row, int c, int n) {
 }
 
 // The 8-key chunk of a mask or bias row that starts at key kk (a multiple of 8), for rows that may start at any address
-// (mask: any byte, bias: any element).  chunk8_at: the key the chunk is fetched from -- one that keeps the 16-byte load
-// inside a row of at least 8 keys (shorter rows are readable up to 8: fdma.h) -- and chunk8_fix / chunk8_fix_mask put a
-// chunk that was fetched further in front back in place (only the chunk that straddles the end of the row is; the caller
+// (mask: any byte, bias: any element).  chunk8_at (fdma_params.h): the key the chunk is fetched from, and chunk8_fix / chunk8_fix_mask put
+// a chunk that was fetched further in front back in place (only the chunk that straddles the end of the row is; the caller
 // drops keys at or beyond the end, and chunks that start there hold anything).  ODD = false: rows of whole, aligned chunks,
 // nothing to put back -- a kernel of its own, because the test for it costs the memory-bound kernels 7 % at head dim 64.
 typedef u32x2_t __attribute__((aligned(1))) u32x2_any_t;
 typedef u32x4_t __attribute__((aligned(2))) u32x4_el_t;
-template <bool ODD> __device__ __forceinline__ int chunk8_at(int kk, int Lk) {
-    if (!ODD) return kk < Lk ? kk : 0;
-    const int last = Lk >= 8 ? Lk - 8 : 0;
-    return kk < last ? kk : last;
-}
 template <bool ODD> __device__ __forceinline__ u32x2_t chunk8_fix_mask(u32x2_t m, int kk, int Lk) {
     if (!ODD) return m;
     const int by = kk - chunk8_at<true>(kk, Lk);

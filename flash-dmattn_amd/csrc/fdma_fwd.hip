@@ -155,19 +155,19 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     // same swizzle)
     const int kc_g = kc ^ (int)TL::swz(kr0), kcol_g = kc_g * 8 < p.d ? kc_g * 8 : 0;
     // (a mask that comes packed to bits: one byte per 8-key chunk instead of eight, expanded where it is looked at)
-    const uint8_t *mbits = (mbase && p.mbits) ? p.mbits + b * p.mb_b + hm * p.mb_h : nullptr;
+    const bool bits = mbase && p.mbits;
+    const uint8_t *mrows = bits ? p.mbits + b * p.mb_b + hm * p.mb_h : mbase;
+    const int64_t mrow_bytes = bits ? p.mb_r : p.m_r;
+    // One 8-byte load from one address: with the choice left to the loads they become two, in branches (d = 256, 2316 x 2/1, causal 170
+    // us, so 155; 4 x 2047 x 16, d = 128 200, so 188).
     auto load_mask = [&](int j, u32x2_t (&dst)[F_IT]) {
         if (!mbase) return;
-        int kk = j * BN + 8 * fc;
-        kk = kk < p.Lk ? kk : 0;
+        const int at = mask_piece_at(bits, j * BN + 8 * fc, p.Lk);
 #pragma unroll
         for (int it = 0; it < F_IT; it++) {
             int row = m0 + fr0 + F_RPP * it;
             row = row < p.Lq ? row : p.Lq - 1;
-            // (one 8-byte load either way, from an address chosen without a branch: mask bytes of the chunk, or the
-            // aligned piece of the bit row that holds the chunk's byte)
-            const uint8_t *src = mbits ? mbits + (int64_t)row * p.mb_r + ((kk >> 3) & ~7) : mbase + (int64_t)row * p.m_r + kk;
-            dst[it] = *(const u32x2_t *)src;
+            dst[it] = *(const u32x2_any_t *)(mrows + (int64_t)row * mrow_bytes + at);
         }
     };
     // validity of the chunks (rows < Lq, keys < Lk, not entirely above the causal diagonal) applied to the loaded
@@ -178,7 +178,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
 #pragma unroll
         for (int it = 0; it < F_IT; it++) {
             const int row = m0 + fr0 + F_RPP * it;
-            u32x2_t mv = mbase ? (mbits ? mask_bits_to_bytes(mask_bits_byte(dst[it], kk)) : dst[it]) : u32x2_t{0x01010101u, 0x01010101u};
+            u32x2_t mv = mbase ? (bits ? mask_bits_to_bytes(mask_bits_byte(dst[it], kk)) : chunk8_fix_mask<ODD>(dst[it], kk, p.Lk)) : u32x2_t{0x01010101u, 0x01010101u};
             const bool ok = row < p.Lq && kk < p.Lk && !(CAUSAL && kk > row + shift);
             uint64_t keepm = ok ? ~0ull : 0ull;
             if (kk + 8 > p.Lk && kk < p.Lk) keepm = (1ull << (8 * (p.Lk - kk))) - 1ull;  // chunk straddles the end of the keys

@@ -147,6 +147,20 @@ __host__ __device__ inline RowPiece row_piece(int first, int rows, int i, uint32
     return {(int64_t)first * row_bytes, (uint32_t)(i < last ? i : last) * row_bytes};
 }
 
+// The key that an 8-key chunk of a mask or bias row is fetched from, for the chunk that starts at key kk (a multiple of 8): one that keeps
+// the load inside a row of at least 8 keys (shorter rows are readable up to 8: fdma.h).  ODD = false: rows of whole chunks.
+template <bool ODD> __host__ __device__ inline int chunk8_at(int kk, int Lk) {
+    if (!ODD) return kk < Lk ? kk : 0;
+    const int last = Lk >= 8 ? Lk - 8 : 0;
+    return kk < last ? kk : last;
+}
+// Where the 8 bytes lie that hold this chunk of a mask row: its mask bytes or, of a mask packed to bits, the aligned piece of the bit row
+// with the chunk's byte.  (One form for both: a choice between two addresses becomes two loads.)
+__host__ __device__ inline int mask_piece_at(bool bits, int kk, int Lk) {
+    const int last = bits ? Lk - 1 : (Lk >= 8 ? Lk - 8 : 0), k = kk < last ? kk : last;
+    return (k >> (bits ? 3 : 0)) & (bits ? ~7 : ~0);
+}
+
 struct FwdParams {
     const void *q, *k, *v;
     const uint8_t *mask;  // nullptr = absent

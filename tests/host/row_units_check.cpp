@@ -2,7 +2,8 @@
 // run by tests/test_row_units.py with g++), over random batches of one length and ragged ones: every block of rows that a
 // call computes has exactly one workgroup per query head, no other workgroup names one, a launch is made of whole turns over the 8 XCDs,
 // and rounding the blocks of the longest entry up to its lists no more than doubles it.  And of the places of rows in pieces of 16 (row_piece),
-// where a matrix has more bytes than 32 bits count, and of the steps of an entry (kv_head_steps) for lengths below zero.
+// where a matrix has more bytes than 32 bits count, of the steps of an entry (kv_head_steps) for lengths below zero, and
+// of what is fetched for 8-key chunks of mask rows (mask_piece_at).
 #include <cstdio>
 #include <cstring>
 #include <vector>
@@ -83,6 +84,17 @@ int main() {
                         return 1;
                     }
                 }
+    // what is fetched for a chunk of a mask row: inside the row, and the chunk's keys are among it
+    for (int lk = 8; lk < 700; lk++)
+        for (int kk = 0; kk < lk + 512; kk += 8) {
+            const int at = mask_piece_at(false, kk, lk), bits = mask_piece_at(true, kk, lk), row_bytes = ((lk + 7) / 8 + 7) / 8 * 8;
+            const bool in = at >= 0 && at + 8 <= lk && (kk >= lk || (at <= kk && kk < at + 8 && at == (lk % 8 ? chunk8_at<true>(kk, lk) : chunk8_at<false>(kk, lk))));
+            const bool in_bits = bits >= 0 && bits % 8 == 0 && bits + 8 <= row_bytes && (kk >= lk || (8 * bits <= kk && kk < 8 * bits + 64));
+            if (!in || !in_bits) {
+                std::printf("FAILED: chunk %d of %d keys is fetched from %d (bits: byte %d)\n", kk, lk, at, bits);
+                return 1;
+            }
+        }
     std::printf("%s (%lld workgroups, %lld batches of whole entries)\n", whole > 100 ? "OK" : "FAILED", checked, whole);
     return whole > 100 ? 0 : 1;
 }

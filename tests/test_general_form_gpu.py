@@ -109,3 +109,29 @@ def test_rows_of_whole_chunks_at_any_address(B, Lq, Lk, H, Hk, d, hm, hb, rows, 
         assert_grad_close(got.cpu(), want, name)
     for a, b, name in zip(*runs, ("out", "dq", "dk", "dv", "dbias")):
         assert (one_batch and name == "dbias") or torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("causal", [False, True])
+def test_last_rows_end_with_their_memory(d, causal):
+    """Mask rows of 10 MiB in all, which the allocator has from the device as a piece of that size: the last chunk of the last row ends where
+    the memory does.  The same results as rows with room behind them."""
+    from flash_sparse_attn import flash_sparse_attn_func
+
+    print("last rows", d, causal, flush=True)
+    H, Lq, Lk = 16, 32768, 20
+    g = torch.Generator(DEV).manual_seed(d)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV, dtype=torch.bfloat16)
+    q, k, v, dout = r(1, Lq, H, d), r(1, Lk, H, d), r(1, Lk, H, d), r(1, Lq, H, d)
+    keep = torch.rand(1, H, Lq, Lk, generator=g, device=DEV) < 0.5
+    torch.cuda.empty_cache()
+    mask, bias = keep.clone(), r(1, H, Lq, Lk)
+    assert mask.numel() % (2 << 20) == 0
+    runs = []
+    for shape in (lambda t: t, _padded):
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v, shape(bias))]
+        out = flash_sparse_attn_func(*leaves[:3], shape(mask), leaves[3], None, causal)
+        runs.append((out.detach(),) + torch.autograd.grad(out, leaves, dout))
+    assert not runs[0][0].isnan().any()
+    for a, b, name in zip(*runs, ("out", "dq", "dk", "dv", "dbias")):
+        assert torch.equal(a, b), name
