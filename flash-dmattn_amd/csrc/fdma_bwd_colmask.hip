@@ -770,6 +770,7 @@ template <int D, int BN> struct DqcSmem {
     static constexpr int OFF_BIAS = OFF_V + NST * K_BYTES;
     static constexpr int OFF_BITS = OFF_BIAS + 3 * 256;  // three bias columns (a direct load fills 256 bytes)
     static constexpr int TOTAL = OFF_BITS + DQ_MAX_KEYS / BN / 8;
+    static_assert(TOTAL >= RED_LDS, "the workgroups that sum parts use it");
 };
 
 // BARE: no compaction, no mask, no bias (ragged batches, plain attention): there is no bias column, and the K / V tiles can
@@ -813,7 +814,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
         // some workgroups sum partial results of the dK/dV kernel instead
         const int at = lid - p.red_first;
         if (at >= 0 && at < p.red_count) {
-            dkdv_reduce_blocks<T, D>(p, at, p.red_count, threadIdx.x);
+            dkdv_reduce_blocks<T, D>(p, at, p.red_count, threadIdx.x, (float *)smem);
             return;
         }
         if (at >= 0) lid -= p.red_count;
@@ -1281,7 +1282,7 @@ hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
     const int n_dq = row_grid(pr.f, Q_BM);  // a multiple of 8
     if (!f.cmp.on) return launch_dq_grid<T, D, CAUSAL>(pr, n_dq, stream);
     const int units_max = f.B * f.Hk * ((f.Lk + KV_BN - 1) / KV_BN);
-    place_reduction(pr, n_dq, units_max * (D / 16));
+    place_reduction(pr, n_dq, units_max * (f.d / 4 + (f.bias ? 1 : 0)));
     return launch_dq_grid<T, D, CAUSAL>(pr, n_dq + pr.red_count, stream);
 }
 

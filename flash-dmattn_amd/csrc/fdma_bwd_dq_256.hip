@@ -37,6 +37,7 @@ constexpr int OFF_COL = NST * STAGE;   // per stage: 32 floats, twice (what a di
 constexpr int OFF_P = OFF_COL + NST * 256;
 constexpr int OFF_DS = OFF_P + 4 * 4096;
 constexpr int OFF_BITS = OFF_DS + 4 * 2048;
+static_assert(OFF_BITS >= 2 * RED_LDS, "the workgroups that sum parts use it");
 constexpr int SMEM = OFF_BITS + (1 << 20) / BN / 8;  // (bwd_colmask_applicable: 2^20 keys at most)
 
 
@@ -56,7 +57,7 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
     if (CMP) {  // some workgroups sum partial results of the dK/dV kernel instead (see place_reduction, fdma_bwd_colmask.hip)
         const int at = lid - p.red_first;
         if (at >= 0 && at < p.red_count) {
-            dkdv_reduce_blocks<T, D>(p, at * 2 + (wave >> 2), p.red_count * 2, tid & 255);
+            dkdv_reduce_blocks<T, D>(p, at * 2 + (wave >> 2), p.red_count * 2, tid & 255, (float *)(smem + (wave >> 2) * RED_LDS));
             return;
         }
         if (at >= 0) lid -= p.red_count;
