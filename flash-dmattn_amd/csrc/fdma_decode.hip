@@ -49,75 +49,102 @@ __device__ __forceinline__ uint32_t nz_bytes_to_bits(uint32_t x) {
     return ((y >> 7) * 0x10204080u) >> 28;
 }
 
-// LISTS: the caller has handed over the ordered list of kept keys (fdma_kept_keys: the mask builder writes it).  A
-// workgroup then takes its share of the LIST instead of a range of keys and builds nothing: one trip to memory less in a
-// chain of six, and every split has the same number of rows whatever the mask looks like.
-// PERHEAD: mask or bias differ between the query heads of a group, so a lane fetches the mask byte and the
-// bias of its own (key, head) pairs; otherwise one fused value per key serves all columns.
-// out[b,h,:] = sum_s exp(lse_s - lse) * o_s ;  lse = logsumexp_s lse_s  (empty everywhere: 0 / +inf) for one (b, h) row,
-// by ONE wave: lane s (and s + 64) fetches lse_s, the weights are made once and left in the wave's own piece of LDS
-// (`s_w`, room for 128 floats), then lane e sums its head-dim elements over the splits with the loads of eight splits
-// in flight: two dependent trips to memory per row, whatever the number of splits.  COHERENT: the partials were written
-// by other workgroups of the SAME launch (possibly on another XCD, behind another L2): they are fetched with
-// device-scope loads.  Both users of this function sum in the same order, so their results agree bit for bit.
+// COHERENT: the partials were written by other workgroups of the SAME launch (possibly on another XCD, behind another L2):
+// they are fetched with device-scope loads.
 template <bool COHERENT> __device__ __forceinline__ float part_load(const float *ptr) {
     if (COHERENT) return __uint_as_float(__hip_atomic_load((const uint32_t *)ptr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     return *ptr;
+}
+
+template <bool COHERENT> __device__ __forceinline__ f32x2_t part_load2(const float *ptr) {  // (8-byte aligned)
+    union { uint64_t u; f32x2_t f; } x;
+    if (COHERENT) x.u = __hip_atomic_load((const uint64_t *)ptr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else x.f = *(const f32x2_t *)ptr;
+    return x.f;
 }
 
 __device__ __forceinline__ void part_store(float *ptr, float v) {
     __hip_atomic_store((uint32_t *)ptr, __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename T, bool COHERENT>
-__device__ __forceinline__ void combine_row(const FwdParams &p, int64_t row, int lane, float *s_w) {
+// out[b,h,:] = sum_s exp(lse_s - lse) * o_s ;  lse = logsumexp_s lse_s  (empty everywhere: 0 / +inf) for one (b, h) row,
+// by ONE wave: lane s (and s + 64) fetches lse_s and holds the weight of split s, then lane i sums its head-dim elements 2 i,
+// 2 i + 1 (and + 128) over the splits.  Bound by trips to memory: up to CMB_FLIGHT splits are requested together, the first of
+// them beside the LSEs (eight at a time, weights through LDS: 2049 keys x 32 / 8 heads, 9 splits, the call 10.0 -> 9.3 us; 65536 x 2 / 1,
+// 32 splits 10.9 -> 9.8).
+// Both users of this function sum in the same order, so their results agree bit for bit.
+constexpr int CMB_FLIGHT = 32;
+constexpr int CMB_GROUP = 8;  // requested and added without a branch between them
+
+template <typename T, bool COHERENT, bool PAIRS>
+__device__ __forceinline__ void combine_row_as(const FwdParams &p, int64_t row, int lane) {
     using E = Elem<T>;
     const int64_t rows = (int64_t)p.B * p.H;
     const float lv0 = lane < p.splits ? part_load<COHERENT>(p.lse_part + (int64_t)lane * rows + row) : -INFINITY;
     const float lv1 = lane + 64 < p.splits ? part_load<COHERENT>(p.lse_part + (int64_t)(lane + 64) * rows + row) : -INFINITY;
-    // the partial outputs of the first eight splits for this lane's first two elements are requested right behind
-    // the LSEs (they do not depend on them): one trip to memory instead of two for up to eight splits
     const int64_t step = rows * p.d;
-    const float *op_row = p.o_part + row * p.d;
-    const int n0 = p.splits < 8 ? p.splits : 8;
-    float v0[8], v1[8];
+    f32x2_t v[CMB_FLIGHT];
+    auto fetch = [&](int e0, int s0) {
+        const int n = p.splits - s0, e = e0 + 2 * lane;
+        const float *op = p.o_part + row * p.d + (e < p.d ? e : 0) + s0 * step;
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-        v0[u] = (u < n0 && lane < p.d) ? part_load<COHERENT>(op_row + lane + (int64_t)u * step) : 0.f;
-        v1[u] = (u < n0 && lane + 64 < p.d) ? part_load<COHERENT>(op_row + lane + 64 + (int64_t)u * step) : 0.f;
-    }
+        for (int u = 0; u < CMB_FLIGHT; u += CMB_GROUP) {
+            if (u < n) {  // (beyond the last split: that one again, dropped below)
+#pragma unroll
+                for (int q = u; q < u + CMB_GROUP; q++) {
+                    const float *src = op + (q < n ? q : n - 1) * step;
+                    v[q] = PAIRS ? part_load2<COHERENT>(src) : f32x2_t{part_load<COHERENT>(src), part_load<COHERENT>(src + 1)};
+                }
+            }
+        }
+    };
+    fetch(0, 0);
     const float mx = wave_max(fmaxf(lv0, lv1));
     const float w0 = mx == -INFINITY ? 0.f : __expf(lv0 - mx), w1 = mx == -INFINITY ? 0.f : __expf(lv1 - mx);  // exp(-inf) = 0 for empty splits
     const float sum = wave_sum(w0 + w1);
-    s_w[lane] = w0;
-    s_w[lane + 64] = w1;
-    __builtin_amdgcn_wave_barrier();  // (the LDS operations of one wave execute in order: the weights are readable below)
     const float inv = sum > 0.f ? 1.f / sum : 0.f;
-    const int b = (int)(row / p.H), h = (int)(row % p.H);
-    for (int e = lane, n = 0; e < p.d; e += 64, n++) {
-        const float *op = op_row + e;
-        float acc = 0.f;
-        int s = 0;
-        if (n < 2) {  // (the splits in ascending order, as everywhere: sums do not depend on how they were fetched)
-#pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (u < n0) acc = fmaf(s_w[u], n == 0 ? v0[u] : v1[u], acc);
-            s = n0;
-        }
-        for (; s + 8 <= p.splits; s += 8) {
-            float v[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = part_load<COHERENT>(op + (int64_t)(s + u) * step);
-#pragma unroll
-            for (int u = 0; u < 8; u++) acc = fmaf(s_w[s + u], v[u], acc);
-        }
-        for (; s < p.splits; s++) acc = fmaf(s_w[s], part_load<COHERENT>(op + (int64_t)s * step), acc);
-        ((uint16_t *)p.o)[b * p.o_b + h * p.o_h + e] = (uint16_t)(E::pack2(acc * inv, 0.f) & 0xffffu);
-    }
     if (lane == 0) p.lse[row] = mx == -INFINITY ? INFINITY : mx + __logf(sum);
-    __builtin_amdgcn_wave_barrier();  // (s_w is rewritten for the wave's next row)
+    f32x2_t acc = {0.f, 0.f};
+    for (int e0 = 0, s0 = 0;;) {
+        const int n = p.splits - s0;
+        const int w = __float_as_int(s0 < 64 ? w0 : w1);
+#pragma unroll
+        for (int u = 0; u < CMB_FLIGHT; u += CMB_GROUP) {  // (the splits in ascending order: sums do not depend on how they were fetched)
+            if (u < n) {
+#pragma unroll
+                for (int q = u; q < u + CMB_GROUP; q++) {
+                    const float wq = __int_as_float(__builtin_amdgcn_readlane(w, (s0 & 63) + q));
+                    acc[0] = fmaf(wq, q < n ? v[q][0] : 0.f, acc[0]);
+                    acc[1] = fmaf(wq, q < n ? v[q][1] : 0.f, acc[1]);
+                }
+            }
+        }
+        s0 += CMB_FLIGHT;
+        if (s0 >= p.splits) {
+            const int e = e0 + 2 * lane;
+            if (e < p.d)  // (rows of whole 16-byte chunks)
+                *(uint32_t *)((uint16_t *)p.o + (row / p.H) * p.o_b + (row % p.H) * p.o_h + e) = E::pack2(acc[0] * inv, acc[1] * inv);
+            e0 += 128;
+            if (e0 >= p.d) break;
+            s0 = 0;
+            acc = f32x2_t{0.f, 0.f};
+        }
+        fetch(e0, s0);
+    }
 }
 
+template <typename T, bool COHERENT>
+__device__ __forceinline__ void combine_row(const FwdParams &p, int64_t row, int lane) {
+    // (the caller's workspace need not be aligned beyond its floats)
+    if (((uintptr_t)p.o_part & 7) == 0) combine_row_as<T, COHERENT, true>(p, row, lane);
+    else combine_row_as<T, COHERENT, false>(p, row, lane);
+}
+
+// LISTS: the caller has handed over the ordered list of kept keys (fdma_kept_keys: the mask builder writes it).  A
+// workgroup then takes its share of the LIST instead of a range of keys and builds nothing: one trip to memory less in a
+// chain of six, and every split has the same number of rows whatever the mask looks like.
+// PERHEAD: mask or bias differ between the query heads of a group, so a lane fetches the mask byte and the
+// bias of its own (key, head) pairs; otherwise one fused value per key serves all columns.
 template <typename T, int D, bool PERHEAD, bool WIDE, bool LISTS>
 __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(const FwdParams p, int keys_per_split) {
     using E = Elem<T>;
@@ -130,7 +157,7 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
     __shared__ int s_wcount[DEC_NJ][4];
     __shared__ float s_m[4][DEC_COLS], s_l[4][DEC_COLS];
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int r = lane & 31, g = lane >> 5;
     const int split = blockIdx.x, b = blockIdx.z;
     const int G = p.H / p.Hk;
@@ -469,7 +496,10 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
         __shared__ int s_last;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (tid == 0) {
+        // (the lane anew, and `wave` a scalar: at head dim 256 the accumulators leave no registers for what lives through the
+        // loop above, and the compiler reloaded such a value there in the lanes of its last condition alone)
+        const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+        if (wave == 0 && ln == 0) {
             int32_t *cnt = p.dec_counter + ((int64_t)b * gridDim.y + blockIdx.y);
             const int old = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const int last = old == p.splits - 1;
@@ -479,7 +509,7 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
         __syncthreads();
         if (s_last) {
             for (int col = wave; col < ncol; col += 4)
-                combine_row<T, true>(p, (int64_t)b * p.H + hk * G + g0 + col, lane, (float *)(smem + wave * 512));
+                combine_row<T, true>(p, (int64_t)b * p.H + hk * G + g0 + col, ln);
         }
     }
 }
@@ -490,10 +520,9 @@ constexpr int CMB_MAX_SPLITS = 128;  // >= the largest number of splits (decode_
 
 template <typename T>
 __global__ void __launch_bounds__(CMB_THREADS) decode_combine_kernel(const FwdParams p) {
-    __shared__ float s_w[CMB_THREADS / 64][CMB_MAX_SPLITS];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * (CMB_THREADS / 64) + wave;
-    if (row < (int64_t)p.B * p.H) combine_row<T, false>(p, row, lane, s_w[wave]);
+    if (row < (int64_t)p.B * p.H) combine_row<T, false>(p, row, lane);
 }
 
 template <typename T, int D, bool PERHEAD, bool WIDE, bool LISTS>
@@ -545,14 +574,26 @@ bool use_decode_path(int Lq, int H, int Hk) {
     return Lq == 1;
 }
 
-// Workgroups have a fixed cost of several microseconds (mask fetch, list, merge), so few fat ones win: two per CU
-// (all resident at once) when a split then still spans 8192 keys, otherwise one per CU; at least 256 keys per
-// split.  With keys_per_split rounded up to 256 every split is non-empty.
+// Workgroups have a fixed cost of several microseconds (mask fetch, list, arrival, merge), so few fat ones win: two per CU
+// (all resident at once) when a split then still spans 8192 keys, otherwise at most one per CU.
+// Few (batch entry, kv head) pairs do not take the whole chip: every split adds some 60 ns of arrival and merge, so there are at
+// most 32, or one for 1024 keys beyond 32768 -- short enough that a mask that keeps (nearly) every key does not lose by it
+// (the host does not know how many are kept; 16 would serve sparse masks best: 16384 keys 9.0, 65536 8.8 us).  us, up to 128
+// splits of 256 keys and a merge of eight at a time -> now, d = 128: 16384 keys x 8 / 4 heads, 1024 kept 15.9 -> 9.7;
+// 65536 x 2 / 1, 512 kept 19.4 -> 11.2; 65536 x 8 / 2, 4096 kept 21.6 -> 12.9; d = 256, 65536 x 2 / 1, 4096 kept 37.2 -> 19.0;
+// all 65536 kept 25.2 -> 21.3, all 16384 15.9 -> 14.2.
+// A split has at least 256 keys; up to 384 keys there is one split, without partial results and merge: 300 keys x 8 / 2,
+// d = 64, 150 kept 8.2 -> 7.1; 384, all kept, d = 128 10.5 -> 9.7 (512 keys, all kept: 10.7 in two, 11.1 in one).
+// With keys_per_split rounded up to 256 every split is non-empty.
 int decode_num_splits(int B, int Hk, int Lk) {
     const int pairs = B * Hk > 0 ? B * Hk : 1;
     int splits = (512 + pairs - 1) / pairs;
-    if ((int64_t)splits * 8192 > Lk) splits = (256 + pairs - 1) / pairs;
-    const int max_by_len = (Lk + 255) / 256;
+    if ((int64_t)splits * 8192 > Lk) {
+        splits = (256 + pairs - 1) / pairs;
+        const int most = Lk > 32768 ? Lk / 1024 : 32;
+        if (splits > most) splits = most;
+    }
+    const int max_by_len = Lk <= 384 ? 1 : (Lk + 255) / 256;
     if (splits > max_by_len) splits = max_by_len;
     if (splits > CMB_MAX_SPLITS) splits = CMB_MAX_SPLITS;
     if (splits < 1) splits = 1;

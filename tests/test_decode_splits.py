@@ -1,0 +1,68 @@
+"""Splits of a single-token call: how many there are, and that their merge -- in the launch itself or in one of its own, up to 32
+splits requested at a time, the workspace aligned for pairs of floats or not -- gives the same bits and the eager restatement's result."""
+import pytest
+import torch
+
+from oracle import eager
+from _util import assert_out_close, make_inputs
+
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("pairs", [(1, 1), (1, 2), (1, 8), (2, 16), (8, 8), (64, 16)])
+def test_no_split_is_empty(pairs):
+    from flash_sparse_attn import _cabi
+
+    B, Hk = pairs
+    a = _cabi.FwdArgs()
+    for Lk in [1, 255, 256, 257, 384, 385, 512, 513, 4093, 8191, 8193, 32768, 32769, 50001, 65536, 131071, 1 << 20]:
+        a.batch, a.seqlen_q, a.seqlen_k, a.num_heads, a.num_heads_k, a.head_dim = B, 1, Lk, Hk, Hk, 64
+        n, rest = divmod(_cabi.lib.fdma_fwd_workspace_bytes(a), (64 + 1) * 4 * B * Hk)
+        assert rest == 0 and n != 1 and n <= 128
+        if n == 0:  # one split: no partial results
+            assert Lk <= 384 or B * Hk >= 256
+            continue
+        span = (-(-Lk // n) + 255) // 256 * 256
+        assert (n - 1) * span < Lk <= n * span
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Lk,H,Hk,D,kept,dtype", [
+    (1, 384, 2, 1, 128, 384, torch.bfloat16),     # the longest call of one split
+    (1, 385, 2, 1, 64, 200, torch.float16),       # the shortest of two
+    (3, 2049, 6, 2, 72, 700, torch.bfloat16),     # 9 splits: a second group; three of four waves merge, a last pair inside the row
+    (1, 8191, 4, 4, 8, 100, torch.bfloat16),      # 32 splits, most of them without a kept key in some rows
+    (1, 33793, 3, 1, 136, 2500, torch.float16),   # 33 splits: a second request; a second round of elements of 8
+    (1, 66000, 2, 1, 256, 1500, torch.bfloat16),  # 64 splits
+    (1, 131000, 1, 1, 64, 5, torch.float16),      # 128 splits, nearly all of them empty
+])
+def test_merge_of_splits(B, Lk, H, Hk, D, kept, dtype):
+    from flash_sparse_attn import _cabi
+    from flash_sparse_attn.flash_sparse_attn_interface import _pad_key_dim
+
+    print("splits", B, Lk, H, Hk, D, kept, dtype, flush=True)
+    q, k, v, mask, bias = [t.to(DEV) for t in make_inputs(B, 1, Lk, H, Hk, D, (B, Hk, 1, Lk), (B, Hk, 1, Lk), kept, seed=Lk + D, dtype=dtype)]
+    ref, ref_lse = eager.attention_forward(q, k, v, mask, bias, None, False)
+    mask, bias = _pad_key_dim(mask, Lk, 16), _pad_key_dim(bias, Lk, 8)
+
+    def call(offset, merged):
+        out, lse = torch.full_like(q, float("nan")), torch.full((B, H, 1), float("nan"), dtype=torch.float32, device=DEV)
+        a = _cabi.FwdArgs()
+        _cabi.fill_fwd(a, q, k, v, mask, bias, out, lse, D ** -0.5, False, 0.0)
+        need, counted = _cabi.lib.fdma_fwd_workspace_bytes(a), _cabi.lib.fdma_fwd_counter_bytes(a)
+        ws = torch.empty(need + 16, dtype=torch.uint8, device=DEV)
+        counters = torch.zeros(counted // 4 + 1, dtype=torch.int32, device=DEV)
+        a.workspace, a.workspace_bytes = ws.data_ptr() + offset, need
+        if merged:
+            a.counters, a.counters_bytes = counters.data_ptr(), counted
+        assert _cabi.lib.fdma_fwd(a, _cabi.current_stream(q.device)) == 0, _cabi.last_error()
+        torch.cuda.synchronize()
+        assert int(counters.abs().max()) == 0
+        return out, lse
+
+    out, lse = call(0, True)
+    assert_out_close(out, ref)
+    assert torch.allclose(lse, ref_lse.reshape(lse.shape), atol=2e-3, rtol=1e-3)
+    for offset, merged in ((0, False), (4, True), (4, False)):
+        again, lse_again = call(offset, merged)
+        assert torch.equal(again, out) and torch.equal(lse_again, lse)
