@@ -5,15 +5,19 @@
 // call, and the same again backwards.  The column-summed dBias that the attention backward returns in the bias's own
 // [B, Hkv, 1, Lk] shape is consumed here directly.
 //
-// Forward: bound by reading V once.  A wave owns 32 tokens and a range of the columns of V_flat; 256 columns at a time (16 KB)
-// go from global memory straight into the wave's own piece of LDS -- whole 512-byte runs of a row per half wave, all of a
-// piece in flight at once, no barrier -- and from there into the A operand of MFMA 32x32x16; W rows, the B operand, come
-// from the caches.  The accumulator column of lane j < Hkv holds dt of 16 of the tokens; it goes through LDS so that softplus
-// is computed by all lanes and the bias rows leave in runs.  (Every lane fetching 16 bytes of its own row per step asked for
-// 32 lines per instruction: 8 x 4093 tokens of 8 x 128, bf16: 23 us, now 16.5 for 67 MB.)
+// Forward: bound by reading V once.  A wave owns 32 tokens and a range of the columns of V_flat; 128 columns at a time (8 KB)
+// go from global memory straight into one of the wave's two pieces of LDS -- whole 256-byte runs of a row per 16 lanes, no
+// barrier, the next piece in flight while one is worked on -- and from there into the A operand of MFMA 32x32x16; W rows, the B
+// operand, come from the caches.  The accumulator column of lane j < Hkv holds dt of 16 of the tokens; it goes through LDS so that
+// softplus is computed by all lanes and the bias rows leave in runs.  (Every lane fetching 16 bytes of its own row per step asked
+// for 32 lines per instruction.  8 x 4093 tokens of 8 x 128, 67 MB, bf16: 23 us that way, 16.7 with one piece of 256 columns that is
+// waited for whole, 14.4 now; 4 x 2304 of 16 x 256, 288 workgroups of eight pieces in a row: 24.7 -> 20.0; 4 x 2048 of 8 x 64
+// 8.0 -> 5.6.)
 // Backward: a workgroup owns a run of tokens; d_dt = dBias * A * sigmoid(dt) goes to LDS, then a thread owns four
 // columns of V_flat and walks the tokens: dV = d_dt W and the workgroup's share of dW = d_dt^T V_flat, dA and dpb, which
 // go to fp32 partials that a second kernel folds in a fixed order (bit-reproducible).
+#include <type_traits>
+
 #include "fdma_common.h"
 #include "fdma_params.h"
 
@@ -25,8 +29,10 @@ __device__ __forceinline__ float sigmoid_f(float x) { return x > 20.f ? 1.f : 1.
 
 // SPLITK: the four waves of a workgroup share 32 tokens, a quarter of the columns each (few tokens: more waves in
 // flight); otherwise every wave owns 32 tokens of its own and reads whole rows.
-constexpr int PC = 256;                       // columns of V_flat per piece
-constexpr int WAVE_LDS = 32 * PC * 2;         // a wave's piece: 32 tokens
+constexpr int PC = 128;                       // columns of V_flat per piece
+constexpr int PIECE_BYTES = 32 * PC * 2;      // of 32 tokens
+constexpr int PIECE_LOADS = PIECE_BYTES / 1024;
+constexpr int WAVE_LDS = 2 * PIECE_BYTES;     // a wave's two pieces
 constexpr int OFF_OUT = 8192;                 // ... reused: accumulators (4 KB), and from here the 16-bit results [head][token]
 constexpr int OUT_PITCH = 34;
 
@@ -54,37 +60,46 @@ __global__ void __launch_bounds__(256) dyn_bias_fwd_kernel(const DynBiasParams p
 #pragma unroll
     for (int i = 0; i < 16; i++) acc[i] = 0.f;
     constexpr int KU = PC / 16;
-    const int n_ks = K / 16, per_wave = SPLITK ? ((n_ks + 3) / 4 + 7) / 8 * 8 : n_ks;
+    const int n_ks = K / 16, per_wave = SPLITK ? ((n_ks + 3) / 4 + KU - 1) / KU * KU : n_ks;
     const int ks_begin = SPLITK ? wave * per_wave : 0;
     const int ks_end = ks_begin + per_wave < n_ks ? ks_begin + per_wave : n_ks;
-    typedef __attribute__((address_space(3))) void lds_void_t;
-    typedef const __attribute__((address_space(1))) void gvoid_t;
-    for (int ks0 = ks_begin; ks0 < ks_end; ks0 += KU) {
-        // direct load i: tokens 2i and 2i + 1 (clamped duplicates beyond the last), lane l the chunk POSITION l % 32 of its
-        // row, which holds chunk position ^ token: reads of one chunk by 16 tokens then fall into 16 different chunks
+    // direct load i of a piece: tokens 4 i .. 4 i + 3 (clamped duplicates beyond the last), lane l the chunk POSITION l % 16 of row
+    // t = 4 i + l / 16, which holds chunk position ^ (t % 16): reads of one chunk by 16 tokens then fall into 16 different chunks
+    const int cpos = lane & 15, tq = lane >> 4;
+    const uint16_t *vrow[PIECE_LOADS];
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int t = 2 * i + g, chunk = r ^ t;
-            int kk = ks0 * 16 + chunk * 8;
-            kk = kk < ks_end * 16 ? kk : ks_begin * 16;  // (past this wave's columns: any of its chunks, never read)
-            int b, l;
-            place(t < n_tok ? t : n_tok - 1, b, l);
-            const int head = p.v_h == p.d ? 0 : kk / p.d;
-            const uint16_t *src = (const uint16_t *)p.v + b * p.v_b + (int64_t)l * p.v_r + (int64_t)head * p.v_h + (kk - head * p.d);
-            __builtin_amdgcn_global_load_lds((gvoid_t *)src, (lds_void_t *)(piece + i * 1024), 16, 0, 0);
-        }
-        u32x4_t bw[KU];
+    for (int i = 0; i < PIECE_LOADS; i++) {
+        int b, l;
+        place(4 * i + tq < n_tok ? 4 * i + tq : n_tok - 1, b, l);
+        vrow[i] = (const uint16_t *)p.v + b * p.v_b + (int64_t)l * p.v_r;
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(piece));
+    // requests piece n of this wave: W's rows first, so that the youngest PIECE_LOADS requests are those of the columns
+    auto fetch = [&](int n, u32x4_t (&bw)[KU]) {
+        const int ks0 = ks_begin + n * KU;
 #pragma unroll
         for (int u = 0; u < KU; u++) {
             const int ks = ks0 + u < ks_end ? ks0 + u : ks_end - 1;  // (a short last piece re-reads the last step and drops it)
             bw[u] = *(const u32x4_t *)(wrow + ks * 16 + 8 * g);
         }
-        __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-        __builtin_amdgcn_wave_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < PIECE_LOADS; i++) {
+            int kk = ks0 * 16 + ((cpos ^ ((4 * i + tq) & 15)) * 8);
+            kk = kk < ks_end * 16 ? kk : ks_begin * 16;  // (past this wave's columns: any of its chunks, never read)
+            const int head = p.v_h == p.d ? 0 : kk / p.d;
+            const uint16_t *src = vrow[i] + (int64_t)head * p.v_h + (kk - head * p.d);
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds0 + (n & 1) * PIECE_BYTES + i * 1024) : "memory");
+        }
+    };
+    // piece n, which has landed
+    auto work = [&](int n, u32x4_t (&bw)[KU]) {
+        const int ks0 = ks_begin + n * KU;
+        const char *base = piece + (n & 1) * PIECE_BYTES + r * (PC * 2);
 #pragma unroll
         for (int u = 0; u < KU; u++) {
             const uint32_t m = (ks0 + u < ks_end) ? wmask : 0u;
-            u32x4_t a = *(const u32x4_t *)(piece + r * 512 + (((2 * u + g) ^ r) << 4));
+            u32x4_t a = *(const u32x4_t *)(base + (((2 * u + g) ^ (r & 15)) << 4));
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 bw[u][e] &= m;
@@ -92,8 +107,42 @@ __global__ void __launch_bounds__(256) dyn_bias_fwd_kernel(const DynBiasParams p
             }
             acc = E::mfma(a, bw[u], acc);
         }
-        __builtin_amdgcn_wave_barrier();
+    };
+    const int n_pieces = ks_begin < ks_end ? (ks_end - ks_begin + KU - 1) / KU : 0;
+    u32x4_t bw0[KU], bw1[KU];
+    // (a piece's successor is requested before it is worked on.  Where the two ways to a wait differ in what is in flight, the compiler
+    // waits for everything: hence no branch inside)
+    auto reads_done = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };  // (of the piece that is overwritten next)
+    auto landed = [&](auto younger) { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(decltype(younger)::value) : "memory"); };
+    constexpr auto one_more = std::integral_constant<int, PIECE_LOADS>();
+    constexpr auto none = std::integral_constant<int, 0>();
+    if (n_pieces > 0) {
+        int n = 0;
+        fetch(0, bw0);
+#pragma unroll 1
+        for (; n + 2 < n_pieces; n += 2) {
+            reads_done();
+            fetch(n + 1, bw1);
+            landed(one_more);
+            work(n, bw0);
+            reads_done();
+            fetch(n + 2, bw0);
+            landed(one_more);
+            work(n + 1, bw1);
+        }
+        if (n + 1 < n_pieces) {
+            reads_done();
+            fetch(n + 1, bw1);
+            landed(one_more);
+            work(n, bw0);
+            landed(none);
+            work(n + 1, bw1);
+        } else {
+            landed(none);
+            work(n, bw0);
+        }
     }
+    __builtin_amdgcn_wave_barrier();
     // ---- dt of (token, head) = the waves' sums in wave order; bias rows through LDS
     if (r < p.Hk) {
 #pragma unroll

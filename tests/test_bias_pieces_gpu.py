@@ -1,0 +1,38 @@
+"""Bias producer forward: pieces of 128 columns, requested one ahead of the one that is worked on.  Waves with no, one, an odd and an
+even number of pieces, a short last piece, short and batch-crossing token tiles, contiguous and gapped heads (the same bits).  Against
+the closed form in 64 bits; the result is rounded to its 16-bit type once."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from flash_sparse_attn.utils.bias import dynamic_mask_bias
+from _util import rel_err
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("B,L,Hk,d,dtype", [
+    (1, 31, 1, 16, torch.bfloat16),      # one step in wave 0, nothing in the others
+    (2, 45, 2, 72, torch.float16),       # a piece, a step, nothing, nothing
+    (1, 33, 4, 128, torch.bfloat16),     # one piece each
+    (3, 50, 5, 112, torch.bfloat16),     # 2, 2, a short one, none
+    (1, 64, 8, 192, torch.float16),      # 3
+    (2, 40, 8, 256, torch.bfloat16),     # 4
+    (1, 70, 20, 256, torch.bfloat16),    # 10
+    (2, 65600, 3, 112, torch.bfloat16),  # a wave has all columns: 2 and a short one
+])
+def test_pieces(B, L, Hk, d, dtype):
+    print("pieces", B, L, Hk, d, dtype, flush=True)
+    g = torch.Generator().manual_seed(L + d)
+    v = torch.randn(B, L, Hk, d, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(Hk, Hk * d, generator=g) / (Hk * d) ** 0.5).to(dtype).to(DEV)
+    a = torch.linspace(0.5, 1.5, Hk).to(dtype).to(DEV)
+    ref = (a.double() * F.softplus(v.double().reshape(B, L, -1) @ w.double().t())).transpose(-1, -2).unsqueeze(-2)
+    gaps = torch.full((B, L, Hk, d + 16), float("nan"), dtype=dtype, device=DEV)  # (what lies between the heads is not read)
+    gaps[..., :d] = v
+    with torch.no_grad():
+        bias, strided = dynamic_mask_bias(v, w, a), dynamic_mask_bias(gaps[..., :d], w, a)
+    torch.cuda.synchronize()
+    assert rel_err(bias, ref) <= 2.0 ** -8
+    assert torch.equal(bias, strided)
