@@ -36,3 +36,24 @@ def test_pieces(B, L, Hk, d, dtype):
     torch.cuda.synchronize()
     assert rel_err(bias, ref) <= 2.0 ** -8
     assert torch.equal(bias, strided)
+
+
+@pytest.mark.parametrize("B,L,Hk,d", [
+    (1, 16385, 1, 16),   # runs of 40 tokens, the last of 25
+    (2, 8990, 3, 48),    # a run across the batch entries
+    (1, 36900, 9, 64),   # 80 tokens: a pass of 64 and one of 16
+])
+def test_gradients_of_long_runs(B, L, Hk, d):
+    """The backward's runs of tokens are whole eights, not whole passes.  Sums over the tokens in fp32, results rounded to 16 bits once."""
+    print("runs", B, L, Hk, d, flush=True)
+    g = torch.Generator().manual_seed(L)
+    v = torch.randn(B, L, Hk, d, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(Hk, Hk * d, generator=g) / (Hk * d) ** 0.5).to(torch.bfloat16).to(DEV)
+    a = torch.linspace(0.5, 1.5, Hk).to(torch.bfloat16).to(DEV)
+    dbias = torch.randn(B, Hk, 1, L, generator=g).to(torch.bfloat16).to(DEV)
+    leaves = [t.requires_grad_(True) for t in (v, w, a)]
+    got = torch.autograd.grad(dynamic_mask_bias(*leaves), leaves, dbias)
+    v64, w64, a64 = wide = [t.detach().double().requires_grad_(True) for t in leaves]
+    ref = (a64 * F.softplus(v64.reshape(B, L, -1) @ w64.t())).transpose(-1, -2).unsqueeze(-2)
+    for x, y in zip(got, torch.autograd.grad(ref, wide, dbias.double())):
+        assert rel_err(x, y) <= 2.0 ** -7
