@@ -577,11 +577,13 @@ bool use_decode_path(int Lq, int H, int Hk) {
 // Workgroups have a fixed cost of several microseconds (mask fetch, list, arrival, merge), so few fat ones win: two per CU
 // (all resident at once) when a split then still spans 8192 keys, otherwise at most one per CU.
 // Few (batch entry, kv head) pairs do not take the whole chip: every split adds some 60 ns of arrival and merge, so there are at
-// most 32, or one for 1024 keys beyond 32768 -- short enough that a mask that keeps (nearly) every key does not lose by it
-// (the host does not know how many are kept; 16 would serve sparse masks best: 16384 keys 9.0, 65536 8.8 us).  us, up to 128
-// splits of 256 keys and a merge of eight at a time -> now, d = 128: 16384 keys x 8 / 4 heads, 1024 kept 15.9 -> 9.7;
-// 65536 x 2 / 1, 512 kept 19.4 -> 11.2; 65536 x 8 / 2, 4096 kept 21.6 -> 12.9; d = 256, 65536 x 2 / 1, 4096 kept 37.2 -> 19.0;
-// all 65536 kept 25.2 -> 21.3, all 16384 15.9 -> 14.2.
+// most 32, or one for 1280 keys beyond 32768 keys.  Sparse masks are served best by few splits, masks that keep every key by
+// many, and the host does not know which it is.  us, spans of 768 / 1024 / 1280 / 2048 keys, one pair of four heads, d = 64 | 128 | 256:
+// 33001 keys, 512 kept 10.4 / 9.6 / 9.2 / 8.8 | 11.0 / 10.0 / 9.7 / 9.3 | 17.6 / 16.4 / 15.3 / 14.6; 65537, 512 kept
+// 13.0 / 11.8 / 10.7 / 9.8 | 13.8 / 12.5 / 11.6 / 10.3 | 23.2 / 20.9 / 18.5 / 16.4; 4096 kept 13.3 / 11.9 / 10.8 / 10.7 | 14.0 / 12.8 /
+// 11.8 / 11.8 | 23.5 / 21.2 / 19.1 / 20.2; all 33001 kept 14.9 / 16.1 / 16.8 / 21.1 | 19.0 / 20.8 / 22.4 / 29.4 | 36.7 / 42.0 / 45.8 / 61.7; all
+// 65537 18.0 / 18.3 / 18.8 / 22.4 | 22.0 / 23.3 / 24.4 / 30.4 | 43.3 / 47.3 / 49.6 / 64.3.  (Up to 128 splits of 256 keys took 15.9 where 32 of
+// 512 take 9.7: 16384 keys x 8 / 4 heads, 1024 kept.)
 // A split has at least 256 keys; up to 384 keys there is one split, without partial results and merge: 300 keys x 8 / 2,
 // d = 64, 150 kept 8.2 -> 7.1; 384, all kept, d = 128 10.5 -> 9.7 (512 keys, all kept: 10.7 in two, 11.1 in one).
 // With keys_per_split rounded up to 256 every split is non-empty.
@@ -590,7 +592,7 @@ int decode_num_splits(int B, int Hk, int Lk) {
     int splits = (512 + pairs - 1) / pairs;
     if ((int64_t)splits * 8192 > Lk) {
         splits = (256 + pairs - 1) / pairs;
-        const int most = Lk > 32768 ? Lk / 1024 : 32;
+        const int most = Lk > 32768 ? (Lk + 1279) / 1280 : 32;
         if (splits > most) splits = most;
     }
     const int max_by_len = Lk <= 384 ? 1 : (Lk + 255) / 256;

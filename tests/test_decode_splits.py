@@ -26,17 +26,31 @@ def test_no_split_is_empty(pairs):
         assert (n - 1) * span < Lk <= n * span
 
 
+@pytest.mark.parametrize("Lk", [32769, 40960, 50001, 65535, 65536, 65537, 131071, 131072])
+def test_spans_of_long_caches(Lk):
+    """One pair's splits beyond 32768 keys span 1280 keys whatever the length is a multiple of."""
+    from flash_sparse_attn import _cabi
+
+    a = _cabi.FwdArgs()
+    a.batch, a.seqlen_q, a.seqlen_k, a.num_heads, a.num_heads_k, a.head_dim = 1, 1, Lk, 2, 1, 64
+    assert _cabi.lib.fdma_fwd_workspace_bytes(a) == -(-Lk // 1280) * (64 + 1) * 4 * 2
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,Lk,H,Hk,D,kept,dtype", [
-    (1, 384, 2, 1, 128, 384, torch.bfloat16),     # the longest call of one split
-    (1, 385, 2, 1, 64, 200, torch.float16),       # the shortest of two
-    (3, 2049, 6, 2, 72, 700, torch.bfloat16),     # 9 splits: a second group; three of four waves merge, a last pair inside the row
-    (1, 8191, 4, 4, 8, 100, torch.bfloat16),      # 32 splits, most of them without a kept key in some rows
-    (1, 33793, 3, 1, 136, 2500, torch.float16),   # 33 splits: a second request; a second round of elements of 8
-    (1, 66000, 2, 1, 256, 1500, torch.bfloat16),  # 64 splits
-    (1, 131000, 1, 1, 64, 5, torch.float16),      # 128 splits, nearly all of them empty
+@pytest.mark.parametrize("B,Lk,H,Hk,D,kept,splits,dtype", [
+    (1, 384, 2, 1, 128, 384, 1, torch.bfloat16),     # the longest call of one split
+    (1, 385, 2, 1, 64, 200, 2, torch.float16),       # the shortest of two
+    (3, 2049, 6, 2, 72, 700, 9, torch.bfloat16),     # a second group; three of four waves merge, a last pair inside the row
+    (1, 33793, 3, 1, 136, 2500, 27, torch.float16),  # a second round of elements of 8
+    (1, 8191, 4, 4, 8, 100, 32, torch.bfloat16),     # one request whole; most splits without a kept key in some rows
+    (1, 41000, 3, 1, 136, 2500, 33, torch.float16),  # a second request of one split, in both rounds of elements
+    (1, 66000, 2, 1, 256, 1500, 52, torch.bfloat16),
+    (1, 81920, 2, 1, 256, 1500, 64, torch.bfloat16),  # the last lane of the first weights
+    (1, 81921, 2, 1, 72, 900, 65, torch.float16),    # the first of the second
+    (1, 131000, 1, 1, 64, 5, 103, torch.float16),    # nearly all of them empty
+    (1, 163840, 1, 1, 64, 4000, 128, torch.bfloat16),  # as many as there are
 ])
-def test_merge_of_splits(B, Lk, H, Hk, D, kept, dtype):
+def test_merge_of_splits(B, Lk, H, Hk, D, kept, splits, dtype):
     from flash_sparse_attn import _cabi
     from flash_sparse_attn.flash_sparse_attn_interface import _pad_key_dim
 
@@ -50,6 +64,7 @@ def test_merge_of_splits(B, Lk, H, Hk, D, kept, dtype):
         a = _cabi.FwdArgs()
         _cabi.fill_fwd(a, q, k, v, mask, bias, out, lse, D ** -0.5, False, 0.0)
         need, counted = _cabi.lib.fdma_fwd_workspace_bytes(a), _cabi.lib.fdma_fwd_counter_bytes(a)
+        assert need == (splits * (D + 1) * 4 * B * H if splits > 1 else 0)
         ws = torch.empty(need + 16, dtype=torch.uint8, device=DEV)
         counters = torch.zeros(counted // 4 + 1, dtype=torch.int32, device=DEV)
         a.workspace, a.workspace_bytes = ws.data_ptr() + offset, need
