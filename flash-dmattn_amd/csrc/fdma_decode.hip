@@ -38,7 +38,9 @@ template <int D> struct DecSmem {
     static constexpr int TILE_BYTES = DEC_TILE * S * 2;
     static constexpr int WAVE_BYTES = 2 * TILE_BYTES + DEC_TILE * 4;  // K rows, V rows, fused bias
     static constexpr int OFF_IDX = 4 * WAVE_BYTES;
-    static constexpr int TOTAL = OFF_IDX + DEC_RANGE * 2;
+    static constexpr bool Q_LDS = D > 128;  // the Q fragments are kept here, see decode_kernel
+    static constexpr int OFF_Q = OFF_IDX + DEC_RANGE * 2;
+    static constexpr int TOTAL = OFF_Q + (Q_LDS ? D / 16 * 1024 : 0);
     static constexpr int SO = D + 4;  // row stride of a wave's partial output in floats (rows fall into different banks)
     static_assert(DEC_COLS * SO * 4 <= WAVE_BYTES, "a wave's partial output must fit its own piece");
 };
@@ -189,13 +191,18 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
     }
 
     // B operands of S^T = K Q^T: lane supplies Q[head r][16 ks + 8 g .. + 7]; columns without a head are zero
-    u32x4_t qf[KS];
+    // (d > 128: in LDS, the same for all waves and a quarter made by each; the barriers in front of a list's first batch publish
+    // them.  In registers, beside the accumulators and a batch of rows in flight, they cost 6 to 40 registers spilled to scratch:
+    // d = 256, us, 16384 keys x 16 / 4 heads, 4096 kept 20.8 -> 20.1, all kept 30.4 -> 29.2; 65537 x 2 / 1 all kept 48.0 -> 46.4.)
+    u32x4_t qf[SM::Q_LDS ? 1 : KS];
     {
         const uint16_t *qp = (const uint16_t *)p.q + b * p.q_b + (int64_t)h * p.q_h;
+        auto q_frag = [&](int ks) { return col_ok && 2 * ks + g < nchunk ? *(const u32x4_t *)(qp + 16 * ks + 8 * g) : u32x4_t{0, 0, 0, 0}; };
+        if constexpr (SM::Q_LDS) {
+            for (int ks = wave; ks < KS; ks += 4) *(u32x4_t *)(smem + SM::OFF_Q + (ks * 64 + lane) * 16) = q_frag(ks);
+        } else {
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            qf[ks] = u32x4_t{0, 0, 0, 0};
-            if (col_ok && 2 * ks + g < nchunk) qf[ks] = *(const u32x4_t *)(qp + 16 * ks + 8 * g);
+            for (int ks = 0; ks < KS; ks++) qf[ks] = q_frag(ks);
         }
     }
     const int hm = p.Hm == p.H ? h : (p.Hm == 1 ? 0 : hk);
@@ -354,7 +361,7 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
 #pragma unroll
                 for (int ks = 0; ks < KS; ks++) {
                     const u32x4_t a = *(const u32x4_t *)(sK + a_off + ks * 32);
-                    s = E::mfma(a, qf[ks], s);
+                    s = E::mfma(a, SM::Q_LDS ? *(const u32x4_t *)(smem + SM::OFF_Q + (ks * 64 + lane) * 16) : qf[SM::Q_LDS ? 0 : ks], s);
                 }
                 if (!PERHEAD) {
 #pragma unroll
@@ -496,10 +503,7 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
         __shared__ int s_last;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        // (the lane anew, and `wave` a scalar: at head dim 256 the accumulators leave no registers for what lives through the
-        // loop above, and the compiler reloaded such a value there in the lanes of its last condition alone)
-        const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
-        if (wave == 0 && ln == 0) {
+        if (tid == 0) {
             int32_t *cnt = p.dec_counter + ((int64_t)b * gridDim.y + blockIdx.y);
             const int old = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const int last = old == p.splits - 1;
@@ -509,7 +513,7 @@ __global__ void __launch_bounds__(DEC_THREADS, D <= 128 ? 2 : 1) decode_kernel(c
         __syncthreads();
         if (s_last) {
             for (int col = wave; col < ncol; col += 4)
-                combine_row<T, true>(p, (int64_t)b * p.H + hk * G + g0 + col, ln);
+                combine_row<T, true>(p, (int64_t)b * p.H + hk * G + g0 + col, lane);
         }
     }
 }

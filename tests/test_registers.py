@@ -1,0 +1,28 @@
+"""What the compiler says of the kernels' registers, read from the metadata that the built library carries beside them."""
+import os
+
+import pytest
+
+msgpack = pytest.importorskip("msgpack")
+LIB = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "flash-dmattn_amd", "lib", "libfdma_hip.so")
+
+
+def kernels():
+    data, key, found = open(LIB, "rb").read(), b"\xaeamdhsa.kernels", {}
+    at = data.find(key)
+    while at >= 0:
+        unpacker = msgpack.Unpacker(strict_map_key=False)
+        unpacker.feed(data[at - 1:at + (1 << 20)])  # (a map of a few entries starts with one byte)
+        for k in unpacker.unpack()["amdhsa.kernels"]:
+            found[k[".name"]] = k
+        at = data.find(key, at + 1)
+    return found
+
+
+def test_decode_holds_its_state_in_registers():
+    """No lane's state of the decode kernels goes through scratch memory: what was reloaded from there behind the loop over the keys had
+    come back in some of the lanes only."""
+    decode = {n: k for n, k in kernels().items() if "decode_kernel" in n}
+    assert len(decode) == 2 * 3 * 6
+    for name, k in decode.items():
+        assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0, name
