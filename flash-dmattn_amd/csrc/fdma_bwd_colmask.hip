@@ -814,7 +814,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
         // some workgroups sum partial results of the dK/dV kernel instead
         const int at = lid - p.red_first;
         if (at >= 0 && at < p.red_count) {
-            dkdv_reduce_blocks<T, D>(p, at, p.red_count, threadIdx.x, (float *)smem);
+            dkdv_reduce_blocks<T, D>(kernel_args_apart<BwdParams>(), at, p.red_count, threadIdx.x, (float *)smem);
             return;
         }
         if (at >= 0) lid -= p.red_count;

@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
     if (CMP) {  // some workgroups sum partial results of the dK/dV kernel instead (see place_reduction, fdma_bwd_colmask.hip)
         const int at = lid - p.red_first;
         if (at >= 0 && at < p.red_count) {
-            dkdv_reduce_blocks<T, D>(p, at * 2 + (wave >> 2), p.red_count * 2, tid & 255, (float *)(smem + (wave >> 2) * RED_LDS));
+            dkdv_reduce_blocks<T, D>(kernel_args_apart<BwdParams>(), at * 2 + (wave >> 2), p.red_count * 2, tid & 255, (float *)(smem + (wave >> 2) * RED_LDS));
             return;
         }
         if (at >= 0) lid -= p.red_count;

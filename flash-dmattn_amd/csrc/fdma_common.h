@@ -175,6 +175,16 @@ __device__ __forceinline__ gptr_t uniform_ptr(const void *ptr) {
     return (gptr_t)(((uint64_t)hi << 32) | lo);
 }
 
+// The running kernel's first argument, a struct, read where the launch left it through a pointer that the compiler cannot follow: what
+// a branch of its own (another job of the same launch) loads of it is not held in scalar registers by the rest of the kernel, nor the
+// other way round.
+template <typename P> __device__ __forceinline__ const P &kernel_args_apart() {
+    typedef const __attribute__((address_space(4))) P *args_t;
+    args_t args = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    return *(const P *)args;
+}
+
 // Direct loads: every lane's 16 or 4 bytes at `base` + off go to LDS, lane after lane from address `dst` on (both the same for all lanes).
 // In assembly, because behind the compiler's builtin every LDS read waits for all LDS operations in flight.  So the compiler
 // neither waits for them nor knows that they write LDS: a kernel waits by hand (s_waitcnt vmcnt) in front of the barrier that publishes

@@ -26,3 +26,11 @@ def test_decode_holds_its_state_in_registers():
     assert len(decode) == 2 * 3 * 6
     for name, k in decode.items():
         assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0, name
+
+
+def test_sums_of_parts_stay_apart_from_dq():
+    """The compacted dQ kernels carry the sums of the dK / dV parts; neither holds the other's scalars."""
+    dq = {n: k for n, k in kernels().items() if "bwd_dq_256_kernel" in n and "ELb1EEE" in n or "bwd_dq_colmask_kernel" in n and "ELb1ELb0EEE" in n}
+    assert len(dq) == 2 * (2 + 4)
+    for name, k in dq.items():
+        assert k[".sgpr_spill_count"] == 0 and k[".vgpr_spill_count"] == 0, name
