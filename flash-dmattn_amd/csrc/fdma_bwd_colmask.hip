@@ -697,26 +697,6 @@ __global__ void __launch_bounds__(NTHREADS) bwd_dkdv_parts_sum_kernel(const BwdP
     }
 }
 
-// The dQ launch of a compacted backward carries the reduction of the dK/dV partials along: `red_count` consecutive workgroups
-// (a multiple of 8) do that instead of dQ work.  They only move memory, so side by side with dQ workgroups, which keep the matrix
-// units busy, they cost little; as a launch of its own the reduction took as long as its memory traffic.
-// One to a CU, in front of all others: they are done early, and the dQ workgroups then start heaviest first as if they were
-// alone.  Spread through the launch instead, one beside three dQ workgroups, they kept those from their CUs (half of the CUs' time
-// was idle).  Spread / in front (us, the whole step): 4 x 2048 tokens, 16/8 heads, d = 64 with its layer 174 / 165; 8192 x 8/4, d = 64
-// 117 / 104; d = 128: 8192 x 32/8 724 / 718, 2048 x 32/8 126 / 117, 4096 x 16/4 164 / 149, 2 x 4096 x 8/2 132 / 119, 12000 x 8/2 263 / 240;
-// half as many 0.95 to 1.16 times that, twice as many the same.
-// Few query rows against many keys are the other way round: few dQ workgroups, which leave CUs free, and partials by the number
-// of keys.  All that the items ask for then follow the dQ workgroups.  100 rows of 16 heads over 2048 kept keys, d = 128 (16 dQ
-// workgroups): the launch 361 us with 16 summing workgroups, 54 with 1024.  Up to half a dQ workgroup per CU, or one where the keys
-// are more than twice the rows: behind / in front (us, the step) 1300 rows x 16/4 heads over 1500 kept of 4000, d = 128 133.5 / 135.4;
-// 4096 x 8/2, all 4096 keys to choose from, 124 / 121 at d = 128, 98.6 / 96.1 at 64.
-inline void place_reduction(BwdParams &p, int n_dq, int items) {
-    const bool few = (p.f.Lk > 2 * p.f.Lq ? 1 : 2) * n_dq <= device_cus();
-    const int most = few ? 1024 : device_cus();
-    p.red_count = ((items < most ? items : most) + 7) / 8 * 8;
-    p.red_first = few ? n_dq : 0;
-}
-
 template <typename T, int D, bool CAUSAL, bool CMP>
 hipError_t launch_dkdv_grid(const BwdParams &p, int grid, hipStream_t stream) {
     if constexpr (D > 128) {
@@ -1280,13 +1260,33 @@ hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
     const FwdParams &f = p.f;
     BwdParams pr = p;
     const int n_dq = row_grid(pr.f, Q_BM);  // a multiple of 8
-    if (!f.cmp.on) return launch_dq_grid<T, D, CAUSAL>(pr, n_dq, stream);
-    const int units_max = f.B * f.Hk * ((f.Lk + KV_BN - 1) / KV_BN);
-    place_reduction(pr, n_dq, units_max * (f.d / 4 + (f.bias ? 1 : 0)));
-    return launch_dq_grid<T, D, CAUSAL>(pr, n_dq + pr.red_count, stream);
+    return launch_dq_grid<T, D, CAUSAL>(pr, n_dq + (f.cmp.on ? pr.red_count : 0), stream);
 }
 
 }  // namespace
+
+// The dQ launch of a compacted backward carries the reduction of the dK/dV partials along: `red_count` consecutive workgroups
+// (a multiple of 8) do that instead of dQ work.  They only move memory, so side by side with dQ workgroups, which keep the matrix
+// units busy, they cost little; as a launch of its own the reduction took as long as its memory traffic.
+// One to a CU, in front of all others: they are done early, and the dQ workgroups then start heaviest first as if they were
+// alone.  Spread through the launch instead, one beside three dQ workgroups, they kept those from their CUs (half of the CUs' time
+// was idle).  Spread / in front (us, the whole step): 4 x 2048 tokens, 16/8 heads, d = 64 with its layer 174 / 165; 8192 x 8/4, d = 64
+// 117 / 104; d = 128: 8192 x 32/8 724 / 718, 2048 x 32/8 126 / 117, 4096 x 16/4 164 / 149, 2 x 4096 x 8/2 132 / 119, 12000 x 8/2 263 / 240;
+// half as many 0.95 to 1.16 times that, twice as many the same.
+// Few query rows against many keys are the other way round: few dQ workgroups, which leave CUs free, and partials by the number
+// of keys.  All that the items ask for then follow the dQ workgroups.  100 rows of 16 heads over 2048 kept keys, d = 128 (16 dQ
+// workgroups): the launch 361 us with 16 summing workgroups, 54 with 1024.  Up to half a dQ workgroup per CU, or one where the keys
+// are more than twice the rows: behind / in front (us, the step) 1300 rows x 16/4 heads over 1500 kept of 4000, d = 128 133.5 / 135.4;
+// 4096 x 8/2, all 4096 keys to choose from, 124 / 121 at d = 128, 98.6 / 96.1 at 64.
+void place_reduction(BwdParams &p) {
+    FwdParams f = p.f;
+    const int n_dq = row_grid(f, Q_BM), items = f.B * f.Hk * ((f.Lk + KV_BN - 1) / KV_BN) * (f.d / 4 + (f.bias ? 1 : 0));
+    const bool few = (f.Lk > 2 * f.Lq ? 1 : 2) * n_dq <= device_cus();
+    const int most = few ? 1024 : device_cus();
+    p.red_count = ((items < most ? items : most) + 7) / 8 * 8;
+    p.red_first = few ? n_dq : 0;
+    p.red_light = n_dq <= device_cus();
+}
 
 bool bwd_colmask_applicable(const BwdParams &p) {
     const bool mask_ok = !p.f.mask || p.f.m_r == 0;

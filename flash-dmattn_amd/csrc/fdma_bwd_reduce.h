@@ -100,15 +100,19 @@ __device__ __forceinline__ void dkdv_reduce_item(const BwdParams &p, const int u
         } else if (half == 0) {
             float tot = start;
             const int n = Gs * n_seg * gper;
+            int gs = 0, sg = 0, gl = 0;  // of the next column: group of heads, segment, local head
             for (int j = 0; j < n; j += 8) {
                 float v[8];
 #pragma unroll
                 for (int t = 0; t < 8; t++) {
-                    const int jt = j + t < n ? j + t : n - 1, pt = jt / gper;
-                    v[t] = dbp[((int64_t)(pt / n_seg * Sm + pt % n_seg) * G + jt % gper) * KV_BN];
+                    v[t] = j + t < n ? dbp[((int64_t)(gs * Sm + sg) * G + gl) * KV_BN] : 0.f;
+                    if (++gl == gper) {
+                        gl = 0;
+                        if (++sg == n_seg) { sg = 0; gs++; }
+                    }
                 }
 #pragma unroll
-                for (int t = 0; t < 8; t++) tot += j + t < n ? v[t] : 0.f;
+                for (int t = 0; t < 8; t++) tot += v[t];
             }
             emit(f.Hb == 1 ? 0 : hk, tot);
         }
@@ -150,11 +154,15 @@ __device__ __forceinline__ void dkdv_reduce_rows(const float *base, const int n_
 // order, and writes dK (scaled), dV and dBias to the original rows / columns of the kept keys.  Called by the workgroups that the
 // dQ launch sets aside for it: share `rb` of `nrb`.  All threads of the workgroup call it together (it has barriers); `lds`:
 // RED_LDS bytes of this share's own.
-// Many units, hence few slots each: items of 16 columns of dK and dV, 64 loads in flight per thread and no barrier (bound by
-// memory).  Few units: a unit has up to 64 slots, and a thread that walks them waits for memory again and again on few CUs
-// (3968 tokens x 8/2 heads, d = 64, 320 kept: 6 units, 24 items, and their dBias slot by slot, 46 us the launch, 13.7 now).  There
+// Items of 16 columns of dK and dV: 64 loads in flight per thread and no barrier (bound by memory).  But a unit has up to 16 slots per
+// query head of its group, and a thread that walks them waits for memory again and again on few CUs (3968 tokens x 8/2 heads, d = 64, 320
+// kept: 6 units, 24 items, and their dBias slot by slot, 46 us the launch, 13.7 now).  Where that is longer than dQ beside it (plan[7]),
 // an item is eight columns of dK or of dV, or dBias, the slots are spread over the threads, and the sums are added up through LDS.
-// (For few slots that is a little behind, a third as many bytes being in flight: 4 x 2048 x 16/8 heads 43.6 against 40.6 us.)
+// That keeps a third as many bytes in flight and more workgroups busy.  One thread / side by side, the dQ launch of 2048 tokens (us):
+// d = 64: 16/8 heads, 256 kept 23.8 / 12.8, 16/4, 640 kept 21.6 / 19.1, 2 x 16/8, 384 kept 19.6 / 21.4, 4 x 16/8, 384 kept 31.4 / 33.7, 6 x 16/8, 640
+// kept 40.6 / 43.5; d = 128: 16/4, 384 kept 28.4 / 21.8, 32/8, 384 kept 28.1 / 29.9; d = 256: 8/2, 100 kept 30.6 / 18.3, 16/8, 384 kept 37.4 /
+// 39.2, 2 x 16/8, 640 kept 83.8 / 95.7.  Of 815 calls the rule of sums_by_chains costs more than 3 % over the better way on 60; all the one way
+// 250, all the other 110, by the number of units alone 130.
 template <typename T, int D>
 __device__ __forceinline__ void dkdv_reduce_blocks(const BwdParams &p, const int rb, const int nrb, const int tid, float *lds) {
     using E = Elem<T>;
@@ -162,14 +170,19 @@ __device__ __forceinline__ void dkdv_reduce_blocks(const BwdParams &p, const int
     const int32_t *plan = f.cmp.plan;
     const int U = plan[0], Gs = plan[1], Sm = plan[2], Q = plan[4], per = Gs * Sm;
     if (per == 1) return;  // no unit was split: the dK/dV kernel wrote the results itself
-    // a plan whose lists overflowed left parts uncomputed: every sum starts from NaN then
-    const float start = plan[6] != 0 ? __builtin_nanf("") : 0.f;
-    const int G = f.H / f.Hk, gper = G / Gs;
-    if (U >= 64 && U * (D / 16) >= 2 * nrb) {
+    if (!plan[7]) {
         for (int item = rb; item < U * (D / 16); item += nrb) dkdv_reduce_item<T, D>(p, item / (D / 16), item % (D / 16), tid);
         return;
     }
-    const int n_ch = (f.d + 7) / 8, ipu = 2 * n_ch + (f.bias ? 1 : 0);  // items per unit
+    // a plan whose lists overflowed left parts uncomputed: every sum starts from NaN then
+    const float start = plan[6] != 0 ? __builtin_nanf("") : 0.f;
+    // (what the items need of the launch's arguments is read here, and what their results need at the head of an item: read where it is
+    // used, behind barriers, it was a trip to memory each time)
+    const int Hk = f.Hk, G = f.H / Hk, gper = G / Gs, n_pairs = f.B * Hk, Lq = f.Lq, Lk = f.Lk, causal = f.causal, ld = f.cmp.ld;
+    const int32_t *idx0 = f.cmp.idx, *counts = f.cmp.count;
+    const float *dkv_part = p.dkv_part, *db_part = p.db_part;
+    const bool with_bias = f.bias != nullptr, per_head = f.Hb == f.H, one_row = f.Hb == 1;
+    const int n_ch = (f.d + 7) / 8, ipu = 2 * n_ch + (with_bias ? 1 : 0);  // items per unit
     const int total = U * ipu, share = (total + nrb - 1) / nrb;
     const int kk = tid >> 1, hf = tid & 1;  // the key, and half of the eight columns, that this thread writes
     int unit = -1, b = 0, hk = 0, n_seg = 1, okey = 0;
@@ -179,27 +192,30 @@ __device__ __forceinline__ void dkdv_reduce_blocks(const BwdParams &p, const int
         const bool ok = item < total;
         if (ok && item / ipu != unit) {
             unit = item / ipu;
-            int lo = 0, hi = f.B * f.Hk;
+            int lo = 0, hi = n_pairs;
             while (hi - lo > 1) {
                 const int mid = (lo + hi) >> 1;
                 if (plan[DKDV_PLAN_HDR + mid] <= unit) lo = mid;
                 else hi = mid;
             }
-            b = lo / f.Hk;
-            hk = lo % f.Hk;
+            b = lo / Hk;
+            hk = lo % Hk;
             const int n0 = (unit - plan[DKDV_PLAN_HDR + lo]) * KV_BN;
-            const int32_t *idx = f.cmp.idx + (int64_t)lo * f.cmp.ld + n0;
-            live = n0 + kk < f.cmp.count[lo];
+            const int32_t *idx = idx0 + (int64_t)lo * ld + n0;
+            live = n0 + kk < counts[lo];
             okey = live ? idx[kk] : 0;
             // segments of this unit that were written (same rule as in the main kernel)
-            n_seg = dkdv_segments(dkdv_query_blocks(f.Lq, f.Lk, f.causal, idx[0]), Q, Sm);
+            n_seg = dkdv_segments(dkdv_query_blocks(Lq, Lk, causal, idx[0]), Q, Sm);
         }
         const int n_w = Gs * n_seg, mat = y >= n_ch ? 1 : 0, c = y - mat * n_ch;
-        const bool cols = y == 2 * n_ch, per_head = f.Hb == f.H;
+        const bool cols = y == 2 * n_ch;
         const int slots = n_w >= 16 ? 8 : (n_w >= 8 ? 4 : (n_w >= 4 ? 2 : 1));
-        const float *dbp = f.bias ? p.db_part + (int64_t)unit * per * G * KV_BN : nullptr;  // [part][local head][key]
+        const float *dbp = db_part + (int64_t)unit * per * G * KV_BN;  // [part][local head][key]
+        uint16_t *dst = mat == 0 ? (uint16_t *)p.dk + b * p.dk_b + hk * p.dk_h : (uint16_t *)p.dv + b * p.dv_b + hk * p.dv_h;
+        const int64_t dst_r = mat == 0 ? p.dk_r : p.dv_r;
+        const float m = mat == 0 ? f.scale : 1.f;
         if (ok && !cols) {
-            const float *base = p.dkv_part + ((int64_t)unit * per * 2 * D + mat * D + c * 8) * KV_BN;
+            const float *base = dkv_part + ((int64_t)unit * per * 2 * D + mat * D + c * 8) * KV_BN;
             if (slots == 8) dkdv_reduce_rows<8, D>(base, n_w, n_seg, Sm, tid, lds);
             else if (slots == 4) dkdv_reduce_rows<4, D>(base, n_w, n_seg, Sm, tid, lds);
             else if (slots == 2) dkdv_reduce_rows<2, D>(base, n_w, n_seg, Sm, tid, lds);
@@ -232,10 +248,7 @@ __device__ __forceinline__ void dkdv_reduce_blocks(const BwdParams &p, const int
             for (int s = 0; s < slots; s++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) a[e] += lds[(s * 8 + 4 * hf + e) * RED_PITCH + kk];
-            const float m = mat == 0 ? f.scale : 1.f;
-            uint16_t *dst = mat == 0 ? (uint16_t *)p.dk + b * p.dk_b + (int64_t)okey * p.dk_r + hk * p.dk_h
-                                     : (uint16_t *)p.dv + b * p.dv_b + (int64_t)okey * p.dv_r + hk * p.dv_h;
-            *(u32x2_t *)(dst + c * 8 + 4 * hf) = u32x2_t{E::pack2(a[0] * m, a[1] * m), E::pack2(a[2] * m, a[3] * m)};
+            *(u32x2_t *)(dst + (int64_t)okey * dst_r + c * 8 + 4 * hf) = u32x2_t{E::pack2(a[0] * m, a[1] * m), E::pack2(a[2] * m, a[3] * m)};
         } else if (ok && live && per_head) {
             for (int gi = hf; gi < G; gi += 2) {
                 float tot = start;
@@ -247,7 +260,7 @@ __device__ __forceinline__ void dkdv_reduce_blocks(const BwdParams &p, const int
             float tot = start;
 #pragma unroll
             for (int s = 0; s < 8; s++) tot += lds[s * RED_PITCH + kk];
-            emit(f.Hb == 1 ? 0 : hk, tot);
+            emit(one_row ? 0 : hk, tot);
         }
         __syncthreads();
     }

@@ -52,7 +52,7 @@ constexpr int IMG_X_BYTES = IMG_BN * 32;                  // 2048
 // under a causal mask, and the fold gives every list the same mix of heavy and light units.
 //   plan[0] = U, plan[1] = Gs, plan[2] = Sm (segment slots per unit and head group), plan[3] = list length
 //   bound (units), plan[4] = Q, plan[5] = where the lists begin, plan[6] = 1 when a per-XCD list overflowed (the
-//   reduce kernel then writes NaN gradients), plan[8 + i] = first unit of pair i (i = 0..pairs)
+//   reduce kernel then writes NaN gradients), plan[7] = how the parts are summed (sums_by_chains), plan[8 + i] = first unit of pair i (i = 0..pairs)
 constexpr int DKDV_PLAN_HDR = 8;
 #ifndef FDMA_DKDV_TARGET
 #define FDMA_DKDV_TARGET 768
@@ -70,6 +70,16 @@ __host__ __device__ inline void dkdv_split(int U, int G, int &Gs, int &Sm) {
         Sm = 2 * want / G;
         Sm = Sm < 1 ? 1 : (Sm > 16 ? 16 : Sm);
     }
+}
+// How the parts of the units are summed (plan[7], see dkdv_reduce_blocks): by several chains of loads side by side, or every sum by
+// one thread, whose trips to memory for four slots follow each other.  `nwg`: workgroups (halves of one at head dims above 128) that
+// sum; light: beside at most one dQ workgroup per CU.  One thread is enough while its trips hide behind the longest row
+// block's own chain of key tiles, which takes 1.2 / 1.4 / 3 trips' time (1.9 us) per unit of a pair at d = 64 / 128 / 256 (head dims in between: the next
+// larger), about twice that where further dQ workgroups wait for the CU.
+__host__ __device__ inline bool sums_by_chains(int U, int per, int pairs, int d, int nwg, bool light) {
+    const int dpad = d <= 64 ? 64 : (d <= 128 ? 128 : 256), trips = (U * (dpad / 16) + nwg - 1) / nwg * ((per + 3) / 4);
+    const float per_unit = light ? (d <= 64 ? 0.8f : (d <= 128 ? 1.2f : 2.f)) : (d <= 64 ? 2.f : 4.f);
+    return (float)trips > 2.f + per_unit * (float)U / (float)pairs;
 }
 // query blocks (of 64 rows) that see a key block whose first key sits at original column `okey_first`
 __host__ __device__ inline int dkdv_query_blocks(int Lq, int Lk, int causal, int okey_first) {
@@ -310,7 +320,8 @@ struct BwdParams {
     // register order) in dkv_part and [G][128] fp32 (dBias columns) in db_part
     int32_t kv_most, kv_quota, kv_units;
     int32_t dot_done;          // softmax_d has been computed by an earlier launch of this call
-    int32_t red_first, red_count;  // compacted backward: workgroups of the dQ launch that sum the dK/dV partials (set by that launch)
+    int32_t red_first, red_count;  // compacted backward: workgroups of the dQ launch that sum the dK/dV partials (see place_reduction)
+    int32_t red_light;             // ... beside at most one that works on dQ per CU
 };
 
 // Keep-mask builder (fdma_mask.hip): one row of `Lk` 16-bit bias values per (batch, head, row).
@@ -404,6 +415,7 @@ hipError_t launch_bwd(const BwdParams &p, int dtype, hipStream_t stream);
 bool bwd_colmask_applicable(const BwdParams &p);
 hipError_t launch_bwd_dkdv_colmask(const BwdParams &p, int dtype, hipStream_t stream);
 hipError_t launch_bwd_dkdv_256(const BwdParams &p, int dtype, int grid, hipStream_t stream);  // its kernel at head dims 129 .. 256 (fdma_bwd_dkdv_256.hip)
+void place_reduction(BwdParams &p);  // compacted: which workgroups of the dQ launch sum the dK/dV partials
 hipError_t launch_bwd_dq_colmask(const BwdParams &p, int dtype, hipStream_t stream);
 hipError_t launch_bwd_dq_256(const BwdParams &p, int dtype, int grid, hipStream_t stream);  // its kernel at head dims 129 .. 256 (fdma_bwd_dq_256.hip)
 // parts the units of the dK/dV kernel on the original key axis are cut into: fills kv_most / kv_quota / kv_units and returns the
