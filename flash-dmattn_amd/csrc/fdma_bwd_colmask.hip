@@ -1273,6 +1273,10 @@ hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
 // was idle).  Spread / in front (us, the whole step): 4 x 2048 tokens, 16/8 heads, d = 64 with its layer 174 / 165; 8192 x 8/4, d = 64
 // 117 / 104; d = 128: 8192 x 32/8 724 / 718, 2048 x 32/8 126 / 117, 4096 x 16/4 164 / 149, 2 x 4096 x 8/2 132 / 119, 12000 x 8/2 263 / 240;
 // half as many 0.95 to 1.16 times that, twice as many the same.
+// Above head dim 128 a CU holds one workgroup of the launch: a quarter of the CUs is left to the heaviest dQ workgroups from the
+// start.  All CUs / three quarters / half of them summing, the dQ launch, d = 256 (us): 3001 x 8/4 73.0 / 60.6 / 59.4, 2048 x 16/8, 1000 kept
+// 78.4 / 64.3 / 62.0, 1300 x 16/8 52.3 / 47.2 / 44.0, 5000 x 16/4 82.0 / 81.5 / 81.8, 2 x 2048 x 16/8, 1500 kept 170 / 168 / 180; not causal 1300 x
+// 16/8 65.0 / 63.7 / 69.1, 3001 x 8/4 82.1 / 75.8 / 82.2.
 // Few query rows against many keys are the other way round: few dQ workgroups, which leave CUs free, and partials by the number
 // of keys.  All that the items ask for then follow the dQ workgroups.  100 rows of 16 heads over 2048 kept keys, d = 128 (16 dQ
 // workgroups): the launch 361 us with 16 summing workgroups, 54 with 1024.  Up to half a dQ workgroup per CU, or one where the keys
@@ -1282,7 +1286,7 @@ void place_reduction(BwdParams &p) {
     FwdParams f = p.f;
     const int n_dq = row_grid(f, Q_BM), items = f.B * f.Hk * ((f.Lk + KV_BN - 1) / KV_BN) * (f.d / 4 + (f.bias ? 1 : 0));
     const bool few = (f.Lk > 2 * f.Lq ? 1 : 2) * n_dq <= device_cus();
-    const int most = few ? 1024 : device_cus();
+    const int most = few ? 1024 : (f.d > 128 ? device_cus() * 3 / 4 : device_cus());
     p.red_count = ((items < most ? items : most) + 7) / 8 * 8;
     p.red_first = few ? n_dq : 0;
     p.red_light = n_dq <= device_cus();
