@@ -403,13 +403,19 @@ hipError_t launch_dyn_bias_fwd(const DynBiasParams &p, int dtype, hipStream_t st
     return hipGetLastError();
 }
 
-int dyn_bias_bwd_workgroups(int64_t n_rows, int *rows_per_wg) {
-    // runs of 32 tokens while that gives at most 512 workgroups (the partials are Hkv * Hkv * d floats each, and two
-    // workgroups fit a CU), else runs as long as 512 workgroups make them.  Whole passes of 64 tokens instead left up to half of
-    // the chip without a second workgroup: 4 x 9000 tokens of 16 x 64 102.9 -> 75.0 us, 17000 of 8 x 128 47.6 -> 39.6,
-    // 4 x 12672 of 8 x 128 87.0 -> 79.7
+// columns of V_flat per thread: four, where there are enough of them and the sums for them fit the registers
+static bool four_columns(int Hk, int d) { return Hk <= 16 && Hk * d >= 1024; }
+
+int dyn_bias_bwd_workgroups(int64_t n_rows, int Hk, int d, int *rows_per_wg) {
+    // Runs of 32 tokens while the device holds all workgroups at a time (the partials are Hkv * Hkv * d floats each), else runs as long
+    // as that takes, in whole eights.  A CU holds two workgroups of up to 8 heads with two columns a thread (105 registers) and one of
+    // all others (161 to 256): with twice as many as that a second round starts, mostly empty.  us, kernel and fold, 512 / 256 workgroups:
+    // 9000 tokens of 8 x 128 31.0 / 23.8, 16 x 256 140 / 92, 24 x 64 98.6 / 64.7; 16385 39.2 / 32.4, 183 / 136, 120 / 93; 33000 55.1 / 49.0, 280 / 233, 181 / 153;
+    // 131072 155 / 149, 802 / 736, 553 / 534; 8 x 64, which fits twice: 33000 33.2 / 38.3, 98304 61 / 80.  (Runs of whole passes of 64 tokens
+    // instead of whole eights: 33000 of 8 x 64 39.8.)
+    const int most = (Hk <= 8 && !four_columns(Hk, d) ? 2 : 1) * device_cus();
     int64_t rows = 32;
-    if ((n_rows + 31) / 32 > 512) rows = ((n_rows + 511) / 512 + 7) / 8 * 8;
+    if ((n_rows + 31) / 32 > most) rows = ((n_rows + most - 1) / most + 7) / 8 * 8;
     *rows_per_wg = (int)rows;
     return (int)((n_rows + rows - 1) / rows);
 }
@@ -418,7 +424,7 @@ hipError_t launch_dyn_bias_bwd(const DynBiasParams &p, int dtype, hipStream_t st
     const int64_t n_rows = (int64_t)p.B * p.L;
     if (n_rows <= 0) return hipSuccess;
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(p.n_wg), dim3(512), 0, stream, p); };
-    const bool wide = p.Hk * p.d >= 1024;  // enough columns for four per thread
+    const bool wide = four_columns(p.Hk, p.d);
     if (dtype == 0) {
         if (p.Hk <= 8) wide ? go(dyn_bias_bwd_kernel<bf16_tag, 8, 4>) : go(dyn_bias_bwd_kernel<bf16_tag, 8, 2>);
         else if (p.Hk <= 16) wide ? go(dyn_bias_bwd_kernel<bf16_tag, 16, 4>) : go(dyn_bias_bwd_kernel<bf16_tag, 16, 2>);

@@ -8,10 +8,10 @@ import torch.nn.functional as F
 from flash_sparse_attn.utils.bias import dynamic_mask_bias
 from _util import rel_err
 
-pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,L,Hk,d,dtype", [
     (1, 31, 1, 16, torch.bfloat16),      # one step in wave 0, nothing in the others
     (2, 45, 2, 72, torch.float16),       # a piece, a step, nothing, nothing
@@ -38,10 +38,26 @@ def test_pieces(B, L, Hk, d, dtype):
     assert torch.equal(bias, strided)
 
 
+@pytest.mark.parametrize("Hk,d,fit", [(8, 64, 512), (8, 128, 256), (4, 256, 256), (9, 64, 256), (16, 48, 256), (16, 256, 256), (32, 64, 256), (1, 16, 512)])
+def test_no_more_runs_than_the_device_holds_at_a_time(Hk, d, fit):
+    from flash_sparse_attn import _cabi
+
+    a = _cabi.DynBiasArgs()
+    a.batch, a.num_heads_k, a.head_dim = 1, Hk, d
+    stride = -(-(Hk * Hk * d + 2 * Hk) // 4) * 4 * 4
+    for L in (1, 32 * fit - 1, 32 * fit, 32 * fit + 1, 9000, 16385, 20000, 33000, 65537, 131072, 1 << 20):
+        a.seqlen_k = L
+        runs, rest = divmod(_cabi.lib.fdma_dyn_bias_bwd_workspace_bytes(a), stride)
+        assert rest == 0 and -(-L // 32) >= runs > 0 and runs <= fit and (runs > fit * 3 // 4 or L <= 64 * fit)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,L,Hk,d", [
     (1, 16385, 1, 16),   # runs of 40 tokens, the last of 25
     (2, 8990, 3, 48),    # a run across the batch entries
-    (1, 36900, 9, 64),   # 80 tokens: a pass of 64 and one of 16
+    (1, 36900, 9, 64),   # 152 tokens: two passes of 64 and one of 24
+    (1, 8193, 8, 128),   # 40 tokens, the last of 33
+    (3, 3500, 17, 64),   # 48 tokens, across the batch entries
 ])
 def test_gradients_of_long_runs(B, L, Hk, d):
     """The backward's runs of tokens are whole eights, not whole passes.  Sums over the tokens in fp32, results rounded to 16 bits once."""
