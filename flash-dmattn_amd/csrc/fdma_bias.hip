@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(256) dyn_bias_fwd_kernel(const DynBiasParams p
             kk = kk < ks_end * 16 ? kk : ks_begin * 16;  // (past this wave's columns: any of its chunks, never read)
             const int head = p.v_h == p.d ? 0 : kk / p.d;
             const uint16_t *src = vrow[i] + (int64_t)head * p.v_h + (kk - head * p.d);
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds0 + (n & 1) * PIECE_BYTES + i * 1024) : "memory");
+            load_lds16_at(src, lds0 + (n & 1) * PIECE_BYTES + i * 1024);
         }
     };
     // piece n, which has landed

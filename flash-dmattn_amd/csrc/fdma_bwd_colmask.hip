@@ -304,8 +304,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const Bwd
             // partial block the rows beyond the end of the queries read the last row's numbers (masked where used).
             const int over = ld_partial ? (lane & 31) - row_last : 0;
             gptr_t sp = dma_stat - (over > 0 ? over * 4 : 0);
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
-                         : : "v"(sp), "s"(__builtin_amdgcn_readfirstlane(dst + 2 * SM::Q_BYTES)));
+            load_lds4_at(sp, __builtin_amdgcn_readfirstlane(dst + 2 * SM::Q_BYTES));
         }
     };
     // end of a step: a wave waits for its own direct loads (and LDS stores), then the barrier publishes everybody's

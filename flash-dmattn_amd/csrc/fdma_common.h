@@ -197,6 +197,13 @@ template <bool MEMORY = false> __device__ __forceinline__ void load_lds16(uint32
 __device__ __forceinline__ void load_lds4(uint32_t off, gptr_t base, uint32_t dst) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(dst));
 }
+// ... from an address of each lane's own (16: as with MEMORY)
+__device__ __forceinline__ void load_lds16_at(const void *src, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(dst) : "memory");
+}
+__device__ __forceinline__ void load_lds4_at(gptr_t src, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(dst));
+}
 
 // What a lane supplies to a transposing read (lds_ld_tr16): row te of four, its 8-byte piece tc of a 32-byte half row tdh.  tcp: the
 // piece in the order in which the results are rows of an accumulator (see pi_row).
