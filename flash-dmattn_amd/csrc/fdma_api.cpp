@@ -293,7 +293,7 @@ static size_t fwd_scratch_bytes(const fdma_fwd_args *a, size_t *shares) {
         if (splits > 1) *shares = (size_t)splits * a->batch * a->num_heads * a->seqlen_q * (size_t)(a->head_dim + 1) * sizeof(float);
         return (size_t)round_up(fdma::compact_bytes(p, false), 256);
     }
-    const int splits = fdma::decode_num_splits(a->batch, a->num_heads_k, a->seqlen_k);
+    const int splits = fdma::decode_num_splits(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->mask != nullptr);
     if (splits <= 1) return 0;
     const size_t rows = (size_t)splits * a->batch * a->num_heads * a->seqlen_q;
     return rows * (size_t)(a->head_dim + 1) * sizeof(float);
@@ -316,7 +316,7 @@ int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
     hipError_t e;
     if (a->seqlen_q == 0) return FDMA_OK;
     if (fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k) && a->seqlen_k > 0) {
-        p.splits = fdma::decode_num_splits(a->batch, a->num_heads_k, a->seqlen_k);
+        p.splits = fdma::decode_num_splits(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->mask != nullptr);
         if (p.splits > 1) {
             const size_t need = fdma_fwd_workspace_bytes(a);
             if (!a->workspace || a->workspace_bytes < need)

@@ -588,15 +588,21 @@ bool use_decode_path(int Lq, int H, int Hk) {
 // 11.8 / 11.8 | 23.5 / 21.2 / 19.1 / 20.2; all 33001 kept 14.9 / 16.1 / 16.8 / 21.1 | 19.0 / 20.8 / 22.4 / 29.4 | 36.7 / 42.0 / 45.8 / 61.7; all
 // 65537 18.0 / 18.3 / 18.8 / 22.4 | 22.0 / 23.3 / 24.4 / 30.4 | 43.3 / 47.3 / 49.6 / 64.3.  (Up to 128 splits of 256 keys took 15.9 where 32 of
 // 512 take 9.7: 16384 keys x 8 / 4 heads, 1024 kept.)
+// A call without a mask keeps every key, and the host does know: one or two pairs then have 64 splits at least beyond 32768 keys (few query
+// heads, whose partial results stay small).  By spans of 1280 / with 64, one pair of four heads, d = 64 | 128 | 256: 33001 keys 16.2 / 14.2 |
+// 21.7 / 18.0 | 42.8 / 34.8; 50001 16.9 / 16.3 | 22.4 / 20.9 | 44.6 / 41.5; 65536 17.9 / 17.0 | 23.5 / 21.7 | 47.3 / 44.0; two pairs of
+// four heads 33001 16.3 / 14.6 | 21.7 / 18.4 | 44.7 / 36.2, 65536 18.4 / 17.6 | 24.2 / 22.9 | 48.6 / 45.3; four pairs of two heads, 65536
+// 19.1 / 20.3 | 29.1 / 30.0 | 55.2 / 55.7.
 // A split has at least 256 keys; up to 384 keys there is one split, without partial results and merge: 300 keys x 8 / 2,
 // d = 64, 150 kept 8.2 -> 7.1; 384, all kept, d = 128 10.5 -> 9.7 (512 keys, all kept: 10.7 in two, 11.1 in one).
 // With keys_per_split rounded up to 256 every split is non-empty.
-int decode_num_splits(int B, int Hk, int Lk) {
+int decode_num_splits(int B, int H, int Hk, int Lk, bool masked) {
     const int pairs = B * Hk > 0 ? B * Hk : 1;
     int splits = (512 + pairs - 1) / pairs;
     if ((int64_t)splits * 8192 > Lk) {
         splits = (256 + pairs - 1) / pairs;
-        const int most = Lk > 32768 ? (Lk + 1279) / 1280 : 32;
+        const int least = !masked && pairs <= 2 && B * H <= 64 ? 64 : 32, spans = (Lk + 1279) / 1280;
+        const int most = Lk > 32768 ? (spans > least ? spans : least) : 32;
         if (splits > most) splits = most;
     }
     const int max_by_len = Lk <= 384 ? 1 : (Lk + 255) / 256;
@@ -613,7 +619,7 @@ int decode_num_splits(int B, int Hk, int Lk) {
 }
 
 int64_t decode_num_counters(int B, int H, int Hk, int Lk) {
-    if (B <= 0 || Hk <= 0 || decode_num_splits(B, Hk, Lk) <= 1) return 0;
+    if (B <= 0 || Hk <= 0 || decode_num_splits(B, H, Hk, Lk, true) <= 1) return 0;  // (with a mask or without: one split of the same calls)
     const int G = H / Hk;
     return (int64_t)B * Hk * ((G + DEC_COLS - 1) / DEC_COLS);
 }

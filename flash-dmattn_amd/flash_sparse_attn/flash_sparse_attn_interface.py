@@ -199,7 +199,7 @@ def _handoff_get(name):
 # counters of the one-launch decode (fdma_fwd_args.counters) are zero before a call and zero after it: they are
 # cleared when the buffer is made and then serve every later call on that stream.
 _decode_scratch = {}
-_decode_sizes = {}   # (batch, heads, kv heads, keys, head dim) -> (workspace bytes, counter bytes): pure functions of the shape
+_decode_sizes = {}   # (batch, heads, kv heads, keys, head dim, no mask) -> (workspace bytes, counter bytes): pure functions of these
 _empty_probs = {}    # the empty S_dmask tensor per (dtype, device)
 
 
@@ -253,7 +253,7 @@ def _flash_sparse_attn_forward_body(
         workspace = None
         if seqlen_q == 1:
             # split-KV decode: workspace and arrival counters (with them the splits are merged by the same launch)
-            skey = (batch, num_heads, k.shape[2], k.shape[1], q.shape[3])
+            skey = (batch, num_heads, k.shape[2], k.shape[1], q.shape[3], mask is None)
             sizes = _decode_sizes.get(skey)
             if sizes is None:
                 sizes = _decode_sizes[skey] = (_cabi.lib.fdma_fwd_workspace_bytes(args), _cabi.lib.fdma_fwd_counter_bytes(args))

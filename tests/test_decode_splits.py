@@ -33,7 +33,30 @@ def test_spans_of_long_caches(Lk):
 
     a = _cabi.FwdArgs()
     a.batch, a.seqlen_q, a.seqlen_k, a.num_heads, a.num_heads_k, a.head_dim = 1, 1, Lk, 2, 1, 64
+    a.mask = 256  # (there is one; sizes alone are looked at)
     assert _cabi.lib.fdma_fwd_workspace_bytes(a) == -(-Lk // 1280) * (64 + 1) * 4 * 2
+
+
+@pytest.mark.parametrize("B,H,Hk,Lk,masked,unmasked", [
+    (1, 4, 1, 32768, 32, 32),
+    (1, 4, 1, 33001, 26, 43),   # spans of 768
+    (1, 64, 2, 50001, 40, 49),  # 1024
+    (2, 32, 1, 65536, 52, 64),
+    (1, 4, 1, 65537, 52, 52),   # 1280
+    (1, 4, 1, 131072, 103, 103),
+    (1, 65, 1, 33001, 26, 26),  # many query heads: no more partial results than with a mask
+    (3, 3, 1, 33001, 26, 26),   # three pairs
+])
+def test_splits_without_a_mask(B, H, Hk, Lk, masked, unmasked):
+    """A call without a mask keeps every key: few pairs take shorter spans.  The counters do not depend on it."""
+    from flash_sparse_attn import _cabi
+
+    a = _cabi.FwdArgs()
+    a.batch, a.seqlen_q, a.seqlen_k, a.num_heads, a.num_heads_k, a.head_dim = B, 1, Lk, H, Hk, 256
+    counters = _cabi.lib.fdma_fwd_counter_bytes(a)
+    assert _cabi.lib.fdma_fwd_workspace_bytes(a) == unmasked * (256 + 1) * 4 * B * H
+    a.mask = 256
+    assert _cabi.lib.fdma_fwd_workspace_bytes(a) == masked * (256 + 1) * 4 * B * H and _cabi.lib.fdma_fwd_counter_bytes(a) == counters
 
 
 @pytest.mark.gpu
@@ -81,3 +104,18 @@ def test_merge_of_splits(B, Lk, H, Hk, D, kept, splits, dtype):
     for offset, merged in ((0, False), (4, True), (4, False)):
         again, lse_again = call(offset, merged)
         assert torch.equal(again, out) and torch.equal(lse_again, lse)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_without_a_mask_behind_a_call_with_one(native, monkeypatch):
+    """Each of the two has splits and a workspace of its own: the same keys in another order of sums."""
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func
+
+    print("no mask", native, flush=True)
+    if not native:
+        monkeypatch.setattr(_cabi, "host", _cabi._NoHost)
+    q, k, v, _, bias = [t.to(DEV) for t in make_inputs(1, 1, 33003, 32, 1, 256, (1, 1, 1, 33003), (1, 1, 1, 33003), 64, seed=5, dtype=torch.float16)]
+    ref, _ = eager.attention_forward(q, k, v, None, bias, None, False)
+    for mask in (torch.ones(1, 1, 1, 33003, dtype=torch.bool, device=DEV), None):
+        assert_out_close(flash_sparse_attn_func(q, k, v, mask, bias, is_causal=False), ref)
