@@ -1288,7 +1288,9 @@ void place_reduction(BwdParams &p) {
     const int most = few ? 1024 : (f.d > 128 ? device_cus() * 3 / 4 : device_cus());
     p.red_count = ((items < most ? items : most) + 7) / 8 * 8;
     p.red_first = few ? n_dq : 0;
-    p.red_light = n_dq <= device_cus();
+    // (a CU holds two workgroups up to head dim 128, and the second round of those is where the difference is gone)
+    const float more = (float)(n_dq - device_cus()) / (float)(2 * device_cus());
+    p.red_wait = more <= 0.f ? 0.f : (f.d > 128 || more > 1.f ? 1.f : more);
 }
 
 bool bwd_colmask_applicable(const BwdParams &p) {

@@ -642,9 +642,9 @@ __device__ __forceinline__ void zero_block(const BwdParams &p, bool dbias_direct
 
 // One workgroup: prefix of 128-key units over the pairs, the split the dK/dV kernel will use and, when units are
 // split, the per-XCD lists of the parts that exist.  `slots`: workgroups of the dK/dV kernel the device holds at a
-// time; `cap`: entries a per-XCD list has room for (that kernel's workgroups per XCD); `sum_wgs`, `light`: see sums_by_chains.
+// time; `cap`: entries a per-XCD list has room for (that kernel's workgroups per XCD); `sum_wgs`, `wait`: see sums_by_chains.
 __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *idx, int ld, int32_t *plan, int pairs, int G,
-                                           int Lq, int Lk, int causal, int slots, int cap, int d, int sum_wgs, bool light) {
+                                           int Lq, int Lk, int causal, int slots, int cap, int d, int sum_wgs, float wait) {
     constexpr int MAXU = DKDV_ENOUGH_UNITS;  // units are split only below this many (and there are no more pairs than units)
     constexpr int MAXL = 1024;               // ... and with at most this many unit lists (LDS: every block of the launch pays for it)
     __shared__ int s_sum, s_max, s_units, s_wsum[4], s_wmax[4];
@@ -799,7 +799,7 @@ __device__ __forceinline__ void plan_block(const int32_t *count, const int32_t *
         plan[2] = Sm;
         plan[4] = Q;
         plan[5] = DKDV_PLAN_HDR + pairs + 1;  // where the lists begin
-        plan[7] = sums_by_chains(U, Gs0 * Sm, pairs, d, sum_wgs, light);
+        plan[7] = sums_by_chains(U, Gs0 * Sm, pairs, d, sum_wgs, wait);
         s_Q = Q; s_Sm = Sm;
     }
     const int n_lists = pairs * k;  // a multiple of 8, at most MAXL
@@ -874,7 +874,7 @@ __global__ void __launch_bounds__(256) compact_bwd_prepass_kernel(const BwdParam
     const int first_dot = do_gather ? 2 : 1, bx = (int)blockIdx.x - 1;
     if (bx < 0) {
         if (blockIdx.y == 0 && blockIdx.z == 0)
-            plan_block(count, idx, ld, plan, f.B * f.Hk, f.H / f.Hk, f.Lq, f.Lk, f.causal, slots, cap, f.d, bp.red_count * (f.d > 128 ? 2 : 1), bp.red_light != 0);
+            plan_block(count, idx, ld, plan, f.B * f.Hk, f.H / f.Hk, f.Lq, f.Lk, f.causal, slots, cap, f.d, bp.red_count * (f.d > 128 ? 2 : 1), bp.red_wait);
     } else if (blockIdx.z == 0) {
         zero_block(bp, bp.dbias != nullptr && bp.dbias_accum == nullptr, bx, blockIdx.y);
     } else if ((int)blockIdx.z < first_dot) {

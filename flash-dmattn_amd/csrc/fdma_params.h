@@ -73,13 +73,13 @@ __host__ __device__ inline void dkdv_split(int U, int G, int &Gs, int &Sm) {
 }
 // How the parts of the units are summed (plan[7], see dkdv_reduce_blocks): by several chains of loads side by side, or every sum by
 // one thread, whose trips to memory for four slots follow each other.  `nwg`: workgroups (halves of one at head dims above 128) that
-// sum; light: beside at most one dQ workgroup per CU.  One thread is enough while its trips hide behind the longest row
-// block's own chain of key tiles, which takes 1.2 / 1.4 / 3 trips' time (1.9 us) per unit of a pair at d = 64 / 128 / 256 (head dims in between: the next
-// larger), about twice that where further dQ workgroups wait for the CU.
-__host__ __device__ inline bool sums_by_chains(int U, int per, int pairs, int d, int nwg, bool light) {
+// sum; wait: how much of dQ waits for a CU, from 0 (at most one workgroup per CU) to 1.  One thread is enough while its trips hide
+// behind the longest row block's own chain of key tiles: about 0.8 / 1 / 4 trips' time (1.9 us) per unit of a pair at d = 64 / 128 / 256 (head dims in
+// between: the next larger), and 2 / 4 / 8 where dQ goes on behind it anyway.
+__host__ __device__ inline bool sums_by_chains(int U, int per, int pairs, int d, int nwg, float wait) {
     const int dpad = d <= 64 ? 64 : (d <= 128 ? 128 : 256), trips = (U * (dpad / 16) + nwg - 1) / nwg * ((per + 3) / 4);
-    const float per_unit = light ? (d <= 64 ? 0.8f : (d <= 128 ? 1.2f : 2.f)) : (d <= 64 ? 2.f : 4.f);
-    return (float)trips > 2.f + per_unit * (float)U / (float)pairs;
+    const float alone = d <= 64 ? 0.8f : (d <= 128 ? 1.f : 4.f), beside = d <= 64 ? 2.f : (d <= 128 ? 4.f : 8.f);
+    return (float)trips > 2.f + (alone + (beside - alone) * wait) * (float)U / (float)pairs;
 }
 // query blocks (of 64 rows) that see a key block whose first key sits at original column `okey_first`
 __host__ __device__ inline int dkdv_query_blocks(int Lq, int Lk, int causal, int okey_first) {
@@ -321,7 +321,7 @@ struct BwdParams {
     int32_t kv_most, kv_quota, kv_units;
     int32_t dot_done;          // softmax_d has been computed by an earlier launch of this call
     int32_t red_first, red_count;  // compacted backward: workgroups of the dQ launch that sum the dK/dV partials (see place_reduction)
-    int32_t red_light;             // ... beside at most one that works on dQ per CU
+    float red_wait;                // how much of dQ waits for a CU beside them, 0 .. 1
 };
 
 // Keep-mask builder (fdma_mask.hip): one row of `Lk` 16-bit bias values per (batch, head, row).

@@ -32,7 +32,7 @@ def plan_in(ws, pairs, units):
     (1, 1030, 1030, 8, 2, 256, 1, 500, False, (4, 9), 0, torch.float16),  # one bias row for all kv heads: atomics
     (16, 130, 700, 2, 1, 128, 1, 640, False, (2, 3), 0, torch.bfloat16),  # 80 units
     (16, 200, 640, 8, 2, 64, 2, 600, True, (4, 1), 0, torch.float16),     # 160 units
-    (8, 513, 513, 12, 2, 64, 2, 513, True, (6, 3), 0, torch.float16),     # a dBias column of 18, 12 or 6 terms
+    (8, 800, 800, 12, 2, 64, 2, 630, True, (6, 3), 0, torch.float16),     # a dBias column of 18, 12 or 6 terms
     (16, 300, 300, 12, 2, 200, 2, 290, True, (6, 2), 0, torch.bfloat16),  # ... of 12 or 6, by halves of a workgroup
     (32, 300, 300, 12, 2, 64, 2, 290, True, (3, 1), 0, torch.bfloat16),   # several heads in a part: 6 terms
     (24, 200, 200, 32, 2, 64, 2, 200, False, (8, 1), 0, torch.float16),   # ... 16 terms
@@ -46,6 +46,7 @@ def plan_in(ws, pairs, units):
     (1, 1030, 1030, 8, 1, 256, 1, 200, True, (8, 6), 1, torch.float16),   # two halves of a workgroup share the items
     (1, 1030, 1030, 8, 2, 256, 1, 128, False, (4, 9), 1, torch.float16),  # ... one bias row for all kv heads: atomics
     (2, 1030, 1030, 4, 2, 64, 0, 129, False, (2, 9), 1, torch.float16),   # no bias
+    (8, 513, 513, 12, 2, 64, 2, 513, True, (6, 3), 1, torch.float16),     # many units
     (1, 500, 500, 32, 1, 64, 1, 200, True, (32, 8), 1, torch.float16),    # 256 slots
 ])
 def test_part_sums(B, Lq, Lk, H, Hk, D, Hb, kept, causal, parts, chains, dtype, monkeypatch):
