@@ -159,12 +159,11 @@ __device__ __forceinline__ void dkdv_reduce_rows(const float *base, const int n_
 // kept: 6 units, 24 items, and their dBias slot by slot, 46 us the launch, 13.7 now).  Where that is longer than dQ beside it (plan[7]),
 // an item is eight columns of dK or of dV, or dBias, the slots are spread over the threads, and the sums are added up through LDS.
 // That keeps a third as many bytes in flight and more workgroups busy.  One thread / side by side, the dQ launch of 2048 tokens (us):
-// d = 64: 16/8 heads, 256 kept 23.8 / 12.8, 16/4, 640 kept 21.6 / 19.1, 2 x 16/8, 384 kept 19.6 / 21.4, 4 x 16/8, 384 kept 31.4 / 33.7, 6 x 16/8, 640
-// kept 40.6 / 43.5; d = 128: 16/4, 384 kept 28.4 / 21.8, 32/8, 384 kept 28.1 / 29.9; d = 256: 8/2, 100 kept 30.6 / 18.3, 16/8, 384 kept 37.4 /
-// 39.2, 2 x 16/8, 640 kept 83.8 / 95.7.  Of 956 backward calls (256 to 8000 rows, 64 to 2048 kept) the rule of sums_by_chains
-// costs more than 3 % over the better way on 27, 9 % at most; all by one thread 230 and 76 %, all side by side 173 and 16 %.  One thread / side by
-// side where few dQ workgroups wait, the whole backward: 4652 x 8/1, d = 128, 1000 kept 125 / 102, 2 x 2335 x 8/2, 447 kept 67.1 / 60.6; not causal
-// 4 x 1496 x 8/1, d = 256, 224 kept 120 / 135.
+// d = 64: 16/8 heads, 256 kept 19.3 / 13.2, 16/4, 640 kept 20.7 / 19.2, 2 x 16/8, 384 kept 20.6 / 22.3, 4 x 16/8, 384 kept 33.2 / 35.3, 6 x 16/8, 640
+// kept 60.8 / 66.6; d = 128: 16/4, 384 kept 28.3 / 21.8, 32/8, 384 kept 27.7 / 29.8, 4652 x 8/1, 1000 kept 57.9 / 35.7; d = 256: 8/2, 100 kept
+// 30.0 / 17.8, 16/8, 384 kept 38.6 / 40.8, 2 x 16/8, 640 kept 83.4 / 93.3, 4 x 16/16, 256 kept 118 / 129.  Of 956 backward calls (256 to 8000 rows, 64
+// to 2048 kept) the rule of sums_by_chains costs more than 3 % over the better way on 27, 9 % at most (3001 x 8/4, d = 256, 1024 kept, the launch 65.2 /
+// 60.9); all by one thread 230 and 76 %, all side by side 173 and 16 %.
 template <typename T, int D>
 __device__ __forceinline__ void dkdv_reduce_blocks(const BwdParams &p, const int rb, const int nrb, const int tid, float *lds) {
     using E = Elem<T>;

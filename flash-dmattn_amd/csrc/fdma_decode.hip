@@ -72,8 +72,9 @@ __device__ __forceinline__ void part_store(float *ptr, float v) {
 // out[b,h,:] = sum_s exp(lse_s - lse) * o_s ;  lse = logsumexp_s lse_s  (empty everywhere: 0 / +inf) for one (b, h) row,
 // by ONE wave: lane s (and s + 64) fetches lse_s and holds the weight of split s, then lane i sums its head-dim elements 2 i,
 // 2 i + 1 (and + 128) over the splits.  Bound by trips to memory: up to CMB_FLIGHT splits are requested together, the first of
-// them beside the LSEs (eight at a time, weights through LDS: 2049 keys x 32 / 8 heads, 9 splits, the call 10.0 -> 9.3 us; 65536 x 2 / 1,
-// 32 splits 10.9 -> 9.8).
+// them beside the LSEs.  Eight at a time, an element a lane, weights through LDS / now, us: 2049 keys x 32 / 8 heads, 9 splits 10.0 / 9.3; 512 kept
+// of 16384 x 4 / 1, 64 splits d = 64 10.5 / 11.1 (half of the lanes have no element), 128 14.0 / 11.9, 256 25.1 / 19.3; of 65537 in 86
+// 12.8 / 12.8, 18.2 / 13.7, 33.8 / 22.6.
 // Both users of this function sum in the same order, so their results agree bit for bit.
 constexpr int CMB_FLIGHT = 32;
 constexpr int CMB_GROUP = 8;  // requested and added without a branch between them
@@ -586,8 +587,8 @@ bool use_decode_path(int Lq, int H, int Hk) {
 // 33001 keys, 512 kept 10.4 / 9.6 / 9.2 / 8.8 | 11.0 / 10.0 / 9.7 / 9.3 | 17.6 / 16.4 / 15.3 / 14.6; 65537, 512 kept
 // 13.0 / 11.8 / 10.7 / 9.8 | 13.8 / 12.5 / 11.6 / 10.3 | 23.2 / 20.9 / 18.5 / 16.4; 4096 kept 13.3 / 11.9 / 10.8 / 10.7 | 14.0 / 12.8 /
 // 11.8 / 11.8 | 23.5 / 21.2 / 19.1 / 20.2; all 33001 kept 14.9 / 16.1 / 16.8 / 21.1 | 19.0 / 20.8 / 22.4 / 29.4 | 36.7 / 42.0 / 45.8 / 61.7; all
-// 65537 18.0 / 18.3 / 18.8 / 22.4 | 22.0 / 23.3 / 24.4 / 30.4 | 43.3 / 47.3 / 49.6 / 64.3.  (Up to 128 splits of 256 keys took 15.9 where 32 of
-// 512 take 9.7: 16384 keys x 8 / 4 heads, 1024 kept.)
+// 65537 18.0 / 18.3 / 18.8 / 22.4 | 22.0 / 23.3 / 24.4 / 30.4 | 43.3 / 47.3 / 49.6 / 64.3.  (64 splits of 256 keys instead of
+// 32 of 512: 16384 keys x 8 / 4 heads, d = 128, 512 kept 13.3 / 9.6, all kept 15.7 / 14.8.)
 // A call without a mask keeps every key, and the host does know: one or two pairs then have 64 splits at least beyond 32768 keys (few query
 // heads, whose partial results stay small).  By spans of 1280 / with 64, one pair of four heads, d = 64 | 128 | 256: 33001 keys 16.2 / 14.2 |
 // 21.7 / 18.0 | 42.8 / 34.8; 50001 16.9 / 16.3 | 22.4 / 20.9 | 44.6 / 41.5; 65536 17.9 / 17.0 | 23.5 / 21.7 | 47.3 / 44.0; two pairs of
