@@ -209,7 +209,8 @@ int fdma_fwd_noalloc(const fdma_fwd_args *args, void *hip_stream);
  * the same value.  n <= 0 only queries.  Returns the value before the call.  No counterpart in the reference. */
 int fdma_set_stream_min_items(int n);
 
-/* Scratch the caller must provide.  0 when none is needed.  Validate nothing but shapes. */
+/* Scratch the caller must provide.  0 when none is needed.  Validate nothing but shapes.  Ask with the arguments of the call itself:
+ * which tensors there are counts too (a decode call without a mask keeps every key and can take more splits than one with). */
 size_t fdma_fwd_workspace_bytes(const fdma_fwd_args *args);
 /* Size of the optional arrival counters (fdma_fwd_args.counters); 0 when the call would not use them. */
 size_t fdma_fwd_counter_bytes(const fdma_fwd_args *args);
