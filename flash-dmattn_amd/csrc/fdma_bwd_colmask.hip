@@ -787,7 +787,6 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
 
     const FwdParams &f = p.f;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = tid & 63, r = lane & 31, g = lane >> 5;
-    const int G = f.H / f.Hk;
     int lid = blockIdx.x;  // index among the dQ workgroups
     if (CMP) {
         // some workgroups sum partial results of the dK/dV kernel instead
@@ -800,15 +799,32 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
     }
     const RowUnit ru = row_unit(f, lid, Q_BM);  // (heaviest first under causal)
     if (ru.block < 0) return;
-    const int b = ru.pair / f.Hk, hk = ru.pair % f.Hk;
-    const int h = hk * G + (lid / 8) % G;
+    const int b = ru.b, hk = ru.hk, h = ru.h;
     const int m0 = ru.block * Q_BM;
     const SeqInfo sq = seq_info(f, b);  // this batch entry's lengths and first rows (ragged batch: from cu_seqlens)
     const int LqS = sq.Lq, LkS = sq.Lk;
     if (m0 >= LqS) return;
     const int qrow = m0 + wave * 32 + r;
     const int qrow_c = qrow < LqS ? qrow : LqS - 1;
-    const int shift = LkS - LqS;
+
+    // ---- Q and dO fragments (B operands), O and the row statistics: requested first of all, raw, from places that exist (rows
+    // beyond Lq: the last one, chunks beyond d: the first), and looked at when the first tiles are on their way.  One trip to memory
+    // for the counts above the rows, one for all of this and one for the tiles were six behind one another.
+    u32x4_t qf[KS], dof[KS], of[CMP ? 1 : KS];
+    {
+        const uint16_t *qp = (const uint16_t *)f.q + b * f.q_b + (sq.q0 + qrow_c) * f.q_r + h * f.q_h;
+        const uint16_t *dp = (const uint16_t *)p.dout + b * p.do_b + (sq.q0 + qrow_c) * p.do_r + h * p.do_h;
+        const uint16_t *op = (const uint16_t *)f.o + b * f.o_b + (sq.q0 + qrow_c) * f.o_r + h * f.o_h;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const int c = ks * 16 + g * 8 < f.d ? ks * 16 + g * 8 : 0;
+            qf[ks] = *(const u32x4_t *)(qp + c);
+            dof[ks] = *(const u32x4_t *)(dp + c);
+            if constexpr (!CMP) of[ks] = *(const u32x4_t *)(op + c);
+        }
+    }
+    const float lse_raw = f.lse[b * f.lse_b + h * f.lse_h + sq.q0 + qrow_c];
+    const float dd_raw = CMP ? p.softmax_d[b * p.sd_b + h * p.sd_h + sq.q0 + qrow_c] : 0.f;
 
     const int hm = f.mask ? (f.Hm == f.H ? h : (f.Hm == 1 ? 0 : hk)) : 0;
     const int hb = f.bias ? (f.Hb == f.H ? h : (f.Hb == 1 ? 0 : hk)) : 0;
@@ -821,21 +837,13 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
     const int Lk = CMP ? f.cmp.count[ru.pair] : LkS;
     const int32_t *ccnt = CMP ? f.cmp.cnt + (int64_t)ru.pair * f.cmp.ld : nullptr;
     const float *fbrow = CMP ? f.cmp.fb + (int64_t)(b * f.cmp.Hfb + (f.cmp.Hfb == f.H ? h : hk)) * f.cmp.ld : nullptr;
-    auto visible = [&](int row) -> int {  // columns [0, visible(row)) pass the causal test for `row`
-        if (row >= LqS) row = LqS - 1;
-        const int c = row + shift;
-        if (!CMP) return c + 1;
-        if (c < 0) return 0;
-        return ccnt[c < LkS ? c : LkS - 1];
-    };
-    const int vis_lane = CAUSAL ? visible(qrow) : 0;
-    const int vis_wave = CAUSAL ? visible(m0 + wave * 32) : 0;
+    const int vis_lane = CAUSAL ? visible_columns<CMP>(qrow, LqS, LkS, ccnt) : 0;  // columns below it pass the causal test for this lane's row
+    const int vis_wave = CAUSAL ? visible_columns<CMP>(m0 + wave * 32, LqS, LkS, ccnt) : 0;
+    const int vis_block = CAUSAL ? visible_columns<CMP>(m0 + Q_BM - 1, LqS, LkS, ccnt) : 0;
 
     int n_end = (Lk + BN - 1) / BN;
     if (CAUSAL) {
-        int lim = visible(m0 + Q_BM - 1);
-        if (lim < 0) lim = 0;
-        const int ne = (lim + BN - 1) / BN;
+        const int ne = ((vis_block < 0 ? 0 : vis_block) + BN - 1) / BN;
         if (ne < n_end) n_end = ne;
     }
 
@@ -865,7 +873,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
             sBits[w0 + 1] = (uint32_t)(ball >> 32);
         }
     }
-    __syncthreads();
+    if (!CMP) __syncthreads();
     auto next_active = [&](int j) -> int {  // wave-uniform: keeps tile bases and loop conditions scalar
         if (CMP) return j < n_end ? j : n_end;
         while (j < n_end) {
@@ -878,46 +886,6 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
         }
         return n_end;
     };
-
-    // ---- Q and dO fragments (B operands), row statistics
-    u32x4_t qf[KS], dof[KS];
-    {
-        const uint16_t *qp = (const uint16_t *)f.q + b * f.q_b + (sq.q0 + qrow_c) * f.q_r + h * f.q_h;
-        const uint16_t *dp = (const uint16_t *)p.dout + b * p.do_b + (sq.q0 + qrow_c) * p.do_r + h * p.do_h;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const int c = ks * 16 + g * 8;
-            u32x4_t qv = {0, 0, 0, 0}, dv = {0, 0, 0, 0};
-            if (qrow < LqS && c < f.d) { qv = *(const u32x4_t *)(qp + c); dv = *(const u32x4_t *)(dp + c); }
-            // Q only feeds the scores in this kernel: scale it by softmax_scale * log2(e) once
-#pragma unroll
-            for (int e = 0; e < 4; e++) qv[e] = E::pack2(E::lo(qv[e]) * f.scale_log2, E::hi(qv[e]) * f.scale_log2);
-            qf[ks] = qv;
-            dof[ks] = dv;
-        }
-    }
-    float lse2 = INFINITY, dd = 0.f;
-    if (qrow < LqS) {
-        lse2 = f.lse[b * f.lse_b + h * f.lse_h + sq.q0 + qrow] * kLog2e;
-        if (CMP) dd = p.softmax_d[b * p.sd_b + h * p.sd_h + sq.q0 + qrow];
-    }
-    if constexpr (!CMP) {
-        // D = rowsum(dO * O) is made here, from the dO fragments, and left for the dK/dV kernel, which is launched behind
-        // this one: a launch and a second read of dO less (52 us of 2.8 ms on 16384 ragged tokens x 32 heads).  (With
-        // compacted keys this launch also sums that kernel's partial results and comes second; D is a layer of the pre-pass.)
-        const uint16_t *op = (const uint16_t *)f.o + b * f.o_b + (sq.q0 + qrow_c) * f.o_r + h * f.o_h;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const int c = ks * 16 + g * 8;
-            const u32x4_t ov = *(const u32x4_t *)(op + (c < f.d ? c : 0));  // (dO is zero beyond d and beyond Lq)
-#pragma unroll
-            for (int e = 0; e < 4; e++) dd += E::lo(ov[e]) * E::lo(dof[ks][e]) + E::hi(ov[e]) * E::hi(dof[ks][e]);
-        }
-        dd = xhalf_sum(dd);
-        if (qrow >= LqS) dd = 0.f;
-        // (fixed lengths: padded rows are zero)
-        if (g == 0 && (qrow < LqS || (!f.cu_q && qrow < p.Lq_rounded))) p.softmax_d[b * p.sd_b + h * p.sd_h + sq.q0 + qrow] = dd;
-    }
 
     f32x16_t dq[DB];
 #pragma unroll
@@ -1048,15 +1016,43 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
         }
     };
     int jc = next_active(0), jn = n_end, jnn = n_end;
+    // (what was requested above has landed by now; waited for here, the tiles' own loads are not waited for with it)
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qf[ks]), "+v"(dof[ks]));
     if (jc < n_end) {
         jn = next_active(jc + 1);
         load_tile(jc, jc);
-        store_tile(0, 0);
         if constexpr (DMA) {  // the second tile is on its way before the first is looked at
             jnn = next_active(jn + 1);
             dma_stage = 1;
             load_tile(jn < n_end ? jn : jc, jc);
         }
+    }
+    const bool row_ok = qrow < LqS;
+    const float lse2 = row_ok ? lse_raw * kLog2e : INFINITY;
+    float dd = row_ok ? dd_raw : 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+        const bool ok = row_ok && ks * 16 + g * 8 < f.d;
+        qf[ks] = scaled8<T>(qf[ks], f.scale_log2, ok);  // (Q only feeds the scores in this kernel: softmax_scale * log2(e) once)
+        dof[ks] = kept8(dof[ks], ok);
+    }
+    if constexpr (!CMP) {
+        // D = rowsum(dO * O) is made here, from the dO fragments, and left for the dK/dV kernel, which is launched behind
+        // this one: a launch and a second read of dO less (52 us of 2.8 ms on 16384 ragged tokens x 32 heads).  (With
+        // compacted keys this launch also sums that kernel's partial results and comes second; D is a layer of the pre-pass.)
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {  // (dO is zero beyond d and beyond Lq)
+#pragma unroll
+            for (int e = 0; e < 4; e++) dd += E::lo(of[ks][e]) * E::lo(dof[ks][e]) + E::hi(of[ks][e]) * E::hi(dof[ks][e]);
+        }
+        dd = xhalf_sum(dd);
+        if (!row_ok) dd = 0.f;
+        // (fixed lengths: padded rows are zero)
+        if (g == 0 && (row_ok || (!f.cu_q && qrow < p.Lq_rounded))) p.softmax_d[b * p.sd_b + h * p.sd_h + sq.q0 + qrow] = dd;
+    }
+    if (jc < n_end) {
+        store_tile(0, 0);
         publish();
     }
     int i = 0;

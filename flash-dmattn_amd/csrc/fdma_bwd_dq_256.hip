@@ -52,7 +52,6 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
     const FwdParams &f = p.f;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = tid & 63, r = lane & 31, g = lane >> 5;
     const int rw = wave & 3, role = wave >> 2;
-    const int G = f.H / f.Hk;
     int lid = blockIdx.x;  // index among the dQ workgroups
     if (CMP) {  // some workgroups sum partial results of the dK/dV kernel instead (see place_reduction, fdma_bwd_colmask.hip)
         const int at = lid - p.red_first;
@@ -64,8 +63,7 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
     }
     const RowUnit ru = row_unit(f, lid, BM);  // (heaviest first under causal)
     if (ru.block < 0) return;
-    const int b = ru.pair / f.Hk, hk = ru.pair % f.Hk;
-    const int h = hk * G + (lid / 8) % G;
+    const int b = ru.b, hk = ru.hk, h = ru.h;
     const int m0 = ru.block * BM;
     const SeqInfo sq = seq_info(f, b);
     const int LqS = sq.Lq, LkS = sq.Lk;
@@ -85,20 +83,12 @@ __global__ void __launch_bounds__(NT) bwd_dq_256_kernel(const BwdParams p) {
     const int Lk = CMP ? f.cmp.count[ru.pair] : LkS;
     const int32_t *ccnt = CMP ? f.cmp.cnt + (int64_t)ru.pair * f.cmp.ld : nullptr;
     const float *fbrow = CMP ? f.cmp.fb + (int64_t)(b * f.cmp.Hfb + (f.cmp.Hfb == f.H ? h : hk)) * f.cmp.ld : nullptr;
-    auto visible = [&](int row) -> int {
-        if (row >= LqS) row = LqS - 1;
-        const int c = row + shift;
-        if (!CMP) return c + 1;
-        if (c < 0) return 0;
-        return ccnt[c < LkS ? c : LkS - 1];
-    };
-    const int vis_lane = CAUSAL ? visible(qrow) : 0;
-    const int vis_wave = CAUSAL ? visible(m0 + rw * 32) : 0;
+    const int vis_lane = CAUSAL ? visible_columns<CMP>(qrow, LqS, LkS, ccnt) : 0;  // columns below it pass the causal test for this lane's row
+    const int vis_wave = CAUSAL ? visible_columns<CMP>(m0 + rw * 32, LqS, LkS, ccnt) : 0;
+    const int vis_block = CAUSAL ? visible_columns<CMP>(m0 + BM - 1, LqS, LkS, ccnt) : 0;
     int n_end = (Lk + BN - 1) / BN;
     if (CAUSAL) {
-        int lim = visible(m0 + BM - 1);
-        if (lim < 0) lim = 0;
-        const int ne = (lim + BN - 1) / BN;
+        const int ne = ((vis_block < 0 ? 0 : vis_block) + BN - 1) / BN;
         if (ne < n_end) n_end = ne;
     }
 

@@ -285,8 +285,14 @@ template <int N> __device__ __forceinline__ void ld_row16(const uint8_t *row, co
     if (n >= 16) {
 #pragma unroll
         for (int u = 0; u < N; u++) v[u] = *(const u32x4_any_t *)(row + (c[u] + 16 <= n ? c[u] : n - 16));
+        // (nothing to put back in a wave without a piece that crosses the end: thirty instructions a piece)
+        bool cross = false;
 #pragma unroll
-        for (int u = 0; u < N; u++) v[u] = shift_row16(v[u], c[u] + 16 - n);
+        for (int u = 0; u < N; u++) cross = cross || c[u] + 16 > n;
+        if (__any(cross)) {
+#pragma unroll
+            for (int u = 0; u < N; u++) v[u] = shift_row16(v[u], c[u] + 16 - n);
+        }
     } else {
 #pragma unroll
         for (int u = 0; u < N; u++) {
@@ -333,6 +339,31 @@ template <bool ODD> __device__ __forceinline__ u32x4_t chunk8_fix(u32x4_t b, int
         b = u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
     }
     return b;
+}
+
+// Key columns that query row `row` of Lq may see among Lk (CMP: of the kept ones, by the counts `cnt` of their row), below zero
+// or zero: none.  Without a branch around the load: the two or three of a prologue and the number of kept keys are then one trip to memory.
+template <bool CMP> __device__ __forceinline__ int visible_columns(int row, int Lq, int Lk, const int32_t *cnt) {
+    const int c = (row < Lq ? row : Lq - 1) + Lk - Lq;
+    if (!CMP) return c + 1;
+    const int n = cnt[c < 0 ? 0 : (c < Lk ? c : Lk - 1)];
+    return c < 0 ? 0 : n;
+}
+
+// Eight elements times `by`, rounded back to their type; all zero unless `keep` (by a mask of bits: a branch around each of a fragment's
+// registers was ten instructions of them, and what is dropped may be infinite)
+__device__ __forceinline__ u32x4_t kept8(u32x4_t v, bool keep) {
+    uint32_t bits = keep ? ~0u : 0u;
+    asm volatile("" : "+v"(bits));
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] &= bits;
+    return v;
+}
+template <typename T> __device__ __forceinline__ u32x4_t scaled8(u32x4_t v, float by, bool keep) {
+    using E = Elem<T>;
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = E::pack2(E::lo(v[e]) * by, E::hi(v[e]) * by);
+    return kept8(v, keep);
 }
 
 // max / sum across the two 32-lane halves of a wave (lanes l and l ^ 32)

@@ -118,9 +118,7 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
     // tiles then hit in that XCD's L2, and every XCD gets the same amount of work.
     const RowUnit ru = row_unit(p, blockIdx.x, BM);
     if (ru.block < 0) return;
-    const int G = p.H / p.Hk;
-    const int b = ru.pair / p.Hk, hk = ru.pair % p.Hk;
-    const int h = hk * G + (int)(blockIdx.x / 8) % G;
+    const int b = ru.b, hk = ru.hk, h = ru.h;
     const int m0 = ru.block * BM;
     const SeqInfo sq = seq_info(p, b);  // this batch entry's lengths and first rows (ragged batch: from cu_seqlens)
     const int LqS = sq.Lq, LkS = sq.Lk;
@@ -141,8 +139,8 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
         }
     }
 
-    const int hm = p.mask ? (p.Hm == p.H ? h : (p.Hm == 1 ? 0 : h / (p.H / p.Hm))) : 0;
-    const int hb = p.bias ? (p.Hb == p.H ? h : (p.Hb == 1 ? 0 : h / (p.H / p.Hb))) : 0;
+    const int hm = p.mask ? (p.Hm == p.H ? h : (p.Hm == 1 ? 0 : hk)) : 0;
+    const int hb = p.bias ? (p.Hb == p.H ? h : (p.Hb == 1 ? 0 : hk)) : 0;
     const uint8_t *mrow = p.mask ? p.mask + b * p.m_b + hm * p.m_h : nullptr;
     const uint16_t *brow = p.bias ? (const uint16_t *)p.bias + b * p.bi_b + hb * p.bi_h : nullptr;
     const uint16_t *kbase = (const uint16_t *)p.k + b * p.k_b + sq.k0 * p.k_r + hk * p.k_h;
@@ -152,19 +150,15 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
     const int Lk = CMP ? p.cmp.count[b * p.Hk + hk] : LkS;
     const int32_t *ccnt = CMP ? p.cmp.cnt + (int64_t)(b * p.Hk + hk) * p.cmp.ld : nullptr;
     const float *fbrow = CMP ? p.cmp.fb + (int64_t)(b * p.cmp.Hfb + (p.cmp.Hfb == p.H ? h : hk)) * p.cmp.ld : nullptr;
-    auto visible = [&](int row) -> int {  // columns [0, visible(row)) pass the causal test for `row`
-        if (row >= LqS) row = LqS - 1;
-        int c = row + shift;
-        if (!CMP) return c + 1;
-        if (c < 0) return 0;
-        return ccnt[c < LkS ? c : LkS - 1];
-    };
+    // causal limits: columns below vis_lane are visible to this lane's query row, and a half tile that ends at
+    // or below vis_wave (the limit of the wave's first row) needs no masking at all
+    const int vis_lane = CAUSAL ? visible_columns<CMP>(wrow0 + r, LqS, LkS, ccnt) : 0;
+    const int vis_wave = CAUSAL ? visible_columns<CMP>(wrow0, LqS, LkS, ccnt) : 0;
+    const int vis_block = CAUSAL ? visible_columns<CMP>(m0 + BM - 1, LqS, LkS, ccnt) : 0;
 
     int n_end = (Lk + BN - 1) / BN;
     if (CAUSAL) {
-        int lim = visible(m0 + BM - 1);
-        if (lim < 0) lim = 0;
-        int ne = (lim + BN - 1) / BN;
+        const int ne = ((vis_block < 0 ? 0 : vis_block) + BN - 1) / BN;
         if (ne < n_end) n_end = ne;
     }
 
@@ -365,11 +359,6 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
     };
 
     const int a_row = pi_row(r);
-
-    // causal limits: columns below vis_lane are visible to this lane's query row, and a half tile that ends at
-    // or below vis_wave (the limit of the wave's first row) needs no masking at all
-    const int vis_lane = CAUSAL ? visible(wrow0 + r) : 0;
-    const int vis_wave = CAUSAL ? visible(wrow0) : 0;
 
     // Constants of a query row that meet the side rows of the keys (B operand of the extra k-step; the lanes of
     // the upper half supply zeros against the zero half of the side rows): 1 / kPieceScale for the three bias
@@ -604,12 +593,7 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
         {
             const bool row_ok = wrow0 + r < LqS;
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const bool ok = row_ok && ks * 16 + g * 8 < p.d;
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    qf[ks][e] = ok ? E::pack2(E::lo(qf[ks][e]) * p.scale_log2, E::hi(qf[ks][e]) * p.scale_log2) : 0u;
-            }
+            for (int ks = 0; ks < KS; ks++) qf[ks] = scaled8<T>(qf[ks], p.scale_log2, row_ok && ks * 16 + g * 8 < p.d);
         }
         __syncthreads();
 

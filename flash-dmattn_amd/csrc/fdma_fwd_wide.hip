@@ -79,8 +79,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
 
     const RowUnit ru = row_unit(p, blockIdx.x, BM);
     if (ru.block < 0) return;
-    const int G = p.H / p.Hk;
-    const int b = ru.pair / p.Hk, hk = ru.pair % p.Hk, h = hk * G + (int)(blockIdx.x / 8) % G;
+    const int b = ru.b, hk = ru.hk, h = ru.h;
     const int m0 = ru.block * BM;
     const SeqInfo sq = seq_info(p, b);
     const int LqS = sq.Lq, LkS = sq.Lk;
@@ -99,8 +98,8 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         }
     }
 
-    const int hm = p.mask ? (p.Hm == p.H ? h : (p.Hm == 1 ? 0 : h / (p.H / p.Hm))) : 0;
-    const int hb = p.bias ? (p.Hb == p.H ? h : (p.Hb == 1 ? 0 : h / (p.H / p.Hb))) : 0;
+    const int hm = p.mask ? (p.Hm == p.H ? h : (p.Hm == 1 ? 0 : hk)) : 0;
+    const int hb = p.bias ? (p.Hb == p.H ? h : (p.Hb == 1 ? 0 : hk)) : 0;
     const uint8_t *mrow = p.mask ? p.mask + b * p.m_b + hm * p.m_h : nullptr;
     const uint16_t *brow = p.bias ? (const uint16_t *)p.bias + b * p.bi_b + hb * p.bi_h : nullptr;
     const uint16_t *kbase = (const uint16_t *)p.k + b * p.k_b + sq.k0 * p.k_r + hk * p.k_h;
@@ -110,18 +109,12 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     const int Lk = CMP ? p.cmp.count[b * p.Hk + hk] : LkS;
     const int32_t *ccnt = CMP ? p.cmp.cnt + (int64_t)(b * p.Hk + hk) * p.cmp.ld : nullptr;
     const float *fbrow = CMP ? p.cmp.fb + (int64_t)(b * p.cmp.Hfb + (p.cmp.Hfb == p.H ? h : hk)) * p.cmp.ld : nullptr;
-    auto visible = [&](int row) -> int {  // columns [0, visible(row)) pass the causal test for `row`
-        if (row >= LqS) row = LqS - 1;
-        const int c = row + shift;
-        if (!CMP) return c + 1;
-        if (c < 0) return 0;
-        return ccnt[c < LkS ? c : LkS - 1];
-    };
+    const int vis_lane = CAUSAL ? visible_columns<CMP>(qrow, LqS, LkS, ccnt) : 0;  // columns below it pass the causal test for this lane's row
+    const int vis_wave = CAUSAL ? visible_columns<CMP>(wrow0, LqS, LkS, ccnt) : 0;
+    const int vis_block = CAUSAL ? visible_columns<CMP>(m0 + BM - 1, LqS, LkS, ccnt) : 0;
     int n_end = (Lk + BN - 1) / BN;
     if (CAUSAL) {
-        int lim = visible(m0 + BM - 1);
-        if (lim < 0) lim = 0;
-        const int ne = (lim + BN - 1) / BN;
+        const int ne = ((vis_block < 0 ? 0 : vis_block) + BN - 1) / BN;
         if (ne < n_end) n_end = ne;
     }
     // this workgroup's share of the tiles (see fwd_key_splits)
@@ -136,8 +129,6 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         t_first = n_end * y / shares;
         n_end = n_end * (y + 1) / shares;
     }
-    const int vis_lane = CAUSAL ? visible(qrow) : 0;
-    const int vis_wave = CAUSAL ? visible(wrow0) : 0;
 
     // ---- active-tile bitmap (compacted keys: every tile is active)
     for (int base = 0; !CMP && base < n_end; base += NT) {
@@ -256,11 +247,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     // Q is scaled by softmax_scale * log2(e) once (the reference also rounds the scaled Q to the input type,
     // flash_fwd_kernel.h:428-439)
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        const bool ok = qrow < LqS && ks * 16 + g * 8 < p.d;
-#pragma unroll
-        for (int e = 0; e < 4; e++) qf[ks][e] = ok ? E::pack2(E::lo(qf[ks][e]) * p.scale_log2, E::hi(qf[ks][e]) * p.scale_log2) : 0u;
-    }
+    for (int ks = 0; ks < KS; ks++) qf[ks] = scaled8<T>(qf[ks], p.scale_log2, qrow < LqS && ks * 16 + g * 8 < p.d);
     if (jc < n_end) publish();
 
     auto one_tile = [&](auto st_c) {

@@ -171,6 +171,19 @@ __host__ __device__ inline int mask_piece_at(bool bits, int kk, int Lk) {
     return (k >> (bits ? 3 : 0)) & (bits ? ~7 : ~0);
 }
 
+// Division by a number that the launch knows, of anything below 2^31: two products and a shift on the scalar unit where the general one
+// is thirty vector instructions and a reciprocal.  (mul = ceil(2^(31 + shift) / by) with 2^shift >= by is off by less than
+// by / 2^(31 + shift) of the quotient's step.)
+struct Divisor {
+    uint32_t by, mul, shift;
+};
+inline Divisor divisor(uint32_t by) {
+    uint32_t s = 0;
+    while (s < 31 && (1u << s) < by) s++;
+    return {by, (uint32_t)((((uint64_t)1 << (31 + s)) + by - 1) / by), 31 + s};
+}
+__host__ __device__ inline int quotient(int n, const Divisor &d) { return (int)(((uint64_t)(uint32_t)n * d.mul) >> d.shift); }
+
 struct FwdParams {
     const void *q, *k, *v;
     const uint8_t *mask;  // nullptr = absent
@@ -215,7 +228,10 @@ struct FwdParams {
     // broadcast like the mask
     const uint8_t *mbits;
     int64_t mb_b, mb_h, mb_r;
-    int32_t row_lists;  // log2 of the lists that the row blocks of a pair are dealt to, -1: whole ragged entries (set by row_grid)
+    // set by row_grid for row_unit: log2 of the lists that the row blocks of a pair are dealt to, -1: whole ragged entries; query heads
+    // per kv head; workgroups of a turn of lists, lists side by side in it, kv heads
+    int32_t row_lists;
+    Divisor row_group, row_turn, row_side, row_heads;
 };
 
 // the caller's kv head behind head `hk` of the compaction layer (see FwdParams::kv_share)
@@ -261,32 +277,39 @@ inline int row_grid(FwdParams &p, int bm) {
     const int log_k = n % 8 == 0 ? 0 : (n % 4 == 0 ? 1 : (n % 2 == 0 ? 2 : 3)), k = 1 << log_k;
     const bool whole = p.cu_q && n_mb < k;
     p.row_lists = whole ? -1 : log_k;
-    return (whole ? (p.B * p.Hk + 7) / 8 * 8 * n_mb : p.B * p.Hk * k * ((n_mb + k - 1) / k)) * (p.H / p.Hk);
+    const int G = p.H / p.Hk, list_len = (whole ? n_mb : (n_mb + k - 1) / k) * G, side = p.cu_q && !whole ? p.Hk * k / 8 : 1;
+    p.row_group = divisor(G);
+    p.row_turn = divisor(list_len > 0 ? list_len * side : 1);
+    p.row_side = divisor(side);
+    p.row_heads = divisor(p.Hk);
+    return (whole ? (p.B * p.Hk + 7) / 8 * 8 * n_mb : p.B * p.Hk * k * ((n_mb + k - 1) / k)) * G;
 }
 struct RowUnit {
     int pair, block;  // block < 0: none
+    int b, hk, h;     // of the pair: batch entry and kv head; this workgroup's query head
 };
 __host__ __device__ inline RowUnit row_unit(const FwdParams &p, int id, int bm) {
     const bool whole = p.row_lists < 0;
-    const int log_k = whole ? 0 : p.row_lists, k = 1 << log_k, G = p.H / p.Hk, n_mb = (p.Lq + bm - 1) / bm;
-    const int list_len = ((n_mb + k - 1) >> log_k) * G;
+    const int log_k = whole ? 0 : p.row_lists, k = 1 << log_k, n_mb = (p.Lq + bm - 1) / bm;
     // Of a ragged batch an XCD's lists of one entry run side by side, heaviest blocks first (more than 8 kv heads; one after the other /
     // side by side, forward: seven entries of 300 and one of 2000 x 12/12, d = 128 78 / 56; 2500 and 2500 x 24/12, d = 96 114 / 102).
-    const int side = p.cu_q && !whole ? (p.Hk << log_k) / 8 : 1, slot = id / 8, at = slot % (list_len * side) / G;
-    const int vlist = id % 8 + 8 * (slot / (list_len * side) * side + at % side), pos = at / side;
+    const int slot = id / 8, turn = quotient(slot, p.row_turn), in_turn = slot - turn * (int)p.row_turn.by;
+    const int at = quotient(in_turn, p.row_group), g = in_turn - at * (int)p.row_group.by;
+    const int pos = quotient(at, p.row_side), vlist = id % 8 + 8 * (turn * (int)p.row_side.by + at - pos * (int)p.row_side.by);
     int pair = vlist >> log_k;
     if (whole) {
         pair = (pair & ~7) | ((pair - (pair >> 3)) & 7);
-        if (pair >= p.B * p.Hk) return {0, -1};
+        if (pair >= p.B * p.Hk) return {0, -1, 0, 0, 0};
     }
+    const int b = quotient(pair, p.row_heads), hk = pair - b * p.Hk;
     int blocks = n_mb, fold = vlist & (k - 1);  // of this pair; this list
     if (p.cu_q) {
-        const int b = pair / p.Hk, q0 = p.cu_q[b], own = (p.cu_q[b + 1] - q0 + bm - 1) / bm;
+        const int q0 = p.cu_q[b], own = (p.cu_q[b + 1] - q0 + bm - 1) / bm;
         blocks = own < n_mb ? own : n_mb;  // (rows beyond the longest length that the caller names are not computed)
         fold = (fold - q0 / bm - b) & (k - 1);
     }
     const int rank = (pos << log_k) + fold;  // from the last block down
-    return {pair, rank < blocks ? blocks - 1 - rank : -1};
+    return {pair, rank < blocks ? blocks - 1 - rank : -1, b, hk, hk * (int)p.row_group.by + g};
 }
 
 // Lists of units per (batch, kv head) pair, so that the lists of a ragged batch fill the 8 XCDs: the heads of ONE entry go to
