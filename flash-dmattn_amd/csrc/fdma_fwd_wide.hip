@@ -86,15 +86,28 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     const int shift = LkS - LqS;
     const int wrow0 = m0 + rw * 32, qrow = wrow0 + r;
 
-    // ---- Q fragments: requested first of all, scaled behind the set-up
-    u32x4_t qf[KS];
+    // ---- staging: a piece is 1 KB, whole rows; wave w fetches pieces w + 8 i of Q, of K and of V.  A lane fills chunk position
+    // `lane % CH` of its row, which holds chunk position ^ chunk_swz(row) of the global row; rows 16 apart have the same swizzle.  Rows
+    // beyond the keys (queries) are clamped to the last one (their column says -inf; they are not stored), chunks beyond d to chunk 0 (they
+    // meet zero Q and columns of O that are not stored).
+    const int prow = C::RPP * wave + lane / C::CH;
+    const int pchunk = lane % C::CH ^ (int)chunk_swz<D>(prow);
+    const uint32_t pcol = pchunk * 8 < p.d ? pchunk * 16 : 0;
+
+    // ---- Q, requested first of all: through LDS, where the second stage of K (and of V) comes later, or V where there is one stage.
+    // As fragments straight from memory every load of a wave touches 32 rows, one cache line after another (2.7 clocks each), and every key
+    // group loads them again: of the 8 us that a workgroup of two tiles took at d = 128, 1.7 were spent on the lines of Q.  The kernel
+    // before / now, us: 223 tokens x 32/8 heads, d = 128 11.1 / 9.4; 2 x 128 x 32/8, d = 64 7.4 / 6.1; 2 x 256 x 8/4, d = 256 17.6 / 13.8;
+    // 2304 ragged tokens and others x 16/8, d = 256 133 / 118; 512 rows x 32/8 against 2048 kept of 16384 37.2 / 34.4.
+    static_assert(BM * ROW <= (ONE ? 1 : 2) * TILE, "Q fits there");
+    auto q_at = [](uint32_t byte) { return byte + (ONE || byte >= TILE ? OFF_V : TILE); };  // (V's second stage is as far behind V as K's end behind K)
     {
-        const int qc = qrow < LqS ? qrow : LqS - 1;
-        const uint16_t *qp = (const uint16_t *)p.q + b * p.q_b + (sq.q0 + qc) * p.q_r + h * p.q_h;
+        const gptr_t qb = uniform_ptr((const uint16_t *)p.q + b * p.q_b + (sq.q0 + m0) * p.q_r + h * p.q_h);
+        const uint32_t q_r2 = (uint32_t)(p.q_r * 2), last = (uint32_t)(LqS - 1 - m0 < BM - 1 ? LqS - 1 - m0 : BM - 1) * q_r2;
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const int c = ks * 16 + g * 8;
-            qf[ks] = *(const u32x4_t *)(qp + (c < p.d ? c : 0));  // (chunks beyond d are cleared when scaled)
+        for (int i = 0; i < BM * ROW / 8192; i++) {
+            const uint32_t at = (uint32_t)(prow + 8 * C::RPP * i) * q_r2;
+            load_lds16((at < last ? at : last) + pcol, qb, __builtin_amdgcn_readfirstlane(lds0 + q_at(8192 * i) + wave * 1024));
         }
     }
 
@@ -123,6 +136,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         // (no share under 512 keys: the shares that are then left over only say so)
         const int y = (int)blockIdx.y, most = n_end * BN / 512 > 1 ? n_end * BN / 512 : 1, shares = p.splits < most ? p.splits : most;
         if (y >= shares) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (Q is not to land in what is another workgroup's LDS by then)
             if (tid < BM && m0 + tid < LqS) p.lse_part[(((int64_t)y * p.B + b) * p.H + h) * p.Lq + m0 + tid] = -INFINITY;
             return;
         }
@@ -150,13 +164,15 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
             }
         }
         const uint64_t ball = __ballot(act);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (Q: landed with the mask row, which was requested behind it)
         if (lane == 0) {
             const int w0 = (base + wave * 64) >> 5;
             sBits[w0] = (uint32_t)ball;
             sBits[w0 + 1] = (uint32_t)(ball >> 32);
         }
     }
-    if (!CMP) __syncthreads();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (Q, which the barrier publishes)
+    __syncthreads();
     auto next_active = [&](int j) -> int {  // wave-uniform
         if (CMP) return j < n_end ? j : n_end;
         while (j < n_end) {
@@ -170,12 +186,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         return n_end;
     };
 
-    // ---- staging: a piece is 1 KB, whole rows; wave w fetches pieces w + 8 i of K and of V.  A lane fills chunk position
-    // `lane % CH` of its row, which holds chunk position ^ chunk_swz(row) of the global row; rows 16 apart have the same swizzle.  Rows beyond the keys are clamped to the last one (their column says -inf), chunks beyond d to chunk 0 (they
-    // meet zero Q and columns of O that are not stored).
-    const int prow = C::RPP * wave + lane / C::CH;
-    const int pchunk = lane % C::CH ^ (int)chunk_swz<D>(prow);
-    const uint32_t pcol = pchunk * 8 < p.d ? pchunk * 16 : 0;
+    // K and V of a tile (see above)
     const uint32_t k_r2 = (uint32_t)(p.k_r * 2), v_r2 = (uint32_t)(p.v_r * 2);
     uint32_t k_row = prow * k_r2, v_row = prow * v_r2;  // (offsets grow with the row: clamped by the last row's)
     gptr_t tb_k = nullptr, tb_v = nullptr;
@@ -242,10 +253,24 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         jn = next_active(jc + 1);
         set_tile(jc, 0);
 #pragma unroll
-        for (int n = 0; n < 2 * NP; n++) dma_piece(n);
+        for (int n = 0; n < (ONE ? NP : 2 * NP); n++) dma_piece(n);
     }
-    // Q is scaled by softmax_scale * log2(e) once (the reference also rounds the scaled Q to the input type,
-    // flash_fwd_kernel.h:428-439)
+    // ---- Q fragments (B operands): chunk 2 ks + g of row 32 rw + r, scaled by softmax_scale * log2(e) once (the reference also rounds
+    // the scaled Q to the input type, flash_fwd_kernel.h:428-439)
+    u32x4_t qf[KS];
+    {
+        const int row = 32 * rw + r;
+        const uint32_t at = lds0 + q_at(32 * rw * ROW) + (uint32_t)(r * ROW) + (((uint32_t)g ^ chunk_swz<D>(row)) << 4);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) qf[ks] = lds_ld128((at ^ ((uint32_t)(ks & 7) << 5)) + (uint32_t)(ks >> 3) * 256);
+    }
+    if constexpr (ONE) {  // everybody has read Q: V takes its place
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (jc < n_end) {
+#pragma unroll
+            for (int n = NP; n < 2 * NP; n++) dma_piece(n);
+        }
+    }
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) qf[ks] = scaled8<T>(qf[ks], p.scale_log2, qrow < LqS && ks * 16 + g * 8 < p.d);
     if (jc < n_end) publish();
