@@ -305,6 +305,21 @@ size_t fdma_fwd_workspace_bytes(const fdma_fwd_args *a) {
     return need + shares;
 }
 
+// room for the shares of a general-form call with split keys: O, then LSE
+static size_t general_share_bytes(const fdma::FwdParams &p, int shares) {
+    return shares > 1 ? (size_t)shares * p.B * p.H * p.Lq * (size_t)(p.d + 1) * sizeof(float) : 0;
+}
+static bool general_fwd(const fdma_fwd_args *a, const fdma::FwdParams &p) {
+    return p.Lk > 0 && p.Hk > 0 && !fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k) && !fdma::fwd_colmask_applicable(p);
+}
+
+size_t fdma_fwd_optional_bytes(const fdma_fwd_args *a) {
+    if (!a) return 0;
+    fdma::FwdParams p;
+    fill_fwd_params(a, p);
+    return general_fwd(a, p) ? general_share_bytes(p, fdma::general_key_shares(p, false)) : 0;
+}
+
 int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
     if (int cap = refuse_capture(hip_stream, "fdma_fwd")) return cap;
     g_err[0] = 0;
@@ -353,6 +368,14 @@ int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
                 p.splits = splits;
                 p.o_part = reinterpret_cast<float *>(static_cast<char *>(a->workspace) + base);
                 p.lse_part = p.o_part + (size_t)splits * a->batch * a->num_heads * a->seqlen_q * a->head_dim;
+            }
+        }
+        if (general_fwd(a, p)) {
+            const int shares = fdma::general_key_shares(p, false);
+            if (shares > 1 && a->workspace && aligned16(a->workspace) && a->workspace_bytes >= general_share_bytes(p, shares)) {
+                p.splits = shares;
+                p.o_part = static_cast<float *>(a->workspace);
+                p.lse_part = p.o_part + (size_t)shares * p.B * p.H * p.Lq * p.d;
             }
         }
         e = fdma::launch_fwd(p, a->dtype, stream);
@@ -487,13 +510,29 @@ static void take_kv_parts(fdma::BwdParams &p, void *ws, size_t bytes) {
     }
 }
 
+// what decides whether dQ is made from the dS that dBias is (bwd_dq_from_ds_applicable)
+static void fill_dbias(const fdma_bwd_args *a, fdma::BwdParams &p) {
+    p.dbias = a->dbias;
+    if (a->dbias) { p.db_b = a->dbias_strides[0]; p.db_h = a->dbias_strides[1]; p.db_r = a->dbias_strides[2]; }
+}
+// Shares of a general-form dQ's keys and the room for their fp32 sums (1 and 0: whole rows)
+static int dq_shares(const fdma_bwd_args *a, const fdma::BwdParams &p, size_t *bytes) {
+    const bool apart = !fdma::use_compact(p.f) && general_form(p.f) && (dbias_shared(a) || !fdma::bwd_dq_from_ds_applicable(p));
+    const int shares = apart ? fdma::general_key_shares(p.f, true) : 1;
+    *bytes = shares > 1 ? (size_t)shares * p.f.B * p.f.H * p.f.Lq * p.f.d * sizeof(float) : 0;
+    return shares;
+}
+
 size_t fdma_bwd_optional_bytes(const fdma_bwd_args *a) {
     if (!a || a->f.num_heads_k <= 0) return 0;
     fdma::BwdParams p;
     std::memset(&p, 0, sizeof(p));
     fill_fwd_params(&a->f, p.f);
-    size_t kv;
-    return direct_column_form(p) ? kv_parts_bytes(p, &kv) : 0;
+    fill_dbias(a, p);
+    size_t bytes;
+    if (direct_column_form(p)) return kv_parts_bytes(p, &bytes);
+    dq_shares(a, p, &bytes);
+    return bytes;
 }
 
 int fdma_bwd(const fdma_bwd_args *a, void *hip_stream) {
@@ -503,12 +542,12 @@ int fdma_bwd(const fdma_bwd_args *a, void *hip_stream) {
     fdma::BwdParams p;
     std::memset(&p, 0, sizeof(p));
     fill_fwd_params(&a->f, p.f);
-    p.dout = a->dout; p.dq = a->dq; p.dk = a->dk; p.dv = a->dv; p.dbias = a->dbias;
+    p.dout = a->dout; p.dq = a->dq; p.dk = a->dk; p.dv = a->dv;
     p.do_b = a->do_strides[0]; p.do_r = a->do_strides[1]; p.do_h = a->do_strides[2];
     p.dq_b = a->dq_strides[0]; p.dq_r = a->dq_strides[1]; p.dq_h = a->dq_strides[2];
     p.dk_b = a->dk_strides[0]; p.dk_r = a->dk_strides[1]; p.dk_h = a->dk_strides[2];
     p.dv_b = a->dv_strides[0]; p.dv_r = a->dv_strides[1]; p.dv_h = a->dv_strides[2];
-    if (a->dbias) { p.db_b = a->dbias_strides[0]; p.db_h = a->dbias_strides[1]; p.db_r = a->dbias_strides[2]; }
+    fill_dbias(a, p);
     p.softmax_d = a->softmax_d;
     p.Lq_rounded = (int32_t)round_up(a->f.seqlen_q, 128);
     p.sd_b = (int64_t)a->f.num_heads * p.Lq_rounded;
@@ -524,7 +563,7 @@ int fdma_bwd(const fdma_bwd_args *a, void *hip_stream) {
         p.dba_h = nr * lkr;
         p.dba_b = a->f.bias_strides[0] == 0 ? 0 : p.dba_h * a->f.num_heads_bias;
     }
-    p.kv_segs = p.kv_most = 1;
+    p.kv_segs = p.kv_most = p.dq_shares = 1;
     if (direct_column_form(p)) take_kv_parts(p, a->workspace ? static_cast<char *>(a->workspace) + need : nullptr, a->workspace_bytes - need);
     if (!fdma::use_compact(p.f) && general_form(p.f)) {
         p.kv_segs = fdma::general_kv_segments(p.f);
@@ -533,6 +572,13 @@ int fdma_bwd(const fdma_bwd_args *a, void *hip_stream) {
         char *at = static_cast<char *>(a->workspace) + dbias_accum_bytes(a);
         p.dkv_part = reinterpret_cast<float *>(at);
         p.db_part = reinterpret_cast<float *>(at + kv);
+        size_t room;
+        const int shares = dq_shares(a, p, &room);
+        char *behind = a->workspace ? static_cast<char *>(a->workspace) + need : nullptr;
+        if (shares > 1 && behind && aligned16(behind) && a->workspace_bytes - need >= room) {
+            p.dq_shares = shares;
+            p.dq_part = reinterpret_cast<float *>(behind);
+        }
     }
     hipStream_t stream = static_cast<hipStream_t>(hip_stream);
     hipError_t e;

@@ -40,7 +40,8 @@ template <> struct NegInf2<bf16_tag> { static constexpr uint32_t value = 0xFF80F
 template <> struct NegInf2<fp16_tag> { static constexpr uint32_t value = 0xFC00FC00u; };
 
 // GH query heads of a kv group that share mask and bias rows: a workgroup takes BM / GH query rows of GH heads (see fwd_kernel).
-template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD>
+// SHARES: a workgroup takes one of p.dq_shares shares of the key tiles (an instantiation of its own, as in fwd_kernel).
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD, bool SHARES>
 __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_kernel(const BwdParams p) {
     constexpr int NTHREADS = 64 * NW, BM = 32 * NW / KSPLIT / GH, RB = BM / 32, BN = ((NW == 8 && KSPLIT == 1) || D > 128) ? 32 : 64;
     constexpr int BK = BN / KSPLIT;         // keys of a tile per wave
@@ -108,6 +109,13 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         if (lim < 0) lim = 0;
         const int ne = (lim + BN - 1) / BN;
         if (ne < n_end) n_end = ne;
+    }
+    // this workgroup's share of them (see general_key_shares), whole pairs: the LDS stage of a tile stays a compile-time constant
+    int t_first = 0;
+    if constexpr (SHARES) {
+        const int y = (int)blockIdx.y, twos = (n_end + 1) / 2;
+        t_first = 2 * (twos * y / p.dq_shares);
+        if (y + 1 < p.dq_shares) n_end = 2 * (twos * (y + 1) / p.dq_shares);
     }
 
     f32x16_t dq[DB];
@@ -332,16 +340,16 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
 
     // ---- main loop.  At the top of iteration j: tile j sits in LDS stage j&1 if it is active, the mask of tile j+1 is
     // in registers (finished) and `act_next` says whether that tile has any kept element.
-    if (n_end > 0) {
-        load_mask(0, mreg);
-        if (n_end > 1) load_mask(1, mnext);
-        bool act_cur = __syncthreads_or(finish_mask(0, mreg));
+    if (t_first < n_end) {
+        load_mask(t_first, mreg);
+        if (t_first + 1 < n_end) load_mask(t_first + 1, mnext);
+        bool act_cur = __syncthreads_or(finish_mask(t_first, mreg));
         if (act_cur) {
-            load_rest(0);
-            store_stage(0, mreg);
+            load_rest(t_first);
+            store_stage(t_first, mreg);
         }
         if (DMA) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-        bool act_next = __syncthreads_or(n_end > 1 && finish_mask(1, mnext));
+        bool act_next = __syncthreads_or(t_first + 1 < n_end && finish_mask(t_first + 1, mnext));
         auto step = [&](int j, u32x2_t (&m_next)[F_IT], u32x2_t (&m_new)[F_IT]) {
             const bool have_next = j + 1 < n_end && act_next;
             if (have_next) load_rest(j + 1);
@@ -354,7 +362,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
             act_cur = have_next;
             act_next = act_nn;
         };
-        for (int j = 0; j < n_end; j += 2) {
+        for (int j = t_first; j < n_end; j += 2) {
             step(j, mnext, mreg);
             if (j + 1 < n_end) step(j + 1, mreg, mnext);
         }
@@ -381,6 +389,19 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
                 for (int e = 0; e < 4; e++) dq[db][4 * q + e] += v[e];
             }
     }
+    if constexpr (SHARES) {  // its sums in fp32, which bwd_dq_sum_kernel adds up (zeros where it has no tile)
+        if (qrow < f.Lq) {
+            float *at = p.dq_part + ((((int64_t)blockIdx.y * f.B + b) * f.H + h) * f.Lq + qrow) * f.d;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int c = 32 * db + 16 * (q >> 1) + 8 * g + 4 * (q & 1);
+                    if (c < f.d) *(f32x4_t *)(at + c) = f32x4_t{dq[db][4 * q], dq[db][4 * q + 1], dq[db][4 * q + 2], dq[db][4 * q + 3]};
+                }
+        }
+        return;
+    }
     if (qrow < f.Lq) {
         uint16_t *dqp = (uint16_t *)p.dq + b * p.dq_b + (int64_t)qrow * p.dq_r + h * p.dq_h;
 #pragma unroll
@@ -399,16 +420,47 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
     }
 }
 
-template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD>
+// dQ = scale * sum of the shares, in their order.  A thread has 8 elements of one row.
+template <typename T> __global__ void __launch_bounds__(256) bwd_dq_sum_kernel(const BwdParams p) {
+    using E = Elem<T>;
+    const FwdParams &f = p.f;
+    const int CH = f.d / 8;
+    const int64_t rows = (int64_t)f.B * f.H * f.Lq, at = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (at >= rows * CH) return;
+    const int64_t row = at / CH;
+    const int c = (int)(at % CH) * 8;
+    f32x4_t v[MAX_KEY_SPLITS][2];
+#pragma unroll
+    for (int s = 0; s < MAX_KEY_SPLITS; s++) {
+        v[s][0] = v[s][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (s < p.dq_shares) {
+            v[s][0] = *(const f32x4_t *)(p.dq_part + (s * rows + row) * f.d + c);
+            v[s][1] = *(const f32x4_t *)(p.dq_part + (s * rows + row) * f.d + c + 4);
+        }
+    }
+#pragma unroll
+    for (int s = 1; s < MAX_KEY_SPLITS; s++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) { v[0][0][e] += v[s][0][e]; v[0][1][e] += v[s][1][e]; }
+    const int q = (int)(row % f.Lq), h = (int)(row / f.Lq % f.H), b = (int)(row / f.Lq / f.H);
+    u32x4_t w;
+#pragma unroll
+    for (int e = 0; e < 4; e++) w[e] = E::pack2(v[0][e >> 1][2 * (e & 1)] * f.scale, v[0][e >> 1][2 * (e & 1) + 1] * f.scale);
+    *(u32x4_t *)((uint16_t *)p.dq + b * p.dq_b + q * p.dq_r + h * p.dq_h + c) = w;
+}
+
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD, bool SHARES = false>
 hipError_t launch_dq_o(const BwdParams &p, hipStream_t stream) {
     constexpr int BM = 32 * NW / KSPLIT / GH, NTHREADS = 64 * NW, BN = ((NW == 8 && KSPLIT == 1) || D > 128) ? 32 : 64;
-    auto kern = bwd_dq_kernel<T, D, CAUSAL, NW, KSPLIT, GH, ODD>;
+    if constexpr (!SHARES && (KSPLIT == 2 || NW == 4)) if (p.dq_shares > 1) return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, GH, ODD, true>(p, stream);
+    auto kern = bwd_dq_kernel<T, D, CAUSAL, NW, KSPLIT, GH, ODD, SHARES>;
     constexpr int merge = KSPLIT == 2 ? (NW / 2) * (D / 32) * 4096 : 0;  // the upper halves' sums
     constexpr int smem = DqSmem<D, BM, BN>::TOTAL > merge ? DqSmem<D, BM, BN>::TOTAL : merge;
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
     dim3 grid(((p.f.Lq + BM - 1) / BM) * (p.f.H / GH) * p.f.B);
+    grid.y = p.dq_shares;
     hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
     return hipGetLastError();
 }
@@ -441,7 +493,7 @@ hipError_t launch_dq_c(const BwdParams &p, hipStream_t stream) {
 
 }  // namespace
 
-hipError_t launch_bwd_dq(const BwdParams &p, int dtype, hipStream_t stream) {
+static hipError_t launch_dq_d(const BwdParams &p, int dtype, hipStream_t stream) {
     // head dims up to 64 / 128 / 256 (a head dim in between runs in the next larger instantiation)
     const int dc = p.f.d <= 64 ? 0 : (p.f.d <= 128 ? 1 : 2);
     const bool c = p.f.causal != 0;
@@ -453,6 +505,16 @@ hipError_t launch_bwd_dq(const BwdParams &p, int dtype, hipStream_t stream) {
     if (dc == 0) return c ? launch_dq_c<fp16_tag, 64, true>(p, stream) : launch_dq_c<fp16_tag, 64, false>(p, stream);
     if (dc == 1) return c ? launch_dq_c<fp16_tag, 128, true>(p, stream) : launch_dq_c<fp16_tag, 128, false>(p, stream);
     return c ? launch_dq_c<fp16_tag, 256, true>(p, stream) : launch_dq_c<fp16_tag, 256, false>(p, stream);
+}
+
+hipError_t launch_bwd_dq(const BwdParams &p, int dtype, hipStream_t stream) {
+    const hipError_t e = launch_dq_d(p, dtype, stream);
+    if (e != hipSuccess || p.dq_shares <= 1) return e;
+    const int64_t items = (int64_t)p.f.B * p.f.H * p.f.Lq * (p.f.d / 8);
+    const dim3 grid((unsigned)((items + 255) / 256));
+    if (dtype == 0) hipLaunchKernelGGL(bwd_dq_sum_kernel<bf16_tag>, grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL(bwd_dq_sum_kernel<fp16_tag>, grid, dim3(256), 0, stream, p);
+    return hipGetLastError();
 }
 
 }  // namespace fdma

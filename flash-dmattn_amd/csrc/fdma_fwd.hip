@@ -55,7 +55,8 @@ template <> struct NegInf2<fp16_tag> { static constexpr uint32_t value = 0xFC00F
 
 // GH query heads of a kv group that share mask and bias rows: a workgroup takes BM / GH query rows of GH heads, so that a fused tile
 // is fetched, fused and stored once for all of them.
-template <typename T, int D, bool CAUSAL, int NW, int BN, int KSPLIT, int GH, bool ODD>
+// SHARES: a workgroup takes one of p.splits shares of the key tiles (an instantiation of its own: what it adds costs the others 2 %).
+template <typename T, int D, bool CAUSAL, int NW, int BN, int KSPLIT, int GH, bool ODD, bool SHARES>
 __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_kernel(const FwdParams p) {
     constexpr int NTHREADS = 64 * NW, BK = BN / KSPLIT;  // (BK: keys of a tile per wave)
     constexpr int BM = 32 * NW / KSPLIT / GH, RB = BM / 32;  // query rows and 32-row blocks per head
@@ -122,6 +123,13 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
         if (lim < 0) lim = 0;
         const int ne = (lim + BN - 1) / BN;
         if (ne < n_end) n_end = ne;
+    }
+    // this workgroup's share of them (see general_key_shares), whole pairs: the LDS stage of a tile stays a compile-time constant
+    int t_first = 0;
+    if constexpr (SHARES) {
+        const int y = (int)blockIdx.y, twos = (n_end + 1) / 2;
+        t_first = 2 * (twos * y / p.splits);
+        if (y + 1 < p.splits) n_end = 2 * (twos * (y + 1) / p.splits);
     }
 
     f32x16_t o[DB];
@@ -401,22 +409,22 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     // j+2 are requested at the top of iteration j, behind K / V of tile j+1 (cache hits; waiting for those must not
     // mean waiting for the younger requests: loads come back in the order they were issued).
     constexpr bool DEEP = D <= 64 || KSPLIT == 2;
-    if (n_end > 0 && DEEP) {
+    if (t_first < n_end && DEEP) {
         u32x2_t m1[F_IT], m2[F_IT], m3[F_IT];            // with mreg: the masks of tiles j .. j+3 at the top of iteration j
         u32x4_t b1[F_IT], b2[F_IT];                      // bias of tiles j+1 (requested an iteration ago), j+2
-        load_mask(0, mreg);
-        load_mask(1, m1);
-        load_mask(2, m2);
-        load_mask(3, m3);
-        bool act_cur = __syncthreads_or(finish_mask(0, mreg));
+        load_mask(t_first, mreg);
+        load_mask(t_first + 1, m1);
+        load_mask(t_first + 2, m2);
+        load_mask(t_first + 3, m3);
+        bool act_cur = __syncthreads_or(finish_mask(t_first, mreg));
         if (act_cur) {
-            load_rest(0);
-            store_stage(0, mreg, breg);
+            load_rest(t_first);
+            store_stage(t_first, mreg, breg);
         }
         if (DMA) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-        bool act_1 = __syncthreads_or(n_end > 1 && finish_mask(1, m1));
-        if (act_1) load_bias(1, b1);
-        bool act_2 = __syncthreads_or(n_end > 2 && finish_mask(2, m2));
+        bool act_1 = __syncthreads_or(t_first + 1 < n_end && finish_mask(t_first + 1, m1));
+        if (act_1) load_bias(t_first + 1, b1);
+        bool act_2 = __syncthreads_or(t_first + 2 < n_end && finish_mask(t_first + 2, m2));
         // one iteration; the register sets change roles from one iteration to the next (written out four iterations
         // at a time: a move between sets would have to wait for a load that is still in flight)
         auto step = [&](int j, u32x2_t (&ma)[F_IT], u32x2_t (&mc)[F_IT], u32x2_t (&md)[F_IT], u32x4_t (&ba)[F_IT], u32x4_t (&bb)[F_IT]) {
@@ -438,22 +446,22 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             act_2 = act_3;
         };
 #pragma unroll 1
-        for (int j = 0; j < n_end; j += 4) {
+        for (int j = t_first; j < n_end; j += 4) {
             step(j, m1, m3, mreg, b1, b2);  // (mreg, the set of tile j, is free: it receives tile j+4)
             if (j + 1 < n_end) step(j + 1, m2, mreg, m1, b2, b1);
             if (j + 2 < n_end) step(j + 2, m3, m1, m2, b1, b2);
             if (j + 3 < n_end) step(j + 3, mreg, m2, m3, b2, b1);
         }
-    } else if (n_end > 0) {
-        load_mask(0, mreg);
-        if (n_end > 1) load_mask(1, mnext);
-        bool act_cur = __syncthreads_or(finish_mask(0, mreg));
+    } else if (t_first < n_end) {
+        load_mask(t_first, mreg);
+        if (t_first + 1 < n_end) load_mask(t_first + 1, mnext);
+        bool act_cur = __syncthreads_or(finish_mask(t_first, mreg));
         if (act_cur) {
-            load_rest(0);
-            store_stage(0, mreg, breg);
+            load_rest(t_first);
+            store_stage(t_first, mreg, breg);
         }
         if (DMA) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-        bool act_next = __syncthreads_or(n_end > 1 && finish_mask(1, mnext));
+        bool act_next = __syncthreads_or(t_first + 1 < n_end && finish_mask(t_first + 1, mnext));
         // one iteration; `m_next` holds the (finished) mask of tile j+1, `m_new` receives the mask of tile j+2.
         // The scheduling barriers keep the loads at the top and their first use below the compute: their
         // latency is then covered by the MFMA work instead of being waited for right away.
@@ -469,7 +477,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             act_cur = have_next;
             act_next = act_nn;
         };
-        for (int j = 0; j < n_end; j += 2) {
+        for (int j = t_first; j < n_end; j += 2) {
             step(j, mnext, mreg);
             if (j + 1 < n_end) step(j + 1, mreg, mnext);
         }
@@ -508,6 +516,21 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             }
     }
     const float inv = total > 0.f ? 1.f / total : 0.f;
+    if constexpr (SHARES) {  // O in fp32 and its log2-sum-exp, which fwd_merge_kernel adds up
+        if (qrow < p.Lq) {
+            const int64_t at = (((int64_t)blockIdx.y * p.B + b) * p.H + h) * p.Lq + qrow;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int c = 32 * db + 16 * (q >> 1) + 8 * g + 4 * (q & 1);
+                    if (c < p.d) *(f32x4_t *)(p.o_part + at * p.d + c) = f32x4_t{o[db][4 * q] * inv, o[db][4 * q + 1] * inv, o[db][4 * q + 2] * inv, o[db][4 * q + 3] * inv};
+                }
+            // (a sum that is no number has to reach the result: only an empty share is left out)
+            if (g == 0) p.lse_part[at] = total == 0.f ? -INFINITY : row_max + __builtin_amdgcn_logf(total);
+        }
+        return;
+    }
     if (qrow < p.Lq) {
         uint16_t *op = (uint16_t *)p.o + b * p.o_b + (int64_t)qrow * p.o_r + h * p.o_h;
 #pragma unroll
@@ -530,16 +553,18 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
     }
 }
 
-template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD>
+template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD, bool SHARES = false>
 hipError_t launch_fwd_o(const FwdParams &p, hipStream_t stream) {
     constexpr int BM = 32 * NW / KSPLIT / GH, NTHREADS = 64 * NW, BN = D > 128 ? 32 : BN_DEFAULT;
-    auto kern = fwd_kernel<T, D, CAUSAL, NW, BN, KSPLIT, GH, ODD>;
+    if constexpr (!SHARES && (KSPLIT == 2 || NW == 4)) if (p.splits > 1) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, GH, ODD, true>(p, stream);
+    auto kern = fwd_kernel<T, D, CAUSAL, NW, BN, KSPLIT, GH, ODD, SHARES>;
     constexpr int merge = KSPLIT == 2 ? (NW / 2) * 512 + (NW / 2) * (D / 32) * 4096 : 0;  // the upper halves' sums
     constexpr int smem = FwdSmem<D, BM, BN>::TOTAL > merge ? FwdSmem<D, BM, BN>::TOTAL : merge;
     static DynSmemLimit smem_limit;
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
     dim3 grid(((p.Lq + BM - 1) / BM) * (p.H / GH) * p.B);
+    grid.y = p.splits;
     hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
     return hipGetLastError();
 }
@@ -583,12 +608,37 @@ int shared_rows(const FwdParams &p) {
     return p.d > 64 && G % 2 == 0 ? 2 : 1;
 }
 
+// Shares that the key tiles of a row block are cut into, forward and dQ.  A workgroup's time is its chain of tiles (1.5 us each at head dims up
+// to 128, 2.5 per 32 keys above), and few heads or short rows leave most CUs without one.
+//   * As many as the chip holds workgroups at once (one per CU; d <= 64: two, three of 32-row ones), rounded DOWN: 64 blocks of 1000 rows,
+//     d = 128: 4 shares 25.1 us, 5 31.5; 188 blocks 43.1 whole, 48.4 in three.
+//   * Four tiles each at least, and at head dims 65 to 128, where a tile takes 1.1 us, twelve in all: below, the fp32 results, written and
+//     read again, and the launch that adds them up cost more than the tiles (d = 128, whole / in two: 4 x 300 x 8/4 16.6 / 21.8,
+//     4 x 478 x 8/4 19.8 / 23.3; d = 64, 2 x 704 x 16/16 25.8 / 23.5); above 128 twelve where there are more than CUs / 4 blocks (4 x 256
+//     x 16/8 125 / 130 with the backward, 256 x 2/1 24.5 / 21.4).
+//   * dQ from 24 tiles on (16 of 32 keys): below, a backward is bound by its launches, of which this is one more (1024 x 2/1,
+//     d = 128: 66.9 and 69 to 72).
+// Whole / shares, us (forward; backward with its other kernels): 2316 x 2/1 heads, d = 256 162 / 46, 323 / 180; 3000 x 2/1, d = 64 83 / 25,
+// 141 / 75; 2240 x 2/1, d = 96 56 / 24, 107 / 72; 4096 x 2/1, d = 128 98 / 39, 172 / 106; 3000 x 8/2, d = 64 81 / 41, 198 / 171; 1999 x 8/4,
+// not causal 61 / 43, 138 / 119.
+int general_key_shares(const FwdParams &p, bool dq) {
+    if (p.cu_q || p.Lq < 1 || p.Lk < 1) return 1;
+    const int gh = shared_rows(p), rows = 128 / gh, tile = p.d > 128 ? 32 : 64, tiles = (p.Lk + tile - 1) / tile;
+    if (dq && tiles < (p.d > 128 ? 16 : 24)) return 1;
+    const int64_t blocks = (int64_t)((p.Lq + rows - 1) / rows) * (p.H / gh) * p.B;
+    int64_t s = blocks > 0 ? device_cus() * (p.d > 64 ? 1 : (gh == 4 ? 3 : 2)) / blocks : 1;
+    if (s > tiles / 4) s = tiles / 4;
+    if (p.d > 64 && tiles < 12 && (p.d <= 128 || 4 * blocks > device_cus())) return 1;
+    return s < 2 ? 1 : (s > MAX_KEY_SPLITS ? MAX_KEY_SPLITS : (int)s);
+}
+
 hipError_t launch_fwd(const FwdParams &p, int dtype, hipStream_t stream) {
     if (p.Lq <= 0 || p.B <= 0) return hipSuccess;
     if (fwd_colmask_applicable(p)) return launch_fwd_colmask(p, dtype, stream);
     // head dims up to 64 / 128 / 256 (a head dim in between runs in the next larger instantiation)
-    if (dtype == 0) return p.d <= 64 ? launch_fwd_t<bf16_tag, 64>(p, stream) : p.d <= 128 ? launch_fwd_t<bf16_tag, 128>(p, stream) : launch_fwd_t<bf16_tag, 256>(p, stream);
-    return p.d <= 64 ? launch_fwd_t<fp16_tag, 64>(p, stream) : p.d <= 128 ? launch_fwd_t<fp16_tag, 128>(p, stream) : launch_fwd_t<fp16_tag, 256>(p, stream);
+    const hipError_t e = dtype == 0 ? (p.d <= 64 ? launch_fwd_t<bf16_tag, 64>(p, stream) : p.d <= 128 ? launch_fwd_t<bf16_tag, 128>(p, stream) : launch_fwd_t<bf16_tag, 256>(p, stream))
+                                    : (p.d <= 64 ? launch_fwd_t<fp16_tag, 64>(p, stream) : p.d <= 128 ? launch_fwd_t<fp16_tag, 128>(p, stream) : launch_fwd_t<fp16_tag, 256>(p, stream));
+    return e != hipSuccess || p.splits <= 1 ? e : launch_fwd_merge(p, dtype, stream);
 }
 
 }  // namespace fdma

@@ -772,7 +772,6 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
 // 0 and +inf).  A thread has 8 elements of one row; the rows of O of a share without a visible key hold nothing and are not read.
 // Only such a share, l_s = -inf, is left out: an l_s that is no number (a NaN among its keys or in the query) has a weight that is
 // none either, which makes the row what the call with whole keys makes it.
-constexpr int MAX_KEY_SPLITS = 8;
 template <typename T> __global__ void __launch_bounds__(256) fwd_merge_kernel(const FwdParams p) {
     using E = Elem<T>;
     const int CH = p.d / 8;
@@ -857,6 +856,10 @@ hipError_t launch_d(const FwdParams &p, hipStream_t stream) {
 
 }  // namespace
 
+hipError_t launch_fwd_merge(const FwdParams &p, int dtype, hipStream_t stream) {
+    return dtype == 0 ? launch_merge<bf16_tag>(p, stream) : launch_merge<fp16_tag>(p, stream);
+}
+
 // Shares that the key tiles of a row block are cut into: a chunk of a prompt against a long cache has too few row blocks for the
 // chip, and a workgroup's time is the chain of its tiles.  The shares' fp32 results cost what they weigh -- 256 workgroups of 128 rows
 // wrote and read 17 MB, 12 us, and two shares of 128 blocks were no faster than none -- so at most 128 blocks of 128 rows, and only
@@ -910,7 +913,7 @@ hipError_t launch_fwd_colmask(const FwdParams &p, int dtype, hipStream_t stream)
     if (takes_key_groups(p)) {  // (and all calls in shares: three shares are at most a third of a 64-row block per CU, see key_shares)
         const hipError_t e = launch_fwd_wide(p, dtype, stream);
         if (e != hipSuccess || !p.cmp.on || p.splits <= 1) return e;
-        return dtype == 0 ? launch_merge<bf16_tag>(p, stream) : launch_merge<fp16_tag>(p, stream);
+        return launch_fwd_merge(p, dtype, stream);
     }
     if (dtype == 0) return p.d <= 64 ? launch_d<bf16_tag, 64>(p, stream) : launch_d<bf16_tag, 128>(p, stream);
     return p.d <= 64 ? launch_d<fp16_tag, 64>(p, stream) : launch_d<fp16_tag, 128>(p, stream);

@@ -342,6 +342,9 @@ struct BwdParams {
     // lengths on the device), units per (batch, kv head) pair -- ragged: per kv head.  Per part [2][Dpad][128] fp32 (dK, dV, in
     // register order) in dkv_part and [G][128] fp32 (dBias columns) in db_part
     int32_t kv_most, kv_quota, kv_units;
+    // general form, dQ: shares that the key tiles of a row block are cut into (1: none), and their fp32 sums (shares, B, H, Lq, d)
+    int32_t dq_shares;
+    float *dq_part;
     int32_t dot_done;          // softmax_d has been computed by an earlier launch of this call
     int32_t red_first, red_count;  // compacted backward: workgroups of the dQ launch that sum the dK/dV partials (see place_reduction)
     float red_wait;                // how much of dQ waits for a CU beside them, 0 .. 1
@@ -423,6 +426,12 @@ int64_t fwd_blocks64(const FwdParams &p);  // 64-row blocks of all heads (ragged
 // compacted forward: shares the keys of a row block are cut into (1: none); p.o_part / p.lse_part then hold
 // splits * B * H * Lq rows of d / 1 floats
 int fwd_key_splits(const FwdParams &p);
+constexpr int MAX_KEY_SPLITS = 8;
+// adds the shares of a forward call up
+hipError_t launch_fwd_merge(const FwdParams &p, int dtype, hipStream_t stream);
+// general form (mask or bias per query): shares that the key tiles of a row block are cut into (1: none), forward or dQ; what
+// they leave lies in o_part / lse_part or BwdParams::dq_part
+int general_key_shares(const FwdParams &p, bool dq);
 int key_shares(const FwdParams &p);  // ... as far as the sizes go: what they would be if the keys were compacted
 // compacted forward on tile images (fdma_fwd_stream.hip): resident workgroups that walk their share of the
 // (query block, head) items with the tiles of the next item already on their way.  `fwd_stream_applicable` decides from

@@ -45,6 +45,7 @@ struct Api {
     decltype(&::fdma_fwd) fwd;
     decltype(&::fdma_bwd) bwd;
     decltype(&::fdma_fwd_workspace_bytes) fwd_workspace_bytes;
+    decltype(&::fdma_fwd_optional_bytes) fwd_optional_bytes;
     decltype(&::fdma_bwd_workspace_bytes) bwd_workspace_bytes;
     decltype(&::fdma_bwd_optional_bytes) bwd_optional_bytes;
     decltype(&::fdma_fwd_counter_bytes) fwd_counter_bytes;
@@ -383,6 +384,12 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
                 a.counters_bytes = c.nbytes();
             }
     }
+    Tensor shares;  // (of the call alone: the node does not keep it)
+    if (!need)
+        if (size_t room = api.fwd_optional_bytes(&a)) {
+            shares = scratch_with_room(0, room, opt);
+            if (room) { a.workspace = shares.data_ptr(); a.workspace_bytes = room; }
+        }
     check(api.fwd(&a, stream));
     if (is_grad) {
         torch::autograd::set_history(out, node);
@@ -714,6 +721,7 @@ PyObject *bind(PyObject *, PyObject *dict) {
     FDMA_BIND(fwd);
     FDMA_BIND(bwd);
     FDMA_BIND(fwd_workspace_bytes);
+    FDMA_BIND(fwd_optional_bytes);
     FDMA_BIND(bwd_workspace_bytes);
     FDMA_BIND(bwd_optional_bytes);
     FDMA_BIND(fwd_counter_bytes);

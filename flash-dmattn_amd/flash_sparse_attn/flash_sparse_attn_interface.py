@@ -267,6 +267,10 @@ def _flash_sparse_attn_forward_body(
             if nbytes:
                 workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
                 args.workspace, args.workspace_bytes = workspace.data_ptr(), nbytes
+            else:
+                shares = _scratch_with_room(0, _cabi.lib.fdma_fwd_optional_bytes(args), q.device)
+                if shares is not None:
+                    args.workspace, args.workspace_bytes = shares.data_ptr(), shares.numel()
         _cabi.check(_cabi.lib.fdma_fwd(args, stream))
     items = getattr(_tls, "items", None)
     per_query_head = mask is not None and mask.shape[1] == num_heads and num_heads != k.shape[2]

@@ -212,12 +212,16 @@ int fdma_set_stream_min_items(int n);
 /* Scratch the caller must provide.  0 when none is needed.  Validate nothing but shapes.  Ask with the arguments of the call itself:
  * which tensors there are counts too (a decode call without a mask keeps every key and can take more splits than one with). */
 size_t fdma_fwd_workspace_bytes(const fdma_fwd_args *args);
+/* Scratch that a forward call with a mask or bias per query can use (0: none): with workspace_bytes of at least this many the keys of
+ * few query rows are cut into shares, whose fp32 results lie there; with less they stay whole.  Nothing of it outlives the call. */
+size_t fdma_fwd_optional_bytes(const fdma_fwd_args *args);
 /* Size of the optional arrival counters (fdma_fwd_args.counters); 0 when the call would not use them. */
 size_t fdma_fwd_counter_bytes(const fdma_fwd_args *args);
 size_t fdma_bwd_workspace_bytes(const fdma_bwd_args *args);
 /* Further scratch that a backward call can use (0: none): with workspace_bytes of at least fdma_bwd_workspace_bytes() plus this
  * many, key blocks that many queries see are cut into parts, whose fp32 sums lie there; with less they stay whole, and the call
- * takes longer where the chip is not full.  Up to 512 MB and the parts' dBias columns: a caller that is short of memory leaves it out. */
+ * takes longer where the chip is not full.  Up to 512 MB and the parts' dBias columns: a caller that is short of memory leaves it out.
+ * With a mask or bias per query: fp32 sums of dQ, of few query rows' keys in shares. */
 size_t fdma_bwd_optional_bytes(const fdma_bwd_args *args);
 
 /* Argument validation only (no GPU work, callable on a host without a device). */

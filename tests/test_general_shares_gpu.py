@@ -1,0 +1,73 @@
+"""Few query rows of the general form, whose key tiles are cut into shares: at the edges of tiles, of shares and of the head
+dims that a kernel serves, against the C oracle and against the same call with whole keys (the shares' results are fp32, so the two
+differ by the last rounding to 16 bits and, where probabilities are rounded against another reference point, by that)."""
+import pytest
+import torch
+
+from oracle import c_oracle
+from _util import assert_grad_close, assert_out_close
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+CASES = [
+    # B, Lq, Lk, H, Hk, d, mask heads, bias heads, causal
+    (1, 512, 512, 2, 1, 64, 1, 1, True),       # two shares; the first rows see no tile of the second
+    (1, 70, 1537, 2, 1, 64, 1, 1, False),      # a last tile of one key, alone behind its pair
+    (1, 40, 1600, 4, 1, 64, 1, 0, True),       # four heads to a workgroup, no bias
+    (2, 33, 1543, 4, 2, 128, 2, 2, True),      # two heads to a workgroup, two key halves; odd rows
+    (1, 130, 1600, 1, 1, 96, 0, 1, False),     # no mask
+    (1, 577, 577, 2, 1, 256, 1, 1, True),      # tiles of 32 keys
+    (1, 65, 520, 2, 2, 136, 2, 1, False),
+    (1, 1700, 1100, 1, 1, 128, 1, 1, True),    # rows without a key
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x) for x in c))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_shares_vs_oracle_and_whole(case, dtype, monkeypatch):
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func
+
+    print(case, dtype, flush=True)
+    B, Lq, Lk, H, Hk, d, hm, hb, causal = case
+    g = torch.Generator().manual_seed(Lq + Lk)
+    r = lambda *s: torch.randn(*s, generator=g).to(dtype)
+    q, k, v, dout = r(B, Lq, H, d), r(B, Lk, Hk, d), r(B, Lk, Hk, d), r(B, Lq, H, d)
+    mask = torch.rand(B, hm, Lq, Lk, generator=g) < 0.3 if hm else None
+    if mask is not None:
+        mask[:, :, : Lq // 2, Lk // 3:] = False  # whole shares without a kept key
+        mask[:, :, 3] = False                     # and a row without any
+    bias = r(B, hb, Lq, Lk) if hb else None
+    ro, rl = c_oracle.forward(q, k, v, mask, bias, d ** -0.5, causal)
+    ref = c_oracle.backward(q, k, v, dout, mask, bias, d ** -0.5, causal)
+    leaves = [t.to(DEV).requires_grad_(True) for t in (q, k, v)] + ([bias.to(DEV).requires_grad_(True)] if hb else [])
+    asked = {"fdma_fwd_optional_bytes": [], "fdma_bwd_optional_bytes": []}
+
+    def run():
+        out, lse, _ = flash_sparse_attn_func(*leaves[:3], None if mask is None else mask.to(DEV), leaves[3] if hb else None, None, causal, return_attn_probs=True)
+        return (out, lse) + torch.autograd.grad(out, leaves, dout.to(DEV))
+
+    native = run()
+    monkeypatch.setattr(_cabi, "host", _cabi._NoHost)  # (the Python path makes the calls)
+    for name, seen in asked.items():
+        fn = getattr(_cabi.lib, name)
+        monkeypatch.setattr(_cabi.lib, name, lambda a, fn=fn, seen=seen: seen.append(fn(a)) or seen[-1])
+    shares = run()
+    assert asked["fdma_fwd_optional_bytes"][0] > 0
+    for name in asked:
+        monkeypatch.setattr(_cabi.lib, name, lambda a: 0)
+    whole = run()
+    assert_out_close(shares[0].cpu(), ro)
+    finite = torch.isfinite(rl)
+    got = shares[1].cpu()
+    assert torch.equal(torch.isfinite(got), finite) and (got[finite] - rl[finite]).abs().max() < 1e-2
+    for x, want, name in zip(shares[2:], ref, ("dq", "dk", "dv", "dbias")):
+        assert_grad_close(x.cpu(), want, name)
+    eps = torch.finfo(dtype).eps
+    for i, (a, b, c) in enumerate(zip(shares, whole, native)):
+        assert torch.equal(a, c), i
+        if i == 1:
+            ok = (a == b) | ((a - b).abs() <= 1e-5 * (1 + b.abs()))
+        else:  # (a probability is rounded to eps / 2 of itself against either reference point; sums of many of them, and what LSE and O carry on)
+            ok = (a.float() - b.float()).abs() <= eps * (2 * b.float().abs() + b.float().abs().max())
+        assert ok.all(), i
