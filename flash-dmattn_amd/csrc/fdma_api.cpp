@@ -277,7 +277,7 @@ int fdma_set_stream_min_items(int n) {
 
 size_t fdma_fwd_counter_bytes(const fdma_fwd_args *a) {
     if (!a || a->seqlen_k <= 0 || a->num_heads_k <= 0 || !fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k)) return 0;
-    return (size_t)round_up(fdma::decode_num_counters(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k) * 4, 256);
+    return (size_t)round_up(fdma::decode_num_counters(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->head_dim) * 4, 256);
 }
 
 // scratch of a forward call: what it cannot do without, and -- `shares` -- room for the shares of split keys behind it
@@ -293,7 +293,7 @@ static size_t fwd_scratch_bytes(const fdma_fwd_args *a, size_t *shares) {
         if (splits > 1) *shares = (size_t)splits * a->batch * a->num_heads * a->seqlen_q * (size_t)(a->head_dim + 1) * sizeof(float);
         return (size_t)round_up(fdma::compact_bytes(p, false), 256);
     }
-    const int splits = fdma::decode_num_splits(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->mask != nullptr);
+    const int splits = fdma::decode_num_splits(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->head_dim, a->mask != nullptr);
     if (splits <= 1) return 0;
     const size_t rows = (size_t)splits * a->batch * a->num_heads * a->seqlen_q;
     return rows * (size_t)(a->head_dim + 1) * sizeof(float);
@@ -331,7 +331,7 @@ int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
     hipError_t e;
     if (a->seqlen_q == 0) return FDMA_OK;
     if (fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k) && a->seqlen_k > 0) {
-        p.splits = fdma::decode_num_splits(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->mask != nullptr);
+        p.splits = fdma::decode_num_splits(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->head_dim, a->mask != nullptr);
         if (p.splits > 1) {
             const size_t need = fdma_fwd_workspace_bytes(a);
             if (!a->workspace || a->workspace_bytes < need)

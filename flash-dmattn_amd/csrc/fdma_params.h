@@ -527,9 +527,9 @@ inline bool odd_rows(const FwdParams &f) {
 int device_cus();
 
 // number of KV splits the decode path uses for this shape, with a mask or without (1 = no workspace needed)
-int decode_num_splits(int B, int H, int Hk, int Lk, bool masked);
+int decode_num_splits(int B, int H, int Hk, int Lk, int d, bool masked);
 // arrival counters the one-launch decode needs for this shape (0 without splits)
-int64_t decode_num_counters(int B, int H, int Hk, int Lk);
+int64_t decode_num_counters(int B, int H, int Hk, int Lk, int d);
 bool use_decode_path(int Lq, int H, int Hk);
 
 }  // namespace fdma

@@ -59,6 +59,31 @@ def test_splits_without_a_mask(B, H, Hk, Lk, masked, unmasked):
     assert _cabi.lib.fdma_fwd_workspace_bytes(a) == masked * (256 + 1) * 4 * B * H and _cabi.lib.fdma_fwd_counter_bytes(a) == counters
 
 
+@pytest.mark.parametrize("B,Lk,Hk,D,splits", [
+    (5, 20096, 8, 256, 6),    # 240 workgroups of the 256 that run at once above head dim 128
+    (11, 41381, 16, 256, 1),
+    (10, 9000, 8, 128, 3),
+    (9, 1595, 16, 96, 1),
+    (10, 16384, 8, 128, 3),   # 240 are enough ...
+    (11, 16384, 8, 128, 5),   # ... 176 are not: two to a CU
+    (11, 16383, 8, 128, 2),
+    (8, 65536, 8, 128, 8),    # two to a CU, spans of 8192
+    (8, 65535, 8, 128, 4),
+    (12, 61888, 16, 64, 4),   # three
+    (11, 8192, 8, 64, 5),
+    (300, 65536, 1, 128, 1),
+    (2, 4093, 64, 256, 2),
+])
+def test_workgroups_that_run_at_once(B, Lk, Hk, D, splits):
+    from flash_sparse_attn import _cabi
+
+    a = _cabi.FwdArgs()
+    a.batch, a.seqlen_q, a.seqlen_k, a.num_heads, a.num_heads_k, a.head_dim = B, 1, Lk, Hk, Hk, D
+    a.mask = 256  # (there is one; sizes alone are looked at)
+    assert _cabi.lib.fdma_fwd_workspace_bytes(a) == (splits * (D + 1) * 4 * B * Hk if splits > 1 else 0)
+    assert (_cabi.lib.fdma_fwd_counter_bytes(a) > 0) == (splits > 1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,Lk,H,Hk,D,kept,splits,dtype", [
     (1, 384, 2, 1, 128, 384, 1, torch.bfloat16),     # the longest call of one split
