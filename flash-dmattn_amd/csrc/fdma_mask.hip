@@ -12,7 +12,7 @@
 // A row is a chain of dependent steps with hardly any bytes, so make_mask_kernel keeps it in registers from the one load
 // to the last output: a thread holds KPT chunks of 8 columns; every wave finds the bins for itself (no broadcast, five
 // barriers in all), and mask, bit row and the list of kept columns come out of one prefix sum over the workgroup.  (Passes
-// over memory for each step, the list from the stored mask: 64 rows of 4093 keys 16.7 us, now 8.1.)  Rows of fewer than 8
+// over memory for each step, the list from the stored mask: 64 rows of 4093 keys 16.7 us, in registers 8.1, two columns an instruction 6.1.)  Rows of fewer than 8
 // or more than 65536 keys and block smoothing take make_mask_memory_kernel, which walks the row in memory.
 //
 // As in the reference, entries excluded by an incoming mask are pushed to `min_value` before the selection, and a
@@ -83,12 +83,36 @@ __device__ __forceinline__ void find_bin_wave(const uint32_t *h, uint32_t k, uin
     above = __builtin_amdgcn_readlane(mine_above, l);
 }
 
+// ---- pairs of 16-bit values in one register
+typedef __attribute__((ext_vector_type(2))) uint16_t u16x2_t;
+typedef __attribute__((ext_vector_type(2))) int16_t s16x2_t;
+__device__ __forceinline__ uint32_t order_keys(uint32_t x) {  // order_key of both
+    const uint32_t sign = __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16x2_t, x) >> (s16x2_t){15, 15});
+    return x ^ (sign | 0x80008000u);
+}
+// one where a half of x is not zero
+__device__ __forceinline__ uint32_t not_zero2(uint32_t x) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2_t, x), (u16x2_t){1, 1}));
+}
+// one where a half of x is above that of t
+__device__ __forceinline__ uint32_t above2(uint32_t x, uint32_t t) {
+    return not_zero2(__builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2_t, x), __builtin_bit_cast(u16x2_t, t))));
+}
+// the ones of four pairs (columns 2 e, 2 e + 1 of a chunk), gathered as acc |= ones << 2 e, as a bit per column
+__device__ __forceinline__ uint32_t column_bits(uint32_t acc) { return (acc & 0x55u) | ((acc >> 15) & 0xaau); }
+
 // One row in registers: NT threads, chunk c of thread t = columns (c * NT + t) * 8 .. + 7.  Lk >= 8, Lk <= NT * 8 * KPT.
+//
+// Bound by the vector instructions of the one CU that has the row (its load and its barriers are 3 us).  The columns are kept as ordered
+// keys, two to a register, and what is compared, filled and counted is two columns an instruction: some 25 instructions a column,
+// where one at a time, the key made again in each pass, was 60.  Kept and tied columns share a prefix sum, and the list leaves through LDS.
+// Before / now, us (2.5 of them the launch): 64 rows of 4093, 1024 kept 7.2 / 6.1; 4 of 8000, 1024 8.3 / 6.9; 8 of 15738, 1524 12.0 / 9.6; 2 of 26876,
+// 3072 17.6 / 13.2, all of them 27.2 / 12.8; 2 of 60000, 4096 37.4 / 21.4; 8192 rows of 4096 (bit rows) 56.1 / 35.9.
 template <int NT, int KPT>
 __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
-    constexpr int NW = NT / 64, REP1 = NT >= 512 ? 16 : 8, REP2 = 4;
-    __shared__ uint32_t hist1[256 * REP1], hist2[256 * REP2], hsum[2][256];
-    __shared__ uint32_t s_tot[2][KPT * NW];
+    constexpr int NW = NT / 64, LOG1 = NT >= 512 ? 4 : 3, REP1 = 1 << LOG1, LOG2 = 2, REP2 = 1 << LOG2;
+    __shared__ __attribute__((aligned(16))) uint32_t hist1[256 * REP1], hist2[256 * REP2], hsum[2][256];
+    __shared__ uint32_t s_tot[KPT * NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int row = blockIdx.x;
     const int r = row % p.rows, h = (row / p.rows) % p.heads, b = row / (p.rows * p.heads);
@@ -96,9 +120,15 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
     const uint8_t *mrow = p.mask_in ? p.mask_in + b * p.mi_b + h * p.mi_h + (int64_t)r * p.mi_r : nullptr;
     uint8_t *orow = p.mask_out + b * p.mo_b + h * p.mo_h + (int64_t)r * p.mo_r;
     const int Lk = p.Lk;
-    const uint32_t min_bits = p.min_bits;
+    const uint32_t min_key = order_key(p.min_bits);
+    const bool min_zero = (p.min_bits & 0x7fffu) == 0;  // ("is the fill value" compares numerically: +0 == -0)
     auto first_col = [&](int c) -> int { return (c * NT + tid) * 8; };
-    // ---- the row, after the masked fill, as bits of the bias type
+    auto valid = [&](int c) -> int {  // columns of the chunk inside the row
+        const int n = Lk - first_col(c);
+        return n >= 8 ? 8 : (n < 0 ? 0 : n);
+    };
+    // ---- the row, after the masked fill, as ordered keys.  Columns beyond its end: the lowest key, which moves no threshold (there are
+    // at least k columns inside); their bits are dropped at the end
     uint32_t v[KPT][4];
     {
         u32x4_t raw[KPT];
@@ -108,49 +138,69 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
             raw[c] = *(const u32x4_el_t *)(brow + chunk8_at<true>(first_col(c), Lk));
             if (mrow) mm[c] = *(const u32x2_any_t *)(mrow + chunk8_at<true>(first_col(c), Lk));
         }
-        for (int i = tid; i < 256 * REP1; i += NT) hist1[i] = 0;
-        for (int i = tid; i < 256 * REP2; i += NT) hist2[i] = 0;
+        for (int i = tid; i < 64 * REP1; i += NT) ((u32x4_t *)hist1)[i] = u32x4_t{0, 0, 0, 0};
+        for (int i = tid; i < 64 * REP2; i += NT) ((u32x4_t *)hist2)[i] = u32x4_t{0, 0, 0, 0};
+        const uint32_t fill = min_key | (min_key << 16);
 #pragma unroll
         for (int c = 0; c < KPT; c++) {
             const u32x4_t x = chunk8_fix<true>(raw[c], first_col(c), Lk);
-            const u32x2_t m = mrow ? chunk8_fix_mask<true>(mm[c], first_col(c), Lk) : u32x2_t{0x01010101u, 0x01010101u};
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t two = m[e >> 1] >> (16 * (e & 1));
-                const uint32_t lo = (two & 0xffu) ? x[e] & 0xffffu : min_bits, hi = (two & 0xff00u) ? x[e] >> 16 : min_bits;
-                v[c][e] = lo | (hi << 16);
+            for (int e = 0; e < 4; e++) v[c][e] = order_keys(x[e]);
+            if (mrow) {
+                const u32x2_t m = chunk8_fix_mask<true>(mm[c], first_col(c), Lk);
+#pragma unroll
+                for (int hlf = 0; hlf < 2; hlf++) {
+                    uint32_t o = m[hlf];
+                    o = ((((o & 0x7f7f7f7fu) + 0x7f7f7f7fu) | o) >> 7) & 0x01010101u;  // nonzero byte -> 0x01
+                    const uint32_t z = (o << 8) - o;                                     // 0x01 -> 0xFF per byte
+                    const uint32_t k0 = __builtin_amdgcn_perm(0, z, 0x01010000u), k1 = __builtin_amdgcn_perm(0, z, 0x03030202u);
+                    v[c][2 * hlf] = (v[c][2 * hlf] & k0) | (fill & ~k0);
+                    v[c][2 * hlf + 1] = (v[c][2 * hlf + 1] & k1) | (fill & ~k1);
+                }
+            }
+            const int n = valid(c);
+            if (n < 8) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[c][e] &= (n > 2 * e ? 0xffffu : 0u) | (n > 2 * e + 1 ? 0xffff0000u : 0u);
             }
         }
     }
-    auto bits_of = [&](int c, int j) -> uint32_t { return (v[c][j >> 1] >> (16 * (j & 1))) & 0xffffu; };
-    auto valid = [&](int c) -> int {  // columns of the chunk inside the row
-        const int n = Lk - first_col(c);
-        return n >= 8 ? 8 : (n < 0 ? 0 : n);
-    };
-    // "is the fill value" compares numerically (+0 == -0)
-    auto is_min = [&](uint32_t x) -> bool { return x == min_bits || (((x | min_bits) & 0x7fffu) == 0); };
-    // exclusive prefix, in column order, of a count per chunk: inside the wave (which leaves its totals), and -- behind a
-    // barrier -- of the totals, which every wave sums for itself, two per lane; returns the row's
-    auto prefix_wave = [&](uint32_t *tot, const int (&n)[KPT], int (&before)[KPT]) {
+    // exclusive prefix, in column order, of a count per chunk -- or of two, in the halves of a register --: inside the wave (which leaves its
+    // totals), and -- behind a barrier -- of the totals, which every wave sums for itself, two per lane; returns the row's
+    auto prefix = [&](const uint32_t (&n)[KPT], uint32_t (&before)[KPT]) -> uint32_t {
+        constexpr int N = KPT * NW;
+        static_assert(N <= 128, "two totals per lane");
 #pragma unroll
         for (int c = 0; c < KPT; c++) {
             int total;
-            before[c] = wave_scan(n[c], lane, total) - n[c];
-            if (lane == 0) tot[c * NW + wave] = (uint32_t)total;
+            before[c] = (uint32_t)wave_scan((int)n[c], lane, total) - n[c];
+            if (lane == 0) s_tot[c * NW + wave] = (uint32_t)total;
         }
-    };
-    auto prefix_row = [&](const uint32_t *tot, int (&before)[KPT]) -> int {
-        constexpr int N = KPT * NW;
-        static_assert(N <= 128, "two totals per lane");
-        const int t0 = 2 * lane < N ? (int)tot[2 * lane] : 0, t1 = 2 * lane + 1 < N ? (int)tot[2 * lane + 1] : 0;
+        __syncthreads();
+        const int t0 = 2 * lane < N ? (int)s_tot[2 * lane] : 0, t1 = 2 * lane + 1 < N ? (int)s_tot[2 * lane + 1] : 0;
         int total;
         const int e1 = wave_scan(t0 + t1, lane, total) - t1, e0 = e1 - t0;
 #pragma unroll
         for (int c = 0; c < KPT; c++) {
             const int i = c * NW + __builtin_amdgcn_readfirstlane(wave);
-            before[c] += __builtin_amdgcn_readlane((i & 1) ? e1 : e0, i >> 1);
+            before[c] += (uint32_t)__builtin_amdgcn_readlane((i & 1) ? e1 : e0, i >> 1);
         }
-        return total;
+        return (uint32_t)total;
+    };
+    // bits of the columns of a chunk whose key is above t (both halves the same)
+    auto above = [&](int c, uint32_t t) -> uint32_t {
+        uint32_t acc = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc |= above2(v[c][e], t) << (2 * e);
+        return column_bits(acc);
+    };
+    auto twice = [](uint32_t x) -> uint32_t { return x | (x << 16); };
+    // ... whose key is x
+    auto equal = [&](int c, uint32_t x) -> uint32_t {
+        uint32_t acc = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc |= not_zero2(v[c][e] ^ twice(x)) << (2 * e);
+        return column_bits(acc) ^ 0xffu;
     };
 
     // one bit per column of the chunk: kept whatever else there is; equal to the threshold, of which `need` are kept
@@ -162,87 +212,99 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
     if (p.type == 1) {  // relu: keep strictly positive values (NaN is not > 0)
         const uint32_t inf = p.dtype == 0 ? 0x7f80u : 0x7c00u;
 #pragma unroll
-        for (int c = 0; c < KPT; c++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const uint32_t x = bits_of(c, j), mag = x & 0x7fffu;
-                if (j < valid(c) && !(x & 0x8000u) && mag != 0 && mag <= inf) keep[c] |= 1u << j;
-            }
+        for (int c = 0; c < KPT; c++) keep[c] = above(c, twice(0x8000u)) & ~above(c, twice(0x8000u | inf));
     } else if (p.window > 0) {
         const uint32_t k = (uint32_t)(p.window < Lk ? p.window : Lk);
-        auto fold = [&](const uint32_t *hist, auto rep_c, uint32_t *sum) {
-            constexpr int REP = decltype(rep_c)::value;
-            for (int t = tid; t < 256; t += NT) {
-                uint32_t s = 0;
+        // sums of the copies of every bin: four copies a thread, a bin's threads side by side
+        auto fold = [&](const uint32_t *hist, auto log_c, uint32_t *sum) {
+            constexpr int PER = 1 << (decltype(log_c)::value - 2);  // threads of a bin: 1, 2 or 4
 #pragma unroll
-                for (int i = 0; i < REP; i++) s += hist[t * REP + ((t + i) & (REP - 1))];  // (the lanes on different banks)
-                sum[t] = s;
+            for (int t = tid; t < 256 * PER; t += NT) {
+                const u32x4_t q = ((const u32x4_t *)hist)[t];
+                int s = (int)(q[0] + q[1] + q[2] + q[3]);
+                if (PER >= 2) s += __builtin_amdgcn_update_dpp(0, s, 0xb1, 0xf, 0xf, false);  // quad_perm:[1,0,3,2]
+                if (PER >= 4) s += __builtin_amdgcn_update_dpp(0, s, 0x4e, 0xf, 0xf, false);  // quad_perm:[2,3,0,1]
+                if (t % PER == 0) sum[t / PER] = (uint32_t)s;
             }
             __syncthreads();
         };
         __syncthreads();
+        const uint32_t copy1 = (uint32_t)(lane & (REP1 - 1)) * 4, copy2 = (uint32_t)(lane & (REP2 - 1)) * 4;
+        auto count = [](uint32_t *hist, uint32_t at) { atomicAdd((uint32_t *)((char *)hist + at), 1u); };
 #pragma unroll
         for (int c = 0; c < KPT; c++)
+            if (first_col(c) < Lk) {
 #pragma unroll
-            for (int j = 0; j < 8; j++)
-                if (j < valid(c)) atomicAdd(&hist1[(order_key(bits_of(c, j)) >> 8) * REP1 + (lane & (REP1 - 1))], 1u);
-        __syncthreads();
-        fold(hist1, std::integral_constant<int, REP1>(), hsum[0]);
-        uint32_t bin1, above1, bin2, above2;
-        find_bin_wave(hsum[0], k, bin1, above1);
-#pragma unroll
-        for (int c = 0; c < KPT; c++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const uint32_t key = order_key(bits_of(c, j));
-                if (j < valid(c) && (key >> 8) == bin1) atomicAdd(&hist2[(key & 0xffu) * REP2 + (lane & (REP2 - 1))], 1u);
+                for (int e = 0; e < 4; e++) {  // (byte offset of a copy of a bin: high byte of the key x 4 REP1)
+                    count(hist1, ((v[c][e] >> (6 - LOG1)) & (0xffu << (LOG1 + 2))) | copy1);
+                    count(hist1, ((v[c][e] >> (22 - LOG1)) & (0xffu << (LOG1 + 2))) | copy1);
+                }
             }
         __syncthreads();
-        fold(hist2, std::integral_constant<int, REP2>(), hsum[1]);
-        find_bin_wave(hsum[1], k - above1, bin2, above2);
+        fold(hist1, std::integral_constant<int, LOG1>(), hsum[0]);
+        uint32_t bin1, above1, bin2, above_2;
+        find_bin_wave(hsum[0], k, bin1, above1);
+        const uint32_t high = twice(bin1 << 8);
+#pragma unroll
+        for (int c = 0; c < KPT; c++)
+            if (first_col(c) < Lk) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const uint32_t x = v[c][e] ^ high, lo = x & 0xffffu, hi = x >> 16;  // (below 256: in this bin, and where in it)
+                    if (lo < 256) count(hist2, (lo << (LOG2 + 2)) | copy2);
+                    if (hi < 256) count(hist2, (hi << (LOG2 + 2)) | copy2);
+                }
+            }
+        __syncthreads();
+        fold(hist2, std::integral_constant<int, LOG2>(), hsum[1]);
+        find_bin_wave(hsum[1], k - above1, bin2, above_2);
         const uint32_t T = (bin1 << 8) | bin2;
+        auto is_min_key = [&](uint32_t x) -> bool { return x == min_key || (min_zero && (x == 0x8000u || x == 0x7fffu)); };
         // entries equal to T still to take, >= 1 of hsum[1][bin2]: in column order (none where T is the fill value)
-        const uint32_t t_bits = (T & 0x8000u) ? T ^ 0x8000u : ~T & 0xffffu;
-        need = is_min(t_bits) ? 0u : k - above1 - above2;
+        need = is_min_key(T) ? 0u : k - above1 - above_2;
         some_ties = need != 0 && need < hsum[1][bin2];
 #pragma unroll
-        for (int c = 0; c < KPT; c++)
+        for (int c = 0; c < KPT; c++) keep[c] = above(c, twice(T));
+        if (need != 0) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const uint32_t x = bits_of(c, j), key = order_key(x);
-                if (j < valid(c) && key > T && !is_min(x)) keep[c] |= 1u << j;
-                if (j < valid(c) && key == T && need != 0) ties[c] |= 1u << j;
-            }
+            for (int c = 0; c < KPT; c++) ties[c] = equal(c, T);
+        }
+        if (T < (min_zero ? 0x8000u : min_key)) {  // (the fill value may lie above the threshold)
+#pragma unroll
+            for (int c = 0; c < KPT; c++) keep[c] &= ~(equal(c, min_key) | (min_zero ? equal(c, 0x8000u) | equal(c, 0x7fffu) : 0u));
+        }
     }
-    // ---- columns kept in front of each chunk, and the first `need` of the ties
-    int run[KPT], total = 0;
+#pragma unroll
+    for (int c = 0; c < KPT; c++) {
+        const uint32_t inside = (1u << valid(c)) - 1u;
+        keep[c] &= inside;
+        ties[c] &= inside;
+    }
+    // ---- columns kept in front of each chunk, and the first `need` of the ties (with ties, neither count reaches 65536)
+    uint32_t run[KPT], total = 0;
+    if (!some_ties) {
+#pragma unroll
+        for (int c = 0; c < KPT; c++) { keep[c] |= ties[c]; ties[c] = 0; }
+    }
     if (some_ties || p.kept_idx) {
-        int n[KPT], m[KPT], tied[KPT];
+        uint32_t n[KPT];
 #pragma unroll
-        for (int c = 0; c < KPT; c++) {
-            n[c] = __builtin_popcount(keep[c]);
-            m[c] = __builtin_popcount(ties[c]);
-        }
-        prefix_wave(s_tot[0], n, run);
-        prefix_wave(s_tot[1], m, tied);
-        __syncthreads();
-        total = prefix_row(s_tot[0], run);
-        const int all = prefix_row(s_tot[1], tied);
-        total += all < (int)need ? all : (int)need;
+        for (int c = 0; c < KPT; c++) n[c] = (uint32_t)__builtin_popcount(keep[c]) | ((uint32_t)__builtin_popcount(ties[c]) << 16);
+        total = prefix(n, run);
+        if (some_ties) {
+            total = (total & 0xffffu) + need;  // (there are more ties than that)
 #pragma unroll
-        for (int c = 0; c < KPT; c++) {
-            int left = (int)need - tied[c];
-            run[c] += left > 0 ? tied[c] : (int)need;
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-                if ((ties[c] >> j) & 1u) {
-                    if (left > 0) keep[c] |= 1u << j;
-                    left--;
+            for (int c = 0; c < KPT; c++) {
+                const int tied = (int)(run[c] >> 16);
+                int left = (int)need - tied;
+                run[c] = (run[c] & 0xffffu) + (uint32_t)(left > 0 ? tied : (int)need);
+                if (left >= __builtin_popcount(ties[c])) {
+                    keep[c] |= ties[c];
+                } else {  // (the last ones kept lie in one chunk)
+                    for (uint32_t u = ties[c]; left > 0; left--, u &= u - 1) keep[c] |= u & (0u - u);
                 }
+            }
         }
-    } else {
-#pragma unroll
-        for (int c = 0; c < KPT; c++) keep[c] |= ties[c];
     }
 
     // ---- the mask row, and its bits (key j of a row in bit j % 8 of byte j / 8)
@@ -262,23 +324,32 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
     // ---- the row as an ordered list of kept columns with inclusive prefix counts (fdma_scan.h), written up to
     // round_up(Lk, 16): the row has room
     if (p.kept_idx) {
+        // (a wave's columns of a chunk go through LDS, 512 at most, and leave 64 at a time: a store for each of a lane's eight touched
+        // every line of the list eight times)
         int32_t *irow = p.kept_idx + (size_t)row * p.kept_ld, *crow = p.kept_cnt + (size_t)row * p.kept_ld;
+        static_assert(256 * REP1 * 4 >= NW * 1024, "the lists of a chunk take the place of the first histogram");
+        uint16_t *list = (uint16_t *)hist1 + wave * 512;
 #pragma unroll
         for (int c = 0; c < KPT; c++) {
             const int col = first_col(c);
-            if (col < (Lk + 15) / 16 * 16) {
-                uint32_t cv[8];
-                int at = run[c];
+            const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)run[c], 0);
+            const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)run[c] + __builtin_popcount(keep[c]), 63) - first;
+            uint32_t at = run[c], cv[8];
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    if ((keep[c] >> j) & 1u) irow[at++] = col + j;
-                    cv[j] = (uint32_t)at;
-                }
+            for (int j = 0; j < 8; j++) {
+                const uint32_t one = (keep[c] >> j) & 1u;
+                if (one) list[at - first] = (uint16_t)(col + j);
+                cv[j] = at += one;
+            }
+            __builtin_amdgcn_wave_barrier();
+            for (uint32_t i = lane; i < n; i += 64) irow[first + i] = list[i];
+            __builtin_amdgcn_wave_barrier();
+            if (col < (Lk + 15) / 16 * 16) {
                 *(u32x4_t *)(crow + col) = u32x4_t{cv[0], cv[1], cv[2], cv[3]};
                 *(u32x4_t *)(crow + col + 4) = u32x4_t{cv[4], cv[5], cv[6], cv[7]};
             }
         }
-        if (tid == 0) p.kept_count[row] = total;
+        if (tid == 0) p.kept_count[row] = (int32_t)total;
     }
 }
 
