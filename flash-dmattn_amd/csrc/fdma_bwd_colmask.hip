@@ -749,14 +749,17 @@ template <int D, int BN> struct DqcSmem {
     static constexpr int OFF_BIAS = OFF_V + NST * K_BYTES;
     static constexpr int OFF_BITS = OFF_BIAS + 3 * 256;  // three bias columns (a direct load fills 256 bytes)
     static constexpr int TOTAL = OFF_BITS + DQ_MAX_KEYS / BN / 8;
+    static constexpr int GROUP = (TOTAL + 255) / 256 * 256;  // of a key group
     static_assert(TOTAL >= RED_LDS, "the workgroups that sum parts use it");
 };
 
 // BARE: no compaction, no mask, no bias (ragged batches, plain attention): there is no bias column, and the K / V tiles can
 // go the direct way as with compacted keys (a column made from mask bytes and bias values would have to come through
 // registers, whose wait is a wait for every direct load in front of it).
-template <typename T, int D, int BN, bool CAUSAL, bool CMP, bool BARE>
-__global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdParams p) {
+// KG: key groups of four waves.  Two take the tiles in turn, each with LDS and barriers' worth of stages of its own, and add their sums
+// up through LDS at the end: half the chain of tiles for grids that leave CUs empty (see dq_key_groups).
+template <typename T, int D, int BN, bool CAUSAL, bool CMP, bool BARE, int KG>
+__device__ __forceinline__ void dq_colmask(const BwdParams &p) {
     using E = Elem<T>;
     using SM = DqcSmem<D, BN>;
     using TL = LdsTile<D>;
@@ -781,12 +784,14 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
 
     // (LDS is read and written by absolute address in the tile loop: an access through a pointer into `smem` makes the
     // compiler wait for every direct load in flight first)
-    extern __shared__ __attribute__((aligned(256))) char smem[];
+    extern __shared__ __attribute__((aligned(256))) char smem_all[];
+    const int kgrp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NTHREADS);  // key group of this wave
+    char *const smem = smem_all + kgrp * SM::GROUP;
     const uint32_t lds0 = lds_addr(smem);  // (a multiple of 256)
     uint32_t *sBits = (uint32_t *)(smem + SM::OFF_BITS);
 
     const FwdParams &f = p.f;
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = tid & 63, r = lane & 31, g = lane >> 5;
+    const int tid = KG == 1 ? threadIdx.x : threadIdx.x % NTHREADS, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 31, g = lane >> 5;
     int lid = blockIdx.x;  // index among the dQ workgroups
     if (CMP) {
         // some workgroups sum partial results of the dK/dV kernel instead
@@ -848,7 +853,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
     }
 
     // ---- active-tile bitmap (tiles with at least one kept key)
-    for (int base = 0; !CMP && base < n_end; base += NTHREADS) {
+    for (int base = 0; !CMP && !BARE && base < n_end; base += NTHREADS) {
         const int j = base + tid;
         bool act = false;
         if (j < n_end) {
@@ -873,9 +878,9 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
             sBits[w0 + 1] = (uint32_t)(ball >> 32);
         }
     }
-    if (!CMP) __syncthreads();
+    if (!CMP && !BARE) __syncthreads();
     auto next_active = [&](int j) -> int {  // wave-uniform: keeps tile bases and loop conditions scalar
-        if (CMP) return j < n_end ? j : n_end;
+        if (CMP || BARE) return j < n_end ? j : n_end;
         while (j < n_end) {
             const uint32_t w = __builtin_amdgcn_readfirstlane(lds_ld32(lds0 + SM::OFF_BITS + 4 * (j >> 5))) >> (j & 31);
             if (w) {
@@ -1015,15 +1020,23 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
             __syncthreads();
         }
     };
-    int jc = next_active(0), jn = n_end, jnn = n_end;
+    // The tiles in turns of KG, one for each group.  jc, jn, jnn: the group's own of this turn and the two behind it; the leads: the first
+    // group's, which end the loop alike for all; tail: the newest turn's last
+    int lead = 0, lead_n = n_end, lead_nn = n_end, tail = -1;
+    auto next_turn = [&](int &first) -> int {
+        first = next_active(tail + 1);
+        tail = KG == 1 ? first : next_active(first + 1);
+        return KG == 2 && kgrp ? tail : first;
+    };
+    int jc = next_turn(lead), jn = n_end, jnn = n_end;
     // (what was requested above has landed by now; waited for here, the tiles' own loads are not waited for with it)
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qf[ks]), "+v"(dof[ks]));
+    jn = next_turn(lead_n);
+    if constexpr (DMA) jnn = next_turn(lead_nn);
     if (jc < n_end) {
-        jn = next_active(jc + 1);
         load_tile(jc, jc);
         if constexpr (DMA) {  // the second tile is on its way before the first is looked at
-            jnn = next_active(jn + 1);
             dma_stage = 1;
             load_tile(jn < n_end ? jn : jc, jc);
         }
@@ -1049,17 +1062,16 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
         dd = xhalf_sum(dd);
         if (!row_ok) dd = 0.f;
         // (fixed lengths: padded rows are zero)
-        if (g == 0 && (row_ok || (!f.cu_q && qrow < p.Lq_rounded))) p.softmax_d[b * p.sd_b + h * p.sd_h + sq.q0 + qrow] = dd;
+        if (g == 0 && kgrp == 0 && (row_ok || (!f.cu_q && qrow < p.Lq_rounded))) p.softmax_d[b * p.sd_b + h * p.sd_h + sq.q0 + qrow] = dd;
     }
-    if (jc < n_end) {
-        store_tile(0, 0);
+    if (lead < n_end) {
+        if (KG == 1 || jc < n_end) store_tile(0, 0);
         publish();
     }
     int i = 0;
     constexpr bool S_EARLY = DMA && MB == 1;
     f32x16_t s[MB];
-    while (jc < n_end) {
-        if constexpr (!DMA) jn = next_active(jc + 1);
+    auto one_tile = [&]() {
         const int n0 = jc * BN;
         const int st = DMA ? i % 3 : (i & 1);
         const uint32_t st_off = (uint32_t)(st * SM::K_BYTES);  // (a multiple of 256: the swizzles stay XORs)
@@ -1201,24 +1213,55 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
             }
         }
         if (!DMA && jn < n_end) store_tile((i + 1) & 1, (i + 1) % 3);
+    };
+    while (lead < n_end) {
+        // (a group without a tile in the last turn only takes part in its barrier)
+        if (KG == 1 || jc < n_end) one_tile();
         publish();
         i++;
         jc = jn;
+        lead = lead_n;
         if constexpr (DMA) {
             jn = jnn;
-            jnn = next_active(jn + 1);
+            lead_n = lead_nn;
+            jnn = next_turn(lead_nn);
+        } else {
+            jn = next_turn(lead_n);
         }
     }
 
     // (direct loads still in flight -- tiles fetched past the last one -- must not land in LDS that belongs to the next
     // workgroup by then)
     if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0x0070);
+    if constexpr (KG == 2) {  // each group hands the other's half of the head dim over and finishes its own
+        __syncthreads();  // (every wave's reads of the last tiles, and its direct loads)
+        static_assert(2 * 4 * (DB / 2) * 4096 <= 2 * SM::GROUP, "the halves lie where the tiles were");
+        f32x4_t *theirs = (f32x4_t *)smem_all + ((1 - kgrp) * 4 + wave) * (DB / 2) * 4 * 64 + lane, *mine = (f32x4_t *)smem_all + (kgrp * 4 + wave) * (DB / 2) * 4 * 64 + lane;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+            if (db / (DB / 2) != kgrp) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) theirs[(db % (DB / 2) * 4 + q) * 64] = f32x4_t{dq[db][4 * q], dq[db][4 * q + 1], dq[db][4 * q + 2], dq[db][4 * q + 3]};
+            }
+        __syncthreads();
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+            if (db / (DB / 2) == kgrp) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const f32x4_t t = mine[(db % (DB / 2) * 4 + q) * 64];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) dq[db][4 * q + e] += t[e];
+                }
+            }
+    }
     if (qrow < LqS) {
         uint16_t *dqp = (uint16_t *)p.dq + b * p.dq_b + (sq.q0 + qrow) * p.dq_r + h * p.dq_h;
 #pragma unroll
         for (int db = 0; db < DB; db++)
 #pragma unroll
             for (int blk = 0; blk < 2; blk++) {
+                if (KG == 2 && db / (DB / 2) != kgrp) continue;
                 const int c = 32 * db + 16 * blk + 8 * g;
                 if (c < f.d) {
                     u32x4_t w;
@@ -1229,6 +1272,27 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdPa
                 }
             }
     }
+}
+
+template <typename T, int D, int BN, bool CAUSAL, bool CMP, bool BARE>
+__global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdParams p) {
+    dq_colmask<T, D, BN, CAUSAL, CMP, BARE, 1>(p);
+}
+template <typename T, int D, int BN, bool CAUSAL, bool BARE>
+__global__ void __launch_bounds__(2 * NTHREADS, 2) bwd_dq_groups_kernel(const BwdParams p) {
+    dq_colmask<T, D, BN, CAUSAL, false, BARE, 2>(p);
+}
+
+// Two key groups to a workgroup of dQ where there is no mask and no bias, the rows are long and there are no more workgroups than CUs
+// hold at once: a SIMD works a tile off in 0.65 us with two waves, in 0.75 with one, and the hand-over at the end is 2 us.  dQ with one group / two,
+// us: ragged 3520 and others (4443 tokens) x 2/1 heads, d = 128 73 / 63; 3392 (7028) x 2/1, d = 96 77 / 61; 4717 (5549) x 8/2, d = 64 90.5 / 71;
+// 3904 (3914) x 16/4, d = 64, 528 blocks, 87 / 74; short rows 334 (632) x 8/2 14.5 / 16.4; more blocks (1984 of 2708 x 32/8, 896)
+// 69 / 90.  Not with a mask, where one group's fixed part weighs as much as its few tiles (768 tokens x 16/8 32.2 / 31.6, 576 x 16/8 x 2
+// 25.4 / 26.5), nor with compacted keys, of which the host does not know how many there are (1733 x 16/4, 130 kept 16.1 / 21.1).
+bool dq_key_groups(const FwdParams &f) {
+    if (f.d > 128 || f.cmp.on || f.mask || f.bias || f.Lk < 1024) return false;
+    const int64_t blocks = f.cu_q ? (int64_t)f.H * (f.total_q / Q_BM + f.B) : (int64_t)f.B * f.H * ((f.Lq + Q_BM - 1) / Q_BM);
+    return blocks <= 9 * (int64_t)device_cus() / 4;
 }
 
 template <typename T, int D, bool CAUSAL>
@@ -1242,11 +1306,13 @@ hipError_t launch_dq_grid(const BwdParams &p, int grid, hipStream_t stream) {
         const int which = f.cmp.on ? 1 : (SWZ && !f.mask && !f.bias ? 2 : 0);
         auto kern = which == 1 ? bwd_dq_colmask_kernel<T, D, BN, CAUSAL, true, false>
                                : (which == 2 ? bwd_dq_colmask_kernel<T, D, BN, CAUSAL, false, SWZ> : bwd_dq_colmask_kernel<T, D, BN, CAUSAL, false, false>);
-        const int smem = DqcSmem<D, BN>::TOTAL;
-        static DynSmemLimit smem_limit[3];  // one per instantiation: the limit is a property of the kernel
-        hipError_t e = smem_limit[which].ensure((const void *)kern, (int)smem);
+        const bool two = dq_key_groups(f);
+        if (two) kern = bwd_dq_groups_kernel<T, D, BN, CAUSAL, SWZ>;
+        const int smem = two ? 2 * DqcSmem<D, BN>::GROUP : DqcSmem<D, BN>::TOTAL;
+        static DynSmemLimit smem_limit[4];  // one per instantiation: the limit is a property of the kernel
+        hipError_t e = smem_limit[two ? 3 : which].ensure((const void *)kern, (int)smem);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(NTHREADS), smem, stream, p);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(two ? 2 * NTHREADS : NTHREADS), smem, stream, p);
         return hipGetLastError();
     }
 }

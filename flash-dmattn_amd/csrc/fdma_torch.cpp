@@ -385,7 +385,7 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             }
     }
     Tensor shares;  // (of the call alone: the node does not keep it)
-    if (!need)
+    if (!need && ((mask.defined() && mask.size(2) > 1) || (bias.defined() && bias.size(2) > 1)))
         if (size_t room = api.fwd_optional_bytes(&a)) {
             shares = scratch_with_room(0, room, opt);
             if (room) { a.workspace = shares.data_ptr(); a.workspace_bytes = room; }
