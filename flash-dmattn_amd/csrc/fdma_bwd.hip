@@ -11,12 +11,12 @@
 //     dQ = scale * dS K ; dK = scale * dS^T Q ; dV = P^T dO ; dBias = dS (summed over broadcast dims)
 //
 // Different structure: no fp32 dQ accumulator, no atomics on dQ/dK/dV, no expanded GQA buffers.
-//   1. bwd_dot_kernel   : D = rowsum(dO * O)
+//   1. bwd_dq_kernel    : (fdma_bwd_dq.hip) one workgroup per (query block, batch, head); loops over key blocks like
+//                         the forward kernel (transposed scores, a lane owns one query row); makes D on the way;
 //   2. bwd_dkdv_kernel  : one workgroup per (key block, batch, KV head); K/V stationary, loops over the
 //                         query heads of the group and over query blocks; dK, dV and dBias complete in
-//                         registers (S is computed un-transposed so a lane owns one key column);
-//   3. bwd_dq_kernel    : (fdma_bwd_dq.hip) one workgroup per (query block, batch, head); loops over key blocks like
-//                         the forward kernel (transposed scores, a lane owns one query row).
+//                         registers (S is computed un-transposed so a lane owns one key column).
+// (Where dBias is dS itself, bwd_dot_kernel makes D, and dQ comes last, from that dS: fdma_bwd_dq_ds.hip.)
 // Work is therefore 7 tile GEMMs instead of 5, in exchange for a deterministic result and no
 // read-modify-write traffic.
 #include "fdma_common.h"
@@ -599,9 +599,10 @@ template <typename T, int D>
 hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
     const FwdParams &f = p.f;
     hipError_t e;
-    // 1. D = rowsum(dO * O)  (the compacted backward has done it in its pre-pass launch; the column-mask form without
-    // compaction makes it in its dQ kernel, which then comes first)
-    const bool colmask = bwd_colmask_applicable(p), dq_first = colmask && !f.cmp.on;
+    // 1. D = rowsum(dO * O)  (the compacted backward has done it in its pre-pass launch; the others make it in their dQ kernel, which
+    // then comes first, unless dQ is made from the dS that step 2 writes)
+    const bool colmask = bwd_colmask_applicable(p), from_ds = !colmask && f.Lk > 0 && bwd_dq_from_ds_applicable(p);
+    const bool dq_first = colmask ? !f.cmp.on : !from_ds;
     if (!p.dot_done && !dq_first) {
         const int rpb = bwd_dot_rows_per_block(f.d);
         dim3 grid(((f.cu_q ? f.total_q : p.Lq_rounded) + rpb - 1) / rpb, f.H, f.cu_q ? 1 : f.B);
@@ -616,7 +617,7 @@ hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
     }
     // 2. dK, dV, dBias
     const int dtype_code = std::is_same<T, bf16_tag>::value ? 0 : 1;
-    if (dq_first && (e = launch_bwd_dq_colmask(p, dtype_code, stream)) != hipSuccess) return e;
+    if (dq_first && (e = colmask ? launch_bwd_dq_colmask(p, dtype_code, stream) : launch_bwd_dq(p, dtype_code, stream)) != hipSuccess) return e;
     if (f.Lk > 0 && colmask) {
         if ((e = launch_bwd_dkdv_colmask(p, dtype_code, stream)) != hipSuccess) return e;
     } else if (f.Lk > 0) {
@@ -656,11 +657,9 @@ hipError_t launch_bwd_t(const BwdParams &p, hipStream_t stream) {
     // 3. dQ (the launch of a compacted backward also sums the dK / dV / dBias partial results of step 2)
     if (colmask) {
         if (!dq_first && (e = launch_bwd_dq_colmask(p, dtype_code, stream)) != hipSuccess) return e;
-    } else if (f.Lk > 0 && bwd_dq_from_ds_applicable(p)) {
+    } else if (from_ds) {
         // (step 2 has written dS itself as dBias: dQ = scale * dS K without a second pass over mask and bias)
         if ((e = launch_bwd_dq_from_ds(p, dtype_code, stream)) != hipSuccess) return e;
-    } else {
-        if ((e = launch_bwd_dq(p, dtype_code, stream)) != hipSuccess) return e;
     }
     // 4. shared dBias elements: fp32 sums to the output type
     if (p.dbias_accum) {

@@ -1,6 +1,6 @@
 // Backward dynamic-mask attention for gfx950, general form (mask and / or bias vary per query row): the dQ kernel.
 //
-// Third kernel of the backward pass (see fdma_bwd.hip): one workgroup per (128-query block, batch, head) loops over
+// First kernel of the backward pass (see fdma_bwd.hip), which also leaves D = rowsum(dO * O) for the next: one workgroup per (128-query block, batch, head) loops over
 // the key tiles like the forward kernel and computes, per 64-key tile,
 //     S^T = K Q^T (+ bias, mask),  P^T = exp2(S^T - LSE),  dP^T = V dO^T,  dS^T = P^T o (dP^T - D),  dQ^T += K^T dS^T
 // -- the dQ part of compute_dq_dk_dv_1colblock (csrc/flash_sparse_attn/src/flash_bwd_kernel.h:79-1142 of the
@@ -32,7 +32,8 @@ template <int D, int BM, int BN> struct DqSmem {
     static constexpr int F_BYTES = BM * SF * 2;
     static constexpr int STAGE = (2 * K_BYTES + F_BYTES + 255) / 256 * 256;
     static constexpr int OFF_VOTE = 2 * STAGE;  // three words: "a tile has a kept element"
-    static constexpr int TOTAL = OFF_VOTE + 16;
+    static constexpr int OFF_D = OFF_VOTE + 16;  // KSPLIT: D of the workgroup's 128 rows
+    static constexpr int TOTAL = OFF_D + 512;
 };
 
 template <typename T> struct NegInf2;
@@ -97,9 +98,29 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         }
     }
     float lse2 = INFINITY, dd = 0.f;
-    if (qrow < f.Lq) {
-        lse2 = f.lse[((int64_t)b * f.H + h) * f.Lq + qrow] * kLog2e;
-        dd = p.softmax_d[((int64_t)b * f.H + h) * p.Lq_rounded + qrow];
+    if (qrow < f.Lq) lse2 = f.lse[((int64_t)b * f.H + h) * f.Lq + qrow] * kLog2e;
+    // D = rowsum(dO * O) is made here, from the dO fragments, and left for the dK/dV kernel, which is launched behind this one: a launch less
+    // (forward + backward, us: 1212 tokens x 8/4 heads, d = 64 124.5 / 121.8, 4 x 511 x 16/8, d = 256 242.1 / 236.8, 576 x 16/4, d = 128 89.9 / 86.1).  Of two waves with the same rows the first makes it, and the other finds it in LDS.
+    if (KSPLIT == 1 || kh == 0) {
+        const uint16_t *op = (const uint16_t *)f.o + b * f.o_b + (int64_t)qrow_c * f.o_r + h * f.o_h;
+        u32x4_t of[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) of[ks] = *(const u32x4_t *)(op + (ks * 16 + g * 8 < f.d ? ks * 16 + g * 8 : 0));
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const bool on = qrow < f.Lq && ks * 16 + g * 8 < f.d;
+            u32x4_t v = kept8(of[ks], on);  // (what is clamped need not be a number; dO is zero there)
+#pragma unroll
+            for (int e = 0; e < 4; e++) dd += E::lo(v[e]) * E::lo(dof[ks][e]) + E::hi(v[e]) * E::hi(dof[ks][e]);
+        }
+        dd = xhalf_sum(dd);
+        float *d_out = p.softmax_d + b * p.sd_b + h * p.sd_h;
+        if (g == 0 && (!SHARES || blockIdx.y == 0)) {
+            if (qrow < p.Lq_rounded) d_out[qrow] = dd;  // (padded rows are zero)
+            if (m0 + BM >= f.Lq && rw == 0)
+                for (int row = m0 + BM + r; row < p.Lq_rounded; row += 32) d_out[row] = 0.f;
+        }
+        if (KSPLIT == 2 && g == 0) lds_st32(lds0 + SM::OFF_D + (xw * 32 + r) * 4, __float_as_uint(dd));
     }
 
     int n_end = (f.Lk + BN - 1) / BN;
@@ -344,6 +365,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) bwd_dq_
         load_mask(t_first, mreg);
         if (t_first + 1 < n_end) load_mask(t_first + 1, mnext);
         bool act_cur = __syncthreads_or(finish_mask(t_first, mreg));
+        if (KSPLIT == 2 && kh == 1) dd = __uint_as_float(lds_ld32(lds0 + SM::OFF_D + (xw * 32 + r) * 4));
         if (act_cur) {
             load_rest(t_first);
             store_stage(t_first, mreg);
