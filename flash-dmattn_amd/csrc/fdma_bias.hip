@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(256) dyn_bias_fwd_kernel(const DynBiasParams p
 
 // Backward, first stage.  Latency: a workgroup's tokens are one trip to memory when their loads are issued together, ahead of
 // d_dt (eight trips of four tokens each before), and the two halves of a workgroup take half of a pass's tokens each: 4 x 2048
-// tokens of 8 x 64 took 18 us, now 14.  Workgroup `c` owns token rows [c * rows_per_wg, ...).  HM = Hkv rounded up to 8, 16 or 32:
+// tokens of 8 x 64 took 18 us, now 12.  Workgroup `c` owns token rows [c * rows_per_wg, ...).  HM = Hkv rounded up to 8, 16 or 32:
 // thread t works on output head t % HM for the per-head sums, so each sum is built in a fixed order; in the main part
 // a thread owns CPT adjacent columns of V_flat (4; 2 when 32 heads' worth of accumulators must fit the registers or
 // when V_flat has too few columns to give every thread four).
@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(512) dyn_bias_bwd_kernel(const DynBiasParams p
     constexpr int TB = 16;                   // tokens whose loads are in flight together (registers)
     constexpr int NT = 512, HC = 16 / CPT < HM ? 16 / CPT : HM;  // HC: heads whose sums the halves exchange at a time
     __shared__ float s_ddt[RB * HM];
-    __shared__ float s_red[2 * NT];
+    __shared__ float s_red[2][NT / 64][HM];
     __shared__ float s_x[HC * CPT * 256];
     const int tid = threadIdx.x, half = __builtin_amdgcn_readfirstlane(tid >> 8), ctid = tid & 255;  // (columns are owned by a thread of each half)
     const int Hk = p.Hk, K = Hk * p.d;
@@ -204,7 +204,7 @@ __global__ void __launch_bounds__(512) dyn_bias_bwd_kernel(const DynBiasParams p
     float *part_w = p.part + (int64_t)blockIdx.x * p.part_stride;
     const int n_groups = (K + 256 * CPT - 1) / (256 * CPT);  // column groups: the same trip count for every thread
 
-    for (int grp = 0; grp < n_groups; grp++) {
+    for (int grp = blockIdx.y; grp < n_groups; grp += gridDim.y) {
         const int k0 = grp * 256 * CPT + ctid * CPT;
         const bool has_cols = k0 < K;
         const int head = has_cols ? k0 / p.d : 0, dd = has_cols ? k0 - head * p.d : 0;
@@ -337,16 +337,34 @@ __global__ void __launch_bounds__(512) dyn_bias_bwd_kernel(const DynBiasParams p
             }
         }
     }
-    // per-head sums: the NT / HM threads of a head, folded in thread order
-    __syncthreads();
-    s_red[tid] = sum_a;
-    s_red[NT + tid] = sum_pb;
+    // per-head sums: a head's threads in a wave, by lane swaps, then the waves in order.  (All of a head's NT / HM through LDS by one
+    // thread were a chain of 64 reads.)
+    if (blockIdx.y) return;
+    auto fold = [&](float x) -> float {
+        const uint32_t u = __float_as_uint(x);
+        const auto r32 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        x = __uint_as_float((uint32_t)r32[0]) + __uint_as_float((uint32_t)r32[1]);
+        if (HM <= 16) {
+            const uint32_t w = __float_as_uint(x);
+            const auto r16 = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+            x = __uint_as_float((uint32_t)r16[0]) + __uint_as_float((uint32_t)r16[1]);
+        }
+        if (HM <= 8) x += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), 0x128, 0xf, 0xf, false));  // row_ror:8
+        return x;
+    };
+    sum_a = fold(sum_a);
+    sum_pb = fold(sum_pb);
+    if ((tid & 63) < HM) {
+        s_red[0][tid >> 6][tid & 63] = sum_a;
+        s_red[1][tid >> 6][tid & 63] = sum_pb;
+    }
     __syncthreads();
     if (tid < Hk) {
         float sa = 0.f, sb = 0.f;
-        for (int t = tid; t < NT; t += HM) {
-            sa += s_red[t];
-            sb += s_red[NT + t];
+#pragma unroll
+        for (int w = 0; w < NT / 64; w++) {
+            sa += s_red[0][w][tid];
+            sb += s_red[1][w][tid];
         }
         part_w[(int64_t)Hk * K + tid] = sa;
         part_w[(int64_t)Hk * K + Hk + tid] = sb;
@@ -423,8 +441,13 @@ int dyn_bias_bwd_workgroups(int64_t n_rows, int Hk, int d, int *rows_per_wg) {
 hipError_t launch_dyn_bias_bwd(const DynBiasParams &p, int dtype, hipStream_t stream) {
     const int64_t n_rows = (int64_t)p.B * p.L;
     if (n_rows <= 0) return hipSuccess;
-    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(p.n_wg), dim3(512), 0, stream, p); };
     const bool wide = four_columns(p.Hk, p.d);
+    const int groups = (p.Hk * p.d + (wide ? 1023 : 511)) / (wide ? 1024 : 512);  // column groups of the kernel
+    // (side by side where all of them run at once: a workgroup's time is its groups one behind the other.  us, before / now, the lane swaps of
+    // the per-head sums among them: 500 tokens of 16 x 256 52.9 / 17.8, 122 of 16 x 96 28.2 / 15.6, 2396 of 8 x 96 18.4 / 10.4, 2048 of 16 x 128
+    // 32.8 / 20.2; the sums alone: 4 x 2048 of 8 x 64 15.0 / 12.3, 83 of 4 x 128 11.5 / 8.5)
+    const dim3 grid(p.n_wg, p.n_wg * groups <= device_cus() ? groups : 1);
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(512), 0, stream, p); };
     if (dtype == 0) {
         if (p.Hk <= 8) wide ? go(dyn_bias_bwd_kernel<bf16_tag, 8, 4>) : go(dyn_bias_bwd_kernel<bf16_tag, 8, 2>);
         else if (p.Hk <= 16) wide ? go(dyn_bias_bwd_kernel<bf16_tag, 16, 4>) : go(dyn_bias_bwd_kernel<bf16_tag, 16, 2>);
@@ -437,9 +460,9 @@ hipError_t launch_dyn_bias_bwd(const DynBiasParams &p, int dtype, hipStream_t st
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int64_t per = (int64_t)p.Hk * p.Hk * p.d + 2 * p.Hk;
-    const dim3 grid((unsigned)((per + 63) / 64));
-    if (dtype == 0) hipLaunchKernelGGL(dyn_bias_reduce_kernel<bf16_tag>, grid, dim3(64 * RED_WAVES), 0, stream, p);
-    else hipLaunchKernelGGL(dyn_bias_reduce_kernel<fp16_tag>, grid, dim3(64 * RED_WAVES), 0, stream, p);
+    const dim3 fold((unsigned)((per + 63) / 64));
+    if (dtype == 0) hipLaunchKernelGGL(dyn_bias_reduce_kernel<bf16_tag>, fold, dim3(64 * RED_WAVES), 0, stream, p);
+    else hipLaunchKernelGGL(dyn_bias_reduce_kernel<fp16_tag>, fold, dim3(64 * RED_WAVES), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -73,3 +73,29 @@ def test_gradients_of_long_runs(B, L, Hk, d):
     ref = (a64 * F.softplus(v64.reshape(B, L, -1) @ w64.t())).transpose(-1, -2).unsqueeze(-2)
     for x, y in zip(got, torch.autograd.grad(ref, wide, dbias.double())):
         assert rel_err(x, y) <= 2.0 ** -7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L,Hk,d,dtype", [
+    (1, 33, 8, 96, torch.bfloat16),     # two groups of 512 columns, the second short; a run of one token
+    (2, 45, 16, 72, torch.float16),     # two of 1024, a run across the batch entries
+    (1, 70, 20, 256, torch.bfloat16),   # ten of 512
+    (1, 64, 32, 40, torch.bfloat16),    # every head of a wave's lanes
+    (1, 4100, 16, 128, torch.float16),  # too many runs for the groups side by side
+    (3, 1, 1, 16, torch.bfloat16),
+])
+def test_gradients_of_column_groups(B, L, Hk, d, dtype):
+    """The backward's groups of columns run side by side where there are few runs of tokens; the per-head sums are taken once.  Two calls
+    give the same bits; sums over the tokens in fp32, results rounded to 16 bits once."""
+    print("groups", B, L, Hk, d, dtype, flush=True)
+    g = torch.Generator().manual_seed(L + Hk)
+    v = torch.randn(B, L, Hk, d, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(Hk, Hk * d, generator=g) / (Hk * d) ** 0.5).to(dtype).to(DEV)
+    a = torch.linspace(0.5, 1.5, Hk).to(dtype).to(DEV)
+    dbias = torch.randn(B, Hk, 1, L, generator=g).to(dtype).to(DEV)
+    leaves = [t.requires_grad_(True) for t in (v, w, a)]
+    got, again = [torch.autograd.grad(dynamic_mask_bias(*leaves), leaves, dbias) for _ in range(2)]
+    v64, w64, a64 = wide = [t.detach().double().requires_grad_(True) for t in leaves]
+    ref = (a64 * F.softplus(v64.reshape(B, L, -1) @ w64.t())).transpose(-1, -2).unsqueeze(-2)
+    for x, y, z in zip(got, torch.autograd.grad(ref, wide, dbias.double()), again):
+        assert rel_err(x, y) <= 2.0 ** -7 and torch.equal(x, z)
