@@ -275,11 +275,41 @@ int fdma_set_stream_min_items(int n) {
     return before;
 }
 
+static bool general_fwd(const fdma_fwd_args *a, const fdma::FwdParams &p) {
+    return p.Lk > 0 && p.Hk > 0 && !fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k) && !fdma::fwd_colmask_applicable(p);
+}
+
+// (Above head dim 128 the general form's shares are added up by a launch: a row block's weigh up to a megabyte, which one workgroup takes
+// 10 us for.  2316 tokens x 2/1 heads, d = 256, forward and backward 195 us with a launch, 203 without.)
 size_t fdma_fwd_counter_bytes(const fdma_fwd_args *a) {
-    if (!a || a->seqlen_k <= 0 || a->num_heads_k <= 0 || !fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k)) return 0;
+    if (!a || a->seqlen_k <= 0 || a->num_heads_k <= 0 || a->seqlen_q <= 0) return 0;
+    if (!fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k)) {
+        fdma::FwdParams p, pv;
+        fill_fwd_params(a, p);
+        if (general_fwd(a, p)) return p.d <= 128 && fdma::general_key_shares(p, false) > 1 ? (size_t)round_up(fdma::general_share_units(p) * 4, 256) : 0;
+        if (fdma::compact_per_query_head(p, pv)) p = pv;
+        return fdma::fwd_key_splits(p) > 1 ? (size_t)round_up(fdma::fwd_share_units(p) * 4, 256) : 0;
+    }
     return (size_t)round_up(fdma::decode_num_counters(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->head_dim) * 4, 256);
 }
 
+// room for the shares of a call with split keys: O, then LSE
+// (for either form: row by row, or as the lanes hold it, with the rows and elements that a row block rounds up to)
+static size_t share_rows(const fdma::FwdParams &p, bool general) {
+    if (general) return (size_t)fdma::general_share_units(p) * 128;
+    return (size_t)fdma::fwd_share_units(p) * fdma::fwd_share_block(p);
+}
+static size_t share_bytes(const fdma::FwdParams &p, bool general, int shares) {
+    const size_t dpad = p.d <= 64 ? 64 : (p.d <= 128 ? 128 : 256);
+    return shares > 1 ? (size_t)shares * share_rows(p, general) * (dpad + 1) * sizeof(float) : 0;
+}
+static void take_shares(fdma::FwdParams &p, bool general, int shares, void *at, int32_t *counters) {
+    const size_t dpad = p.d <= 64 ? 64 : (p.d <= 128 ? 128 : 256);
+    p.splits = shares;
+    p.dec_counter = counters;
+    p.o_part = static_cast<float *>(at);
+    p.lse_part = p.o_part + shares * share_rows(p, general) * dpad;
+}
 // scratch of a forward call: what it cannot do without, and -- `shares` -- room for the shares of split keys behind it
 static size_t fwd_scratch_bytes(const fdma_fwd_args *a, size_t *shares) {
     *shares = 0;
@@ -290,7 +320,7 @@ static size_t fwd_scratch_bytes(const fdma_fwd_args *a, size_t *shares) {
         if (fdma::compact_per_query_head(p, pv)) p = pv;
         else if (!fdma::use_compact(p)) return 0;
         const int splits = fdma::fwd_key_splits(p);
-        if (splits > 1) *shares = (size_t)splits * a->batch * a->num_heads * a->seqlen_q * (size_t)(a->head_dim + 1) * sizeof(float);
+        *shares = share_bytes(p, false, splits);
         return (size_t)round_up(fdma::compact_bytes(p, false), 256);
     }
     const int splits = fdma::decode_num_splits(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->head_dim, a->mask != nullptr);
@@ -305,19 +335,11 @@ size_t fdma_fwd_workspace_bytes(const fdma_fwd_args *a) {
     return need + shares;
 }
 
-// room for the shares of a general-form call with split keys: O, then LSE
-static size_t general_share_bytes(const fdma::FwdParams &p, int shares) {
-    return shares > 1 ? (size_t)shares * p.B * p.H * p.Lq * (size_t)(p.d + 1) * sizeof(float) : 0;
-}
-static bool general_fwd(const fdma_fwd_args *a, const fdma::FwdParams &p) {
-    return p.Lk > 0 && p.Hk > 0 && !fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k) && !fdma::fwd_colmask_applicable(p);
-}
-
 size_t fdma_fwd_optional_bytes(const fdma_fwd_args *a) {
-    if (!a) return 0;
+    if (!a || a->num_heads_k <= 0) return 0;
     fdma::FwdParams p;
     fill_fwd_params(a, p);
-    return general_fwd(a, p) ? general_share_bytes(p, fdma::general_key_shares(p, false)) : 0;
+    return general_fwd(a, p) ? share_bytes(p, true, fdma::general_key_shares(p, false)) : 0;
 }
 
 int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
@@ -350,6 +372,8 @@ int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
         e = fdma::launch_fwd_decode(p, a->dtype, stream);
     } else {
         // seqlen_k == 0 falls out of the kernel as O = 0, LSE = +inf (flash_api.cpp:535-539)
+        const size_t cneed = a->counters ? fdma_fwd_counter_bytes(a) : 0;
+        int32_t *counters = cneed && a->counters_bytes >= cneed && !(reinterpret_cast<uintptr_t>(a->counters) & 3) ? a->counters : nullptr;
         // (a query-broadcast mask with a row per query head: compacted per query head -- forward only; the backward of
         // that form skips tiles instead)
         fdma::FwdParams pv;
@@ -364,19 +388,11 @@ int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
             const size_t base = fwd_scratch_bytes(a, &shares);
             if ((e = fdma::compact_setup(p, a->workspace, a->dtype, stream)) != hipSuccess)
                 return fail(FDMA_ERR_LAUNCH, "forward launch failed: %s", hipGetErrorString(e));
-            if (splits > 1 && a->workspace_bytes >= base + shares) {
-                p.splits = splits;
-                p.o_part = reinterpret_cast<float *>(static_cast<char *>(a->workspace) + base);
-                p.lse_part = p.o_part + (size_t)splits * a->batch * a->num_heads * a->seqlen_q * a->head_dim;
-            }
+            if (splits > 1 && a->workspace_bytes >= base + shares) take_shares(p, false, splits, static_cast<char *>(a->workspace) + base, counters);
         }
         if (general_fwd(a, p)) {
             const int shares = fdma::general_key_shares(p, false);
-            if (shares > 1 && a->workspace && aligned16(a->workspace) && a->workspace_bytes >= general_share_bytes(p, shares)) {
-                p.splits = shares;
-                p.o_part = static_cast<float *>(a->workspace);
-                p.lse_part = p.o_part + (size_t)shares * p.B * p.H * p.Lq * p.d;
-            }
+            if (shares > 1 && a->workspace && aligned16(a->workspace) && a->workspace_bytes >= share_bytes(p, true, shares)) take_shares(p, true, shares, a->workspace, counters);
         }
         e = fdma::launch_fwd(p, a->dtype, stream);
     }

@@ -27,6 +27,7 @@
 
 #include "fdma_common.h"
 #include "fdma_params.h"
+#include "fdma_fwd_merge.h"
 
 namespace fdma {
 
@@ -500,7 +501,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
                     xo[(db * 4 + q) * 64] = f32x4_t{o[db][4 * q], o[db][4 * q + 1], o[db][4 * q + 2], o[db][4 * q + 3]};
         }
         __syncthreads();
-        if (kh == 1) return;
+        if (!SHARES && kh == 1) return;
         const float m1 = xm[0], t1 = xm[(RB * GH) * 64];
         const float mx = fmaxf(row_max, m1), safe = mx == -INFINITY ? 0.f : mx;
         const float w0 = fast_exp2(row_max - safe), w1 = fast_exp2(m1 - safe);
@@ -516,19 +517,51 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
             }
     }
     const float inv = total > 0.f ? 1.f / total : 0.f;
-    if constexpr (SHARES) {  // O in fp32 and its log2-sum-exp, which fwd_merge_kernel adds up
-        if (qrow < p.Lq) {
-            const int64_t at = (((int64_t)blockIdx.y * p.B + b) * p.H + h) * p.Lq + qrow;
+    if constexpr (SHARES) {  // O in fp32 and its log2-sum-exp, which the last workgroup of the rows, or fwd_merge_kernel, adds up
+        // (a sum that is no number has to reach the result: only an empty share is left out)
+        const float l = total == 0.f ? -INFINITY : row_max + __builtin_amdgcn_logf(total);
+        if (!p.dec_counter) {
+            if (qrow < p.Lq && kh == 0) {
+                const int64_t at = (((int64_t)blockIdx.y * p.B + b) * p.H + h) * p.Lq + qrow;
+#pragma unroll
+                for (int db = 0; db < DB; db++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int c = 32 * db + 16 * (q >> 1) + 8 * g + 4 * (q & 1);
+                        if (c < p.d) *(f32x4_t *)(p.o_part + at * p.d + c) = f32x4_t{o[db][4 * q] * inv, o[db][4 * q + 1] * inv, o[db][4 * q + 2] * inv, o[db][4 * q + 3] * inv};
+                    }
+                if (g == 0) p.lse_part[at] = l;
+            }
+            return;
+        }
+        // (counters: [workgroup][share][wave of the lower half][32-wide block of O][quarter][lane] and [workgroup][share][row])
+        constexpr int ROWS = 32 * RB * GH;
+        const int64_t first = (int64_t)blockIdx.x * p.splits;
+        float *o_lane = p.o_part + first * (ROWS * D) + xw * (32 * D) + lane * 2, *l_lane = p.lse_part + first * ROWS + xw * 32 + r;
+        if (kh == 0) {
+            float *at = o_lane + (int64_t)blockIdx.y * (ROWS * D);
 #pragma unroll
             for (int db = 0; db < DB; db++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const int c = 32 * db + 16 * (q >> 1) + 8 * g + 4 * (q & 1);
-                    if (c < p.d) *(f32x4_t *)(p.o_part + at * p.d + c) = f32x4_t{o[db][4 * q] * inv, o[db][4 * q + 1] * inv, o[db][4 * q + 2] * inv, o[db][4 * q + 3] * inv};
-                }
-            // (a sum that is no number has to reach the result: only an empty share is left out)
-            if (g == 0) p.lse_part[at] = total == 0.f ? -INFINITY : row_max + __builtin_amdgcn_logf(total);
+                for (int q = 0; q < 4; q++)
+                    share_store4(at + (db * 4 + q) * 256, f32x4_t{o[db][4 * q] * inv, o[db][4 * q + 1] * inv, o[db][4 * q + 2] * inv, o[db][4 * q + 3] * inv});
+            if (g == 0) share_store(l_lane + (int64_t)blockIdx.y * ROWS, l);
         }
+        if (!last_share(p.dec_counter + blockIdx.x, p.splits, (int *)(smem + SM::OFF_VOTE)) || kh || qrow >= p.Lq) return;
+        bool on[MAX_KEY_SPLITS];
+        const ShareWeights sw = lane_share_weights(l_lane, ROWS, p.splits, on);
+        uint16_t *op = (uint16_t *)p.o + b * p.o_b + (int64_t)qrow * p.o_r + h * p.o_h;
+#pragma unroll 1
+        for (int i = 0; i < 2 * DB; i += 4) {
+            u32x4_t y[4];
+            lane_merged<T, 4>(sw, o_lane + i * 512, ROWS * D, p.splits, on, y);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int c = 16 * (i + u) + 8 * g;
+                if (c < p.d) *(u32x4_t *)(op + c) = y[u];
+            }
+        }
+        if (g == 0) p.lse[((int64_t)b * p.H + h) * p.Lq + qrow] = sw.lse;
         return;
     }
     if (qrow < p.Lq) {
@@ -608,6 +641,11 @@ int shared_rows(const FwdParams &p) {
     return p.d > 64 && G % 2 == 0 ? 2 : 1;
 }
 
+int64_t general_share_units(const FwdParams &p) {
+    const int gh = shared_rows(p), rows = 128 / gh;
+    return (int64_t)((p.Lq + rows - 1) / rows) * (p.H / gh) * p.B;
+}
+
 // Shares that the key tiles of a row block are cut into, forward and dQ.  A workgroup's time is its chain of tiles (1.5 us each at head dims up
 // to 128, 2.5 per 32 keys above), and few heads or short rows leave most CUs without one.
 //   * As many as the chip holds workgroups at once (one per CU; d <= 64: two, three of 32-row ones), rounded DOWN: 64 blocks of 1000 rows,
@@ -618,14 +656,16 @@ int shared_rows(const FwdParams &p) {
 //     x 16/8 125 / 130 with the backward, 256 x 2/1 24.5 / 21.4).
 //   * dQ from 24 tiles on (16 of 32 keys): below, a backward is bound by its launches, of which this is one more (1024 x 2/1,
 //     d = 128: 66.9 and 69 to 72).
+// (Up to head dim 128 the last workgroup of the rows adds the forward's shares up; a launch of its own: 3883 x 8/2, d = 64 66.7 / 55.9, 2 x 1198 x
+// 8/4, d = 64 30.6 / 26.9, 2 x 1039 x 8/2 24.5 / 21.0.)
 // Whole / shares, us (forward; backward with its other kernels): 2316 x 2/1 heads, d = 256 162 / 46, 323 / 180; 3000 x 2/1, d = 64 83 / 25,
 // 141 / 75; 2240 x 2/1, d = 96 56 / 24, 107 / 72; 4096 x 2/1, d = 128 98 / 39, 172 / 106; 3000 x 8/2, d = 64 81 / 41, 198 / 171; 1999 x 8/4,
 // not causal 61 / 43, 138 / 119.
 int general_key_shares(const FwdParams &p, bool dq) {
     if (p.cu_q || p.Lq < 1 || p.Lk < 1) return 1;
-    const int gh = shared_rows(p), rows = 128 / gh, tile = p.d > 128 ? 32 : 64, tiles = (p.Lk + tile - 1) / tile;
+    const int gh = shared_rows(p), tile = p.d > 128 ? 32 : 64, tiles = (p.Lk + tile - 1) / tile;
     if (dq && tiles < (p.d > 128 ? 16 : 24)) return 1;
-    const int64_t blocks = (int64_t)((p.Lq + rows - 1) / rows) * (p.H / gh) * p.B;
+    const int64_t blocks = general_share_units(p);
     int64_t s = blocks > 0 ? device_cus() * (p.d > 64 ? 1 : (gh == 4 ? 3 : 2)) / blocks : 1;
     if (s > tiles / 4) s = tiles / 4;
     if (p.d > 64 && tiles < 12 && (p.d <= 128 || 4 * blocks > device_cus())) return 1;
@@ -638,7 +678,7 @@ hipError_t launch_fwd(const FwdParams &p, int dtype, hipStream_t stream) {
     // head dims up to 64 / 128 / 256 (a head dim in between runs in the next larger instantiation)
     const hipError_t e = dtype == 0 ? (p.d <= 64 ? launch_fwd_t<bf16_tag, 64>(p, stream) : p.d <= 128 ? launch_fwd_t<bf16_tag, 128>(p, stream) : launch_fwd_t<bf16_tag, 256>(p, stream))
                                     : (p.d <= 64 ? launch_fwd_t<fp16_tag, 64>(p, stream) : p.d <= 128 ? launch_fwd_t<fp16_tag, 128>(p, stream) : launch_fwd_t<fp16_tag, 256>(p, stream));
-    return e != hipSuccess || p.splits <= 1 ? e : launch_fwd_merge(p, dtype, stream);
+    return e != hipSuccess || p.splits <= 1 || p.dec_counter ? e : launch_fwd_merge(p, dtype, stream);
 }
 
 }  // namespace fdma

@@ -47,6 +47,7 @@
 
 #include "fdma_common.h"
 #include "fdma_params.h"
+#include "fdma_fwd_merge.h"
 
 namespace fdma {
 
@@ -768,12 +769,8 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
 }
 #undef FWD_LDS
 
-// Adds up the shares of a call with split keys: out = sum_s 2^(l_s - l) O_s, l = log2 sum_s 2^l_s (no share with a visible key:
-// 0 and +inf).  A thread has 8 elements of one row; the rows of O of a share without a visible key hold nothing and are not read.
-// Only such a share, l_s = -inf, is left out: an l_s that is no number (a NaN among its keys or in the query) has a weight that is
-// none either, which makes the row what the call with whole keys makes it.
+// Adds up the shares of a call with split keys and no arrival counters.  A thread has 8 elements of one row.
 template <typename T> __global__ void __launch_bounds__(256) fwd_merge_kernel(const FwdParams p) {
-    using E = Elem<T>;
     const int CH = p.d / 8;
     const int64_t rows = (int64_t)p.B * p.H * p.Lq, at = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (at >= rows * CH) return;
@@ -784,35 +781,20 @@ template <typename T> __global__ void __launch_bounds__(256) fwd_merge_kernel(co
 #pragma unroll
     for (int s = 0; s < MAX_KEY_SPLITS; s++) l[s] = s < p.splits ? p.lse_part[s * rows + row] : -INFINITY;
 #pragma unroll
-    for (int s = 0; s < MAX_KEY_SPLITS; s++) {
+    for (int s = 0; s < MAX_KEY_SPLITS; s++) {  // (the rows of O of a share without a visible key hold nothing and are not read)
         v[s][0] = v[s][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         if (l[s] != -INFINITY) {
             v[s][0] = *(const f32x4_t *)(p.o_part + (s * rows + row) * p.d + c);
             v[s][1] = *(const f32x4_t *)(p.o_part + (s * rows + row) * p.d + c + 4);
         }
     }
-    float top = l[0];
-#pragma unroll
-    for (int s = 1; s < MAX_KEY_SPLITS; s++) top = fmaxf(top, l[s]);
-    float sum = 0.f;
+    const ShareWeights r = share_weights(l);
     f32x4_t a[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int s = 0; s < MAX_KEY_SPLITS; s++) {
-        const float w = l[s] != -INFINITY ? fast_exp2(l[s] - top) : 0.f;
-        sum += w;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            a[0][e] = fmaf(w, v[s][0][e], a[0][e]);
-            a[1][e] = fmaf(w, v[s][1][e], a[1][e]);
-        }
-    }
-    const float inv = sum > 0.f ? 1.f / sum : 0.f;
+    for (int s = 0; s < MAX_KEY_SPLITS; s++) add_share(a, r.w[s], v[s]);
     const int q = (int)(row % p.Lq), h = (int)(row / p.Lq % p.H), b = (int)(row / p.Lq / p.H);
-    u32x4_t w;
-#pragma unroll
-    for (int e = 0; e < 4; e++) w[e] = E::pack2(a[e >> 1][2 * (e & 1)] * inv, a[e >> 1][2 * (e & 1) + 1] * inv);
-    *(u32x4_t *)((uint16_t *)p.o + b * p.o_b + q * p.o_r + h * p.o_h + c) = w;
-    if (c == 0) p.lse[b * p.lse_b + h * p.lse_h + q] = sum > 0.f ? (top + __builtin_amdgcn_logf(sum)) * kLn2 : INFINITY;
+    *(u32x4_t *)((uint16_t *)p.o + b * p.o_b + q * p.o_r + h * p.o_h + c) = merged8<T>(r.inv, a);
+    if (c == 0) p.lse[b * p.lse_b + h * p.lse_h + q] = r.lse;
 }
 
 template <typename T> hipError_t launch_merge(const FwdParams &p, hipStream_t stream) {
@@ -871,8 +853,11 @@ hipError_t launch_fwd_merge(const FwdParams &p, int dtype, hipStream_t stream) {
 // keys kept:
 //   3072 keys   13.1 / 16.3    19.1 / 22.7    41.2 / 28.4        16384 keys   21.5 / 20.9    49.7 / 26.2    157.2 / 45.7
 //   6144 keys   15.2 / 18.6    26.0 / 21.0    70.0 / 33.7        32768 keys   31.6 / 23.1    87.3 / 34.2    297.6 / 70.2
-// How much is kept is not known here: with under 1024 kept keys there is a single share and the merge costs its 3 to 4 us for
-// nothing; the other way round a share too few costs more.
+// How much is kept is not known here: with under 1024 kept keys there is a single share, whose workgroup writes the result itself
+// (arrival counters; without, a merge of 3 to 4 us for nothing: 214 rows x 16/8 heads, 216 kept of 5056 16.2 / 12.8, 27 x 2/1, 644 of
+// 3456, d = 64 16.6 / 13.8, in shares 223 x 16/4, 2496 of 23360 28.3 / 26.8); the other way round a share too few costs more.
+// Causal calls whose last row block takes twice the average gain nothing from shares: d = 256, whole / in two, 3001 x 8/4 heads, 1024
+// kept 44.7 / 53.1, 8192 x 2/1, 2048 kept 51.7 / 55.1, all 3001 kept 92 / 80; d = 128, 2048 x 8/4, all kept 32.8 / 37.9.
 int key_shares(const FwdParams &p) {
     if (p.cu_q || p.d > 128 || p.Lq < 2 || p.Lk / 2 < p.Lq) return 1;
     const int64_t blocks = (int64_t)p.B * p.H * ((p.Lq + 127) / 128);
@@ -906,13 +891,19 @@ static bool takes_key_groups(const FwdParams &p) {
     return 2 * blocks64 <= 5 * (int64_t)device_cus();
 }
 
+int64_t fwd_share_units(const FwdParams &p) {
+    FwdParams pr = p;
+    return row_grid(pr, fwd_share_block(p));
+}
+int fwd_share_block(const FwdParams &p) { return p.d > 128 && fwd_blocks64(p) > device_cus() ? 128 : 64; }
+
 hipError_t launch_fwd_colmask(const FwdParams &p, int dtype, hipStream_t stream) {
     if (p.cmp.on && p.cmp.img_kv) return launch_fwd_stream(p, dtype, stream);  // (the pre-pass has written tile images)
     // head dims up to 64 / 128 (a head dim in between runs in the next larger instantiation), above in a kernel of their own
     if (p.d > 128) return launch_fwd_wide(p, dtype, stream);
     if (takes_key_groups(p)) {  // (and all calls in shares: three shares are at most a third of a 64-row block per CU, see key_shares)
         const hipError_t e = launch_fwd_wide(p, dtype, stream);
-        if (e != hipSuccess || !p.cmp.on || p.splits <= 1) return e;
+        if (e != hipSuccess || !p.cmp.on || p.splits <= 1 || p.dec_counter) return e;
         return launch_fwd_merge(p, dtype, stream);
     }
     if (dtype == 0) return p.d <= 64 ? launch_d<bf16_tag, 64>(p, stream) : launch_d<bf16_tag, 128>(p, stream);

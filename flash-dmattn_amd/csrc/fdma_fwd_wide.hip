@@ -32,6 +32,7 @@
 
 #include "fdma_common.h"
 #include "fdma_params.h"
+#include "fdma_fwd_merge.h"
 
 namespace fdma {
 
@@ -57,7 +58,7 @@ template <int D_, int RG> struct Cfg {
     static constexpr int PASSES = KG * (KG - 1) * RG * UPW * 2048 > 128 * 1024 ? 2 : 1, UPP = UPW / PASSES;  // ... in so many passes
     static constexpr int OFF_SUMS = KG * (KG - 1) * RG * UPP * 2048;  // the others' shares of a pass's units, then row sums and references
     static constexpr int MERGE_BYTES = OFF_SUMS + 2 * 8 * 64 * 4;
-    static constexpr int SMEM = LOOP_BYTES > MERGE_BYTES ? LOOP_BYTES : MERGE_BYTES;
+    static constexpr int SMEM = LOOP_BYTES > MERGE_BYTES + 16 ? LOOP_BYTES : MERGE_BYTES + 16;  // (a word behind the merge: last_share)
     static_assert(SMEM <= 160 * 1024, "one workgroup per CU");
     static_assert(UPW * KG * 16 == D, "every unit of O is finished by one key group");
     static_assert(8 * RPP % 16 == 0, "a wave's pieces lie rows of one swizzle apart");
@@ -78,6 +79,7 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     const int rw = wave % RG, kg = wave / RG;  // 32-row group and key group of this wave
 
     const RowUnit ru = row_unit(p, blockIdx.x, BM);
+    const int part = SHARES ? (int)blockIdx.y : 0;  // (all first shares first: workgroups that turn out to have none come when CUs are free)
     if (ru.block < 0) return;
     const int b = ru.b, hk = ru.hk, h = ru.h;
     const int m0 = ru.block * BM;
@@ -131,17 +133,18 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
         if (ne < n_end) n_end = ne;
     }
     // this workgroup's share of the tiles (see fwd_key_splits)
-    int t_first = 0;
+    int t_first = 0, shares = 1;
     if (SHARES && p.splits > 1) {
-        // (no share under 512 keys: the shares that are then left over only say so)
-        const int y = (int)blockIdx.y, most = n_end * BN / 512 > 1 ? n_end * BN / 512 : 1, shares = p.splits < most ? p.splits : most;
-        if (y >= shares) {
+        // (no share under 512 keys: the workgroups that are then left over end, and without counters say so)
+        const int most = n_end * BN / 512 > 1 ? n_end * BN / 512 : 1;
+        shares = p.splits < most ? p.splits : most;
+        if (part >= shares) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (Q is not to land in what is another workgroup's LDS by then)
-            if (tid < BM && m0 + tid < LqS) p.lse_part[(((int64_t)y * p.B + b) * p.H + h) * p.Lq + m0 + tid] = -INFINITY;
+            if (!p.dec_counter && tid < BM && m0 + tid < LqS) p.lse_part[(((int64_t)part * p.B + b) * p.H + h) * p.Lq + m0 + tid] = -INFINITY;
             return;
         }
-        t_first = n_end * y / shares;
-        n_end = n_end * (y + 1) / shares;
+        t_first = n_end * part / shares;
+        n_end = n_end * (part + 1) / shares;
     }
 
     // ---- active-tile bitmap (compacted keys: every tile is active)
@@ -431,8 +434,16 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     }
     const bool row_ok = qrow < LqS;
     const float inv = total > 0.f ? 1.f / total : 0.f;
-    const bool share = SHARES && p.splits > 1;  // this share's O in fp32 and its log2-sum-exp; fwd_merge_kernel adds the shares up
-    const int64_t prow_at = (((int64_t)blockIdx.y * p.B + b) * p.H + h) * p.Lq + qrow;
+    // this share's O in fp32 and its log2-sum-exp, which the last workgroup of the row block, or fwd_merge_kernel, adds up
+    const bool share = SHARES && (p.dec_counter ? shares > 1 : p.splits > 1);
+    const int64_t prow_at = (((int64_t)part * p.B + b) * p.H + h) * p.Lq + qrow;
+    // (counters: [unit][share][wave][16-wide unit of O][half][lane] and [unit][share][row])
+    float *o_lane = nullptr, *l_lane = nullptr;
+    if (SHARES && p.dec_counter) {
+        const int64_t first = (int64_t)blockIdx.x * p.splits;
+        o_lane = p.o_part + first * (BM * D) + wave * (UPW * 512) + lane * 2;
+        l_lane = p.lse_part + first * BM + rw * 32 + r;
+    }
     uint16_t *op = (uint16_t *)p.o + b * p.o_b + (sq.q0 + qrow) * p.o_r + h * p.o_h;
 #pragma unroll
     for (int pass = 0; pass < C::PASSES; pass++) {
@@ -462,7 +473,11 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
 #pragma unroll
                         for (int e = 0; e < 4; e++) y[q][e] *= inv;
                     }
-                    if (row_ok && c < p.d) {
+                    if (share && p.dec_counter) {
+                        float *at = o_lane + part * (BM * D) + (pass * UPP + j) * 512;
+                        share_store4(at, y[0]);
+                        share_store4(at + 256, y[1]);
+                    } else if (row_ok && c < p.d) {
                         if (share) {
                             *(f32x4_t *)(p.o_part + prow_at * p.d + c) = y[0];
                             *(f32x4_t *)(p.o_part + prow_at * p.d + c + 4) = y[1];
@@ -475,8 +490,22 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     }
     if (g == 0 && kg == 0 && row_ok) {
         // (a sum that is no number has to reach the result: only an empty share is left out)
-        if (share) p.lse_part[prow_at] = total == 0.f ? -INFINITY : top + __builtin_amdgcn_logf(total);
+        if (share) share_store(p.dec_counter ? l_lane + part * BM : p.lse_part + prow_at, total == 0.f ? -INFINITY : top + __builtin_amdgcn_logf(total));
         else p.lse[b * p.lse_b + h * p.lse_h + sq.q0 + qrow] = total > 0.f ? (top + __builtin_amdgcn_logf(total)) * kLn2 : INFINITY;
+    }
+    if constexpr (SHARES) {
+        if (share && p.dec_counter && last_share(p.dec_counter + blockIdx.x, shares, (int *)(smem + C::MERGE_BYTES)) && row_ok) {
+            bool on[MAX_KEY_SPLITS];
+            const ShareWeights sw = lane_share_weights(l_lane, BM, shares, on);
+            u32x4_t y[UPW];
+            lane_merged<T, UPW>(sw, o_lane, BM * D, shares, on, y);
+#pragma unroll
+            for (int j = 0; j < UPW; j++) {
+                const int c = 16 * (kg * UPW + j) + 8 * g;
+                if (c < p.d) *(u32x4_t *)(op + c) = y[j];
+            }
+            if (g == 0 && kg == 0) p.lse[b * p.lse_b + h * p.lse_h + sq.q0 + qrow] = sw.lse;
+        }
     }
 }
 

@@ -428,10 +428,15 @@ int64_t fwd_blocks64(const FwdParams &p);  // 64-row blocks of all heads (ragged
 int fwd_key_splits(const FwdParams &p);
 constexpr int MAX_KEY_SPLITS = 8;
 // adds the shares of a forward call up
+// (without arrival counters; with them, FwdParams::dec_counter, the last workgroup of a row block does it)
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, hipStream_t stream);
 // general form (mask or bias per query): shares that the key tiles of a row block are cut into (1: none), forward or dQ; what
 // they leave lies in o_part / lse_part or BwdParams::dq_part
 int general_key_shares(const FwdParams &p, bool dq);
+int64_t general_share_units(const FwdParams &p);  // row blocks of a forward in shares, a counter each
+// compacted forward in shares (fwd_key_splits): row blocks, a counter each
+int64_t fwd_share_units(const FwdParams &p);
+int fwd_share_block(const FwdParams &p);  // rows of a row block
 int key_shares(const FwdParams &p);  // ... as far as the sizes go: what they would be if the keys were compacted
 // compacted forward on tile images (fdma_fwd_stream.hip): resident workgroups that walk their share of the
 // (query block, head) items with the tiles of the next item already on their way.  `fwd_stream_applicable` decides from

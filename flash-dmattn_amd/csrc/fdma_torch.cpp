@@ -377,18 +377,18 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (need) {
         a.workspace = (char *)buf.data_ptr() + lse_bytes;
         a.workspace_bytes = need;
-        if (Lq == 1)
-            if (const size_t cbytes = api.fwd_counter_bytes(&a)) {
-                Tensor &c = counters_for(dev, stream, cbytes, bytes);
-                a.counters = (int32_t *)c.data_ptr();
-                a.counters_bytes = c.nbytes();
-            }
     }
     Tensor shares;  // (of the call alone: the node does not keep it)
     if (!need && ((mask.defined() && mask.size(2) > 1) || (bias.defined() && bias.size(2) > 1)))
         if (size_t room = api.fwd_optional_bytes(&a)) {
             shares = scratch_with_room(0, room, opt);
             if (room) { a.workspace = shares.data_ptr(); a.workspace_bytes = room; }
+        }
+    if (a.workspace)
+        if (const size_t cbytes = api.fwd_counter_bytes(&a)) {
+            Tensor &c = counters_for(dev, stream, cbytes, bytes);
+            a.counters = (int32_t *)c.data_ptr();
+            a.counters_bytes = c.nbytes();
         }
     check(api.fwd(&a, stream));
     if (is_grad) {

@@ -264,13 +264,15 @@ def _flash_sparse_attn_forward_body(
                     args.counters, args.counters_bytes = counters.data_ptr(), counters.numel() * 4
         else:
             nbytes = _cabi.lib.fdma_fwd_workspace_bytes(args)
-            if nbytes:
-                workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-                args.workspace, args.workspace_bytes = workspace.data_ptr(), nbytes
-            else:
-                shares = _scratch_with_room(0, _cabi.lib.fdma_fwd_optional_bytes(args), q.device)
-                if shares is not None:
-                    args.workspace, args.workspace_bytes = shares.data_ptr(), shares.numel()
+            # (a workspace that a backward will want is kept until then; the room for shares is of this call alone)
+            scratch = _scratch_with_room(nbytes, 0 if nbytes else _cabi.lib.fdma_fwd_optional_bytes(args), q.device)
+            workspace = scratch if nbytes else None
+            if scratch is not None:
+                args.workspace, args.workspace_bytes = scratch.data_ptr(), scratch.numel()
+                cbytes = _cabi.lib.fdma_fwd_counter_bytes(args)
+                if cbytes:
+                    counters = _decode_buffers(q.device, stream, 0, cbytes)[1]
+                    args.counters, args.counters_bytes = counters.data_ptr(), counters.numel() * 4
         _cabi.check(_cabi.lib.fdma_fwd(args, stream))
     items = getattr(_tls, "items", None)
     per_query_head = mask is not None and mask.shape[1] == num_heads and num_heads != k.shape[2]

@@ -144,7 +144,8 @@ typedef struct fdma_fwd_args {
      * reference always runs its combine as a second kernel, flash_fwd_launch_template.h:91-143) and puts its counter
      * back to zero, so the same buffer serves the next call as it is -- clear it once, when it is allocated.  Calls
      * that may overlap on the device (different streams) need a buffer each.  NULL = the merge is a second launch.
-     * Results are the same bit for bit either way.  Other paths ignore the field. */
+     * Results are the same bit for bit either way.  Forward calls with keys in shares (few query rows; see workspace_bytes and
+     * fdma_fwd_optional_bytes) use them alike, a counter per block of query rows; other paths ignore the field. */
     int32_t *counters;
     size_t counters_bytes; /* >= fdma_fwd_counter_bytes(args) */
 } fdma_fwd_args;

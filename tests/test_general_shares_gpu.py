@@ -27,6 +27,7 @@ CASES = [
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_shares_vs_oracle_and_whole(case, dtype, monkeypatch):
     from flash_sparse_attn import _cabi, flash_sparse_attn_func
+    from flash_sparse_attn import flash_sparse_attn_interface as interface
 
     print(case, dtype, flush=True)
     B, Lq, Lk, H, Hk, d, hm, hb, causal = case
@@ -54,6 +55,11 @@ def test_shares_vs_oracle_and_whole(case, dtype, monkeypatch):
         monkeypatch.setattr(_cabi.lib, name, lambda a, fn=fn, seen=seen: seen.append(fn(a)) or seen[-1])
     shares = run()
     assert asked["fdma_fwd_optional_bytes"][0] > 0
+    assert not any(int(c.abs().max()) for _, c in interface._decode_scratch.values())  # (arrival counters are left zero)
+    with monkeypatch.context() as m:
+        m.setattr(_cabi.lib, "fdma_fwd_counter_bytes", lambda a: 0)
+        apart = run()  # (added up by a launch of its own)
+    assert torch.equal(apart[0], shares[0]) and torch.equal(apart[1], shares[1])
     for name in asked:
         monkeypatch.setattr(_cabi.lib, name, lambda a: 0)
     whole = run()
@@ -71,3 +77,35 @@ def test_shares_vs_oracle_and_whole(case, dtype, monkeypatch):
         else:  # (a probability is rounded to eps / 2 of itself against either reference point; sums of many of them, and what LSE and O carry on)
             ok = (a.float() - b.float()).abs() <= eps * (2 * b.float().abs() + b.float().abs().max())
         assert ok.all(), i
+
+
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,d,kept", [
+    (1, 70, 5003, 4, 2, 128, 3000),   # four shares; a row block of six rows
+    (2, 16, 8200, 2, 1, 64, 8200),    # eight
+    (1, 130, 4100, 3, 3, 72, 900),    # offered four, one taken: the result is written whole
+    (1, 64, 6000, 2, 1, 96, 1100),    # two of five
+])
+def test_few_rows_against_many_keys(B, Lq, Lk, H, Hk, d, kept, monkeypatch):
+    """The column form's shares: added up by the last workgroup of a row block or by a launch, the same bits."""
+    from oracle import eager
+    from _util import make_inputs
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func
+    from flash_sparse_attn import flash_sparse_attn_interface as interface
+
+    print("few rows", B, Lq, Lk, H, Hk, d, kept, flush=True)
+    q, k, v, mask, bias = [t.to(DEV) for t in make_inputs(B, Lq, Lk, H, Hk, d, (B, Hk, 1, Lk), (B, Hk, 1, Lk), kept, seed=Lk)]
+    ref, ref_lse = eager.attention_forward(q, k, v, mask, bias, None, True)
+    call = lambda: flash_sparse_attn_func(q, k, v, mask, bias, None, True, return_attn_probs=True)[:2]
+    with torch.no_grad():
+        native = flash_sparse_attn_func(q, k, v, mask, bias, None, True)
+        monkeypatch.setattr(_cabi, "host", _cabi._NoHost)
+        asked = []
+        fn = _cabi.lib.fdma_fwd_counter_bytes
+        monkeypatch.setattr(_cabi.lib, "fdma_fwd_counter_bytes", lambda a: asked.append(fn(a)) or asked[-1])
+        out, lse = call()
+        assert asked[0] > 0 and not any(int(c.abs().max()) for _, c in interface._decode_scratch.values())
+        monkeypatch.setattr(_cabi.lib, "fdma_fwd_counter_bytes", lambda a: 0)
+        apart, lse_apart = call()
+    assert torch.equal(out, native) and torch.equal(out, apart) and torch.equal(lse, lse_apart)
+    assert_out_close(out, ref)
+    assert torch.allclose(lse, ref_lse.reshape(lse.shape), atol=2e-3, rtol=1e-3)
