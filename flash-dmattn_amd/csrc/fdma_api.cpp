@@ -803,7 +803,7 @@ static void fill_dyn_bias(const fdma_dyn_bias_args *a, fdma::DynBiasParams &p) {
     p.dbias = a->dbias; p.dbias_b = a->dbias_strides[0]; p.dbias_h = a->dbias_strides[1];
     p.dv = a->dvalue; p.dv_b = a->dvalue_strides[0]; p.dv_r = a->dvalue_strides[1]; p.dv_h = a->dvalue_strides[2];
     p.dw = a->dweight; p.da = a->da; p.dpb = a->dproj_bias;
-    p.n_wg = fdma::dyn_bias_bwd_workgroups((int64_t)a->batch * a->seqlen_k, a->num_heads_k, a->head_dim, &p.rows_per_wg);
+    p.n_wg = fdma::dyn_bias_bwd_workgroups((int64_t)a->batch * a->seqlen_k, a->num_heads_k, a->head_dim, &p.rows_per_wg, &p.col_waves);
     p.part_stride = round_up((int64_t)a->num_heads_k * a->num_heads_k * a->head_dim + 2 * a->num_heads_k, 4);
 }
 

@@ -13,9 +13,8 @@
 // for 32 lines per instruction.  8 x 4093 tokens of 8 x 128, 67 MB, bf16: 23 us that way, 16.7 with one piece of 256 columns that is
 // waited for whole, 14.4 now; 4 x 2304 of 16 x 256, 288 workgroups of eight pieces in a row: 24.7 -> 20.0; 4 x 2048 of 8 x 64
 // 8.0 -> 5.6.)
-// Backward: a workgroup owns a run of tokens; d_dt = dBias * A * sigmoid(dt) goes to LDS, then a thread owns four
-// columns of V_flat and walks the tokens: dV = d_dt W and the workgroup's share of dW = d_dt^T V_flat, dA and dpb, which
-// go to fp32 partials that a second kernel folds in a fixed order (bit-reproducible).
+// Backward: a workgroup owns a run of tokens: d_dt = dBias * A * sigmoid(dt), dV = d_dt W and the run's share of dW = d_dt^T V_flat, dA and
+// dpb, which go to fp32 partials that a second kernel folds in a fixed order (bit-reproducible).
 #include <type_traits>
 
 #include "fdma_common.h"
@@ -177,197 +176,215 @@ __global__ void __launch_bounds__(256) dyn_bias_fwd_kernel(const DynBiasParams p
     }
 }
 
-// Backward, first stage.  Latency: a workgroup's tokens are one trip to memory when their loads are issued together, ahead of
-// d_dt (eight trips of four tokens each before), and the two halves of a workgroup take half of a pass's tokens each: 4 x 2048
-// tokens of 8 x 64 took 18 us, now 12.  Workgroup `c` owns token rows [c * rows_per_wg, ...).  HM = Hkv rounded up to 8, 16 or 32:
-// thread t works on output head t % HM for the per-head sums, so each sum is built in a fixed order; in the main part
-// a thread owns CPT adjacent columns of V_flat (4; 2 when 32 heads' worth of accumulators must fit the registers or
-// when V_flat has too few columns to give every thread four).
-template <typename T, int HM, int CPT>
-__global__ void __launch_bounds__(512) dyn_bias_bwd_kernel(const DynBiasParams p) {
-    using E = Elem<T>;
-    constexpr int RB = 64;                   // tokens per pass through LDS
-    constexpr int TB = 16;                   // tokens whose loads are in flight together (registers)
-    constexpr int NT = 512, HC = 16 / CPT < HM ? 16 / CPT : HM;  // HC: heads whose sums the halves exchange at a time
-    __shared__ float s_ddt[RB * HM];
-    __shared__ float s_red[2][NT / 64][HM];
-    __shared__ float s_x[HC * CPT * 256];
-    const int tid = threadIdx.x, half = __builtin_amdgcn_readfirstlane(tid >> 8), ctid = tid & 255;  // (columns are owned by a thread of each half)
-    const int Hk = p.Hk, K = Hk * p.d;
-    const int64_t wg_row0 = (int64_t)blockIdx.x * p.rows_per_wg;
-    const int64_t n_rows = (int64_t)p.B * p.L;
-    const int64_t wg_row1 = wg_row0 + p.rows_per_wg < n_rows ? wg_row0 + p.rows_per_wg : n_rows;
-    const int j_mine = tid % HM, rgroup = tid / HM;
-    constexpr int RSTEP = NT / HM;
-    const float a_mine = j_mine < Hk ? E::lo((uint32_t)((const uint16_t *)p.a)[j_mine]) : 0.f;
-    float sum_a = 0.f, sum_pb = 0.f;  // this thread's share of dA[j_mine], dpb[j_mine]
-    float *part_w = p.part + (int64_t)blockIdx.x * p.part_stride;
-    const int n_groups = (K + 256 * CPT - 1) / (256 * CPT);  // column groups: the same trip count for every thread
+// Backward, first stage: two contractions, dV = d_dt W over the heads and dW = d_dt^T V_flat over the tokens, on MFMA 16x16x4 in fp32
+// (operands and sums stay 32 bits; twice the rate of the vector unit, which the products were bound by, and its registers spilled).
+// A wave owns 128 columns of V_flat and 16 tokens at a time, workgroup (x, y) the tokens [x * rows_per_wg, ...) and col_waves such
+// column ranges; what is left of its eight waves takes tiles of tokens in turn, and their dW meet in LDS at the end, in order.
+//   * dW: lane (c, g) holds columns 8 c .. 8 c + 7 of tokens 4 q + g -- 16-byte loads, a row of 256 bytes per 16 lanes -- and step e takes
+//     the e-th of them.  The sum of head j lies in lanes j, 16 + j, ..: 32 columns each.
+//   * dV: the step's rows are columns 32 m + 8 (rho / 4) + 2 (rho % 4) + h of W, so a lane ends with eight columns of its token.
+//   * d_dt of (token, head) is made in the lane that dV wants it in; dW wants it transposed: through a KB of LDS of the wave's own.
+// HM = Hkv rounded up to 8, 16 or 32.  Bound by memory where there are many tokens (4 x 17701 of 16 x 64, 290 MB: 56 of the 92 at the rate of a
+// copy), else by a chain of one trip to memory, three barriers and the fold.  us, kernel and fold, products on the vector unit by columns of
+// one thread / now: 4 x 2048 of 8 x 64 14.6 / 11.3, 122 of 16 x 96 17.8 / 11.8, 2 x 8566 of 2 x 128 20.9 / 13.8, 4000 of 16 x 256 65.3 / 29.6,
+// 33000 of 8 x 128 45.2 / 37.5, of 1 x 64 25.4 / 13.0, 4 x 17701 of 16 x 64 117 / 92, 131072 of 8 x 128 156 / 127.
+constexpr int BWD_COLS = 128, BWD_TOK = 16, BWD_WAVES = 8;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef u32x4_t u32x4_a8_t __attribute__((aligned(8)));
 
-    for (int grp = blockIdx.y; grp < n_groups; grp += gridDim.y) {
-        const int k0 = grp * 256 * CPT + ctid * CPT;
-        const bool has_cols = k0 < K;
-        const int head = has_cols ? k0 / p.d : 0, dd = has_cols ? k0 - head * p.d : 0;
-        // (raw, unconditional loads: the pass below requests its own before anything looks at these)
-        uint32_t wraw[HM][CPT / 2];
-        float wj[HM][CPT], dw[HM][CPT];
+template <typename T, int HM>
+__global__ void __launch_bounds__(64 * BWD_WAVES) __attribute__((amdgpu_waves_per_eu(HM <= 16 ? 4 : 2))) dyn_bias_bwd_kernel(const DynBiasParams p) {
+    using E = Elem<T>;
+    constexpr int NS = HM / 4, NB = (HM + 15) / 16;  // steps of dV over the heads; sixteens of heads
+    constexpr int PITCH = 16 * NB + 4;
+    __shared__ __attribute__((aligned(256))) char smem[BWD_WAVES * 8192 + 2 * BWD_WAVES * HM * 4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
+    const int Hk = p.Hk, K = Hk * p.d;
+    const int col_waves = p.col_waves, tok_waves = BWD_WAVES / col_waves, cw = wave % col_waves, tw = wave / col_waves;
+    const int k0 = ((int)blockIdx.y * col_waves + cw) * BWD_COLS;
+    const int64_t row0 = (int64_t)blockIdx.x * p.rows_per_wg, n_rows = (int64_t)p.B * p.L;  // (fewer than 2^31 tokens: their values fill the memory)
+    const int n_tok = (int)(row0 + p.rows_per_wg < n_rows ? p.rows_per_wg : n_rows - row0);
+    const bool per_head = blockIdx.y == 0 && cw == 0;  // these waves make the sums of dA and dpb as well
+    float *part_w = p.part + (int64_t)blockIdx.x * p.part_stride;
+    float *s_wave = (float *)(smem + wave * 8192), *s_red = (float *)(smem + BWD_WAVES * 8192);
+
+    // batch entry and position of token t of the tile whose first one is (b0, l0)
+    auto place = [&](int b0, int l0, int t, int &b, int &l) {
+        b = b0;
+        l = l0 + t;
+        while (l >= p.L) { l -= p.L; b++; }
+    };
+    u32x4_t vraw[4];
+    uint16_t gb_raw[NS];
+    float dt_raw[NS];
+    const int kv = k0 + 8 * c < K ? k0 + 8 * c : 0, kv_head = kv / p.d;  // (columns beyond the last: any, their results go nowhere)
+    const int64_t col_v = (int64_t)kv_head * p.v_h + (kv - kv_head * p.d);
+    // requests tile i (tokens past the last one: it again)
+    auto fetch = [&](int i) {
+        const int at = 16 * i < n_tok ? 16 * i : n_tok - 1, left = n_tok - 1 - at;
+        const uint32_t base = (uint32_t)row0 + (uint32_t)at;
+        const int b0 = (int)(base / (uint32_t)p.L), l0 = (int)(base - (uint32_t)b0 * (uint32_t)p.L);
+        int b, l;
 #pragma unroll
-        for (int j = 0; j < HM; j++) {
+        for (int q = 0; q < 4; q++) {
+            place(b0, l0, 4 * q + g < left ? 4 * q + g : left, b, l);
+            vraw[q] = *(const u32x4_t *)((const uint16_t *)p.v + b * p.v_b + (int64_t)l * p.v_r + col_v);
+        }
+        const int t = c < left ? c : left;
+        place(b0, l0, t, b, l);
+        int g_mine = g;
+        asm volatile("" : "+v"(g_mine));  // (where the heads' rows begin is not kept over the tiles: registers)
 #pragma unroll
-            for (int e = 0; e < CPT; e += 2) {
-                wraw[j][e / 2] = *(const uint32_t *)((const uint16_t *)p.w + (int64_t)(j < Hk ? j : 0) * K + (has_cols ? k0 : 0) + e);
-                dw[j][e] = dw[j][e + 1] = 0.f;
+        for (int s = 0; s < NS; s++) {
+            const int j = 4 * s + g_mine < Hk ? 4 * s + g_mine : 0;
+            gb_raw[s] = ((const uint16_t *)p.dbias)[b * p.dbias_b + (int64_t)j * p.dbias_h + l];
+            dt_raw[s] = p.dt[(int64_t)(base + (uint32_t)t) * Hk + j];
+        }
+    };
+
+    f32x4_t dw[NB][8];
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) dw[nb][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float sum_a[NS], sum_pb[NS], a_mine[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) sum_a[s] = sum_pb[s] = 0.f;
+
+    if (k0 < K && 16 * tw < n_tok) {
+        fetch(tw);
+        uint32_t wraw[4][NS];
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const int j = 4 * s + g < Hk ? 4 * s + g : 0;
+            const uint32_t keep = 4 * s + g < Hk ? 0xffffffffu : 0u;
+            a_mine[s] = E::lo((uint32_t)((const uint16_t *)p.a)[j] & keep);
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                const int col = k0 + 32 * m + 8 * (c >> 2) + 2 * (c & 3);
+                wraw[m][s] = *(const uint32_t *)((const uint16_t *)p.w + (int64_t)j * K + (col < K ? col : 0)) & keep;
             }
         }
-        for (int64_t base = wg_row0; base < wg_row1; base += RB) {
-            // the first TB tokens' values are requested in front of everything else of the pass
-            const int n = (int)(wg_row1 - base < RB ? wg_row1 - base : RB);
-            uint32_t vraw[TB][CPT / 2];
-            const int b0 = (int)((uint32_t)base / (uint32_t)p.L), l0 = (int)base - b0 * p.L;  // (fewer than 2^31 tokens: their values fill the memory)
-            auto place = [&](int t, int &b, int &l) {  // batch entry and position of token base + t
-                b = b0;
-                l = l0 + t;
-                while (l >= p.L) { l -= p.L; b++; }
-            };
-            // (rows are walked by adding strides, not by a product per token and matrix in scalar arithmetic)
-            const int64_t col_v = (int64_t)head * p.v_h + dd, col_dv = (int64_t)head * p.dv_h + dd;
-            auto load_v = [&](int rr0) {
-                int b, l;
-                place(rr0 < n ? rr0 : n - 1, b, l);
-                const uint16_t *row = (const uint16_t *)p.v + b * p.v_b + (int64_t)l * p.v_r;
+        uint32_t heads = 0;  // a byte each: the heads that this lane's four pieces of a dV row lie in
 #pragma unroll
-                for (int u = 0; u < TB; u++) {
+        for (int m = 0; m < 4; m++) heads |= (uint32_t)((k0 + 32 * m + 8 * g) / p.d & 0xff) << (8 * m);
+        for (int i = tw; 16 * i < n_tok; i += tok_waves) {
+            const int left = n_tok - 16 * i;
+            // d_dt, where dV wants it and in LDS
+            float ddt[NS];
 #pragma unroll
-                    for (int e = 0; e < CPT / 2; e++) vraw[u][e] = *(const uint32_t *)(row + col_v + 2 * e);
-                    if (rr0 + u + 1 < n) {  // (past the last token: it again)
-                        row += p.v_r;
-                        if (++l == p.L) { l = 0; row += p.v_b - p.L * p.v_r; }
+            for (int s = 0; s < NS; s++) {
+                const float gb = E::lo((uint32_t)gb_raw[s]), dt = dt_raw[s];
+                const bool ok = c < left && 4 * s + g < Hk;
+                ddt[s] = ok ? gb * a_mine[s] * sigmoid_f(dt) : 0.f;
+                if (per_head) {
+                    sum_a[s] += ok ? gb * softplus_f(dt) : 0.f;
+                    sum_pb[s] += ddt[s];
+                }
+                s_wave[c * PITCH + 4 * s + g] = ddt[s];
+            }
+            __builtin_amdgcn_wave_barrier();  // (the LDS operations of one wave execute in order)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const uint32_t keep = 4 * q + g < left ? 0xffffffffu : 0u;  // (an infinity past the last token is not multiplied by its zero)
+                float dd[NB];
+#pragma unroll
+                for (int nb = 0; nb < NB; nb++) dd[nb] = s_wave[(4 * q + g) * PITCH + 16 * nb + (HM < 16 ? c & (HM - 1) : c)];
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    const uint32_t x = vraw[q][e / 2] & keep;
+#pragma unroll
+                    for (int nb = 0; nb < NB; nb++) {
+                        dw[nb][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(E::lo(x), dd[nb], dw[nb][e], 0, 0, 0);
+                        dw[nb][e + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(E::hi(x), dd[nb], dw[nb][e + 1], 0, 0, 0);
                     }
                 }
-            };
-            const int nh = (n + 1) / 2, h_lo = half ? nh : 0, h_hi = half ? n : nh;  // this half's tokens
-            load_v(h_lo);
-            uint16_t gb_raw[RB / RSTEP];
-            float dt_raw[RB / RSTEP];
-#pragma unroll
-            for (int i = 0; i < RB / RSTEP; i++) {
-                const int rr = rgroup + i * RSTEP;
-                int b, l;
-                place(rr < n ? rr : n - 1, b, l);
-                const int j = j_mine < Hk ? j_mine : 0;
-                gb_raw[i] = ((const uint16_t *)p.dbias)[b * p.dbias_b + (int64_t)j * p.dbias_h + l];
-                dt_raw[i] = p.dt[(base + (rr < n ? rr : n - 1)) * Hk + j];
             }
-            __syncthreads();
-            if (base == wg_row0) {
-#pragma unroll
-                for (int j = 0; j < HM; j++)
-#pragma unroll
-                    for (int e = 0; e < CPT; e += 2) {
-                        wj[j][e] = j < Hk ? E::lo(wraw[j][e / 2]) : 0.f;
-                        wj[j][e + 1] = j < Hk ? E::hi(wraw[j][e / 2]) : 0.f;
-                    }
+            __builtin_amdgcn_wave_barrier();
+            if (16 * (i + tok_waves) < n_tok) fetch(i + tok_waves);  // (on its way while dV is made)
+            int b, l;
+            {
+                const uint32_t base = (uint32_t)row0 + (uint32_t)(16 * i);
+                const int b0 = (int)(base / (uint32_t)p.L);
+                place(b0, (int)(base - (uint32_t)b0 * (uint32_t)p.L), c < left ? c : 0, b, l);
             }
-            // d_dt of the RB tokens of this pass -> LDS; the per-head sums are taken on the first column group
+            asm volatile("" : "+v"(heads));  // (the places themselves, computed in front of the loop, are eight registers)
+            uint16_t *orow = (uint16_t *)p.dv + b * p.dv_b + (int64_t)l * p.dv_r;
 #pragma unroll
-            for (int i = 0; i < RB / RSTEP; i++) {
-                const int rr = rgroup + i * RSTEP;
-                float ddt = 0.f;
-                if (j_mine < Hk && rr < n) {
-                    const float gb = E::lo((uint32_t)gb_raw[i]), dt = dt_raw[i];
-                    ddt = gb * a_mine * sigmoid_f(dt);
-                    if (grp == 0) {
-                        sum_a += gb * softplus_f(dt);
-                        sum_pb += ddt;
+            for (int m = 0; m < 4; m++) {
+                if (k0 + 32 * m < K) {
+                    f32x4_t lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int s = 0; s < NS; s++) {
+                        asm volatile("" : "+v"(wraw[m][s]));  // (kept packed: unpacked in front of the loop it is twice the registers)
+                        lo = __builtin_amdgcn_mfma_f32_16x16x4f32(E::lo(wraw[m][s]), ddt[s], lo, 0, 0, 0);
+                        hi = __builtin_amdgcn_mfma_f32_16x16x4f32(E::hi(wraw[m][s]), ddt[s], hi, 0, 0, 0);
                     }
+                    u32x4_t out;
+#pragma unroll
+                    for (int x = 0; x < 4; x++) out[x] = E::pack2(lo[x], hi[x]);
+                    const int kd = k0 + 32 * m + 8 * g, head = (int)(heads >> (8 * m) & 0xffu);
+                    if (c < left && kd < K) *(u32x4_a8_t *)(orow + head * p.dv_h + (kd - head * p.d)) = out;
                 }
-                s_ddt[rr * HM + j_mine] = ddt;
-            }
-            __syncthreads();
-            for (int rr0 = h_lo; rr0 < h_hi; rr0 += TB) {
-                if (rr0 > h_lo) load_v(rr0);
-                int b, l;
-                place(rr0, b, l);
-                uint16_t *orow = (uint16_t *)p.dv + b * p.dv_b + (int64_t)l * p.dv_r;
-#pragma unroll
-                for (int u = 0; u < TB; u++) {
-                    if (rr0 + u < h_hi && has_cols) {
-                        float v4[CPT], dv[CPT];
-#pragma unroll
-                        for (int e = 0; e < CPT; e += 2) {
-                            v4[e] = E::lo(vraw[u][e / 2]);
-                            v4[e + 1] = E::hi(vraw[u][e / 2]);
-                            dv[e] = dv[e + 1] = 0.f;
-                        }
-#pragma unroll
-                        for (int j = 0; j < HM; j++) {
-                            const float ddt = s_ddt[(rr0 + u) * HM + j];  // same address for the whole wave: a broadcast read; 0 beyond Hkv
-#pragma unroll
-                            for (int e = 0; e < CPT; e++) {
-                                dw[j][e] += ddt * v4[e];
-                                dv[e] += ddt * wj[j][e];
-                            }
-                        }
-#pragma unroll
-                        for (int e = 0; e < CPT; e += 2) *(uint32_t *)(orow + col_dv + e) = E::pack2(dv[e], dv[e + 1]);
-                    }
-                    orow += p.dv_r;
-                    if (++l == p.L) { l = 0; orow += p.dv_b - p.L * p.dv_r; }
-                }
-            }
-        }
-        // the halves' sums, in order, HC heads at a time
-#pragma unroll
-        for (int j0 = 0; j0 < HM; j0 += HC) {
-            __syncthreads();
-            if (half) {
-#pragma unroll
-                for (int j = 0; j < HC; j++)
-#pragma unroll
-                    for (int e = 0; e < CPT; e++) s_x[(j * CPT + e) * 256 + ctid] = dw[j0 + j][e];
-            }
-            __syncthreads();
-            if (!half && has_cols) {
-#pragma unroll
-                for (int j = 0; j < HC; j++)
-                    if (j0 + j < Hk) {
-#pragma unroll
-                        for (int e = 0; e < CPT; e++) part_w[(int64_t)(j0 + j) * K + k0 + e] = dw[j0 + j][e] + s_x[(j * CPT + e) * 256 + ctid];
-                    }
             }
         }
     }
-    // per-head sums: a head's threads in a wave, by lane swaps, then the waves in order.  (All of a head's NT / HM through LDS by one
-    // thread were a chain of 64 reads.)
+    // dW: lane (j, g) has columns 32 g + 4 r .. of head j in piece r = 2 i + e / 4 of eight; a wave adds up its share of the pieces
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) {
+        auto store = [&](int r, f32x4_t x) {
+            const int j = 16 * nb + c, col = k0 + 32 * g + 4 * r;
+            if (j < Hk && col < K) *(f32x4_t *)(part_w + (int64_t)j * K + col) = x;
+        };
+        auto piece = [&](int r) {
+            const int i = r >> 1, e = (r & 1) * 4;
+            return f32x4_t{dw[nb][e][i], dw[nb][e + 1][i], dw[nb][e + 2][i], dw[nb][e + 3][i]};
+        };
+        if (tok_waves == 1) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) store(r, piece(r));
+            continue;
+        }
+        if (nb) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 8; r++) *(f32x4_t *)(s_wave + (r * 64 + lane) * 4) = piece(r);
+        __syncthreads();
+        for (int r = tw * (8 / tok_waves); r < (tw + 1) * (8 / tok_waves); r++) {
+            const float *src = (const float *)(smem + cw * 8192) + (r * 64 + lane) * 4;
+            f32x4_t x = *(const f32x4_t *)src;
+            for (int w = 1; w < tok_waves; w++) x += *(const f32x4_t *)(src + w * col_waves * 2048);
+            store(r, x);
+        }
+    }
+    // dA and dpb: the sixteen tokens' lanes by swaps, then the waves in order
     if (blockIdx.y) return;
     auto fold = [&](float x) -> float {
-        const uint32_t u = __float_as_uint(x);
-        const auto r32 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-        x = __uint_as_float((uint32_t)r32[0]) + __uint_as_float((uint32_t)r32[1]);
-        if (HM <= 16) {
-            const uint32_t w = __float_as_uint(x);
-            const auto r16 = __builtin_amdgcn_permlane16_swap(w, w, false, false);
-            x = __uint_as_float((uint32_t)r16[0]) + __uint_as_float((uint32_t)r16[1]);
-        }
-        if (HM <= 8) x += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), 0x128, 0xf, 0xf, false));  // row_ror:8
+        auto ror = [&](auto ctrl) { x += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), decltype(ctrl)::value, 0xf, 0xf, false)); };
+        ror(std::integral_constant<int, 0x128>{});  // row_ror: 8, 4, 2, 1
+        ror(std::integral_constant<int, 0x124>{});
+        ror(std::integral_constant<int, 0x122>{});
+        ror(std::integral_constant<int, 0x121>{});
         return x;
     };
-    sum_a = fold(sum_a);
-    sum_pb = fold(sum_pb);
-    if ((tid & 63) < HM) {
-        s_red[0][tid >> 6][tid & 63] = sum_a;
-        s_red[1][tid >> 6][tid & 63] = sum_pb;
+    if (cw == 0) {
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const float sa = fold(sum_a[s]), sb = fold(sum_pb[s]);
+            if (c == 0) {
+                s_red[tw * HM + 4 * s + g] = sa;
+                s_red[(BWD_WAVES + tw) * HM + 4 * s + g] = sb;
+            }
+        }
     }
     __syncthreads();
-    if (tid < Hk) {
+    if ((int)threadIdx.x < Hk) {
         float sa = 0.f, sb = 0.f;
-#pragma unroll
-        for (int w = 0; w < NT / 64; w++) {
-            sa += s_red[0][w][tid];
-            sb += s_red[1][w][tid];
+        for (int w = 0; w < tok_waves; w++) {
+            sa += s_red[w * HM + threadIdx.x];
+            sb += s_red[(BWD_WAVES + w) * HM + threadIdx.x];
         }
-        part_w[(int64_t)Hk * K + tid] = sa;
-        part_w[(int64_t)Hk * K + Hk + tid] = sb;
+        part_w[(int64_t)Hk * K + threadIdx.x] = sa;
+        part_w[(int64_t)Hk * K + Hk + threadIdx.x] = sb;
     }
 }
 
@@ -421,19 +438,25 @@ hipError_t launch_dyn_bias_fwd(const DynBiasParams &p, int dtype, hipStream_t st
     return hipGetLastError();
 }
 
-// columns of V_flat per thread: four, where there are enough of them and the sums for them fit the registers
-static bool four_columns(int Hk, int d) { return Hk <= 16 && Hk * d >= 1024; }
-
-int dyn_bias_bwd_workgroups(int64_t n_rows, int Hk, int d, int *rows_per_wg) {
-    // Runs of 32 tokens while the device holds all workgroups at a time (the partials are Hkv * Hkv * d floats each), else runs as long
-    // as that takes, in whole eights.  A CU holds two workgroups of up to 8 heads with two columns a thread (105 registers) and one of
-    // all others (161 to 256): with twice as many as that a second round starts, mostly empty.  us, kernel and fold, 512 / 256 workgroups:
-    // 9000 tokens of 8 x 128 31.0 / 23.8, 16 x 256 140 / 92, 24 x 64 98.6 / 64.7; 16385 39.2 / 32.4, 183 / 136, 120 / 93; 33000 55.1 / 49.0, 280 / 233, 181 / 153;
-    // 131072 155 / 149, 802 / 736, 553 / 534; 8 x 64, which fits twice: 33000 33.2 / 38.3, 98304 61 / 80.  (Runs of whole passes of 64 tokens
-    // instead of whole eights: 33000 of 8 x 64 39.8.)
-    const int most = (Hk <= 8 && !four_columns(Hk, d) ? 2 : 1) * device_cus();
-    int64_t rows = 32;
-    if ((n_rows + 31) / 32 > most) rows = ((n_rows + most - 1) / most + 7) / 8 * 8;
+// Runs of tokens (what it returns), their length, and the column ranges that a workgroup takes.
+int dyn_bias_bwd_workgroups(int64_t n_rows, int Hk, int d, int *rows_per_wg, int *col_waves) {
+    const int groups = (Hk * d + BWD_COLS - 1) / BWD_COLS, cus = device_cus();
+    const int most = (Hk <= 8 && Hk * d < 1024 ? 2 : 1) * cus;  // (the partial results, Hkv * Hkv * d floats each, cost what a run of tokens does)
+    // Few tokens: a tile each for the eight waves of a workgroup of one column range; fewest partial results.  Up to two rounds of the two
+    // workgroups that a CU holds: us, up to one / two: 9000 tokens of 16 x 64 26.5 / 23.0, 4000 of 16 x 256 34.4 / 29.6, 9000 of 8 x 128
+    // 19.5 / 18.7, 30000 of 8 x 64 25.5 / 26.4.
+    if ((n_rows + 127) / 128 * groups <= 4 * cus && n_rows <= 64 * most) {
+        *rows_per_wg = BWD_WAVES * BWD_TOK;
+        *col_waves = 1;
+        return (int)((n_rows + 127) / 128);
+    }
+    // Else up to four column ranges to a workgroup, two waves each; eight, one each, where the registers of more than 16 heads leave room
+    // for one workgroup on a CU, or more than 16 ranges are rounds of their own (us, two / four / eight: 4 x 17701 of 16 x 64 92 / 92 / 101,
+    // 33000 of 8 x 128 39.7 / 37.5 / 39.4, of 32 x 64 196 / 175 / 167, 9000 of 16 x 256 66.7 / 60.8 / 55.6).
+    const int side = Hk > 16 || groups > 16 ? BWD_WAVES : BWD_WAVES / 2, in_turn = (groups + side - 1) / side;
+    *col_waves = (groups + in_turn - 1) / in_turn;
+    int64_t rows = 2 * BWD_TOK;
+    if ((n_rows + rows - 1) / rows > most) rows = ((n_rows + most - 1) / most + BWD_TOK - 1) / BWD_TOK * BWD_TOK;
     *rows_per_wg = (int)rows;
     return (int)((n_rows + rows - 1) / rows);
 }
@@ -441,21 +464,17 @@ int dyn_bias_bwd_workgroups(int64_t n_rows, int Hk, int d, int *rows_per_wg) {
 hipError_t launch_dyn_bias_bwd(const DynBiasParams &p, int dtype, hipStream_t stream) {
     const int64_t n_rows = (int64_t)p.B * p.L;
     if (n_rows <= 0) return hipSuccess;
-    const bool wide = four_columns(p.Hk, p.d);
-    const int groups = (p.Hk * p.d + (wide ? 1023 : 511)) / (wide ? 1024 : 512);  // column groups of the kernel
-    // (side by side where all of them run at once: a workgroup's time is its groups one behind the other.  us, before / now, the lane swaps of
-    // the per-head sums among them: 500 tokens of 16 x 256 52.9 / 17.8, 122 of 16 x 96 28.2 / 15.6, 2396 of 8 x 96 18.4 / 10.4, 2048 of 16 x 128
-    // 32.8 / 20.2; the sums alone: 4 x 2048 of 8 x 64 15.0 / 12.3, 83 of 4 x 128 11.5 / 8.5)
-    const dim3 grid(p.n_wg, p.n_wg * groups <= device_cus() ? groups : 1);
-    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(512), 0, stream, p); };
+    const int groups = (p.Hk * p.d + BWD_COLS - 1) / BWD_COLS, waves = p.col_waves * (BWD_WAVES / p.col_waves);
+    const dim3 grid(p.n_wg, (groups + p.col_waves - 1) / p.col_waves);
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64 * waves), 0, stream, p); };
     if (dtype == 0) {
-        if (p.Hk <= 8) wide ? go(dyn_bias_bwd_kernel<bf16_tag, 8, 4>) : go(dyn_bias_bwd_kernel<bf16_tag, 8, 2>);
-        else if (p.Hk <= 16) wide ? go(dyn_bias_bwd_kernel<bf16_tag, 16, 4>) : go(dyn_bias_bwd_kernel<bf16_tag, 16, 2>);
-        else go(dyn_bias_bwd_kernel<bf16_tag, 32, 2>);
+        if (p.Hk <= 8) go(dyn_bias_bwd_kernel<bf16_tag, 8>);
+        else if (p.Hk <= 16) go(dyn_bias_bwd_kernel<bf16_tag, 16>);
+        else go(dyn_bias_bwd_kernel<bf16_tag, 32>);
     } else {
-        if (p.Hk <= 8) wide ? go(dyn_bias_bwd_kernel<fp16_tag, 8, 4>) : go(dyn_bias_bwd_kernel<fp16_tag, 8, 2>);
-        else if (p.Hk <= 16) wide ? go(dyn_bias_bwd_kernel<fp16_tag, 16, 4>) : go(dyn_bias_bwd_kernel<fp16_tag, 16, 2>);
-        else go(dyn_bias_bwd_kernel<fp16_tag, 32, 2>);
+        if (p.Hk <= 8) go(dyn_bias_bwd_kernel<fp16_tag, 8>);
+        else if (p.Hk <= 16) go(dyn_bias_bwd_kernel<fp16_tag, 16>);
+        else go(dyn_bias_bwd_kernel<fp16_tag, 32>);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

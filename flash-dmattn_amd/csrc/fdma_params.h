@@ -390,11 +390,11 @@ struct DynBiasParams {
     void *dw, *da, *dpb;  // (Hk, Hk * d), (Hk), (Hk) or nullptr
     float *part;          // n_wg partials of part_stride floats: dW (Hk * Hk * d), dA (Hk), dpb (Hk)
     int64_t part_stride;
-    int32_t n_wg, rows_per_wg;
+    int32_t n_wg, rows_per_wg, col_waves;
 };
 hipError_t launch_dyn_bias_fwd(const DynBiasParams &p, int dtype, hipStream_t stream);
 hipError_t launch_dyn_bias_bwd(const DynBiasParams &p, int dtype, hipStream_t stream);
-int dyn_bias_bwd_workgroups(int64_t n_rows, int Hk, int d, int *rows_per_wg);
+int dyn_bias_bwd_workgroups(int64_t n_rows, int Hk, int d, int *rows_per_wg, int *col_waves);
 
 // Dynamic-LDS limit of a kernel, raised once per device (and again only for a larger request) instead of on every
 // launch: one `static DynSmemLimit` per launch site.  Later launches make no runtime call besides the launch itself.

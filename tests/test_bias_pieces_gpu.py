@@ -99,3 +99,31 @@ def test_gradients_of_column_groups(B, L, Hk, d, dtype):
     ref = (a64 * F.softplus(v64.reshape(B, L, -1) @ w64.t())).transpose(-1, -2).unsqueeze(-2)
     for x, y, z in zip(got, torch.autograd.grad(ref, wide, dbias.double()), again):
         assert rel_err(x, y) <= 2.0 ** -7 and torch.equal(x, z)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L,Hk,d,dtype", [
+    (1, 15, 8, 16, torch.bfloat16),      # a short tile, a full range of columns
+    (1, 17, 9, 16, torch.float16),       # a tile and a token; a range and half a block of columns; rows of up to sixteen heads
+    (2, 64, 1, 64, torch.bfloat16),      # a tile for every wave, half a range
+    (1, 129, 17, 16, torch.float16),     # a run of one token; more than sixteen heads; two whole ranges and a short one
+    (40, 3, 3, 80, torch.bfloat16),      # tiles that cross several batch entries
+    (1, 16400, 8, 128, torch.bfloat16),  # four ranges to a workgroup
+    (1, 9300, 16, 80, torch.float16),    # ten ranges: four, four and two
+    (1, 4200, 32, 72, torch.bfloat16),   # 18 of eight, eight and two
+])
+def test_gradients_of_column_ranges(B, L, Hk, d, dtype):
+    """The backward's products, tiles of 16 tokens by ranges of 128 columns.  Sums over the tokens in fp32, results rounded to 16 bits once."""
+    print("ranges", B, L, Hk, d, dtype, flush=True)
+    g = torch.Generator().manual_seed(L + Hk + d)
+    v = torch.randn(B, L, Hk, d, generator=g).to(dtype).to(DEV)
+    w = (torch.randn(Hk, Hk * d, generator=g) / (Hk * d) ** 0.5).to(dtype).to(DEV)
+    a, pb = torch.linspace(0.5, 1.5, Hk).to(dtype).to(DEV), torch.linspace(-1, 1, Hk).to(dtype).to(DEV)
+    dbias = torch.randn(B, Hk, 1, L, generator=g).to(dtype).to(DEV)
+    leaves = [t.requires_grad_(True) for t in (v, w, a, pb)]
+    got = torch.autograd.grad(dynamic_mask_bias(*leaves), leaves, dbias)
+    wide = [t.detach().double().requires_grad_(True) for t in leaves]
+    v64, w64, a64, pb64 = wide
+    ref = (a64 * F.softplus(v64.reshape(B, L, -1) @ w64.t() + pb64)).transpose(-1, -2).unsqueeze(-2)
+    for x, y in zip(got, torch.autograd.grad(ref, wide, dbias.double())):
+        assert rel_err(x, y) <= 2.0 ** -7
