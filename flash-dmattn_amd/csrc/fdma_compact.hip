@@ -86,23 +86,61 @@ __global__ void __launch_bounds__(SCAN_THREADS) compact_scan_kernel(const FwdPar
                                 count + pair, s_wave);
 }
 
+// K and V rows s_src[0 .. n) (below zero: left out) to rows 0, step, 2 step .. of kd / vd, by a workgroup of 256: up to four pieces of either
+// per thread are requested before the first is stored (one after the other each was a trip to memory of its own, and a wait for the store in front).
+__device__ __forceinline__ void copy_rows(const uint16_t *kb, int64_t k_r, const uint16_t *vb, int64_t v_r, uint16_t *kd, uint16_t *vd, int64_t step,
+                                          const int *s_src, int n, int d) {
+    const int CH = d / 8, rows = 256 / CH, left = 256 - rows * CH;  // 256 pieces on: so many rows and pieces
+    int rr = (int)threadIdx.x / CH, ch = (int)threadIdx.x - rr * CH;
+    while (rr < n) {
+        u32x4_t kv[4], vv[4];
+        int row[4], at[4];
+        bool on[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int src = s_src[rr < n ? rr : 0];
+            on[u] = rr < n && src >= 0;
+            row[u] = rr;
+            at[u] = ch * 8;
+            kv[u] = *(const u32x4_t *)(kb + (src >= 0 ? src : 0) * k_r + ch * 8);
+            vv[u] = *(const u32x4_t *)(vb + (src >= 0 ? src : 0) * v_r + ch * 8);
+            rr += rows;
+            ch += left;
+            if (ch >= CH) { ch -= CH; rr++; }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (on[u]) {
+                *(u32x4_t *)(kd + row[u] * step + at[u]) = kv[u];
+                *(u32x4_t *)(vd + row[u] * step + at[u]) = vv[u];
+            }
+    }
+}
+
 // orig: the caller's tensors.  kc / vc: dense [B*Hk, Lk, d] destinations.
 // copies_only: the per-pair lists and the fused bias exist already (made by the forward call whose workspace this is);
 // only the K / V rows are copied.
+// The kept keys are dealt to all workgroups of the pair in turn, so that each has its share of however few there are, and the count and the
+// list entries are one trip to memory, the rows and their bias another.  (64 keys in a row to each of the first workgroups, pieces of rows one
+// after the other: 1024 kept of 3001 x 4 heads, d = 256 8.4 us, now 6.0; 512 of 2048 x 32, d = 64 6.6 / 6.4, 2396 x 8, d = 96 7.5 either way.)
 template <typename T>
 __device__ __forceinline__ void gather_block(const FwdParams &p, const int32_t *idx, int32_t *cnt, const int32_t *count, float *fb,
                                              uint16_t *kc, uint16_t *vc, int ld, int Hfb, int block_x, int pair, bool copies_only = false) {
     using E = Elem<T>;
     const int b = pair / p.Hk, hk = pair % p.Hk;
     const int tid = threadIdx.x;
-    const int c0 = block_x * GATHER_KEYS;
+    const int c0 = block_x * GATHER_KEYS, blocks = (p.Lk + GATHER_KEYS - 1) / GATHER_KEYS;
+    const int rank = block_x + tid * blocks;  // the compacted key of thread `tid`, for the first GATHER_KEYS of them
     // Lists handed over by the caller (one row per mask row): this block copies its 64 entries of the row into the
     // per-pair arrays the kernels index (in place of the scan), and reads its own inputs from the source
     const int32_t *src_idx = idx + (size_t)pair * ld;
+    const bool lists = p.kept_idx && !copies_only;
+    const int srow = (p.m_b == 0 ? 0 : b) * p.Hm + (p.Hm == 1 ? 0 : hk);
+    if (lists) src_idx = p.kept_idx + (size_t)srow * p.kept_ld;
+    int src = -1;
+    if (tid < GATHER_KEYS && rank < p.Lk) src = src_idx[rank];
     int n;
-    if (p.kept_idx && !copies_only) {
-        const int srow = (p.m_b == 0 ? 0 : b) * p.Hm + (p.Hm == 1 ? 0 : hk);
-        src_idx = p.kept_idx + (size_t)srow * p.kept_ld;
+    if (lists) {
         // (lists are device data the host cannot check: a list made for a longer key axis than this call's must not
         // take reads or gradient writes past the tensors, so counts and columns are held inside [0, Lk))
         n = p.kept_count[srow];
@@ -116,43 +154,29 @@ __device__ __forceinline__ void gather_block(const FwdParams &p, const int32_t *
     } else {
         n = count[pair];
     }
-    if (c0 >= n) return;
+    if (block_x >= n) return;
+    const int mine = (n - 1 - block_x) / blocks + 1;
     __shared__ int s_src[GATHER_KEYS];
-    if (tid < GATHER_KEYS) {
-        const int32_t col = (c0 + tid < n) ? src_idx[c0 + tid] : -1;
-        s_src[tid] = col < p.Lk ? col : p.Lk - 1;
-    }
+    if (tid < GATHER_KEYS) s_src[tid] = rank < n ? (src < p.Lk ? src : p.Lk - 1) : -1;
     __syncthreads();
-    const int CH = p.d / 8;
     const uint16_t *kb = (const uint16_t *)p.k + b * p.k_b + kv_head(p, hk) * p.k_h;
     const uint16_t *vb = (const uint16_t *)p.v + b * p.v_b + kv_head(p, hk) * p.v_h;
-    uint16_t *kd = kc + ((size_t)pair * p.Lk + c0) * p.d;
-    uint16_t *vd = vc + ((size_t)pair * p.Lk + c0) * p.d;
-    for (int it = tid; it < GATHER_KEYS * CH; it += 256) {
-        const int rr = it / CH, ch = it - rr * CH;
-        const int src = s_src[rr];
-        if (src >= 0) {
-            const u32x4_t kv = *(const u32x4_t *)(kb + (int64_t)src * p.k_r + ch * 8);
-            const u32x4_t vv = *(const u32x4_t *)(vb + (int64_t)src * p.v_r + ch * 8);
-            *(u32x4_t *)(kd + (size_t)rr * p.d + ch * 8) = kv;
-            *(u32x4_t *)(vd + (size_t)rr * p.d + ch * 8) = vv;
-        }
-    }
-    if (copies_only) return;
-    // fused bias of the compacted keys, one vector per bias class of this kv head
-    const int G = p.H / p.Hk;
-    const int nfb = Hfb == p.H ? G : 1;
-    for (int it = tid; it < GATHER_KEYS * nfb; it += 256) {
-        const int gi = it / GATHER_KEYS, rr = it - gi * GATHER_KEYS;
-        const int src = s_src[rr];
-        if (src < 0) continue;
-        const int hfb = Hfb == p.H ? hk * G + gi : hk;
-        float v = 0.f;
-        if (p.bias) {
-            const int hb = p.Hb == p.H ? hfb : (p.Hb == 1 ? 0 : kv_head(p, hk));
-            v = E::lo((uint32_t)((const uint16_t *)p.bias)[b * p.bi_b + hb * p.bi_h + src]) * kLog2e;
-        }
-        fb[((size_t)b * Hfb + hfb) * ld + c0 + rr] = v;
+    // fused bias of the compacted keys, one vector per bias class of this kv head; requested in front of the rows
+    const int G = p.H / p.Hk, nfb = copies_only ? 0 : Hfb == p.H ? G : 1;
+    auto bias_head = [&](int gi) { return Hfb == p.H ? hk * G + gi : hk; };
+    auto bias_of = [&](int gi, int col) -> uint32_t {
+        if (!p.bias || col < 0) return 0u;
+        const int hb = p.Hb == p.H ? bias_head(gi) : (p.Hb == 1 ? 0 : kv_head(p, hk));
+        return (uint32_t)((const uint16_t *)p.bias)[b * p.bi_b + hb * p.bi_h + col];
+    };
+    const int gi0 = tid / GATHER_KEYS, rr = tid % GATHER_KEYS;
+    const uint32_t braw0 = gi0 < nfb ? bias_of(gi0, s_src[rr]) : 0u;
+    copy_rows(kb, p.k_r, vb, p.v_r, kc + ((size_t)pair * p.Lk + block_x) * p.d, vc + ((size_t)pair * p.Lk + block_x) * p.d, (int64_t)blocks * p.d,
+              s_src, mine, p.d);
+    for (int gi = gi0; gi < nfb; gi += 256 / GATHER_KEYS) {
+        if (s_src[rr] < 0) continue;
+        const uint32_t braw = gi == gi0 ? braw0 : bias_of(gi, s_src[rr]);
+        fb[((size_t)b * Hfb + bias_head(gi)) * ld + block_x + rr * blocks] = E::lo(braw) * kLog2e;
     }
 }
 

@@ -90,6 +90,27 @@ def test_attention_with_handed_over_lists_is_bit_identical(case, mode):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("Lk,H,Hk,D,bias_heads,W", [
+    (63, 2, 1, 8, 1, 63),        # a workgroup per pair, a piece to a row
+    (65, 2, 1, 64, 1, 64),       # two; the second has every other key
+    (640, 2, 2, 96, 2, 9),       # fewer keys than workgroups; twelve pieces to a row
+    (641, 4, 2, 256, 2, 11),     # as many
+    (1000, 10, 1, 128, 10, 700), # a bias of ten heads: three passes over them
+    (1000, 12, 2, 200, 12, 1000),
+])
+def test_handed_over_lists_are_dealt_to_the_workgroups(Lk, H, Hk, D, bias_heads, W):
+    """The gather of handed-over lists deals the keys to all workgroups of a pair; the one-launch scan does not.  The same bits."""
+    q, k, v, bias = _inputs(2, 70, Lk, H, Hk, D, bias_heads, seed=Lk + D)
+    set_compact("2")
+    try:
+        mask = M.topk_mask(bias[:, :Hk], None, W, torch.finfo(bias.dtype).min)
+        assert M.kept_keys_of(mask) is not None
+        for a, b in zip(_run(q, k, v, mask, bias), _run(q, k, v, mask.clone(), bias)):
+            assert torch.equal(a, b)
+    finally:
+        set_compact("auto")
+
+
 @pytest.mark.parametrize("Lk", [1, 15, 16, 17, 255, 256, 257, 511, 512, 513, 1000, 1281])
 @pytest.mark.parametrize("pattern", ["random", "all", "last_only", "first_segments_empty", "every_256th"])
 def test_forward_scan_and_gather_in_one_launch_at_segment_boundaries(Lk, pattern):
