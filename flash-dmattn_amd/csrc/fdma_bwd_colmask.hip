@@ -48,7 +48,12 @@ template <int D> constexpr bool RAGGED_TURNS = D <= 128;
 
 // CMP: the key axis is the compacted list of kept columns (fdma_compact.hip); a lane still owns one key,
 // reads it from the dense copies, and writes its gradients to the key's original row / column.
-template <typename T, int D, bool CAUSAL, bool CMP>
+// DC: the head dims that are worked on, 96 of a 128-wide tile for head dims 65 to 96 (here and in dQ).  The tile itself stays as wide: its
+// swizzle and the direct loads are made for rows of 256 bytes.  A quarter of the products is gone, and with it the spilled registers (256 and up
+// to 52 bytes of scratch a lane; 223 and none).  Forward + backward at d = 96, 128 dims / 96 of them, us: ragged 3601 and others x 32/8
+// heads 658 / 587, 4466 and others x 16/16 519 / 461, 2752 and others x 2/1 137 / 126; layer of 4 x 2432 x 16/8 365 / 333; 8256 x 16/8, 128 kept
+// 124 / 116.
+template <typename T, int D, int DC, bool CAUSAL, bool CMP>
 __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const BwdParams p) {
     using E = Elem<T>;
     using SM = KvcSmem<D>;
@@ -56,8 +61,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const Bwd
     constexpr int BM = SM::BM;       // query rows per step
     constexpr int SUB = KV_BM / BM;  // steps per planning block
     constexpr bool V_LDS = SM::V_LDS;
-    constexpr int KS = D / 16;
-    constexpr int DB = D / 32;
+    constexpr int KS = DC / 16;
+    constexpr int DB = DC / 32;
     constexpr int MB = BM / 32;
     constexpr int CH = D / 8, RPP = NTHREADS / CH, Q_IT = BM / RPP;
     // DMA: the Q / dO tiles and the row statistics of a step go from global memory straight into LDS
@@ -406,7 +411,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const Bwd
                 if (which) dp[mb] = E::mfma(a[fi], V_LDS ? vl[V_LDS ? ks : 0] : vf[V_LDS ? 0 : ks], dp[mb]);
                 else s[mb] = E::mfma(a[fi], kf[ks], s[mb]);
                 if constexpr (DMA) {
-                    if (fi % 3 == 1 && fi / 3 <= 2 * Q_IT) dma_piece(fi / 3);
+                    constexpr int EVERY = NF / (2 * Q_IT + 1);
+                    if (fi % EVERY == 1 && fi / EVERY <= 2 * Q_IT) dma_piece(fi / EVERY);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -584,7 +590,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const Bwd
             for (int gh = 0; gh < G; gh++)
                 if (gh < gi0 || gh > g_end) p.db_part[((int64_t)slot * G + gh) * KV_BN + (key - n0)] = 0.f;
         }
-        f32x4_t *dst = (f32x4_t *)p.dkv_part + (int64_t)slot * (2 * KV_BN * D / 4) + wave * DB * 4 * 64 + lane;
+        f32x4_t *dst = (f32x4_t *)p.dkv_part + (int64_t)slot * (2 * KV_BN * D / 4) + wave * (D / 32) * 4 * 64 + lane;
 #pragma unroll
         for (int db = 0; db < DB; db++)
 #pragma unroll
@@ -665,14 +671,14 @@ __global__ void __launch_bounds__(NTHREADS) bwd_dkdv_parts_sum_kernel(const BwdP
         const int lane = t & 63, w = t >> 6;  // w = ((mat * 4 + wave) * DB + db) * 2 + blk
         const int blk = w & 1, db = (w >> 1) % DB, kw = (w >> 1) / DB % 4, mat = (w >> 1) / DB / 4;
         const float *src = p.dkv_part + (int64_t)slot * 2 * PER + mat * PER + (((kw * DB + db) * 4 + 2 * blk) * 64 + lane) * 4;
+        const int key = n0 + kw * 32 + (lane & 31), c = 32 * db + 16 * blk + 8 * (lane >> 5);
         f32x4_t a0 = {0, 0, 0, 0}, a1 = {0, 0, 0, 0};
 #pragma unroll 4
-        for (int i = 0; i < n; i++) {
+        for (int i = 0; i < (c < f.d ? n : 0); i++) {  // (columns beyond d need not have been written)
             const float *q = src + (int64_t)i * 2 * PER;
             a0 += *(const f32x4_t *)q;
             a1 += *(const f32x4_t *)(q + 256);
         }
-        const int key = n0 + kw * 32 + (lane & 31), c = 32 * db + 16 * blk + 8 * (lane >> 5);
         if (key < sq.Lk && c < f.d) {
             const float m = mat == 0 ? f.scale : 1.f;
             const u32x4_t o = {E::pack2(a0[0] * m, a0[1] * m), E::pack2(a0[2] * m, a0[3] * m), E::pack2(a1[0] * m, a1[1] * m), E::pack2(a1[2] * m, a1[3] * m)};
@@ -701,10 +707,12 @@ hipError_t launch_dkdv_grid(const BwdParams &p, int grid, hipStream_t stream) {
     if constexpr (D > 128) {
         return launch_bwd_dkdv_256(p, std::is_same<T, bf16_tag>::value ? 0 : 1, grid, stream);
     } else {
-        auto kern = bwd_dkdv_colmask_kernel<T, D, CAUSAL, CMP>;
+        constexpr int LESS = D == 128 ? 96 : D;
+        const bool less = p.f.d <= LESS;
+        auto kern = less ? bwd_dkdv_colmask_kernel<T, D, LESS, CAUSAL, CMP> : bwd_dkdv_colmask_kernel<T, D, D, CAUSAL, CMP>;
         const int smem = KvcSmem<D>::TOTAL;
-        static DynSmemLimit smem_limit;
-        hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
+        static DynSmemLimit smem_limit[2];  // one per instantiation
+        hipError_t e = smem_limit[less].ensure((const void *)kern, (int)smem);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(kern, dim3(grid), dim3(NTHREADS), smem, stream, p);
         return hipGetLastError();
@@ -758,13 +766,13 @@ template <int D, int BN> struct DqcSmem {
 // registers, whose wait is a wait for every direct load in front of it).
 // KG: key groups of four waves.  Two take the tiles in turn, each with LDS and barriers' worth of stages of its own, and add their sums
 // up through LDS at the end: half the chain of tiles for grids that leave CUs empty (see dq_key_groups).
-template <typename T, int D, int BN, bool CAUSAL, bool CMP, bool BARE, int KG>
+template <typename T, int D, int DC, int BN, bool CAUSAL, bool CMP, bool BARE, int KG>
 __device__ __forceinline__ void dq_colmask(const BwdParams &p) {
     using E = Elem<T>;
     using SM = DqcSmem<D, BN>;
     using TL = LdsTile<D>;
-    constexpr int KS = D / 16;
-    constexpr int DB = D / 32;
+    constexpr int KS = DC / 16;
+    constexpr int DB = DC / 32;
     constexpr int MB = BN / 32;
     constexpr int KB = BN / 16;
     constexpr int CH = D / 8, RPP = NTHREADS / CH, K_IT = BN / RPP;
@@ -1203,11 +1211,15 @@ __device__ __forceinline__ void dq_colmask(const BwdParams &p) {
                     // (this wave's own copy of that column was fetched a tile ago, in front of the N_DMA loads of the
                     // tile after it: wait for it alone -- vmcnt N_DMA, no wait for LDS reads or exports)
                     if (DMA_COL && kb == 0 && db == 0) __builtin_amdgcn_s_waitcnt(0x0F70 | N_DMA);
-                    if (DMA_COL && kb == 0 && db < 4) nb[db] = __builtin_bit_cast(f32x4_t, lds_ld128(bs_n + 16 * (db & 1) + 64 * (db >> 1)));
-                    if (kb == KB - 1 && db < 4) {
 #pragma unroll
-                        for (int e = 0; e < 4; e++) s[0][4 * db + e] = DMA_COL ? nb[db][e] - lse2 : -lse2;
-                    }
+                    for (int x = 0; x < 4; x++)  // (four pieces over the block's slots)
+                        if (x * DB / 4 == db) {
+                            if (DMA_COL && kb == 0) nb[x] = __builtin_bit_cast(f32x4_t, lds_ld128(bs_n + 16 * (x & 1) + 64 * (x >> 1)));
+                            if (kb == KB - 1) {
+#pragma unroll
+                                for (int e = 0; e < 4; e++) s[0][4 * x + e] = DMA_COL ? nb[x][e] - lse2 : -lse2;
+                            }
+                        }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -1235,23 +1247,27 @@ __device__ __forceinline__ void dq_colmask(const BwdParams &p) {
     if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0x0070);
     if constexpr (KG == 2) {  // each group hands the other's half of the head dim over and finishes its own
         __syncthreads();  // (every wave's reads of the last tiles, and its direct loads)
-        static_assert(2 * 4 * (DB / 2) * 4096 <= 2 * SM::GROUP, "the halves lie where the tiles were");
-        f32x4_t *theirs = (f32x4_t *)smem_all + ((1 - kgrp) * 4 + wave) * (DB / 2) * 4 * 64 + lane, *mine = (f32x4_t *)smem_all + (kgrp * 4 + wave) * (DB / 2) * 4 * 64 + lane;
+        static_assert(2 * 4 * DB * 2048 <= 2 * SM::GROUP, "the halves lie where the tiles were");
+        // (eight head-dim elements, 2 db + blk, at a time: the first DB of them are group 0's)
+        f32x4_t *theirs = (f32x4_t *)smem_all + ((1 - kgrp) * 4 + wave) * DB * 2 * 64 + lane, *mine = (f32x4_t *)smem_all + (kgrp * 4 + wave) * DB * 2 * 64 + lane;
 #pragma unroll
-        for (int db = 0; db < DB; db++)
-            if (db / (DB / 2) != kgrp) {
+        for (int u = 0; u < 2 * DB; u++)
+            if (u / DB != kgrp) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) theirs[(db % (DB / 2) * 4 + q) * 64] = f32x4_t{dq[db][4 * q], dq[db][4 * q + 1], dq[db][4 * q + 2], dq[db][4 * q + 3]};
+                for (int q = 0; q < 2; q++) {
+                    const int e = 8 * (u & 1) + 4 * q;
+                    theirs[(u % DB * 2 + q) * 64] = f32x4_t{dq[u / 2][e], dq[u / 2][e + 1], dq[u / 2][e + 2], dq[u / 2][e + 3]};
+                }
             }
         __syncthreads();
 #pragma unroll
-        for (int db = 0; db < DB; db++)
-            if (db / (DB / 2) == kgrp) {
+        for (int u = 0; u < 2 * DB; u++)
+            if (u / DB == kgrp) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const f32x4_t t = mine[(db % (DB / 2) * 4 + q) * 64];
+                for (int q = 0; q < 2; q++) {
+                    const f32x4_t t = mine[(u % DB * 2 + q) * 64];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) dq[db][4 * q + e] += t[e];
+                    for (int e = 0; e < 4; e++) dq[u / 2][8 * (u & 1) + 4 * q + e] += t[e];
                 }
             }
     }
@@ -1261,7 +1277,7 @@ __device__ __forceinline__ void dq_colmask(const BwdParams &p) {
         for (int db = 0; db < DB; db++)
 #pragma unroll
             for (int blk = 0; blk < 2; blk++) {
-                if (KG == 2 && db / (DB / 2) != kgrp) continue;
+                if (KG == 2 && (2 * db + blk) / DB != kgrp) continue;
                 const int c = 32 * db + 16 * blk + 8 * g;
                 if (c < f.d) {
                     u32x4_t w;
@@ -1276,11 +1292,15 @@ __device__ __forceinline__ void dq_colmask(const BwdParams &p) {
 
 template <typename T, int D, int BN, bool CAUSAL, bool CMP, bool BARE>
 __global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_colmask_kernel(const BwdParams p) {
-    dq_colmask<T, D, BN, CAUSAL, CMP, BARE, 1>(p);
+    dq_colmask<T, D, D, BN, CAUSAL, CMP, BARE, 1>(p);
 }
-template <typename T, int D, int BN, bool CAUSAL, bool BARE>
+template <typename T, bool CAUSAL, bool CMP, bool BARE>
+__global__ void __launch_bounds__(NTHREADS, 2) bwd_dq_96_kernel(const BwdParams p) {
+    dq_colmask<T, 128, 96, 32, CAUSAL, CMP, BARE, 1>(p);
+}
+template <typename T, int D, int DC, int BN, bool CAUSAL, bool BARE>
 __global__ void __launch_bounds__(2 * NTHREADS, 2) bwd_dq_groups_kernel(const BwdParams p) {
-    dq_colmask<T, D, BN, CAUSAL, false, BARE, 2>(p);
+    dq_colmask<T, D, DC, BN, CAUSAL, false, BARE, 2>(p);
 }
 
 // Two key groups to a workgroup of dQ where there is no mask and no bias, the rows are long and there are no more workgroups than CUs
@@ -1295,26 +1315,32 @@ bool dq_key_groups(const FwdParams &f) {
     return blocks <= 9 * (int64_t)device_cus() / 4;
 }
 
+template <typename T, int D, int DC, bool CAUSAL>
+hipError_t launch_dq_dims(const BwdParams &p, int grid, hipStream_t stream) {
+    const FwdParams &f = p.f;
+    constexpr int BN = D > 64 ? 32 : 64;  // at d = 128 a 64-key tile would spill registers
+    constexpr bool SWZ = LdsTile<D>::SWZ;
+    const int which = f.cmp.on ? 1 : (SWZ && !f.mask && !f.bias ? 2 : 0);
+    const bool two = dq_key_groups(f);
+    auto kern = bwd_dq_groups_kernel<T, D, DC, BN, CAUSAL, SWZ>;
+    if constexpr (DC == D) {
+        if (!two) kern = which == 1 ? bwd_dq_colmask_kernel<T, D, BN, CAUSAL, true, false>
+                                    : (which == 2 ? bwd_dq_colmask_kernel<T, D, BN, CAUSAL, false, SWZ> : bwd_dq_colmask_kernel<T, D, BN, CAUSAL, false, false>);
+    } else {
+        if (!two) kern = which == 1 ? bwd_dq_96_kernel<T, CAUSAL, true, false> : (which == 2 ? bwd_dq_96_kernel<T, CAUSAL, false, true> : bwd_dq_96_kernel<T, CAUSAL, false, false>);
+    }
+    const int smem = two ? 2 * DqcSmem<D, BN>::GROUP : DqcSmem<D, BN>::TOTAL;
+    static DynSmemLimit smem_limit[4];  // one per instantiation: the limit is a property of the kernel
+    hipError_t e = smem_limit[two ? 3 : which].ensure((const void *)kern, (int)smem);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(two ? 2 * NTHREADS : NTHREADS), smem, stream, p);
+    return hipGetLastError();
+}
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_dq_grid(const BwdParams &p, int grid, hipStream_t stream) {
-    const FwdParams &f = p.f;
-    if constexpr (D > 128) {
-        return launch_bwd_dq_256(p, std::is_same<T, bf16_tag>::value ? 0 : 1, grid, stream);
-    } else {
-        constexpr int BN = D > 64 ? 32 : 64;  // at d = 128 a 64-key tile would spill registers
-        constexpr bool SWZ = LdsTile<D>::SWZ;
-        const int which = f.cmp.on ? 1 : (SWZ && !f.mask && !f.bias ? 2 : 0);
-        auto kern = which == 1 ? bwd_dq_colmask_kernel<T, D, BN, CAUSAL, true, false>
-                               : (which == 2 ? bwd_dq_colmask_kernel<T, D, BN, CAUSAL, false, SWZ> : bwd_dq_colmask_kernel<T, D, BN, CAUSAL, false, false>);
-        const bool two = dq_key_groups(f);
-        if (two) kern = bwd_dq_groups_kernel<T, D, BN, CAUSAL, SWZ>;
-        const int smem = two ? 2 * DqcSmem<D, BN>::GROUP : DqcSmem<D, BN>::TOTAL;
-        static DynSmemLimit smem_limit[4];  // one per instantiation: the limit is a property of the kernel
-        hipError_t e = smem_limit[two ? 3 : which].ensure((const void *)kern, (int)smem);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(two ? 2 * NTHREADS : NTHREADS), smem, stream, p);
-        return hipGetLastError();
-    }
+    if constexpr (D > 128) return launch_bwd_dq_256(p, std::is_same<T, bf16_tag>::value ? 0 : 1, grid, stream);
+    else if constexpr (D == 128) return p.f.d <= 96 ? launch_dq_dims<T, D, 96, CAUSAL>(p, grid, stream) : launch_dq_dims<T, D, D, CAUSAL>(p, grid, stream);
+    else return launch_dq_dims<T, D, D, CAUSAL>(p, grid, stream);
 }
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_dq(const BwdParams &p, hipStream_t stream) {
