@@ -72,7 +72,11 @@ template <int D, int BN> struct CmSmem {
 // CMP: K / V are the compacted copies of the kept columns (see fdma_compact.hip).  The key axis then has
 // `count` columns, all kept; the fused bias vector comes pre-gathered, and the causal limit of a query row
 // is the number of kept columns at or below its diagonal instead of the column index itself.
-template <typename T, int D, int BN, bool CAUSAL, int NW, bool CMP, int KG>
+// DC: the head dims that are worked on, 96 of a 128-wide tile for head dims 65 to 96 (here and in fdma_fwd_wide.hip): a quarter of the products
+// less, the staging as it is.  d = 96, 128 dims / 96 of them, us: 4 x 13120 x 8/4 heads, 3606 kept 390 / 335; 22912 x 16/16, 1280 kept, not
+// causal 235 / 204; ragged 4026 and others x 16/8 95.4 / 82.5; key groups 2 x 128 x 16/8 against 861 kept of 1817 24.2 / 22.7, 4 x 1152 x
+// 16/8, 128 kept 22.7 / 21.8.
+template <typename T, int D, int DC, int BN, bool CAUSAL, int NW, bool CMP, int KG>
 __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fwd_colmask_kernel(const FwdParams p) {
     constexpr int NTHREADS = 64 * NW;         // of a key group
     static_assert(KG == 1 || NW == 4, "key groups are for small grids, which have 128-row workgroups");
@@ -83,8 +87,8 @@ __global__ void __launch_bounds__(64 * NW * KG, (NW == 4 && KG == 1) ? 2 : 1) fw
     using E = Elem<T>;
     using SM = CmSmem<D, BN>;
     constexpr int KQ = BN / 4;                // key quads per tile
-    constexpr int KS = D / 16;
-    constexpr int DB = D / 32;
+    constexpr int KS = DC / 16;
+    constexpr int DB = DC / 32;
     constexpr int BM = 32 * NW;
     constexpr int CH = D / 8;                 // 16-byte chunks per K row
     constexpr int K_RPP = STHREADS / CH;      // K rows staged per pass
@@ -806,10 +810,12 @@ template <typename T> hipError_t launch_merge(const FwdParams &p, hipStream_t st
 template <typename T, int D, int BN, bool CAUSAL, bool CMP, int NW = 4, int KG = 1>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     constexpr int BM = 32 * NW;
-    auto kern = fwd_colmask_kernel<T, D, BN, CAUSAL, NW, CMP, KG>;
+    constexpr int LESS = D == 128 ? 96 : D;
+    const bool less = p.d <= LESS;
+    auto kern = less ? fwd_colmask_kernel<T, D, LESS, BN, CAUSAL, NW, CMP, KG> : fwd_colmask_kernel<T, D, D, BN, CAUSAL, NW, CMP, KG>;
     const int smem = KG * CmSmem<D, BN>::TOTAL;
-    static DynSmemLimit smem_limit;
-    hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
+    static DynSmemLimit smem_limit[2];  // one per instantiation
+    hipError_t e = smem_limit[less].ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
     FwdParams pr = p;
     const int grid = row_grid(pr, BM);

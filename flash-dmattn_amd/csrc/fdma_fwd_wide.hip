@@ -64,11 +64,12 @@ template <int D_, int RG> struct Cfg {
     static_assert(8 * RPP % 16 == 0, "a wave's pieces lie rows of one swizzle apart");
 };
 
-template <typename T, int D, int RG, bool CAUSAL, bool CMP>
+// DC: the head dims that are worked on, 96 of a 128-wide tile for head dims 65 to 96 (the merge takes the others along as zeros).
+template <typename T, int D, int DC, int RG, bool CAUSAL, bool CMP>
 __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const FwdParams p) {
     using E = Elem<T>;
     using C = Cfg<D, RG>;
-    constexpr int KG = C::KG, BM = C::BM, BN = C::BN, ROW = C::ROW, TILE = C::TILE, NP = C::NP, KS = D / 16, DB = D / 32;
+    constexpr int KG = C::KG, BM = C::BM, BN = C::BN, ROW = C::ROW, TILE = C::TILE, NP = C::NP, KS = DC / 16, DB = DC / 32;
     constexpr int OFF_V = C::OFF_V, OFF_COL = C::OFF_COL, OFF_BITS = C::OFF_BITS, UPW = C::UPW, UPP = C::UPP;
     constexpr bool ONE = C::ONE, SHARES = CMP && D <= 128;  // (key_shares cuts nothing above)
     extern __shared__ __attribute__((aligned(256))) char smem[];
@@ -244,9 +245,9 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
     uint32_t tr_off = lds0 + OFF_V + (uint32_t)(32 * kg) * ROW + tr_chunk<D>(g, tr_lane(lane));
     const uint32_t col_off = lds0 + OFF_COL + 128 * kg + 32 * g;
 
-    f32x16_t o[DB];
+    f32x16_t o[D / 32];
 #pragma unroll
-    for (int db = 0; db < DB; db++)
+    for (int db = 0; db < D / 32; db++)
 #pragma unroll
         for (int i = 0; i < 16; i++) o[db][i] = 0.f;
     float row_sum = 0.f, row_ref = -INFINITY;  // relative to exp2(row_ref); -inf: no visible key met yet
@@ -512,9 +513,11 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
 template <typename T, int D, int RG, bool CAUSAL, bool CMP>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     using C = Cfg<D, RG>;
-    auto kern = fwd_wide_kernel<T, D, RG, CAUSAL, CMP>;
-    static DynSmemLimit smem_limit;
-    hipError_t e = smem_limit.ensure((const void *)kern, C::SMEM);
+    constexpr int LESS = D == 128 ? 96 : D;
+    const bool less = p.d <= LESS;
+    auto kern = less ? fwd_wide_kernel<T, D, LESS, RG, CAUSAL, CMP> : fwd_wide_kernel<T, D, D, RG, CAUSAL, CMP>;
+    static DynSmemLimit smem_limit[2];  // one per instantiation
+    hipError_t e = smem_limit[less].ensure((const void *)kern, C::SMEM);
     if (e != hipSuccess) return e;
     FwdParams pr = p;
     const int grid = row_grid(pr, C::BM);
