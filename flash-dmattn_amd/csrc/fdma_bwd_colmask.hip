@@ -566,6 +566,22 @@ __global__ void __launch_bounds__(NTHREADS, 2) bwd_dkdv_colmask_kernel(const Bwd
         }
         publish();
     };
+    if constexpr (DMA && CMP) {
+        // A wave behind the last kept key fetches its share of the tiles and leaves the products to the others.  Forward + backward, d = 128, us:
+        // 2 x 16000 x 16/4 heads, 400 kept, not causal 677 / 651, 2 x 19776 x 8/2, 96 kept 244 / 237, 4 x 8192 x 16/8, 170 kept 445 / 438; where no
+        // wave is without, 2048 kept of 8192 x 32/8, 706 / 704.  (At head dims up to 64 it costs more scalar registers than it gives: 12000 x 32/8,
+        // 300 kept 206 / 213; ragged calls, with few such blocks, the same either way.)
+        if (n0 + wave * 32 >= Lk) {
+            for (int step = 0; step < n_steps; step++) {
+                dma_begin(~step & 1);
+#pragma unroll
+                for (int n = 0; n <= 2 * Q_IT; n++) dma_piece(n);
+                dma_advance(step + 2 < n_steps);
+                publish();
+            }
+            return;
+        }
+    }
     for (int step = 0; step < n_steps; step += 2) {
         one_step(std::integral_constant<int, 0>(), step);
         if (step + 1 < n_steps) one_step(std::integral_constant<int, 1>(), step + 1);
