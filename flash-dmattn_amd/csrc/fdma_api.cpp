@@ -811,7 +811,7 @@ size_t fdma_dyn_bias_bwd_workspace_bytes(const fdma_dyn_bias_args *a) {
     if (!a || (int64_t)a->batch * a->seqlen_k <= 0) return 0;
     fdma::DynBiasParams p;
     fill_dyn_bias(a, p);
-    return (size_t)p.n_wg * p.part_stride * sizeof(float);
+    return (size_t)fdma::dyn_bias_bwd_parts((int64_t)a->batch * a->seqlen_k, a->num_heads_k, a->head_dim) * p.part_stride * sizeof(float);
 }
 
 int fdma_dyn_bias_fwd(const fdma_dyn_bias_args *a, void *hip_stream) {

@@ -438,10 +438,20 @@ hipError_t launch_dyn_bias_fwd(const DynBiasParams &p, int dtype, hipStream_t st
     return hipGetLastError();
 }
 
-// Runs of tokens (what it returns), their length, and the column ranges that a workgroup takes.
+// runs of tokens at most (their partial results, Hkv * Hkv * d floats each, cost what a run does)
+static int most_runs(int Hk, int d) { return (Hk <= 8 && Hk * d < 1024 ? 2 : 1) * device_cus(); }
+
+// The size of the workspace: a partial result for every 32 tokens or, where those are more than the most, for runs of whole eights.
+int dyn_bias_bwd_parts(int64_t n_rows, int Hk, int d) {
+    const int most = most_runs(Hk, d);
+    int64_t rows = 32;
+    if ((n_rows + rows - 1) / rows > most) rows = ((n_rows + most - 1) / most + 7) / 8 * 8;
+    return (int)((n_rows + rows - 1) / rows);
+}
+
+// Runs of tokens (what it returns: as many as dyn_bias_bwd_parts or fewer), their length, and the column ranges that a workgroup takes.
 int dyn_bias_bwd_workgroups(int64_t n_rows, int Hk, int d, int *rows_per_wg, int *col_waves) {
-    const int groups = (Hk * d + BWD_COLS - 1) / BWD_COLS, cus = device_cus();
-    const int most = (Hk <= 8 && Hk * d < 1024 ? 2 : 1) * cus;  // (the partial results, Hkv * Hkv * d floats each, cost what a run of tokens does)
+    const int groups = (Hk * d + BWD_COLS - 1) / BWD_COLS, cus = device_cus(), most = most_runs(Hk, d);
     // Few tokens: a tile each for the eight waves of a workgroup of one column range; fewest partial results.  Up to two rounds of the two
     // workgroups that a CU holds: us, up to one / two: 9000 tokens of 16 x 64 26.5 / 23.0, 4000 of 16 x 256 34.4 / 29.6, 9000 of 8 x 128
     // 19.5 / 18.7, 30000 of 8 x 64 25.5 / 26.4.

@@ -395,6 +395,7 @@ struct DynBiasParams {
 hipError_t launch_dyn_bias_fwd(const DynBiasParams &p, int dtype, hipStream_t stream);
 hipError_t launch_dyn_bias_bwd(const DynBiasParams &p, int dtype, hipStream_t stream);
 int dyn_bias_bwd_workgroups(int64_t n_rows, int Hk, int d, int *rows_per_wg, int *col_waves);
+int dyn_bias_bwd_parts(int64_t n_rows, int Hk, int d);  // partial results that a caller makes room for: at least as many
 
 // Dynamic-LDS limit of a kernel, raised once per device (and again only for a larger request) instead of on every
 // launch: one `static DynSmemLimit` per launch site.  Later launches make no runtime call besides the launch itself.
