@@ -66,7 +66,7 @@ template <int D_, int RG> struct Cfg {
 
 // DC: the head dims that are worked on, 96 of a 128-wide tile for head dims 65 to 96 (the merge takes the others along as zeros).
 template <typename T, int D, int DC, int RG, bool CAUSAL, bool CMP>
-__global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const FwdParams p) {
+__device__ __forceinline__ void fwd_wide(const FwdParams &p) {
     using E = Elem<T>;
     using C = Cfg<D, RG>;
     constexpr int KG = C::KG, BM = C::BM, BN = C::BN, ROW = C::ROW, TILE = C::TILE, NP = C::NP, KS = DC / 16, DB = DC / 32;
@@ -511,11 +511,22 @@ __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const Fwd
 }
 
 template <typename T, int D, int RG, bool CAUSAL, bool CMP>
+__global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const FwdParams p) {
+    fwd_wide<T, D, D, RG, CAUSAL, CMP>(p);
+}
+template <typename T, bool CAUSAL, bool CMP>
+__global__ void __launch_bounds__(NT, 2) fwd_96_kernel(const FwdParams p) {
+    fwd_wide<T, 128, 96, 2, CAUSAL, CMP>(p);
+}
+
+template <typename T, int D, int RG, bool CAUSAL, bool CMP>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     using C = Cfg<D, RG>;
-    constexpr int LESS = D == 128 ? 96 : D;
-    const bool less = p.d <= LESS;
-    auto kern = less ? fwd_wide_kernel<T, D, LESS, RG, CAUSAL, CMP> : fwd_wide_kernel<T, D, D, RG, CAUSAL, CMP>;
+    auto kern = fwd_wide_kernel<T, D, RG, CAUSAL, CMP>;
+    const bool less = D == 128 && p.d <= 96;
+    if constexpr (D == 128) {
+        if (less) kern = fwd_96_kernel<T, CAUSAL, CMP>;
+    }
     static DynSmemLimit smem_limit[2];  // one per instantiation
     hipError_t e = smem_limit[less].ensure((const void *)kern, C::SMEM);
     if (e != hipSuccess) return e;

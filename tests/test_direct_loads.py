@@ -71,3 +71,14 @@ def test_no_direct_load_in_flight_at_the_merge_of_key_groups(tmp_path):
         loads, early = _early_stores(body)
         assert loads > 0 and "ds_write_b128" in body, name
         assert not early, (name, early[:3])
+
+
+def test_nor_at_that_of_their_variants(tmp_path):
+    """The same kernels for head dims 65 to 96."""
+    text = _assembly("fdma_fwd_wide", tmp_path)
+    kernels = re.findall(r"^(_Z\S*fwd_96_kernel\S*):.*?\n(.*?)^\.Lfunc_end", text, re.M | re.S)
+    assert len(kernels) == 8
+    for name, body in kernels:
+        loads, early = _early_stores(body)
+        assert loads > 0 and "ds_write_b128" in body, name
+        assert not early, (name, early[:3])
