@@ -335,6 +335,13 @@ size_t fdma_fwd_workspace_bytes(const fdma_fwd_args *a) {
     return need + shares;
 }
 
+int fdma_fwd_takes_lists(const fdma_fwd_args *a) {
+    if (!a || a->seqlen_k <= 0 || a->num_heads_k <= 0 || a->seqlen_q <= 0 || fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k)) return 0;
+    fdma::FwdParams p;
+    fill_fwd_params(a, p);
+    return fdma::fwd_from_lists(p);
+}
+
 size_t fdma_fwd_optional_bytes(const fdma_fwd_args *a) {
     if (!a || a->num_heads_k <= 0) return 0;
     fdma::FwdParams p;
@@ -378,7 +385,7 @@ int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
         // that form skips tiles instead)
         fdma::FwdParams pv;
         if (fdma::compact_per_query_head(p, pv)) p = pv;
-        if (fdma::use_compact(p)) {
+        if (fdma::use_compact(p) && !(!a->workspace && fdma::fwd_from_lists(p))) {
             const size_t need = fdma::compact_bytes(p, false);
             if (!a->workspace || a->workspace_bytes < need)
                 return fail(FDMA_ERR_WORKSPACE, "forward workspace too small: need %zu bytes, got %zu", need, a->workspace_bytes);

@@ -897,6 +897,18 @@ static bool takes_key_groups(const FwdParams &p) {
     return 2 * blocks64 <= 5 * (int64_t)device_cus();
 }
 
+// Whether the forward can take handed-over lists of kept keys as they are, without copies of their rows (which a backward wants: a call whose
+// workspace holds them makes them).  The gather in front, 5 to 7 us, is gone; a tile pays two reads of LDS and a product per row piece.  Copies /
+// rows where they lie, us, the whole layer: 3001 tokens x 8/4 heads, d = 256, 1024 kept 50.7 / 47.4, 8192 x 8/4, 2048 kept 101 / 100, 2 x 6000
+// x 8/4, all kept 321 / 319; d = 128: 2000 x 8/4, 500 kept 25.2 / 21.5, 2 x 1024 x 8/4, all kept 31.1 / 26.1, 7000 x 2/1, 3000 kept 48.4 / 43.9;
+// d = 96 2000 x 8/4, 128 kept 22.0 / 20.1; d = 64 2 x 3000 x 2/1, 900 kept 25.5 / 21.7.  Above head dim 128 not with 64-row blocks, whose
+// registers it spills (1000 x 8/4, 300 kept 36.7 / 37.3).
+bool fwd_from_lists(const FwdParams &p) {
+    if (!p.kept_idx || !p.mask || p.cmp.on || p.cu_q || p.kv_share > 1 || !use_compact(p) || !fwd_colmask_applicable(p) || fwd_stream_applicable(p)) return false;
+    const int64_t r = p.k_r > p.v_r ? p.k_r : p.v_r;  // (row offsets are 32-bit numbers)
+    return (p.d > 128 ? fwd_blocks64(p) > device_cus() : takes_key_groups(p)) && key_shares(p) == 1 && p.k_r >= 0 && p.v_r >= 0 && (p.Lk * r + p.d) * 2 < (int64_t)1 << 32;
+}
+
 int64_t fwd_share_units(const FwdParams &p) {
     FwdParams pr = p;
     return row_grid(pr, fwd_share_block(p));

@@ -65,13 +65,15 @@ template <int D_, int RG> struct Cfg {
 };
 
 // DC: the head dims that are worked on, 96 of a 128-wide tile for head dims 65 to 96 (the merge takes the others along as zeros).
-template <typename T, int D, int DC, int RG, bool CAUSAL, bool CMP>
+// LIST (with CMP): the keys are those of a handed-over list, and K, V and bias are read where they lie (see fwd_from_lists).
+template <typename T, int D, int DC, int RG, bool CAUSAL, bool CMP, bool LIST>
 __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
     using E = Elem<T>;
     using C = Cfg<D, RG>;
     constexpr int KG = C::KG, BM = C::BM, BN = C::BN, ROW = C::ROW, TILE = C::TILE, NP = C::NP, KS = DC / 16, DB = DC / 32;
     constexpr int OFF_V = C::OFF_V, OFF_COL = C::OFF_COL, OFF_BITS = C::OFF_BITS, UPW = C::UPW, UPP = C::UPP;
-    constexpr bool ONE = C::ONE, SHARES = CMP && D <= 128;  // (key_shares cuts nothing above)
+    static_assert(CMP || !LIST, "a list's keys are counted like compacted ones");
+    constexpr bool ONE = C::ONE, SHARES = CMP && !LIST && D <= 128;  // (key_shares cuts nothing above)
     extern __shared__ __attribute__((aligned(256))) char smem[];
     const uint32_t lds0 = lds_addr(smem);  // (a multiple of 256)
     uint32_t *sBits = (uint32_t *)(smem + OFF_BITS);
@@ -93,9 +95,17 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
     // `lane % CH` of its row, which holds chunk position ^ chunk_swz(row) of the global row; rows 16 apart have the same swizzle.  Rows
     // beyond the keys (queries) are clamped to the last one (their column says -inf; they are not stored), chunks beyond d to chunk 0 (they
     // meet zero Q and columns of O that are not stored).
-    const int prow = C::RPP * wave + lane / C::CH;
+    int prow = C::RPP * wave + lane / C::CH;
     const int pchunk = lane % C::CH ^ (int)chunk_swz<D>(prow);
     const uint32_t pcol = pchunk * 8 < p.d ? pchunk * 16 : 0;
+
+    // LIST: original columns of the keys of two tiles, the parity of a tile deciding where, held inside [0, Lk) (lists are device data the host
+    // cannot check); those of the first tile are requested here and published with Q
+    const int lrow = LIST ? (p.m_b == 0 ? 0 : b) * p.Hm + (p.Hm == 1 ? 0 : hk) : 0;
+    const int32_t *list = LIST ? p.kept_idx + (int64_t)lrow * p.kept_ld : nullptr;
+    auto column_at = [&](int c) { return list[c < LkS ? c : LkS - 1]; };
+    const uint32_t idx_off = lds0 + OFF_BITS;
+    int32_t list_raw = LIST ? column_at(tid) : 0;
 
     // ---- Q, requested first of all: through LDS, where the second stage of K (and of V) comes later, or V where there is one stage.
     // As fragments straight from memory every load of a wave touches 32 rows, one cache line after another (2.7 clocks each), and every key
@@ -122,9 +132,10 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
     const uint16_t *vbase = (const uint16_t *)p.v + b * p.v_b + sq.k0 * p.v_r + hk * p.v_h;
 
     // key columns this workgroup iterates over, and the number of them a query row may see
-    const int Lk = CMP ? p.cmp.count[b * p.Hk + hk] : LkS;
-    const int32_t *ccnt = CMP ? p.cmp.cnt + (int64_t)(b * p.Hk + hk) * p.cmp.ld : nullptr;
-    const float *fbrow = CMP ? p.cmp.fb + (int64_t)(b * p.cmp.Hfb + (p.cmp.Hfb == p.H ? h : hk)) * p.cmp.ld : nullptr;
+    int Lk = LIST ? p.kept_count[lrow] : CMP ? p.cmp.count[b * p.Hk + hk] : LkS;
+    if (LIST) Lk = Lk < 0 ? 0 : (Lk < LkS ? Lk : LkS);
+    const int32_t *ccnt = LIST ? p.kept_cnt + (int64_t)lrow * p.kept_ld : CMP ? p.cmp.cnt + (int64_t)(b * p.Hk + hk) * p.cmp.ld : nullptr;
+    const float *fbrow = CMP && !LIST ? p.cmp.fb + (int64_t)(b * p.cmp.Hfb + (p.cmp.Hfb == p.H ? h : hk)) * p.cmp.ld : nullptr;
     const int vis_lane = CAUSAL ? visible_columns<CMP>(qrow, LqS, LkS, ccnt) : 0;  // columns below it pass the causal test for this lane's row
     const int vis_wave = CAUSAL ? visible_columns<CMP>(wrow0, LqS, LkS, ccnt) : 0;
     const int vis_block = CAUSAL ? visible_columns<CMP>(m0 + BM - 1, LqS, LkS, ccnt) : 0;
@@ -175,7 +186,12 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
             sBits[w0 + 1] = (uint32_t)(ball >> 32);
         }
     }
+    auto keep_column = [&](int tile) {
+        const uint32_t c = (uint32_t)list_raw, last = (uint32_t)LkS - 1;
+        lds_st32(idx_off + (uint32_t)((tile & 1) * BN + tid) * 4, c < last ? c : last);
+    };
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (Q, which the barrier publishes)
+    if (LIST && tid < BN) keep_column(0);
     __syncthreads();
     auto next_active = [&](int j) -> int {  // wave-uniform
         if (CMP) return j < n_end ? j : n_end;
@@ -194,12 +210,13 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
     const uint32_t k_r2 = (uint32_t)(p.k_r * 2), v_r2 = (uint32_t)(p.v_r * 2);
     uint32_t k_row = prow * k_r2, v_row = prow * v_r2;  // (offsets grow with the row: clamped by the last row's)
     gptr_t tb_k = nullptr, tb_v = nullptr;
-    int t_rows = 0, t_stage = 0;     // last row of the tile being fetched, its stage
+    int t_rows = 0, t_stage = 0, t_tile = 0;  // last row of the tile being fetched, its stage, the tile
     uint32_t braw = 0, mraw = 0;     // first waves: raw bias and mask of key `tid` of that tile
     bool col_ok = false;
     auto set_tile = [&](int j, int stage) {
-        tb_k = uniform_ptr(kbase + (int64_t)j * BN * p.k_r);
-        tb_v = uniform_ptr(vbase + (int64_t)j * BN * p.v_r);
+        tb_k = uniform_ptr(kbase + (LIST ? 0 : (int64_t)j * BN * p.k_r));
+        tb_v = uniform_ptr(vbase + (LIST ? 0 : (int64_t)j * BN * p.v_r));
+        t_tile = j;
         const int left = Lk - 1 - j * BN;
         t_rows = left < BN - 1 ? left : BN - 1;
         t_stage = stage;
@@ -207,7 +224,10 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
             const int col = j * BN + tid;
             col_ok = col < Lk;
             const int cc = col_ok ? col : 0;
-            if (CMP) {
+            if (LIST) {
+                braw = (brow ? brow : kbase)[brow ? lds_ld32(idx_off + (uint32_t)((j & 1) * BN + tid) * 4) : 0];
+                list_raw = column_at(col + BN);
+            } else if (CMP) {
                 braw = __float_as_uint(fbrow[cc]);
             } else {
                 mraw = (mrow ? mrow : (const uint8_t *)kbase)[mrow ? cc : 0];
@@ -218,8 +238,15 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
     // (in assembly and waited for by hand: behind the compiler's builtin every LDS read waits for all LDS operations in flight)
     auto dma_piece = [&](int n) {  // NP pieces of K, NP of V
         const int i = n % NP;
-        const uint32_t r2 = n < NP ? k_r2 : v_r2, at = (n < NP ? k_row : v_row) + 8 * C::RPP * i * r2, last = (uint32_t)t_rows * r2;
-        const uint32_t off = (at < last ? at : last) + pcol;
+        const uint32_t r2 = n < NP ? k_r2 : v_r2;
+        uint32_t off;
+        if constexpr (LIST) {  // (rows beyond the last kept key: it again)
+            const int row = prow + 8 * C::RPP * i;
+            off = lds_ld32(idx_off + (uint32_t)((t_tile & 1) * BN + (row < t_rows ? row : t_rows)) * 4) * r2 + pcol;
+        } else {
+            const uint32_t at = (n < NP ? k_row : v_row) + 8 * C::RPP * i * r2, last = (uint32_t)t_rows * r2;
+            off = (at < last ? at : last) + pcol;
+        }
         const uint32_t dst = lds0 + (n < NP ? 0 : OFF_V) + (uint32_t)((ONE ? 0 : t_stage * TILE) + (wave + 8 * i) * 1024);
         load_lds16(off, n < NP ? tb_k : tb_v, __builtin_amdgcn_readfirstlane(dst));
     };
@@ -228,7 +255,10 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
         if (wave < BN / 64) {
             float v = 0.f;
             bool keep = col_ok;
-            if (CMP) {
+            if (LIST) {
+                if (brow) v = E::lo(braw) * kLog2e;
+                keep_column(t_tile + 1);
+            } else if (CMP) {
                 v = __uint_as_float(braw);
             } else {
                 keep = keep && (!mrow || mraw);
@@ -282,7 +312,8 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
     auto one_tile = [&](auto st_c) {
         constexpr int st = decltype(st_c)::value;
         // (the swizzled addresses are these constants XOR a compile-time value, recomputed where used)
-        asm volatile("" : "+v"(a_off), "+v"(tr_off), "+v"(k_row), "+v"(v_row));
+        if constexpr (LIST) asm volatile("" : "+v"(a_off), "+v"(tr_off), "+v"(prow));
+        else asm volatile("" : "+v"(a_off), "+v"(tr_off), "+v"(k_row), "+v"(v_row));
         const int n0 = jc * BN + 32 * kg;
         set_tile(jn < n_end ? jn : jc, st ^ 1);  // (past the last tile it is fetched again and dropped)
         __builtin_amdgcn_sched_barrier(0);
@@ -512,11 +543,15 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
 
 template <typename T, int D, int RG, bool CAUSAL, bool CMP>
 __global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_wide_kernel(const FwdParams p) {
-    fwd_wide<T, D, D, RG, CAUSAL, CMP>(p);
+    fwd_wide<T, D, D, RG, CAUSAL, CMP, false>(p);
 }
 template <typename T, bool CAUSAL, bool CMP>
 __global__ void __launch_bounds__(NT, 2) fwd_96_kernel(const FwdParams p) {
-    fwd_wide<T, 128, 96, 2, CAUSAL, CMP>(p);
+    fwd_wide<T, 128, 96, 2, CAUSAL, CMP, false>(p);
+}
+template <typename T, int D, int DC, int RG, bool CAUSAL>
+__global__ void __launch_bounds__(NT, D == 64 ? 4 : 2) fwd_list_kernel(const FwdParams p) {
+    fwd_wide<T, D, DC, RG, CAUSAL, true, true>(p);
 }
 
 template <typename T, int D, int RG, bool CAUSAL, bool CMP>
@@ -536,6 +571,23 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     return hipGetLastError();
 }
 
+template <typename T, int D, int DC, int RG> hipError_t launch_list(const FwdParams &p, hipStream_t stream) {
+    auto kern = p.causal ? fwd_list_kernel<T, D, DC, RG, true> : fwd_list_kernel<T, D, DC, RG, false>;
+    static DynSmemLimit smem_limit[2];  // one per instantiation
+    using C = Cfg<D, RG>;
+    hipError_t e = smem_limit[p.causal != 0].ensure((const void *)kern, C::SMEM);
+    if (e != hipSuccess) return e;
+    FwdParams pr = p;
+    const int grid = row_grid(pr, C::BM);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), C::SMEM, stream, pr);
+    return hipGetLastError();
+}
+template <typename T> hipError_t launch_lists(const FwdParams &p, hipStream_t stream) {
+    if (p.d > 128) return launch_list<T, 256, 256, 4>(p, stream);
+    if (p.d > 96) return launch_list<T, 128, 128, 2>(p, stream);
+    return p.d > 64 ? launch_list<T, 128, 96, 2>(p, stream) : launch_list<T, 64, 64, 2>(p, stream);
+}
+
 template <typename T, int D, int RG> hipError_t launch_t(const FwdParams &p, hipStream_t stream) {
     if (p.cmp.on) return p.causal ? launch_one<T, D, RG, true, true>(p, stream) : launch_one<T, D, RG, false, true>(p, stream);
     return p.causal ? launch_one<T, D, RG, true, false>(p, stream) : launch_one<T, D, RG, false, false>(p, stream);
@@ -548,6 +600,7 @@ template <typename T, int D, int RG> hipError_t launch_t(const FwdParams &p, hip
 // against 2000 kept of 8000 63.8 / 54.8; 1500 x 8, all kept 62.2 / 55.2; 2 x 700 x 4 27.7 / 24.6; 1024 x 2 23.8 / 23.9; beyond a block per
 // CU 3001 x 8 (376 blocks) 45.6 / 51.1, 2000 x 16 (512) 34.4 / 45.7.
 hipError_t launch_fwd_wide(const FwdParams &p, int dtype, hipStream_t stream) {
+    if (fwd_from_lists(p)) return dtype == 0 ? launch_lists<bf16_tag>(p, stream) : launch_lists<fp16_tag>(p, stream);
     if (p.d > 128 && fwd_blocks64(p) <= device_cus()) return dtype == 0 ? launch_t<bf16_tag, 256, 2>(p, stream) : launch_t<fp16_tag, 256, 2>(p, stream);
     if (p.d > 128) return dtype == 0 ? launch_t<bf16_tag, 256, 4>(p, stream) : launch_t<fp16_tag, 256, 4>(p, stream);
     if (p.d > 64) return dtype == 0 ? launch_t<bf16_tag, 128, 2>(p, stream) : launch_t<fp16_tag, 128, 2>(p, stream);

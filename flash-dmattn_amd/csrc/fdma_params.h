@@ -421,6 +421,7 @@ struct DynSmemLimit {
 hipError_t launch_fwd(const FwdParams &p, int dtype, hipStream_t stream);
 // column-mask specialisation (mask / bias absent or broadcast over queries); nq = 32-row blocks per wave
 bool fwd_colmask_applicable(const FwdParams &p);
+bool fwd_from_lists(const FwdParams &p);
 hipError_t launch_fwd_colmask(const FwdParams &p, int dtype, hipStream_t stream);
 hipError_t launch_fwd_wide(const FwdParams &p, int dtype, hipStream_t stream);  // head dims 129 .. 256 (fdma_fwd_wide.hip)
 int64_t fwd_blocks64(const FwdParams &p);  // 64-row blocks of all heads (ragged batches: at most)

@@ -45,6 +45,7 @@ struct Api {
     decltype(&::fdma_fwd) fwd;
     decltype(&::fdma_bwd) bwd;
     decltype(&::fdma_fwd_workspace_bytes) fwd_workspace_bytes;
+    decltype(&::fdma_fwd_takes_lists) fwd_takes_lists;
     decltype(&::fdma_fwd_optional_bytes) fwd_optional_bytes;
     decltype(&::fdma_bwd_workspace_bytes) bwd_workspace_bytes;
     decltype(&::fdma_bwd_optional_bytes) bwd_optional_bytes;
@@ -366,7 +367,8 @@ PyObject *attention(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     // LSE and workspace in one piece -- except where a backward will want the LSE and there is no workspace to go with it, or
     // saved-tensor hooks are waiting (they may move it off the device until then): it is a tensor of its own there, which the
     // node saves as autograd does
-    const size_t need = api.fwd_workspace_bytes(&a);
+    // (without a backward nobody else wants the compacted copies)
+    const size_t need = !is_grad && side.idx.defined() && api.fwd_takes_lists(&a) ? 0 : api.fwd_workspace_bytes(&a);
     const bool apart = is_grad && (need == 0 || Lq == 1 || !at::SavedTensorDefaultHooks::get_tls_state().stack.empty());
     const size_t lse_bytes = apart ? 0 : up256((size_t)B * H * Lq * 4);
     Tensor lse, buf;
@@ -721,6 +723,7 @@ PyObject *bind(PyObject *, PyObject *dict) {
     FDMA_BIND(fwd);
     FDMA_BIND(bwd);
     FDMA_BIND(fwd_workspace_bytes);
+    FDMA_BIND(fwd_takes_lists);
     FDMA_BIND(fwd_optional_bytes);
     FDMA_BIND(bwd_workspace_bytes);
     FDMA_BIND(bwd_optional_bytes);

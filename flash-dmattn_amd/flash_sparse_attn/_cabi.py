@@ -124,7 +124,7 @@ class DynBiasArgs(ctypes.Structure):
 
 
 EXPORTS = (
-    "fdma_fwd", "fdma_fwd_noalloc", "fdma_bwd", "fdma_fwd_workspace_bytes", "fdma_fwd_counter_bytes", "fdma_bwd_workspace_bytes",
+    "fdma_fwd", "fdma_fwd_noalloc", "fdma_bwd", "fdma_fwd_workspace_bytes", "fdma_fwd_takes_lists", "fdma_fwd_counter_bytes", "fdma_bwd_workspace_bytes",
     "fdma_fwd_optional_bytes", "fdma_bwd_optional_bytes", "fdma_varlen_bwd_ws", "fdma_varlen_bwd_optional_bytes",
     "fdma_set_stream_min_items",
     "fdma_fwd_validate", "fdma_bwd_validate", "fdma_last_error", "fdma_abi_version",
@@ -203,6 +203,8 @@ def _load() -> ctypes.CDLL:
     lib.fdma_fwd_workspace_bytes.restype = ctypes.c_size_t
     lib.fdma_fwd_optional_bytes.argtypes = [ctypes.POINTER(FwdArgs)]
     lib.fdma_fwd_optional_bytes.restype = ctypes.c_size_t
+    lib.fdma_fwd_takes_lists.argtypes = [ctypes.POINTER(FwdArgs)]
+    lib.fdma_fwd_takes_lists.restype = ctypes.c_int
     lib.fdma_fwd_counter_bytes.argtypes = [ctypes.POINTER(FwdArgs)]
     lib.fdma_fwd_counter_bytes.restype = ctypes.c_size_t
     lib.fdma_set_stream_min_items.argtypes = [ctypes.c_int]
@@ -258,7 +260,7 @@ lib = _load()
 
 _HOST_PATH = os.path.normpath(os.path.join(_HERE, "..", "lib", "_fdma_torch.so"))
 _HOST_CALLS = (
-    "fdma_fwd", "fdma_bwd", "fdma_fwd_workspace_bytes", "fdma_fwd_optional_bytes", "fdma_bwd_workspace_bytes", "fdma_bwd_optional_bytes", "fdma_fwd_counter_bytes",
+    "fdma_fwd", "fdma_bwd", "fdma_fwd_workspace_bytes", "fdma_fwd_takes_lists", "fdma_fwd_optional_bytes", "fdma_bwd_workspace_bytes", "fdma_bwd_optional_bytes", "fdma_fwd_counter_bytes",
     "fdma_set_stream_min_items", "fdma_varlen_fwd", "fdma_varlen_bwd_ws", "fdma_varlen_bwd_optional_bytes", "fdma_create_mask", "fdma_dyn_bias_fwd",
     "fdma_dyn_bias_bwd", "fdma_dyn_bias_bwd_workspace_bytes", "fdma_last_error",
 )

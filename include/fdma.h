@@ -213,6 +213,9 @@ int fdma_set_stream_min_items(int n);
 /* Scratch the caller must provide.  0 when none is needed.  Validate nothing but shapes.  Ask with the arguments of the call itself:
  * which tensors there are counts too (a decode call without a mask keeps every key and can take more splits than one with). */
 size_t fdma_fwd_workspace_bytes(const fdma_fwd_args *args);
+/* Whether a forward call with handed-over lists (args->kept) can do without that scratch: 1: with workspace NULL it reads the kept rows
+ * where they lie, with the same bits as results.  (A backward makes the compacted copies itself then.)  0: it cannot. */
+int fdma_fwd_takes_lists(const fdma_fwd_args *args);
 /* Scratch that a forward call with a mask or bias per query can use (0: none): with workspace_bytes of at least this many the keys of
  * few query rows are cut into shares, whose fp32 results lie there; with less they stay whole.  Nothing of it outlives the call. */
 size_t fdma_fwd_optional_bytes(const fdma_fwd_args *args);

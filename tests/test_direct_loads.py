@@ -74,10 +74,10 @@ def test_no_direct_load_in_flight_at_the_merge_of_key_groups(tmp_path):
 
 
 def test_nor_at_that_of_their_variants(tmp_path):
-    """The same kernels for head dims 65 to 96."""
+    """The same kernels for head dims 65 to 96, and those that read a list's rows where they lie."""
     text = _assembly("fdma_fwd_wide", tmp_path)
-    kernels = re.findall(r"^(_Z\S*fwd_96_kernel\S*):.*?\n(.*?)^\.Lfunc_end", text, re.M | re.S)
-    assert len(kernels) == 8
+    kernels = re.findall(r"^(_Z\S*(?:fwd_96|fwd_list)_kernel\S*):.*?\n(.*?)^\.Lfunc_end", text, re.M | re.S)
+    assert len(kernels) == 8 + 16
     for name, body in kernels:
         loads, early = _early_stores(body)
         assert loads > 0 and "ds_write_b128" in body, name
