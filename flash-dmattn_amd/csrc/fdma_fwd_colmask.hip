@@ -903,10 +903,16 @@ static bool takes_key_groups(const FwdParams &p) {
 // x 8/4, all kept 321 / 319; d = 128: 2000 x 8/4, 500 kept 25.2 / 21.5, 2 x 1024 x 8/4, all kept 31.1 / 26.1, 7000 x 2/1, 3000 kept 48.4 / 43.9;
 // d = 96 2000 x 8/4, 128 kept 22.0 / 20.1; d = 64 2 x 3000 x 2/1, 900 kept 25.5 / 21.7.  Above head dim 128 not with 64-row blocks, whose
 // registers it spills (1000 x 8/4, 300 kept 36.7 / 37.3).
+// Causal calls up to two blocks of 64 rows per CU, three at head dims up to 64, beyond what takes_key_groups gives the kernel where it reads copies.  96 / 500 / all
+// kept: d = 128 2048 x 16/8 (512 blocks) 28.4 / 25.6, 33.8 / 30.5, 55.2 / 45.2; d = 96 4000 x 8/4 (504) 25.4 / 23.6, 29.4 / 27.4, 69.1 / 58.6;
+// d = 64 3072 x 16/8 (768) 25.2 / 22.1, 29.0 / 25.2, 64.8 / 49.2; 30 layers near the lines 1.12 times, none slower.  Beyond: d = 128 1500 x 32/16 (768),
+// 128, 512, 1400 kept 30.9 / 33.6, 38.8 / 41.2, 57.9 / 55.6, d = 64 4096 x 16/8 (1024) 24.8 / 25.7, 29.1 / 29.5, 42.4 / 37.9.
 bool fwd_from_lists(const FwdParams &p) {
     if (!p.kept_idx || !p.mask || p.cmp.on || p.cu_q || p.kv_share > 1 || !use_compact(p) || !fwd_colmask_applicable(p) || fwd_stream_applicable(p)) return false;
     const int64_t r = p.k_r > p.v_r ? p.k_r : p.v_r;  // (row offsets are 32-bit numbers)
-    return (p.d > 128 ? fwd_blocks64(p) > device_cus() : takes_key_groups(p)) && key_shares(p) == 1 && p.k_r >= 0 && p.v_r >= 0 && (p.Lk * r + p.d) * 2 < (int64_t)1 << 32;
+    const int64_t blocks64 = fwd_blocks64(p), cus = device_cus();
+    const bool grid_ok = p.d > 128 ? blocks64 > cus : takes_key_groups(p) || (p.causal && p.Lk > 128 && blocks64 <= (p.d > 64 ? 2 : 3) * cus);
+    return grid_ok && key_shares(p) == 1 && p.k_r >= 0 && p.v_r >= 0 && (p.Lk * r + p.d) * 2 < (int64_t)1 << 32;
 }
 
 int64_t fwd_share_units(const FwdParams &p) {
@@ -919,7 +925,7 @@ hipError_t launch_fwd_colmask(const FwdParams &p, int dtype, hipStream_t stream)
     if (p.cmp.on && p.cmp.img_kv) return launch_fwd_stream(p, dtype, stream);  // (the pre-pass has written tile images)
     // head dims up to 64 / 128 (a head dim in between runs in the next larger instantiation), above in a kernel of their own
     if (p.d > 128) return launch_fwd_wide(p, dtype, stream);
-    if (takes_key_groups(p)) {  // (and all calls in shares: three shares are at most a third of a 64-row block per CU, see key_shares)
+    if (fwd_from_lists(p) || takes_key_groups(p)) {  // (and all calls in shares: three shares are at most a third of a 64-row block per CU, see key_shares)
         const hipError_t e = launch_fwd_wide(p, dtype, stream);
         if (e != hipSuccess || !p.cmp.on || p.splits <= 1 || p.dec_counter) return e;
         return launch_fwd_merge(p, dtype, stream);

@@ -5,7 +5,7 @@ import torch
 
 from flash_sparse_attn import flash_sparse_attn_func
 from flash_sparse_attn.utils import mask as M
-from _util import set_compact
+from _util import rel_err, set_compact
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -18,6 +18,9 @@ DEV = "cuda"
     (3, 200, 501, 2, 1, 96, 1, 1, True, torch.bfloat16),    # rows of an odd length
     (1, 515, 515, 8, 8, 64, 8, 8, True, torch.float16),
     (2, 130, 700, 2, 2, 40, 2, 0, False, torch.bfloat16),   # no bias
+    (1, 1900, 1900, 16, 8, 128, 8, 8, True, torch.bfloat16),  # 480 blocks of 64 rows: copies go to another kernel, see below
+    (1, 1500, 1500, 16, 8, 72, 8, 8, True, torch.float16),
+    (2, 1500, 1500, 16, 8, 64, 8, 8, True, torch.bfloat16),
     (5, 512, 512, 8, 4, 256, 4, 4, True, torch.bfloat16),   # 128-row blocks
     (4, 700, 500, 8, 2, 200, 2, 1, True, torch.float16),    # ... rows that see nothing
 ])
@@ -42,6 +45,10 @@ def test_same_bits(B, Lq, Lk, H, Hk, d, mask_heads, bias_heads, causal, dtype, k
             peak = torch.cuda.max_memory_allocated() - before
     finally:
         set_compact("auto")
-    assert torch.isfinite(direct.float()).all() and torch.equal(direct, copied)
+    assert torch.isfinite(direct.float()).all()
+    if B * H * -(-Lq // 64) <= 256 or d > 128:
+        assert torch.equal(direct, copied)
+    else:  # (another order of summation: P rounded to 16 bits against another reference point, both results rounded once)
+        assert rel_err(direct, copied) <= 2.0 * torch.finfo(dtype).eps
     # the output and the row statistics, in blocks of 512 bytes, and a mask or bias brought to whole chunks; no copies of K and V
     assert peak < direct.numel() * 2 + B * H * Lq * 4 + 4 * 1024 + (mask.numel() + (bias.numel() if bias_heads else 0)) * 8
