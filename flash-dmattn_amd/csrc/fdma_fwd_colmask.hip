@@ -889,10 +889,16 @@ bool fwd_colmask_applicable(const FwdParams &p) {
 //     either way).
 //   * d <= 64, two to a CU: up to two and a half blocks per CU 1.25 to 1.65 times over 11 calls; 768 blocks (2 x 1500 x 16 heads, 700
 //     kept) 29.3 against 27.8 us, ragged 4000 to 1000 x 16 140 against 125.
+// Causal ragged batches further, up to two blocks per CU, three at d <= 64, where one entry of 1024 rows or more has half of them all: the call
+// takes what the last blocks of that entry take.  128-row blocks / these, us: 2000, 100, 700, 30 x 8/4 heads, d = 128 45.5 / 27.7 (forward + backward
+// 146 / 129), 3000, 1000 x 8/4 58.6 / 42.1, 4000, 4000 x 4/2 60.7 / 55.6; d = 96 5000, 50, 60 x 4/2 89 / 51; d = 64 1500, 1500 x 16/4 29.7 / 26.3.
+// Entries of one length keep the line: four of 1024 x 8/8, d = 128 25.2 / 26.2, three of 1100 24.7 / 26.9, not causal or compacted calls as well
+// (2600 x 8/2, d = 128, causal, 96 / 500 / all kept 15.9 / 17.6, 21.3 / 19.7, 48.8 / 39.4, not causal 15.0 / 17.2, 20.9 / 24.5, 51.0 / 66.2).
 // (A ragged batch has at most total / 64 blocks per head and one more per entry.)
 int64_t fwd_blocks64(const FwdParams &p) { return p.cu_q ? (int64_t)p.H * (p.total_q / 64 + p.B) : (int64_t)p.B * p.H * ((p.Lq + 63) / 64); }
 static bool takes_key_groups(const FwdParams &p) {
     const int64_t blocks64 = fwd_blocks64(p);
+    if (p.cu_q && p.causal && p.Lq >= 1024 && 2 * (int64_t)p.Lq >= p.total_q && blocks64 <= (p.d > 64 ? 2 : 3) * device_cus()) return true;
     if (p.d > 64) return blocks64 <= device_cus() && p.Lk > 128;
     return 2 * blocks64 <= 5 * (int64_t)device_cus();
 }

@@ -74,6 +74,9 @@ def test_climbing_scores_and_empty_groups(D, mode):
     ([1, 200, 64, 65, 300], 4, 2, 128),
     ([1, 200, 64, 65, 300], 4, 2, 64),
     ([2500, 1800], 8, 4, 64),
+    ([1100, 300, 5, 790], 13, 13, 96),  # an entry of half of the rows: up to two blocks of 64 rows per CU (481 here) ...
+    ([7, 1300, 40], 32, 8, 64),         # ... or three (736)
+    ([1024, 1023], 14, 14, 128),        # (476)
 ])
 def test_ragged(lens, H, Hk, D):
     from flash_sparse_attn import flash_sparse_attn_varlen_func
