@@ -474,7 +474,12 @@ template <typename T> __global__ void __launch_bounds__(256) bwd_dq_sum_kernel(c
 template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD, bool SHARES = false>
 hipError_t launch_dq_o(const BwdParams &p, hipStream_t stream) {
     constexpr int BM = 32 * NW / KSPLIT / GH, NTHREADS = 64 * NW, BN = ((NW == 8 && KSPLIT == 1) || D > 128) ? 32 : 64;
-    if constexpr (!SHARES && (KSPLIT == 2 || NW == 4)) if (p.dq_shares > 1) return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, GH, ODD, true>(p, stream);
+    if constexpr (!SHARES) {
+        if (p.dq_shares > 1) {
+            if constexpr (KSPLIT == 2 || NW == 4) return launch_dq_o<T, D, CAUSAL, NW, KSPLIT, GH, ODD, true>(p, stream);
+            else return hipErrorInvalidValue;  // (general_key_shares plans none for the kernels of 256 rows)
+        }
+    }
     auto kern = bwd_dq_kernel<T, D, CAUSAL, NW, KSPLIT, GH, ODD, SHARES>;
     constexpr int merge = KSPLIT == 2 ? (NW / 2) * (D / 32) * 4096 : 0;  // the upper halves' sums
     constexpr int smem = DqSmem<D, BM, BN>::TOTAL > merge ? DqSmem<D, BM, BN>::TOTAL : merge;
@@ -482,7 +487,7 @@ hipError_t launch_dq_o(const BwdParams &p, hipStream_t stream) {
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
     dim3 grid(((p.f.Lq + BM - 1) / BM) * (p.f.H / GH) * p.f.B);
-    grid.y = p.dq_shares;
+    if constexpr (SHARES) grid.y = p.dq_shares;
     hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
     return hipGetLastError();
 }
@@ -505,8 +510,7 @@ hipError_t launch_dq_n(const BwdParams &p, hipStream_t stream) {
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_dq_c(const BwdParams &p, hipStream_t stream) {
     if constexpr (D > 64 && D <= 128) {
-        // 256-row workgroups while the grid still covers the chip about twice
-        if ((int64_t)p.f.B * p.f.H * ((p.f.Lq + 255) / 256) >= 512) return launch_dq_n<T, D, CAUSAL, 8>(p, stream);
+        if (general_rows_256(p.f)) return launch_dq_n<T, D, CAUSAL, 8>(p, stream);
         return launch_dq_n<T, D, CAUSAL, 8, 2>(p, stream);
     } else {
         return launch_dq_n<T, D, CAUSAL, 4>(p, stream);

@@ -620,8 +620,7 @@ hipError_t launch_fwd_c(const FwdParams &p, hipStream_t stream) {
 template <typename T, int D>
 hipError_t launch_fwd_t(const FwdParams &p, hipStream_t stream) {
     if constexpr (D > 64 && D <= 128) {
-        // 256-row workgroups while the grid still covers the chip about twice
-        if ((int64_t)p.B * p.H * ((p.Lq + 255) / 256) >= 512)
+        if (general_rows_256(p))
             return p.causal ? launch_fwd_c<T, D, true, 8>(p, stream) : launch_fwd_c<T, D, false, 8>(p, stream);
         return p.causal ? launch_fwd_c<T, D, true, 8, 2>(p, stream) : launch_fwd_c<T, D, false, 8, 2>(p, stream);
     } else {
@@ -641,6 +640,9 @@ int shared_rows(const FwdParams &p) {
     return p.d > 64 && G % 2 == 0 ? 2 : 1;
 }
 
+// At head dims 65 to 128, forward and dQ: 256-row workgroups while the grid still covers the chip about twice
+bool general_rows_256(const FwdParams &p) { return p.d > 64 && p.d <= 128 && (int64_t)p.B * p.H * ((p.Lq + 255) / 256) >= 512; }
+
 int64_t general_share_units(const FwdParams &p) {
     const int gh = shared_rows(p), rows = 128 / gh;
     return (int64_t)((p.Lq + rows - 1) / rows) * (p.H / gh) * p.B;
@@ -656,6 +658,7 @@ int64_t general_share_units(const FwdParams &p) {
 //     x 16/8 125 / 130 with the backward, 256 x 2/1 24.5 / 21.4).
 //   * dQ from 24 tiles on (16 of 32 keys): below, a backward is bound by its launches, of which this is one more (1024 x 2/1,
 //     d = 128: 66.9 and 69 to 72).
+//   * None of a dQ that the kernels of 256 rows take: they work on whole keys.
 // (Up to head dim 128 the last workgroup of the rows adds the forward's shares up; a launch of its own: 3883 x 8/2, d = 64 66.7 / 55.9, 2 x 1198 x
 // 8/4, d = 64 30.6 / 26.9, 2 x 1039 x 8/2 24.5 / 21.0.)
 // Whole / shares, us (forward; backward with its other kernels): 2316 x 2/1 heads, d = 256 162 / 46, 323 / 180; 3000 x 2/1, d = 64 83 / 25,
@@ -664,7 +667,7 @@ int64_t general_share_units(const FwdParams &p) {
 int general_key_shares(const FwdParams &p, bool dq) {
     if (p.cu_q || p.Lq < 1 || p.Lk < 1) return 1;
     const int gh = shared_rows(p), tile = p.d > 128 ? 32 : 64, tiles = (p.Lk + tile - 1) / tile;
-    if (dq && tiles < (p.d > 128 ? 16 : 24)) return 1;
+    if (dq && (tiles < (p.d > 128 ? 16 : 24) || general_rows_256(p))) return 1;
     const int64_t blocks = general_share_units(p);
     int64_t s = blocks > 0 ? device_cus() * (p.d > 64 ? 1 : (gh == 4 ? 3 : 2)) / blocks : 1;
     if (s > tiles / 4) s = tiles / 4;

@@ -471,6 +471,7 @@ bool bwd_dkdv_64_applicable(const BwdParams &p);  // general form, head dims up 
 hipError_t launch_bwd_dkdv_64(const BwdParams &p, int dtype, hipStream_t stream);
 // general forward and dQ kernels: query heads to a workgroup (fdma_fwd.hip)
 int shared_rows(const FwdParams &p);
+bool general_rows_256(const FwdParams &p);  // whether those of 256 rows take the call, which do not work on shares of the keys
 // general dQ kernel (mask / bias per query row), fdma_bwd_dq.hip
 hipError_t launch_bwd_dq(const BwdParams &p, int dtype, hipStream_t stream);
 

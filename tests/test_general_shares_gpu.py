@@ -23,6 +23,21 @@ CASES = [
 ]
 
 
+def _many_heads(B, Lq, Lk, H, Hk, d, bias_heads):
+    g = torch.Generator().manual_seed(Lq + Lk + d)
+    r = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    mask = (torch.rand(B, Hk, Lq, Lk, generator=g) < 0.3).to(DEV)
+    mask[:, :, Lq // 2, Lk // 3:] = False  # (a row that keeps nothing of the last share)
+    return r(B, Lq, H, d), r(B, Lk, Hk, d), r(B, Lk, Hk, d), r(B, Lq, H, d), mask, r(B, bias_heads, Lq, Lk) if bias_heads else None
+
+
+def _not_a_number_everywhere():
+    """Memory that the allocator hands out next holds NaN."""
+    held = [torch.full((n << 18,), float("nan"), device=DEV) for n in (1, 4, 16, 64, 256) for _ in range(4)]
+    torch.cuda.synchronize()
+    del held
+
+
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x) for x in c))
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_shares_vs_oracle_and_whole(case, dtype, monkeypatch):
@@ -77,6 +92,39 @@ def test_shares_vs_oracle_and_whole(case, dtype, monkeypatch):
         else:  # (a probability is rounded to eps / 2 of itself against either reference point; sums of many of them, and what LSE and O carry on)
             ok = (a.float() - b.float()).abs() <= eps * (2 * b.float().abs() + b.float().abs().max())
         assert ok.all(), i
+
+
+LINE = [
+    (16, 2, 1473, 32, 8, 96, 0),     # 512 blocks of 256 rows: whole keys, by the kernels that have no shares
+    (16, 16, 4096, 32, 8, 128, 0),
+    (16, 32, 1473, 32, 8, 128, 1),   # a bias that kv heads share: dQ is not made from dS
+    (32, 33, 1473, 16, 4, 96, 0),
+    (32, 32, 4096, 16, 4, 128, 1),
+    (15, 32, 1537, 32, 8, 128, 0),   # 480: two shares, four heads to a workgroup
+    (15, 16, 4096, 32, 8, 96, 1),
+    (15, 30, 1539, 32, 8, 72, 0),    # ... rows of an odd length
+    (2, 65, 1600, 8, 2, 128, 1),     # more shares; a row block of one row
+]
+
+
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,d,bias_heads", LINE)
+@pytest.mark.parametrize("native", [True, False])
+def test_gradients_where_the_kernel_changes(B, Lq, Lk, H, Hk, d, bias_heads, native, monkeypatch):
+    """Either side of the line at which kernels of 256 query rows take a call: the gradients do not hold what lay in the scratch before."""
+    from oracle import eager
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func
+
+    print("line", B, Lq, Lk, H, Hk, d, bias_heads, native, flush=True)
+    q, k, v, dout, mask, bias = _many_heads(B, Lq, Lk, H, Hk, d, bias_heads)
+    ref = eager.attention_forward_backward(q, k, v, mask, bias, None, True, dout)
+    if not native:
+        monkeypatch.setattr(_cabi, "host", _cabi._NoHost)
+    leaves = [t.requires_grad_(True) for t in (q, k, v) + ((bias,) if bias_heads else ())]
+    out = flash_sparse_attn_func(*leaves[:3], mask, leaves[3] if bias_heads else None, None, True)
+    _not_a_number_everywhere()
+    grads = torch.autograd.grad(out, leaves, dout)
+    for x, want, name in zip(grads, ref[1:], ("dq", "dk", "dv", "dbias")):
+        assert_grad_close(x, want, name)
 
 
 @pytest.mark.parametrize("B,Lq,Lk,H,Hk,d,kept", [
