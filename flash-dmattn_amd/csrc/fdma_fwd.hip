@@ -589,7 +589,12 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && NW == 4) ? 2 : 1) fwd_ker
 template <typename T, int D, bool CAUSAL, int NW, int KSPLIT, int GH, bool ODD, bool SHARES = false>
 hipError_t launch_fwd_o(const FwdParams &p, hipStream_t stream) {
     constexpr int BM = 32 * NW / KSPLIT / GH, NTHREADS = 64 * NW, BN = D > 128 ? 32 : BN_DEFAULT;
-    if constexpr (!SHARES && (KSPLIT == 2 || NW == 4)) if (p.splits > 1) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, GH, ODD, true>(p, stream);
+    if constexpr (!SHARES) {
+        if (p.splits > 1) {
+            if constexpr (KSPLIT == 2 || NW == 4) return launch_fwd_o<T, D, CAUSAL, NW, KSPLIT, GH, ODD, true>(p, stream);
+            else return hipErrorInvalidValue;  // (general_key_shares plans none for the kernels of 256 rows)
+        }
+    }
     auto kern = fwd_kernel<T, D, CAUSAL, NW, BN, KSPLIT, GH, ODD, SHARES>;
     constexpr int merge = KSPLIT == 2 ? (NW / 2) * 512 + (NW / 2) * (D / 32) * 4096 : 0;  // the upper halves' sums
     constexpr int smem = FwdSmem<D, BM, BN>::TOTAL > merge ? FwdSmem<D, BM, BN>::TOTAL : merge;
@@ -597,7 +602,7 @@ hipError_t launch_fwd_o(const FwdParams &p, hipStream_t stream) {
     hipError_t e = smem_limit.ensure((const void *)kern, (int)smem);
     if (e != hipSuccess) return e;
     dim3 grid(((p.Lq + BM - 1) / BM) * (p.H / GH) * p.B);
-    grid.y = p.splits;
+    if constexpr (SHARES) grid.y = p.splits;
     hipLaunchKernelGGL(kern, grid, dim3(NTHREADS), smem, stream, p);
     return hipGetLastError();
 }
@@ -658,7 +663,7 @@ int64_t general_share_units(const FwdParams &p) {
 //     x 16/8 125 / 130 with the backward, 256 x 2/1 24.5 / 21.4).
 //   * dQ from 24 tiles on (16 of 32 keys): below, a backward is bound by its launches, of which this is one more (1024 x 2/1,
 //     d = 128: 66.9 and 69 to 72).
-//   * None of a dQ that the kernels of 256 rows take: they work on whole keys.
+//   * None where the kernels of 256 rows take the call: they work on whole keys.
 // (Up to head dim 128 the last workgroup of the rows adds the forward's shares up; a launch of its own: 3883 x 8/2, d = 64 66.7 / 55.9, 2 x 1198 x
 // 8/4, d = 64 30.6 / 26.9, 2 x 1039 x 8/2 24.5 / 21.0.)
 // Whole / shares, us (forward; backward with its other kernels): 2316 x 2/1 heads, d = 256 162 / 46, 323 / 180; 3000 x 2/1, d = 64 83 / 25,
@@ -667,7 +672,7 @@ int64_t general_share_units(const FwdParams &p) {
 int general_key_shares(const FwdParams &p, bool dq) {
     if (p.cu_q || p.Lq < 1 || p.Lk < 1) return 1;
     const int gh = shared_rows(p), tile = p.d > 128 ? 32 : 64, tiles = (p.Lk + tile - 1) / tile;
-    if (dq && (tiles < (p.d > 128 ? 16 : 24) || general_rows_256(p))) return 1;
+    if (general_rows_256(p) || (dq && tiles < (p.d > 128 ? 16 : 24))) return 1;
     const int64_t blocks = general_share_units(p);
     int64_t s = blocks > 0 ? device_cus() * (p.d > 64 ? 1 : (gh == 4 ? 3 : 2)) / blocks : 1;
     if (s > tiles / 4) s = tiles / 4;

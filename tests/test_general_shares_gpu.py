@@ -127,6 +127,30 @@ def test_gradients_where_the_kernel_changes(B, Lq, Lk, H, Hk, d, bias_heads, nat
         assert_grad_close(x, want, name)
 
 
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,d,bias_heads", LINE + [(16, 32, 705, 32, 8, 128, 0), (15, 32, 769, 32, 8, 128, 1)])
+def test_forward_where_the_kernel_changes(B, Lq, Lk, H, Hk, d, bias_heads, monkeypatch):
+    """... nor does the forward, with arrival counters or without."""
+    from oracle import eager
+    from flash_sparse_attn import _cabi, flash_sparse_attn_func
+
+    print("line, forward", B, Lq, Lk, H, Hk, d, bias_heads, flush=True)
+    q, k, v, _, mask, bias = _many_heads(B, Lq, Lk, H, Hk, d, bias_heads)
+    ref, ref_lse = eager.attention_forward(q, k, v, mask, bias, None, True)
+
+    def call():
+        _not_a_number_everywhere()
+        with torch.no_grad():
+            return flash_sparse_attn_func(q, k, v, mask, bias, None, True, return_attn_probs=True)[:2]
+
+    runs = [call()]
+    for name in ("fdma_fwd_counter_bytes", "fdma_fwd_optional_bytes"):  # (added up by a launch of its own; whole keys)
+        monkeypatch.setattr(_cabi.lib, name, lambda a: 0)
+        runs.append(call())
+    for out, lse in runs:
+        assert_out_close(out, ref)
+        assert torch.allclose(lse, ref_lse.reshape(lse.shape), atol=2e-3, rtol=1e-3)
+
+
 @pytest.mark.parametrize("B,Lq,Lk,H,Hk,d,kept", [
     (1, 70, 5003, 4, 2, 128, 3000),   # four shares; a row block of six rows
     (2, 16, 8200, 2, 1, 64, 8200),    # eight

@@ -15,7 +15,7 @@ def _ask(B, Lq, Lk, H, Hk, d, bias_heads):
         f.bias, f.num_heads_bias, a.dbias = 256, bias_heads, 256
         for strides in (f.bias_strides, a.dbias_strides):
             strides[0], strides[1], strides[2] = bias_heads * Lq * Lk, Lq * Lk, Lk
-    return a, _cabi.lib.fdma_bwd_optional_bytes(a)
+    return _cabi.lib.fdma_fwd_optional_bytes(f), _cabi.lib.fdma_fwd_counter_bytes(f), _cabi.lib.fdma_bwd_optional_bytes(a)
 
 
 SIZES = [(B, H, Hk) for B in (1, 3, 15, 16, 17, 31, 32, 128, 512, 1024) for H in (1, 2, 4, 8, 12, 16, 32, 64) for Hk in (1, 2, 4, 8, 32) if H % Hk == 0]
@@ -29,9 +29,10 @@ def test_room_only_where_a_kernel_works_on_shares(bias_heads):
             for Lk in (704, 1472, 1473, 4096):
                 for d in (64, 72, 96, 128, 136, 256):
                     rows256 = 64 < d <= 128 and B * H * -(-Lq // 256) >= 512
-                    _, backward = _ask(B, Lq, Lk, H, Hk, d, bias_heads)
+                    forward, counters, backward = _ask(B, Lq, Lk, H, Hk, d, bias_heads)
                     offered += backward > 0
-                    assert not (rows256 and backward), (B, Lq, Lk, H, Hk, d)
+                    assert not (rows256 and (forward or counters or backward)), (B, Lq, Lk, H, Hk, d)
+                    assert (counters > 0) == (forward > 0 and d <= 128)
     assert offered > 1000
 
 
@@ -42,5 +43,6 @@ def test_room_only_where_a_kernel_works_on_shares(bias_heads):
     (1, 32, 4, 1, 128, 8),
 ])
 def test_either_side_of_the_line(B, Lq, H, Hk, d, shares):
-    _, backward = _ask(B, Lq, 4096, H, Hk, d, 0)
+    forward, counters, backward = _ask(B, Lq, 4096, H, Hk, d, 0)
+    assert (forward > 0, counters > 0) == (shares > 1, shares > 1)
     assert backward == (shares * B * H * Lq * d * 4 if shares > 1 else 0)
