@@ -280,7 +280,9 @@ __global__ void __launch_bounds__(NT) make_mask_kernel(const MaskParams p) {
         keep[c] &= inside;
         ties[c] &= inside;
     }
-    // ---- columns kept in front of each chunk, and the first `need` of the ties (with ties, neither count reaches 65536)
+    // ---- columns kept in front of each chunk, and the first `need` of the ties.  Where only some ties are kept, both are counted in the halves of a
+    // register: the others are below 65536, and so is what lies in front of any chunk; the row's ties may be 65536, whose half of the total wraps to
+    // zero and is not looked at
     uint32_t run[KPT], total = 0;
     if (!some_ties) {
 #pragma unroll

@@ -45,3 +45,20 @@ def test_rows(L, fill, kind, dtype):
     assert torch.equal(count.long(), m.sum(-1)) and torch.equal(cnt[:, :L].long(), m.cumsum(-1))
     for i in range(2):
         assert torch.equal(idx[i, : count[i]].long(), m[i].nonzero().flatten())
+
+
+@pytest.mark.parametrize("window", [1, 9, 4096, 65528, 65535, 65536])
+@pytest.mark.parametrize("above", [0, 1, 9])
+def test_largest_row_of_equal_values(window, above):
+    """65536 ties, or nearly as many: the first ones in column order are kept, behind what lies above them."""
+    from flash_sparse_attn.utils.mask import create_mask, kept_keys_of
+
+    L = 65536
+    x = torch.full((1, 1, 1, L), 0.25, dtype=torch.bfloat16)
+    x[..., torch.arange(above) * 7000 + 3] = 1.0
+    got = create_mask(x.to(DEV), None, 1, 1, L, window, torch.finfo(x.dtype).min, type="topk")
+    want = torch.zeros(L, dtype=torch.bool)
+    want[torch.argsort(-x.flatten().float(), stable=True)[:window]] = True
+    assert torch.equal(got.cpu().flatten(), want)
+    idx, cnt, count, _ = [t.cpu() if torch.is_tensor(t) else t for t in kept_keys_of(got)]
+    assert int(count) == window and torch.equal(idx[0, :window].long(), want.nonzero().flatten()) and torch.equal(cnt[0, :L].long(), want.cumsum(0))
