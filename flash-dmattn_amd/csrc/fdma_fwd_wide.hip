@@ -115,12 +115,16 @@ __device__ __forceinline__ void fwd_wide(const FwdParams &p) {
     static_assert(BM * ROW <= (ONE ? 1 : 2) * TILE, "Q fits there");
     auto q_at = [](uint32_t byte) { return byte + (ONE || byte >= TILE ? OFF_V : TILE); };  // (V's second stage is as far behind V as K's end behind K)
     {
-        const gptr_t qb = uniform_ptr((const uint16_t *)p.q + b * p.q_b + (sq.q0 + m0) * p.q_r + h * p.q_h);
-        const uint32_t q_r2 = (uint32_t)(p.q_r * 2), last = (uint32_t)(LqS - 1 - m0 < BM - 1 ? LqS - 1 - m0 : BM - 1) * q_r2;
+        // (offsets are not negative: rows that lie in descending order are counted from the last one)
+        const bool down = p.q_r < 0;
+        const int rows = LqS - 1 - m0 < BM - 1 ? LqS - 1 - m0 : BM - 1;
+        const gptr_t qb = uniform_ptr((const uint16_t *)p.q + b * p.q_b + (sq.q0 + m0 + (down ? rows : 0)) * p.q_r + h * p.q_h);
+        const uint32_t q_r2 = (uint32_t)((down ? -p.q_r : p.q_r) * 2), last = (uint32_t)rows * q_r2;
 #pragma unroll
         for (int i = 0; i < BM * ROW / 8192; i++) {
-            const uint32_t at = (uint32_t)(prow + 8 * C::RPP * i) * q_r2;
-            load_lds16((at < last ? at : last) + pcol, qb, __builtin_amdgcn_readfirstlane(lds0 + q_at(8192 * i) + wave * 1024));
+            uint32_t at = (uint32_t)(prow + 8 * C::RPP * i) * q_r2;
+            at = at < last ? at : last;
+            load_lds16((down ? last - at : at) + pcol, qb, __builtin_amdgcn_readfirstlane(lds0 + q_at(8192 * i) + wave * 1024));
         }
     }
 

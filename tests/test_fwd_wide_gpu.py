@@ -113,3 +113,38 @@ def test_ragged_above_head_dim_128(lens, H, Hk, D, causal):
         s = slice(at, at + n)
         assert_out_close(out[s], eager.attention_forward(q[None, s], k[None, s], v[None, s], None, None, None, causal)[0][0])
         at += n
+
+
+@pytest.mark.parametrize("B,Lq,Lk,H,Hk,D,lists", [
+    (2, 131, 300, 4, 2, 64, False),
+    (1, 3, 300, 4, 2, 96, False),
+    (2, 70, 300, 4, 2, 128, True),
+    (1, 200, 300, 4, 2, 256, False),
+    (5, 512, 512, 8, 4, 256, True),   # 128-row blocks
+])
+def test_query_rows_in_descending_order(B, Lq, Lk, H, Hk, D, lists):
+    """A negative row stride of Q (plain C callers): the same bits as from rows in ascending order."""
+    from flash_sparse_attn import _cabi
+    from flash_sparse_attn.utils import mask as M
+
+    print("descending", B, Lq, Lk, H, Hk, D, lists, flush=True)
+    q, k, v, _, bias = [t if t is None else t.to(DEV) for t in make_inputs(B, Lq, Lk, H, Hk, D, (B, Hk, 1, Lk), seed=Lq + D)]
+    mask = M.topk_mask(bias, None, Lk // 3, torch.finfo(q.dtype).min) if lists else None
+    idx, cnt, count, ld = M.kept_keys_of(mask) if lists else (None,) * 4
+    rows = [q, q.flip(1).contiguous()]
+    results = []
+    set_compact("2" if lists else "0")
+    for i in range(2):
+        out, lse = torch.full_like(q, float("nan")), torch.full((B, H, Lq), float("nan"), dtype=torch.float32, device=DEV)
+        a = _cabi.FwdArgs()
+        _cabi.fill_fwd(a, q, k, v, mask, bias, out, lse, D ** -0.5, True, 0.0, kept=(idx, cnt, count, ld) if lists else None)
+        if lists:
+            assert _cabi.lib.fdma_fwd_takes_lists(a)
+        if i:
+            a.q, a.q_strides[1] = rows[1].data_ptr() + (Lq - 1) * q.stride(1) * 2, -q.stride(1)
+        assert _cabi.lib.fdma_fwd(a, _cabi.current_stream(q.device)) == 0, _cabi.last_error()
+        torch.cuda.synchronize()
+        results.append((out, lse))
+    for x, y in zip(*results):
+        assert torch.equal(x, y)
+    assert torch.isfinite(results[0][0].float()).all()
