@@ -584,10 +584,12 @@ bool use_decode_path(int Lq, int H, int Hk) {
 // 48 pairs, 1000 kept of 30000 keys, 5 splits (240) 20.5 us, 6 (288) 31.0; d = 128, 80 pairs, 2000 of 9000, 3 (240) 21.0, 4 (320) 24.0.
 //   * Up to head dim 128 a CU holds two (three at 64), and where a split then still spans 8192 keys that many are taken, rounded
 //     down too; also two per CU beyond 16384 keys (8192 at 64) where a CU's one would leave a fifth of them idle (88 pairs of 13235 keys,
-//     all kept, d = 64: 2 splits 73.2, 3 62.0, 5 59.4).
-// 4773 calls of 12 to 256 pairs over 1024 to 65536 keys, against the same numbers rounded up: 1.026 / 1.044 / 1.149 times as fast at d = 64 / 128 /
-// 256 (4 % to 6 % behind the best number of each call, 2 % at 256), 40 of them more than 3 % slower, one more than 10 (10 x 21738
-// x 8/2, d = 128, 128 kept: 11.5 / 13.8), 1695 more than 3 % faster.
+//     all kept, d = 64: 2 splits 73.2, 3 62.0, 5 59.4), and at 64 where a CU's one is two splits: 104 to 127 pairs, 220
+//     calls of 8192 to 65536 keys, by length and share kept: 2 are 0.87 to 1.04 times as fast as the number rounded up, 4 1.01 to 1.08
+//     (108 pairs of 11806, all kept, 3 / 2 / 4: 67.2 / 71.8 / 64.8).
+// Against the same numbers rounded up, 2400 calls of 12 to 256 pairs over 1024 to 65536 keys, 128 to all of them kept, whose number differs: 1.18
+// times as fast, 26 of them more than 3 % slower and three more than 10 (192 pairs, d = 64: 12 x 26023 x 32/16, all kept 256 / 294,
+// 24 x 27510 x 8/8, half 144 / 164; d = 128: 18 x 53394 x 4/4, 128 kept 10.8 / 12.4).
 // Few (batch entry, kv head) pairs do not take the whole chip: every split adds some 60 ns of arrival and merge, so there are at
 // most 32, or one for 1280 keys beyond 32768 keys.  Sparse masks are served best by few splits, masks that keep every key by
 // many, and the host does not know which it is.  us, spans of 768 / 1024 / 1280 / 2048 keys, one pair of four heads, d = 64 | 128 | 256:
@@ -605,13 +607,14 @@ bool use_decode_path(int Lq, int H, int Hk) {
 // d = 64, 150 kept 8.2 -> 7.1; 384, all kept, d = 128 10.5 -> 9.7 (512 keys, all kept: 10.7 in two, 11.1 in one).
 // With keys_per_split rounded up to 256 every split is non-empty.
 int decode_num_splits(int B, int H, int Hk, int Lk, int d, bool masked) {
-    const int pairs = B * Hk > 0 ? B * Hk : 1;
+    const int pairs = B * Hk > 0 ? B * Hk : 1, cus = device_cus();
     int splits = 0;
     for (int per_cu = d <= 64 ? 3 : (d <= 128 ? 2 : 1); per_cu > 1 && splits == 0; per_cu--)
-        if ((int64_t)(256 * per_cu / pairs) * 8192 <= Lk) splits = 256 * per_cu / pairs;
+        if ((int64_t)(cus * per_cu / pairs) * 8192 <= Lk) splits = cus * per_cu / pairs;
     if (splits == 0) {
-        splits = 256 / pairs;
-        if (d <= 128 && splits * pairs < 208 && Lk >= (d <= 64 ? 8192 : 16384)) splits = 512 / pairs;
+        splits = cus / pairs;
+        const bool idle = 16 * splits * pairs < 13 * cus || (d <= 64 && splits == 2 && 2 * pairs < cus);
+        if (d <= 128 && idle && Lk >= (d <= 64 ? 8192 : 16384)) splits = 2 * cus / pairs;
         const int least = !masked && pairs <= 2 && B * H <= 64 ? 64 : 32, spans = (Lk + 1279) / 1280;
         const int most = Lk > 32768 ? (spans > least ? spans : least) : 32;
         if (splits > most) splits = most;

@@ -71,6 +71,11 @@ def test_splits_without_a_mask(B, H, Hk, Lk, masked, unmasked):
     (8, 65535, 8, 128, 4),
     (12, 61888, 16, 64, 4),   # three
     (11, 8192, 8, 64, 5),
+    (13, 28627, 8, 64, 4),    # two splits of 104 pairs to 127 would be one workgroup to most CUs, which hold three at d = 64
+    (127, 8192, 1, 64, 4),
+    (127, 8191, 1, 64, 2),
+    (16, 28627, 8, 64, 2),    # (128 pairs: one to every CU)
+    (13, 28627, 8, 72, 2),
     (300, 65536, 1, 128, 1),
     (2, 4093, 64, 256, 2),
 ])
