@@ -668,7 +668,8 @@ int64_t general_share_units(const FwdParams &p) {
 // 8/4, d = 64 30.6 / 26.9, 2 x 1039 x 8/2 24.5 / 21.0.)
 // Whole / shares, us (forward; backward with its other kernels): 2316 x 2/1 heads, d = 256 162 / 46, 323 / 180; 3000 x 2/1, d = 64 83 / 25,
 // 141 / 75; 2240 x 2/1, d = 96 56 / 24, 107 / 72; 4096 x 2/1, d = 128 98 / 39, 172 / 106; 3000 x 8/2, d = 64 81 / 41, 198 / 171; 1999 x 8/4,
-// not causal 61 / 43, 138 / 119.
+// not causal 61 / 43, 138 / 119.  Rows that are not whole chunks, in instantiations of their own (forward; backward without a bias): 2999 x 2/1, d = 64
+// 101 / 28, 143 / 69; 2239 x 2/1, d = 96 60 / 28, 104 / 64; 4095 x 2/2, d = 128 130 / 48, 182 / 102; 3001 x 8/2, d = 64 85 / 45, 177 / 135.
 int general_key_shares(const FwdParams &p, bool dq) {
     if (p.cu_q || p.Lq < 1 || p.Lk < 1) return 1;
     const int gh = shared_rows(p), tile = p.d > 128 ? 32 : 64, tiles = (p.Lk + tile - 1) / tile;

@@ -35,3 +35,13 @@ def test_sums_of_parts_stay_apart_from_dq():
     assert len(dq) == 2 * (2 + 4)
     for name, k in dq.items():
         assert k[".sgpr_spill_count"] <= 20 and k[".vgpr_spill_count"] == 0, name
+
+
+def test_forward_with_key_groups():
+    """The forward with key groups keeps a lane's state in registers up to head dim 128; above, where O alone is 128 of them and Q 64, up
+    to five do not fit (20 bytes a lane, in the kernel that reads a list's rows where they lie)."""
+    fwd = {n: k for n, k in kernels().items() if "fwd_wide_kernel" in n or "fwd_96_kernel" in n or "fwd_list_kernel" in n}
+    assert len(fwd) == 2 * (4 * 4 + 4 + 4 * 2)
+    for name, k in fwd.items():
+        most = (5, 20) if "Li256E" in name else (0, 0)
+        assert (k[".vgpr_spill_count"], k[".private_segment_fixed_size"]) <= most and k[".private_segment_fixed_size"] <= most[1], name
