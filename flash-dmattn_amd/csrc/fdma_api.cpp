@@ -349,7 +349,8 @@ size_t fdma_fwd_optional_bytes(const fdma_fwd_args *a) {
     return general_fwd(a, p) ? share_bytes(p, true, fdma::general_key_shares(p, false)) : 0;
 }
 
-int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
+// `most_splits`: of a decode call (0: as many as decode_num_splits says, what callers make room for)
+static int forward(const fdma_fwd_args *a, void *hip_stream, int most_splits) {
     if (int cap = refuse_capture(hip_stream, "fdma_fwd")) return cap;
     g_err[0] = 0;
     int rc = validate_common(a, false);
@@ -361,11 +362,11 @@ int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
     if (a->seqlen_q == 0) return FDMA_OK;
     if (fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k) && a->seqlen_k > 0) {
         p.splits = fdma::decode_num_splits(a->batch, a->num_heads, a->num_heads_k, a->seqlen_k, a->head_dim, a->mask != nullptr);
+        if (most_splits && p.splits > most_splits) p.splits = most_splits;
         if (p.splits > 1) {
-            const size_t need = fdma_fwd_workspace_bytes(a);
+            const size_t rows = (size_t)p.splits * a->batch * a->num_heads * a->seqlen_q, need = rows * (size_t)(a->head_dim + 1) * sizeof(float);
             if (!a->workspace || a->workspace_bytes < need)
                 return fail(FDMA_ERR_WORKSPACE, "forward workspace too small: need %zu bytes, got %zu", need, a->workspace_bytes);
-            const size_t rows = (size_t)p.splits * a->batch * a->num_heads * a->seqlen_q;
             p.o_part = static_cast<float *>(a->workspace);
             p.lse_part = p.o_part + rows * a->head_dim;
             if (a->counters) {
@@ -407,6 +408,8 @@ int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) {
     return FDMA_OK;
 }
 
+int fdma_fwd(const fdma_fwd_args *a, void *hip_stream) { return forward(a, hip_stream, 0); }
+
 int fdma_fwd_noalloc(const fdma_fwd_args *a, void *hip_stream) {
     g_err[0] = 0;
     int rc = validate_common(a, false);
@@ -415,7 +418,12 @@ int fdma_fwd_noalloc(const fdma_fwd_args *a, void *hip_stream) {
     size_t need = fwd_scratch_bytes(a, &shares);
     constexpr size_t kUsable = (size_t)FDMA_NOALLOC_SCRATCH_BYTES - FDMA_NOALLOC_COUNTER_BYTES;
     fdma_fwd_args with_scratch = *a;
-    if (need > kUsable && !fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k)) {
+    int most_splits = 0;
+    if (need > kUsable && fdma::use_decode_path(a->seqlen_q, a->num_heads, a->num_heads_k)) {
+        const size_t split = (size_t)a->batch * a->num_heads * (size_t)(a->head_dim + 1) * sizeof(float);
+        most_splits = fdma::decode_splits_at_most((int)(kUsable / split), a->seqlen_k);
+        need = most_splits > 1 ? most_splits * split : 0;
+    } else if (need > kUsable) {
         fdma::FwdParams p, pv;
         fill_fwd_params(a, p);
         if (fdma::compact_per_query_head(p, pv)) p = pv;
@@ -443,7 +451,7 @@ int fdma_fwd_noalloc(const fdma_fwd_args *a, void *hip_stream) {
             with_scratch.counters_bytes = FDMA_NOALLOC_COUNTER_BYTES;
         }
     }
-    return fdma_fwd(&with_scratch, hip_stream);
+    return forward(&with_scratch, hip_stream, most_splits);
 }
 
 int fdma_bwd_validate(const fdma_bwd_args *a) {

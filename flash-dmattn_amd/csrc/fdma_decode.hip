@@ -622,8 +622,12 @@ int decode_num_splits(int B, int H, int Hk, int Lk, int d, bool masked) {
     const int max_by_len = Lk <= 384 ? 1 : (Lk + 255) / 256;
     if (splits > max_by_len) splits = max_by_len;
     if (splits > CMB_MAX_SPLITS) splits = CMB_MAX_SPLITS;
+    return decode_splits_at_most(splits, Lk);
+}
+
+// shrinks so that no split is empty after rounding keys_per_split up to a multiple of 256
+int decode_splits_at_most(int splits, int Lk) {
     if (splits < 1) splits = 1;
-    // shrink so that no split is empty after rounding keys_per_split up to a multiple of 256
     while (splits > 1) {
         const int kps = ((Lk + splits - 1) / splits + 255) / 256 * 256;
         if ((int64_t)(splits - 1) * kps < Lk) break;

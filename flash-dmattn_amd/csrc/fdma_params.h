@@ -536,6 +536,7 @@ int device_cus();
 
 // number of KV splits the decode path uses for this shape, with a mask or without (1 = no workspace needed)
 int decode_num_splits(int B, int H, int Hk, int Lk, int d, bool masked);
+int decode_splits_at_most(int splits, int Lk);
 // arrival counters the one-launch decode needs for this shape (0 without splits)
 int64_t decode_num_counters(int B, int H, int Hk, int Lk, int d);
 bool use_decode_path(int Lq, int H, int Hk);

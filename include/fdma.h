@@ -189,7 +189,7 @@ int fdma_bwd(const fdma_bwd_args *args, void *hip_stream);
  * decode path (split-KV partials) or of the compaction path lives in a static device array of
  * FDMA_NOALLOC_SCRATCH_BYTES inside the library, which every GPU the library runs on holds until the process ends.
  * A problem whose fdma_fwd_workspace_bytes() exceeds that returns FDMA_ERR_WORKSPACE and launches nothing -- unless all that
- * does not fit are the partial results of split keys (the keys stay whole) or, under FDMA_COMPACT_AUTO, copies that are made
+ * does not fit are the partial results of split keys (fewer splits; or the keys stay whole) or, under FDMA_COMPACT_AUTO, copies that are made
  * for few query rows against many keys (tiles are skipped instead).  The call makes no hipMalloc / hipFree (nor any other
  * allocating call); apart from those two, results are bit-identical to fdma_fwd's.
  * Every call on a GPU uses that GPU's one array: calls that overlap on one GPU (different streams or host

@@ -79,6 +79,28 @@ def test_noalloc_entry_point_rejects_what_does_not_fit():
     assert torch.isnan(out.float()).all()   # nothing was launched
 
 
+@pytest.mark.parametrize("size", [(127, 8192, 64, 1, 64), (64, 4096, 64, 1, 256), (100, 16384, 64, 1, 72)])
+def test_noalloc_decode_takes_the_splits_that_fit(size):
+    """Partial results of more splits than the static array holds: fewer splits (of the second call, one), the same up to a rounding."""
+    from flash_sparse_attn import _cabi
+
+    print(f"no-alloc splits {size}", flush=True)
+    B, Lk, H, Hk, D = size
+    g = torch.Generator(device=DEV).manual_seed(Lk)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)
+    q, k, v, bias = r(B, 1, H, D), r(B, Lk, Hk, D), r(B, Lk, Hk, D), r(B, 1, 1, Lk)
+    mask = torch.rand(B, 1, 1, Lk, generator=g, device=DEV) < 0.1
+    rc0, out0, lse0, need = _call("fdma_fwd", q, k, v, mask, bias, False, _cabi.COMPACT_AUTO, own_workspace=True)
+    assert rc0 == 0, _cabi.last_error()
+    assert need > _cabi.NOALLOC_SCRATCH_BYTES - (64 << 10)
+    rc1, out1, lse1, _ = _call("fdma_fwd_noalloc", q, k, v, mask, bias, False, _cabi.COMPACT_AUTO, own_workspace=False)
+    assert rc1 == 0, _cabi.last_error()
+    assert ((lse1 - lse0).abs() <= 1e-5 * (1 + lse0.abs())).all()
+    # (a probability is rounded to eps / 2 of itself against the reference point of either split)
+    a, b = out1.float(), out0.float()
+    assert ((a - b).abs() <= torch.finfo(torch.bfloat16).eps * (2 * b.abs() + b.abs().max())).all()
+
+
 def test_noalloc_entry_point_allocates_no_device_memory():
     """The property the entry point exists for: after one warm-up call (code object, per-device scratch address), a
     call changes neither the device's free memory (hipMemGetInfo) nor the tensor library's allocation counters.  The
